@@ -170,8 +170,10 @@ def _w4a16_handler(op, bound, env, stream) -> bool:
             cands = [16 * rows + waves for rows in (8, 4) for waves in ((4, 8) if M == 1 else (4,))]
         else:
             counts = [v for v in (1, 2, 3, 4, 5, 6, 8, 10, 12, 16, 20, 24, 32) if v <= K // 128]
-            # 512 + v: v K-splits over blocks of 64 rows; 256 + v: over blocks of 32 rows (twice the blocks)
+            # 512 + v: v K-splits over blocks of 64 rows; 256 + v: over blocks of 32 rows (twice the blocks);
+            # 1024 + v, 2048 + v: over blocks of 128 and 256 rows
             cands = [0] + [512 + v for v in counts] + ([256 + v for v in counts] if M > 32 else [])
+            cands += [rows + v for rows in (1024, 2048) for v in counts if v <= 16] if M > 64 else []
         saved = tune_hand_kernel(op, key, cands, lambda v, t: run(v, t, torch.cuda.current_stream().cuda_stream), trials, clones)
         del clones
     run(saved['value'] if saved is not None else 0, (x, q, s, z, y))

@@ -26,18 +26,12 @@
 //   * split-K without atomics (5.6 M float atomics cost 75 us on this chip): each K-split writes its fp32 tile to the
 //     library workspace and a second small kernel adds the splits in a fixed order and rounds once to fp16 - results
 //     do not depend on timing.
-#include "art_common.h"
+#include "art_w4_mfma.h"
 
 namespace {
 
-typedef _Float16 h8 __attribute__((ext_vector_type(8)));
-typedef _Float16 h4 __attribute__((ext_vector_type(4)));
-typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-typedef float f16v __attribute__((ext_vector_type(16)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
-typedef int i32x2 __attribute__((ext_vector_type(2)));
-typedef __attribute__((address_space(3))) i32x2 lds_i32x2;
+using namespace art::w4;
+
 
 constexpr int kThreads = 512;                       // 8 wavefronts: 4 column quarters x 2 k halves
 constexpr int BM = 64, BN = 256, GK = 128;          // rows and columns of a block, k of a quantisation group
@@ -49,27 +43,6 @@ constexpr int STAGE = W_BYTES + X_BYTES + Q_BYTES;
 constexpr int RLD = BN + 4;                         // floats per row of a result tile in LDS
 constexpr size_t kLdsBytes = (size_t)NS * STAGE;    // 139264; the two result tiles of the epilogue (133120) reuse it
 static_assert(2 * BM * RLD * sizeof(float) <= kLdsBytes, "the result tiles fit the ring");
-
-struct Magic {
-  unsigned int mask_lo, mask_hi, bias_lo, bias_hi;   // 0x000F000F 0x00F000F0 0x64006400 0x54005400
-};
-
-__device__ __forceinline__ h2 as_h2(unsigned int v) { return __builtin_bit_cast(h2, v); }
-
-// (w & mask) | bias in one v_bitop3_b32 (truth table 0xEA = (a & b) | c).
-__device__ __forceinline__ unsigned int and_or(unsigned int w, unsigned int mask, unsigned int bias) {
-  return __builtin_amdgcn_bitop3_b32(w, mask, bias, 0xEA);
-}
-
-// 8 halves of x in the k order the nibble extraction leaves in a B operand: k0 k4 k1 k5 k2 k6 k3 k7.
-__device__ __forceinline__ h8 permute_k(u32x4 v) {
-  u32x4 o;
-  o[0] = __builtin_amdgcn_perm(v[2], v[0], 0x05040100u);
-  o[1] = __builtin_amdgcn_perm(v[2], v[0], 0x07060302u);
-  o[2] = __builtin_amdgcn_perm(v[3], v[1], 0x05040100u);
-  o[3] = __builtin_amdgcn_perm(v[3], v[1], 0x07060302u);
-  return __builtin_bit_cast(h8, o);
-}
 
 // 64 lanes x 16 (4) bytes from global memory straight into LDS: lane l's bytes land at lds_dst + 16 l (4 l); the lane
 // chooses its global address freely.  The instruction takes the LDS address from m0, which is put back afterwards.
@@ -338,6 +311,77 @@ int choose_splits(int rows, int N, int K, size_t scratch_bytes, int compute_unit
   return s < 1 ? 1 : s;
 }
 
+// Rows per block of this file's kernel at the library's choice.  32 rows where twice the blocks fill the chip better than
+// twice the K-splits do - a block of 32 rows unpacks the same weights for half the matrix instructions, but every K-split
+// it saves is an fp32 copy of the output less to write and read back.  Measured at M = 64 and 128 on MI355X: 32-row
+// blocks win where one block per compute unit then covers at least four K-splits' worth of (column tile, row block)
+// pairs (M = 64: up to 8192 columns, M = 128: 4096), and lose where they would need a second round of blocks; beyond
+// 64 rows also where the loop over K is long (128 rows over 11008 x 4096: 27.2 us against 25.8 with 64-row blocks; over
+// 4096 x 4096: 17.3 against 19.7).
+int choose_block_rows(int M, int K, int N, int compute_units) {
+  if (M <= 32) return 32;
+  const int col_tiles = (N + BN - 1) / BN;
+  return (M <= 64 || (M <= 128 && K <= 8192)) && col_tiles * ((M + 31) / 32) * 4 <= compute_units ? 32 : BM;
+}
+
+constexpr int kMaxRowBlocks = 8;                    // row blocks of one launch: they share the weight stream through L2
+
+// ---- What a launch takes, in microseconds, from sweeps of 48 to 1003 rows over eight weight shapes (1024 x 3072 to
+// 4096 x 22016 and 11008 x 4096) on MI355X; within 10 % of the measured times above 96 rows.
+double split_cost(double rows, double N, int splits) {     // the second launch, and the fp32 tiles at 6 TB/s
+  return splits == 1 ? 0.0 : 2.5 + (8.0 * splits + 2.0) * rows * N / 6.0e6;
+}
+double estimate_narrow(int M, int K, int N, size_t scratch_bytes, int compute_units) {
+  const int block_rows = choose_block_rows(M, K, N, compute_units), col_tiles = (N + BN - 1) / BN, G = K / GK;
+  double t = 0;
+  for (int m0 = 0; m0 < M; m0 += block_rows * kMaxRowBlocks) {
+    const int rows = M - m0 < block_rows * kMaxRowBlocks ? M - m0 : block_rows * kMaxRowBlocks;
+    const int m_blocks = (rows + block_rows - 1) / block_rows;
+    const int splits = choose_splits(rows, N, K, scratch_bytes, compute_units / m_blocks);
+    const int rounds = (col_tiles * m_blocks * splits + compute_units - 1) / compute_units;
+    t += 5.0 + rounds * ((G + splits - 1) / splits) * (block_rows == BM ? 1.05 : 0.8) + split_cost(rows, N, splits);
+  }
+  return t;
+}
+double estimate_wide(int M, int K, int N, int row_tiles, int splits, int compute_units) {
+  const int col_tiles = (N + 255) / 256, m_blocks = (M + 32 * row_tiles - 1) / (32 * row_tiles), G = K / GK;
+  const double stages = 2 * ((G + splits - 1) / splits), blocks = (double)col_tiles * m_blocks * splits;
+  double t = 6.0 + split_cost(M, N, splits);
+  if (row_tiles == 8) {             // one block per compute unit; a fuller chip clocks lower
+    const int rounds = (int)((blocks + compute_units - 1) / compute_units);
+    t += rounds * stages * (1.05 + 0.25 * blocks / ((double)rounds * compute_units));
+  } else {                          // two
+    const int full = (int)(blocks / (2 * compute_units));
+    const double rest = blocks - 2.0 * full * compute_units;
+    t += full * stages * 1.62;
+    if (rest > compute_units) t += stages * 1.62;
+    else if (rest > 0) t += stages * (0.70 + 0.15 * rest / compute_units);
+  }
+  return t;
+}
+// Row tiles and K-splits for art_gemm_w4_wide.hip, or 0 where this file's kernel is the better one: blocks of 32 and 64
+// rows start sooner and fill the chip at smaller sizes, those of 128 and 256 rows multiply faster (M = 1003 over
+// 4096 x 12288: 93 against 156 us, 4096 x 22016: 166 against 248; M = 128 over 4096 x 4096: 21 against 17).
+int choose_wide(int M, int K, int N, size_t scratch_bytes, int compute_units, int* splits) {
+  if (M <= 64) return 0;
+  double best = estimate_narrow(M, K, N, scratch_bytes, compute_units) - 1.5;
+  int row_tiles = 0;
+  for (int rt = 4; rt <= 8; rt += 4)
+    for (int s = 1; s <= 16 && s <= K / (2 * GK); ++s) {
+      if (s > 1 && (size_t)s * M * N * sizeof(float) > scratch_bytes) break;
+      const double t = estimate_wide(M, K, N, rt, s, compute_units);
+      if (t < best) { best = t; row_tiles = rt; *splits = s; }
+    }
+  return row_tiles;
+}
+
+int combine(const float* partial, _Float16* y, int rows, int N, int splits, const _Float16* residual, hipStream_t stream) {
+  const long long count4 = (long long)rows * N / 4;
+  gemm_w4a16_combine_kernel<<<dim3((unsigned)((count4 + 255) / 256)), 256, 0, stream>>>(partial, y, count4, (long long)rows * N, splits, residual);
+  ART_LAUNCH_CHECK();
+  return 0;
+}
+
 }  // namespace
 
 extern "C" int art_gemm_w4a16(const void* x_dev, const void* qweight_dev, const void* scales_dev, const void* qzeros_dev,
@@ -352,7 +396,9 @@ extern "C" int art_gemm_w4a16_tuned(const void* x_dev, const void* qweight_dev, 
 
 extern "C" int art_gemm_w4a16_residual(const void* x_dev, const void* qweight_dev, const void* scales_dev, const void* qzeros_dev,
                                        void* y_dev, const void* residual_dev, int M, int K, int N, int k_splits, void* stream) {
-  ART_REQUIRE(k_splits >= 0 && k_splits < 0x300, "art_gemm_w4a16: k_splits must be 0 (library's choice) or 1..255, plus 256 x the rows-per-block code (got %d)", k_splits);
+  const int want_rows = k_splits >> 8;              // 0: library's choice; else rows of a block / 32
+  ART_REQUIRE(k_splits >= 0 && (want_rows <= 2 || want_rows == 4 || want_rows == 8),
+              "art_gemm_w4a16: k_splits must be 0 (library's choice) or 1..255, plus 256 x the rows-per-block code 1, 2, 4 or 8 (got %d)", k_splits);
   ART_REQUIRE(((uintptr_t)residual_dev % 8) == 0, "art_gemm_w4a16: the residual must be 8-byte aligned");
   ART_REQUIRE(!art::overlaps(x_dev, (size_t)M * K * 2, y_dev, (size_t)M * N * 2), "art_gemm_w4a16: y must not overlap x");
   ART_REQUIRE(x_dev && qweight_dev && scales_dev && qzeros_dev && y_dev, "art_gemm_w4a16: null pointer");
@@ -379,24 +425,23 @@ extern "C" int art_gemm_w4a16_residual(const void* x_dev, const void* qweight_de
   const Magic mg{0x000F000Fu, 0x00F000F0u, 0x64006400u, 0x54005400u};
   hipStream_t st = (hipStream_t)stream;
   const int G = K / GK, col_tiles = (N + BN - 1) / BN;
-  // Up to kMaxRowBlocks row blocks go into one launch (they share the weight stream through L2, and the K-splits
-  // are combined once); longer batches take several passes over the weights.
-  // Rows per block: 64, or 32 where twice the blocks fill the chip better than twice the K-splits do - a block of 32
-  // rows unpacks the same weights for half the matrix instructions, but every K-split it saves is an fp32 copy of
-  // the output less to write and read back.  The caller's choice arrives in the upper bits of k_splits.
-  constexpr int kMaxRowBlocks = 8;
-  const int want_rows = k_splits >> 8;              // 0: library's choice, 1: 32-row blocks, 2: 64-row blocks
+  // Up to kMaxRowBlocks row blocks of this file's kernel go into one launch; longer batches take several passes over the
+  // weights.  The caller's choice of kernel and rows per block arrives in the upper bits of k_splits.
   k_splits &= 0xff;
-  ART_REQUIRE(want_rows <= 2, "art_gemm_w4a16: rows-per-block code must be 0, 1 or 2 (got %d)", want_rows);
-  int block_rows = BM;
-  if (want_rows == 1 || M <= 32) block_rows = 32;
-  else if (want_rows == 0 && (M <= 64 || (M <= 128 && K <= 8192))) {
-    // measured at M = 64 and 128 on MI355X: 32-row blocks win where one block per compute unit then covers at least
-    // four K-splits' worth of (column tile, row block) pairs (M = 64: up to 8192 columns, M = 128: 4096), and lose
-    // where they would need a second round of blocks; beyond 64 rows also where the loop over K is long (128 rows
-    // over 11008 x 4096: 27.2 us against 25.8 with 64-row blocks; over 4096 x 4096: 17.3 against 19.7)
-    if (col_tiles * ((M + 31) / 32) * 4 <= compute_units) block_rows = 32;
+  int row_tiles = want_rows >= 4 ? want_rows : 0, wide_splits = k_splits;
+  if (want_rows == 0 && k_splits == 0) row_tiles = choose_wide(M, K, N, scratch_bytes, compute_units, &wide_splits);
+  if (row_tiles) {
+    const size_t per_split = (size_t)M * N * sizeof(float);
+    if (wide_splits > G) wide_splits = G;
+    if ((size_t)wide_splits * per_split > scratch_bytes) wide_splits = (int)(scratch_bytes / per_split);
+    if (wide_splits < 1) wide_splits = 1;
+    if (art::w4::gemm_wide((const _Float16*)x_dev, (const unsigned char*)qweight_dev, (const _Float16*)scales_dev,
+                           (const unsigned char*)qzeros_dev, (_Float16*)y_dev, scratch, M, K, N, wide_splits, row_tiles,
+                           (const _Float16*)residual_dev, st))
+      return 1;
+    return wide_splits > 1 ? combine(scratch, (_Float16*)y_dev, M, N, wide_splits, (const _Float16*)residual_dev, st) : 0;
   }
+  const int block_rows = want_rows == 1 ? 32 : want_rows == 2 ? (M <= 32 ? 32 : BM) : choose_block_rows(M, K, N, compute_units);
   for (int m0 = 0; m0 < M; m0 += block_rows * kMaxRowBlocks) {
     const int rows = M - m0 < block_rows * kMaxRowBlocks ? M - m0 : block_rows * kMaxRowBlocks;
     const int m_blocks = (rows + block_rows - 1) / block_rows;
@@ -419,12 +464,7 @@ extern "C" int art_gemm_w4a16_residual(const void* x_dev, const void* qweight_de
                                                          (const unsigned char*)qzeros_dev, ys, scratch, rows, K, N, splits,
                                                          col_tiles, m_blocks, mg, rs);
     ART_LAUNCH_CHECK();
-    if (splits > 1) {
-      const long long count4 = (long long)rows * N / 4;
-      gemm_w4a16_combine_kernel<<<dim3((unsigned)((count4 + 255) / 256)), 256, 0, st>>>(scratch, ys, count4, (long long)rows * N,
-                                                                                        splits, rs);
-      ART_LAUNCH_CHECK();
-    }
+    if (splits > 1 && combine(scratch, ys, rows, N, splits, rs, st)) return 1;
   }
   return 0;
 }

@@ -1,0 +1,333 @@
+// Weight-only int4 GEMM for large batches (whole prompts): the arithmetic of art_gemm_w4.hip,
+//     y[m,n] = sum_k x[m,k] * w[k,n],   w[k,n] = fp16(s[g,n] * fp16(q[k,n] - z[g,n])),   group g = k / 128,
+// on the matrix cores with fp32 accumulation.  Blocks of 64 rows spend more time unpacking weights than multiplying
+// them (166 vector instructions per 16 MFMAs and wavefront); here a block owns 128 or 256 rows, so that an unpacked
+// weight is multiplied by four or eight row tiles.
+//
+//   * four wavefronts, each 32 MT rows x 64 columns (MT = 4: 128 accumulator registers and two blocks per compute
+//     unit, MT = 8: 256 and one wavefront per SIMD).  No two wavefronts unpack the same weight.  What bounds the loop is
+//     the issue of vector instructions beside the MFMAs: one wavefront alone gets four of them into the shadow of an
+//     MFMA (32 cycles) and pays 7 cycles for every further one, two wavefronts get six each.  Hence pairs of k in
+//     natural order (one v_perm more per pair of weights) instead of a permutation of every x operand: 2.9 vector
+//     instructions per MFMA at MT = 8 against 4.6 (90 us against 103 for 1003 rows over 4096 x 4096);
+//   * per 64 values of k a block needs 8 KiB of packed weights, 4 MT KiB of x and the group's scales and zero points;
+//     they go from global memory straight into LDS (global_load_lds, no registers in flight), a ring of three slots.
+//     The weights run a stage ahead of x, so that the first operands of a stage can be unpacked in the stage before;
+//   * the chunk positions are swizzled so that every 16 lanes of a 16-byte read of x (rows 128 bytes apart), and of a
+//     transposing byte read of the weights, touch every bank once (SQ_LDS_BANK_CONFLICT 5.9 M -> 0.3 M per launch);
+//   * one round = 16 values of k per lane half = 2 MT MFMAs.  The operands of round e + 1 are read and unpacked between
+//     the MFMAs of round e, in four chunks fenced against the scheduler; each chunk also issues at most one load.  Left
+//     together the loads of a stage blocked every wavefront of the compute unit at once (about 700 cycles per stage:
+//     90 -> 71 us).
+// Measured (MI355X, 1003 rows): 4096 x 12288 93 us = 1.09 PFLOP/s, 4096 x 22016 166 us, 11008 x 4096 96 us, 4096 x 4096
+// 46 us with two K-splits; the 64-row blocks of art_gemm_w4.hip: 156, 248, 130 and 62 us.
+#include "art_w4_mfma.h"
+
+#include <type_traits>
+
+namespace {
+
+using namespace art::w4;
+
+constexpr int kThreads = 256;
+constexpr int BN = 256, SK = 64;                    // columns of a block, k of a stage
+constexpr int NS = 3;                               // stages of the LDS ring
+constexpr int W_BYTES = (SK / 2) * BN;              // 32 byte-rows x 256 columns
+constexpr int Q_BYTES = 1024;                       // scales (512 B), zero points (128 B), idle lanes
+constexpr int C_LD = BN + 8;                        // halves per row of the staged output
+constexpr int stage_bytes(int MT) { return W_BYTES + Q_BYTES + MT * 32 * SK * 2; }
+constexpr size_t lds_bytes(int MT) { return (size_t)NS * stage_bytes(MT); }
+static_assert(128 * C_LD * 2 <= NS * stage_bytes(4), "128 staged output rows fit the ring");
+
+// 64 lanes x 16 (4) bytes from base + lane offset straight into LDS at lds_dst + 16 (4) * lane.  The instruction takes
+// the LDS address from m0, which is put back.  The waits are written by hand: the compiler does not see these loads.
+__device__ __forceinline__ void load_lds_x4(const void* base, unsigned int off, unsigned int lds_dst) {
+  unsigned int keep;
+  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b32 m0, %0"
+               : "=&s"(keep) : "v"(off), "s"(base), "s"(lds_dst));
+}
+__device__ __forceinline__ void load_lds_x1(const void* base, unsigned int off, unsigned int lds_dst) {
+  unsigned int keep;
+  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2\n\ts_mov_b32 m0, %0"
+               : "=&s"(keep) : "v"(off), "s"(base), "s"(lds_dst));
+}
+
+template <int MT>
+__global__ __launch_bounds__(kThreads, MT == 8 ? 1 : 2) void gemm_w4a16_wide_kernel(
+    const _Float16* __restrict__ x, const unsigned char* __restrict__ qweight, const _Float16* __restrict__ scales,
+    const unsigned char* __restrict__ qzeros, _Float16* y, float* __restrict__ partial, int M, int K, int N, int splits,
+    int col_tiles, int m_blocks, Magic mg, const _Float16* residual) {       // residual may be y itself
+  constexpr int STAGE = stage_bytes(MT), BM = 32 * MT;
+  constexpr int L = 2 + MT + 1;                     // loads per wavefront and stage
+  extern __shared__ __align__(1024) unsigned char smem[];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // the row blocks of one (column tile, K split) have block ids 8 apart: the same XCD, whose L2 then serves the weights
+  const int unit = (int)(blockIdx.x / (8 * m_blocks)) * 8 + (int)(blockIdx.x % 8);
+  const int m_block = (int)(blockIdx.x % (8 * m_blocks)) / 8;
+  if (unit >= col_tiles * splits) return;
+  const int split = unit / col_tiles;
+  const int n0 = (unit % col_tiles) * BN, m0 = m_block * BM;
+  const int G = K / 128;
+  const int g_begin = (int)((long long)G * split / splits), g_end = (int)((long long)G * (split + 1) / splits);
+  const int steps = 2 * (g_end - g_begin);          // splits <= G: at least two
+  const unsigned int lds0 = (unsigned int)(size_t)(__attribute__((address_space(3))) unsigned char*)smem;
+
+  // ---- what this lane fetches per stage.  Columns past N and rows past M re-read valid memory; nothing of them is stored.
+  unsigned int woff[2], xoff[MT], qoff;
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const int r = 4 * (wave + 4 * u) + (lane >> 4);
+    const int col = n0 + ((lane & 15) ^ (r & 7)) * 16;
+    woff[u] = (unsigned int)r * N + (col < N ? col : 0);
+  }
+#pragma unroll
+  for (int u = 0; u < MT; ++u) {
+    const int r = 8 * (wave + 4 * u) + (lane >> 3), row = m0 + r < M ? m0 + r : M - 1;
+    xoff[u] = (unsigned int)(row - m0) * (2 * K) + (((lane & 7) ^ ((r >> 1) & 7)) * 16);
+  }
+  const unsigned char* wbase = qweight + (size_t)g_begin * 64 * N;
+  const unsigned char* xbase = reinterpret_cast<const unsigned char*>(x + (size_t)m0 * K + (size_t)g_begin * 128);
+  // scales and zero points share one load: wavefronts 0 and 1 fetch the scales of columns 2 d, 2 d + 1, half of
+  // wavefront 2 the zero points of columns 8 (d - 128) .. + 7, the others repeat the first scales
+  const bool is_zero = tid >= 128 && tid < 160;
+  const int qcol = tid < 128 ? n0 + 2 * tid : n0 + 8 * (tid - 128);
+  qoff = is_zero ? (unsigned int)((qcol < N ? qcol : 0) >> 1) : (tid < 128 ? 2u * (qcol < N ? qcol : 0) : 0u);
+  const unsigned char* qbase = wave == 2 ? qzeros + (size_t)g_begin * (N / 2) : reinterpret_cast<const unsigned char*>(scales + (size_t)g_begin * N);
+  const unsigned int qstep = wave == 2 ? N / 2 : 2 * N;
+
+  // Load j of ring slot `slot`: 0, 1 packed weights, 2 scales and zero points, 3 .. MT + 2 x.  The weights run one
+  // stage ahead of x: slot of stage i holds x of stage i and the weights of stage i + 1.
+  auto issue = [&](unsigned int slot, int j) {
+    const unsigned int st = lds0 + slot;
+    if (j < 2) load_lds_x4(wbase, woff[j], st + (wave + 4 * j) * 1024);
+    else if (j == 2) load_lds_x1(qbase, qoff, st + W_BYTES + wave * 256);
+    else load_lds_x4(xbase, xoff[j - 3], st + W_BYTES + Q_BYTES + (wave + 4 * (j - 3)) * 1024);
+  };
+  // The bases move on behind the loads of a stage.  At the end they stay at the last one: it is fetched again, into
+  // slots that nobody reads, and the loop needs neither branches nor a varying count of loads.
+  auto next_weights = [&](int fetched) {            // stage whose weights were just fetched
+    if (fetched + 1 < steps) {
+      wbase += (size_t)32 * N;
+      if (fetched & 1) qbase += qstep;
+    }
+  };
+  auto next_x = [&](int fetched) { if (fetched + 1 < steps) xbase += SK * 2; };
+
+  // ---- operand roles.  A transposing read takes 8 byte-rows x 16 columns per 16 lanes: lane s16 supplies the 8-byte
+  // piece (row s16 / 2, half s16 % 2) and receives the 8 bytes (16 values of k) of column s16.  Lanes 16-31 take the
+  // chunk 8 further on, so that the 32 lanes of a pass touch 16 different chunk positions.
+  const int s16 = lane & 15, hi16 = (lane >> 4) & 1, h = lane >> 5;
+  int b_off[2], colpos[2];
+#pragma unroll
+  for (int ct = 0; ct < 2; ++ct) {
+    const int chunk = wave * 2 + ct + 8 * hi16;
+    b_off[ct] = (h * 16 + (s16 >> 1)) * 256 + ((chunk ^ (s16 >> 1)) * 16) + (s16 & 1) * 8;      // + q * 2048
+    colpos[ct] = chunk * 16 + s16;
+  }
+  int a_off[4];                                     // x chunk 4 h + e of row lane % 32; + 4096 per row tile
+#pragma unroll
+  for (int e = 0; e < 4; ++e) a_off[e] = W_BYTES + Q_BYTES + (lane & 31) * 128 + (((4 * h + e) ^ ((lane >> 1) & 7)) * 16);
+
+  f16v acc[MT][2];
+#pragma unroll
+  for (int t = 0; t < MT; ++t)
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[t][c][r] = 0.f;
+
+  i32x2 pk[2][2][2];                                // packed weights: [stage parity][q][column tile]
+  _Float16 raw_s[2];
+  unsigned int raw_z[2];
+  h2 s2[2], zz2[2];                                 // scale, 1024 + zero point of this lane's two columns
+  h8 fa[2][MT];                                     // operands of a round, double buffered: x
+  h2 fb[2][2][4];                                   // ... weights, in pairs of k
+  auto read_weights = [&](unsigned int slot, int par, int part) {
+    const unsigned char* st = smem + slot;
+    if (part < 4) pk[par][part >> 1][part & 1] = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_i32x2*)(st + b_off[part & 1] + (part >> 1) * 2048));
+  };
+  auto read_scales = [&](unsigned int slot, int ct) {
+    const unsigned char* st = smem + slot + W_BYTES;
+    raw_s[ct] = *reinterpret_cast<const _Float16*>(st + colpos[ct] * 2);
+    raw_z[ct] = st[512 + (colpos[ct] >> 1)];
+  };
+  auto decode_scales = [&](int ct) {
+    const unsigned int z = (raw_z[ct] >> ((colpos[ct] & 1) * 4)) & 15u;
+    const _Float16 s = (n0 + colpos[ct] < N) ? raw_s[ct] : (_Float16)0.f;
+    s2[ct] = h2{s, s};
+    zz2[ct] = as_h2(z | (z << 16) | mg.bias_lo);
+  };
+  auto read_x = [&](unsigned int slot, int e, int t) {
+    fa[e & 1][t] = *reinterpret_cast<const h8*>(smem + slot + a_off[e] + t * 4096);
+  };
+  // pair j of column tile ct for round e.  Byte j of the word holds k = 2 j (low nibble) and 2 j + 1 (high nibble).
+  auto unpack = [&](int par, int e, int ct, int j) {
+    const unsigned int w = (unsigned int)pk[par][e >> 1][ct][e & 1], u = w >> 4;
+    const unsigned int q = __builtin_amdgcn_perm(u, w, 0x0c040c00u + 0x00010001u * j);
+    fb[e & 1][ct][j] = (as_h2(and_or(q, mg.mask_lo, mg.bias_lo)) - zz2[ct]) * s2[ct];
+  };
+  auto multiply = [&](int slot, int t) {
+#pragma unroll
+    for (int ct = 0; ct < 2; ++ct) {
+      const h2* p = fb[slot][ct];
+      const h8 b = h8{p[0][0], p[0][1], p[1][0], p[1][1], p[2][0], p[2][1], p[3][0], p[3][1]};
+      acc[t][ct] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fa[slot][t], b, acc[t][ct], 0, 0, 0);
+    }
+  };
+
+  // ---- prologue: weights of stage 0 into slot 2, then slots 0 and 1
+#pragma unroll
+  for (int j = 0; j < 3; ++j) issue(2 * STAGE, j);
+  next_weights(0);
+#pragma unroll
+  for (int j = 0; j < L; ++j) issue(0, j);
+  next_weights(1);
+  next_x(0);
+#pragma unroll
+  for (int j = 0; j < L; ++j) issue(STAGE, j);
+  next_weights(2);
+  next_x(1);
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(L) : "memory");       // loads return in order
+  art_lds_barrier();
+#pragma unroll
+  for (int part = 0; part < 4; ++part) read_weights(2 * STAGE, 0, part);
+#pragma unroll
+  for (int ct = 0; ct < 2; ++ct) { read_scales(2 * STAGE, ct); decode_scales(ct); }
+#pragma unroll
+  for (int t = 0; t < MT; ++t) read_x(0, 0, t);
+#pragma unroll
+  for (int ct = 0; ct < 2; ++ct)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) unpack(0, 0, ct, j);
+  art_lds_barrier();                                // slot 2 is free again
+  unsigned int s_cur = 0, s_next = STAGE, s_fill = 2 * STAGE;
+
+  // A round multiplies 16 values of k per lane half and prepares the operands of the round behind it, in four chunks:
+  // MT / 2 MFMAs, MT / 4 reads of x, two unpacked pairs and one load for the stage two ahead.
+  constexpr int CT_ = MT / 4;                       // row tiles per chunk
+  auto round = [&](int i, auto par_tag, auto e_tag) {
+    constexpr int PAR = decltype(par_tag)::value, E = decltype(e_tag)::value;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      __builtin_amdgcn_sched_barrier(0);
+      constexpr int kFirst[4] = {3, 7, 11, 0};      // loads of rounds 0, 1, 2; round 3 starts the next stage's
+      const int j = kFirst[E] + c;
+      if (E == 3 ? c < 3 : j < L) issue(s_fill, j);
+      if (E == 2) read_weights(s_cur, PAR ^ 1, c);  // the weights of stage i + 1 came with x of stage i
+      if (E == 2 && PAR == 1 && c < 2) read_scales(s_cur, c);
+      if (E == 3 && PAR == 1 && c == 0) { decode_scales(0); decode_scales(1); }
+#pragma unroll
+      for (int t = c * CT_; t < (c + 1) * CT_; ++t) E == 3 ? read_x(s_next, 0, t) : read_x(s_cur, (E + 1) & 3, t);
+#pragma unroll
+      for (int p = 2 * c; p < 2 * c + 2; ++p) unpack(E == 3 ? PAR ^ 1 : PAR, (E + 1) & 3, p >> 2, p & 3);
+#pragma unroll
+      for (int t = c * CT_; t < (c + 1) * CT_; ++t) multiply(E & 1, t);
+#pragma unroll
+      for (int m = 0; m < 2 * CT_; ++m) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x002, MT == 8 ? 3 : 5, 0);
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto stage = [&](int i, auto par_tag) {
+    using E0 = std::integral_constant<int, 0>;
+    using E1 = std::integral_constant<int, 1>;
+    using E2 = std::integral_constant<int, 2>;
+    using E3 = std::integral_constant<int, 3>;
+    round(i, par_tag, E0{});
+    round(i, par_tag, E1{});
+    round(i, par_tag, E2{});
+    next_x(i + 2);
+    // The next slot is complete once only the x loads of stage i + 2 are outstanding ... and everybody has read all of
+    // this one, which then takes stage i + 3.  Behind the last stage the reads return old bytes; nothing uses them.
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(L) : "memory");
+    art_lds_barrier();
+    const unsigned int free_slot = s_cur;
+    s_fill = free_slot;
+    round(i, par_tag, E3{});
+    next_weights(i + 4);
+    s_cur = s_next;
+    s_next = 3 * STAGE - s_cur - s_fill;
+  };
+  // the weights of slot 2 (stage 3) open the pattern: from here on every round 3 fetches the weights of the next slot
+#pragma unroll
+  for (int j = 0; j < 3; ++j) issue(s_fill, j);
+  next_weights(3);
+#pragma unroll 1
+  for (int i = 0; i < steps; i += 2) {
+    stage(i, std::integral_constant<int, 0>{});
+    stage(i + 1, std::integral_constant<int, 1>{});
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // nothing of the ring is on its way when its space is reused or given back
+
+  // Accumulator element r of row tile t is row t * 32 + (r / 4) * 8 + 4 h + r % 4.
+  if (splits > 1) {
+#pragma unroll
+    for (int t = 0; t < MT; ++t)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int row = m0 + t * 32 + (r >> 2) * 8 + h * 4 + (r & 3);
+#pragma unroll
+        for (int ct = 0; ct < 2; ++ct)
+          if (row < M && n0 + colpos[ct] < N) partial[((size_t)split * M + row) * N + n0 + colpos[ct]] = acc[t][ct][r];
+      }
+    return;
+  }
+  _Float16* cs = reinterpret_cast<_Float16*>(smem);
+#pragma unroll
+  for (int p = 0; p < MT / 4; ++p) {                // 128 rows at a time through LDS, out as 16-byte stores
+    __syncthreads();
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int ct = 0; ct < 2; ++ct)
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          cs[(t * 32 + (r >> 2) * 8 + h * 4 + (r & 3)) * C_LD + colpos[ct]] = (_Float16)acc[4 * p + t][ct][r];
+    __syncthreads();
+#pragma unroll 4
+    for (int c = tid; c < 128 * (BN / 8); c += kThreads) {
+      const int row = c >> 5, col = (c & 31) * 8, grow = m0 + p * 128 + row;
+      if (grow >= M || n0 + col >= N) continue;
+      h8 o = *reinterpret_cast<const h8*>(cs + row * C_LD + col);
+      if (residual) {                               // y = fp16(fp16(product) + residual)
+        const h4 r0 = *reinterpret_cast<const h4*>(residual + (size_t)grow * N + n0 + col);
+        const h4 r1 = *reinterpret_cast<const h4*>(residual + (size_t)grow * N + n0 + col + 4);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          o[k] = (_Float16)((float)o[k] + (float)r0[k]);
+          o[k + 4] = (_Float16)((float)o[k + 4] + (float)r1[k]);
+        }
+      }
+      // y is 8-byte aligned
+      *reinterpret_cast<h4*>(y + (size_t)grow * N + n0 + col) = h4{o[0], o[1], o[2], o[3]};
+      *reinterpret_cast<h4*>(y + (size_t)grow * N + n0 + col + 4) = h4{o[4], o[5], o[6], o[7]};
+    }
+  }
+}
+
+template <int MT>
+int launch(const _Float16* x, const unsigned char* qweight, const _Float16* scales, const unsigned char* qzeros, _Float16* y,
+           float* partial, int M, int K, int N, int splits, const _Float16* residual, hipStream_t stream) {
+  static bool configured = false;
+  if (!configured) {
+    ART_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_w4a16_wide_kernel<MT>), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                (int)lds_bytes(MT)));
+    configured = true;
+  }
+  const int col_tiles = (N + BN - 1) / BN, m_blocks = (M + 32 * MT - 1) / (32 * MT);
+  gemm_w4a16_wide_kernel<MT><<<dim3((unsigned)((col_tiles * splits + 7) / 8 * 8 * m_blocks)), kThreads, lds_bytes(MT), stream>>>(
+      x, qweight, scales, qzeros, y, partial, M, K, N, splits, col_tiles, m_blocks, kMagic, residual);
+  ART_LAUNCH_CHECK();
+  return 0;
+}
+
+}  // namespace
+
+int art::w4::gemm_wide(const _Float16* x, const unsigned char* qweight, const _Float16* scales, const unsigned char* qzeros, _Float16* y,
+                       float* partial, int M, int K, int N, int splits, int row_tiles, const _Float16* residual, hipStream_t stream) {
+  return row_tiles == 8 ? launch<8>(x, qweight, scales, qzeros, y, partial, M, K, N, splits, residual, stream)
+                        : launch<4>(x, qweight, scales, qzeros, y, partial, M, K, N, splits, residual, stream);
+}

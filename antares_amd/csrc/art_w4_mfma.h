@@ -1,0 +1,46 @@
+// What the int4 GEMM kernels share: operand types, the nibble -> fp16 extraction and the order of k it leaves.
+#pragma once
+#include "art_common.h"
+
+namespace art {
+namespace w4 {
+
+typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+typedef _Float16 h4 __attribute__((ext_vector_type(4)));
+typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+typedef float f16v __attribute__((ext_vector_type(16)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+typedef int i32x2 __attribute__((ext_vector_type(2)));
+typedef __attribute__((address_space(3))) i32x2 lds_i32x2;
+
+struct Magic {
+  unsigned int mask_lo, mask_hi, bias_lo, bias_hi;   // 0x000F000F 0x00F000F0 0x64006400 0x54005400
+};
+
+__device__ __forceinline__ h2 as_h2(unsigned int v) { return __builtin_bit_cast(h2, v); }
+
+// (w & mask) | bias in one v_bitop3_b32 (truth table 0xEA = (a & b) | c).
+__device__ __forceinline__ unsigned int and_or(unsigned int w, unsigned int mask, unsigned int bias) {
+  return __builtin_amdgcn_bitop3_b32(w, mask, bias, 0xEA);
+}
+
+// 8 halves of x in the k order the nibble extraction leaves in a B operand: k0 k4 k1 k5 k2 k6 k3 k7.
+__device__ __forceinline__ h8 permute_k(u32x4 v) {
+  u32x4 o;
+  o[0] = __builtin_amdgcn_perm(v[2], v[0], 0x05040100u);
+  o[1] = __builtin_amdgcn_perm(v[2], v[0], 0x07060302u);
+  o[2] = __builtin_amdgcn_perm(v[3], v[1], 0x05040100u);
+  o[3] = __builtin_amdgcn_perm(v[3], v[1], 0x07060302u);
+  return __builtin_bit_cast(h8, o);
+}
+
+constexpr Magic kMagic{0x000F000Fu, 0x00F000F0u, 0x64006400u, 0x54005400u};
+
+// Large batches (art_gemm_w4_wide.hip): one launch over blocks of 32 row_tiles rows x 256 columns, K cut into `splits`;
+// with splits > 1 the fp32 tiles go to `partial` [splits][M][N].  row_tiles is 4 or 8.
+int gemm_wide(const _Float16* x, const unsigned char* qweight, const _Float16* scales, const unsigned char* qzeros, _Float16* y,
+              float* partial, int M, int K, int N, int splits, int row_tiles, const _Float16* residual, hipStream_t stream);
+
+}  // namespace w4
+}  // namespace art

@@ -525,6 +525,29 @@ def test_w4a16_gemm_with_the_residual_folded_in(autort, M, K, N):
     assert np.allclose(plain.float().cpu().numpy(), prod.astype(np.float32), **FP16_TOL)
 
 
+# one group and many; one row past and one short of a block; the last column tile a chunk of 16; more K-splits than groups
+@pytest.mark.parametrize('M,K,N', [(65, 128, 16), (128, 256, 272), (129, 384, 528), (255, 1024, 240), (257, 640, 256), (300, 2048, 1040)])
+def test_w4a16_gemm_over_blocks_of_128_and_256_rows(autort, M, K, N):
+    from ctypes import c_void_p
+    from antares_amd.runtime import capi
+    from oracle import hot_ops
+    dev = autort.device()
+    p = workloads.w4_problem(K + N + M, M, K, N)
+    res = torch.randn(M, N, generator=torch.Generator().manual_seed(M)).half()
+    prod = hot_ops.gemm_w4a16(p['x'].numpy(), p['qweight'].numpy(), p['scales'].numpy(), p['qzeros'].numpy()).astype(np.float32)
+    d = [p[k].to(dev) for k in ('x', 'qweight', 'scales', 'qzeros')] + [torch.empty(M, N, dtype=torch.float16, device=dev), res.to(dev)]
+    ptr = [c_void_p(t.data_ptr()) for t in d]
+    for rows in (128, 256):
+        for splits in (1, 2, 3, 16):
+            note(f'w4a16 gemm M={M} K={K} N={N} blocks of {rows} rows, {splits} splits')
+            code = rows // 32 * 256 + splits
+            for residual, want in ((c_void_p(0), prod), (ptr[5], (prod + res.numpy().astype(np.float32)))):
+                d[4].fill_(float('nan'))
+                capi.check(capi.lib().art_gemm_w4a16_residual(*ptr[:5], residual, M, K, N, code, c_void_p(torch.cuda.current_stream().cuda_stream)))
+                torch.cuda.synchronize()
+                assert np.allclose(d[4].float().cpu().numpy(), want, **FP16_TOL)
+
+
 ROW_VECTOR_CASES = [
     # program, inputs, shapes of the inputs, does the row-vector variant apply to these extents
     ('output0[N, C] = input0[N, C] + input1[C]', ['input0=float32[N:300, C:1024]', 'input1=float32[C:1024]'], [(300, 1024), (1024,)], True),
