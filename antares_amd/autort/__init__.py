@@ -30,6 +30,8 @@ class _Ops:
 
     def _register(self, name: str, op):
         self._table[name] = op
+        if not hasattr(type(self), name):          # an attribute of its own: found without entering __getattr__
+            object.__setattr__(self, name, op)
 
     def __getattr__(self, name: str):
         table = object.__getattribute__(self, '_table')
@@ -40,12 +42,12 @@ class _Ops:
         if record is not None:
             op = ExportedOp(record['ir'], list(record['inputs']), config=record['config'], name=record['name'],
                             extra_outputs=record['extra_outputs'], tuned=record.get('tuned') or None)
-            table[name] = op
+            self._register(name, op)
             return op
         op = builtin.lookup(name)
         if op is None:
             raise AttributeError(f'autort.ops has no operator `{name}`; create it with autort.export(..., name="{name}")')
-        table[name] = op
+        self._register(name, op)
         return op
 
     def __dir__(self):

@@ -1,13 +1,13 @@
 """Operators that ship with the package: the fused partition and the Llama
 decode operators.  Each is a thin Python wrapper that checks shapes on the
-host and calls one typed entry point of libantares_amd.so."""
+host and calls one typed entry point of libantares_amd.so; a call whose
+signature has been seen before is replayed in native code (runtime/calls.py)."""
 from __future__ import annotations
-
-from ctypes import c_void_p
 
 import torch
 
-from ..runtime import capi
+from ..runtime import calls, capi
+from ..runtime.calls import STREAM, Number
 from .builtin import builtin
 from .op import current_stream_handle
 
@@ -21,7 +21,15 @@ def _require_cuda(*tensors):
     capi.init(tensors[0].device.index or 0)
 
 
-class PartitionEvenFirst:
+def _run(op, pending, result, fn, *args):
+    """Calls a library entry point on the current stream and leaves the recipe of the call with the operator."""
+    call = calls.Call(current_stream_handle())
+    call.library(fn, *args, STREAM)
+    call.keep(op, pending, [result], device_stream=False)
+    return result
+
+
+class PartitionEvenFirst(calls.Operator):
     """``autort.ops.partition_even_first_i32(x[, out])``: all even values of an
     int32 vector in input order, then all odd values in input order — the result
     of the classify / cumsum / bucket pipeline of samples/01_sort_even_first.py:9-27
@@ -32,6 +40,7 @@ class PartitionEvenFirst:
     def __init__(self):
         self.tuned = {}                                 # str(n) -> {'value': cap on blocks, 'us': ...}
         self._loaded = False
+        self._bind(('x', 'out', 'extra'), ())
 
     def _saved(self):
         """Winners of earlier tuning runs, kept in the operator store as `partition_even_first_i32.tuned.json`."""
@@ -61,8 +70,7 @@ class PartitionEvenFirst:
             pass
 
     def _launch(self, x, out, cap):
-        capi.check(capi.lib().art_partition_even_first_i32_tuned(c_void_p(x.data_ptr()), c_void_p(out.data_ptr()), x.numel(),
-                                                                int(cap), c_void_p(current_stream_handle())))
+        capi.check(capi.lib().art_partition_even_first_i32_tuned(x.data_ptr(), out.data_ptr(), x.numel(), int(cap), current_stream_handle()))
 
     def tune(self, x: torch.Tensor, trials: int = 5):
         """Times up to `trials` caps on the number of blocks for vectors of x's length (on rotating copies of x, into
@@ -75,7 +83,7 @@ class PartitionEvenFirst:
         self.config = {}
         return tune_hand_kernel(self, str(n), list(self.BLOCK_CAPS), lambda v, t: self._launch(t[0], t[1], v), trials, clones)
 
-    def __call__(self, x: torch.Tensor, out: torch.Tensor = None, extra=None):
+    def _call(self, pending, x: torch.Tensor, out: torch.Tensor = None, extra=None):
         if x.dtype != torch.int32 or x.dim() != 1:
             raise TypeError('partition_even_first_i32 expects a 1-D int32 tensor')
         if out is None:
@@ -84,8 +92,7 @@ class PartitionEvenFirst:
             raise TypeError('partition_even_first_i32: out must be int32 with as many elements as the input')
         _require_cuda(x, out)
         saved = self._saved().get(str(x.numel()))
-        self._launch(x, out, saved['value'] if saved else 0)
-        return out
+        return _run(self, pending, out, capi.lib().art_partition_even_first_i32_tuned, x, out, x.numel(), saved['value'] if saved else 0)
 
 
 @builtin('partition_even_first_i32')
@@ -106,20 +113,21 @@ def _dt(t: torch.Tensor, what: str) -> int:
     return _DT[t.dtype]
 
 
-def _pos_args(extra, what: str):
+def _pos_args(extra, what: str, params: int):
     """``extra=[pos]``: a Python int, or a 1-element int32 GPU tensor (read on the
-    device, so a recorded HIP graph can be replayed for every position)."""
+    device, so a recorded HIP graph can be replayed for every position).  ``params``:
+    parameters of the operator, behind which the numbers of ``extra`` are counted."""
     if not extra:
         raise TypeError(f'{what} needs extra=[pos]')
     pos = extra[0]
     if isinstance(pos, torch.Tensor):
         if pos.dtype != torch.int32 or pos.numel() != 1 or not pos.is_cuda:
             raise TypeError(f'{what}: a tensor position must be a 1-element int32 GPU tensor')
-        return c_void_p(pos.data_ptr()), 0
-    return c_void_p(0), int(pos)
+        return pos, 0
+    return None, Number(int(pos), params, 'I')
 
 
-class RmsNorm:
+class RmsNorm(calls.Operator):
     """``rmsnorm_f32(x[N], vsum[1], w[N], extra=[1/N]) -> out[N]``:
     ``out = x * rsqrt(vsum * extra[0] + eps) * w`` with eps = 1e-5 (``extra[1]``
     overrides it).  ``vsum`` is the caller's fp32 sum of squares; passing ``None``
@@ -128,42 +136,38 @@ class RmsNorm:
     def __init__(self, out_dtype: torch.dtype):
         self.out_dtype = out_dtype
         self.name = 'rmsnorm_f32' if out_dtype == torch.float32 else 'rmsnorm_f16'
+        self._bind(('x', 'vsum', 'w', 'out', 'extra'), ('extra',))
 
-    def __call__(self, x, vsum, w, out=None, extra=None):
+    def _call(self, pending, x, vsum, w, out=None, extra=None):
         n = w.numel()
         rows = x.numel() // n
         if rows * n != x.numel() or n == 0:
             raise ValueError(f'{self.name}: x has {x.numel()} elements, weight {n}')
-        inv_n = float(extra[0]) if extra else 1.0 / n
-        eps = float(extra[1]) if extra and len(extra) > 1 else RMS_EPS
+        inv_n = Number(float(extra[0]), 5, 'F') if extra else 1.0 / n
+        eps = Number(float(extra[1]), 6, 'F') if extra and len(extra) > 1 else RMS_EPS
         if out is None:
             out = torch.empty(x.shape, dtype=self.out_dtype, device=x.device)
         if out.numel() != x.numel():
             raise ValueError(f'{self.name}: out has the wrong size')
         tensors = [x, w, out]
-        vptr = c_void_p(0)
         if vsum is not None:
-            vsum = vsum.view(-1)
             if vsum.dtype != torch.float32 or vsum.numel() != rows:
                 raise TypeError(f'{self.name}: vsum must be float32 with one value per row')
             tensors.append(vsum)
-            vptr = c_void_p(vsum.data_ptr())
         _require_cuda(*tensors)
-        capi.check(capi.lib().art_rmsnorm(c_void_p(x.data_ptr()), vptr, c_void_p(w.data_ptr()), c_void_p(out.data_ptr()),
-                                         rows, n, inv_n, eps, _dt(x, 'x'), _dt(w, 'weight'), _dt(out, 'out'),
-                                         c_void_p(current_stream_handle())))
-        return out
+        return _run(self, pending, out, capi.lib().art_rmsnorm, x, vsum, w, out, rows, n, inv_n, eps, _dt(x, 'x'), _dt(w, 'weight'), _dt(out, 'out'))
 
 
-class Rotary:
+class Rotary(calls.Operator):
     """``rotary_f32(x[H,2,D/2], inv_freq[D], out[H,D], extra=[pos])`` (rotate-half
     form) and ``rotate_f32(coef[1,dim/2], data[dim], out[dim], extra=[pos])``
     (interleaved pairs, samples/03_llama_tiny.py:68-70)."""
 
     def __init__(self, name: str, interleaved: bool):
         self.name, self.interleaved = name, interleaved
+        self._bind(('a', 'b', 'out', 'extra'), ('extra',))
 
-    def __call__(self, a, b, out=None, extra=None):
+    def _call(self, pending, a, b, out=None, extra=None):
         x, freq = (b, a) if self.interleaved else (a, b)
         if out is None:
             out = torch.empty_like(x)
@@ -178,22 +182,20 @@ class Rotary:
             if freq.numel() < head_dim // 2:
                 raise ValueError(f'{self.name}: inv_freq is too short')
         _require_cuda(x, freq, out)
-        pos_dev, pos = _pos_args(extra, self.name)
+        pos_dev, pos = _pos_args(extra, self.name, 4)
         stride, out_rows = 0, 0
         if out.numel() != x.numel():
             # a whole [positions, heads*head_dim] cache: the row is chosen by the device-side position
-            if not pos_dev.value or out.numel() % x.numel() != 0:
+            if pos_dev is None or out.numel() % x.numel() != 0:
                 raise ValueError(f'{self.name}: out must match x in size (or be a cache with extra=[position tensor])')
             stride, out_rows = x.numel(), out.numel() // x.numel()
         if out.dtype != x.dtype:
             raise ValueError(f'{self.name}: out must have the dtype of x')
-        capi.check(capi.lib().art_rotary(c_void_p(x.data_ptr()), c_void_p(freq.data_ptr()), c_void_p(out.data_ptr()), heads,
-                                        head_dim, int(self.interleaved), pos_dev, pos, stride, out_rows, _dt(x, 'x'), _dt(freq, 'inv_freq'),
-                                        _dt(out, 'out'), c_void_p(current_stream_handle())))
-        return out
+        return _run(self, pending, out, capi.lib().art_rotary, x, freq, out, heads, head_dim, int(self.interleaved), pos_dev, pos, stride, out_rows,
+                    _dt(x, 'x'), _dt(freq, 'inv_freq'), _dt(out, 'out'))
 
 
-class DecodeAttention:
+class DecodeAttention(calls.Operator):
     """``attention_f32(q[H,D], k[S,H,D], v[S,H,D], att_f[1]) -> out[H,D]``: scores
     ``att_f * q.k``, softmax over S, weighted sum of v (the torch spelling is at
     samples/03_llama_tiny.py:94-99).  ``extra=[pos]`` with a 1-element int32 GPU
@@ -202,8 +204,9 @@ class DecodeAttention:
 
     def __init__(self, name: str):
         self.name = name
+        self._bind(('q', 'k', 'v', 'att_f', 'out', 'extra'), ())
 
-    def __call__(self, q, k, v, att_f, out=None, extra=None):
+    def _call(self, pending, q, k, v, att_f, out=None, extra=None):
         if q.dim() != 2 or k.dim() != 3 or k.shape != v.shape or k.shape[1:] != q.shape:
             raise ValueError(f'{self.name}: expected q[H,D], k[S,H,D], v[S,H,D]; got {list(q.shape)}, {list(k.shape)}, {list(v.shape)}')
         if att_f.dtype != torch.float32 or att_f.numel() != 1:
@@ -213,23 +216,23 @@ class DecodeAttention:
         if out is None:
             out = torch.empty_like(q)
         _require_cuda(q, k, v, att_f, out)
-        pos_dev = c_void_p(0)
+        pos_dev = None
         if extra and isinstance(extra[0], torch.Tensor):
-            pos_dev, _ = _pos_args(extra, self.name)
-        capi.check(capi.lib().art_decode_attention(c_void_p(q.data_ptr()), c_void_p(k.data_ptr()), c_void_p(v.data_ptr()),
-                                                  c_void_p(att_f.data_ptr()), c_void_p(out.data_ptr()), k.shape[0], q.shape[0],
-                                                  q.shape[1], pos_dev, _dt(q, 'q'), _dt(k, 'k'), _dt(out, 'out'),
-                                                  c_void_p(current_stream_handle())))
-        return out
+            pos_dev, _ = _pos_args(extra, self.name, 6)
+        return _run(self, pending, out, capi.lib().art_decode_attention, q, k, v, att_f, out, k.shape[0], q.shape[0], q.shape[1], pos_dev,
+                    _dt(q, 'q'), _dt(k, 'k'), _dt(out, 'out'))
 
 
-class CausalAttention:
+class CausalAttention(calls.Operator):
     """``attention_causal_f16(q[T,H,D], k[S,H,D], v[S,H,D], att_f[1]) -> out[T,H,D]`` with S >= T: position t attends to
     rows 0..t of k and v (views of the key / value cache), i.e. ``attention_f16`` for the T positions of a prompt in
     one launch on the matrix cores."""
     name = 'attention_causal_f16'
 
-    def __call__(self, q, k, v, att_f, out=None, extra=None):
+    def __init__(self):
+        self._bind(('q', 'k', 'v', 'att_f', 'out', 'extra'), ())
+
+    def _call(self, pending, q, k, v, att_f, out=None, extra=None):
         if q.dim() != 3 or k.dim() != 3 or k.shape != v.shape or k.shape[1:] != q.shape[1:] or k.shape[0] < q.shape[0]:
             raise ValueError(f'{self.name}: expected q[T,H,D], k[S,H,D], v[S,H,D] with S >= T; got {list(q.shape)}, {list(k.shape)}, {list(v.shape)}')
         for t in (q, k, v):
@@ -243,10 +246,7 @@ class CausalAttention:
             raise TypeError(f'{self.name}: out must be float16 of the shape of q')
         _require_cuda(q, k, v, att_f, out)
         T, H, D = q.shape
-        capi.check(capi.lib().art_prefill_attention(c_void_p(q.data_ptr()), c_void_p(k.data_ptr()), c_void_p(v.data_ptr()),
-                                                   c_void_p(att_f.data_ptr()), c_void_p(out.data_ptr()), T, H, D, H * D,
-                                                   c_void_p(current_stream_handle())))
-        return out
+        return _run(self, pending, out, capi.lib().art_prefill_attention, q, k, v, att_f, out, T, H, D, H * D)
 
 
 builtin('attention_causal_f16')(lambda: CausalAttention())
@@ -271,17 +271,17 @@ def _sumsq_buffers(who, *buffers):
     return given
 
 
-def _ptr_or_null(t):
-    return c_void_p(t.data_ptr() if t is not None else 0)
-
-
-class GemvW4Fused:
+class GemvW4Fused(calls.Operator):
     """``gemv_w4a16_fused(x[K], qweight, scales, qzeros, out[N], norm_weight=None, residual=None, eps=1e-5)``:
     the packed int4 GEMV with an RMSNorm of its input and/or a residual add of its output folded in
     (the operators around every projection of the decode step, samples/05_llama2_7b_int4.py:150-173)."""
     name = 'gemv_w4a16_fused'
 
-    def __call__(self, x, qweight, scales, qzeros, out=None, norm_weight=None, residual=None, eps=RMS_EPS, swiglu=False,
+    def __init__(self):
+        self._bind(('x', 'qweight', 'scales', 'qzeros', 'out', 'norm_weight', 'residual', 'eps', 'swiglu', 'extra', 'sumsq_in', 'sumsq_out',
+                    'sumsq_clear'), ())
+
+    def _call(self, pending, x, qweight, scales, qzeros, out=None, norm_weight=None, residual=None, eps=RMS_EPS, swiglu=False,
                  extra=None, sumsq_in=None, sumsq_out=None, sumsq_clear=None):
         """``swiglu=True``: ``x`` holds gate | up (2*K values) and the product is taken with silu(gate) * up.
         ``sumsq_*``: int64[256] buffers that hand sum(y^2) from the projection that writes a residual stream
@@ -304,12 +304,8 @@ class GemvW4Fused:
                 tensors.append(t)
         tensors += _sumsq_buffers('gemv_w4a16_fused', sumsq_in, sumsq_out, sumsq_clear)
         _require_cuda(*tensors)
-        capi.check(capi.lib().art_gemv_w4a16_fused_sumsq(
-            c_void_p(x.data_ptr()), c_void_p(qweight.data_ptr()), c_void_p(scales.data_ptr()), c_void_p(qzeros.data_ptr()),
-            c_void_p(out.data_ptr()), K, N, c_void_p(norm_weight.data_ptr() if norm_weight is not None else 0), float(eps),
-            c_void_p(residual.data_ptr() if residual is not None else 0), int(bool(swiglu)), _ptr_or_null(sumsq_in),
-            _ptr_or_null(sumsq_out), _ptr_or_null(sumsq_clear), c_void_p(current_stream_handle())))
-        return out
+        return _run(self, pending, out, capi.lib().art_gemv_w4a16_fused_sumsq, x, qweight, scales, qzeros, out, K, N, norm_weight, float(eps),
+                    residual, int(bool(swiglu)), sumsq_in, sumsq_out, sumsq_clear)
 
 
 class W4Prepack:
@@ -336,13 +332,13 @@ class W4Prepack:
             if not t.is_contiguous():
                 raise ValueError('w4_prepack: operands must be contiguous')
         _require_cuda(qweight, scales, qzeros, out)
-        capi.check(capi.lib().art_w4_prepack(c_void_p(qweight.data_ptr()), c_void_p(scales.data_ptr()), c_void_p(qzeros.data_ptr()),
-                                            c_void_p(out.data_ptr()), K, N, c_void_p(current_stream_handle())))
+        capi.check(capi.lib().art_w4_prepack(qweight.data_ptr(), scales.data_ptr(), qzeros.data_ptr(),
+                                            out.data_ptr(), K, N, current_stream_handle()))
         out.w4_shape = (K, N)
         return out
 
 
-class GemvW4Packed:
+class GemvW4Packed(calls.Operator):
     """``gemv_w4p(x[K], packed, out=None, norm_weight=None, residual=None, eps=1e-5, swiglu_out=False, shape=None)``:
     the int4 GEMV over weights repacked by ``w4_prepack`` - one block per 16 columns over all of K, no K-splits.
     ``norm_weight``: RMSNorm of x folded in; ``residual``: added to the rounded product (``out`` may be the residual);
@@ -350,7 +346,10 @@ class GemvW4Packed:
     ``out[N/2]`` receives fp16(silu(gate) * up).  ``shape`` = (K, N) when ``packed`` does not carry ``w4_shape``."""
     name = 'gemv_w4p'
 
-    def __call__(self, x, packed, out=None, norm_weight=None, residual=None, eps=RMS_EPS, swiglu_out=False, shape=None, extra=None):
+    def __init__(self):
+        self._bind(('x', 'packed', 'out', 'norm_weight', 'residual', 'eps', 'swiglu_out', 'shape', 'extra'), ())
+
+    def _call(self, pending, x, packed, out=None, norm_weight=None, residual=None, eps=RMS_EPS, swiglu_out=False, shape=None, extra=None):
         K, N = shape if shape is not None else getattr(packed, 'w4_shape', (None, None))
         if K is None:
             raise ValueError('gemv_w4p: pass shape=(K, N) or a tensor returned by w4_prepack')
@@ -370,10 +369,9 @@ class GemvW4Packed:
                     raise TypeError(f'gemv_w4p: {what} must be float16 of {n} values')
                 tensors.append(t)
         _require_cuda(*tensors)
-        capi.check(capi.lib().art_gemv_w4p(c_void_p(x.data_ptr()), c_void_p(packed.data_ptr()), c_void_p(out.data_ptr()), K, N,
-                                          _ptr_or_null(norm_weight), float(eps), _ptr_or_null(residual), int(bool(swiglu_out)),
-                                          c_void_p(current_stream_handle())))
-        return out
+        # without `shape` K and N hang on the tensor, where a recipe does not look
+        return _run(self, pending if shape is not None else None, out, capi.lib().art_gemv_w4p, x, packed, out, K, N, norm_weight, float(eps), residual,
+                    int(bool(swiglu_out)))
 
 
 def interleave_gate_up(gate: dict, up: dict) -> dict:
@@ -392,12 +390,15 @@ builtin('w4_prepack')(lambda: W4Prepack())
 builtin('gemv_w4p')(lambda: GemvW4Packed())
 
 
-class AttentionRope:
+class AttentionRope(calls.Operator):
     """``attention_rope_f16(qkv[3*H*D], inv_freq[D], key_cache[S,H*D], val_cache[S,H*D], att_f[1], out[H,D], extra=[pos_tensor])``:
     rotary embedding of q and k, both cache writes and the attention over rows 0..pos, one launch per layer."""
     name = 'attention_rope_f16'
 
-    def __call__(self, qkv, inv_freq, key_cache, val_cache, att_f, out, extra=None):
+    def __init__(self):
+        self._bind(('qkv', 'inv_freq', 'key_cache', 'val_cache', 'att_f', 'out', 'extra'), ())
+
+    def _call(self, pending, qkv, inv_freq, key_cache, val_cache, att_f, out, extra=None):
         heads, head_dim = out.shape
         if qkv.numel() != 3 * heads * head_dim or key_cache.shape[-1] != heads * head_dim or val_cache.shape != key_cache.shape:
             raise ValueError('attention_rope_f16: shapes do not fit together')
@@ -407,23 +408,23 @@ class AttentionRope:
         if att_f.dtype != torch.float32 or att_f.numel() != 1:
             raise TypeError('attention_rope_f16: att_f must be a 1-element float32 tensor')
         _require_cuda(qkv, inv_freq, key_cache, val_cache, att_f, out)
-        pos_dev, _ = _pos_args(extra, self.name)
-        if not pos_dev.value:
+        pos_dev, _ = _pos_args(extra, self.name, 0)
+        if pos_dev is None:
             raise TypeError('attention_rope_f16: extra=[pos] must be a 1-element int32 GPU tensor')
-        capi.check(capi.lib().art_decode_attention_rope(c_void_p(qkv.data_ptr()), c_void_p(inv_freq.data_ptr()),
-                                                       c_void_p(key_cache.data_ptr()), c_void_p(val_cache.data_ptr()),
-                                                       c_void_p(att_f.data_ptr()), c_void_p(out.data_ptr()), heads, head_dim, pos_dev,
-                                                       key_cache.numel() // (heads * head_dim), c_void_p(current_stream_handle())))
-        return out
+        return _run(self, pending, out, capi.lib().art_decode_attention_rope, qkv, inv_freq, key_cache, val_cache, att_f, out, heads, head_dim, pos_dev,
+                    key_cache.numel() // (heads * head_dim))
 
 
-class AttentionRopeSplit:
+class AttentionRopeSplit(calls.Operator):
     """``attention_rope_split_f16(qkv[3*H*D], inv_freq[D], key_cache, val_cache, att_f[1], partial[H, P, 132], extra=[pos_tensor])``:
     ``attention_rope_f16`` spread over P blocks per head.  ``partial`` (float32) receives, per head and part, 128
     unnormalised sums, the running maximum and the running sum; ``gemv_w4a16_attn`` merges them while it loads x."""
     name = 'attention_rope_split_f16'
 
-    def __call__(self, qkv, inv_freq, key_cache, val_cache, att_f, partial, extra=None):
+    def __init__(self):
+        self._bind(('qkv', 'inv_freq', 'key_cache', 'val_cache', 'att_f', 'partial', 'extra'), ())
+
+    def _call(self, pending, qkv, inv_freq, key_cache, val_cache, att_f, partial, extra=None):
         if partial.dim() != 3 or partial.shape[2] != 132 or partial.dtype != torch.float32:
             raise TypeError('attention_rope_split_f16: partial must be float32 [heads, parts, 132]')
         heads, parts = partial.shape[0], partial.shape[1]
@@ -436,23 +437,22 @@ class AttentionRopeSplit:
         if att_f.dtype != torch.float32 or att_f.numel() != 1:
             raise TypeError('attention_rope_split_f16: att_f must be a 1-element float32 tensor')
         _require_cuda(qkv, inv_freq, key_cache, val_cache, att_f, partial)
-        pos_dev, _ = _pos_args(extra, self.name)
-        if not pos_dev.value:
+        pos_dev, _ = _pos_args(extra, self.name, 0)
+        if pos_dev is None:
             raise TypeError('attention_rope_split_f16: extra=[pos] must be a 1-element int32 GPU tensor')
-        capi.check(capi.lib().art_decode_attention_rope_split(
-            c_void_p(qkv.data_ptr()), c_void_p(inv_freq.data_ptr()), c_void_p(key_cache.data_ptr()), c_void_p(val_cache.data_ptr()),
-            c_void_p(att_f.data_ptr()), c_void_p(partial.data_ptr()), heads, head_dim, pos_dev,
-            key_cache.numel() // (heads * head_dim), parts,
-            c_void_p(current_stream_handle())))
-        return partial
+        return _run(self, pending, partial, capi.lib().art_decode_attention_rope_split, qkv, inv_freq, key_cache, val_cache, att_f, partial, heads,
+                    head_dim, pos_dev, key_cache.numel() // (heads * head_dim), parts)
 
 
-class GemmW4Residual:
+class GemmW4Residual(calls.Operator):
     """``gemm_w4a16_residual(x[M,K], qweight, scales, qzeros, out[M,N], residual=None)``: the packed int4 product for a
     batch of rows on the matrix cores with the residual add folded in (``out`` may be the residual itself)."""
     name = 'gemm_w4a16_residual'
 
-    def __call__(self, x, qweight, scales, qzeros, out, residual=None):
+    def __init__(self):
+        self._bind(('x', 'qweight', 'scales', 'qzeros', 'out', 'residual'), ())
+
+    def _call(self, pending, x, qweight, scales, qzeros, out, residual=None):
         M, K = x.shape
         N = qweight.shape[1]
         if qweight.shape[0] * 2 != K or scales.shape != (K // 128, N) or qzeros.shape != (K // 128, N // 2) or out.shape != (M, N):
@@ -461,22 +461,21 @@ class GemmW4Residual:
                 (residual is not None and (residual.dtype != torch.float16 or residual.shape != out.shape)):
             raise TypeError('gemm_w4a16_residual: x, scales, out and residual must be float16 (residual of the shape of out)')
         _require_cuda(*([x, qweight, scales, qzeros, out] + ([residual] if residual is not None else [])))
-        capi.check(capi.lib().art_gemm_w4a16_residual(
-            c_void_p(x.data_ptr()), c_void_p(qweight.data_ptr()), c_void_p(scales.data_ptr()), c_void_p(qzeros.data_ptr()),
-            c_void_p(out.data_ptr()), c_void_p(residual.data_ptr() if residual is not None else 0), M, K, N, 0,
-            c_void_p(current_stream_handle())))
-        return out
+        return _run(self, pending, out, capi.lib().art_gemm_w4a16_residual, x, qweight, scales, qzeros, out, residual, M, K, N, 0)
 
 
 builtin('gemm_w4a16_residual')(lambda: GemmW4Residual())
 
 
-class GemvW4Attn:
+class GemvW4Attn(calls.Operator):
     """``gemv_w4a16_attn(partial[H, P, 132], qweight, scales, qzeros, out[N], residual=None)``: the int4 projection of a
     split attention's output (merged on the fly) with the residual add folded in."""
     name = 'gemv_w4a16_attn'
 
-    def __call__(self, partial, qweight, scales, qzeros, out, residual=None, sumsq_out=None, sumsq_clear=None):
+    def __init__(self):
+        self._bind(('partial', 'qweight', 'scales', 'qzeros', 'out', 'residual', 'sumsq_out', 'sumsq_clear'), ())
+
+    def _call(self, pending, partial, qweight, scales, qzeros, out, residual=None, sumsq_out=None, sumsq_clear=None):
         K, N = qweight.shape[0] * 2, qweight.shape[1]
         if partial.dim() != 3 or partial.shape[2] != 132 or partial.dtype != torch.float32 or partial.shape[0] * 128 != K:
             raise TypeError('gemv_w4a16_attn: partial must be float32 [K/128, parts, 132]')
@@ -486,43 +485,41 @@ class GemvW4Attn:
             raise TypeError('gemv_w4a16_attn: scales, out and residual must be float16')
         _require_cuda(*([partial, qweight, scales, qzeros, out] + ([residual] if residual is not None else []) +
                         _sumsq_buffers('gemv_w4a16_attn', sumsq_out, sumsq_clear)))
-        capi.check(capi.lib().art_gemv_w4a16_attn_sumsq(
-            c_void_p(partial.data_ptr()), partial.shape[1], c_void_p(qweight.data_ptr()), c_void_p(scales.data_ptr()),
-            c_void_p(qzeros.data_ptr()), c_void_p(out.data_ptr()), K, N,
-            c_void_p(residual.data_ptr() if residual is not None else 0), _ptr_or_null(sumsq_out), _ptr_or_null(sumsq_clear),
-            c_void_p(current_stream_handle())))
-        return out
+        return _run(self, pending, out, capi.lib().art_gemv_w4a16_attn_sumsq, partial, partial.shape[1], qweight, scales, qzeros, out, K, N, residual,
+                    sumsq_out, sumsq_clear)
 
 
-class RopeQkvStore:
+class RopeQkvStore(calls.Operator):
     """``rope_qkv_store_f16(qkv[3*H*D], inv_freq[D], q_out[H,D], key_cache[S,H*D], val_cache[S,H*D], extra=[pos_tensor])``:
     rotary embedding of q and k (k straight into its cache row) and the copy of v into its cache row, one launch."""
 
     def __init__(self, name):
         self.name = name
+        self._bind(('qkv', 'inv_freq', 'q_out', 'key_cache', 'val_cache', 'extra'), ())
 
-    def __call__(self, qkv, inv_freq, q_out, key_cache, val_cache, extra=None):
+    def _call(self, pending, qkv, inv_freq, q_out, key_cache, val_cache, extra=None):
         heads, head_dim = q_out.shape
         if qkv.numel() != 3 * heads * head_dim or key_cache.shape[-1] != heads * head_dim or val_cache.shape != key_cache.shape:
             raise ValueError(f'{self.name}: shapes do not fit together')
         if not (qkv.dtype == q_out.dtype == key_cache.dtype == val_cache.dtype):
             raise TypeError(f'{self.name}: qkv, q_out and the caches must share one dtype')
         _require_cuda(qkv, inv_freq, q_out, key_cache, val_cache)
-        pos_dev, _ = _pos_args(extra, self.name)
-        if not pos_dev.value:
+        pos_dev, _ = _pos_args(extra, self.name, 0)
+        if pos_dev is None:
             raise TypeError(f'{self.name}: extra=[pos] must be a 1-element int32 GPU tensor')
-        capi.check(capi.lib().art_rope_qkv_store(c_void_p(qkv.data_ptr()), c_void_p(inv_freq.data_ptr()), c_void_p(q_out.data_ptr()),
-                                                c_void_p(key_cache.data_ptr()), c_void_p(val_cache.data_ptr()), heads, head_dim,
-                                                pos_dev, key_cache.numel() // (heads * head_dim), _dt(qkv, 'qkv'), _dt(inv_freq, 'inv_freq'), c_void_p(current_stream_handle())))
-        return q_out
+        return _run(self, pending, q_out, capi.lib().art_rope_qkv_store, qkv, inv_freq, q_out, key_cache, val_cache, heads, head_dim, pos_dev,
+                    key_cache.numel() // (heads * head_dim), _dt(qkv, 'qkv'), _dt(inv_freq, 'inv_freq'))
 
 
-class RopeQkvStoreRows:
+class RopeQkvStoreRows(calls.Operator):
     """``rope_qkv_store_rows_f16(qkv[T, 3*H*D], inv_freq[D], q_out[T,H,D], key_cache[S,H*D], val_cache[S,H*D], extra=[first_pos])``:
     ``rope_qkv_store_f16`` for the T tokens of a prompt, token t at position first_pos + t (a host integer, default 0)."""
     name = 'rope_qkv_store_rows_f16'
 
-    def __call__(self, qkv, inv_freq, q_out, key_cache, val_cache, extra=None):
+    def __init__(self):
+        self._bind(('qkv', 'inv_freq', 'q_out', 'key_cache', 'val_cache', 'extra'), ())
+
+    def _call(self, pending, qkv, inv_freq, q_out, key_cache, val_cache, extra=None):
         T, heads, head_dim = q_out.shape
         if qkv.shape != (T, 3 * heads * head_dim) or key_cache.shape[-1] != heads * head_dim or val_cache.shape != key_cache.shape:
             raise ValueError(f'{self.name}: shapes do not fit together')
@@ -531,22 +528,23 @@ class RopeQkvStoreRows:
                 raise TypeError(f'{self.name}: tensors must be float16')
         first = int(extra[0]) if extra else 0
         _require_cuda(qkv, inv_freq, q_out, key_cache, val_cache)
-        capi.check(capi.lib().art_rope_qkv_store_rows(c_void_p(qkv.data_ptr()), c_void_p(inv_freq.data_ptr()), c_void_p(q_out.data_ptr()),
-                                                     c_void_p(key_cache.data_ptr()), c_void_p(val_cache.data_ptr()), T, heads, head_dim,
-                                                     first, key_cache.numel() // (heads * head_dim), c_void_p(current_stream_handle())))
-        return q_out
+        return _run(self, pending, q_out, capi.lib().art_rope_qkv_store_rows, qkv, inv_freq, q_out, key_cache, val_cache, T, heads, head_dim, first,
+                    key_cache.numel() // (heads * head_dim))
 
 
 builtin('rope_qkv_store_rows_f16')(lambda: RopeQkvStoreRows())
 
 
-class GreedyNext:
+class GreedyNext(calls.Operator):
     """``greedy_next_f16(logits[V], prompt[L] or None, token[1], pos[1], embed[V, D], x[D])``: the bookkeeping
     between two decode steps in one launch - pos += 1; token = prompt[pos] while the prompt lasts, else
     argmax(logits); x = embed[token].  token, pos and prompt are int32 GPU tensors."""
     name = 'greedy_next_f16'
 
-    def __call__(self, logits, prompt, token, pos, embed, x):
+    def __init__(self):
+        self._bind(('logits', 'prompt', 'token', 'pos', 'embed', 'x'), ())
+
+    def _call(self, pending, logits, prompt, token, pos, embed, x):
         vocab, dim = embed.shape
         if logits.numel() != vocab or x.numel() != dim or token.numel() != 1 or pos.numel() != 1:
             raise ValueError('greedy_next_f16: shapes do not fit together')
@@ -557,10 +555,8 @@ class GreedyNext:
             raise TypeError('greedy_next_f16: token, pos and prompt must be int32')
         _require_cuda(logits, embed, x, *ints)
         has_prompt = len(ints) == 3
-        capi.check(capi.lib().art_greedy_next(c_void_p(logits.data_ptr()), vocab, c_void_p(prompt.data_ptr() if has_prompt else 0),
-                                             prompt.numel() if has_prompt else 0, c_void_p(token.data_ptr()), c_void_p(pos.data_ptr()),
-                                             c_void_p(embed.data_ptr()), dim, c_void_p(x.data_ptr()), c_void_p(current_stream_handle())))
-        return token
+        return _run(self, pending, token, capi.lib().art_greedy_next, logits, vocab, prompt if has_prompt else None, prompt.numel() if has_prompt else 0,
+                    token, pos, embed, dim, x)
 
 
 builtin('greedy_next_f16')(lambda: GreedyNext())

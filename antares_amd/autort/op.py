@@ -20,7 +20,7 @@ import torch
 
 from ..ir import Graph, bake_small_reduce_extents, fuse_elementwise, pad_guarded_factors, parse_program, split_wide_reductions
 from ..lower import contraction_slices, lower_graph
-from ..runtime import capi
+from ..runtime import calls, capi
 
 TORCH_DTYPE = {'float64': torch.float64, 'float32': torch.float32, 'float16': torch.float16,
                'int64': torch.int64, 'int32': torch.int32, 'int16': torch.int16, 'int8': torch.int8,
@@ -64,7 +64,7 @@ def compile_cached(source: str) -> bytes:
     return image
 
 
-class ExportedOp:
+class ExportedOp(calls.Operator):
     """One einstein_v2 program bound to gfx950 kernels."""
 
     def __init__(self, ir: str, inputs, config: Optional[str] = None, name: Optional[str] = None,
@@ -100,7 +100,9 @@ class ExportedOp:
             info = self.fused.tensors.get(n) or self.graph.tensors[n]
             self._wanted_dtype[n] = (TORCH_DTYPE[info.dtype], info.dtype)
         self._declared_in_graph = [n for n in self.declared if n in self.fused.tensors]
-        self._shape_cache: Dict[tuple, tuple] = {}     # shapes of the declared tensors -> (dimension values, output shapes)
+        # the call's arguments in order: tensors by position (no keyword has a name that starts with `/`), the last
+        # output also as `out`; `extra` is taken and ignored
+        self._bind(tuple(['/' + n for n in self.declared + self.fresh_outputs[:-1]] + ['out', 'extra']), ())
 
     # -- persistence ---------------------------------------------------------
     def persist(self) -> Optional[str]:
@@ -127,7 +129,7 @@ class ExportedOp:
         return self._module
 
     # -- calling -------------------------------------------------------------
-    def __call__(self, *tensors, extra=None, out=None):
+    def _call(self, pending, *tensors, extra=None, out=None):
         g = self.fused
         nd = len(self.declared)
         if len(tensors) < nd:
@@ -147,32 +149,29 @@ class ExportedOp:
         for n, t in bound.items():
             self._check_tensor(n, t)
             dev = dev or t.device
+            if t.device != dev:            # a kernel must never see a host address or another device's
+                raise RuntimeError(f'{self.name}(): tensor `{n}` is on {t.device}, the ones before it on {dev}')
         if dev is None:
             dev = torch.device('cuda', torch.cuda.current_device())
         if dev.type != 'cuda':
             raise RuntimeError(f'{self.name}(): tensors must live on the GPU (got {dev}); there is no CPU fallback')
-        # dimension values and output shapes depend on the shapes of the declared tensors only: worked out once per
-        # combination of shapes (a decode loop calls with the same shapes every time)
-        key = tuple([bound[n].shape for n in self._declared_in_graph])
-        hit = self._shape_cache.get(key)
-        if hit is None:
-            env = g.bind_dims({n: tuple(bound[n].shape) for n in self._declared_in_graph})
-            hit = (env, {n: g.shape_of(n, env) for n in self.fresh_outputs})
-            if len(self._shape_cache) < 64:
-                self._shape_cache[key] = hit
-        env, wants = hit
+        env = g.bind_dims({n: tuple(bound[n].shape) for n in self._declared_in_graph})
         for n in self.fresh_outputs:
-            want = wants[n]
+            want = g.shape_of(n, env)
             if n in bound:
                 if bound[n].numel() != _numel(want):
                     raise ValueError(f'output `{n}` expects {want} ({_numel(want)} elements), got {list(bound[n].shape)}')
             else:
                 bound[n] = torch.empty(want, dtype=self._wanted_dtype[n][0], device=dev)
         capi.init(dev.index or 0)
-        stream = current_stream_handle(dev.index)
-        if self.fast_path is None or not self.fast_path(self, bound, env, stream):
-            self._run_generic(bound, env, dev, stream)
+        call = calls.Call(current_stream_handle(dev.index))
+        if self.fast_path is None or not self.fast_path(self, bound, env, call):
+            self._run_generic(bound, env, dev, call)
         outs = [bound[o] for o in self.graph.outputs]
+        # a call under capture could not search its launch parameters: it leaves no recipe, a later one still may
+        trials = self.config.get('tune')
+        if not (isinstance(trials, int) and trials > 0 and torch.cuda.is_current_stream_capturing()):
+            call.keep(self, pending, outs, device_stream=True)
         return outs[0] if len(outs) == 1 else tuple(outs)
 
     def _check_tensor(self, name: str, t: torch.Tensor):
@@ -218,7 +217,7 @@ class ExportedOp:
         dimensions launches from."""
         return self._variant(env)['plans']
 
-    def _run_generic(self, bound: Dict[str, torch.Tensor], env: Dict[str, int], dev, stream: int):
+    def _run_generic(self, bound: Dict[str, torch.Tensor], env: Dict[str, int], dev, call: calls.Call):
         variant = self._variant(env)
         module, g, plans_ = variant['module'], variant['graph'], variant['plans']
         dims = [env[d] for d in g.dim_names]
@@ -236,7 +235,7 @@ class ExportedOp:
                         bound[n] = torch.empty(g.shape_of(n, env), dtype=TORCH_DTYPE[g.tensors[n].dtype], device=dev)
                 sym, grid = group.choose(env, {n: bound[n].data_ptr() for n in group.args})
                 if grid:
-                    capi.launch(module.function(sym), (grid, 1, 1), (256, 1, 1), stream, [bound[n].data_ptr() for n in group.args] + dims)
+                    call.kernel(module.function(sym), grid, 256, [bound[n] for n in group.args] + dims)
                     skip = group.count - 1
                     continue
             for n in plan.args:
@@ -254,8 +253,7 @@ class ExportedOp:
             skip = plan.covers - 1         # a map applied at this reduction's stores
             if grid == 0:
                 continue
-            capi.launch(module.function(sym), (grid, 1, 1), (block, 1, 1), stream,
-                        [ptrs[n] for n in plan.args] + dims)
+            call.kernel(module.function(sym), grid, block, [bound[n] for n in plan.args] + dims)
 
     def _tune(self, plan, key: str, bound, dims, ptrs, env, module, trials: int):
         """``config="tune:N"``: times up to N launch configurations of one kernel for the extents of this call

@@ -19,6 +19,7 @@ import torch
 
 from ..ir import Graph, fuse_elementwise, parse_program
 from ..runtime import capi
+from ..runtime.calls import STREAM
 
 _TABLE: Dict[str, Tuple[Callable, list]] = {}      # canonical key -> (handler, the registered program's tensor order)
 
@@ -77,16 +78,14 @@ def _gptq_inputs(xdt: str, sdt: str):
     return [f'input0={xdt}[S:4096]', 'qweight=int32[L:512, N:12288]', f'scales={sdt}[K:32, N:12288]']
 
 
-def _gptq_handler(op, bound, env, stream) -> bool:
+def _gptq_handler(op, bound, env, call) -> bool:
     r = op.fast_roles
     x, q, s, out = bound[r['input0']], bound[r['qweight']], bound[r['scales']], bound[r['my_result']]
     x_f16, s_f16 = int(x.dtype == torch.float16), int(s.dtype == torch.float16)
     K, N = x.shape[0], q.shape[1]
-    qp = q.data_ptr()
-    if K % 128 or N % 4 or q.shape[0] * 8 != K or s.shape[0] * 128 != K or qp % 16:
+    if K % 128 or N % 4 or q.shape[0] * 8 != K or s.shape[0] * 128 != K or q.data_ptr() % 16:
         return False
-    capi.check(capi.lib().art_gemv_gptq(c_void_p(x.data_ptr()), c_void_p(qp), c_void_p(s.data_ptr()),
-                                       c_void_p(out.data_ptr()), K, N, x_f16, s_f16, c_void_p(stream)))
+    call.library(capi.lib().art_gemv_gptq, x, q, s, out, K, N, x_f16, s_f16, STREAM)
     return True
 
 
@@ -134,7 +133,7 @@ def tune_hand_kernel(op, key: str, candidates, run, trials: int, clones):
     return best
 
 
-def _w4a16_handler(op, bound, env, stream) -> bool:
+def _w4a16_handler(op, bound, env, call) -> bool:
     r = op.fast_roles
     x, q, s, z, y = bound[r['x']], bound[r['qweight']], bound[r['scales']], bound[r['qzeros']], bound[r['y']]
     M, K = x.shape
@@ -148,13 +147,14 @@ def _w4a16_handler(op, bound, env, stream) -> bool:
     lib = capi.lib()
     gemv = M <= 3
 
-    def run(value, t, st=None):
-        args = (c_void_p(t[0].data_ptr()), c_void_p(t[1].data_ptr()), c_void_p(t[2].data_ptr()), c_void_p(t[3].data_ptr()),
-                c_void_p(t[4].data_ptr()), M, K, N)
-        if gemv:         # value = 16 * rows per lane + wavefronts per block (0: the library's choice of both)
-            capi.check(lib.art_gemv_w4a16_knobs(*args, int(value) >> 4, int(value) & 15, c_void_p(stream if st is None else st)))
-        else:
-            capi.check(lib.art_gemm_w4a16_tuned(*args, int(value), c_void_p(stream if st is None else st)))
+    # the entry point and its launch parameters (GEMV: 16 * rows per lane + wavefronts per block, 0: the library's choice)
+    entry = lib.art_gemv_w4a16_knobs if gemv else lib.art_gemm_w4a16_tuned
+
+    def knobs(value):
+        return (int(value) >> 4, int(value) & 15) if gemv else (int(value),)
+
+    def run(value, t):
+        capi.check(entry(*(c_void_p(v.data_ptr()) for v in t), M, K, N, *knobs(value), c_void_p(torch.cuda.current_stream().cuda_stream)))
 
     # the launch parameters of the kernel that runs: (rows per lane, wavefronts per block) of the GEMV - two factors
     # searched as a product space, as the reference's tuner walks the factor spaces of a schedule's knobs
@@ -174,9 +174,9 @@ def _w4a16_handler(op, bound, env, stream) -> bool:
             # 1024 + v, 2048 + v: over blocks of 128 and 256 rows
             cands = [0] + [512 + v for v in counts] + ([256 + v for v in counts] if M > 32 else [])
             cands += [rows + v for rows in (1024, 2048) for v in counts if v <= 16] if M > 64 else []
-        saved = tune_hand_kernel(op, key, cands, lambda v, t: run(v, t, torch.cuda.current_stream().cuda_stream), trials, clones)
+        saved = tune_hand_kernel(op, key, cands, run, trials, clones)
         del clones
-    run(saved['value'] if saved is not None else 0, (x, q, s, z, y))
+    call.library(entry, x, q, s, z, y, M, K, N, *knobs(saved['value'] if saved is not None else 0), STREAM)
     return True
 
 
@@ -194,7 +194,7 @@ GEMM_F16_IR = """
 GEMM_F16_INPUTS = ['a=float16[M:4096, K:4096]', 'b=float16[K:4096, N:4096]']
 
 
-def _gemm_f16_handler(op, bound, env, stream) -> bool:
+def _gemm_f16_handler(op, bound, env, call) -> bool:
     r = op.fast_roles
     a, b, c = bound[r['a']], bound[r['b']], bound[r['c']]
     M, K = a.shape
@@ -202,17 +202,17 @@ def _gemm_f16_handler(op, bound, env, stream) -> bool:
     if N % 8 or K % 64 or a.data_ptr() % 16 or b.data_ptr() % 16 or c.data_ptr() % 16:
         return False
 
-    def run(value, t, st=None):
+    def run(value, t):
         capi.check(capi.lib().art_gemm_f16_tuned(c_void_p(t[0].data_ptr()), c_void_p(t[1].data_ptr()), c_void_p(t[2].data_ptr()), M, N, K,
-                                                 int(value), c_void_p(stream if st is None else st)))
+                                                 int(value), c_void_p(torch.cuda.current_stream().cuda_stream)))
     # the launch parameter: threads per block (2 x 2 wavefronts of 128 x 128 outputs, or 2 x 4 of 128 x 64)
     key = f'gemm_f16.threads|{M},{K},{N}'
     saved = op.tuned.get(key)
     trials = op.config.get('tune')
     if saved is None and isinstance(trials, int) and trials > 0 and not torch.cuda.is_current_stream_capturing():
-        saved = tune_hand_kernel(op, key, [256, 512], lambda v, t: run(v, t, torch.cuda.current_stream().cuda_stream), trials,
+        saved = tune_hand_kernel(op, key, [256, 512], run, trials,
                                  [(a, b, torch.empty_like(c))])
-    run(saved['value'] if saved is not None else 0, (a, b, c))
+    call.library(capi.lib().art_gemm_f16_tuned, a, b, c, M, N, K, int(saved['value'] if saved is not None else 0), STREAM)
     return True
 
 
@@ -226,7 +226,7 @@ GEMM_F32_IR = 'c[M, N] +=! a[M, K] * b[K, N]'
 GEMM_F32_INPUTS = ['a=float32[M:4096, K:4096]', 'b=float32[K:4096, N:4096]']
 
 
-def _gemm_f32_handler(op, bound, env, stream) -> bool:
+def _gemm_f32_handler(op, bound, env, call) -> bool:
     r = op.fast_roles
     a, b, c = bound[r['a']], bound[r['b']], bound[r['c']]
     M, K = a.shape
@@ -235,15 +235,15 @@ def _gemm_f32_handler(op, bound, env, stream) -> bool:
     if N % 4 or K % 32 or N < 4 or M * N < 128 * 128 * 32 or a.data_ptr() % 16 or b.data_ptr() % 16:
         return False
 
-    def run(_, t, st=None):
+    def run(_, t):
         capi.check(capi.lib().art_gemm_f32(c_void_p(t[0].data_ptr()), c_void_p(t[1].data_ptr()), c_void_p(t[2].data_ptr()), M, N, K,
-                                          c_void_p(stream if st is None else st)))
+                                          c_void_p(torch.cuda.current_stream().cuda_stream)))
     # the kernel has no launch parameter to search; a tuning run records its time for the shape in the module file
     key = f'gemm_f32|{M},{K},{N}'
     trials = op.config.get('tune')
     if key not in op.tuned and isinstance(trials, int) and trials > 0 and not torch.cuda.is_current_stream_capturing():
-        tune_hand_kernel(op, key, [0], lambda v, t: run(v, t, torch.cuda.current_stream().cuda_stream), 1, [(a, b, torch.empty_like(c))])
-    run(0, (a, b, c))
+        tune_hand_kernel(op, key, [0], run, 1, [(a, b, torch.empty_like(c))])
+    call.library(capi.lib().art_gemm_f32, a, b, c, M, N, K, STREAM)
     return True
 
 
@@ -257,7 +257,7 @@ BATCH_GEMM_F32_IR = 'c[B, M, N] +=! a[B, M, K] * b[B, K, N]'
 BATCH_GEMM_F32_INPUTS = ['a=float32[B:3, M:1024, K:512]', 'b=float32[B:3, K:512, N:512]']
 
 
-def _batch_gemm_f32_handler(op, bound, env, stream) -> bool:
+def _batch_gemm_f32_handler(op, bound, env, call) -> bool:
     r = op.fast_roles
     a, b, c = bound[r['a']], bound[r['b']], bound[r['c']]
     batch, M, K = a.shape
@@ -266,8 +266,7 @@ def _batch_gemm_f32_handler(op, bound, env, stream) -> bool:
     if N % 4 or K % 32 or N < 4 or batch > 65535 or batch * M * N < 128 * 128 * 32 or a.data_ptr() % 16 or b.data_ptr() % 16 \
             or (M * K) % 4 or (K * N) % 4:
         return False
-    capi.check(capi.lib().art_gemm_f32_batched(c_void_p(a.data_ptr()), c_void_p(b.data_ptr()), c_void_p(c.data_ptr()), batch, M, N, K,
-                                              c_void_p(stream)))
+    call.library(capi.lib().art_gemm_f32_batched, a, b, c, batch, M, N, K, STREAM)
     return True
 
 
@@ -278,15 +277,14 @@ register(BATCH_GEMM_F32_IR, BATCH_GEMM_F32_INPUTS, _batch_gemm_f32_handler)
 # fp32 GEMM with an operand stored the other way round: A as [K, M], B as [N, K] (a linear layer's weight)
 # ---------------------------------------------------------------------------
 def _gemm_f32_layout_handler(trans_a: bool, trans_b: bool):
-    def handler(op, bound, env, stream) -> bool:
+    def handler(op, bound, env, call) -> bool:
         r = op.fast_roles
         a, b, c = bound[r['a']], bound[r['b']], bound[r['c']]
         (K, M) = a.shape if trans_a else a.shape[::-1]
         N = b.shape[0] if trans_b else b.shape[1]
         if K % 32 or (not trans_b and N % 4) or (trans_a and M % 4) or M * N < 128 * 128 * 32 or a.data_ptr() % 16 or b.data_ptr() % 16:
             return False
-        capi.check(capi.lib().art_gemm_f32_ex(c_void_p(a.data_ptr()), c_void_p(b.data_ptr()), c_void_p(c.data_ptr()), 1, M, N, K,
-                                             int(trans_a), int(trans_b), c_void_p(stream)))
+        call.library(capi.lib().art_gemm_f32_ex, a, b, c, 1, M, N, K, int(trans_a), int(trans_b), STREAM)
         return True
     return handler
 

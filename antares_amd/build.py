@@ -1,4 +1,4 @@
-"""Builds libantares_amd.so for gfx950 with hipcc (cross-compiles without a GPU).
+"""Builds libantares_amd.so for gfx950 with hipcc (cross-compiles without a GPU) and the host extension with g++.
 
     python -m antares_amd.build
 """
@@ -12,10 +12,32 @@ import sys
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, 'csrc')
 OUT = os.path.join(CSRC, 'libantares_amd.so')
+CALLS_OUT = os.path.join(HERE, 'runtime', '_calls.so')
 
 # packed-FP32 instruction selection is switched off for all device code
 FLAGS = ['--offload-arch=gfx950', '-O3', '-std=c++17', '-fPIC', '-shared',
          '-Xclang', '-target-feature', '-Xclang', '-packed-fp32-ops', '-Wno-unused-result']
+
+
+def build_calls(verbose: bool = True) -> str:
+    """The host-side extension (operator calls replayed in native code) against torch's C++ headers."""
+    import sysconfig
+
+    import torch
+    root = os.path.dirname(torch.__file__)
+    include = [os.path.join(root, 'include'), os.path.join(root, 'include', 'torch', 'csrc', 'api', 'include'), '/opt/rocm/include',
+               sysconfig.get_paths()['include']]
+    cmd = ['g++', '-O2', '-std=c++17', '-fPIC', '-shared', '-w', '-D__HIP_PLATFORM_AMD__', '-DUSE_ROCM',
+           f'-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}'] + [f'-I{i}' for i in include] + \
+        [os.path.join(CSRC, 'host', 'calls.cpp'), '-o', CALLS_OUT + '.tmp', f'-L{os.path.join(root, "lib")}',
+         '-ltorch_python', '-ltorch_hip', '-ltorch_cpu', '-lc10_hip', '-lc10']
+    if verbose:
+        print('[antares_amd.build]', ' '.join(cmd), flush=True)
+    p = subprocess.run(cmd, capture_output=True, text=True)
+    if p.returncode != 0:
+        raise RuntimeError(f'g++ failed:\n{p.stdout}\n{p.stderr}')
+    os.replace(CALLS_OUT + '.tmp', CALLS_OUT)
+    return CALLS_OUT
 
 
 def build(verbose: bool = True) -> str:
@@ -30,6 +52,7 @@ def build(verbose: bool = True) -> str:
     if err.strip() and verbose:
         print(err)
     os.replace(OUT + '.tmp', OUT)
+    build_calls(verbose)
     return OUT
 
 

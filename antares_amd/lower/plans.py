@@ -8,12 +8,26 @@ from dataclasses import dataclass, field
 from typing import Callable, Dict, List, Optional, Tuple
 
 from ..ir.nodes import Expr, ITEMSIZE, walk
+from ..runtime import calls
 from .emit_common import BLOCK, MAX_GRID
 
 
+class _Rule:
+    """A launch rule (`choose`) that is replaced on a plan - a forced variant - also ends the recipes made by the old one."""
+
+    def __setattr__(self, name, value):
+        object.__setattr__(self, name, value)
+        if name == 'choose':
+            calls.forget()
+
+    def __delattr__(self, name):
+        object.__delattr__(self, name)
+        if name == 'choose':
+            calls.forget()
+
 
 @dataclass
-class RowGroup:
+class RowGroup(_Rule):
     """A run of statements that one kernel computes row by row: reductions over the last axis of a row followed by
     the map that uses their results (softmax, layer normalisation, AntaresIR.md:226-232)."""
     symbol: str                    # the kernel for rows of any length: a block per row, the row walked per statement
@@ -66,7 +80,7 @@ class RowGroup:
 
 
 @dataclass
-class KernelPlan:
+class KernelPlan(_Rule):
     """Everything the runtime needs to launch one statement."""
     name: str                      # base kernel name
     args: List[str]                # tensor argument order

@@ -1,0 +1,124 @@
+"""Operators whose calls are replayed in native code.
+
+``Operator`` (``csrc/host/calls.cpp``) is the base class of everything callable in ``autort.ops``.  A call whose
+signature - dtypes, shapes, devices, contiguity and 16-byte alignment of the tensors, which arguments are given - has been
+seen before is replayed from a recipe without entering Python; any other call reaches the subclass's ``_call(pending,
+...)``, which checks the arguments, runs the operator and leaves the recipe with ``pending`` (None when the arguments are
+nothing a recipe can be kept for).
+"""
+from __future__ import annotations
+
+import ctypes
+from ctypes import c_void_p
+
+import torch
+
+from . import capi
+
+try:
+    from . import _calls
+    Operator = _calls.Operator
+except ImportError as _e:                     # not built: operators can still be made (lowering, compiling), not called
+    _calls, _reason = None, str(_e)
+
+    class Operator:
+        tuned = config = fast_path = None
+
+        def _bind(self, names, dynamic):
+            pass
+
+        def __call__(self, *args, **kwargs):
+            raise capi.ArtError(f'antares_amd/runtime/_calls.so cannot be loaded ({_reason}): build it with `python -m antares_amd.build`')
+
+_ready = False
+
+
+def setup():
+    """Hands the native side the library's launch entry point; before the first recipe is kept."""
+    global _ready
+    if not _ready:
+        lib = capi.lib()
+        _calls.setup(ctypes.cast(lib.art_launch, c_void_p).value, ctypes.cast(lib.art_last_error, c_void_p).value, capi.ArtError,
+                     torch.nn.Parameter)
+        _ready = True
+
+
+def forget():
+    """Every recipe is worked out again at its next call (the rules of a launch plan have changed)."""
+    if _calls is not None:
+        _calls.forget()
+
+
+class Stream:
+    """The stream of the call, as an argument."""
+
+
+STREAM = Stream()
+
+
+class Number:
+    """Number ``index`` of the call's list argument, passed on as it is: its value now, and its place in later calls."""
+    __slots__ = ('value', 'slot', 'kind')
+
+    def __init__(self, value, slot: int, kind: str):
+        self.value, self.slot, self.kind = value, slot, kind
+
+
+class Call:
+    """What one call of an operator launches, in order: kernels and entry points of the library, with tensors as
+    tensors, the stream as STREAM, list numbers as Number, and constants."""
+
+    def __init__(self, stream: int):
+        self.stream = stream
+        self.steps = []
+
+    def library(self, fn, *args):
+        self.steps.append((fn, None, None, args))
+        values = [c_void_p(a.data_ptr()) if isinstance(a, torch.Tensor) else c_void_p(self.stream) if a is STREAM else
+                  a.value if isinstance(a, Number) else c_void_p(0) if a is None else a for a in args]
+        capi.check(fn(*values))
+
+    def kernel(self, func, grid: int, block: int, args):
+        self.steps.append((func, (grid, 1, 1), (block, 1, 1), args))
+        capi.launch(func, (grid, 1, 1), (block, 1, 1), self.stream, [a.data_ptr() if isinstance(a, torch.Tensor) else a for a in args])
+
+    def keep(self, op: Operator, pending, results, device_stream: bool):
+        """Leaves the recipe of this call with the operator.  Tensors that are not among the call's arguments are
+        allocated afresh by every later call."""
+        if pending is None:
+            return
+        setup()
+        key, slots, device = pending
+        place, owned = {}, set()
+        for i, s in enumerate(slots):             # one tensor in two places is part of the signature
+            if isinstance(s, torch.Tensor):
+                place.setdefault(id(s), i)
+                owned.add(s.untyped_storage().data_ptr())
+        fresh = []
+
+        def index(t):
+            at = place.get(id(t))
+            if at is None:
+                if t.numel() and t.untyped_storage().data_ptr() in owned:
+                    raise RuntimeError('a recipe takes its arguments as they were passed, not views of them')
+                at = place[id(t)] = len(slots) + len(fresh)
+                fresh.append(t)
+            return at
+
+        def encode(fn, a):
+            if isinstance(a, torch.Tensor):
+                return ('p', index(a))
+            if a is STREAM:
+                return ('s',)
+            if isinstance(a, Number):
+                return (a.kind, a.slot)
+            if isinstance(a, float):
+                return ('f', a)
+            return ('i', int(a or 0))
+        launches = []
+        for fn, grid, block, args in self.steps:
+            address = fn.value if grid is not None else ctypes.cast(fn, c_void_p).value
+            launches.append((address, grid, block, [encode(fn, a) for a in args]))
+        outs = [index(t) for t in results]
+        if len(fresh) <= 16:
+            op._commit(key, len(slots), device, int(device_stream), [(t.dtype, tuple(t.shape)) for t in fresh], launches, outs)

@@ -1,0 +1,96 @@
+"""Calls replayed in native code: what belongs to a signature (shapes, alignment, one tensor in two places, which
+arguments are given) leads to a recipe of its own, what does not (addresses, numbers in `extra`) is taken from the call,
+and a call that cannot be replayed still raises what it raised before."""
+import threading
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope='module')
+def op():
+    import autort
+    return autort.export(ir='output0[N] = input0[N] + input1[N]', inputs=['input0=float32[N:64]', 'input1=float32[N:64]'], name='calls_add')
+
+
+@pytest.mark.parametrize('n', [0, 1, 3, 4, 1000, 4099])
+def test_every_signature_gets_its_own_recipe(op, n):
+    import autort
+    print(f'[case] calls n={n}', flush=True)
+    dev = autort.device()
+    for offset in (0, 1, 4):                                 # aligned, not aligned, aligned again
+        for _ in range(3):
+            a, b = torch.randn(n + 4, device=dev)[offset:n + offset], torch.randn(n, device=dev)
+            assert a.numel() == n and torch.equal(op(a, b), a + b)
+            assert torch.equal(op(a, a), a + a)              # one tensor in two places ...
+            assert torch.equal(op(b, a), a + b)              # ... is not what two tensors are
+            out = torch.empty(n, device=dev)
+            assert op(a, b, out=out) is out and torch.equal(out, a + b)
+            assert op(a, b, out) is out
+            kept = a.clone()
+            assert op(a, b, out=a) is a and torch.equal(a, kept + b)
+
+
+def test_errors_are_raised_after_a_replayed_call_too(op):
+    import autort
+    dev = autort.device()
+    a = torch.randn(100, device=dev)
+    op(a, a)
+    op(a, a)
+    for bad in ((a,), (a, a.half()), (a, a.cpu()), (a, torch.randn(200, device=dev)[::2]), (a, 1.0), (a, a, torch.empty(7, device=dev)), (a, torch.randn(99, device=dev))):
+        with pytest.raises(Exception):
+            op(*bad)
+    with pytest.raises(TypeError):
+        op(a, input1=a)
+    assert torch.equal(op(a, a), a + a)
+
+
+def test_numbers_in_extra_and_the_stream_are_taken_from_the_call():
+    import autort
+    dev = autort.device()
+    x, w = torch.randn(256, device=dev), torch.randn(256, device=dev)
+    vsum = (x * x).sum().view(1)
+    for inv_n in (1 / 256, 1 / 64, 1.0, 1):
+        want = x * torch.rsqrt(vsum * inv_n + 1e-5) * w
+        assert torch.allclose(autort.ops.rmsnorm_f32(x, vsum, w, extra=[inv_n]), want, rtol=1e-4, atol=1e-5)
+    q = torch.randn(2, 2, 64, device=dev)
+    inv = torch.rand(128, device=dev)
+    for pos in (0, 1, 77, torch.tensor([77], dtype=torch.int32, device=dev), torch.tensor([3], dtype=torch.int32, device=dev)):
+        angle = float(pos) * inv[:64]
+        want = torch.cat([q[:, 0] * angle.cos() - q[:, 1] * angle.sin(), q[:, 1] * angle.cos() + q[:, 0] * angle.sin()], 1)
+        got = autort.ops.rotary_f32(q, inv, torch.empty(2, 128, device=dev), extra=[pos])
+        assert torch.allclose(got, want, rtol=1e-4, atol=1e-4)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        g = torch.cuda.CUDAGraph()
+        out = torch.zeros(256, device=dev)
+        autort.ops.rmsnorm_f32(x, vsum, w, out, extra=[1.0])
+        side.synchronize()
+        with torch.cuda.graph(g, stream=side):               # recorded on the capturing stream: not run yet
+            autort.ops.rmsnorm_f32(x, vsum, w, out, extra=[0.25])
+        first = out.clone()
+        g.replay()
+    side.synchronize()
+    assert not torch.equal(first, out) and torch.allclose(out, x * torch.rsqrt(vsum * 0.25 + 1e-5) * w, rtol=1e-4, atol=1e-5)
+
+
+def test_several_threads_call_one_operator(op):
+    import autort
+    dev = autort.device()
+    wrong = []
+
+    def work(i):
+        with torch.cuda.stream(torch.cuda.Stream()):
+            for k in range(50):
+                a = torch.full((64 + (i + k) % 7,), float(i), device=dev)
+                if not torch.equal(op(a, a), a + a):
+                    wrong.append((i, k))
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong
