@@ -467,6 +467,30 @@ class GemmW4Residual(calls.Operator):
 builtin('gemm_w4a16_residual')(lambda: GemmW4Residual())
 
 
+class GemmW4Swiglu(calls.Operator):
+    """``gemm_w4a16_swiglu(x[M,K], qweight[K/2,2F], scales, qzeros, out[M,F])``: the packed int4 product of a batch of rows
+    with a gate | up matrix and the SwiGLU of its two halves, out = fp16(silu(gate) * up)."""
+    name = 'gemm_w4a16_swiglu'
+
+    def __init__(self):
+        self._bind(('x', 'qweight', 'scales', 'qzeros', 'out'), ())
+
+    def _call(self, pending, x, qweight, scales, qzeros, out=None):
+        M, K = x.shape
+        N = qweight.shape[1]
+        if out is None:
+            out = torch.empty(M, N // 2, dtype=torch.float16, device=x.device)
+        if qweight.shape[0] * 2 != K or scales.shape != (K // 128, N) or qzeros.shape != (K // 128, N // 2) or out.shape != (M, N // 2):
+            raise ValueError('gemm_w4a16_swiglu: operand shapes do not match M, K, N')
+        if x.dtype != torch.float16 or scales.dtype != torch.float16 or out.dtype != torch.float16:
+            raise TypeError('gemm_w4a16_swiglu: x, scales and out must be float16')
+        _require_cuda(x, qweight, scales, qzeros, out)
+        return _run(self, pending, out, capi.lib().art_gemm_w4a16_swiglu, x, qweight, scales, qzeros, out, M, K, N, 0)
+
+
+builtin('gemm_w4a16_swiglu')(lambda: GemmW4Swiglu())
+
+
 class GemvW4Attn(calls.Operator):
     """``gemv_w4a16_attn(partial[H, P, 132], qweight, scales, qzeros, out[N], residual=None)``: the int4 projection of a
     split attention's output (merged on the fly) with the residual add folded in."""

@@ -59,7 +59,8 @@ __device__ __forceinline__ void load_lds_x1(const void* g, unsigned int lds_dst)
                : "=&s"(keep) : "v"(g), "s"(lds_dst) : "memory");
 }
 
-template <int MT>   // MT accumulator tiles of 32 rows: a block owns 32 MT rows
+// MT accumulator tiles of 32 rows: a block owns 32 MT rows.  SWIGLU: see art_gemm_w4_wide.hip
+template <int MT, bool SWIGLU>
 __global__ __launch_bounds__(kThreads) void gemm_w4a16_kernel(const _Float16* __restrict__ x, const unsigned char* __restrict__ qweight,
                                                               const _Float16* __restrict__ scales,
                                                               const unsigned char* __restrict__ qzeros, _Float16* y,
@@ -78,13 +79,13 @@ __global__ __launch_bounds__(kThreads) void gemm_w4a16_kernel(const _Float16* __
   const int m_block = (int)(blockIdx.x % (8 * m_blocks)) / 8;
   if (unit >= col_tiles * splits) return;
   const int split = unit / col_tiles;
-  const int n0 = (unit % col_tiles) * BN;
+  const TileColumns<SWIGLU> cols{(unit % col_tiles) * (SWIGLU ? BN / 2 : BN), N};
   constexpr int RB = 32 * MT;                       // rows of a block
   constexpr int kLoadsPerGroup = 3 + MT;            // LDS-direct loads per wavefront and group: 2 weights, MT x, 1 scales / zero points
   const int m0 = m_block * RB;
   const int M = M_total - m0 < RB ? M_total - m0 : RB;          // rows of this block
   x += (size_t)m0 * K;
-  y += (size_t)m0 * N;
+  y += (size_t)m0 * (SWIGLU ? N / 2 : N);
   if (residual) residual += (size_t)m0 * N;
   const int g_begin = (int)((long long)G * split / splits), g_end = (int)((long long)G * (split + 1) / splits);
   const int groups = g_end - g_begin;
@@ -98,8 +99,7 @@ __global__ __launch_bounds__(kThreads) void gemm_w4a16_kernel(const _Float16* __
 #pragma unroll
   for (int u = 0; u < 2; ++u) {
     const int r = 4 * (wave + 8 * u) + (lane >> 4);
-    const int col = n0 + ((lane & 15) ^ (r & 7)) * 16;            // N % 16 == 0: a chunk is inside or outside as a whole
-    wsrc[u] = qweight + ((size_t)g_begin * (GK / 2) + r) * N + (col < N ? col : 0);
+    wsrc[u] = qweight + ((size_t)g_begin * (GK / 2) + r) * N + cols.safe(((lane & 15) ^ (r & 7)) * 16);
     xsrc[u] = x + (size_t)(r < M ? r : M - 1) * K + (size_t)g_begin * GK + ((lane & 15) ^ (r & 15)) * 8;
   }
   const unsigned char* qsrc;
@@ -107,12 +107,10 @@ __global__ __launch_bounds__(kThreads) void gemm_w4a16_kernel(const _Float16* __
   {
     const int d = wave * 64 + lane;                 // dword of the 2 KiB area
     if (d < 128) {                                  // scales of columns 2 d, 2 d + 1
-      const int col = n0 + 2 * d;
-      qsrc = reinterpret_cast<const unsigned char*>(scales + (size_t)g_begin * N + (col < N ? col : 0));
+      qsrc = reinterpret_cast<const unsigned char*>(scales + (size_t)g_begin * N + cols.safe(2 * d));
       qstep = 2 * N;
     } else if (d < 160) {                           // zero points of columns 8 (d - 128) .. + 7
-      const int col = n0 + 8 * (d - 128);
-      qsrc = qzeros + (size_t)g_begin * (N / 2) + ((col < N ? col : 0) >> 1);
+      qsrc = qzeros + (size_t)g_begin * (N / 2) + (cols.safe(8 * (d - 128)) >> 1);
       qstep = N / 2;
     } else {                                        // idle lanes re-read the first scales into the padding
       qsrc = reinterpret_cast<const unsigned char*>(scales + (size_t)g_begin * N);
@@ -170,7 +168,7 @@ __global__ __launch_bounds__(kThreads) void gemm_w4a16_kernel(const _Float16* __
     for (int ct = 0; ct < 2; ++ct) {
       const _Float16 sc = *reinterpret_cast<const _Float16*>(st + W_BYTES + X_BYTES + colpos[ct] * 2);
       const unsigned int zb = st[W_BYTES + X_BYTES + 512 + (colpos[ct] >> 1)];
-      const _Float16 s = (n0 + colpos[ct] < N) ? sc : (_Float16)0.f;
+      const _Float16 s = cols.inside(colpos[ct]) ? sc : (_Float16)0.f;
       s2[ct] = h2{s, s};
       const unsigned int z = (zb >> ((colpos[ct] & 1) * 4)) & 15u;
       const unsigned int zz = z | (z << 16);
@@ -246,44 +244,53 @@ __global__ __launch_bounds__(kThreads) void gemm_w4a16_kernel(const _Float16* __
 #pragma unroll 1
   for (int e = tid; e < MT * 32 * (BN / 4); e += kThreads) {
     const int row = e >> 6, c4 = (e & 63) * 4;
-    if (row >= M || n0 + c4 >= N) continue;         // N % 4 == 0: four columns are inside or outside as a whole
+    if (row >= M || !cols.inside(c4)) continue;
+    const size_t at = (size_t)row * N + cols.at(c4);
     const f32x4 v = *reinterpret_cast<const f32x4*>(red + (size_t)row * RLD + c4) +
                     *reinterpret_cast<const f32x4*>(red + ((size_t)BM + row) * RLD + c4);
-    if (splits == 1) {
+    if (SWIGLU && splits == 1) {                    // the gate half of the tile works, with the up half 128 columns further on
+      if (c4 >= 128) continue;
+      const f32x4 u = *reinterpret_cast<const f32x4*>(red + (size_t)row * RLD + 128 + c4) +
+                      *reinterpret_cast<const f32x4*>(red + ((size_t)BM + row) * RLD + 128 + c4);
+      *reinterpret_cast<h4*>(y + (size_t)row * (N / 2) + cols.at(c4)) =
+          swiglu4(h4{(_Float16)v[0], (_Float16)v[1], (_Float16)v[2], (_Float16)v[3]}, h4{(_Float16)u[0], (_Float16)u[1], (_Float16)u[2], (_Float16)u[3]});
+    } else if (splits == 1) {
       h4 o = h4{(_Float16)v[0], (_Float16)v[1], (_Float16)v[2], (_Float16)v[3]};
       if (residual) {                               // y = fp16(fp16(product) + residual); may alias y: same elements
-        const h4 res = *reinterpret_cast<const h4*>(residual + (size_t)row * N + n0 + c4);
+        const h4 res = *reinterpret_cast<const h4*>(residual + at);
         o = h4{(_Float16)((float)o[0] + (float)res[0]), (_Float16)((float)o[1] + (float)res[1]),
                (_Float16)((float)o[2] + (float)res[2]), (_Float16)((float)o[3] + (float)res[3])};
       }
-      *reinterpret_cast<h4*>(y + (size_t)row * N + n0 + c4) = o;
+      *reinterpret_cast<h4*>(y + at) = o;
     } else {
-      *reinterpret_cast<f32x4*>(partial + ((size_t)split * M_total + m0 + row) * N + n0 + c4) = v;
+      *reinterpret_cast<f32x4*>(partial + ((size_t)split * M_total + m0) * N + at) = v;
     }
   }
 }
 
-// y[m,n] = fp16(sum over splits, in split order); four columns per thread (N % 4 == 0).
+// Four neighbouring sums over the K-splits, in split order: eight splits at a time, all eight loads issued before the
+// first is added (a loop of load-then-add runs one memory round trip per split).  Past the last split a load repeats
+// split 0 and is not added.
+__device__ __forceinline__ f32x4 sum_splits(const float* partial, long long split_stride, int splits) {
+  f32x4 t = *reinterpret_cast<const f32x4*>(partial);
+  for (int s0 = 1; s0 < splits; s0 += 8) {
+    f32x4 v[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = *reinterpret_cast<const f32x4*>(partial + (s0 + j < splits ? s0 + j : 0) * split_stride);
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      if (s0 + j < splits) t += v[j];
+  }
+  return t;
+}
+
+// y[m,n] = fp16(sum over splits); four columns per thread (N % 4 == 0).
 __global__ __launch_bounds__(256) void gemm_w4a16_combine_kernel(const float* __restrict__ partial, _Float16* y,
                                                                   long long count4, long long split_stride, int splits,
                                                                   const _Float16* residual) {
   const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
   if (i >= count4) return;
-  // eight splits at a time: all eight loads are issued before the first is added (a loop of load-then-add runs one
-  // memory round trip per split); the additions keep the split order.  Past the last split a load repeats split 0
-  // and is not added.
-  f32x4 t = *reinterpret_cast<const f32x4*>(partial + i * 4);
-  for (int s0 = 1; s0 < splits; s0 += 8) {
-    f32x4 v[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const int s = s0 + j < splits ? s0 + j : 0;
-      v[j] = *reinterpret_cast<const f32x4*>(partial + s * split_stride + i * 4);
-    }
-#pragma unroll
-    for (int j = 0; j < 8; ++j)
-      if (s0 + j < splits) t += v[j];
-  }
+  const f32x4 t = sum_splits(partial + i * 4, split_stride, splits);
   h4 out = h4{(_Float16)t[0], (_Float16)t[1], (_Float16)t[2], (_Float16)t[3]};
   if (residual) {                    // y = fp16(fp16(product) + residual); residual may be y itself
     const h4 res = *reinterpret_cast<const h4*>(residual + i * 4);
@@ -291,6 +298,18 @@ __global__ __launch_bounds__(256) void gemm_w4a16_combine_kernel(const float* __
              (_Float16)((float)out[2] + (float)res[2]), (_Float16)((float)out[3] + (float)res[3])};
   }
   *reinterpret_cast<h4*>(y + i * 4) = out;
+}
+
+// The same for gate | up: y[m, n] of N / 2 columns from the sums of columns n and N / 2 + n.
+__global__ __launch_bounds__(256) void gemm_w4a16_combine_swiglu_kernel(const float* __restrict__ partial, _Float16* y, int rows, int N,
+                                                                         int splits) {
+  const int quads = N / 8;           // groups of four output columns
+  const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
+  if (i >= (long long)rows * quads) return;
+  const long long row = i / quads, col = (i % quads) * 4, stride = (long long)rows * N;
+  const f32x4 g = sum_splits(partial + row * N + col, stride, splits), u = sum_splits(partial + row * N + N / 2 + col, stride, splits);
+  *reinterpret_cast<h4*>(y + row * (N / 2) + col) = swiglu4(h4{(_Float16)g[0], (_Float16)g[1], (_Float16)g[2], (_Float16)g[3]},
+                                                            h4{(_Float16)u[0], (_Float16)u[1], (_Float16)u[2], (_Float16)u[3]});
 }
 
 // Number of K-splits: as many blocks as the chip holds at once (one per compute unit), but at least
@@ -375,10 +394,85 @@ int choose_wide(int M, int K, int N, size_t scratch_bytes, int compute_units, in
   return row_tiles;
 }
 
-int combine(const float* partial, _Float16* y, int rows, int N, int splits, const _Float16* residual, hipStream_t stream) {
+int combine(const float* partial, _Float16* y, int rows, int N, int splits, const _Float16* residual, bool swiglu, hipStream_t stream) {
+  if (swiglu) {
+    gemm_w4a16_combine_swiglu_kernel<<<dim3((unsigned)(((long long)rows * (N / 8) + 255) / 256)), 256, 0, stream>>>(partial, y, rows, N, splits);
+    ART_LAUNCH_CHECK();
+    return 0;
+  }
   const long long count4 = (long long)rows * N / 4;
   gemm_w4a16_combine_kernel<<<dim3((unsigned)((count4 + 255) / 256)), 256, 0, stream>>>(partial, y, count4, (long long)rows * N, splits, residual);
   ART_LAUNCH_CHECK();
+  return 0;
+}
+
+int run(const void* x_dev, const void* qweight_dev, const void* scales_dev, const void* qzeros_dev, void* y_dev, const void* residual_dev,
+        int M, int K, int N, int k_splits, bool swiglu, void* stream) {
+  const int n_out = swiglu ? N / 2 : N;
+  const int want_rows = k_splits >> 8;              // 0: library's choice; else rows of a block / 32
+  ART_REQUIRE(k_splits >= 0 && (want_rows <= 2 || want_rows == 4 || want_rows == 8),
+              "art_gemm_w4a16: k_splits must be 0 (library's choice) or 1..255, plus 256 x the rows-per-block code 1, 2, 4 or 8 (got %d)", k_splits);
+  ART_REQUIRE(((uintptr_t)residual_dev % 8) == 0, "art_gemm_w4a16: the residual must be 8-byte aligned");
+  ART_REQUIRE(!art::overlaps(x_dev, (size_t)M * K * 2, y_dev, (size_t)M * n_out * 2), "art_gemm_w4a16: y must not overlap x");
+  ART_REQUIRE(x_dev && qweight_dev && scales_dev && qzeros_dev && y_dev, "art_gemm_w4a16: null pointer");
+  ART_REQUIRE(M >= 1, "art_gemm_w4a16: M must be positive (got %d)", M);
+  ART_REQUIRE(K > 0 && N > 0 && K % 128 == 0 && N % 16 == 0, "art_gemm_w4a16: need K %% 128 == 0 and N %% 16 == 0 (K=%d N=%d)", K, N);
+  ART_REQUIRE(((uintptr_t)qweight_dev % 16) == 0 && ((uintptr_t)x_dev % 16) == 0 && ((uintptr_t)qzeros_dev % 8) == 0 &&
+                  ((uintptr_t)y_dev % 8) == 0 && ((uintptr_t)scales_dev % 4) == 0,
+              "art_gemm_w4a16: x and qweight must be 16-byte aligned, qzeros and y 8-byte aligned, scales 4-byte aligned");
+  art::Workspace* wsp = art::workspace((hipStream_t)stream);
+  if (!wsp) return 1;
+  art::Workspace& ws = *wsp;
+  float* scratch = reinterpret_cast<float*>((char*)ws.base + art::kScratchOffset);
+  const size_t scratch_bytes = ws.bytes - art::kScratchOffset;
+  static int compute_units = 0;
+  if (compute_units == 0) {
+    int dev = 0;
+    ART_HIP(hipGetDevice(&dev));
+    ART_HIP(hipDeviceGetAttribute(&compute_units, hipDeviceAttributeMultiprocessorCount, dev));
+    for (const auto kernel : {gemm_w4a16_kernel<1, false>, gemm_w4a16_kernel<2, false>, gemm_w4a16_kernel<1, true>, gemm_w4a16_kernel<2, true>})
+      ART_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLdsBytes));
+  }
+  hipStream_t st = (hipStream_t)stream;
+  const int G = K / GK, col_tiles = tile_count(N, swiglu);
+  // Up to kMaxRowBlocks row blocks of this file's kernel go into one launch; longer batches take several passes over the
+  // weights.  The caller's choice of kernel and rows per block arrives in the upper bits of k_splits.
+  k_splits &= 0xff;
+  int row_tiles = want_rows >= 4 ? want_rows : 0, wide_splits = k_splits;
+  if (want_rows == 0 && k_splits == 0) row_tiles = choose_wide(M, K, N, scratch_bytes, compute_units, &wide_splits);
+  if (row_tiles) {
+    const size_t per_split = (size_t)M * N * sizeof(float);
+    if (wide_splits > G) wide_splits = G;
+    if ((size_t)wide_splits * per_split > scratch_bytes) wide_splits = (int)(scratch_bytes / per_split);
+    if (wide_splits < 1) wide_splits = 1;
+    if (art::w4::gemm_wide((const _Float16*)x_dev, (const unsigned char*)qweight_dev, (const _Float16*)scales_dev,
+                           (const unsigned char*)qzeros_dev, (_Float16*)y_dev, scratch, M, K, N, wide_splits, row_tiles,
+                           (const _Float16*)residual_dev, swiglu, st))
+      return 1;
+    return wide_splits > 1 ? combine(scratch, (_Float16*)y_dev, M, N, wide_splits, (const _Float16*)residual_dev, swiglu, st) : 0;
+  }
+  const int block_rows = want_rows == 1 ? 32 : want_rows == 2 ? (M <= 32 ? 32 : BM) : choose_block_rows(M, K, N, compute_units);
+  for (int m0 = 0; m0 < M; m0 += block_rows * kMaxRowBlocks) {
+    const int rows = M - m0 < block_rows * kMaxRowBlocks ? M - m0 : block_rows * kMaxRowBlocks;
+    const int m_blocks = (rows + block_rows - 1) / block_rows;
+    int splits = choose_splits(rows, N, K, scratch_bytes, compute_units / m_blocks);
+    if (k_splits > 0) {           // the caller's choice, within what the kernel and the scratch space take
+      const int cap = (int)(scratch_bytes / ((size_t)rows * N * sizeof(float)));
+      splits = k_splits > G ? G : k_splits;
+      if (splits > cap) splits = cap < 1 ? 1 : cap;
+    }
+    const _Float16* xs = (const _Float16*)x_dev + (size_t)m0 * K;
+    _Float16* ys = (_Float16*)y_dev + (size_t)m0 * n_out;
+    const _Float16* rs = residual_dev ? (const _Float16*)residual_dev + (size_t)m0 * N : nullptr;
+    const dim3 grid((unsigned)((col_tiles * splits + 7) / 8 * 8 * m_blocks));
+    const auto kernel = block_rows == 32 ? (swiglu ? gemm_w4a16_kernel<1, true> : gemm_w4a16_kernel<1, false>)
+                                         : (swiglu ? gemm_w4a16_kernel<2, true> : gemm_w4a16_kernel<2, false>);
+    kernel<<<grid, kThreads, kLdsBytes, st>>>(xs, (const unsigned char*)qweight_dev, (const _Float16*)scales_dev,
+                                              (const unsigned char*)qzeros_dev, ys, scratch, rows, K, N, splits, col_tiles, m_blocks,
+                                              kMagic, rs);
+    ART_LAUNCH_CHECK();
+    if (splits > 1 && combine(scratch, ys, rows, N, splits, rs, swiglu, st)) return 1;
+  }
   return 0;
 }
 
@@ -396,75 +490,11 @@ extern "C" int art_gemm_w4a16_tuned(const void* x_dev, const void* qweight_dev, 
 
 extern "C" int art_gemm_w4a16_residual(const void* x_dev, const void* qweight_dev, const void* scales_dev, const void* qzeros_dev,
                                        void* y_dev, const void* residual_dev, int M, int K, int N, int k_splits, void* stream) {
-  const int want_rows = k_splits >> 8;              // 0: library's choice; else rows of a block / 32
-  ART_REQUIRE(k_splits >= 0 && (want_rows <= 2 || want_rows == 4 || want_rows == 8),
-              "art_gemm_w4a16: k_splits must be 0 (library's choice) or 1..255, plus 256 x the rows-per-block code 1, 2, 4 or 8 (got %d)", k_splits);
-  ART_REQUIRE(((uintptr_t)residual_dev % 8) == 0, "art_gemm_w4a16: the residual must be 8-byte aligned");
-  ART_REQUIRE(!art::overlaps(x_dev, (size_t)M * K * 2, y_dev, (size_t)M * N * 2), "art_gemm_w4a16: y must not overlap x");
-  ART_REQUIRE(x_dev && qweight_dev && scales_dev && qzeros_dev && y_dev, "art_gemm_w4a16: null pointer");
-  ART_REQUIRE(M >= 1, "art_gemm_w4a16: M must be positive (got %d)", M);
-  ART_REQUIRE(K > 0 && N > 0 && K % 128 == 0 && N % 16 == 0, "art_gemm_w4a16: need K %% 128 == 0 and N %% 16 == 0 (K=%d N=%d)", K, N);
-  ART_REQUIRE(((uintptr_t)qweight_dev % 16) == 0 && ((uintptr_t)x_dev % 16) == 0 && ((uintptr_t)qzeros_dev % 8) == 0 &&
-                  ((uintptr_t)y_dev % 8) == 0 && ((uintptr_t)scales_dev % 4) == 0,
-              "art_gemm_w4a16: x and qweight must be 16-byte aligned, qzeros and y 8-byte aligned, scales 4-byte aligned");
-  art::Workspace* wsp = art::workspace((hipStream_t)stream);
-  if (!wsp) return 1;
-  art::Workspace& ws = *wsp;
-  float* scratch = reinterpret_cast<float*>((char*)ws.base + art::kScratchOffset);
-  const size_t scratch_bytes = ws.bytes - art::kScratchOffset;
-  static int compute_units = 0;
-  if (compute_units == 0) {
-    int dev = 0;
-    ART_HIP(hipGetDevice(&dev));
-    ART_HIP(hipDeviceGetAttribute(&compute_units, hipDeviceAttributeMultiprocessorCount, dev));
-    ART_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_w4a16_kernel<1>), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)kLdsBytes));
-    ART_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_w4a16_kernel<2>), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)kLdsBytes));
-  }
-  const Magic mg{0x000F000Fu, 0x00F000F0u, 0x64006400u, 0x54005400u};
-  hipStream_t st = (hipStream_t)stream;
-  const int G = K / GK, col_tiles = (N + BN - 1) / BN;
-  // Up to kMaxRowBlocks row blocks of this file's kernel go into one launch; longer batches take several passes over the
-  // weights.  The caller's choice of kernel and rows per block arrives in the upper bits of k_splits.
-  k_splits &= 0xff;
-  int row_tiles = want_rows >= 4 ? want_rows : 0, wide_splits = k_splits;
-  if (want_rows == 0 && k_splits == 0) row_tiles = choose_wide(M, K, N, scratch_bytes, compute_units, &wide_splits);
-  if (row_tiles) {
-    const size_t per_split = (size_t)M * N * sizeof(float);
-    if (wide_splits > G) wide_splits = G;
-    if ((size_t)wide_splits * per_split > scratch_bytes) wide_splits = (int)(scratch_bytes / per_split);
-    if (wide_splits < 1) wide_splits = 1;
-    if (art::w4::gemm_wide((const _Float16*)x_dev, (const unsigned char*)qweight_dev, (const _Float16*)scales_dev,
-                           (const unsigned char*)qzeros_dev, (_Float16*)y_dev, scratch, M, K, N, wide_splits, row_tiles,
-                           (const _Float16*)residual_dev, st))
-      return 1;
-    return wide_splits > 1 ? combine(scratch, (_Float16*)y_dev, M, N, wide_splits, (const _Float16*)residual_dev, st) : 0;
-  }
-  const int block_rows = want_rows == 1 ? 32 : want_rows == 2 ? (M <= 32 ? 32 : BM) : choose_block_rows(M, K, N, compute_units);
-  for (int m0 = 0; m0 < M; m0 += block_rows * kMaxRowBlocks) {
-    const int rows = M - m0 < block_rows * kMaxRowBlocks ? M - m0 : block_rows * kMaxRowBlocks;
-    const int m_blocks = (rows + block_rows - 1) / block_rows;
-    int splits = choose_splits(rows, N, K, scratch_bytes, compute_units / m_blocks);
-    if (k_splits > 0) {           // the caller's choice, within what the kernel and the scratch space take
-      const int cap = (int)(scratch_bytes / ((size_t)rows * N * sizeof(float)));
-      splits = k_splits > G ? G : k_splits;
-      if (splits > cap) splits = cap < 1 ? 1 : cap;
-    }
-    const _Float16* xs = (const _Float16*)x_dev + (size_t)m0 * K;
-    _Float16* ys = (_Float16*)y_dev + (size_t)m0 * N;
-    const _Float16* rs = residual_dev ? (const _Float16*)residual_dev + (size_t)m0 * N : nullptr;
-    const dim3 grid((unsigned)((col_tiles * splits + 7) / 8 * 8 * m_blocks));
-    if (block_rows == 32)
-      gemm_w4a16_kernel<1><<<grid, kThreads, kLdsBytes, st>>>(xs, (const unsigned char*)qweight_dev, (const _Float16*)scales_dev,
-                                                         (const unsigned char*)qzeros_dev, ys, scratch, rows, K, N, splits,
-                                                         col_tiles, m_blocks, mg, rs);
-    else
-      gemm_w4a16_kernel<2><<<grid, kThreads, kLdsBytes, st>>>(xs, (const unsigned char*)qweight_dev, (const _Float16*)scales_dev,
-                                                         (const unsigned char*)qzeros_dev, ys, scratch, rows, K, N, splits,
-                                                         col_tiles, m_blocks, mg, rs);
-    ART_LAUNCH_CHECK();
-    if (splits > 1 && combine(scratch, ys, rows, N, splits, rs, st)) return 1;
-  }
-  return 0;
+  return run(x_dev, qweight_dev, scales_dev, qzeros_dev, y_dev, residual_dev, M, K, N, k_splits, false, stream);
+}
+
+extern "C" int art_gemm_w4a16_swiglu(const void* x_dev, const void* qweight_dev, const void* scales_dev, const void* qzeros_dev,
+                                     void* y_dev, int M, int K, int N, int k_splits, void* stream) {
+  ART_REQUIRE(N % 32 == 0, "art_gemm_w4a16_swiglu: the gate and up halves must be multiples of 16 columns (N=%d)", N);
+  return run(x_dev, qweight_dev, scales_dev, qzeros_dev, y_dev, nullptr, M, K, N, k_splits, true, stream);
 }

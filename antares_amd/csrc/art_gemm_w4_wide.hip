@@ -52,7 +52,9 @@ __device__ __forceinline__ void load_lds_x1(const void* base, unsigned int off, 
                : "=&s"(keep) : "v"(off), "s"(base), "s"(lds_dst));
 }
 
-template <int MT>
+// SWIGLU: the matrix is gate | up (N / 2 columns each); a block owns 128 gate columns and the matching 128 up columns and
+// stores y[m, n] = fp16(silu(fp16(gate)) * fp16(up)), N / 2 columns.
+template <int MT, bool SWIGLU>
 __global__ __launch_bounds__(kThreads, MT == 8 ? 1 : 2) void gemm_w4a16_wide_kernel(
     const _Float16* __restrict__ x, const unsigned char* __restrict__ qweight, const _Float16* __restrict__ scales,
     const unsigned char* __restrict__ qzeros, _Float16* y, float* __restrict__ partial, int M, int K, int N, int splits,
@@ -66,7 +68,8 @@ __global__ __launch_bounds__(kThreads, MT == 8 ? 1 : 2) void gemm_w4a16_wide_ker
   const int m_block = (int)(blockIdx.x % (8 * m_blocks)) / 8;
   if (unit >= col_tiles * splits) return;
   const int split = unit / col_tiles;
-  const int n0 = (unit % col_tiles) * BN, m0 = m_block * BM;
+  const TileColumns<SWIGLU> cols{(unit % col_tiles) * (SWIGLU ? BN / 2 : BN), N};
+  const int m0 = m_block * BM;
   const int G = K / 128;
   const int g_begin = (int)((long long)G * split / splits), g_end = (int)((long long)G * (split + 1) / splits);
   const int steps = 2 * (g_end - g_begin);          // splits <= G: at least two
@@ -77,8 +80,7 @@ __global__ __launch_bounds__(kThreads, MT == 8 ? 1 : 2) void gemm_w4a16_wide_ker
 #pragma unroll
   for (int u = 0; u < 2; ++u) {
     const int r = 4 * (wave + 4 * u) + (lane >> 4);
-    const int col = n0 + ((lane & 15) ^ (r & 7)) * 16;
-    woff[u] = (unsigned int)r * N + (col < N ? col : 0);
+    woff[u] = (unsigned int)r * N + cols.safe(((lane & 15) ^ (r & 7)) * 16);
   }
 #pragma unroll
   for (int u = 0; u < MT; ++u) {
@@ -90,18 +92,23 @@ __global__ __launch_bounds__(kThreads, MT == 8 ? 1 : 2) void gemm_w4a16_wide_ker
   // scales and zero points share one load: wavefronts 0 and 1 fetch the scales of columns 2 d, 2 d + 1, half of
   // wavefront 2 the zero points of columns 8 (d - 128) .. + 7, the others repeat the first scales
   const bool is_zero = tid >= 128 && tid < 160;
-  const int qcol = tid < 128 ? n0 + 2 * tid : n0 + 8 * (tid - 128);
-  qoff = is_zero ? (unsigned int)((qcol < N ? qcol : 0) >> 1) : (tid < 128 ? 2u * (qcol < N ? qcol : 0) : 0u);
+  qoff = is_zero ? (unsigned int)cols.safe(8 * (tid - 128)) >> 1 : (tid < 128 ? 2u * cols.safe(2 * tid) : 0u);
   const unsigned char* qbase = wave == 2 ? qzeros + (size_t)g_begin * (N / 2) : reinterpret_cast<const unsigned char*>(scales + (size_t)g_begin * N);
   const unsigned int qstep = wave == 2 ? N / 2 : 2 * N;
 
   // Load j of ring slot `slot`: 0, 1 packed weights, 2 scales and zero points, 3 .. MT + 2 x.  The weights run one
   // stage ahead of x: slot of stage i holds x of stage i and the weights of stage i + 1.
+  // (the bases are the same for every lane; said so explicitly, they stay in scalar registers whatever surrounds the loop)
+  auto uniform = [](const void* p) {
+    const unsigned long long v = (unsigned long long)p;
+    return (const void*)((unsigned long long)(unsigned int)__builtin_amdgcn_readfirstlane((int)v) |
+                         (unsigned long long)(unsigned int)__builtin_amdgcn_readfirstlane((int)(v >> 32)) << 32);
+  };
   auto issue = [&](unsigned int slot, int j) {
     const unsigned int st = lds0 + slot;
-    if (j < 2) load_lds_x4(wbase, woff[j], st + (wave + 4 * j) * 1024);
-    else if (j == 2) load_lds_x1(qbase, qoff, st + W_BYTES + wave * 256);
-    else load_lds_x4(xbase, xoff[j - 3], st + W_BYTES + Q_BYTES + (wave + 4 * (j - 3)) * 1024);
+    if (j < 2) load_lds_x4(uniform(wbase), woff[j], st + (wave + 4 * j) * 1024);
+    else if (j == 2) load_lds_x1(uniform(qbase), qoff, st + W_BYTES + wave * 256);
+    else load_lds_x4(uniform(xbase), xoff[j - 3], st + W_BYTES + Q_BYTES + (wave + 4 * (j - 3)) * 1024);
   };
   // The bases move on behind the loads of a stage.  At the end they stay at the last one: it is fetched again, into
   // slots that nobody reads, and the loop needs neither branches nor a varying count of loads.
@@ -153,7 +160,7 @@ __global__ __launch_bounds__(kThreads, MT == 8 ? 1 : 2) void gemm_w4a16_wide_ker
   };
   auto decode_scales = [&](int ct) {
     const unsigned int z = (raw_z[ct] >> ((colpos[ct] & 1) * 4)) & 15u;
-    const _Float16 s = (n0 + colpos[ct] < N) ? raw_s[ct] : (_Float16)0.f;
+    const _Float16 s = cols.inside(colpos[ct]) ? raw_s[ct] : (_Float16)0.f;
     s2[ct] = h2{s, s};
     zz2[ct] = as_h2(z | (z << 16) | mg.bias_lo);
   };
@@ -271,7 +278,7 @@ __global__ __launch_bounds__(kThreads, MT == 8 ? 1 : 2) void gemm_w4a16_wide_ker
         const int row = m0 + t * 32 + (r >> 2) * 8 + h * 4 + (r & 3);
 #pragma unroll
         for (int ct = 0; ct < 2; ++ct)
-          if (row < M && n0 + colpos[ct] < N) partial[((size_t)split * M + row) * N + n0 + colpos[ct]] = acc[t][ct][r];
+          if (row < M && cols.inside(colpos[ct])) partial[((size_t)split * M + row) * N + cols.at(colpos[ct])] = acc[t][ct][r];
       }
     return;
   }
@@ -287,14 +294,26 @@ __global__ __launch_bounds__(kThreads, MT == 8 ? 1 : 2) void gemm_w4a16_wide_ker
         for (int r = 0; r < 16; ++r)
           cs[(t * 32 + (r >> 2) * 8 + h * 4 + (r & 3)) * C_LD + colpos[ct]] = (_Float16)acc[4 * p + t][ct][r];
     __syncthreads();
+    if constexpr (SWIGLU) {
+#pragma unroll 1
+      for (int c = tid; c < 128 * (BN / 16); c += kThreads) {
+        const int row = c >> 4, col = (c & 15) * 8, grow = m0 + p * 128 + row;
+        if (grow >= M || !cols.inside(col)) continue;
+        const h8 g = *reinterpret_cast<const h8*>(cs + row * C_LD + col), u = *reinterpret_cast<const h8*>(cs + row * C_LD + 128 + col);
+        _Float16* dst = y + (size_t)grow * (N / 2) + cols.at(col);      // y is 8-byte aligned
+        *reinterpret_cast<h4*>(dst) = swiglu4(h4{g[0], g[1], g[2], g[3]}, h4{u[0], u[1], u[2], u[3]});
+        *reinterpret_cast<h4*>(dst + 4) = swiglu4(h4{g[4], g[5], g[6], g[7]}, h4{u[4], u[5], u[6], u[7]});
+      }
+      continue;
+    }
 #pragma unroll 4
     for (int c = tid; c < 128 * (BN / 8); c += kThreads) {
       const int row = c >> 5, col = (c & 31) * 8, grow = m0 + p * 128 + row;
-      if (grow >= M || n0 + col >= N) continue;
+      if (grow >= M || !cols.inside(col)) continue;
+      const size_t at = (size_t)grow * N + cols.at(col);
       h8 o = *reinterpret_cast<const h8*>(cs + row * C_LD + col);
       if (residual) {                               // y = fp16(fp16(product) + residual)
-        const h4 r0 = *reinterpret_cast<const h4*>(residual + (size_t)grow * N + n0 + col);
-        const h4 r1 = *reinterpret_cast<const h4*>(residual + (size_t)grow * N + n0 + col + 4);
+        const h4 r0 = *reinterpret_cast<const h4*>(residual + at), r1 = *reinterpret_cast<const h4*>(residual + at + 4);
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
           o[k] = (_Float16)((float)o[k] + (float)r0[k]);
@@ -302,23 +321,23 @@ __global__ __launch_bounds__(kThreads, MT == 8 ? 1 : 2) void gemm_w4a16_wide_ker
         }
       }
       // y is 8-byte aligned
-      *reinterpret_cast<h4*>(y + (size_t)grow * N + n0 + col) = h4{o[0], o[1], o[2], o[3]};
-      *reinterpret_cast<h4*>(y + (size_t)grow * N + n0 + col + 4) = h4{o[4], o[5], o[6], o[7]};
+      *reinterpret_cast<h4*>(y + at) = h4{o[0], o[1], o[2], o[3]};
+      *reinterpret_cast<h4*>(y + at + 4) = h4{o[4], o[5], o[6], o[7]};
     }
   }
 }
 
-template <int MT>
+template <int MT, bool SWIGLU>
 int launch(const _Float16* x, const unsigned char* qweight, const _Float16* scales, const unsigned char* qzeros, _Float16* y,
            float* partial, int M, int K, int N, int splits, const _Float16* residual, hipStream_t stream) {
   static bool configured = false;
   if (!configured) {
-    ART_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_w4a16_wide_kernel<MT>), hipFuncAttributeMaxDynamicSharedMemorySize,
+    ART_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_w4a16_wide_kernel<MT, SWIGLU>), hipFuncAttributeMaxDynamicSharedMemorySize,
                                 (int)lds_bytes(MT)));
     configured = true;
   }
-  const int col_tiles = (N + BN - 1) / BN, m_blocks = (M + 32 * MT - 1) / (32 * MT);
-  gemm_w4a16_wide_kernel<MT><<<dim3((unsigned)((col_tiles * splits + 7) / 8 * 8 * m_blocks)), kThreads, lds_bytes(MT), stream>>>(
+  const int col_tiles = tile_count(N, SWIGLU), m_blocks = (M + 32 * MT - 1) / (32 * MT);
+  gemm_w4a16_wide_kernel<MT, SWIGLU><<<dim3((unsigned)((col_tiles * splits + 7) / 8 * 8 * m_blocks)), kThreads, lds_bytes(MT), stream>>>(
       x, qweight, scales, qzeros, y, partial, M, K, N, splits, col_tiles, m_blocks, kMagic, residual);
   ART_LAUNCH_CHECK();
   return 0;
@@ -327,7 +346,10 @@ int launch(const _Float16* x, const unsigned char* qweight, const _Float16* scal
 }  // namespace
 
 int art::w4::gemm_wide(const _Float16* x, const unsigned char* qweight, const _Float16* scales, const unsigned char* qzeros, _Float16* y,
-                       float* partial, int M, int K, int N, int splits, int row_tiles, const _Float16* residual, hipStream_t stream) {
-  return row_tiles == 8 ? launch<8>(x, qweight, scales, qzeros, y, partial, M, K, N, splits, residual, stream)
-                        : launch<4>(x, qweight, scales, qzeros, y, partial, M, K, N, splits, residual, stream);
+                       float* partial, int M, int K, int N, int splits, int row_tiles, const _Float16* residual, bool swiglu, hipStream_t stream) {
+  if (swiglu)
+    return row_tiles == 8 ? launch<8, true>(x, qweight, scales, qzeros, y, partial, M, K, N, splits, nullptr, stream)
+                          : launch<4, true>(x, qweight, scales, qzeros, y, partial, M, K, N, splits, nullptr, stream);
+  return row_tiles == 8 ? launch<8, false>(x, qweight, scales, qzeros, y, partial, M, K, N, splits, residual, stream)
+                        : launch<4, false>(x, qweight, scales, qzeros, y, partial, M, K, N, splits, residual, stream);
 }

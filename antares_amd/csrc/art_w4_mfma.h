@@ -37,10 +37,33 @@ __device__ __forceinline__ h8 permute_k(u32x4 v) {
 
 constexpr Magic kMagic{0x000F000Fu, 0x00F000F0u, 0x64006400u, 0x54005400u};
 
+// The 256 columns of a block: neighbours, or (SWIGLU, the matrix is gate | up) 128 of the gate half and the matching 128 of
+// the up half.  N % 16 == 0 (SWIGLU: N % 32), so a piece of 16 columns is inside or outside as a whole.
+template <bool SWIGLU>
+struct TileColumns {
+  int n0, N;
+  __device__ __forceinline__ int at(int pos) const { return SWIGLU && pos >= 128 ? N / 2 + n0 + pos - 128 : n0 + pos; }
+  __device__ __forceinline__ bool inside(int pos) const { return SWIGLU ? n0 + (pos & 127) < N / 2 : n0 + pos < N; }
+  __device__ __forceinline__ int safe(int pos) const { return inside(pos) ? at(pos) : 0; }
+};
+inline int tile_count(int N, bool swiglu) { return swiglu ? (N / 2 + 127) / 128 : (N + 255) / 256; }
+
+// fp16(silu(gate) * up) of fp16 operands in fp32, as the decode step's GEMV and the sample's torch line round it.
+__device__ __forceinline__ h4 swiglu4(h4 g, h4 u) {
+  h4 o;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const float gf = (float)g[k];
+    o[k] = (_Float16)(gf / (1.0f + expf(0.0f - gf)) * (float)u[k]);
+  }
+  return o;
+}
+
 // Large batches (art_gemm_w4_wide.hip): one launch over blocks of 32 row_tiles rows x 256 columns, K cut into `splits`;
-// with splits > 1 the fp32 tiles go to `partial` [splits][M][N].  row_tiles is 4 or 8.
+// with splits > 1 the fp32 tiles go to `partial` [splits][M][N].  row_tiles is 4 or 8.  swiglu: y[M, N/2] from
+// gate | up, no residual.
 int gemm_wide(const _Float16* x, const unsigned char* qweight, const _Float16* scales, const unsigned char* qzeros, _Float16* y,
-              float* partial, int M, int K, int N, int splits, int row_tiles, const _Float16* residual, hipStream_t stream);
+              float* partial, int M, int K, int N, int splits, int row_tiles, const _Float16* residual, bool swiglu, hipStream_t stream);
 
 }  // namespace w4
 }  // namespace art

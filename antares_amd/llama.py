@@ -283,14 +283,10 @@ class LlamaInt4Decoder:
             # there is one set of these per prompt length
             return ExportedOp(ir, list(inputs), name=name)
         cfg = self.cfg
-        d, H, D, F, V = cfg.dim, cfg.n_heads, cfg.head_dim, cfg.ffn, cfg.vocab
-        f32 = '.to(`float32`)'
+        d, V = cfg.dim, cfg.vocab
         ops = {
             'embed': program(ir='emb[T, D] = table[tok[T], D]', inputs=[f'table=float16[{V}, {d}]', f'tok=int32[{T}]'],
                               name=f'prefill_embed_{T}'),
-            'silu_mul': program(
-                ir=f'hid[T, N] = (gu[T, N]{f32} / (1.0 + (0.0 - gu[T, N]{f32}).call(`exp`)) * gu[T, {F} + N]{f32}).to(`float16`) where N in {F}',
-                inputs=[f'gu=float16[{T}, {2 * F}]'], name=f'prefill_silu_mul_{T}'),
         }
         self._prefill_cache[T] = ops
         return ops
@@ -339,7 +335,7 @@ class LlamaInt4Decoder:
         f16 = dict(dtype=torch.float16, device=self.dev)
         x = ops['embed'](self.w['embed'], tokens.view(T))
         qkv = torch.empty(T, 3 * d, **f16)
-        gu = torch.empty(T, 2 * F, **f16)
+        hid = torch.empty(T, F, **f16)
         qr = torch.empty(T, H, D, **f16)
 
         def linear(inp, lin, out):
@@ -359,8 +355,8 @@ class LlamaInt4Decoder:
                                                        self.val_cache[l].view(cfg.max_seq, H, D), self.att_f)
             gemm_res(att.view(T, d), lw['o'], x)
             xb = rms(x, lw['ffn_norm'])
-            linear(xb, lw['gate_up'], gu)
-            hid = ops['silu_mul'](gu)
+            gu = lw['gate_up']
+            self.autort.ops.gemm_w4a16_swiglu(xb, gu['qweight'], gu['scales'], gu['qzeros'], hid)
             gemm_res(hid, lw['down'], x)
         self.x.copy_(x[T - 1])
         self.pos.fill_(T - 1)

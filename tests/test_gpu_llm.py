@@ -45,6 +45,26 @@ def test_rmsnorm_f32_like_the_sample(autort, n):
     assert np.allclose(out2.cpu().numpy(), hot_ops.rmsnorm(x.numpy(), None, w.numpy()), **FP32_TOL)
 
 
+# rows one vector long, not a whole number of vectors, as long as registers hold and longer; a row off the 16-byte grid
+@pytest.mark.parametrize('rows,n,offset', [(1, 8, 0), (3, 1000, 0), (5, 1001, 0), (2, 2056, 0), (130, 4096, 0), (2, 8192, 0), (2, 8200, 0), (1, 4096, 1)])
+def test_rmsnorm_rows_of_any_length(autort, rows, n, offset):
+    from oracle import hot_ops
+    note(f'rmsnorm {rows} x {n} offset {offset}')
+    dev = autort.device()
+    for xdt, odt in ((torch.float16, torch.float16), (torch.float32, torch.float32), (torch.float16, torch.float32)):
+        x = torch.randn(rows * n + offset, generator=gen(n)).to(xdt)[offset:].view(rows, n)
+        w = (1 + 0.1 * torch.randn(n, generator=gen(2))).to(xdt)
+        op = autort.ops.rmsnorm_f16 if odt == torch.float16 else autort.ops.rmsnorm_f32
+        xd = torch.zeros(rows * n + offset, dtype=xdt, device=dev)[offset:].view(rows, n).copy_(x)
+        got = op(xd, None, w.to(dev)).float().cpu().numpy()
+        vsum = (xd.float() ** 2).sum(1)
+        given = op(xd, vsum, w.to(dev)).float().cpu().numpy()
+        for r in range(rows):
+            want = hot_ops.rmsnorm(x[r].numpy(), None, w.numpy(), out_dtype=np.float16 if odt == torch.float16 else np.float32).astype(np.float32)
+            tol = FP16_TOL if odt == torch.float16 else FP32_TOL
+            assert np.allclose(got[r], want, **tol) and np.allclose(given[r], want, **tol)
+
+
 def test_rmsnorm_f16_variants(autort):
     from oracle import hot_ops
     note('rmsnorm_f16: fp32 x + fp16 w (sample 04), fp16 x + fp16 w')
@@ -320,6 +340,29 @@ def test_causal_attention_over_a_prompt_against_the_oracle(T, H):
     sc = sc.masked_fill(torch.triu(torch.ones(T, T, dtype=torch.bool), 1), float('-inf'))
     exact = torch.einsum('hts,shd->thd', torch.softmax(sc, -1), vd[:T]).numpy()
     assert np.allclose(out.astype(np.float64), exact, rtol=1e-2, atol=1e-2)
+
+
+# the 16-byte form at its smallest and largest head, then heads and addresses it leaves to the one-pair-per-lane form
+@pytest.mark.parametrize('H,D,offset', [(1, 16, 0), (3, 256, 0), (33, 128, 0), (2, 72, 0), (2, 272, 0), (2, 128, 1)])
+def test_rope_qkv_store_rows_of_any_head_size(H, D, offset):
+    import autort
+    from oracle import hot_ops
+    dev = autort.device()
+    T, S, first = 3, 8, 2
+    note(f'rope_qkv_store_rows H={H} D={D} offset={offset}')
+    g = torch.Generator().manual_seed(D)
+    qkv = torch.randn(T, 3 * H * D, generator=g).half()
+    inv = (1.0 / (10000 ** (torch.arange(0, D, 2).float() / D))).half()
+    inv_freq = torch.cat([inv, inv])
+    qd = torch.zeros(T * 3 * H * D + offset, dtype=torch.float16, device=dev)[offset:].view(T, -1).copy_(qkv)
+    kd, vd = torch.zeros(S, H * D, dtype=torch.float16, device=dev), torch.zeros(S, H * D, dtype=torch.float16, device=dev)
+    q_out = torch.zeros(T, H, D, dtype=torch.float16, device=dev)
+    autort.ops.rope_qkv_store_rows_f16(qd, inv_freq.to(dev), q_out, kd, vd, extra=[first])
+    for t in range(T):
+        q, k, v = (qkv[t, i * H * D:(i + 1) * H * D].numpy() for i in range(3))
+        assert np.allclose(q_out[t].float().cpu().numpy(), hot_ops.rotary(q.reshape(H, 2, D // 2), inv_freq.numpy(), first + t).astype(np.float32).reshape(H, D), **FP16_TOL)
+        assert np.allclose(kd[first + t].float().cpu().numpy(), hot_ops.rotary(k.reshape(H, 2, D // 2), inv_freq.numpy(), first + t).astype(np.float32).reshape(-1), **FP16_TOL)
+        assert np.array_equal(vd[first + t].cpu().numpy(), v)
 
 
 @pytest.mark.usefixtures('oracle_built')

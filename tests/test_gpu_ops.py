@@ -548,6 +548,30 @@ def test_w4a16_gemm_over_blocks_of_128_and_256_rows(autort, M, K, N):
                 assert np.allclose(d[4].float().cpu().numpy(), want, **FP16_TOL)
 
 
+# both kernels, with and without K-splits (code 0: the library's choice); halves of 16 columns and past a tile of 128
+@pytest.mark.parametrize('M,K,F', [(5, 128, 16), (33, 512, 144), (64, 1024, 112), (65, 256, 128), (130, 2048, 272), (257, 640, 400)])
+def test_w4a16_gemm_with_swiglu_behind_it(autort, M, K, F):
+    from ctypes import c_void_p
+    from antares_amd.runtime import capi
+    from oracle import hot_ops
+    dev = autort.device()
+    p = workloads.w4_problem(K + F + M, M, K, 2 * F)
+    p['scales'] = p['scales'] * 0.1
+    prod = hot_ops.gemm_w4a16(p['x'].numpy(), p['qweight'].numpy(), p['scales'].numpy(), p['qzeros'].numpy()).astype(np.float32)
+    gate, up = prod[:, :F], prod[:, F:]
+    want = gate / (1 + np.exp(-gate)) * up
+    d = [p[k].to(dev) for k in ('x', 'qweight', 'scales', 'qzeros')]
+    for code in (0, 256 + 1, 256 + 2, 512 + 1, 512 + 3, 1024 + 1, 1024 + 4, 2048 + 1, 2048 + 2):
+        note(f'w4a16 gemm + swiglu M={M} K={K} F={F} code {code}')
+        out = torch.full((M, F), float('nan'), dtype=torch.float16, device=dev)
+        capi.check(capi.lib().art_gemm_w4a16_swiglu(*(c_void_p(t.data_ptr()) for t in d), c_void_p(out.data_ptr()), M, K, 2 * F, code,
+                                                    c_void_p(torch.cuda.current_stream().cuda_stream)))
+        torch.cuda.synchronize()
+        assert np.allclose(out.float().cpu().numpy(), want, **FP16_TOL)
+    got = autort.ops.gemm_w4a16_swiglu(*d)
+    assert got.shape == (M, F) and np.allclose(got.float().cpu().numpy(), want, **FP16_TOL)
+
+
 ROW_VECTOR_CASES = [
     # program, inputs, shapes of the inputs, does the row-vector variant apply to these extents
     ('output0[N, C] = input0[N, C] + input1[C]', ['input0=float32[N:300, C:1024]', 'input1=float32[C:1024]'], [(300, 1024), (1024,)], True),
