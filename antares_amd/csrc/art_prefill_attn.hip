@@ -7,8 +7,13 @@
 // softmax times V) that the reference's tiled schedule would produce for a prompt
 // (backends/c-rocm/schedule/standard/algo_tiling.py:35-98).
 //
-// One wavefront per (head, tile of 32 queries); it walks the key tiles 0..its own, so nothing is computed above the
-// diagonal and no block barrier exists.  Everything is kept transposed so that a lane owns ONE query:
+// One block of four wavefronts per (head, tile of 32 queries).  The key tiles 0 .. the block's own are dealt out to the
+// wavefronts in turn, each keeps an online softmax of its share, and the four states are merged through LDS at the end:
+// nothing is computed above the diagonal, no barrier exists in the loop, and the longest chain of tiles - which bounds the
+// launch, 1.6 us a tile with one wavefront per SIMD - is a quarter of the tiles.  1003 tokens of 32 heads: 52 us with one
+// wavefront for all of them, 63 with four while the blocks of a head were neighbours (every XCD read all keys and values
+// past its L2), 28 with a head on one XCD; 128 tokens: 8.1 and 6.1 us.  Everything is kept transposed so that a lane owns
+// ONE query:
 //   * S^T = K Q^T on v_mfma_f32_32x32x16_f16: A = a K tile as it lies in the cache (32 rows of 128 dims, staged in LDS
 //     with coalesced 16-byte loads, read back as 16-byte rows), B = the lane's query row from registers.  The 32 x 32
 //     result has query lane % 32 in every lane, 16 keys per lane: the running maximum and sum of the online softmax
@@ -16,7 +21,8 @@
 //   * O^T += V^T P^T: the probabilities go from the accumulator layout straight into the B operand (the order of
 //     the summed index is free as long as both operands agree), V^T comes out of the row-major V tile through the
 //     transposing LDS read ds_read_b64_tr_b16, with the row quadruples chosen to match that order.
-//   * the rescaling by e^(m_old - m_new) is one multiplication per accumulator register.
+//   * the rescaling by 2^(m_old - m_new) is one multiplication per accumulator register, skipped where no maximum grew;
+//     exponentials are of base 2, log2(e) being folded into the scale; only the diagonal tile is masked.
 #include "art_common.h"
 
 namespace {
@@ -29,8 +35,10 @@ typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
 
 constexpr int D = 128;                 // head dimension
-constexpr int QT = 32, KT = 32;        // queries per wavefront, keys per step
+constexpr int QT = 32, KT = 32;        // queries per block, keys per step
+constexpr int kWaves = 4;
 constexpr int K_LD = D + 8;            // halves per K row in LDS (272 bytes)
+constexpr int O_LD = D + 4;            // floats per output row of the merge
 constexpr int V_LD = D + 32;           // halves per V row in LDS (320 bytes: the four rows of a transposing read fall on disjoint banks)
 
 __device__ __forceinline__ float max_with_lane_xor_32(float v) {
@@ -45,18 +53,23 @@ __device__ __forceinline__ float sum_with_lane_xor_32(float v) {
 }
 
 // q: [T, heads, 128]; k, v: rows of kv_stride halves, row s holding [heads, 128]; out: [T, heads, 128]
-__global__ __launch_bounds__(64) void prefill_attention_kernel(const _Float16* __restrict__ q, const _Float16* __restrict__ k,
+__global__ __launch_bounds__(64 * kWaves, 2) void prefill_attention_kernel(const _Float16* __restrict__ q, const _Float16* __restrict__ k,
                                                                 const _Float16* __restrict__ v, _Float16* __restrict__ out, int T,
                                                                 int heads, long long kv_stride, const float* __restrict__ att_f,
                                                                 int q_tiles) {
-  __shared__ __align__(16) _Float16 Ks[KT * K_LD];
-  __shared__ __align__(16) _Float16 Vs[KT * V_LD];
-  const int lane = threadIdx.x, half = lane >> 5, qi = lane & 31;
-  // the longest walks (last query tiles) are handed out first
-  const int qt = q_tiles - 1 - (int)(blockIdx.x % q_tiles), h = blockIdx.x / q_tiles;
+  constexpr int TILE = KT * (K_LD + V_LD);           // halves of a wavefront's K and V tile
+  static_assert(TILE * 2 >= QT * O_LD * 4, "a wavefront's outputs take the place of its tiles");
+  __shared__ __align__(16) _Float16 tiles[kWaves][TILE];
+  __shared__ float s_m[kWaves][QT], s_l[kWaves][QT];
+  const int lane = threadIdx.x & 63, half = lane >> 5, qi = lane & 31, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  _Float16* const Ks = tiles[wave];
+  _Float16* const Vs = Ks + KT * K_LD;
+  // The longest walks (last query tiles) are handed out first; blocks of one head are `heads` apart, i.e. on one XCD for
+  // a multiple of 8 heads, whose L2 then holds the keys and values of its heads.
+  const int qt = q_tiles - 1 - (int)(blockIdx.x / heads), h = blockIdx.x % heads;
   const int query = qt * QT + qi;
   const int qrow = query < T ? query : T - 1;                    // rows past T repeat the last one and are never stored
-  const float scale = att_f[0];
+  const float scale = att_f[0] * 1.44269504088896341f;            // scores in units of log2(e)
 
   // B operand of S^T = K Q^T: query lane % 32, dims 16 s + 8 half .. + 8 of step s
   h8 bq[D / 16];
@@ -77,7 +90,7 @@ __global__ __launch_bounds__(64) void prefill_attention_kernel(const _Float16* _
       vreg[i] = *reinterpret_cast<const u32x4*>(v + off);
     }
   };
-  load_tile(0);
+  if (wave <= qt) load_tile(wave);
 
   float m_run = -INFINITY, l_run = 0.f;
   f16v o[D / 32];
@@ -90,14 +103,14 @@ __global__ __launch_bounds__(64) void prefill_attention_kernel(const _Float16* _
   const int s16 = lane & 15;
   const int tr_row = s16 >> 2, tr_col = ((lane & 31) >> 4) * 16 + (s16 & 3) * 4;
 
-  for (int kt = 0; kt <= qt; ++kt) {
+  for (int kt = wave; kt <= qt; kt += kWaves) {
     // registers -> LDS (a wavefront's LDS operations execute in order: the reads of the previous tile are done)
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       *reinterpret_cast<u32x4*>(&Ks[(st_row + 4 * i) * K_LD + st_col]) = kreg[i];
       *reinterpret_cast<u32x4*>(&Vs[(st_row + 4 * i) * V_LD + st_col]) = vreg[i];
     }
-    if (kt < qt) load_tile(kt + 1);                              // next tile's loads fly during this tile's arithmetic
+    if (kt + kWaves <= qt) load_tile(kt + kWaves);                // next tile's loads fly during this tile's arithmetic
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
@@ -113,30 +126,38 @@ __global__ __launch_bounds__(64) void prefill_attention_kernel(const _Float16* _
     }
     // element r of the accumulator: key (r / 4) * 8 + 4 * half + r % 4 of the tile, query lane % 32
     float mx = -INFINITY;
+    if (kt == qt) {
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int key = kt * KT + (r >> 2) * 8 + 4 * half + (r & 3);
-      st[r] = key <= query ? st[r] * scale : -INFINITY;
-      mx = fmaxf(mx, st[r]);
+      for (int r = 0; r < 16; ++r) {
+        const int key = kt * KT + (r >> 2) * 8 + 4 * half + (r & 3);
+        st[r] = key <= query ? st[r] * scale : -INFINITY;
+      }
+    } else {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) st[r] *= scale;
     }
+#pragma unroll
+    for (int r = 0; r < 16; ++r) mx = fmaxf(mx, st[r]);
     mx = max_with_lane_xor_32(mx);
-    // key kt * 32 <= query for every query of this wavefront's tile, so the maximum is finite from the first tile on
+    // key kt * 32 <= query for every query of this block's tile, so the maximum is finite from the first tile on
     const float m_new = fmaxf(m_run, mx);
-    const float alpha = __expf(m_run - m_new);                   // first tile: e^(-inf) = 0
+    if (__builtin_amdgcn_ballot_w64(m_new > m_run) != 0) {       // first tile: 2^(-inf) = 0
+      const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
+      l_run *= alpha;
+#pragma unroll
+      for (int t = 0; t < D / 32; ++t)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o[t][r] *= alpha;
+    }
     float lsum = 0.f;
     float p[16];
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-      p[r] = __expf(st[r] - m_new);                              // masked: e^(-inf) = 0
+      p[r] = __builtin_amdgcn_exp2f(st[r] - m_new);              // masked: 2^(-inf) = 0
       lsum += p[r];
     }
-    lsum = sum_with_lane_xor_32(lsum);
-    l_run = l_run * alpha + lsum;
+    l_run += sum_with_lane_xor_32(lsum);
     m_run = m_new;
-#pragma unroll
-    for (int t = 0; t < D / 32; ++t)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) o[t][r] *= alpha;
 
     // ---- O^T += V^T P^T.  Step j sums over 16 keys; lane half `half` supplies, as elements 0..7, the keys
     // (2j) * 8 + 4 half + 0..3 and (2j + 1) * 8 + 4 half + 0..3 - exactly p[8j .. 8j + 7] - and V^T is read with the same
@@ -159,18 +180,34 @@ __global__ __launch_bounds__(64) void prefill_attention_kernel(const _Float16* _
     __builtin_amdgcn_wave_barrier();
   }
 
-  if (query >= T) return;
-  const float inv = 1.0f / l_run;
-  _Float16* op = out + ((size_t)query * heads + h) * D;
+  // ---- merge: every wavefront scales its outputs to the common maximum and leaves them in LDS, where its tiles were
+  if (half == 0) { s_m[wave][qi] = m_run; s_l[wave][qi] = l_run; }
+  __syncthreads();
+  float m_all = s_m[0][qi], l_all = 0.f;             // wavefront 0 has had tile 0: finite
+#pragma unroll
+  for (int w = 1; w < kWaves; ++w) m_all = fmaxf(m_all, s_m[w][qi]);
+#pragma unroll
+  for (int w = 0; w < kWaves; ++w) l_all += s_l[w][qi] * __builtin_amdgcn_exp2f(s_m[w][qi] - m_all);
+  const float mine = __builtin_amdgcn_exp2f(m_run - m_all) / l_all;
+  typedef float f32x4 __attribute__((ext_vector_type(4)));
+  float* const O = reinterpret_cast<float*>(tiles[wave]);
   // element r of tile t: dim t * 32 + (r / 4) * 8 + 4 * half + r % 4
 #pragma unroll
   for (int t = 0; t < D / 32; ++t)
 #pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      const h4 w = {(_Float16)(o[t][4 * g] * inv), (_Float16)(o[t][4 * g + 1] * inv), (_Float16)(o[t][4 * g + 2] * inv),
-                    (_Float16)(o[t][4 * g + 3] * inv)};
-      *reinterpret_cast<h4*>(op + t * 32 + g * 8 + 4 * half) = w;
-    }
+    for (int g = 0; g < 4; ++g)
+      *reinterpret_cast<f32x4*>(O + qi * O_LD + t * 32 + g * 8 + 4 * half) =
+          f32x4{o[t][4 * g] * mine, o[t][4 * g + 1] * mine, o[t][4 * g + 2] * mine, o[t][4 * g + 3] * mine};
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < QT * D / 4 / (64 * kWaves); ++i) {
+    const int e = threadIdx.x + i * 64 * kWaves, row = e >> 5, c = (e & 31) * 4;
+    if (qt * QT + row >= T) break;
+    f32x4 v = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) v += *reinterpret_cast<const f32x4*>(reinterpret_cast<const float*>(tiles[w]) + row * O_LD + c);
+    *reinterpret_cast<h4*>(out + ((size_t)(qt * QT + row) * heads + h) * D + c) = h4{(_Float16)v[0], (_Float16)v[1], (_Float16)v[2], (_Float16)v[3]};
+  }
 }
 
 }  // namespace
@@ -187,7 +224,7 @@ extern "C" int art_prefill_attention(const void* q_dev, const void* k_dev, const
   const int q_tiles = (T + QT - 1) / QT;
   const long long blocks = (long long)q_tiles * heads;
   ART_REQUIRE(blocks <= 0x7fffffffLL, "art_prefill_attention: too many blocks");
-  prefill_attention_kernel<<<dim3((unsigned)blocks), dim3(64), 0, (hipStream_t)stream>>>(
+  prefill_attention_kernel<<<dim3((unsigned)blocks), dim3(64 * kWaves), 0, (hipStream_t)stream>>>(
       (const _Float16*)q_dev, (const _Float16*)k_dev, (const _Float16*)v_dev, (_Float16*)out_dev, T, heads, kv_row_stride,
       (const float*)att_f_dev, q_tiles);
   ART_LAUNCH_CHECK();
