@@ -171,9 +171,9 @@ def _w4a16_handler(op, bound, env, call) -> bool:
         else:
             counts = [v for v in (1, 2, 3, 4, 5, 6, 8, 10, 12, 16, 20, 24, 32) if v <= K // 128]
             # 512 + v: v K-splits over blocks of 64 rows; 256 + v: over blocks of 32 rows (twice the blocks);
-            # 1024 + v, 2048 + v: over blocks of 128 and 256 rows
+            # 1280 + v: over blocks of 128 rows; 1024 + v, 2048 + v: of 128 and 256 rows and twice the columns
             cands = [0] + [512 + v for v in counts] + ([256 + v for v in counts] if M > 32 else [])
-            cands += [rows + v for rows in (1024, 2048) for v in counts if v <= 16] if M > 64 else []
+            cands += [rows + v for rows in (1280, 1024, 2048) for v in counts if v <= 16] if M > 64 else []
         saved = tune_hand_kernel(op, key, cands, run, trials, clones)
         del clones
     call.library(entry, x, q, s, z, y, M, K, N, *knobs(saved['value'] if saved is not None else 0), STREAM)

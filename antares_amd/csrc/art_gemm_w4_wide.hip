@@ -39,19 +39,6 @@ constexpr int stage_bytes(int MT) { return W_BYTES + Q_BYTES + MT * 32 * SK * 2;
 constexpr size_t lds_bytes(int MT) { return (size_t)NS * stage_bytes(MT); }
 static_assert(128 * C_LD * 2 <= NS * stage_bytes(4), "128 staged output rows fit the ring");
 
-// 64 lanes x 16 (4) bytes from base + lane offset straight into LDS at lds_dst + 16 (4) * lane.  The instruction takes
-// the LDS address from m0, which is put back.  The waits are written by hand: the compiler does not see these loads.
-__device__ __forceinline__ void load_lds_x4(const void* base, unsigned int off, unsigned int lds_dst) {
-  unsigned int keep;
-  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b32 m0, %0"
-               : "=&s"(keep) : "v"(off), "s"(base), "s"(lds_dst));
-}
-__device__ __forceinline__ void load_lds_x1(const void* base, unsigned int off, unsigned int lds_dst) {
-  unsigned int keep;
-  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2\n\ts_mov_b32 m0, %0"
-               : "=&s"(keep) : "v"(off), "s"(base), "s"(lds_dst));
-}
-
 // SWIGLU: the matrix is gate | up (N / 2 columns each); a block owns 128 gate columns and the matching 128 up columns and
 // stores y[m, n] = fp16(silu(fp16(gate)) * fp16(up)), N / 2 columns.
 template <int MT, bool SWIGLU>
@@ -68,7 +55,7 @@ __global__ __launch_bounds__(kThreads, MT == 8 ? 1 : 2) void gemm_w4a16_wide_ker
   const int m_block = (int)(blockIdx.x % (8 * m_blocks)) / 8;
   if (unit >= col_tiles * splits) return;
   const int split = unit / col_tiles;
-  const TileColumns<SWIGLU> cols{(unit % col_tiles) * (SWIGLU ? BN / 2 : BN), N};
+  const TileColumns<SWIGLU, BN> cols{(unit % col_tiles) * (SWIGLU ? BN / 2 : BN), N};
   const int m0 = m_block * BM;
   const int G = K / 128;
   const int g_begin = (int)((long long)G * split / splits), g_end = (int)((long long)G * (split + 1) / splits);
@@ -98,12 +85,6 @@ __global__ __launch_bounds__(kThreads, MT == 8 ? 1 : 2) void gemm_w4a16_wide_ker
 
   // Load j of ring slot `slot`: 0, 1 packed weights, 2 scales and zero points, 3 .. MT + 2 x.  The weights run one
   // stage ahead of x: slot of stage i holds x of stage i and the weights of stage i + 1.
-  // (the bases are the same for every lane; said so explicitly, they stay in scalar registers whatever surrounds the loop)
-  auto uniform = [](const void* p) {
-    const unsigned long long v = (unsigned long long)p;
-    return (const void*)((unsigned long long)(unsigned int)__builtin_amdgcn_readfirstlane((int)v) |
-                         (unsigned long long)(unsigned int)__builtin_amdgcn_readfirstlane((int)(v >> 32)) << 32);
-  };
   auto issue = [&](unsigned int slot, int j) {
     const unsigned int st = lds0 + slot;
     if (j < 2) load_lds_x4(uniform(wbase), woff[j], st + (wave + 4 * j) * 1024);
@@ -336,7 +317,7 @@ int launch(const _Float16* x, const unsigned char* qweight, const _Float16* scal
                                 (int)lds_bytes(MT)));
     configured = true;
   }
-  const int col_tiles = tile_count(N, SWIGLU), m_blocks = (M + 32 * MT - 1) / (32 * MT);
+  const int col_tiles = tile_count(N, SWIGLU, BN), m_blocks = (M + 32 * MT - 1) / (32 * MT);
   gemm_w4a16_wide_kernel<MT, SWIGLU><<<dim3((unsigned)((col_tiles * splits + 7) / 8 * 8 * m_blocks)), kThreads, lds_bytes(MT), stream>>>(
       x, qweight, scales, qzeros, y, partial, M, K, N, splits, col_tiles, m_blocks, kMagic, residual);
   ART_LAUNCH_CHECK();

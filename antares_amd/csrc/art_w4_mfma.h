@@ -25,28 +25,39 @@ __device__ __forceinline__ unsigned int and_or(unsigned int w, unsigned int mask
   return __builtin_amdgcn_bitop3_b32(w, mask, bias, 0xEA);
 }
 
-// 8 halves of x in the k order the nibble extraction leaves in a B operand: k0 k4 k1 k5 k2 k6 k3 k7.
-__device__ __forceinline__ h8 permute_k(u32x4 v) {
-  u32x4 o;
-  o[0] = __builtin_amdgcn_perm(v[2], v[0], 0x05040100u);
-  o[1] = __builtin_amdgcn_perm(v[2], v[0], 0x07060302u);
-  o[2] = __builtin_amdgcn_perm(v[3], v[1], 0x05040100u);
-  o[3] = __builtin_amdgcn_perm(v[3], v[1], 0x07060302u);
-  return __builtin_bit_cast(h8, o);
+// 64 lanes x 16 (4) bytes from base + lane offset straight into LDS at lds_dst + 16 (4) * lane.  The instruction takes
+// the LDS address from m0, which nothing else here uses (the compiler warns that it does not preserve a reserved register
+// that is named as clobbered; nothing has to be preserved).  The waits are written by hand: the compiler does not see
+// these loads.
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+__device__ __forceinline__ void load_lds_x4(const void* base, unsigned int off, unsigned int lds_dst) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds_dst) : "m0");
+}
+__device__ __forceinline__ void load_lds_x1(const void* base, unsigned int off, unsigned int lds_dst) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" ::"v"(off), "s"(base), "s"(lds_dst) : "m0");
+}
+#pragma clang diagnostic pop
+
+// A base address that is the same for every lane, in scalar registers whatever surrounds the load.
+__device__ __forceinline__ const void* uniform(const void* p) {
+  const unsigned long long v = (unsigned long long)p;
+  return (const void*)((unsigned long long)(unsigned int)__builtin_amdgcn_readfirstlane((int)v) |
+                       (unsigned long long)(unsigned int)__builtin_amdgcn_readfirstlane((int)(v >> 32)) << 32);
 }
 
 constexpr Magic kMagic{0x000F000Fu, 0x00F000F0u, 0x64006400u, 0x54005400u};
 
-// The 256 columns of a block: neighbours, or (SWIGLU, the matrix is gate | up) 128 of the gate half and the matching 128 of
+// The BN columns of a block: neighbours, or (SWIGLU, the matrix is gate | up) BN / 2 of the gate half and the matching ones of
 // the up half.  N % 16 == 0 (SWIGLU: N % 32), so a piece of 16 columns is inside or outside as a whole.
-template <bool SWIGLU>
+template <bool SWIGLU, int BN>
 struct TileColumns {
   int n0, N;
-  __device__ __forceinline__ int at(int pos) const { return SWIGLU && pos >= 128 ? N / 2 + n0 + pos - 128 : n0 + pos; }
-  __device__ __forceinline__ bool inside(int pos) const { return SWIGLU ? n0 + (pos & 127) < N / 2 : n0 + pos < N; }
+  __device__ __forceinline__ int at(int pos) const { return SWIGLU && pos >= BN / 2 ? N / 2 + n0 + pos - BN / 2 : n0 + pos; }
+  __device__ __forceinline__ bool inside(int pos) const { return SWIGLU ? n0 + (pos & (BN / 2 - 1)) < N / 2 : n0 + pos < N; }
   __device__ __forceinline__ int safe(int pos) const { return inside(pos) ? at(pos) : 0; }
 };
-inline int tile_count(int N, bool swiglu) { return swiglu ? (N / 2 + 127) / 128 : (N + 255) / 256; }
+inline int tile_count(int N, bool swiglu, int bn) { return swiglu ? (N / 2 + bn / 2 - 1) / (bn / 2) : (N + bn - 1) / bn; }
 
 // fp16(silu(gate) * up) of fp16 operands in fp32, as the decode step's GEMV and the sample's torch line round it.
 __device__ __forceinline__ h4 swiglu4(h4 g, h4 u) {

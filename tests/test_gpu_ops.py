@@ -526,8 +526,8 @@ def test_w4a16_gemm_with_the_residual_folded_in(autort, M, K, N):
 
 
 # one group and many; one row past and one short of a block; the last column tile a chunk of 16; more K-splits than groups
-@pytest.mark.parametrize('M,K,N', [(65, 128, 16), (128, 256, 272), (129, 384, 528), (255, 1024, 240), (257, 640, 256), (300, 2048, 1040)])
-def test_w4a16_gemm_over_blocks_of_128_and_256_rows(autort, M, K, N):
+@pytest.mark.parametrize('M,K,N', [(1, 128, 16), (33, 640, 144), (65, 128, 16), (128, 256, 272), (129, 384, 528), (255, 1024, 240), (257, 640, 256), (300, 2048, 1040)])
+def test_w4a16_gemm_in_every_form(autort, M, K, N):
     from ctypes import c_void_p
     from antares_amd.runtime import capi
     from oracle import hot_ops
@@ -537,10 +537,10 @@ def test_w4a16_gemm_over_blocks_of_128_and_256_rows(autort, M, K, N):
     prod = hot_ops.gemm_w4a16(p['x'].numpy(), p['qweight'].numpy(), p['scales'].numpy(), p['qzeros'].numpy()).astype(np.float32)
     d = [p[k].to(dev) for k in ('x', 'qweight', 'scales', 'qzeros')] + [torch.empty(M, N, dtype=torch.float16, device=dev), res.to(dev)]
     ptr = [c_void_p(t.data_ptr()) for t in d]
-    for rows in (128, 256):
+    for form in (1, 2, 5, 4, 8):          # 32, 64 and 128 rows over 128 columns, 128 and 256 rows over 256 columns
         for splits in (1, 2, 3, 16):
-            note(f'w4a16 gemm M={M} K={K} N={N} blocks of {rows} rows, {splits} splits')
-            code = rows // 32 * 256 + splits
+            note(f'w4a16 gemm M={M} K={K} N={N} form {form}, {splits} splits')
+            code = form * 256 + splits
             for residual, want in ((c_void_p(0), prod), (ptr[5], (prod + res.numpy().astype(np.float32)))):
                 d[4].fill_(float('nan'))
                 capi.check(capi.lib().art_gemm_w4a16_residual(*ptr[:5], residual, M, K, N, code, c_void_p(torch.cuda.current_stream().cuda_stream)))
@@ -561,7 +561,7 @@ def test_w4a16_gemm_with_swiglu_behind_it(autort, M, K, F):
     gate, up = prod[:, :F], prod[:, F:]
     want = gate / (1 + np.exp(-gate)) * up
     d = [p[k].to(dev) for k in ('x', 'qweight', 'scales', 'qzeros')]
-    for code in (0, 256 + 1, 256 + 2, 512 + 1, 512 + 3, 1024 + 1, 1024 + 4, 2048 + 1, 2048 + 2):
+    for code in (0, 256 + 1, 256 + 2, 512 + 1, 512 + 3, 1280 + 1, 1280 + 2, 1024 + 1, 1024 + 4, 2048 + 1, 2048 + 2):
         note(f'w4a16 gemm + swiglu M={M} K={K} F={F} code {code}')
         out = torch.full((M, F), float('nan'), dtype=torch.float16, device=dev)
         capi.check(capi.lib().art_gemm_w4a16_swiglu(*(c_void_p(t.data_ptr()) for t in d), c_void_p(out.data_ptr()), M, K, 2 * F, code,
