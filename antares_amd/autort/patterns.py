@@ -34,6 +34,9 @@ def register(ir: str, inputs, handler: Callable):
 def match(fused: Graph) -> Optional[Tuple[Callable, Dict[str, str]]]:
     """(handler, roles) for a recognised program, else None.  ``roles`` maps the registered program's tensor names
     to the names the caller's program uses for the tensors in the same places."""
+    conv = _conv2d(fused)
+    if conv is not None:
+        return _conv2d_handler(fused.statements[0], *conv[3:]), dict(zip('xwy', conv[:3]))
     hit = _TABLE.get(fused.canonical_key())
     if hit is None or not _axes_span_their_dimensions(fused):
         return None
@@ -292,3 +295,139 @@ def _gemm_f32_layout_handler(trans_a: bool, trans_b: bool):
 register('c[M, N] +=! a[K, M] * b[K, N]', ['a=float32[K:512, M:512]', 'b=float32[K:512, N:512]'], _gemm_f32_layout_handler(True, False))
 register('c[M, N] +=! a[M, K] * b[N, K]', ['a=float32[M:512, K:512]', 'b=float32[N:512, K:512]'], _gemm_f32_layout_handler(False, True))
 register('c[M, N] +=! a[K, M] * b[N, K]', ['a=float32[K:512, M:512]', 'b=float32[N:512, K:512]'], _gemm_f32_layout_handler(True, True))
+
+
+# ---------------------------------------------------------------------------
+# 2-D convolution, stride 1, zeros outside the image (AntaresIR.md:166): y[N, F, HO, WO] +=! x[N, C, HO + KH - ph,
+# WO + KW - pw] * w[F, C, KH, KW], both factors float32 or float16 cast to float32.  Padding, extents and guards are part of
+# the program's text, so it is recognised by its structure.
+# ---------------------------------------------------------------------------
+def _shifted_sum(ix):
+    """``A + B - 3`` -> ([names of the axes added], constant); None for anything else."""
+    if ix.kind == 'axis':
+        return [ix.name], 0
+    if ix.kind == 'const' and isinstance(ix.value, int):
+        return [], ix.value
+    if ix.kind == 'op' and ix.name in '+-' and len(ix.args) == 2:
+        l, r = _shifted_sum(ix.args[0]), _shifted_sum(ix.args[1])
+        if l is not None and r is not None and (ix.name == '+' or not r[0]):
+            return sorted(l[0] + r[0]), l[1] + (r[1] if ix.name == '+' else -r[1])
+    return None
+
+
+def _guards(conds):
+    """[lowest, past the highest] value that the conditions leave to each index expression, by its axes and constant;
+    None when a condition is anything but an expression of that kind compared with an integer."""
+    out = {}
+    for c in conds:
+        if c.kind != 'op' or c.name not in ('<', '<=', '>', '>=') or len(c.args) != 2:
+            return None
+        l, r = _shifted_sum(c.args[0]), _shifted_sum(c.args[1])
+        if l is None or r is None or bool(l[0]) == bool(r[0]):
+            return None
+        op = c.name
+        if r[0]:
+            l, r, op = r, l, {'<': '>', '<=': '>=', '>': '<', '>=': '<='}[op]
+        lo, hi = out.get((tuple(l[0]), l[1]), (None, None))
+        value = r[1] + (op in ('<=', '>'))
+        if op in ('<', '<='):
+            hi = value if hi is None else min(hi, value)
+        else:
+            lo = value if lo is None else max(lo, value)
+        out[(tuple(l[0]), l[1])] = (lo, hi)
+    return out
+
+
+def _conv2d(fused: Graph):
+    """-> (x, w, y, axes by part, {index: (padding, lowest, past the highest)}) of a convolution, else None."""
+    if len(fused.statements) != 1:
+        return None
+    st = fused.statements[0]
+    if st.scatter or st.reduce != '+' or st.out_dtype != 'float32' or len(st.data_axes) != 4 or len(st.reduce_axes) != 3:
+        return None
+    n, f, ho, wo = (a for a, _ in st.data_axes)
+    if [i.name if i.kind == 'axis' else None for i in st.out_index] != [n, f, ho, wo]:
+        return None
+    if st.root.kind != 'op' or st.root.name != '*' or len(st.root.args) != 2:
+        return None
+    factors = []
+    for e in st.root.args:
+        conds = []
+        while e.kind in ('cast', 'when'):
+            if e.kind == 'when':
+                if len(e.args) != 2 or e.merge != 'all' or e.args[1].kind != 'const' or e.args[1].value != 0:
+                    return None
+                conds += list(e.conds)
+            elif e.dtype != 'float32':
+                return None
+            e = e.args[0]
+        if e.kind != 'load' or e.dtype not in ('float16', 'float32') or len(e.args) != 4 or e.name == st.output:
+            return None
+        factors.append((e, conds))
+    if factors[0][0].args[0].kind == 'axis' and factors[0][0].args[0].name == f:
+        factors.reverse()
+    (x, conds), (w, w_conds) = factors
+    if x.dtype != w.dtype or w_conds or not all(i.kind == 'axis' for i in w.args):
+        return None
+    wf, c, kh, kw = (i.name for i in w.args)
+    if wf != f or sorted((c, kh, kw)) != sorted(a for a, _ in st.reduce_axes):
+        return None
+    if [i.name if i.kind == 'axis' else None for i in x.args[:2]] != [n, c]:
+        return None
+    guards, window = _guards(conds), {}
+    if guards is None:
+        return None
+    for ix, axes, key in ((x.args[2], (ho, kh), 'h'), (x.args[3], (wo, kw), 'w')):
+        s = _shifted_sum(ix)
+        if s is None or s[0] != sorted(axes):
+            return None
+        window[key] = (-s[1],) + guards.pop((tuple(s[0]), s[1]), (None, None))
+    if guards:                                    # a condition on something else than the two indices
+        return None
+    return x.name, w.name, st.output, {'n': n, 'f': f, 'c': c, 'kh': kh, 'kw': kw, 'ho': ho, 'wo': wo}, window
+
+
+def _conv2d_handler(st, axes, window):
+    extent = dict(st.data_axes + st.reduce_axes)
+
+    def handler(op, bound, env, call) -> bool:
+        x, w, y = (bound[op.fast_roles[r]] for r in 'xwy')
+        e = {part: extent[a] if isinstance(extent[a], int) else env[extent[a]] for part, a in axes.items()}
+        if x.dim() != 4 or w.dim() != 4 or (x.shape[0], x.shape[1]) != (e['n'], e['c']) or \
+                tuple(w.shape) != (e['f'], e['c'], e['kh'], e['kw']) or \
+                (e['kh'], e['kw']) != (3, 3) or not x.numel() or not y.numel():
+            return False
+        # The kernel reads zeros outside the image and the image everywhere else: that has to be what the guards say, and
+        # an index without a guard on one side must not reach past it.
+        for key, size in (('h', x.shape[2]), ('w', x.shape[3])):
+            pad, lo, hi = window[key]
+            highest = e[key + 'o'] - 1 + e['k' + key] - 1 - pad
+            if (lo != 0 if lo is not None else pad > 0) or (hi != size if hi is not None else highest >= size):
+                return False
+        size = x.element_size()
+        if any(t.data_ptr() < y.data_ptr() + 4 * y.numel() and y.data_ptr() < t.data_ptr() + size * t.numel() for t in (x, w)):
+            return False                          # a result over an operand: the generic kernels' order is kept
+        lib = capi.lib()
+        shape = (int(x.dtype == torch.float16), e['n'], e['c'], x.shape[2], x.shape[3], e['f'], e['ho'], e['wo'],
+                 window['h'][0], window['w'][0])
+        if max(abs(v) for v in shape) >= 1 << 31:
+            return False
+        form = lib.art_conv2d_form(*shape, 0)
+        if not form:
+            return False
+        packed = torch.empty(lib.art_conv2d_packed_bytes(shape[0], e['c'], e['f']), dtype=torch.uint8, device=x.device)
+
+        def run(value, t):
+            capi.check(lib.art_conv2d(*(c_void_p(v.data_ptr()) for v in t), *shape, int(value), c_void_p(torch.cuda.current_stream().cuda_stream)))
+        # the launch parameter: the shape of a block
+        key = 'conv2d.form|' + ','.join(str(v) for v in shape)
+        saved = op.tuned.get(key)
+        trials = op.config.get('tune')
+        if saved is None and isinstance(trials, int) and trials > 0 and not torch.cuda.is_current_stream_capturing():
+            forms = [form] + [v for v in (1, 2, 3) if v != form and lib.art_conv2d_form(*shape, v)]
+            saved = tune_hand_kernel(op, key, forms, run, trials, [(x, w, packed, torch.empty_like(y))])
+        if saved is not None and lib.art_conv2d_form(*shape, int(saved['value'])):
+            form = int(saved['value'])
+        call.library(lib.art_conv2d, x, w, packed, y, *shape, form, STREAM)
+        return True
+    return handler

@@ -1,0 +1,364 @@
+// 3 x 3 convolution, stride 1, NCHW image and FCHW filter, float32 sums, on the gfx950 matrix cores:
+//
+//   y[n, f, ho, wo] = sum over c, kh, kw of x[n, c, ho + kh - ph, wo + kw - pw] * w[f, c, kh, kw]        (0 outside x)
+//
+// Replaces, for these programs (AntaresIR.md:166), what the reference's tiled schedule generates
+// (backends/c-rocm/schedule/standard/algo_tiling.py:35-98).
+//
+// Design for MI355X.  As a matrix product (features x output points, k = channels x taps) the operation is bound by the
+// matrix cores, but a kernel that gathers the image once per tap is bound by the gathering: it fetches every image value
+// nine times in pieces of one element, with an address and two comparisons each.  Here:
+//   * the output points of a block (64 or 128 in a row of n, ho, wo) need one CONTIGUOUS run of points of the image
+//     padded to HO + 2 rows of WO + 2: the run is staged in LDS once per 64 bytes of channels (32 float16 or
+//     16 float32), as [point][channel], and a tap is a constant number of points added to a lane's LDS address.  Global
+//     reads run along the points (a wavefront reads 64 of them from one channel), 16-byte LDS writes put a lane's 8 or 4
+//     channels side by side; 80 bytes from point to point keep reads and writes on distinct banks;
+//   * the offset of each staged point (or "outside") is worked out once per block;
+//   * the filter is packed first, by a launch of its own, in the order in which wavefronts feed it to the matrix
+//     instructions: [64 bytes of channels][tap][32 features][half][lane] with 16 bytes per lane, so that a wavefront's
+//     operand is one contiguous kilobyte that comes from L2 straight into registers, a tap ahead of its use;
+//   * the next 64 bytes of channels travel to registers while these are multiplied, two LDS buffers, one LDS-only barrier
+//     per 64 bytes of channels (18 to 72 matrix instructions per wavefront and barrier for a 3 x 3 filter, not 2 to 8);
+//   * 2 x 2 wavefronts of MT x NT tiles of 32 features x 32 points; blocks of one run of points are neighbours on one XCD.
+// Measured, padding 1, both launches, against the generic lowering (a padded copy, then a gathering product): float16
+// 32 x 128 x 28 x 28 -> 128 41.4 -> 21.1 us, 24 x 200 x 33 x 33 -> 48 89 -> 23 us, 2 x 160 x 18 x 18 -> 64 57 -> 14 us;
+// float32 32 x 128 x 28 x 28 -> 128 113 -> 81 us (the matrix instructions alone take 47), 23 x 128 x 30 x 30 -> 176 119 -> 86.
+// The first of these spends 7 us of the matrix cores' time in 18.6 us: one block per compute unit and only 4 chunks, so the
+// first image fetch, the waits between chunks and the stores of 12.8 MB stay in sight; packing the filter takes 2.3 us.
+#include <type_traits>
+
+#include "art_common.h"
+
+namespace {
+
+constexpr int kThreads = 256;
+constexpr int kTaps = 9;                        // 3 x 3
+constexpr int kChunkBytes = 64;                 // channels of a point that are staged at a time
+constexpr int kPitchBytes = kChunkBytes + 16;   // from one point to the next in LDS
+constexpr unsigned kOutside = 0xffffffffu;
+constexpr size_t kMaxLds = 64 * 1024;
+
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+template <typename T> struct Elem;
+template <> struct Elem<_Float16> {
+  typedef _Float16 vec __attribute__((ext_vector_type(8)));
+  typedef unsigned short raw;
+  static __device__ __forceinline__ f32x16 multiply(vec a, vec b, f32x16 c) { return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0); }
+};
+template <> struct Elem<float> {
+  typedef float vec __attribute__((ext_vector_type(4)));
+  typedef float raw;
+  // instruction m multiplies k = m (lanes 0-31) and k = 4 + m (lanes 32-63) of 8
+  static __device__ __forceinline__ f32x16 multiply(vec a, vec b, f32x16 c) {
+#pragma unroll
+    for (int m = 0; m < 4; ++m) c = __builtin_amdgcn_mfma_f32_32x32x2f32(a[m], b[m], c, 0, 0, 0);
+    return c;
+  }
+};
+
+struct Geometry {
+  int N, C, H, W, F, HO, WO, ph, pw;
+  int columns;          // output points: N * HO * WO
+  int chunks;           // runs of 64 bytes of channels
+  int row_tiles;        // 32-feature tiles of the packed filter
+  int row_blocks;       // blocks along the features
+  int span;             // points the LDS buffers hold
+};
+
+// Output point -> its place in the padded image (where tap (0, 0) reads).
+__device__ __forceinline__ int place_of(int column, const Geometry& g) {
+  const unsigned hw = (unsigned)(g.HO * g.WO), n = (unsigned)column / hw, r = (unsigned)column % hw;
+  const unsigned ho = r / (unsigned)g.WO, wo = r % (unsigned)g.WO;
+  return (int)((n * (unsigned)(g.HO + 2) + ho) * (unsigned)(g.WO + 2) + wo);
+}
+
+// Filter [F][C][taps] -> [chunk][tap][32 features][half][lane][16 bytes], zeros past F and C.  A thread gathers the 16
+// bytes of one lane; bound by latency (about 2 us).
+template <typename T>
+__global__ __launch_bounds__(kThreads) void conv2d_pack_kernel(const T* __restrict__ w, T* __restrict__ packed, Geometry g) {
+  constexpr int V = 16 / sizeof(T);
+  const long long id = (long long)blockIdx.x * kThreads + threadIdx.x;
+  if (id >= (long long)g.chunks * kTaps * g.row_tiles * 128) return;
+  const int lane = (int)(id & 63), half = (int)(id >> 6) & 1;
+  const unsigned rest = (unsigned)(id >> 7);
+  const int r = (int)(rest % (unsigned)g.row_tiles);
+  const unsigned qt = rest / (unsigned)g.row_tiles;
+  const int t = (int)(qt % (unsigned)kTaps), q = (int)(qt / (unsigned)kTaps);
+  const int f = r * 32 + (lane & 31), c0 = (q * 4 + half * 2 + (lane >> 5)) * V;
+  typename Elem<T>::vec v;
+#pragma unroll
+  for (int j = 0; j < V; ++j) v[j] = (f < g.F && c0 + j < g.C) ? w[((size_t)f * g.C + c0 + j) * kTaps + t] : (T)0;
+  reinterpret_cast<typename Elem<T>::vec*>(packed)[id] = v;
+}
+
+template <typename T, int MT, int NT>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 4))) void conv2d_kernel(const T* __restrict__ x, const T* __restrict__ packed, float* __restrict__ y, Geometry g) {
+  typedef typename Elem<T>::vec vec;
+  constexpr int kHeld = NT == 1 ? 3 : 5;              // points per lane that travel while the channels before them are multiplied (more: fetched behind them)
+  constexpr int V = 16 / sizeof(T), TN = 64 * NT, kPitch = kPitchBytes / sizeof(T);
+  extern __shared__ __align__(16) char lds[];
+  T* image = reinterpret_cast<T*>(lds);                                                 // [2][span][pitch]
+  unsigned* where = reinterpret_cast<unsigned*>(lds + 2 * (size_t)g.span * kPitchBytes);   // [span]: byte offset into x without the channel, or kOutside
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave >> 1, wn = wave & 1;
+  const int wide = g.WO + 2, high = g.HO + 2;
+  // workgroups go to the eight XCDs round robin: an XCD gets a contiguous run of blocks
+  const int per = gridDim.x >> 3, left = gridDim.x & 7, xcd = blockIdx.x & 7;
+  const int block = xcd * per + (xcd < left ? xcd : left) + (blockIdx.x >> 3);
+  const int rb = block % g.row_blocks, column0 = (block / g.row_blocks) * TN;
+  const int last = (column0 + TN < g.columns ? column0 + TN : g.columns) - 1;
+  const int place0 = place_of(column0, g);
+  const int points = place_of(last, g) - place0 + 2 * wide + 3;            // <= span
+
+  for (int i = tid; i < points; i += kThreads) {
+    const unsigned p = (unsigned)(place0 + i), n = p / (unsigned)(high * wide), r = p % (unsigned)(high * wide);
+    const int h = (int)(r / (unsigned)wide) - g.ph, w = (int)(r % (unsigned)wide) - g.pw;
+    const bool in = h >= 0 && h < g.H && w >= 0 && w < g.W;
+    where[i] = in ? ((n * (unsigned)g.C * (unsigned)g.H + (unsigned)h) * (unsigned)g.W + (unsigned)w) * (unsigned)sizeof(T) : kOutside;
+  }
+
+  // this lane's output points: LDS place of tap (0, 0), and where the result goes
+  int at[NT];
+  size_t to[NT];
+#pragma unroll
+  for (int j = 0; j < NT; ++j) {
+    int column = column0 + wn * 32 * NT + j * 32 + (lane & 31);
+    if (column > last) column = last;
+    at[j] = (place_of(column, g) - place0) * kPitch + (lane >> 5) * V;
+    const unsigned hw = (unsigned)(g.HO * g.WO);
+    to[j] = (size_t)((unsigned)column / hw) * g.F * hw + (unsigned)column % hw;
+  }
+  // Item i of a lane: point lane + 64 i, channels wave * V .. + V - 1 of the chunk.  Loads go out without a branch between
+  // them (points and channels past the end re-read the last one) and stay as they came until they are put into LDS: a
+  // branch or a conversion behind each load is a wait for it.
+  const size_t plane = (size_t)g.H * g.W * sizeof(T);
+  const int items = (points + 63) >> 6;
+  struct Item { typename Elem<T>::raw v[V]; };
+  auto fetch = [&](int q, int i) {
+    const int point = lane + 64 * i, c0 = (q * 4 + wave) * V;
+    const unsigned o = where[point < points ? point : points - 1];
+    const unsigned from = o == kOutside ? 0u : o;
+    Item r;
+#pragma unroll
+    for (int j = 0; j < V; ++j) {
+      const int c = c0 + j < g.C ? c0 + j : g.C - 1;                                    // the same in all lanes
+      const char* base = reinterpret_cast<const char*>(x) + c * plane;
+      r.v[j] = *reinterpret_cast<const typename Elem<T>::raw*>(base + (size_t)from);
+    }
+    return r;
+  };
+  auto put = [&](int q, int i, const Item& r) {
+    const int point = lane + 64 * i, c0 = (q * 4 + wave) * V;
+    vec v;
+#pragma unroll
+    for (int j = 0; j < V; ++j) v[j] = __builtin_bit_cast(T, r.v[j]);
+    if (c0 + V > g.C) {
+#pragma unroll
+      for (int j = 0; j < V; ++j) if (c0 + j >= g.C) v[j] = (T)0;
+    }
+    if (point >= points) return;
+    if (where[point] == kOutside) v = vec(0);
+    *reinterpret_cast<vec*>(image + ((size_t)(q & 1) * g.span + point) * kPitch + wave * V) = v;
+  };
+
+  // The filter: a wavefront's MT x 2 operands of a tap, 64 x 16 bytes each, asked for kAhead taps before their use (a
+  // tap is 64 to 256 cycles of matrix instructions, L2 answers after several hundred).
+  constexpr int kSets = MT == 1 ? kTaps : 3, kAhead = kSets - 1;
+  const vec* filter = reinterpret_cast<const vec*>(packed) + ((size_t)rb * 2 + wm) * MT * 128 + lane;
+  const size_t filter_step = (size_t)g.row_tiles * 128;
+  constexpr int kSum = MT == 1 && NT == 1 ? 3 : kTaps;            // taps summed by themselves
+  constexpr int kPerTap = MT == 1 ? kHeld : 2;        // points per lane asked for with a tap
+  vec a[kSets][MT][2];
+  auto fetch_filter = [&](int set, int tap) {
+    const vec* p = filter + (size_t)tap * filter_step;
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) a[set][i][h] = p[(i * 2 + h) * 64];
+  };
+
+  art_lds_barrier();                                  // `where` is written
+  Item held[kHeld];
+#pragma unroll
+  for (int i = 0; i < kHeld; ++i) held[i] = fetch(0, i);
+#pragma unroll
+  for (int t = 0; t < kAhead; ++t) fetch_filter(t, t);      // asked for last: loads come back in order
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int i = 0; i < kHeld; ++i) put(0, i, held[i]);
+  for (int i = kHeld; i < items; ++i) put(0, i, fetch(0, i));
+  art_lds_barrier();
+  f32x16 total[MT][NT];
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) total[i][j][e] = 0.f;
+  auto chunk = [&](int q, auto last_chunk) {
+    constexpr bool kMore = !decltype(last_chunk)::value;
+    const T* tile = image + (size_t)(q & 1) * g.span * kPitch;
+    // a chunk is summed by itself and then added to the total (where registers allow, a row of taps by itself before
+    // that): the error of a sum grows with the length of its chain
+    f32x16 acc[MT][NT], row[MT][NT];
+    vec b[2][NT];
+    auto look = [&](int h, int t) {
+      const T* from = tile + ((t / 3) * wide + t % 3) * kPitch;
+#pragma unroll
+      for (int j = 0; j < NT; ++j) b[h][j] = *reinterpret_cast<const vec*>(from + at[j] + h * 2 * V);
+    };
+    look(0, 0);
+#pragma unroll
+    for (int t = 0; t < kTaps; ++t) {
+      if (kMore) {
+#pragma unroll
+        for (int i = t * kPerTap; i < (t + 1) * kPerTap && i < kHeld; ++i) held[i] = fetch(q + 1, i);
+      }
+      if (kMore || t + kAhead < kTaps) fetch_filter((t + kAhead) % kSets, q * kTaps + t + kAhead);
+      __builtin_amdgcn_sched_barrier(0);              // left to the scheduler, the loads sink to their use
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        if (h == 0 || t + 1 < kTaps) look(h ^ 1, t + h);        // the other half, or the next tap's first
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+          for (int j = 0; j < NT; ++j)
+            row[i][j] = Elem<T>::multiply(a[t % kSets][i][h], b[h][j], h == 0 && t % kSum == 0 ? f32x16(0) : row[i][j]);
+      }
+      if (t % kSum != kSum - 1) continue;
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) acc[i][j] = t < kSum ? row[i][j] : acc[i][j] + row[i][j];
+    }
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int j = 0; j < NT; ++j) total[i][j] += acc[i][j];
+    if (kMore) {
+#pragma unroll
+      for (int i = 0; i < kHeld; ++i) put(q + 1, i, held[i]);
+      for (int i = kHeld; i < items; ++i) put(q + 1, i, fetch(q + 1, i));
+      art_lds_barrier();      // the other buffer is written, this one is free
+    }
+  };
+  for (int q = 0; q + 1 < g.chunks; ++q) chunk(q, std::false_type{});
+  chunk(g.chunks - 1, std::true_type{});
+
+  // accumulator element e: feature (e / 4) * 8 + (lane / 32) * 4 + e % 4 of the tile, point lane % 32
+#pragma unroll
+  for (int j = 0; j < NT; ++j) {
+    if (column0 + wn * 32 * NT + j * 32 + (lane & 31) > last) continue;
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const int f = ((rb * 2 + wm) * MT + i) * 32 + (e >> 2) * 8 + (lane >> 5) * 4 + (e & 3);
+        if (f < g.F) __builtin_nontemporal_store(total[i][j][e], y + to[j] + (size_t)f * g.HO * g.WO);
+      }
+  }
+}
+
+// The most points a block of `columns` output points can need: every step to the next row skips two points, every
+// step to the next image two rows.
+int span_of(const Geometry& g, int columns) {
+  if (columns > g.columns) columns = g.columns;
+  const long long wide = g.WO + 2, hw = (long long)g.HO * g.WO;
+  const long long rows = (columns - 1 + g.WO - 1) / g.WO, images = (columns - 1 + hw - 1) / hw;
+  const long long span = columns - 1 + rows * 2 + images * 2 * wide + 2 * wide + 3;
+  return span > (1 << 20) ? 1 << 20 : (int)span;
+}
+
+size_t lds_of(int span) { return (size_t)span * (2 * kPitchBytes + 4); }
+
+// Forms: 1 = 64 features x 64 points per block, 2 = 64 x 128, 3 = 128 x 128.
+int features_of(int form) { return form == 3 ? 128 : 64; }
+int points_of(int form) { return form == 1 ? 64 : 128; }
+
+bool geometry(Geometry& g, int f16, int N, int C, int H, int W, int F, int HO, int WO, int ph, int pw) {
+  g = Geometry{N, C, H, W, F, HO, WO, ph, pw, 0, 0, 0, 0, 0};
+  if (N < 1 || C < 1 || H < 1 || W < 1 || F < 1 || HO < 1 || WO < 1) return false;
+  // byte offsets into x and places in the padded image are 32-bit
+  if ((long long)HO > (1 << 20) || (long long)WO > (1 << 20)) return false;
+  const long long image = (long long)(HO + 2) * (WO + 2);
+  if (image > (1LL << 30) / N || (long long)H * W > (1LL << 30) / ((long long)N * C)) return false;
+  if ((long long)N * C * H * W * (f16 ? 2 : 4) > (1LL << 31)) return false;
+  g.columns = N * HO * WO;
+  g.chunks = (C + (f16 ? 31 : 15)) / (f16 ? 32 : 16);
+  return (long long)g.chunks * kTaps * ((F + 127) / 128) * 4 < (1 << 22);      // packed filter below 4 GiB
+}
+
+bool fits(const Geometry& g, int form) { return form >= 1 && form <= 3 && lds_of(span_of(g, points_of(form))) <= kMaxLds; }
+
+long long blocks_of(const Geometry& g, int form) {
+  return (long long)((g.columns + points_of(form) - 1) / points_of(form)) * ((g.F + features_of(form) - 1) / features_of(form));
+}
+
+// The form for these sizes, or 0: the generic kernels are faster or sum more exactly there.  Lines from sweeps of 90 sizes
+// (C 16-256, F 16-256, images of 7-56 squared, batches 1-32), times in us generic / here.
+//  * fewer than 32 features, or fewer than 16 blocks of 64 x 64: the generic path sums on the vector units in short
+//    chains.  In float32 that error (0.8e-7 against 64 bits) is below the matrix instructions' (1.3e-7): left alone.  In
+//    float16 it is the same (0.7-1.1e-7 both) from 64 channels on, and the times are 62 / 16 (1 x 224 -> 24, 35 x 35) and
+//    120 / 14 (2 x 128 -> 24, 46 x 46); below 8192 results the generic path wins (7 / 9 for 7 x 40 -> 16, 7 x 7).
+//  * from 1024 terms per result on the generic path slices the sum over an idle chip: 13 / 18 (float16, 5 x 216 -> 40,
+//    14 x 14, 16 blocks), 22 / 14 at 144 blocks; float32 23 / 43 at 40 blocks, 80 / 55 at 475.
+//  * 64 x 128 from 128 such blocks on (float16, 150 blocks: 28.8 with 64 x 64, 27.1; 92 blocks: 18.7, 21.0), 128 x 128
+//    from 192 on where it pads no more features (32 x 128 -> 128, 28 x 28: 27.1, 21.7, 21.1).
+int choose(const Geometry& g, int f16) {
+  const long long small = blocks_of(g, 1);
+  const bool vector_units = g.F < 32 || small < 16;
+  if (vector_units && (!f16 || (long long)g.columns * g.F < 8192 || (g.F < 32 && g.C < 64))) return 0;
+  if (!vector_units && 9LL * g.C >= 1024 && small < (f16 ? 64 : 192)) return 0;
+  if (g.F >= 32) {
+    if ((g.F + 127) / 128 * 2 == (g.F + 63) / 64 && blocks_of(g, 3) >= 192 && fits(g, 3)) return 3;
+    if (blocks_of(g, 2) >= 128 && fits(g, 2)) return 2;
+  }
+  return fits(g, 1) ? 1 : 0;
+}
+
+template <typename T, int MT, int NT>
+void launch(const void* x, const void* packed, void* y, const Geometry& g, unsigned blocks, hipStream_t st) {
+  conv2d_kernel<T, MT, NT><<<dim3(blocks), dim3(kThreads), lds_of(g.span), st>>>((const T*)x, (const T*)packed, (float*)y, g);
+}
+
+template <typename T>
+int run(const void* x, const void* w, void* packed, void* y, const Geometry& g, int form, hipStream_t st) {
+  const long long lanes = (long long)g.chunks * kTaps * g.row_tiles * 128;
+  conv2d_pack_kernel<T><<<dim3((unsigned)((lanes + kThreads - 1) / kThreads)), dim3(kThreads), 0, st>>>((const T*)w, (T*)packed, g);
+  ART_LAUNCH_CHECK();
+  const unsigned blocks = (unsigned)blocks_of(g, form);
+  if (form == 1) launch<T, 1, 1>(x, packed, y, g, blocks, st);
+  else if (form == 2) launch<T, 1, 2>(x, packed, y, g, blocks, st);
+  else launch<T, 2, 2>(x, packed, y, g, blocks, st);
+  ART_LAUNCH_CHECK();
+  return 0;
+}
+
+}  // namespace
+
+extern "C" int art_conv2d_form(int f16, int N, int C, int H, int W, int F, int HO, int WO, int ph, int pw, int form) {
+  Geometry g;
+  if (!geometry(g, f16, N, C, H, W, F, HO, WO, ph, pw)) return 0;
+  return form ? (fits(g, form) ? form : 0) : choose(g, f16);
+}
+
+extern "C" size_t art_conv2d_packed_bytes(int f16, int C, int F) {
+  const size_t chunks = ((size_t)C + (f16 ? 31 : 15)) / (f16 ? 32 : 16);
+  return chunks * kTaps * (((size_t)F + 127) / 128) * 4 * 2048;
+}
+
+extern "C" int art_conv2d(const void* x_dev, const void* w_dev, void* packed_dev, void* y_dev, int f16, int N, int C, int H, int W, int F, int HO,
+                          int WO, int ph, int pw, int form, void* stream) {
+  Geometry g;
+  ART_REQUIRE(geometry(g, f16, N, C, H, W, F, HO, WO, ph, pw) && fits(g, form), "art_conv2d: sizes the kernel does not take (form %d)", form);
+  ART_REQUIRE(x_dev && w_dev && packed_dev && y_dev, "art_conv2d: null pointer");
+  const uintptr_t size = f16 ? 2 : 4;
+  ART_REQUIRE((uintptr_t)x_dev % size == 0 && (uintptr_t)w_dev % size == 0 && (uintptr_t)packed_dev % 16 == 0 && (uintptr_t)y_dev % 4 == 0,
+              "art_conv2d: misaligned tensor");
+  g.row_blocks = (F + features_of(form) - 1) / features_of(form);
+  g.row_tiles = g.row_blocks * (features_of(form) / 32);
+  g.span = span_of(g, points_of(form));
+  return f16 ? run<_Float16>(x_dev, w_dev, packed_dev, y_dev, g, form, (hipStream_t)stream)
+             : run<float>(x_dev, w_dev, packed_dev, y_dev, g, form, (hipStream_t)stream);
+}

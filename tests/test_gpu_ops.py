@@ -1172,3 +1172,75 @@ def test_fp32_gemm_with_operands_stored_the_other_way_round(autort, ir, ta, tb, 
         sel[torch.arange(M), torch.arange(M) % K] = 1.0              # row m of the result = row m % K of B
         sel_in = sel.t().contiguous() if ta else sel
         assert torch.equal(op(sel_in.to(dev), b.to(dev)).cpu(), (b.t() if tb else b)[torch.arange(M) % K].contiguous())
+
+
+def conv_program(dtype, hw, out, pads, guard=True):
+    """A 3 x 3 convolution over hw = (H, W) with pads = (ph, pw) and results of out = (HO, WO)."""
+    cast = '.to(`float32`)' if dtype == 'float16' else ''
+    idx = [f'{a}O + K{a} - {p}' if p > 0 else f'{a}O + K{a} + {-p}' for a, p in zip('HW', pads)]
+    when = f'.when([{idx[0]} >= 0, {idx[0]} < {hw[0]}, {idx[1]} >= 0, {idx[1]} < {hw[1]}], 0.0)' if guard else ''
+    return (f'output0[N, F, HO, WO] +=! input0[N, C, {idx[0]}, {idx[1]}]{cast}{when} * input1[F, C, KH, KW]{cast} '
+            f'where HO in {out[0]}, WO in {out[1]}')
+
+
+CONV_CASES = [  # N, C, (H, W), F, (ph, pw), (HO, WO), guarded
+    (2, 16, (9, 9), 33, (1, 1), (9, 9), True),             # a block spans several images, one more feature than a tile
+    (3, 33, (13, 17), 64, (1, 1), (13, 17), True),         # channels one past a chunk, a wide image
+    (1, 70, (40, 3), 130, (1, 1), (40, 3), True),          # rows of three points, a block of two features
+    (5, 24, (8, 8), 48, (0, 0), (6, 6), False),            # no padding: no guards
+    (2, 20, (12, 10), 40, (2, 0), (14, 7), True),          # padded on one axis by two, results short of the other's end
+    (1, 16, (1, 1), 32, (1, 1), (1, 1), True),             # one point
+    (4, 8, (30, 31), 20, (-1, 1), (27, 31), True),         # taps that start inside
+]
+
+
+@pytest.mark.parametrize('dtype', ['float16', 'float32'])
+@pytest.mark.parametrize('form', [1, 2, 3])
+@pytest.mark.parametrize('case', CONV_CASES)
+def test_convolution_blocks_match_float64(autort, dtype, form, case):
+    """Each block shape of the convolution kernel against the same sum in 64 bits: products of float16 are exact in
+    float32, so the error is that of float32 sums of 9 C terms in any order."""
+    from ctypes import c_void_p
+    from antares_amd.runtime import capi
+    N, C, (H, W), F, (ph, pw), (HO, WO), _ = case
+    note(f'convolution {dtype} form {form} {case}')
+    g = torch.Generator().manual_seed(N * 1000 + C)
+    x = torch.randn(N, C, H, W, generator=g).to(getattr(torch, dtype))
+    w = torch.randn(F, C, 3, 3, generator=g).to(getattr(torch, dtype))
+    f16 = int(dtype == 'float16')
+    shape = (f16, N, C, H, W, F, HO, WO, ph, pw)
+    lib = capi.lib()
+    assert lib.art_conv2d_form(*shape, form) == form
+    dev = autort.device()
+    xd, wd = x.to(dev), w.to(dev)
+    y = torch.full((N, F, HO, WO), 7.0, device=dev)
+    packed = torch.empty(lib.art_conv2d_packed_bytes(f16, C, F), dtype=torch.uint8, device=dev)
+    capi.check(lib.art_conv2d(*(c_void_p(t.data_ptr()) for t in (xd, wd, packed, y)), *shape, form, c_void_p(torch.cuda.current_stream().cuda_stream)))
+    pad = max(ph, pw, 0) + 2
+    big = torch.nn.functional.conv2d(torch.nn.functional.pad(x.double(), (pad, pad + 2, pad, pad + 2)), w.double())
+    want = big[:, :, pad - ph:pad - ph + HO, pad - pw:pad - pw + WO]
+    bound = 2.0 ** -23 * 9 * C * torch.nn.functional.conv2d(
+        torch.nn.functional.pad(x.double().abs(), (pad, pad + 2, pad, pad + 2)), w.double().abs())[:, :, pad - ph:pad - ph + HO, pad - pw:pad - pw + WO]
+    assert ((y.cpu().double() - want).abs() <= bound + 1e-30).all()
+
+
+@pytest.mark.parametrize('dtype,n,c,f,hw', [('float16', 4, 40, 72, 20), ('float16', 2, 64, 24, 23), ('float32', 5, 20, 72, 21), ('float16', 30, 16, 256, 28)])
+def test_convolution_operator_takes_the_kernel_and_agrees_with_the_generic_one(autort, dtype, n, c, f, hw):
+    note(f'convolution operator {dtype} {n}x{c}x{hw}x{hw} -> {f}')
+    dev = autort.device()
+    dt = getattr(torch, dtype)
+    op = autort.export(ir=conv_program(dtype, (hw, hw), (hw, hw), (1, 1)),
+                       inputs=[f'input0={dtype}[N:{n}, C:{c}, H:{hw}, W:{hw}]', f'input1={dtype}[F:{f}, C:{c}, KH:3, KW:3]'], name=f'conv_hand_{dtype}_{n}_{c}')
+    x, w = torch.randn(n, c, hw, hw, device=dev).to(dt), torch.randn(f, c, 3, 3, device=dev).to(dt)
+    x[0, 0, 0, 0], x[0, 0, hw - 1, hw - 1] = float('inf'), float('nan')
+    taken = []
+    handler = op.fast_path
+    op.fast_path = lambda *a: taken.append(handler(*a)) or taken[-1]
+    got, again = op(x, w), op(x, w)
+    assert taken and all(taken) and torch.equal(got.isnan(), again.isnan()) and torch.equal(got.nan_to_num(), again.nan_to_num())
+    op = autort.export(ir=op.ir, inputs=op.input_specs, name=f'conv_generic_{dtype}_{n}_{c}')
+    op.fast_path = None
+    want = op(x, w)
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf())
+    fin = want.isfinite()
+    assert ((got - want)[fin].norm() / want[fin].norm()).item() < 2.0 ** -23 * 9 * c       # float32 sums of 9 c terms, another order

@@ -235,3 +235,34 @@ def test_programs_that_restrict_an_axis_do_not_take_a_hand_kernel():
     # a `where` that only repeats the dimension, or static shapes of the full extent, still match
     assert patterns.match(fuse_elementwise(parse_program('c[M, N] +=! a[M, K] * b[K, N] where K in 4096',
                                                          ['a=float32[4096, 4096]', 'b=float32[4096, 4096]']))) is not None
+
+
+def test_convolutions_are_recognised_by_structure():
+    """What the hand-written 3 x 3 convolution is asked about, and what it must not be."""
+    from antares_amd.autort import patterns
+    from antares_amd.ir import fuse_elementwise, parse_program
+    ins = ['input0={}[N:2, C:8, H:20, W:20]', 'input1={}[F:16, C:8, KH:3, KW:3]']
+
+    def conv(ir, dtype='float32'):
+        return patterns._conv2d(fuse_elementwise(parse_program(ir, [i.format(dtype) for i in ins])))
+    head, tail = 'output0[N, F, HO, WO] +=! ', ' * input1[F, C, KH, KW]'
+    x = 'input0[N, C, HO + KH - 1, WO + KW - 1]'
+    when = '.when([HO + KH - 1 >= 0, 20 > HO + KH - 1, -1 < WO + KW - 1, WO + KW - 1 <= 19], 0.0)'
+    where = ' where HO in 20, WO in 20'
+    got = conv(head + x + when + tail + where)
+    assert got[:3] == ('input0', 'input1', 'output0') and got[4] == {'h': (1, 0, 20), 'w': (1, 0, 20)}
+    assert conv(head + 'input1[F, C, KH, KW] * ' + x + when + where)[:3] == got[:3]
+    assert conv(head + 'input0[N, C, HO + KH, WO + KW]' + tail + ' where HO in 18, WO in 18')[4] == {'h': (0, None, None), 'w': (0, None, None)}
+    half = head + x + '.to(`float32`)' + when + tail + '.to(`float32`)' + where
+    assert conv(half, 'float16')[4] == got[4]
+    for ir in (head + 'input0[N, C, HO * 2 + KH, WO + KW]' + tail + ' where HO in 9, WO in 18',           # a stride
+               head + 'input0[N, C, HO + KH * 2, WO + KW]' + tail + ' where HO in 16, WO in 18',          # a dilation
+               head + 'input0[N, C, HO - KH + 2, WO + KW]' + tail + ' where HO in 18, WO in 18',          # a mirrored filter
+               head + 'input0[N, C, WO + KH, HO + KW]' + tail + ' where HO in 18, WO in 18',              # a transposed image
+               head + x + when.replace('0.0)', '1.0)') + tail + where,                                    # padded with ones
+               head + x + when.replace('HO + KH - 1 >= 0', 'HO + KH >= 1 + N') + tail + where,            # a guard on something else
+               head + x + '.when([HO + KH - 1 >= 0, WO + KW - 1 >= 0], 0.0, merge_op="any")' + tail + where,
+               'output0[N, F, WO, HO] +=! ' + x + when + tail + where,                                    # results transposed
+               'output0[N, F, HO, WO] >=! ' + x + when + tail + where):                                   # not a sum
+        assert conv(ir) is None, ir
+    assert conv(head + 'input0[N, C, HO + KH, WO + KW]' + tail + ' where HO in 18, WO in 18', 'float16') is None     # sums in float16 are another program
