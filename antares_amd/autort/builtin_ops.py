@@ -467,6 +467,33 @@ class GemmW4Residual(calls.Operator):
 builtin('gemm_w4a16_residual')(lambda: GemmW4Residual())
 
 
+class GemmW4ResidualNorm(calls.Operator):
+    """``gemm_w4a16_residual_norm(x[M,K], qweight, scales, qzeros, out[M,N], norm_weight[N], residual=None, norm_out=None,
+    eps=1e-5)``: ``gemm_w4a16_residual`` and the RMSNorm of its result, which is returned."""
+    name = 'gemm_w4a16_residual_norm'
+
+    def __init__(self):
+        self._bind(('x', 'qweight', 'scales', 'qzeros', 'out', 'norm_weight', 'residual', 'norm_out', 'eps'), ())
+
+    def _call(self, pending, x, qweight, scales, qzeros, out, norm_weight, residual=None, norm_out=None, eps=RMS_EPS):
+        M, K = x.shape
+        N = qweight.shape[1]
+        if norm_out is None:
+            norm_out = torch.empty(M, N, dtype=torch.float16, device=x.device)
+        if qweight.shape[0] * 2 != K or scales.shape != (K // 128, N) or qzeros.shape != (K // 128, N // 2) or out.shape != (M, N) or \
+                norm_out.shape != (M, N) or norm_weight.numel() != N:
+            raise ValueError('gemm_w4a16_residual_norm: operand shapes do not match M, K, N')
+        if any(t.dtype != torch.float16 for t in (x, scales, out, norm_weight, norm_out)) or \
+                (residual is not None and (residual.dtype != torch.float16 or residual.shape != out.shape)):
+            raise TypeError('gemm_w4a16_residual_norm: x, scales, out, residual, norm_weight and norm_out must be float16 (residual of the shape of out)')
+        _require_cuda(*([x, qweight, scales, qzeros, out, norm_weight, norm_out] + ([residual] if residual is not None else [])))
+        return _run(self, pending, norm_out, capi.lib().art_gemm_w4a16_residual_norm, x, qweight, scales, qzeros, out, residual, norm_weight, norm_out,
+                    M, K, N, float(eps), 0)
+
+
+builtin('gemm_w4a16_residual_norm')(lambda: GemmW4ResidualNorm())
+
+
 class GemmW4Swiglu(calls.Operator):
     """``gemm_w4a16_swiglu(x[M,K], qweight[K/2,2F], scales, qzeros, out[M,F])``: the packed int4 product of a batch of rows
     with a gate | up matrix and the SwiGLU of its two halves, out = fp16(silu(gate) * up)."""

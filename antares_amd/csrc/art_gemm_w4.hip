@@ -305,6 +305,56 @@ __global__ __launch_bounds__(256) void gemm_w4a16_combine_kernel(const float* __
   *reinterpret_cast<h4*>(y + i * 4) = out;
 }
 
+// The same with the RMSNorm that follows (norm_out = fp16(y / rms(y) * weight), from the rounded y): a block owns a row, whose
+// elements stay in registers, 8 per thread and turn (N % 8 == 0, N <= 8192; as many threads as a row of up to 4096 has
+// pieces of 8).  Bound by the launch: instead of two launches of 2 us and more, one; a layer of the 32-layer model's prompt pass has
+// two of them: 8 layers 611 -> 596 us at 8 tokens, 938 -> 911 at 100, 1318 -> 1311 at 200 (fewer K-splits meet).
+constexpr int kNormThreads = 512, kNormTurns = 2;
+__global__ __launch_bounds__(kNormThreads) void gemm_w4a16_combine_norm_kernel(const float* __restrict__ partial, _Float16* y, int N,
+                                                                                long long split_stride, int splits, const _Float16* residual,
+                                                                                const _Float16* __restrict__ weight, _Float16* __restrict__ norm_out, float eps) {
+  typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+  __shared__ float s_part[kNormThreads / 64];
+  const int tid = threadIdx.x, threads = blockDim.x, chunks = N >> 3;
+  const size_t row = (size_t)blockIdx.x * N;
+  h8 v[kNormTurns];
+  float a = 0.f;
+#pragma unroll
+  for (int i = 0; i < kNormTurns; ++i) {
+    const int c = tid + i * threads;
+    if (c >= chunks) break;
+    const size_t at = row + 8 * (size_t)c;
+    const f32x4 lo = sum_splits(partial + at, split_stride, splits), hi = sum_splits(partial + at + 4, split_stride, splits);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) v[i][k] = (_Float16)(k < 4 ? lo[k] : hi[k - 4]);
+    if (residual) {
+      const h8 res = *reinterpret_cast<const h8*>(residual + at);
+#pragma unroll
+      for (int k = 0; k < 8; ++k) v[i][k] = (_Float16)((float)v[i][k] + (float)res[k]);
+    }
+    *reinterpret_cast<h8*>(y + at) = v[i];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) a = fmaf((float)v[i][k], (float)v[i][k], a);
+  }
+#pragma unroll
+  for (int m = 1; m < 64; m <<= 1) a += __shfl_xor(a, m, 64);
+  if ((tid & 63) == 0) s_part[tid >> 6] = a;
+  __syncthreads();
+  float ss = 0.f;
+  for (int k = 0; k < threads >> 6; ++k) ss += s_part[k];
+  const float r = 1.0f / sqrtf(ss * (1.0f / (float)N) + eps);
+#pragma unroll
+  for (int i = 0; i < kNormTurns; ++i) {
+    const int c = tid + i * threads;
+    if (c >= chunks) break;
+    const h8 w = *reinterpret_cast<const h8*>(weight + 8 * (size_t)c);
+    h8 o;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) o[k] = (_Float16)((float)v[i][k] * r * (float)w[k]);
+    *reinterpret_cast<h8*>(norm_out + row + 8 * (size_t)c) = o;
+  }
+}
+
 // The same for gate | up: y[m, n] of N / 2 columns from the sums of columns n and N / 2 + n.
 __global__ __launch_bounds__(256) void gemm_w4a16_combine_swiglu_kernel(const float* __restrict__ partial, _Float16* y, int rows, int N,
                                                                          int splits) {
@@ -356,7 +406,22 @@ Plan choose(int M, int K, int N, size_t scratch_bytes, int compute_units, int co
   }
   return best;
 }
-int combine(const float* partial, _Float16* y, int rows, int N, int splits, const _Float16* residual, bool swiglu, hipStream_t stream) {
+// An RMSNorm of the result: out = fp16(y / rms(y) * weight).
+struct Norm {
+  const void* weight;
+  void* out;
+  float eps;
+};
+
+int combine(const float* partial, _Float16* y, int rows, int N, int splits, const _Float16* residual, bool swiglu, const Norm* norm,
+            hipStream_t stream) {
+  if (norm) {
+    const int threads = N < 8 * kNormThreads ? (N / 8 + 63) / 64 * 64 : kNormThreads;
+    gemm_w4a16_combine_norm_kernel<<<dim3(rows), threads, 0, stream>>>(partial, y, N, (long long)rows * N, splits, residual,
+                                                                            (const _Float16*)norm->weight, (_Float16*)norm->out, norm->eps);
+    ART_LAUNCH_CHECK();
+    return 0;
+  }
   if (swiglu) {
     gemm_w4a16_combine_swiglu_kernel<<<dim3((unsigned)(((long long)rows * (N / 8) + 255) / 256)), 256, 0, stream>>>(partial, y, rows, N, splits);
     ART_LAUNCH_CHECK();
@@ -369,7 +434,7 @@ int combine(const float* partial, _Float16* y, int rows, int N, int splits, cons
 }
 
 int run(const void* x_dev, const void* qweight_dev, const void* scales_dev, const void* qzeros_dev, void* y_dev, const void* residual_dev,
-        int M, int K, int N, int k_splits, bool swiglu, void* stream) {
+        int M, int K, int N, int k_splits, bool swiglu, const Norm* norm, void* stream) {
   const int n_out = swiglu ? N / 2 : N;
   const int code = k_splits >> 8;                   // 0: library's choice; else rows of a block / 32, 5: 128 rows x 128 columns
   ART_REQUIRE(k_splits >= 0 && (code <= 2 || code == 4 || code == 5 || code == 8),
@@ -391,6 +456,10 @@ int run(const void* x_dev, const void* qweight_dev, const void* scales_dev, cons
   const _Float16* xs = (const _Float16*)x_dev;
   const _Float16* res = (const _Float16*)residual_dev;
   _Float16* ys = (_Float16*)y_dev;
+  // Where K-splits meet in a pass of their own, the norm is part of that pass, up to 256 rows: beyond them
+  // nothing is gained (8 layers of 4096 columns: 966 -> 944 us at 100 rows, 1881 -> 1879 at 300).
+  const bool norm_there = norm && p.splits > 1 && M <= 256 && N % 8 == 0 && N <= 8 * kNormThreads * kNormTurns &&
+                          (((uintptr_t)y_dev | (uintptr_t)residual_dev | (uintptr_t)norm->weight | (uintptr_t)norm->out) % 16) == 0;
   if (p.wide) {
     if (art::w4::gemm_wide(xs, (const unsigned char*)qweight_dev, (const _Float16*)scales_dev, (const unsigned char*)qzeros_dev, ys, scratch, M,
                            K, N, p.splits, p.row_tiles, res, swiglu, st))
@@ -418,7 +487,8 @@ int run(const void* x_dev, const void* qweight_dev, const void* scales_dev, cons
                                                            (const unsigned char*)qzeros_dev, ys, scratch, M, K, N, work, kMagic, res);
     ART_LAUNCH_CHECK();
   }
-  return p.splits > 1 ? combine(scratch, ys, M, N, p.splits, res, swiglu, st) : 0;
+  if (p.splits > 1 && combine(scratch, ys, M, N, p.splits, res, swiglu, norm_there ? norm : nullptr, st)) return 1;
+  return norm && !norm_there ? art_rmsnorm(y_dev, nullptr, norm->weight, norm->out, M, N, 1.0f / (float)N, norm->eps, 1, 1, 1, stream) : 0;
 }
 
 }  // namespace
@@ -435,11 +505,25 @@ extern "C" int art_gemm_w4a16_tuned(const void* x_dev, const void* qweight_dev, 
 
 extern "C" int art_gemm_w4a16_residual(const void* x_dev, const void* qweight_dev, const void* scales_dev, const void* qzeros_dev,
                                        void* y_dev, const void* residual_dev, int M, int K, int N, int k_splits, void* stream) {
-  return run(x_dev, qweight_dev, scales_dev, qzeros_dev, y_dev, residual_dev, M, K, N, k_splits, false, stream);
+  return run(x_dev, qweight_dev, scales_dev, qzeros_dev, y_dev, residual_dev, M, K, N, k_splits, false, nullptr, stream);
 }
 
 extern "C" int art_gemm_w4a16_swiglu(const void* x_dev, const void* qweight_dev, const void* scales_dev, const void* qzeros_dev,
                                      void* y_dev, int M, int K, int N, int k_splits, void* stream) {
   ART_REQUIRE(N % 32 == 0, "art_gemm_w4a16_swiglu: the gate and up halves must be multiples of 16 columns (N=%d)", N);
-  return run(x_dev, qweight_dev, scales_dev, qzeros_dev, y_dev, nullptr, M, K, N, k_splits, true, stream);
+  return run(x_dev, qweight_dev, scales_dev, qzeros_dev, y_dev, nullptr, M, K, N, k_splits, true, nullptr, stream);
+}
+
+extern "C" int art_gemm_w4a16_residual_norm(const void* x_dev, const void* qweight_dev, const void* scales_dev, const void* qzeros_dev,
+                                            void* y_dev, const void* residual_dev, const void* norm_weight_dev, void* norm_out_dev, int M, int K,
+                                            int N, float eps, int k_splits, void* stream) {
+  ART_REQUIRE(norm_weight_dev && norm_out_dev, "art_gemm_w4a16_residual_norm: null pointer");
+  ART_REQUIRE((((uintptr_t)norm_weight_dev | (uintptr_t)norm_out_dev) % 2) == 0, "art_gemm_w4a16_residual_norm: misaligned tensor");
+  ART_REQUIRE(!art::overlaps(norm_out_dev, (size_t)M * N * 2, y_dev, (size_t)M * N * 2) &&
+                  !art::overlaps(norm_out_dev, (size_t)M * N * 2, residual_dev, residual_dev ? (size_t)M * N * 2 : 0) &&
+                  !art::overlaps(norm_out_dev, (size_t)M * N * 2, norm_weight_dev, (size_t)N * 2) &&
+                  !art::overlaps(norm_out_dev, (size_t)M * N * 2, x_dev, (size_t)M * K * 2),
+              "art_gemm_w4a16_residual_norm: the normalised result must not overlap an operand or the result");
+  const Norm norm{norm_weight_dev, norm_out_dev, eps};
+  return run(x_dev, qweight_dev, scales_dev, qzeros_dev, y_dev, residual_dev, M, K, N, k_splits, false, &norm, stream);
 }

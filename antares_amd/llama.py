@@ -297,7 +297,7 @@ class LlamaInt4Decoder:
         prompt (`attention_causal_f16`, matrix cores), keys and values land in cache rows 0..T-1.  Leaves the step
         state at the last prompt position (self.pos = T - 1, self.x = its hidden state, self.logits = its logits), so
         `advance()` and the recorded decode step continue from there.  Same operators and roundings as the one-token
-        step, applied to T rows.  With ``graph`` the pass is recorded once per prompt length in a HIP graph (about 420
+        step, applied to T rows.  With ``graph`` the pass is recorded once per prompt length in a HIP graph (about 360
         launches) and replayed on later calls with the new tokens copied into the recorded input."""
         T = int(tokens.numel())
         if not 4 <= T <= self.cfg.max_seq:
@@ -341,23 +341,25 @@ class LlamaInt4Decoder:
         def linear(inp, lin, out):
             self.gemv(inp, lin['qweight'], lin['scales'], lin['qzeros'], out=out)
 
-        def gemm_res(inp, lin, acc):    # acc += inp @ W, the residual add folded into the projection
-            self.autort.ops.gemm_w4a16_residual(inp, lin['qweight'], lin['scales'], lin['qzeros'], acc, residual=acc)
+        def gemm_res(inp, lin, acc, norm_weight):    # acc += inp @ W -> the RMSNorm in front of the next projection
+            return self.autort.ops.gemm_w4a16_residual_norm(inp, lin['qweight'], lin['scales'], lin['qzeros'], acc, norm_weight, residual=acc,
+                                                            eps=cfg.rms_eps)
 
-        def rms(inp, weight):           # the built-in operator takes rows: one launch for the T positions
-            return self.autort.ops.rmsnorm_f16(inp, None, weight, extra=[1.0 / d, cfg.rms_eps])
-
-        for l, lw in enumerate(self.w['layers']):
-            xb = rms(x, lw['att_norm'])
+        layers = self.w['layers']
+        # the built-in operator takes rows: one launch for the T positions
+        xb = self.autort.ops.rmsnorm_f16(x, None, layers[0]['att_norm'], extra=[1.0 / d, cfg.rms_eps])
+        for l, lw in enumerate(layers):
             linear(xb, lw['qkv'], qkv)
             self.autort.ops.rope_qkv_store_rows_f16(qkv, self.inv_freq, qr, self.key_cache[l], self.val_cache[l])
             att = self.autort.ops.attention_causal_f16(qr, self.key_cache[l].view(cfg.max_seq, H, D),
                                                        self.val_cache[l].view(cfg.max_seq, H, D), self.att_f)
-            gemm_res(att.view(T, d), lw['o'], x)
-            xb = rms(x, lw['ffn_norm'])
-            gu = lw['gate_up']
+            xb = gemm_res(att.view(T, d), lw['o'], x, lw['ffn_norm'])
+            gu, down = lw['gate_up'], lw['down']
             self.autort.ops.gemm_w4a16_swiglu(xb, gu['qweight'], gu['scales'], gu['qzeros'], hid)
-            gemm_res(hid, lw['down'], x)
+            if l + 1 < len(layers):
+                xb = gemm_res(hid, down, x, layers[l + 1]['att_norm'])
+            else:                       # the final norm is folded into the last projection
+                self.autort.ops.gemm_w4a16_residual(hid, down['qweight'], down['scales'], down['qzeros'], x, residual=x)
         self.x.copy_(x[T - 1])
         self.pos.fill_(T - 1)
         self.token.copy_(tokens.view(T)[T - 1:T])

@@ -153,6 +153,11 @@ int art_partition_even_first_i32_tuned(const void* in_dev, void* out_dev, long l
  * into the last pass: y = fp16(fp16(product) + residual).  residual_dev: fp16 [M,N], may be y itself, may be NULL. */
 int art_gemm_w4a16_residual(const void* x_dev, const void* qweight_dev, const void* scales_dev, const void* qzeros_dev,
                             void* y_dev, const void* residual_dev, int M, int K, int N, int k_splits, void* stream);
+/* ... and with the RMSNorm in front of the next projection behind it (:150): norm_out = fp16(y / sqrt(mean(y^2) + eps) *
+ * norm_weight), both fp16; norm_out [M,N] overlaps none of the other tensors. */
+int art_gemm_w4a16_residual_norm(const void* x_dev, const void* qweight_dev, const void* scales_dev, const void* qzeros_dev, void* y_dev,
+                                 const void* residual_dev, const void* norm_weight_dev, void* norm_out_dev, int M, int K, int N, float eps,
+                                 int k_splits, void* stream);
 /* The same product with a gate | up matrix (N/2 columns each, N % 32 == 0): y[M, N/2] = fp16(silu(fp16(gate)) * fp16(up)),
  * i.e. the projection and the SwiGLU behind it (samples/05_llama2_7b_int4.py:171) for a batch of rows. */
 int art_gemm_w4a16_swiglu(const void* x_dev, const void* qweight_dev, const void* scales_dev, const void* qzeros_dev,

@@ -1244,3 +1244,39 @@ def test_convolution_operator_takes_the_kernel_and_agrees_with_the_generic_one(a
     assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf())
     fin = want.isfinite()
     assert ((got - want)[fin].norm() / want[fin].norm()).item() < 2.0 ** -23 * 9 * c       # float32 sums of 9 c terms, another order
+
+
+# with and without K-splits, one and two turns of a block, a row that is not whole 16-byte pieces of 8 (two launches)
+@pytest.mark.parametrize('M,K,N', [(1, 256, 16), (5, 512, 272), (33, 1024, 4096), (130, 640, 8192), (20, 512, 8208), (300, 256, 144)])
+def test_w4a16_gemm_with_residual_and_rmsnorm_behind_it(autort, M, K, N):
+    """gemm_w4a16_residual_norm gives gemm_w4a16_residual's result bit for bit, and its RMSNorm: the square root's argument is
+    a float32 sum in another order (N 2^-24 at most), the result is rounded to float16 (2^-11)."""
+    from ctypes import c_void_p
+    from antares_amd.runtime import capi
+    dev = autort.device()
+    capi.init(0)
+    p = workloads.w4_problem(K + N + M, M, K, N)
+    d = [p[k].to(dev) for k in ('x', 'qweight', 'scales', 'qzeros')]
+    g = torch.Generator().manual_seed(M)
+    res, weight = torch.randn(M, N, generator=g).half().to(dev), (torch.randn(N, generator=g) * 0.1 + 1).half().to(dev)
+    stream = c_void_p(torch.cuda.current_stream().cuda_stream)
+    for code in (0, 256 + 1, 256 + 2, 512 + 3, 1024 + 2, 2048 + 1):
+        for residual in (None, res):
+            note(f'w4a16 gemm + residual + norm M={M} K={K} N={N} code {code} {"with" if residual is not None else "no"} residual')
+            want, got, norm = (torch.full((M, N), float('nan'), dtype=torch.float16, device=dev) for _ in range(3))
+            ptr = [c_void_p(t.data_ptr()) for t in d]
+            r = c_void_p(residual.data_ptr() if residual is not None else 0)
+            capi.check(capi.lib().art_gemm_w4a16_residual(*ptr, c_void_p(want.data_ptr()), r, M, K, N, code, stream))
+            capi.check(capi.lib().art_gemm_w4a16_residual_norm(*ptr, c_void_p(got.data_ptr()), r, c_void_p(weight.data_ptr()), c_void_p(norm.data_ptr()),
+                                                               M, K, N, 1e-5, code, stream))
+            assert torch.equal(got, want)
+            y = want.cpu().double()
+            exact = y / torch.sqrt((y * y).mean(1, keepdim=True) + 1e-5) * weight.cpu().double()
+            assert ((norm.cpu().double() - exact).abs() <= exact.abs() * (2.0 ** -11 + N * 2.0 ** -24) + 2.0 ** -24).all()
+    acc = res.clone()
+    out = autort.ops.gemm_w4a16_residual_norm(*d, acc, weight, residual=acc)
+    plain = res.clone()
+    autort.ops.gemm_w4a16_residual(*d, plain, residual=plain)
+    assert torch.equal(acc, plain) and torch.equal(out, autort.ops.gemm_w4a16_residual_norm(*d, res.clone(), weight, residual=res))
+    assert capi.lib().art_gemm_w4a16_residual_norm(*ptr, c_void_p(acc.data_ptr()), None, c_void_p(weight.data_ptr()), c_void_p(acc.data_ptr()),
+                                                   M, K, N, 1e-5, 0, stream) != 0
