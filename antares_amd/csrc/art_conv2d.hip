@@ -356,6 +356,9 @@ extern "C" int art_conv2d(const void* x_dev, const void* w_dev, void* packed_dev
   const uintptr_t size = f16 ? 2 : 4;
   ART_REQUIRE((uintptr_t)x_dev % size == 0 && (uintptr_t)w_dev % size == 0 && (uintptr_t)packed_dev % 16 == 0 && (uintptr_t)y_dev % 4 == 0,
               "art_conv2d: misaligned tensor");
+  ART_REQUIRE(!art::overlaps(y_dev, (size_t)N * F * HO * WO * 4, x_dev, (size_t)N * C * H * W * size) &&
+                  !art::overlaps(y_dev, (size_t)N * F * HO * WO * 4, w_dev, (size_t)F * C * 9 * size),
+              "art_conv2d: the result must not overlap an operand");
   g.row_blocks = (F + features_of(form) - 1) / features_of(form);
   g.row_tiles = g.row_blocks * (features_of(form) / 32);
   g.span = span_of(g, points_of(form));
