@@ -60,7 +60,9 @@ struct Recipe {
   int slots;
   std::vector<Alloc> allocs;
   std::vector<Launch> launches;
+  std::vector<std::pair<int, bool>> numbers;             // slots whose numbers are passed on; true: as a float
   std::vector<int> results;
+  bool uses_stream;
 };
 
 struct Operator {
@@ -194,6 +196,20 @@ int call_library(void* fn, const uint64_t* a, const float* f) {
                  a[18], a[19], f[0], f[1], f[2], f[3]);
 }
 
+// A number of the call as an entry point takes it: what the Python method's int() or float() of it and ctypes' c_int or
+// c_float make of that, errors included - whatever kind of number the call that left the recipe had there.
+bool pass_number(PyObject* o, bool as_float, uint64_t& i, float& f) {
+  if (as_float) {
+    f = (float)PyFloat_AsDouble(o);
+  } else if (PyLong_Check(o)) {
+    i = (uint64_t)PyLong_AsUnsignedLongLongMask(o);
+  } else if (PyObject* whole = PyNumber_Long(o)) {
+    i = (uint64_t)PyLong_AsUnsignedLongLongMask(whole);
+    Py_DECREF(whole);
+  }
+  return !PyErr_Occurred();
+}
+
 PyObject* execute(const std::shared_ptr<Recipe>& keep, const Slots& s) {
   const Recipe& r = *keep;
   at::Tensor fresh[kMaxSlots];
@@ -203,18 +219,10 @@ PyObject* execute(const std::shared_ptr<Recipe>& keep, const Slots& s) {
   for (int i = 0; i < s.n; ++i) {
     pointer[i] = 0;
     PyObject* o = s.obj[i];
-    if (o == nullptr || o == Py_None) continue;
-    if (is_tensor(o)) {
-      pointer[i] = (uint64_t)(uintptr_t)THPVariable_Unpack(o).const_data_ptr();
-    } else if (PyLong_Check(o)) {
-      slot_int[i] = (uint64_t)PyLong_AsLongLong(o);
-      slot_float[i] = (float)PyLong_AsDouble(o);
-      if (PyErr_Occurred()) return nullptr;
-    } else if (PyFloat_Check(o)) {
-      slot_float[i] = (float)PyFloat_AS_DOUBLE(o);
-      slot_int[i] = 0;
-    }
+    if (o && is_tensor(o)) pointer[i] = (uint64_t)(uintptr_t)THPVariable_Unpack(o).const_data_ptr();
   }
+  for (const auto& n : r.numbers)
+    if (!pass_number(s.obj[n.first], n.second, slot_int[n.first], slot_float[n.first])) return nullptr;
   try {
     for (size_t i = 0; i < r.allocs.size(); ++i) {
       fresh[i] = at::Tensor(at::detail::empty_cuda(r.allocs[i].sizes, r.allocs[i].dtype, at::Device(at::kCUDA, (c10::DeviceIndex)r.device), std::nullopt));
@@ -230,7 +238,7 @@ PyObject* execute(const std::shared_ptr<Recipe>& keep, const Slots& s) {
     Py_XDECREF(type);
     return nullptr;
   }
-  const uint64_t stream = (uint64_t)(uintptr_t)c10::hip::getCurrentHIPStream(r.device_stream ? (c10::DeviceIndex)r.device : (c10::DeviceIndex)-1).stream();
+  const uint64_t stream = !r.uses_stream ? 0 : (uint64_t)(uintptr_t)c10::hip::getCurrentHIPStream(r.device_stream ? (c10::DeviceIndex)r.device : (c10::DeviceIndex)-1).stream();
   int rc = 0;
   Py_BEGIN_ALLOW_THREADS
   for (const Launch& l : r.launches) {
@@ -350,6 +358,7 @@ PyObject* operator_commit(PyObject* self, PyObject* args) {
   r->config_version = version_of(op->config);
   r->device = device;
   r->device_stream = device_stream != 0;
+  r->uses_stream = false;
   r->slots = slots;
   if (!PyList_Check(allocs) || !PyList_Check(launches) || !PyList_Check(results) || PyList_GET_SIZE(allocs) > kMaxSlots) {
     PyErr_SetString(PyExc_TypeError, "commit: allocs (at most 24), launches and results are lists");
@@ -373,6 +382,7 @@ PyObject* operator_commit(PyObject* self, PyObject* args) {
     Launch l;
     l.fn = (void*)(uintptr_t)fn;
     l.kernel = grid != Py_None;
+    r->uses_stream |= l.kernel;
     if (l.kernel && (!PyArg_ParseTuple(grid, "III", &l.grid[0], &l.grid[1], &l.grid[2]) || !PyArg_ParseTuple(block, "III", &l.block[0], &l.block[1], &l.block[2])))
       return nullptr;
     int ints = 0, floats = 0;
@@ -381,7 +391,7 @@ PyObject* operator_commit(PyObject* self, PyObject* args) {
       PyObject* v = nullptr;
       if (!PyArg_ParseTuple(PyList_GET_ITEM(list, k), "C|O", &kind, &v)) return nullptr;
       Arg g{};
-      if (kind == 's') g.kind = Arg::kStream;
+      if (kind == 's') { g.kind = Arg::kStream; r->uses_stream = true; }
       else if (kind == 'i') { g.kind = Arg::kInt; g.i = (uint64_t)PyLong_AsUnsignedLongLongMask(v); }
       else if (kind == 'f') { g.kind = Arg::kFloat; g.f = (float)PyFloat_AsDouble(v); }
       else {
@@ -389,6 +399,7 @@ PyObject* operator_commit(PyObject* self, PyObject* args) {
         g.index = (int)PyLong_AsLong(v);
         if (!PyErr_Occurred() && (g.index < 0 || g.index >= (kind == 'p' ? tensors : slots)))
           PyErr_SetString(PyExc_IndexError, "commit: an argument refers to a slot that does not exist");
+        else if (kind != 'p') r->numbers.emplace_back(g.index, g.kind == Arg::kSlotFloat);
       }
       if (PyErr_Occurred()) return nullptr;
       (g.kind == Arg::kFloat || g.kind == Arg::kSlotFloat ? floats : ints)++;

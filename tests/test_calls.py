@@ -1,0 +1,63 @@
+"""Calls replayed in native code, as far as that needs no GPU: what a recipe passes on to an entry point (here a
+recording callback), with arguments that are numbers."""
+import ctypes
+
+import pytest
+
+from antares_amd.runtime import calls
+
+
+class Recording(calls.Operator):
+    """Passes the numbers of `extra` on to a callback: as whole numbers, or as floats."""
+
+    def __init__(self, kind='I', during=None):
+        self.kind, self.seen, self.python_calls = kind, [], 0
+
+        def entry(*values):
+            self.seen.append(values[0])
+            if during is not None:
+                during()
+            return 0
+        # whole numbers are int arguments of the library's entry points
+        self.entry = ctypes.CFUNCTYPE(ctypes.c_int, ctypes.c_int if kind == 'I' else ctypes.c_float)(entry)
+        self._bind(('x', 'extra'), ('extra',))
+
+    def _call(self, pending, x=None, extra=None):
+        self.python_calls += 1
+        value = int(extra[0]) if self.kind == 'I' else float(extra[0])
+        call = calls.Call(0)
+        call.library(self.entry, calls.Number(value, 2, self.kind))
+        call.keep(self, pending, [], device_stream=False)
+
+
+@pytest.mark.parametrize('values', [(5, 6, 2 ** 31 - 1, -1, 0), (5.0, 6.0, 7.9, -7.9, 0.0), (True, False, True)])
+def test_a_whole_number_is_passed_on_whatever_kind_of_number_it_is(values):
+    op = Recording('I')
+    for v in values:
+        op(None, extra=[v])
+        op(extra=(v,))
+    assert op.seen == [int(v) for v in values for _ in range(2)]
+
+
+def test_a_position_that_changes_its_kind():
+    op = Recording('I')
+    for v in (5, 6.0, 7, 8.0, 9.5, True, 10):
+        op(None, extra=[v])
+    assert op.seen == [5, 6, 7, 8, 9, 1, 10]
+
+
+def test_a_float_is_passed_on_whatever_kind_of_number_it_is():
+    op = Recording('F')
+    for v in (0.5, 0.25, 3, 4, 1e30):
+        op(None, extra=[v])
+    assert op.seen == [ctypes.c_float(float(v)).value for v in (0.5, 0.25, 3, 4, 1e30)]
+
+
+def test_a_number_that_is_none_raises_what_it_raises_at_the_first_call():
+    op = Recording('I')
+    for first in (True, False):
+        for v, error in ((float('nan'), ValueError), (float('inf'), OverflowError), (-float('inf'), OverflowError)):
+            with pytest.raises(error):
+                op(None, extra=[v])
+        op(None, extra=[3.0])
+    assert op.python_calls == 4 and op.seen == [3, 3]

@@ -94,3 +94,24 @@ def test_several_threads_call_one_operator(op):
     for t in threads:
         t.join()
     assert not wrong
+
+
+# a position is taken by its value in every call, also where an earlier call of the signature had another kind of number
+@pytest.mark.parametrize('positions', [(5.0, 6.0, 77.9), (5, 6.0, 7, True, 8.0)])
+@pytest.mark.parametrize('name', ['rotary_f32', 'rotate_f32'])
+def test_a_position_may_be_any_number(name, positions):
+    import autort
+    print(f'[case] {name} {positions}', flush=True)
+    dev = autort.device()
+    x, inv = torch.randn(2, 2, 64, device=dev), torch.rand(128, device=dev)
+    for pos in positions:
+        angle = float(int(pos)) * inv[:64]
+        if name == 'rotary_f32':
+            want = torch.cat([x[:, 0] * angle.cos() - x[:, 1] * angle.sin(), x[:, 1] * angle.cos() + x[:, 0] * angle.sin()], 1)
+            got = autort.ops.rotary_f32(x, inv, torch.empty(2, 128, device=dev), extra=[pos])
+        else:
+            data = x.view(2, 128)[0]
+            re, im = data[0::2], data[1::2]
+            want = torch.stack([re * angle.cos() - im * angle.sin(), im * angle.cos() + re * angle.sin()], 1).view(128)
+            got = autort.ops.rotate_f32(inv[:64].view(1, 64), data, torch.empty(128, device=dev), extra=[pos])
+        assert torch.allclose(got, want, rtol=1e-4, atol=1e-4)
