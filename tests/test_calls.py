@@ -3,7 +3,9 @@ recording callback), with arguments that are numbers."""
 import ctypes
 
 import pytest
+import torch
 
+from antares_amd.autort import builtin_ops
 from antares_amd.runtime import calls
 
 
@@ -61,3 +63,23 @@ def test_a_number_that_is_none_raises_what_it_raises_at_the_first_call():
                 op(None, extra=[v])
         op(None, extra=[3.0])
     assert op.python_calls == 4 and op.seen == [3, 3]
+
+
+def test_a_number_given_as_a_tensor_leaves_no_recipe(monkeypatch):
+    """The value of a tensor that no launch takes may be part of the call's constants: the next call has another one."""
+    monkeypatch.setattr(builtin_ops, 'current_stream_handle', lambda: 0)
+    kept = []
+    monkeypatch.setattr(calls.Call, 'keep', lambda self, *a, **k: kept.append(self))
+    entry = ctypes.CFUNCTYPE(ctypes.c_int, ctypes.c_void_p, ctypes.c_int, ctypes.c_void_p)(lambda *a: 0)
+    x, out, number, empty = torch.ones(4), torch.empty(4), torch.tensor([3]), torch.empty(0)
+
+    def run(slots, *args):
+        kept.clear()
+        builtin_ops._run(None, None if slots is None else (b'', slots, -1), out, entry, *args)
+        return len(kept)
+    assert run((x, out), x, 3) == 1
+    assert run((x, out, [5], 5), x, calls.Number(5, 3, 'I')) == 1
+    assert run((x, None, empty), x, 3) == 1               # a tensor without elements has no value
+    assert run((x, out, [number], number), x, int(number)) == 0
+    assert run((x, number, out), x, int(number)) == 0
+    assert run(None, x, 3) == 0

@@ -115,3 +115,20 @@ def test_a_position_may_be_any_number(name, positions):
             want = torch.stack([re * angle.cos() - im * angle.sin(), im * angle.cos() + re * angle.sin()], 1).view(128)
             got = autort.ops.rotate_f32(inv[:64].view(1, 64), data, torch.empty(128, device=dev), extra=[pos])
         assert torch.allclose(got, want, rtol=1e-4, atol=1e-4)
+
+
+def test_a_number_given_as_a_tensor_is_read_in_every_call():
+    import autort
+    dev = autort.device()
+    x, w = torch.randn(256, device=dev), torch.randn(256, device=dev)
+    vsum = (x * x).sum().view(1)
+    for inv_n in (1 / 256, 1 / 64, 1.0):
+        want = x * torch.rsqrt(vsum * inv_n + 1e-5) * w
+        for extra in ([torch.tensor(inv_n, device=dev)], [torch.tensor([inv_n], device=dev), 1e-5]):
+            assert torch.allclose(autort.ops.rmsnorm_f32(x, vsum, w, extra=extra), want, rtol=1e-4, atol=1e-5)
+    qkv, inv = torch.randn(3, 3 * 256, device=dev).half(), torch.rand(128, device=dev).half()
+    for first in (0, 2, 5):
+        got, want = ([torch.zeros(3, 2, 128, device=dev).half()] + [torch.zeros(8, 256, device=dev).half() for _ in range(2)] for _ in range(2))
+        autort.ops.rope_qkv_store_rows_f16(qkv, inv, *got, extra=[torch.tensor([first], device=dev)])
+        autort.ops.rope_qkv_store_rows_f16(qkv, inv, *want, extra=[first])
+        assert all(torch.equal(a, b) for a, b in zip(got, want)) and torch.equal(got[2][first:first + 3], qkv[:, 512:])
