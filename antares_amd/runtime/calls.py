@@ -64,6 +64,10 @@ class Number:
         self.value, self.slot, self.kind = value, slot, kind
 
 
+class _ViewOfAnArgument(Exception):
+    pass
+
+
 class Call:
     """What one call of an operator launches, in order: kernels and entry points of the library, with tensors as
     tensors, the stream as STREAM, list numbers as Number, and constants."""
@@ -84,7 +88,7 @@ class Call:
 
     def keep(self, op: Operator, pending, results, device_stream: bool):
         """Leaves the recipe of this call with the operator.  Tensors that are not among the call's arguments are
-        allocated afresh by every later call."""
+        allocated afresh by every later call; a view of an argument is neither, and a call that uses one leaves no recipe."""
         if pending is None:
             return
         setup()
@@ -100,7 +104,7 @@ class Call:
             at = place.get(id(t))
             if at is None:
                 if t.numel() and t.untyped_storage().data_ptr() in owned:
-                    raise RuntimeError('a recipe takes its arguments as they were passed, not views of them')
+                    raise _ViewOfAnArgument
                 at = place[id(t)] = len(slots) + len(fresh)
                 fresh.append(t)
             return at
@@ -116,9 +120,12 @@ class Call:
                 return ('f', a)
             return ('i', int(a or 0))
         launches = []
-        for fn, grid, block, args in self.steps:
-            address = fn.value if grid is not None else ctypes.cast(fn, c_void_p).value
-            launches.append((address, grid, block, [encode(fn, a) for a in args]))
-        outs = [index(t) for t in results]
+        try:
+            for fn, grid, block, args in self.steps:
+                address = fn.value if grid is not None else ctypes.cast(fn, c_void_p).value
+                launches.append((address, grid, block, [encode(fn, a) for a in args]))
+            outs = [index(t) for t in results]
+        except _ViewOfAnArgument:
+            return
         if len(fresh) <= 16:
             op._commit(key, len(slots), device, int(device_stream), [(t.dtype, tuple(t.shape)) for t in fresh], launches, outs)

@@ -83,3 +83,23 @@ def test_a_number_given_as_a_tensor_leaves_no_recipe(monkeypatch):
     assert run((x, out, [number], number), x, int(number)) == 0
     assert run((x, number, out), x, int(number)) == 0
     assert run(None, x, 3) == 0
+
+
+def test_a_view_of_an_argument_leaves_no_recipe(monkeypatch):
+    monkeypatch.setattr(calls, 'setup', lambda: None)
+    kept = []
+
+    class Keeping:
+        def _commit(self, *recipe):
+            kept.append(recipe)
+    entry = ctypes.CFUNCTYPE(ctypes.c_int, ctypes.c_void_p)(lambda *a: 0)
+    x, fresh = torch.ones(4), torch.empty(4)
+
+    def keep(arg, result):
+        kept.clear()
+        call = calls.Call(0)
+        call.library(entry, arg)
+        call.keep(Keeping(), (b'', (x,), -1), [result], device_stream=False)
+        return len(kept)
+    assert keep(x, fresh) == 1 and keep(fresh, x) == 1 and keep(x[:0], x) == 1
+    assert keep(x[:2], fresh) == 0 and keep(x, x[1:]) == 0 and keep(x.view(2, 2), fresh) == 0

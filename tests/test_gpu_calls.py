@@ -132,3 +132,12 @@ def test_a_number_given_as_a_tensor_is_read_in_every_call():
         autort.ops.rope_qkv_store_rows_f16(qkv, inv, *got, extra=[torch.tensor([first], device=dev)])
         autort.ops.rope_qkv_store_rows_f16(qkv, inv, *want, extra=[first])
         assert all(torch.equal(a, b) for a, b in zip(got, want)) and torch.equal(got[2][first:first + 3], qkv[:, 512:])
+
+
+def test_a_tensor_of_positions_in_the_place_of_the_list():
+    import autort
+    dev = autort.device()
+    x, inv = torch.randn(2, 2, 64, device=dev), torch.rand(128, device=dev)
+    for pos in (3, 4):
+        got = autort.ops.rotary_f32(x, inv, torch.empty(2, 128, device=dev), extra=torch.tensor([pos], dtype=torch.int32, device=dev))
+        assert torch.equal(got, autort.ops.rotary_f32(x, inv, torch.empty(2, 128, device=dev), extra=[pos]))
