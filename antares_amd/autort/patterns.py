@@ -397,6 +397,8 @@ def _conv2d_handler(st, axes, window):
                 tuple(w.shape) != (e['f'], e['c'], e['kh'], e['kw']) or \
                 (e['kh'], e['kw']) != (3, 3) or not x.numel() or not y.numel():
             return False
+        if op.fused.shape_of(op.fast_roles['y'], env) != [e[part] for part in ('n', 'f', 'ho', 'wo')]:
+            return False                          # the kernel stores a dense result, not a part of a larger one
         # The kernel reads zeros outside the image and the image everywhere else: that has to be what the guards say, and
         # an index without a guard on one side must not reach past it.
         for key, size in (('h', x.shape[2]), ('w', x.shape[3])):

@@ -1280,3 +1280,23 @@ def test_w4a16_gemm_with_residual_and_rmsnorm_behind_it(autort, M, K, N):
     assert torch.equal(acc, plain) and torch.equal(out, autort.ops.gemm_w4a16_residual_norm(*d, res.clone(), weight, residual=res))
     assert capi.lib().art_gemm_w4a16_residual_norm(*ptr, c_void_p(acc.data_ptr()), None, c_void_p(weight.data_ptr()), c_void_p(acc.data_ptr()),
                                                    M, K, N, 1e-5, 0, stream) != 0
+
+
+@pytest.mark.parametrize('dtype', ['float16', 'float32'])
+def test_convolution_into_part_of_a_larger_result(autort, dtype):
+    """A declared result that is larger than what the program computes: only its part is written, in its place."""
+    note(f'convolution {dtype} into part of a larger result')
+    dev = autort.device()
+    n, c, f, hw = 4, 64, 64, 28
+    op = autort.export(ir=conv_program(dtype, (hw, hw), (hw, hw), (1, 1)), name=f'conv_part_{dtype}',
+                       inputs=[f'input0={dtype}[N:{n}, C:{c}, H:{hw}, W:{hw}]', f'input1={dtype}[F:{f}, C:{c}, KH:3, KW:3]', 'output0=float32[N, F, A:32, B:30]'])
+    g = torch.Generator().manual_seed(hw)
+    x, w = torch.randn(n, c, hw, hw, generator=g).to(getattr(torch, dtype)), torch.randn(f, c, 3, 3, generator=g).to(getattr(torch, dtype))
+    want, bound = (torch.nn.functional.conv2d(a, b, padding=1) for a, b in ((x.double(), w.double()), (x.double().abs(), w.double().abs())))
+    for size in ((32, 30), (28, 28), (28, 30)):
+        for _ in range(2):
+            y = torch.full((n, f) + size, 7.0, device=dev)
+            op(x.to(dev), w.to(dev), y)
+            got = y.cpu().double()
+            assert ((got[:, :, :hw, :hw] - want).abs() <= 2.0 ** -23 * 9 * c * bound).all()
+            assert (got[:, :, hw:] == 7.0).all() and (got[:, :, :, hw:] == 7.0).all()

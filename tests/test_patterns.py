@@ -1,0 +1,39 @@
+"""Which calls the handlers of hand-written kernels take, decided on the host: no GPU."""
+import pytest
+import torch
+
+from antares_amd.autort.op import ExportedOp
+
+CONV = ('output0[N, F, HO, WO] +=! input0[N, C, HO + KH - 1, WO + KW - 1].when([HO + KH - 1 >= 0, HO + KH - 1 < 28, WO + KW - 1 >= 0, '
+        'WO + KW - 1 < 28], 0.0) * input1[F, C, KH, KW] where HO in 28, WO in 28')
+CONV_INPUTS = ['input0=float32[N:4, C:64, H:28, W:28]', 'input1=float32[F:64, C:64, KH:3, KW:3]']
+
+
+class Launches:
+    def __init__(self):
+        self.taken = []
+
+    def library(self, fn, *args):
+        self.taken.append(fn.__name__)
+
+
+def taken_by(op, *tensors):
+    """What the hand-written kernel's handler launches for these tensors; [] when it leaves the call to the generic kernels."""
+    bound = dict(zip(op.declared + op.fresh_outputs, tensors))
+    env = op.fused.bind_dims({n: tuple(bound[n].shape) for n in op._declared_in_graph})
+    call = Launches()
+    ran = op.fast_path(op, bound, env, call)
+    assert ran == bool(call.taken)
+    return call.taken
+
+
+@pytest.mark.parametrize('spec,shape,dense', [
+    (None, (4, 64, 28, 28), True), (None, (4 * 64 * 28 * 28,), True),                # the program's own result, in any shape
+    ('output0=float32[4, 64, 28, 28]', (4, 64, 28, 28), True),
+    ('output0=float32[N:4, F:64, A:32, B:28]', (4, 64, 32, 28), False), ('output0=float32[N:4, F:64, A:28, B:32]', (4, 64, 28, 32), False),
+    ('output0=float32[N:4, F:64, A:32, B:28]', (4, 64, 28, 28), True),              # of the size of the result in this call
+    ('output0=float32[5, 64, 28, 28]', (5, 64, 28, 28), False), ('output0=float32[4, 65, 28, 28]', (4, 65, 28, 28), False)])
+def test_a_convolution_into_part_of_a_larger_result_is_left_to_the_generic_kernels(spec, shape, dense):
+    op = ExportedOp(CONV, CONV_INPUTS + ([spec] if spec else []), name='conv_part')
+    x, w, y = torch.zeros(4, 64, 28, 28), torch.zeros(64, 64, 3, 3), torch.zeros(shape)
+    assert taken_by(op, x, w, y) == (['art_conv2d'] if dense else [])
