@@ -100,6 +100,10 @@ class ExportedOp(calls.Operator):
             info = self.fused.tensors.get(n) or self.graph.tensors[n]
             self._wanted_dtype[n] = (TORCH_DTYPE[info.dtype], info.dtype)
         self._declared_in_graph = [n for n in self.declared if n in self.fused.tensors]
+        # (declared result, dimension, its extent, how far the program writes along it) wherever the two may differ
+        self._written = [(st.output, i, dim, dict(st.data_axes)[ix.name]) for st in self.fused.statements if st.output in self.inout and not st.scatter
+                         for i, (ix, dim) in enumerate(zip(st.out_index, self.fused.tensors[st.output].shape))
+                         if ix.kind == 'axis' and dict(st.data_axes).get(ix.name, dim) != dim]
         # the call's arguments in order: tensors by position (no keyword has a name that starts with `/`), the last
         # output also as `out`; `extra` is taken and ignored
         self._bind(tuple(['/' + n for n in self.declared + self.fresh_outputs[:-1]] + ['out', 'extra']), ())
@@ -156,6 +160,10 @@ class ExportedOp(calls.Operator):
         if dev.type != 'cuda':
             raise RuntimeError(f'{self.name}(): tensors must live on the GPU (got {dev}); there is no CPU fallback')
         env = g.bind_dims({n: tuple(bound[n].shape) for n in self._declared_in_graph})
+        for n, i, dim, extent in self._written:
+            room, extent = (v if isinstance(v, int) else env[v] for v in (dim, extent))
+            if extent > room:
+                raise ValueError(f'output `{n}` has {room} elements along dimension {i}, {self.name}() writes {extent}')
         for n in self.fresh_outputs:
             want = g.shape_of(n, env)
             if n in bound:

@@ -3,10 +3,23 @@ import pytest
 import torch
 
 from antares_amd.autort.op import ExportedOp
+from antares_amd.runtime import capi
 
 CONV = ('output0[N, F, HO, WO] +=! input0[N, C, HO + KH - 1, WO + KW - 1].when([HO + KH - 1 >= 0, HO + KH - 1 < 28, WO + KW - 1 >= 0, '
         'WO + KW - 1 < 28], 0.0) * input1[F, C, KH, KW] where HO in 28, WO in 28')
 CONV_INPUTS = ['input0=float32[N:4, C:64, H:28, W:28]', 'input1=float32[F:64, C:64, KH:3, KW:3]']
+
+
+class GpuShaped(torch.Tensor):
+    """Dtype, shape and device of a GPU tensor, without one."""
+
+    @staticmethod
+    def __new__(cls, shape):
+        return torch.Tensor._make_wrapper_subclass(cls, shape, dtype=torch.float32, device='cuda:0')
+
+    @classmethod
+    def __torch_dispatch__(cls, func, types, args=(), kwargs=None):
+        raise NotImplementedError(func)
 
 
 class Launches:
@@ -37,3 +50,19 @@ def test_a_convolution_into_part_of_a_larger_result_is_left_to_the_generic_kerne
     op = ExportedOp(CONV, CONV_INPUTS + ([spec] if spec else []), name='conv_part')
     x, w, y = torch.zeros(4, 64, 28, 28), torch.zeros(64, 64, 3, 3), torch.zeros(shape)
     assert taken_by(op, x, w, y) == (['art_conv2d'] if dense else [])
+
+
+@pytest.mark.parametrize('spec,shape,fits', [
+    ('output0=float32[N, F, A, B]', (4, 64, 28, 28), True), ('output0=float32[N, F, A, B]', (4, 64, 30, 29), True),
+    ('output0=float32[N, F, A, B]', (4, 64, 27, 28), False), ('output0=float32[N, F, A, B]', (4, 64, 28, 27), False),
+    ('output0=float32[4, 64, 28, 20]', (4, 64, 28, 20), False), ('output0=float32[3, 64, 28, 28]', (3, 64, 28, 28), False)])
+def test_a_declared_result_too_small_for_the_program_is_refused(monkeypatch, spec, shape, fits):
+    class Checked(Exception):
+        pass
+
+    def init(device):
+        raise Checked
+    monkeypatch.setattr(capi, 'init', init)              # what follows the checks
+    op = ExportedOp(CONV, CONV_INPUTS + [spec], name='conv_room')
+    with pytest.raises(Checked if fits else ValueError):
+        op._call(None, *(GpuShaped(s) for s in ((4, 64, 28, 28), (64, 64, 3, 3), shape)))
