@@ -172,6 +172,8 @@ class ExportedOp(calls.Operator):
             else:
                 bound[n] = torch.empty(want, dtype=self._wanted_dtype[n][0], device=dev)
         capi.init(dev.index or 0)
+        for t in bound.values():
+            calls.address(t)
         call = calls.Call(current_stream_handle(dev.index))
         if self.fast_path is None or not self.fast_path(self, bound, env, call):
             self._run_generic(bound, env, dev, call)

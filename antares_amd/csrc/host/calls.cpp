@@ -11,6 +11,7 @@
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <ATen/hip/EmptyTensor.h>
@@ -102,14 +103,17 @@ bool is_tensor(PyObject* o) { return (PyObject*)Py_TYPE(o) == THPVariableClass |
 
 bool describe_tensor(PyObject* o, Key& key, Slots& s) {
   const at::Tensor& t = THPVariable_Unpack(o);
-  if (t.layout() != at::kStrided || !t.is_cuda() || !t.is_contiguous()) return false;
+  // wrappers of torch.func are plain tensors to Python and have no storage (vmap, grad, jvp) or no memory (functionalize)
+  if (t.layout() != at::kStrided || !t.is_cuda() || !t.has_storage() || !t.is_contiguous()) return false;
+  const uintptr_t address = (uintptr_t)t.const_data_ptr();
+  if (address == 0 && t.numel() != 0) return false;
   const int device = t.device().index();
   if (s.device < 0) s.device = device;
   const auto sizes = t.sizes();
   int first = 0;                                         // one tensor in two places: which place it had first
   while (s.obj[first] != o) ++first;
   if (!key.put(1 | (int64_t)t.scalar_type() << 8 | (int64_t)device << 16 | (int64_t)sizes.size() << 24 |
-               (int64_t)((uintptr_t)t.const_data_ptr() & 15) << 32 | (int64_t)first << 40))
+               (int64_t)(address & 15) << 32 | (int64_t)first << 40))
     return false;
   for (int64_t v : sizes)
     if (!key.put(v)) return false;
@@ -210,38 +214,15 @@ bool pass_number(PyObject* o, bool as_float, uint64_t& i, float& f) {
   return !PyErr_Occurred();
 }
 
-PyObject* execute(const std::shared_ptr<Recipe>& keep, const Slots& s) {
-  const Recipe& r = *keep;
-  at::Tensor fresh[kMaxSlots];
-  uint64_t pointer[2 * kMaxSlots];
-  uint64_t slot_int[kMaxSlots];
-  float slot_float[kMaxSlots];
-  for (int i = 0; i < s.n; ++i) {
-    pointer[i] = 0;
-    PyObject* o = s.obj[i];
-    if (o && is_tensor(o)) pointer[i] = (uint64_t)(uintptr_t)THPVariable_Unpack(o).const_data_ptr();
-  }
-  for (const auto& n : r.numbers)
-    if (!pass_number(s.obj[n.first], n.second, slot_int[n.first], slot_float[n.first])) return nullptr;
-  try {
-    for (size_t i = 0; i < r.allocs.size(); ++i) {
-      fresh[i] = at::Tensor(at::detail::empty_cuda(r.allocs[i].sizes, r.allocs[i].dtype, at::Device(at::kCUDA, (c10::DeviceIndex)r.device), std::nullopt));
-      pointer[s.n + i] = (uint64_t)(uintptr_t)fresh[i].const_data_ptr();
-    }
-  } catch (const std::exception& e) {
-    PyObject* type = nullptr;
-    if (std::string(e.what()).find("out of memory") != std::string::npos) {
-      if (PyObject* torch = PyImport_ImportModule("torch")) { type = PyObject_GetAttrString(torch, "OutOfMemoryError"); Py_DECREF(torch); }
-      PyErr_Clear();
-    }
-    PyErr_SetString(type ? type : PyExc_RuntimeError, e.what());
-    Py_XDECREF(type);
-    return nullptr;
-  }
-  const uint64_t stream = !r.uses_stream ? 0 : (uint64_t)(uintptr_t)c10::hip::getCurrentHIPStream(r.device_stream ? (c10::DeviceIndex)r.device : (c10::DeviceIndex)-1).stream();
-  int rc = 0;
-  Py_BEGIN_ALLOW_THREADS
+struct Unlocked {                                        // other threads run meanwhile, whichever way this scope is left
+  PyThreadState* state = PyEval_SaveThread();
+  ~Unlocked() { PyEval_RestoreThread(state); }
+};
+
+int launch_all(const Recipe& r, const uint64_t* pointer, const uint64_t* slot_int, const float* slot_float, uint64_t stream) {
+  Unlocked unlocked;
   for (const Launch& l : r.launches) {
+    int rc;
     uint64_t a[64];
     float f[kMaxFloats] = {0.f, 0.f, 0.f, 0.f};
     int na = 0, nf = 0;
@@ -261,9 +242,30 @@ PyObject* execute(const std::shared_ptr<Recipe>& keep, const Slots& s) {
       while (na < kMaxInts) a[na++] = 0;
       rc = call_library(l.fn, a, f);
     }
-    if (rc) break;
+    if (rc) return rc;
   }
-  Py_END_ALLOW_THREADS
+  return 0;
+}
+
+PyObject* execute(const std::shared_ptr<Recipe>& keep, const Slots& s) {
+  const Recipe& r = *keep;
+  at::Tensor fresh[kMaxSlots];
+  uint64_t pointer[2 * kMaxSlots];
+  uint64_t slot_int[kMaxSlots];
+  float slot_float[kMaxSlots];
+  for (int i = 0; i < s.n; ++i) {
+    pointer[i] = 0;
+    PyObject* o = s.obj[i];
+    if (o && is_tensor(o)) pointer[i] = (uint64_t)(uintptr_t)THPVariable_Unpack(o).const_data_ptr();
+  }
+  for (const auto& n : r.numbers)
+    if (!pass_number(s.obj[n.first], n.second, slot_int[n.first], slot_float[n.first])) return nullptr;
+  for (size_t i = 0; i < r.allocs.size(); ++i) {
+    fresh[i] = at::Tensor(at::detail::empty_cuda(r.allocs[i].sizes, r.allocs[i].dtype, at::Device(at::kCUDA, (c10::DeviceIndex)r.device), std::nullopt));
+    pointer[s.n + i] = (uint64_t)(uintptr_t)fresh[i].const_data_ptr();
+  }
+  const uint64_t stream = !r.uses_stream ? 0 : (uint64_t)(uintptr_t)c10::hip::getCurrentHIPStream(r.device_stream ? (c10::DeviceIndex)r.device : (c10::DeviceIndex)-1).stream();
+  const int rc = launch_all(r, pointer, slot_int, slot_float, stream);
   if (rc) {
     PyErr_SetString(g_error ? g_error : PyExc_RuntimeError, g_last_error());
     return nullptr;
@@ -285,7 +287,9 @@ PyObject* execute(const std::shared_ptr<Recipe>& keep, const Slots& s) {
   return out;
 }
 
+// C++ exceptions of torch (no storage, out of memory, no device) leave as the Python exceptions that torch makes of them.
 PyObject* operator_call(PyObject* self, PyObject* args, PyObject* kwargs) {
+  HANDLE_TH_ERRORS
   Operator* op = (Operator*)self;
   Key key;
   Slots s;
@@ -337,6 +341,7 @@ PyObject* operator_call(PyObject* self, PyObject* args, PyObject* kwargs) {
   Py_DECREF(full);
   Py_DECREF(method);
   return out;
+  END_HANDLE_TH_ERRORS
 }
 
 // commit(key, slots, device, device_stream, allocs, launches, results)

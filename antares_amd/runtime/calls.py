@@ -68,6 +68,14 @@ class _ViewOfAnArgument(Exception):
     pass
 
 
+def address(t: torch.Tensor) -> int:
+    """Where a tensor's elements are; an error for a wrapper (torch.func, functionalisation) that has none."""
+    at = t.data_ptr()
+    if not at and t.numel():
+        raise capi.ArtError(f'a tensor of shape {list(t.shape)} has no memory')
+    return at
+
+
 class Call:
     """What one call of an operator launches, in order: kernels and entry points of the library, with tensors as
     tensors, the stream as STREAM, list numbers as Number, and constants."""
@@ -77,14 +85,15 @@ class Call:
         self.steps = []
 
     def library(self, fn, *args):
-        self.steps.append((fn, None, None, args))
-        values = [c_void_p(a.data_ptr()) if isinstance(a, torch.Tensor) else c_void_p(self.stream) if a is STREAM else
+        values = [c_void_p(address(a)) if isinstance(a, torch.Tensor) else c_void_p(self.stream) if a is STREAM else
                   a.value if isinstance(a, Number) else c_void_p(0) if a is None else a for a in args]
+        self.steps.append((fn, None, None, args))
         capi.check(fn(*values))
 
     def kernel(self, func, grid: int, block: int, args):
+        values = [address(a) if isinstance(a, torch.Tensor) else a for a in args]
         self.steps.append((func, (grid, 1, 1), (block, 1, 1), args))
-        capi.launch(func, (grid, 1, 1), (block, 1, 1), self.stream, [a.data_ptr() if isinstance(a, torch.Tensor) else a for a in args])
+        capi.launch(func, (grid, 1, 1), (block, 1, 1), self.stream, values)
 
     def keep(self, op: Operator, pending, results, device_stream: bool):
         """Leaves the recipe of this call with the operator.  Tensors that are not among the call's arguments are

@@ -103,3 +103,89 @@ def test_a_view_of_an_argument_leaves_no_recipe(monkeypatch):
         return len(kept)
     assert keep(x, fresh) == 1 and keep(fresh, x) == 1 and keep(x[:0], x) == 1
     assert keep(x[:2], fresh) == 0 and keep(x, x[1:]) == 0 and keep(x.view(2, 2), fresh) == 0
+
+
+class GpuShaped(torch.Tensor):
+    """Dtype, shape and device of a GPU tensor, without one."""
+
+    @staticmethod
+    def __new__(cls, *shape):
+        return torch.Tensor._make_wrapper_subclass(cls, shape, dtype=torch.float32, device='cuda:0')
+
+    @classmethod
+    def __torch_dispatch__(cls, func, types, args=(), kwargs=None):
+        raise NotImplementedError(func)
+
+
+class Reached(Exception):
+    pass
+
+
+class Noting(calls.Operator):
+    def __init__(self):
+        self.pending = []
+        self._bind(('x', 'extra'), ())
+
+    def _call(self, pending, x=None, extra=None):
+        self.pending.append(pending)
+        raise Reached
+
+
+TRANSFORMS = [
+    lambda f: torch.vmap(f)(GpuShaped(3, 4)),
+    lambda f: torch.vmap(torch.vmap(f))(GpuShaped(3, 4, 5)),
+    lambda f: torch.func.grad(f)(GpuShaped(3, 4)),
+    lambda f: torch.func.functionalize(f)(GpuShaped(3, 4))]
+
+
+@pytest.mark.parametrize('transform', TRANSFORMS)
+def test_a_tensor_without_memory_reaches_the_python_method(transform):
+    """Inside torch.func's transformations a GPU tensor is a plain torch.Tensor without storage, or without memory."""
+    op = Noting()
+
+    def call(x):
+        assert type(x) is torch.Tensor and x.is_cuda
+        with pytest.raises(Reached):
+            op(x)
+        with pytest.raises(Reached):
+            op(None, extra=[x])
+        raise Reached
+    with pytest.raises(Reached):
+        transform(call)
+    assert op.pending == [None, None]
+
+
+@pytest.mark.skipif(torch.cuda.is_available(), reason='the error of a machine without a GPU')
+def test_an_error_of_torch_in_a_replayed_call_is_a_python_exception():
+    entry = ctypes.CFUNCTYPE(ctypes.c_int, ctypes.c_void_p)(lambda *a: 0)
+
+    class Streaming(calls.Operator):
+        def __init__(self):
+            self._bind(('x',), ())
+
+        def _call(self, pending, x=None):
+            call = calls.Call(0)
+            call.library(entry, calls.STREAM)
+            call.keep(self, pending, [], device_stream=False)
+    op = Streaming()
+    op(None)
+    for _ in range(3):
+        with pytest.raises(RuntimeError):               # no device, hence no current stream
+            op(None)
+
+
+def test_a_tensor_without_memory_is_refused_before_the_launch():
+    called = []
+    entry = ctypes.CFUNCTYPE(ctypes.c_int, ctypes.c_void_p)(lambda *a: called.append(a) or 0)
+
+    def launch(x):
+        call = calls.Call(0)
+        with pytest.raises(RuntimeError):
+            call.library(entry, x)
+        with pytest.raises(RuntimeError):
+            call.kernel(None, 1, 64, [x])
+        raise Reached
+    for transform in TRANSFORMS:
+        with pytest.raises(Reached):
+            transform(launch)
+    assert not called

@@ -141,3 +141,25 @@ def test_a_tensor_of_positions_in_the_place_of_the_list():
     for pos in (3, 4):
         got = autort.ops.rotary_f32(x, inv, torch.empty(2, 128, device=dev), extra=torch.tensor([pos], dtype=torch.int32, device=dev))
         assert torch.equal(got, autort.ops.rotary_f32(x, inv, torch.empty(2, 128, device=dev), extra=[pos]))
+
+
+def test_errors_of_torch_are_python_exceptions_in_replayed_calls_too(op):
+    import autort
+    dev = autort.device()
+    big = torch.zeros(32 << 20, device=dev)
+    op(big, big)
+    op(big, big)
+    for transform in (lambda f: torch.vmap(f)(torch.zeros(2, 64, device=dev)), lambda f: torch.func.functionalize(f)(torch.zeros(64, device=dev)),
+                      lambda f: torch.func.grad(lambda x: f(x).sum())(torch.zeros(64, device=dev))):
+        with pytest.raises(RuntimeError):
+            transform(lambda x: op(x, x))
+    kept = [op(big, big) for _ in range(2)]
+    del kept
+    torch.cuda.empty_cache()
+    try:
+        torch.cuda.set_per_process_memory_fraction(1e-4)
+        with pytest.raises(torch.OutOfMemoryError):
+            op(big, big)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    assert not op(big, big).any()
