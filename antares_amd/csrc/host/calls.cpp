@@ -2,8 +2,8 @@
 //
 // An operator call from Python used to cost 9 to 10 us of host time (argument checks, shape look-ups, output
 // allocation through torch.empty, ctypes conversions), more than most of the kernels it launches.  What a call does
-// depends only on the dtypes, shapes, devices, contiguity and 16-byte alignment of its tensors and on which arguments are
-// given, so the Python side works it out once per such signature - a recipe: outputs and intermediates to allocate,
+// depends only on the dtypes, shapes, devices, contiguity and 16-byte alignment of its tensors, on which of them share
+// memory and on which arguments are given, so the Python side works it out once per such signature - a recipe: outputs and intermediates to allocate,
 // kernels and library entry points to call, and where each argument comes from - and this file replays it: signature,
 // look-up, allocation, launches.  Anything unusual (an argument that is no plain tensor, a signature not seen before)
 // goes to the operator's Python method, which checks everything and raises the errors; a recipe holds no data and no
@@ -87,6 +87,8 @@ struct Slots {
   PyObject* obj[kMaxSlots];
   int n = 0;
   int device = -1;
+  struct Range { uintptr_t from, to; int slot; } memory[kMaxSlots];      // of the tensors that have elements
+  int tensors = 0;
 };
 
 struct Key {
@@ -117,6 +119,19 @@ bool describe_tensor(PyObject* o, Key& key, Slots& s) {
     return false;
   for (int64_t v : sizes)
     if (!key.put(v)) return false;
+  if (t.numel() != 0) s.memory[s.tensors++] = {address, address + (uintptr_t)t.nbytes(), s.n - 1};
+  return true;
+}
+
+// Which tensors share memory: a kernel may be the right one only where its result is not over an operand.  One word per
+// tensor that overlaps earlier ones (behind everything else, so that the rest of the key says whether there can be any).
+bool describe_overlaps(Key& key, const Slots& s) {
+  for (int i = 1; i < s.tensors; ++i) {
+    int64_t with = 0;
+    for (int j = 0; j < i; ++j)
+      if (s.memory[i].from < s.memory[j].to && s.memory[j].from < s.memory[i].to) with |= (int64_t)1 << s.memory[j].slot;
+    if (with && !key.put((int64_t)s.memory[i].slot << 32 | with)) return false;
+  }
   return true;
 }
 
@@ -187,7 +202,7 @@ bool signature(Operator* op, PyObject* args, PyObject* kwargs, Key& key, Slots& 
   for (int l = 0; l < nlists; ++l)
     for (Py_ssize_t i = 0; i < PySequence_Fast_GET_SIZE(lists[l]); ++i)
       if (!describe(PySequence_Fast_GET_ITEM(lists[l], i), list_dynamic[l], true, key, s)) return false;
-  return true;
+  return describe_overlaps(key, s);
 }
 
 // A library entry point with any mix of up to kMaxInts integer / pointer and kMaxFloats float arguments: the x86-64

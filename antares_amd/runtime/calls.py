@@ -1,8 +1,8 @@
 """Operators whose calls are replayed in native code.
 
 ``Operator`` (``csrc/host/calls.cpp``) is the base class of everything callable in ``autort.ops``.  A call whose
-signature - dtypes, shapes, devices, contiguity and 16-byte alignment of the tensors, which arguments are given - has been
-seen before is replayed from a recipe without entering Python; any other call reaches the subclass's ``_call(pending,
+signature - dtypes, shapes, devices, contiguity and 16-byte alignment of the tensors, which of them share memory, which
+arguments are given - has been seen before is replayed from a recipe without entering Python; any other call reaches the subclass's ``_call(pending,
 ...)``, which checks the arguments, runs the operator and leaves the recipe with ``pending`` (None when the arguments are
 nothing a recipe can be kept for).
 """

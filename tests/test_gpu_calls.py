@@ -163,3 +163,58 @@ def test_errors_of_torch_are_python_exceptions_in_replayed_calls_too(op):
     finally:
         torch.cuda.set_per_process_memory_fraction(1.0)
     assert not op(big, big).any()
+
+
+def conv_op(name):
+    import autort
+    return autort.export(ir='output0[N, F, HO, WO] +=! input0[N, C, HO + KH - 1, WO + KW - 1].when([HO + KH - 1 >= 0, HO + KH - 1 < 28, WO + KW - 1 >= 0, '
+                            'WO + KW - 1 < 28], 0.0) * input1[F, C, KH, KW] where HO in 28, WO in 28',
+                         inputs=['input0=float32[N:4, C:64, H:28, W:28]', 'input1=float32[F:64, C:64, KH:3, KW:3]'], name=name)
+
+
+@pytest.mark.parametrize('order', ['over its image first', 'apart first'])
+def test_a_convolution_over_its_image_and_one_apart_from_it_do_not_depend_on_each_other(order):
+    import autort
+    dev = autort.device()
+    op = conv_op('calls_conv_' + order.split()[0])
+    g = torch.Generator().manual_seed(1)
+    x, w = torch.randn(4, 64, 28, 28, generator=g), torch.randn(64, 64, 3, 3, generator=g) / 24
+    want, bound = (torch.nn.functional.conv2d(a, b, padding=1) for a, b in ((x.double(), w.double()), (x.double().abs(), w.double().abs())))
+    taken = []
+    handler = op.fast_path
+    op.fast_path = lambda *a: taken.append(handler(*a)) or taken[-1]
+
+    def check(got):
+        assert ((got.cpu().double() - want).abs() <= 2.0 ** -23 * 9 * 64 * bound).all()
+    for where in (['over', 'apart', 'behind'] if order.startswith('over') else ['apart', 'behind', 'over']) * 3:
+        print(f'[case] convolution {where}', flush=True)
+        memory = torch.zeros(2 * x.numel(), device=dev)
+        image = memory[:x.numel()].view_as(x).copy_(x)
+        at = {'over': 0, 'apart': None, 'behind': x.numel()}[where]        # behind: the first element past the image
+        check(op(image, w.to(dev), out=None if at is None else memory[at:at + x.numel()].view_as(x)))
+    assert sorted(taken) == [False, True, True]          # one recipe each: by hand where the memory is apart
+
+
+def test_which_tensors_share_memory_is_part_of_the_signature():
+    from antares_amd.runtime import calls
+    import autort
+    dev = autort.device()
+
+    class Keys(calls.Operator):
+        def __init__(self):
+            self._bind(('a', 'b', 'c', 'extra'), ())
+
+        def _call(self, pending, *args, **kwargs):
+            return pending[0]
+    key = Keys()
+    m = torch.zeros(64, device=dev)
+    a, b, c = m[0:16], m[16:32], m[32:48]
+    base = key(a, b, c)
+    assert base == key(a, c, b) == key(b, c, a) == key(c.clone(), b, a) and base != key(a, b, [c])
+    keys = [base, key(a, a, c), key(a, b, a), key(a, b, b), key(a, m[12:28], c), key(a, b, m[12:28]), key(a, b, m[20:36]),
+            key(m[4:20], m[12:28], m[20:36]), key(m[4:20], m[8:24], m[12:28])]
+    assert len(set(keys)) == len(keys)
+    assert key(a, m[4:20], c) == key(b, m[12:28], c) == key(a, m[0:16], c)  # how they overlap is not
+    assert key(a, b, extra=[c]) != key(a, b, extra=[b])
+    none = m[:0]
+    assert key(none, m[:0], c) == key(none, m[4:4], a)                     # nothing to share without elements
