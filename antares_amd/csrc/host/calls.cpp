@@ -229,6 +229,17 @@ bool pass_number(PyObject* o, bool as_float, uint64_t& i, float& f) {
   return !PyErr_Occurred();
 }
 
+// The arguments of a call stay alive until it is over: while other threads run, one of them may empty a list argument.
+struct Held {
+  const Slots& s;
+  explicit Held(const Slots& slots) : s(slots) {
+    for (int i = 0; i < s.n; ++i) Py_XINCREF(s.obj[i]);
+  }
+  ~Held() {
+    for (int i = 0; i < s.n; ++i) Py_XDECREF(s.obj[i]);
+  }
+};
+
 struct Unlocked {                                        // other threads run meanwhile, whichever way this scope is left
   PyThreadState* state = PyEval_SaveThread();
   ~Unlocked() { PyEval_RestoreThread(state); }
@@ -264,6 +275,7 @@ int launch_all(const Recipe& r, const uint64_t* pointer, const uint64_t* slot_in
 
 PyObject* execute(const std::shared_ptr<Recipe>& keep, const Slots& s) {
   const Recipe& r = *keep;
+  const Held held(s);
   at::Tensor fresh[kMaxSlots];
   uint64_t pointer[2 * kMaxSlots];
   uint64_t slot_int[kMaxSlots];

@@ -1,6 +1,7 @@
 """Calls replayed in native code, as far as that needs no GPU: what a recipe passes on to an entry point (here a
 recording callback), with arguments that are numbers."""
 import ctypes
+import sys
 
 import pytest
 import torch
@@ -189,3 +190,23 @@ def test_a_tensor_without_memory_is_refused_before_the_launch():
         with pytest.raises(Reached):
             transform(launch)
     assert not called
+
+
+@pytest.mark.parametrize('as_list', [True, False])
+def test_arguments_live_until_the_call_is_over(as_list):
+    """Other threads run while a recipe's entry points do, and may change a list argument."""
+    value, counts = float('1234.5'), []
+    extra = [value] if as_list else (value,)
+
+    def during():
+        if op.seen[1:] and as_list:
+            extra.clear()
+        counts.append(sys.getrefcount(value))
+    op = Recording('F', during)
+    op(None, extra=[value])                              # leaves the recipe
+    counts.clear()
+    before = sys.getrefcount(value)
+    op(None, extra=extra)
+    assert op.seen == [1234.5] * 2 and op.python_calls == 1
+    assert counts == [before + (0 if as_list else 1)]           # the list's reference is gone, the call's is there
+    assert sys.getrefcount(value) == before - as_list
