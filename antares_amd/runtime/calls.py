@@ -17,11 +17,11 @@ from . import capi
 
 try:
     from . import _calls
-    Operator = _calls.Operator
+    _Base = _calls.Operator
 except ImportError as _e:                     # not built: operators can still be made (lowering, compiling), not called
     _calls, _reason = None, str(_e)
 
-    class Operator:
+    class _Base:
         tuned = config = fast_path = None
 
         def _bind(self, names, dynamic):
@@ -29,6 +29,23 @@ except ImportError as _e:                     # not built: operators can still b
 
         def __call__(self, *args, **kwargs):
             raise capi.ArtError(f'antares_amd/runtime/_calls.so cannot be loaded ({_reason}): build it with `python -m antares_amd.build`')
+
+
+class Operator(_Base):
+    """Copies and pickles like an object of Python's: with its attributes, without its recipes."""
+
+    def _bind(self, names, dynamic):
+        self._parameters = (names, dynamic)
+        super()._bind(names, dynamic)
+
+    def __getstate__(self):
+        return {**vars(self), **{n: getattr(self, n) for n in ('tuned', 'config', 'fast_path') if getattr(self, n) is not None}}
+
+    def __setstate__(self, state):
+        for name, value in state.items():
+            setattr(self, name, value)
+        self._bind(*self._parameters)
+
 
 _ready = False
 

@@ -1,12 +1,15 @@
 """Calls replayed in native code, as far as that needs no GPU: what a recipe passes on to an entry point (here a
 recording callback), with arguments that are numbers."""
+import copy
 import ctypes
+import pickle
 import sys
 
 import pytest
 import torch
 
-from antares_amd.autort import builtin_ops
+from antares_amd.autort import builtin_ops, patterns
+from antares_amd.autort.op import ExportedOp
 from antares_amd.runtime import calls
 
 
@@ -210,3 +213,47 @@ def test_arguments_live_until_the_call_is_over(as_list):
     assert op.seen == [1234.5] * 2 and op.python_calls == 1
     assert counts == [before + (0 if as_list else 1)]           # the list's reference is gone, the call's is there
     assert sys.getrefcount(value) == before - as_list
+
+
+def exported(name, **kw):
+    return ExportedOp('output0[N] = input0[N] + input1[N]', ['input0=float32[N:64]', 'input1=float32[N:64]'], name=name, **kw)
+
+
+def by_hand(name):
+    op = ExportedOp(patterns.W4A16_IR, patterns.W4A16_INPUTS, name=name, config='tune:3', tuned={'k': {'value': 2}})
+    assert op.fast_path is not None
+    return op
+
+
+@pytest.mark.parametrize('duplicate', [copy.copy, copy.deepcopy])
+@pytest.mark.parametrize('make', [exported, by_hand, lambda name: builtin_ops.RmsNorm(torch.float16), lambda name: builtin_ops.PartitionEvenFirst()])
+def test_operators_can_be_copied(make, duplicate):
+    op = make('copied')
+    holder = torch.nn.Module()
+    holder.op = op
+    twin, held = duplicate(op), copy.deepcopy(holder).op
+    assert held is not op
+    for t in (twin, held):
+        assert type(t) is type(op) and vars(t).keys() == vars(op).keys() and t.name == op.name
+        assert t.tuned == op.tuned and t.config == op.config and (t.fast_path is None) == (op.fast_path is None)
+    assert twin is not op and (op.tuned is None or (twin.tuned is op.tuned) == (duplicate is copy.copy))
+    twin.fast_path = None                                # its own attributes
+    twin.tuned = {'other': {'value': 1}}
+    assert op.tuned != twin.tuned and (op.fast_path is None) == (make is not by_hand)
+
+
+def test_a_copy_is_called_like_the_operator_it_is_a_copy_of():
+    op = Recording('I')
+    op(None, extra=[1])
+    twin = copy.copy(op)
+    twin(None, extra=[2])
+    twin(extra=[3], x=None)
+    twin(None, extra=[4])
+    op(None, extra=[5])
+    assert op.seen == [1, 2, 3, 4, 5] and (op.python_calls, twin.python_calls) == (1, 2)
+
+
+def test_built_in_operators_can_be_pickled():
+    for op in (builtin_ops.RmsNorm(torch.float32), builtin_ops.Rotary('rotary_f32', False), builtin_ops.GemvW4Fused(), builtin_ops.PartitionEvenFirst()):
+        twin = pickle.loads(pickle.dumps(op))
+        assert type(twin) is type(op) and vars(twin) == vars(op) and twin.tuned == op.tuned

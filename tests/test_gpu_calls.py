@@ -218,3 +218,16 @@ def test_which_tensors_share_memory_is_part_of_the_signature():
     assert key(a, b, extra=[c]) != key(a, b, extra=[b])
     none = m[:0]
     assert key(none, m[:0], c) == key(none, m[4:4], a)                     # nothing to share without elements
+
+
+def test_copies_of_an_operator_are_called_like_it(op):
+    import copy
+    import autort
+    dev = autort.device()
+    fresh = autort.export(ir=op.ir, inputs=op.input_specs, name='calls_add_fresh')
+    norm = autort.ops.rmsnorm_f32
+    a, b = torch.randn(1000, device=dev), torch.randn(1000, device=dev)
+    op(a, b)
+    for twin in (copy.deepcopy(fresh), copy.copy(fresh), copy.copy(op)):
+        assert all(torch.equal(twin(a, b), a + b) for _ in range(3))
+    assert all(torch.equal(copy.deepcopy(norm)(a, None, b), norm(a, None, b)) for _ in range(2))
