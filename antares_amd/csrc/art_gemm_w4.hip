@@ -388,23 +388,33 @@ double estimate(int M, int K, int N, const Plan& p, int compute_units) {
   else if (rest > 0) per_group += c.per_cu == 2 || blocks > round ? c.one : c.one + (c.two - c.one) * rest / compute_units;
   return c.fixed + groups * per_group + (p.splits > 1 ? 2.4 + (8.0 * p.splits + 2.0) * M * N / 4.4e6 : 0.0);
 }
-Plan choose(int M, int K, int N, size_t scratch_bytes, int compute_units, int code, int splits) {
+// What a form's 32-bit offsets (a block's rows of x and of the packed weights) and its division by the number of column
+// tiles hold.
+bool holds(const Plan& p, int K, int N, bool swiglu) {
+  return 64LL * p.row_tiles * K <= 1LL << 32 && 64LL * N <= 1LL << 32 && (p.wide || (long long)tile_count(N, swiglu, BN) * p.splits < 65536);
+}
+// False: no form takes these sizes.  `code` and `splits` are the caller's wishes (0: none); a form that does not hold the
+// sizes is replaced by one that does.
+bool choose(Plan& best, int M, int K, int N, bool swiglu, size_t scratch_bytes, int compute_units, int code, int splits) {
   const int G = K / GK;
   const size_t per_split = (size_t)M * N * sizeof(float);
   const int cap = (int)(scratch_bytes / per_split), most = G < cap ? G : (cap < 1 ? 1 : cap);
-  Plan best{false, 1, 1};
   double t_best = 1e30;
-  for (const Plan form : {Plan{false, 1, 1}, Plan{false, 2, 1}, Plan{false, 4, 1}, Plan{true, 4, 1}, Plan{true, 8, 1}}) {
-    const int form_code = form.wide ? form.row_tiles : form.row_tiles == 4 ? 5 : form.row_tiles;
-    if (code != 0 ? code != form_code : 16 * form.row_tiles >= M && form.row_tiles > 1) continue;     // not over twice the rows
-    for (int s = splits > 0 ? splits : 1; s <= (splits > 0 ? splits : 32); ++s) {
-      if (splits == 0 && s > 1 && (s > most || 2 * s > G + 1)) break;
-      const Plan p{form.wide, form.row_tiles, s > most ? most : s};
-      const double t = estimate(M, K, N, p, compute_units);
-      if (t < t_best) { t_best = t; best = p; }
+  for (int pass = 0; pass < 2 && t_best == 1e30; ++pass) {
+    for (const Plan form : {Plan{false, 1, 1}, Plan{false, 2, 1}, Plan{false, 4, 1}, Plan{true, 4, 1}, Plan{true, 8, 1}}) {
+      const int form_code = form.wide ? form.row_tiles : form.row_tiles == 4 ? 5 : form.row_tiles;
+      if (pass == 0 && (code != 0 ? code != form_code : 16 * form.row_tiles >= M && form.row_tiles > 1)) continue;     // not over twice the rows
+      for (int s = splits > 0 ? splits : 1; s <= (splits > 0 ? splits : 32); ++s) {
+        if (splits == 0 && s > 1 && (s > most || 2 * s > G + 1)) break;
+        const Plan p{form.wide, form.row_tiles, s > most ? most : s};
+        if (!holds(p, K, N, swiglu)) break;
+        const double t = estimate(M, K, N, p, compute_units);
+        if (t < t_best) { t_best = t; best = p; }
+      }
     }
+    if (t_best == 1e30) splits = 1;
   }
-  return best;
+  return t_best < 1e30;
 }
 // An RMSNorm of the result: out = fp16(y / rms(y) * weight).
 struct Norm {
@@ -433,6 +443,43 @@ int combine(const float* partial, _Float16* y, int rows, int N, int splits, cons
   return 0;
 }
 
+// One launch of the product (and of the pass behind it) over up to kMaxRows rows.
+constexpr int kMaxRows = 1 << 18;                   // 8192 blocks of 32 rows
+int run_rows(const _Float16* xs, const unsigned char* qweight, const _Float16* scales, const unsigned char* qzeros, _Float16* ys, const _Float16* res,
+             int M, int K, int N, int code, int splits, bool swiglu, const Norm* norm, float* scratch, size_t scratch_bytes, hipStream_t st) {
+  Plan p;
+  ART_REQUIRE(choose(p, M, K, N, swiglu, scratch_bytes, art::compute_units(), code, splits), "art_gemm_w4a16: K=%d N=%d are too large", K, N);
+  // Where K-splits meet in a pass of their own, the norm is part of that pass, up to 256 rows: beyond them
+  // nothing is gained (8 layers of 4096 columns: 966 -> 944 us at 100 rows, 1881 -> 1879 at 300).
+  const bool norm_there = norm && p.splits > 1 && M <= 256 && N % 8 == 0 && N <= 8 * kNormThreads * kNormTurns &&
+                          (((uintptr_t)ys | (uintptr_t)res | (uintptr_t)norm->weight | (uintptr_t)norm->out) % 16) == 0;
+  if (p.wide) {
+    if (art::w4::gemm_wide(xs, qweight, scales, qzeros, ys, scratch, M, K, N, p.splits, p.row_tiles, res, swiglu, st)) return 1;
+  } else {
+    static bool configured = false;
+    if (!configured) {
+      const void* kernels[3][2] = {{(const void*)gemm_w4a16_kernel<1, false>, (const void*)gemm_w4a16_kernel<1, true>},
+                                   {(const void*)gemm_w4a16_kernel<2, false>, (const void*)gemm_w4a16_kernel<2, true>},
+                                   {(const void*)gemm_w4a16_kernel<4, false>, (const void*)gemm_w4a16_kernel<4, true>}};
+      for (int i = 0; i < 3; ++i)
+        for (int j = 0; j < 2; ++j)
+          ART_HIP(hipFuncSetAttribute(kernels[i][j], hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes(1 << i)));
+      configured = true;
+    }
+    const int col_tiles = tile_count(N, swiglu, BN), m_blocks = (M + 32 * p.row_tiles - 1) / (32 * p.row_tiles);
+    const int units = col_tiles * p.splits, G = K / GK;
+    const Work work{units, col_tiles, p.splits, (unsigned int)((0x100000000ull + col_tiles - 1) / col_tiles), G / p.splits, G % p.splits};
+    const dim3 grid(8 * m_blocks, (units + 7) / 8);
+    const auto kernel = p.row_tiles == 1   ? (swiglu ? gemm_w4a16_kernel<1, true> : gemm_w4a16_kernel<1, false>)
+                        : p.row_tiles == 2 ? (swiglu ? gemm_w4a16_kernel<2, true> : gemm_w4a16_kernel<2, false>)
+                                           : (swiglu ? gemm_w4a16_kernel<4, true> : gemm_w4a16_kernel<4, false>);
+    kernel<<<grid, kThreads, lds_bytes(p.row_tiles), st>>>(xs, qweight, scales, qzeros, ys, scratch, M, K, N, work, kMagic, res);
+    ART_LAUNCH_CHECK();
+  }
+  if (p.splits > 1 && combine(scratch, ys, M, N, p.splits, res, swiglu, norm_there ? norm : nullptr, st)) return 1;
+  return norm && !norm_there ? art_rmsnorm(ys, nullptr, norm->weight, norm->out, M, N, 1.0f / (float)N, norm->eps, 1, 1, 1, st) : 0;
+}
+
 int run(const void* x_dev, const void* qweight_dev, const void* scales_dev, const void* qzeros_dev, void* y_dev, const void* residual_dev,
         int M, int K, int N, int k_splits, bool swiglu, const Norm* norm, void* stream) {
   const int n_out = swiglu ? N / 2 : N;
@@ -451,44 +498,16 @@ int run(const void* x_dev, const void* qweight_dev, const void* scales_dev, cons
   if (!ws) return 1;
   float* scratch = reinterpret_cast<float*>((char*)ws->base + art::kScratchOffset);
   const size_t scratch_bytes = ws->bytes - art::kScratchOffset;
-  hipStream_t st = (hipStream_t)stream;
-  Plan p = choose(M, K, N, scratch_bytes, art::compute_units(), code, k_splits & 0xff);
-  const _Float16* xs = (const _Float16*)x_dev;
-  const _Float16* res = (const _Float16*)residual_dev;
-  _Float16* ys = (_Float16*)y_dev;
-  // Where K-splits meet in a pass of their own, the norm is part of that pass, up to 256 rows: beyond them
-  // nothing is gained (8 layers of 4096 columns: 966 -> 944 us at 100 rows, 1881 -> 1879 at 300).
-  const bool norm_there = norm && p.splits > 1 && M <= 256 && N % 8 == 0 && N <= 8 * kNormThreads * kNormTurns &&
-                          (((uintptr_t)y_dev | (uintptr_t)residual_dev | (uintptr_t)norm->weight | (uintptr_t)norm->out) % 16) == 0;
-  if (p.wide) {
-    if (art::w4::gemm_wide(xs, (const unsigned char*)qweight_dev, (const _Float16*)scales_dev, (const unsigned char*)qzeros_dev, ys, scratch, M,
-                           K, N, p.splits, p.row_tiles, res, swiglu, st))
+  for (int m0 = 0; m0 < M; m0 += kMaxRows) {
+    const size_t out = (size_t)m0 * n_out;
+    const Norm rows_norm = norm ? Norm{norm->weight, (_Float16*)norm->out + out, norm->eps} : Norm{};
+    if (run_rows((const _Float16*)x_dev + (size_t)m0 * K, (const unsigned char*)qweight_dev, (const _Float16*)scales_dev, (const unsigned char*)qzeros_dev,
+                 (_Float16*)y_dev + out, residual_dev ? (const _Float16*)residual_dev + out : nullptr, M - m0 < kMaxRows ? M - m0 : kMaxRows, K, N, code,
+                 k_splits & 0xff, swiglu, norm ? &rows_norm : nullptr, scratch, scratch_bytes, (hipStream_t)stream))
       return 1;
-  } else {
-    static bool configured = false;
-    if (!configured) {
-      const void* kernels[3][2] = {{(const void*)gemm_w4a16_kernel<1, false>, (const void*)gemm_w4a16_kernel<1, true>},
-                                   {(const void*)gemm_w4a16_kernel<2, false>, (const void*)gemm_w4a16_kernel<2, true>},
-                                   {(const void*)gemm_w4a16_kernel<4, false>, (const void*)gemm_w4a16_kernel<4, true>}};
-      for (int i = 0; i < 3; ++i)
-        for (int j = 0; j < 2; ++j)
-          ART_HIP(hipFuncSetAttribute(kernels[i][j], hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes(1 << i)));
-      configured = true;
-    }
-    const int col_tiles = tile_count(N, swiglu, BN), m_blocks = (M + 32 * p.row_tiles - 1) / (32 * p.row_tiles);
-    const int units = col_tiles * p.splits, G = K / GK;
-    ART_REQUIRE(units < 65536 && m_blocks < 8192, "art_gemm_w4a16: too many tiles (M=%d N=%d)", M, N);
-    const Work work{units, col_tiles, p.splits, (unsigned int)((0x100000000ull + col_tiles - 1) / col_tiles), G / p.splits, G % p.splits};
-    const dim3 grid(8 * m_blocks, (units + 7) / 8);
-    const auto kernel = p.row_tiles == 1   ? (swiglu ? gemm_w4a16_kernel<1, true> : gemm_w4a16_kernel<1, false>)
-                        : p.row_tiles == 2 ? (swiglu ? gemm_w4a16_kernel<2, true> : gemm_w4a16_kernel<2, false>)
-                                           : (swiglu ? gemm_w4a16_kernel<4, true> : gemm_w4a16_kernel<4, false>);
-    kernel<<<grid, kThreads, lds_bytes(p.row_tiles), st>>>(xs, (const unsigned char*)qweight_dev, (const _Float16*)scales_dev,
-                                                           (const unsigned char*)qzeros_dev, ys, scratch, M, K, N, work, kMagic, res);
-    ART_LAUNCH_CHECK();
+    if (M - m0 <= kMaxRows) break;                  // m0 does not pass the largest int
   }
-  if (p.splits > 1 && combine(scratch, ys, M, N, p.splits, res, swiglu, norm_there ? norm : nullptr, st)) return 1;
-  return norm && !norm_there ? art_rmsnorm(y_dev, nullptr, norm->weight, norm->out, M, N, 1.0f / (float)N, norm->eps, 1, 1, 1, stream) : 0;
+  return 0;
 }
 
 }  // namespace

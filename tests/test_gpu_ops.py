@@ -1300,3 +1300,48 @@ def test_convolution_into_part_of_a_larger_result(autort, dtype):
             got = y.cpu().double()
             assert ((got[:, :, :hw, :hw] - want).abs() <= 2.0 ** -23 * 9 * c * bound).all()
             assert (got[:, :, hw:] == 7.0).all() and (got[:, :, :, hw:] == 7.0).all()
+
+
+# more rows than one launch of any form takes (and one row more); 32-row blocks asked for; more columns than the narrow forms
+# number, also where one of them is asked for, and a K-split that does not fit
+@pytest.mark.parametrize('M,K,N,code', [(262145, 128, 16, 0), (1048576 + 40, 128, 16, 0), (262144 + 33, 256, 48, 256 + 1), (524288 + 1, 128, 32, 2048 + 1),
+                                        (5, 128, 16384 * 513, 0), (40, 256, 16384 * 513, 512 + 2), (5, 256, 16384 * 300, 256 + 2)])
+def test_w4a16_gemm_of_very_many_rows_or_columns(autort, M, K, N, code):
+    """Rows and columns repeat with a period: the result is that of one period, the oracle's."""
+    from ctypes import c_void_p
+    from antares_amd.runtime import capi
+    from oracle import hot_ops
+    note(f'w4a16 gemm M={M} K={K} N={N} code={code}')
+    dev = autort.device()
+    capi.init(0)
+    m, n, step = min(M, 999), min(N, 16384), 1 << 17
+    p = workloads.w4_problem(M % 1000, m, K, n)
+    x, q, s, z = (p[k] for k in ('x', 'qweight', 'scales', 'qzeros'))
+    want = torch.from_numpy(hot_ops.gemm_w4a16(x.numpy(), q.numpy(), s.numpy(), z.numpy())).to(dev).float()
+    rows = torch.arange(M, device=dev) % m
+    operands = [x.to(dev)[rows]] + [t.to(dev).repeat(1, N // n) for t in (q, s, z)]
+    lib, stream = capi.lib(), c_void_p(torch.cuda.current_stream().cuda_stream)
+
+    def new(columns):
+        return torch.full((M, columns), float('nan'), dtype=torch.float16, device=dev)
+
+    def ptr(*tensors):
+        return [c_void_p(t.data_ptr()) for t in tensors]
+
+    def close(got, period, **tol):
+        for r in range(0, M, step):
+            part = got[r:r + step].float().view(-1, N // n, period.shape[1])
+            assert torch.allclose(part, period[rows[r:r + step]].view(-1, 1, period.shape[1]).expand_as(part), **tol)
+    y = new(N)
+    capi.check(lib.art_gemm_w4a16_tuned(*ptr(*operands, y), M, K, N, code, stream))
+    close(y, want, rtol=1e-2, atol=1e-2)
+    if n < N:
+        return
+    if N % 32 == 0:
+        hid = new(N // 2)
+        capi.check(lib.art_gemm_w4a16_swiglu(*ptr(*operands, hid), M, K, N, code, stream))
+        close(hid, torch.nn.functional.silu(want[:, :N // 2]) * want[:, N // 2:], rtol=2e-2, atol=2e-2)
+    res, weight = torch.randn(m, N, device=dev).half()[rows], torch.rand(N, device=dev).half()
+    acc, out = res.clone(), new(N)                           # the residual and the normalised rows move on with the rows
+    capi.check(lib.art_gemm_w4a16_residual_norm(*ptr(*operands, acc, acc, weight, out), M, K, N, 1e-5, code, stream))
+    assert torch.equal(acc, (y.float() + res.float()).half()) and torch.equal(out, autort.ops.rmsnorm_f16(acc, None, weight))
