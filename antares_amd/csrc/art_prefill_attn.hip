@@ -10,10 +10,11 @@
 // One block of four wavefronts per (head, tile of 32 queries).  The key tiles 0 .. the block's own are dealt out to the
 // wavefronts in turn, each keeps an online softmax of its share, and the four states are merged through LDS at the end:
 // nothing is computed above the diagonal, no barrier exists in the loop, and the longest chain of tiles - which bounds the
-// launch, 1.6 us a tile with one wavefront per SIMD - is a quarter of the tiles.  1003 tokens of 32 heads: 52 us with one
-// wavefront for all of them, 63 with four while the blocks of a head were neighbours (every XCD read all keys and values
-// past its L2), 28 with a head on one XCD; 128 tokens: 8.1 and 6.1 us.  Everything is kept transposed so that a lane owns
-// ONE query:
+// launch, 1.6 us a tile with one wavefront per SIMD - is a quarter of the tiles.  With four wavefronts the L2 has to serve the
+// key tiles: the blocks of a head run on one XCD, those of the heads past a multiple of eight on all.  One wavefront per query
+// tile / four with the blocks of a head wherever they fall / four as here, us: 1003 tokens of 32 heads 50 / 63 / 26, of 31
+// heads 49 / 39 / 27; 4000 tokens of 31 heads 456 / 547 / 276, of 71 heads 917 / 1247 / 653; 128 tokens of 32 heads 8.0 / - / 5.2.
+// Everything is kept transposed so that a lane owns ONE query:
 //   * S^T = K Q^T on v_mfma_f32_32x32x16_f16: A = a K tile as it lies in the cache (32 rows of 128 dims, staged in LDS
 //     with coalesced 16-byte loads, read back as 16-byte rows), B = the lane's query row from registers.  The 32 x 32
 //     result has query lane % 32 in every lane, 16 keys per lane: the running maximum and sum of the online softmax
@@ -64,9 +65,16 @@ __global__ __launch_bounds__(64 * kWaves, 2) void prefill_attention_kernel(const
   const int lane = threadIdx.x & 63, half = lane >> 5, qi = lane & 31, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   _Float16* const Ks = tiles[wave];
   _Float16* const Vs = Ks + KT * K_LD;
-  // The longest walks (last query tiles) are handed out first; blocks of one head are `heads` apart, i.e. on one XCD for
-  // a multiple of 8 heads, whose L2 then holds the keys and values of its heads.
-  const int qt = q_tiles - 1 - (int)(blockIdx.x / heads), h = blockIdx.x % heads;
+  // The longest walks (last query tiles) are handed out first, in chunks (grid y, z) of eight query tiles of all heads.
+  // Workgroups go to the eight XCDs round robin: in a chunk, the tiles of heads & ~7 heads lie that many blocks apart, a head
+  // on one XCD, whose L2 then holds its keys and values; the tiles of the other heads & 7 are dealt to all XCDs, in front.
+  const int chunk = blockIdx.y + blockIdx.z * gridDim.y, ranks = q_tiles - 8 * chunk < 8 ? q_tiles - 8 * chunk : 8;
+  if (ranks <= 0) return;
+  const unsigned whole = heads & ~7, others = heads & 7, dealt = (ranks * others + 7) & ~7u;
+  const bool is_dealt = blockIdx.x < dealt;
+  const unsigned at = is_dealt ? blockIdx.x : blockIdx.x - dealt, per = is_dealt ? others : whole;
+  if (at >= ranks * per) return;
+  const int qt = q_tiles - 1 - (8 * chunk + (int)(at / per)), h = (int)((is_dealt ? whole : 0) + at % per);
   const int query = qt * QT + qi;
   const int qrow = query < T ? query : T - 1;                    // rows past T repeat the last one and are never stored
   const float scale = att_f[0] * 1.44269504088896341f;            // scores in units of log2(e)
@@ -224,7 +232,9 @@ extern "C" int art_prefill_attention(const void* q_dev, const void* k_dev, const
   const int q_tiles = (T + QT - 1) / QT;
   const long long blocks = (long long)q_tiles * heads;
   ART_REQUIRE(blocks <= 0x7fffffffLL, "art_prefill_attention: too many blocks");
-  prefill_attention_kernel<<<dim3((unsigned)blocks), dim3(64 * kWaves), 0, (hipStream_t)stream>>>(
+  const unsigned chunks = (q_tiles + 7) / 8, rows = chunks < 32768 ? chunks : 32768;
+  const unsigned a_chunk = chunks > 1 ? 8 * heads : (q_tiles * (heads & 7) + 7) / 8 * 8 + q_tiles * (heads & ~7);
+  prefill_attention_kernel<<<dim3(a_chunk, rows, (chunks + rows - 1) / rows), dim3(64 * kWaves), 0, (hipStream_t)stream>>>(
       (const _Float16*)q_dev, (const _Float16*)k_dev, (const _Float16*)v_dev, (_Float16*)out_dev, T, heads, kv_row_stride,
       (const float*)att_f_dev, q_tiles);
   ART_LAUNCH_CHECK();

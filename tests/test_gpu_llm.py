@@ -342,6 +342,25 @@ def test_causal_attention_over_a_prompt_against_the_oracle(T, H):
     assert np.allclose(out.astype(np.float64), exact, rtol=1e-2, atol=1e-2)
 
 
+# heads on one XCD each, dealt to all of them, and both; one to nine query tiles past a chunk of eight, the last one not full
+@pytest.mark.parametrize('T,H', [(9, 7), (33, 1), (64, 9), (224, 8), (256, 12), (257, 9), (270, 31), (513, 25), (545, 17), (1003, 20)])
+def test_causal_attention_of_any_number_of_heads(T, H):
+    import autort
+    dev = autort.device()
+    D, S = 128, T + 3
+    g = torch.Generator().manual_seed(T + H)
+    note(f'causal attention T={T} H={H}')
+    q, kc, vc = torch.randn(T, H, D, generator=g).half(), (torch.randn(S, H, D, generator=g) * 0.7).half(), torch.randn(S, H, D, generator=g).half()
+    att_f = 1 / math.sqrt(D)
+    out = torch.full((T, H, D), float('nan'), dtype=torch.float16, device=dev)
+    autort.ops.attention_causal_f16(q.to(dev), kc.to(dev), vc.to(dev), torch.tensor([att_f], device=dev), out)
+    sc = torch.einsum('thd,shd->hts', q.double(), kc[:T].double()) * att_f
+    sc = sc.masked_fill(torch.triu(torch.ones(T, T, dtype=torch.bool), 1), float('-inf'))
+    exact = torch.einsum('hts,shd->thd', torch.softmax(sc, -1), vc[:T].double())
+    # probabilities (2^-11 of each, the sum of their products with v bounded by the largest |v|) and results are rounded to float16
+    assert ((out.cpu().double() - exact).abs() <= 2.0 ** -10 * vc.double().abs().max() + 2.0 ** -10 * exact.abs()).all()
+
+
 # the 16-byte form at its smallest and largest head, then heads and addresses it leaves to the one-pair-per-lane form
 @pytest.mark.parametrize('H,D,offset', [(1, 16, 0), (3, 256, 0), (33, 128, 0), (2, 72, 0), (2, 272, 0), (2, 128, 1)])
 def test_rope_qkv_store_rows_of_any_head_size(H, D, offset):
