@@ -14,6 +14,7 @@
 // key tiles: the blocks of a head run on one XCD, those of the heads past a multiple of eight on all.  One wavefront per query
 // tile / four with the blocks of a head wherever they fall / four as here, us: 1003 tokens of 32 heads 50 / 63 / 26, of 31
 // heads 49 / 39 / 27; 4000 tokens of 31 heads 456 / 547 / 276, of 71 heads 917 / 1247 / 653; 128 tokens of 32 heads 8.0 / - / 5.2.
+// A prompt of one query tile has one key tile: one wavefront, which stores its own outputs (32 tokens: 4.2 us, 4.6 with four).
 // Everything is kept transposed so that a lane owns ONE query:
 //   * S^T = K Q^T on v_mfma_f32_32x32x16_f16: A = a K tile as it lies in the cache (32 rows of 128 dims, staged in LDS
 //     with coalesced 16-byte loads, read back as 16-byte rows), B = the lane's query row from registers.  The 32 x 32
@@ -37,7 +38,7 @@ typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
 
 constexpr int D = 128;                 // head dimension
 constexpr int QT = 32, KT = 32;        // queries per block, keys per step
-constexpr int kWaves = 4;
+constexpr int kMaxWaves = 4;
 constexpr int K_LD = D + 8;            // halves per K row in LDS (272 bytes)
 constexpr int O_LD = D + 4;            // floats per output row of the merge
 constexpr int V_LD = D + 32;           // halves per V row in LDS (320 bytes: the four rows of a transposing read fall on disjoint banks)
@@ -54,6 +55,7 @@ __device__ __forceinline__ float sum_with_lane_xor_32(float v) {
 }
 
 // q: [T, heads, 128]; k, v: rows of kv_stride halves, row s holding [heads, 128]; out: [T, heads, 128]
+template <int kWaves>
 __global__ __launch_bounds__(64 * kWaves, 2) void prefill_attention_kernel(const _Float16* __restrict__ q, const _Float16* __restrict__ k,
                                                                 const _Float16* __restrict__ v, _Float16* __restrict__ out, int T,
                                                                 int heads, long long kv_stride, const float* __restrict__ att_f,
@@ -188,6 +190,19 @@ __global__ __launch_bounds__(64 * kWaves, 2) void prefill_attention_kernel(const
     __builtin_amdgcn_wave_barrier();
   }
 
+  typedef float f32x4 __attribute__((ext_vector_type(4)));
+  // element r of tile t: dim t * 32 + (r / 4) * 8 + 4 * half + r % 4
+  if constexpr (kWaves == 1) {
+    if (query >= T) return;
+    const float mine = 1.0f / l_run;
+#pragma unroll
+    for (int t = 0; t < D / 32; ++t)
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+        *reinterpret_cast<h4*>(out + ((size_t)query * heads + h) * D + t * 32 + g * 8 + 4 * half) =
+            h4{(_Float16)(o[t][4 * g] * mine), (_Float16)(o[t][4 * g + 1] * mine), (_Float16)(o[t][4 * g + 2] * mine), (_Float16)(o[t][4 * g + 3] * mine)};
+    return;
+  }
   // ---- merge: every wavefront scales its outputs to the common maximum and leaves them in LDS, where its tiles were
   if (half == 0) { s_m[wave][qi] = m_run; s_l[wave][qi] = l_run; }
   __syncthreads();
@@ -197,9 +212,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void prefill_attention_kernel(const
 #pragma unroll
   for (int w = 0; w < kWaves; ++w) l_all += s_l[w][qi] * __builtin_amdgcn_exp2f(s_m[w][qi] - m_all);
   const float mine = __builtin_amdgcn_exp2f(m_run - m_all) / l_all;
-  typedef float f32x4 __attribute__((ext_vector_type(4)));
   float* const O = reinterpret_cast<float*>(tiles[wave]);
-  // element r of tile t: dim t * 32 + (r / 4) * 8 + 4 * half + r % 4
 #pragma unroll
   for (int t = 0; t < D / 32; ++t)
 #pragma unroll
@@ -234,7 +247,9 @@ extern "C" int art_prefill_attention(const void* q_dev, const void* k_dev, const
   ART_REQUIRE(blocks <= 0x7fffffffLL, "art_prefill_attention: too many blocks");
   const unsigned chunks = (q_tiles + 7) / 8, rows = chunks < 32768 ? chunks : 32768;
   const unsigned a_chunk = chunks > 1 ? 8 * heads : (q_tiles * (heads & 7) + 7) / 8 * 8 + q_tiles * (heads & ~7);
-  prefill_attention_kernel<<<dim3(a_chunk, rows, (chunks + rows - 1) / rows), dim3(64 * kWaves), 0, (hipStream_t)stream>>>(
+  // one key tile: one wavefront, and no merge
+  const auto kernel = q_tiles == 1 ? prefill_attention_kernel<1> : prefill_attention_kernel<kMaxWaves>;
+  kernel<<<dim3(a_chunk, rows, (chunks + rows - 1) / rows), dim3(q_tiles == 1 ? 64 : 64 * kMaxWaves), 0, (hipStream_t)stream>>>(
       (const _Float16*)q_dev, (const _Float16*)k_dev, (const _Float16*)v_dev, (_Float16*)out_dev, T, heads, kv_row_stride,
       (const float*)att_f_dev, q_tiles);
   ART_LAUNCH_CHECK();
