@@ -149,10 +149,11 @@ __global__ __launch_bounds__(64 * kWaves, 2) void prefill_attention_kernel(const
 #pragma unroll
     for (int r = 0; r < 16; ++r) mx = fmaxf(mx, st[r]);
     mx = max_with_lane_xor_32(mx);
-    // key kt * 32 <= query for every query of this block's tile, so the maximum is finite from the first tile on
-    const float m_new = fmaxf(m_run, mx);
+    // The maximum may stay -infinity (a tile of infinitely negative scores is all that a wavefront has had so far): its terms
+    // are then 2^(-inf - 0) = 0.
+    const float m_new = fmaxf(m_run, mx), base = m_new == -INFINITY ? 0.f : m_new;
     if (__builtin_amdgcn_ballot_w64(m_new > m_run) != 0) {       // first tile: 2^(-inf) = 0
-      const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
+      const float alpha = __builtin_amdgcn_exp2f(m_run - base);
       l_run *= alpha;
 #pragma unroll
       for (int t = 0; t < D / 32; ++t)
@@ -163,7 +164,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void prefill_attention_kernel(const
     float p[16];
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-      p[r] = __builtin_amdgcn_exp2f(st[r] - m_new);              // masked: 2^(-inf) = 0
+      p[r] = __builtin_amdgcn_exp2f(st[r] - base);              // masked: 2^(-inf) = 0
       lsum += p[r];
     }
     l_run += sum_with_lane_xor_32(lsum);
@@ -206,7 +207,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void prefill_attention_kernel(const
   // ---- merge: every wavefront scales its outputs to the common maximum and leaves them in LDS, where its tiles were
   if (half == 0) { s_m[wave][qi] = m_run; s_l[wave][qi] = l_run; }
   __syncthreads();
-  float m_all = s_m[0][qi], l_all = 0.f;             // wavefront 0 has had tile 0: finite
+  float m_all = s_m[0][qi], l_all = 0.f;
 #pragma unroll
   for (int w = 1; w < kWaves; ++w) m_all = fmaxf(m_all, s_m[w][qi]);
 #pragma unroll

@@ -361,6 +361,32 @@ def test_causal_attention_of_any_number_of_heads(T, H):
     assert ((out.cpu().double() - exact).abs() <= 2.0 ** -10 * vc.double().abs().max() + 2.0 ** -10 * exact.abs()).all()
 
 
+@pytest.mark.parametrize('T', [32, 40, 150])
+def test_causal_attention_with_infinitely_negative_scores(T):
+    """Keys whose scores are -infinity count nothing, also where a whole tile of them is all that a wavefront sees first."""
+    import autort
+    dev = autort.device()
+    H, D = 2, 128
+    g = torch.Generator().manual_seed(T)
+    note(f'causal attention with infinite scores T={T}')
+    q, k, v = (torch.randn(T, H, D, generator=g).half() for _ in range(3))
+    q[:, :, 5] = 1.0
+    gone = torch.zeros(T, dtype=torch.bool)
+    gone[[3, 30]] = True
+    gone[32:64] = True
+    gone[96:127] = True
+    k[gone, :, 5] = float('-inf')
+    out = autort.ops.attention_causal_f16(q.to(dev), k.to(dev), v.to(dev), torch.tensor([1 / math.sqrt(D)], device=dev)).cpu().double()
+    sc = torch.einsum('thd,shd->hts', q.double(), k.double()) / math.sqrt(D)
+    sc = sc.masked_fill(torch.triu(torch.ones(T, T, dtype=torch.bool), 1), float('-inf'))
+    exact = torch.einsum('hts,shd->thd', torch.softmax(sc, -1), v.double())
+    assert exact.isfinite().all()
+    assert ((out - exact).abs() <= 2.0 ** -10 * v.double().abs().max() + 2.0 ** -10 * exact.abs()).all()
+    k[:, :, 5] = float('-inf')                               # nothing left: 0 / 0, as in the softmax itself
+    none = autort.ops.attention_causal_f16(q.to(dev), k.to(dev), v.to(dev), torch.tensor([1 / math.sqrt(D)], device=dev))
+    assert none.isnan().all()
+
+
 # the 16-byte form at its smallest and largest head, then heads and addresses it leaves to the one-pair-per-lane form
 @pytest.mark.parametrize('H,D,offset', [(1, 16, 0), (3, 256, 0), (33, 128, 0), (2, 72, 0), (2, 272, 0), (2, 128, 1)])
 def test_rope_qkv_store_rows_of_any_head_size(H, D, offset):
