@@ -107,7 +107,7 @@ bool describe_tensor(PyObject* o, Key& key, Slots& s) {
   const at::Tensor& t = THPVariable_Unpack(o);
   // wrappers of torch.func are plain tensors to Python and have no storage (vmap, grad, jvp) or no memory (functionalize)
   if (t.layout() != at::kStrided || !t.is_cuda() || !t.has_storage() || !t.is_contiguous()) return false;
-  const uintptr_t address = (uintptr_t)t.const_data_ptr();
+  const uintptr_t address = (uintptr_t)t.mutable_data_ptr();     // the call may write: a lazy copy gets its memory here
   if (address == 0 && t.numel() != 0) return false;
   const int device = t.device().index();
   if (s.device < 0) s.device = device;
@@ -283,7 +283,7 @@ PyObject* execute(const std::shared_ptr<Recipe>& keep, const Slots& s) {
   for (int i = 0; i < s.n; ++i) {
     pointer[i] = 0;
     PyObject* o = s.obj[i];
-    if (o && is_tensor(o)) pointer[i] = (uint64_t)(uintptr_t)THPVariable_Unpack(o).const_data_ptr();
+    if (o && is_tensor(o)) pointer[i] = (uint64_t)(uintptr_t)THPVariable_Unpack(o).mutable_data_ptr();
   }
   for (const auto& n : r.numbers)
     if (!pass_number(s.obj[n.first], n.second, slot_int[n.first], slot_float[n.first])) return nullptr;

@@ -231,3 +231,14 @@ def test_copies_of_an_operator_are_called_like_it(op):
     for twin in (copy.deepcopy(fresh), copy.copy(fresh), copy.copy(op)):
         assert all(torch.equal(twin(a, b), a + b) for _ in range(3))
     assert all(torch.equal(copy.deepcopy(norm)(a, None, b), norm(a, None, b)) for _ in range(2))
+
+
+def test_a_lazy_copy_is_written_apart_from_its_original(op):
+    import autort
+    dev = autort.device()
+    a, b, kept = torch.randn(1000, device=dev), torch.randn(1000, device=dev), torch.zeros(1000, device=dev)
+    for _ in range(3):
+        out = torch._lazy_clone(kept)
+        assert torch.equal(op(a, b, out=out), a + b) and not kept.any()
+        both = torch._lazy_clone(kept)
+        assert torch.equal(op(torch._lazy_clone(a), b, out=both), a + b) and not kept.any()
