@@ -16,8 +16,8 @@
 
 #include <ATen/hip/EmptyTensor.h>
 #include <c10/hip/HIPStream.h>
-#include <structmember.h>
 
+#include <cstddef>
 #include <memory>
 #include <string>
 #include <unordered_map>
@@ -54,7 +54,6 @@ struct Alloc {
 };
 struct Recipe {
   unsigned long long generation;
-  PyObject *tuned, *config, *fast_path;                  // identities only, never dereferenced as owners
   uint64_t tuned_version, config_version;
   int device;
   bool device_stream;                                    // the stream of the tensors' device, or of the current device
@@ -68,7 +67,7 @@ struct Recipe {
 
 struct Operator {
   PyObject_HEAD
-  PyObject *tuned, *config, *fast_path;                  // attributes a recipe depends on
+  PyObject *tuned, *config, *fast_path;                  // attributes a recipe depends on: setting one empties the table
   std::vector<PyObject*>* params;                        // interned names of the parameters
   std::vector<char>* dynamic;                            // list parameter whose numbers are not part of the signature
   std::unordered_map<std::string, std::shared_ptr<Recipe>>* table;
@@ -76,11 +75,15 @@ struct Operator {
   std::shared_ptr<Recipe>* last;
 };
 
-uint64_t version_of(PyObject* dict) { return dict && PyDict_CheckExact(dict) ? ((PyDictObject*)dict)->ma_version_tag : 0; }
+// What changes with every change of a dict; an object whose changes cannot be told never has the version it had.
+uint64_t version_of(PyObject* dict) {
+  static uint64_t never = 0;
+  if (!dict || dict == Py_None) return 0;
+  return PyDict_CheckExact(dict) ? ((PyDictObject*)dict)->ma_version_tag : --never;
+}
 
 bool current(const Operator* op, const Recipe& r) {
-  return r.generation == g_generation && r.tuned == op->tuned && r.config == op->config && r.fast_path == op->fast_path &&
-         r.tuned_version == version_of(op->tuned) && r.config_version == version_of(op->config);
+  return r.generation == g_generation && r.tuned_version == version_of(op->tuned) && r.config_version == version_of(op->config);
 }
 
 struct Slots {
@@ -383,9 +386,6 @@ PyObject* operator_commit(PyObject* self, PyObject* args) {
   if (!PyArg_ParseTuple(args, "y#iiiOOO", &key, &key_size, &slots, &device, &device_stream, &allocs, &launches, &results)) return nullptr;
   auto r = std::make_shared<Recipe>();
   r->generation = g_generation;
-  r->tuned = op->tuned;
-  r->config = op->config;
-  r->fast_path = op->fast_path;
   r->tuned_version = version_of(op->tuned);
   r->config_version = version_of(op->config);
   r->device = device;
@@ -521,11 +521,30 @@ void operator_dealloc(PyObject* self) {
   Py_TYPE(self)->tp_free(self);
 }
 
-PyMemberDef operator_members[] = {
-    {"tuned", T_OBJECT, offsetof(Operator, tuned), 0, "choices of tuning runs"},
-    {"config", T_OBJECT, offsetof(Operator, config), 0, "parsed config"},
-    {"fast_path", T_OBJECT, offsetof(Operator, fast_path), 0, "handler of a hand-written kernel, or None"},
-    {nullptr, 0, 0, 0, nullptr}};
+PyObject* attribute_get(PyObject* self, void* offset) {
+  PyObject* v = *(PyObject**)((char*)self + (size_t)offset);
+  if (!v) v = Py_None;
+  Py_INCREF(v);
+  return v;
+}
+
+int attribute_set(PyObject* self, PyObject* value, void* offset) {
+  Operator* op = (Operator*)self;
+  op->table->clear();
+  op->last->reset();
+  Py_XINCREF(value);
+  PyObject** field = (PyObject**)((char*)self + (size_t)offset);
+  PyObject* old = *field;
+  *field = value;
+  Py_XDECREF(old);
+  return 0;
+}
+
+PyGetSetDef operator_attributes[] = {
+    {"tuned", attribute_get, attribute_set, "choices of tuning runs", (void*)offsetof(Operator, tuned)},
+    {"config", attribute_get, attribute_set, "parsed config", (void*)offsetof(Operator, config)},
+    {"fast_path", attribute_get, attribute_set, "handler of a hand-written kernel, or None", (void*)offsetof(Operator, fast_path)},
+    {nullptr, nullptr, nullptr, nullptr, nullptr}};
 
 PyMethodDef operator_methods[] = {
     {"_commit", operator_commit, METH_VARARGS, "keep how a call of this signature is run"},
@@ -570,7 +589,7 @@ PyMODINIT_FUNC PyInit__calls(void) {
   OperatorType.tp_traverse = operator_traverse;
   OperatorType.tp_clear = operator_clear;
   OperatorType.tp_call = operator_call;
-  OperatorType.tp_members = operator_members;
+  OperatorType.tp_getset = operator_attributes;
   OperatorType.tp_methods = operator_methods;
   if (PyType_Ready(&OperatorType) < 0) return nullptr;
   PyObject* m = PyModule_Create(&module_def);

@@ -1,5 +1,6 @@
 """Calls replayed in native code, as far as that needs no GPU: what a recipe passes on to an entry point (here a
 recording callback), with arguments that are numbers."""
+import collections
 import copy
 import ctypes
 import pickle
@@ -257,3 +258,25 @@ def test_built_in_operators_can_be_pickled():
     for op in (builtin_ops.RmsNorm(torch.float32), builtin_ops.Rotary('rotary_f32', False), builtin_ops.GemvW4Fused(), builtin_ops.PartitionEvenFirst()):
         twin = pickle.loads(pickle.dumps(op))
         assert type(twin) is type(op) and vars(twin) == vars(op) and twin.tuned == op.tuned
+
+
+@pytest.mark.parametrize('attribute', ['fast_path', 'tuned', 'config'])
+def test_an_attribute_that_is_replaced_ends_the_recipes(attribute):
+    """Also where the new object takes the old one's place in memory."""
+    op = Recording('I')
+    for i in range(20):
+        setattr(op, attribute, None)
+        setattr(op, attribute, (lambda: i) if attribute == 'fast_path' else {'i': i})
+        for _ in range(3):
+            op(None, extra=[i])
+        assert op.python_calls == i + 1
+    if attribute != 'fast_path':
+        getattr(op, attribute)['i'] = 'changed'              # and one that is changed in place
+        op(None, extra=[1])
+        assert op.python_calls == 21
+        setattr(op, attribute, collections.OrderedDict(i=1))     # whose changes leave no trace
+        for _ in range(2):
+            op(None, extra=[1])
+        assert op.python_calls == 23
+    delattr(op, attribute)
+    assert getattr(op, attribute) is None
