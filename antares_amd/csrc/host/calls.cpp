@@ -14,7 +14,9 @@
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
+#include <ATen/Context.h>
 #include <ATen/hip/EmptyTensor.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
 
 #include <cstddef>
@@ -317,13 +319,20 @@ PyObject* execute(const std::shared_ptr<Recipe>& keep, const Slots& s) {
   return out;
 }
 
+// Where torch.empty is more than memory - a dispatch mode sees it, deterministic algorithms have it filled - results are made
+// by it, in the Python method.
+bool plain_allocations() {
+  const at::Context& context = at::globalContext();
+  return !c10::impl::TorchDispatchModeTLS::any_modes_set() && !(context.deterministicAlgorithms() && context.deterministicFillUninitializedMemory());
+}
+
 // C++ exceptions of torch (no storage, out of memory, no device) leave as the Python exceptions that torch makes of them.
 PyObject* operator_call(PyObject* self, PyObject* args, PyObject* kwargs) {
   HANDLE_TH_ERRORS
   Operator* op = (Operator*)self;
   Key key;
   Slots s;
-  const bool known = signature(op, args, kwargs, key, s);
+  const bool known = plain_allocations() && signature(op, args, kwargs, key, s);
   if (known) {
     const char* bytes = (const char*)key.word;
     const size_t size = (size_t)key.n * sizeof(int64_t);

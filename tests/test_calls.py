@@ -8,6 +8,7 @@ import sys
 
 import pytest
 import torch
+import torch.utils._python_dispatch
 
 from antares_amd.autort import builtin_ops, patterns
 from antares_amd.autort.op import ExportedOp
@@ -280,3 +281,27 @@ def test_an_attribute_that_is_replaced_ends_the_recipes(attribute):
         assert op.python_calls == 23
     delattr(op, attribute)
     assert getattr(op, attribute) is None
+
+
+def test_calls_under_a_dispatch_mode_or_with_filled_memory_are_not_replayed():
+    class Mode(torch.utils._python_dispatch.TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+    op = Recording('I')
+    op(None, extra=[1])
+    op(None, extra=[2])
+    assert op.python_calls == 1
+    with Mode():
+        op(None, extra=[3])
+        op(None, extra=[4])
+    assert op.python_calls == 3
+    before = torch.are_deterministic_algorithms_enabled()
+    try:
+        torch.use_deterministic_algorithms(True)
+        op(None, extra=[5])
+        op(None, extra=[6])
+    finally:
+        torch.use_deterministic_algorithms(before)
+    assert op.python_calls == 5
+    op(None, extra=[7])
+    assert op.python_calls == 5 and op.seen == [1, 2, 3, 4, 5, 6, 7]
