@@ -1,7 +1,7 @@
 """Operators that ship with the package: the fused partition and the Llama
 decode operators.  Each is a thin Python wrapper that checks shapes on the
 host and calls one typed entry point of libantares_amd.so; a call whose
-signature has been seen before is replayed in native code (runtime/calls.py)."""
+signature has a recipe is replayed in native code (runtime/calls.py)."""
 from __future__ import annotations
 
 import torch
@@ -18,7 +18,7 @@ def _require_cuda(*tensors):
             raise RuntimeError('autort built-in operators need GPU tensors; there is no CPU fallback')
         if not t.is_contiguous():
             raise ValueError('autort built-in operators need dense (contiguous) tensors')
-    capi.init(tensors[0].device.index or 0)
+    capi.init(tensors[0].get_device())
 
 
 def _run(op, pending, result, fn, *args):
@@ -571,7 +571,7 @@ class RopeQkvStoreRows(calls.Operator):
     name = 'rope_qkv_store_rows_f16'
 
     def __init__(self):
-        self._bind(('qkv', 'inv_freq', 'q_out', 'key_cache', 'val_cache', 'extra'), ())
+        self._bind(('qkv', 'inv_freq', 'q_out', 'key_cache', 'val_cache', 'extra'), ('extra',))
 
     def _call(self, pending, qkv, inv_freq, q_out, key_cache, val_cache, extra=None):
         T, heads, head_dim = q_out.shape
@@ -580,7 +580,7 @@ class RopeQkvStoreRows(calls.Operator):
         for t in (qkv, inv_freq, q_out, key_cache, val_cache):
             if t.dtype != torch.float16:
                 raise TypeError(f'{self.name}: tensors must be float16')
-        first = int(extra[0]) if extra else 0
+        first = Number(int(extra[0]), 6, 'I') if extra else 0
         _require_cuda(qkv, inv_freq, q_out, key_cache, val_cache)
         return _run(self, pending, q_out, capi.lib().art_rope_qkv_store_rows, qkv, inv_freq, q_out, key_cache, val_cache, T, heads, head_dim, first,
                     key_cache.numel() // (heads * head_dim))

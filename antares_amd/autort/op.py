@@ -105,8 +105,8 @@ class ExportedOp(calls.Operator):
                          for i, (ix, dim) in enumerate(zip(st.out_index, self.fused.tensors[st.output].shape))
                          if ix.kind == 'axis' and dict(st.data_axes).get(ix.name, dim) != dim]
         # the call's arguments in order: tensors by position (no keyword has a name that starts with `/`), the last
-        # output also as `out`; `extra` is taken and ignored
-        self._bind(tuple(['/' + n for n in self.declared + self.fresh_outputs[:-1]] + ['out', 'extra']), ())
+        # output also as `out`; `extra` is taken and ignored, whatever its numbers
+        self._bind(tuple(['/' + n for n in self.declared + self.fresh_outputs[:-1]] + ['out', 'extra']), ('extra',))
 
     # -- persistence ---------------------------------------------------------
     def persist(self) -> Optional[str]:
@@ -172,15 +172,16 @@ class ExportedOp(calls.Operator):
             else:
                 bound[n] = torch.empty(want, dtype=self._wanted_dtype[n][0], device=dev)
         capi.init(dev.index or 0)
-        for t in bound.values():
-            calls.address(t)
+        trials = self.config.get('tune')
+        if trials:                                 # a search launches on these tensors by itself
+            for t in bound.values():
+                calls.address(t)
         call = calls.Call(current_stream_handle(dev.index))
         if self.fast_path is None or not self.fast_path(self, bound, env, call):
             self._run_generic(bound, env, dev, call)
         outs = [bound[o] for o in self.graph.outputs]
         # a call under capture could not search its launch parameters: it leaves no recipe, a later one still may
-        trials = self.config.get('tune')
-        if not (isinstance(trials, int) and trials > 0 and torch.cuda.is_current_stream_capturing()):
+        if pending is not None and not (isinstance(trials, int) and trials > 0 and torch.cuda.is_current_stream_capturing()):
             call.keep(self, pending, outs, device_stream=True)
         return outs[0] if len(outs) == 1 else tuple(outs)
 

@@ -3,11 +3,11 @@
 // An operator call from Python used to cost 9 to 10 us of host time (argument checks, shape look-ups, output
 // allocation through torch.empty, ctypes conversions), more than most of the kernels it launches.  What a call does
 // depends only on the dtypes, shapes, devices, contiguity and 16-byte alignment of its tensors, on which of them share
-// memory and on which arguments are given, so the Python side works it out once per such signature - a recipe: outputs and intermediates to allocate,
-// kernels and library entry points to call, and where each argument comes from - and this file replays it: signature,
-// look-up, allocation, launches.  Anything unusual (an argument that is no plain tensor, a signature not seen before)
-// goes to the operator's Python method, which checks everything and raises the errors; a recipe holds no data and no
-// result, only how to compute it.
+// memory and on which arguments are given, so the Python side works it out once per such signature - a recipe: outputs and
+// intermediates to allocate, kernels and library entry points to call, and where each argument comes from - when the
+// signature is met for the second time, and this file replays it: signature, look-up, allocation, launches.  Anything
+// unusual (an argument that is no plain tensor, a new signature) goes to the operator's Python method, which checks
+// everything and raises the errors; a recipe holds no data and no result, only how to compute it.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
@@ -22,6 +22,7 @@
 #include <cstddef>
 #include <memory>
 #include <string>
+#include <string_view>
 #include <unordered_map>
 #include <vector>
 
@@ -30,7 +31,11 @@ namespace {
 constexpr int kMaxSlots = 24;            // flattened arguments of a call
 constexpr int kMaxInts = 20;             // integer and pointer arguments of a library entry point
 constexpr int kMaxFloats = 4;
-constexpr size_t kMaxRecipes = 256;      // per operator; the table is emptied when it is full
+// A recipe costs as much to make as a call without one (attention over a cache that grows: 10 us of host time a call, 17 with a
+// recipe made each time, 4 replayed): it is made when a signature is met again.  The table holds the positions of a long
+// sequence; it is emptied when it is full.
+constexpr size_t kMaxRecipes = 8192;     // per operator
+constexpr size_t kMet = 8192;            // signatures that are remembered, by a part of their hash
 
 PyObject* g_error = nullptr;             // ArtError
 PyObject* g_parameter = nullptr;         // torch.nn.Parameter
@@ -73,6 +78,7 @@ struct Operator {
   std::vector<PyObject*>* params;                        // interned names of the parameters
   std::vector<char>* dynamic;                            // list parameter whose numbers are not part of the signature
   std::unordered_map<std::string, std::shared_ptr<Recipe>>* table;
+  std::vector<uint32_t>* met;
   std::string* last_key;
   std::shared_ptr<Recipe>* last;
 };
@@ -86,6 +92,17 @@ uint64_t version_of(PyObject* dict) {
 
 bool current(const Operator* op, const Recipe& r) {
   return r.generation == g_generation && r.tuned_version == version_of(op->tuned) && r.config_version == version_of(op->config);
+}
+
+// Whether this signature has been met before (now it has); two may be taken for one another, which only costs time.
+bool met_before(Operator* op, const char* bytes, size_t size) {
+  const uint64_t h = std::hash<std::string_view>{}(std::string_view(bytes, size));
+  if (op->met->empty()) op->met->resize(kMet);
+  uint32_t& place = (*op->met)[h % kMet];
+  const uint32_t mark = (uint32_t)(h >> 32) | 1;
+  if (place == mark) return true;
+  place = mark;
+  return false;
 }
 
 struct Slots {
@@ -332,7 +349,7 @@ PyObject* operator_call(PyObject* self, PyObject* args, PyObject* kwargs) {
   Operator* op = (Operator*)self;
   Key key;
   Slots s;
-  const bool known = plain_allocations() && signature(op, args, kwargs, key, s);
+  bool known = plain_allocations() && signature(op, args, kwargs, key, s);
   if (known) {
     const char* bytes = (const char*)key.word;
     const size_t size = (size_t)key.n * sizeof(int64_t);
@@ -347,6 +364,7 @@ PyObject* operator_call(PyObject* self, PyObject* args, PyObject* kwargs) {
       *op->last = r;
       return execute(r, s);
     }
+    known = it != op->table->end() || met_before(op, bytes, size);
   }
   // not seen before: the Python method runs the call and, where it can, leaves a recipe (commit) for this signature
   static PyObject* name = PyUnicode_InternFromString("_call");
@@ -496,6 +514,7 @@ PyObject* operator_new(PyTypeObject* type, PyObject*, PyObject*) {
   op->params = new std::vector<PyObject*>();
   op->dynamic = new std::vector<char>();
   op->table = new std::unordered_map<std::string, std::shared_ptr<Recipe>>();
+  op->met = new std::vector<uint32_t>();
   op->last_key = new std::string();
   op->last = new std::shared_ptr<Recipe>();
   return (PyObject*)op;
@@ -525,6 +544,7 @@ void operator_dealloc(PyObject* self) {
   delete op->params;
   delete op->dynamic;
   delete op->table;
+  delete op->met;
   delete op->last_key;
   delete op->last;
   Py_TYPE(self)->tp_free(self);

@@ -2,9 +2,9 @@
 
 ``Operator`` (``csrc/host/calls.cpp``) is the base class of everything callable in ``autort.ops``.  A call whose
 signature - dtypes, shapes, devices, contiguity and 16-byte alignment of the tensors, which of them share memory, which
-arguments are given - has been seen before is replayed from a recipe without entering Python; any other call reaches the subclass's ``_call(pending,
-...)``, which checks the arguments, runs the operator and leaves the recipe with ``pending`` (None when the arguments are
-nothing a recipe can be kept for).
+arguments are given - has a recipe is replayed from it without entering Python; any other call reaches the subclass's
+``_call(pending, ...)``, which checks the arguments, runs the operator and leaves the recipe with ``pending`` (None when the
+signature is met for the first time or the arguments are nothing a recipe can be kept for).
 """
 from __future__ import annotations
 
@@ -71,6 +71,7 @@ class Stream:
 
 
 STREAM = Stream()
+_Tensor = torch.Tensor
 
 
 class Number:
@@ -97,18 +98,28 @@ class Call:
     """What one call of an operator launches, in order: kernels and entry points of the library, with tensors as
     tensors, the stream as STREAM, list numbers as Number, and constants."""
 
+    __slots__ = ('stream', 'steps')
+
     def __init__(self, stream: int):
         self.stream = stream
         self.steps = []
 
     def library(self, fn, *args):
-        values = [c_void_p(address(a)) if isinstance(a, torch.Tensor) else c_void_p(self.stream) if a is STREAM else
-                  a.value if isinstance(a, Number) else c_void_p(0) if a is None else a for a in args]
+        values = [a if a.__class__ is int else (a.data_ptr() or address(a)) if a.__class__ is _Tensor else self._value(a) for a in args]
         self.steps.append((fn, None, None, args))
-        capi.check(fn(*values))
+        rc = fn(*values)
+        if rc:
+            capi.check(rc)
+
+    def _value(self, a):
+        if a is STREAM:
+            return self.stream
+        if isinstance(a, _Tensor):
+            return address(a)
+        return a.value if a.__class__ is Number else a
 
     def kernel(self, func, grid: int, block: int, args):
-        values = [address(a) if isinstance(a, torch.Tensor) else a for a in args]
+        values = [a if a.__class__ is int else a.data_ptr() or address(a) for a in args]
         self.steps.append((func, (grid, 1, 1), (block, 1, 1), args))
         capi.launch(func, (grid, 1, 1), (block, 1, 1), self.stream, values)
 

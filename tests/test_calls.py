@@ -41,24 +41,25 @@ class Recording(calls.Operator):
 @pytest.mark.parametrize('values', [(5, 6, 2 ** 31 - 1, -1, 0), (5.0, 6.0, 7.9, -7.9, 0.0), (True, False, True)])
 def test_a_whole_number_is_passed_on_whatever_kind_of_number_it_is(values):
     op = Recording('I')
-    for v in values:
+    for v in values * 2:
         op(None, extra=[v])
         op(extra=(v,))
-    assert op.seen == [int(v) for v in values for _ in range(2)]
+    assert op.seen == [int(v) for v in values * 2 for _ in range(2)] and op.python_calls <= 4
 
 
 def test_a_position_that_changes_its_kind():
     op = Recording('I')
-    for v in (5, 6.0, 7, 8.0, 9.5, True, 10):
+    for v in (5, 6.0, 7, 8.0, 9.5, True, 10, 11.5, 12) * 2:
         op(None, extra=[v])
-    assert op.seen == [5, 6, 7, 8, 9, 1, 10]
+    assert op.seen == [5, 6, 7, 8, 9, 1, 10, 11, 12] * 2
 
 
 def test_a_float_is_passed_on_whatever_kind_of_number_it_is():
     op = Recording('F')
-    for v in (0.5, 0.25, 3, 4, 1e30):
+    values = (0.5, 0.25, 3, 4, 1e30) * 3
+    for v in values:
         op(None, extra=[v])
-    assert op.seen == [ctypes.c_float(float(v)).value for v in (0.5, 0.25, 3, 4, 1e30)]
+    assert op.seen == [ctypes.c_float(float(v)).value for v in values] and op.python_calls == 4
 
 
 def test_a_number_that_is_none_raises_what_it_raises_at_the_first_call():
@@ -175,6 +176,7 @@ def test_an_error_of_torch_in_a_replayed_call_is_a_python_exception():
             call.keep(self, pending, [], device_stream=False)
     op = Streaming()
     op(None)
+    op(None)
     for _ in range(3):
         with pytest.raises(RuntimeError):               # no device, hence no current stream
             op(None)
@@ -204,15 +206,16 @@ def test_arguments_live_until_the_call_is_over(as_list):
     extra = [value] if as_list else (value,)
 
     def during():
-        if op.seen[1:] and as_list:
+        if op.seen[2:] and as_list:
             extra.clear()
         counts.append(sys.getrefcount(value))
     op = Recording('F', during)
+    op(None, extra=[value])
     op(None, extra=[value])                              # leaves the recipe
     counts.clear()
     before = sys.getrefcount(value)
     op(None, extra=extra)
-    assert op.seen == [1234.5] * 2 and op.python_calls == 1
+    assert op.seen == [1234.5] * 3 and op.python_calls == 2
     assert counts == [before + (0 if as_list else 1)]           # the list's reference is gone, the call's is there
     assert sys.getrefcount(value) == before - as_list
 
@@ -247,12 +250,13 @@ def test_operators_can_be_copied(make, duplicate):
 def test_a_copy_is_called_like_the_operator_it_is_a_copy_of():
     op = Recording('I')
     op(None, extra=[1])
+    op(None, extra=[2])
     twin = copy.copy(op)
-    twin(None, extra=[2])
-    twin(extra=[3], x=None)
-    twin(None, extra=[4])
-    op(None, extra=[5])
-    assert op.seen == [1, 2, 3, 4, 5] and (op.python_calls, twin.python_calls) == (1, 2)
+    for i in (3, 4, 5):
+        twin(None, extra=[i])
+    twin(extra=[6], x=None)
+    op(None, extra=[7])
+    assert op.seen == [1, 2, 3, 4, 5, 6, 7] and (op.python_calls, twin.python_calls) == (2, 4)
 
 
 def test_built_in_operators_can_be_pickled():
@@ -270,15 +274,15 @@ def test_an_attribute_that_is_replaced_ends_the_recipes(attribute):
         setattr(op, attribute, (lambda: i) if attribute == 'fast_path' else {'i': i})
         for _ in range(3):
             op(None, extra=[i])
-        assert op.python_calls == i + 1
+        assert op.python_calls == i + 2
     if attribute != 'fast_path':
         getattr(op, attribute)['i'] = 'changed'              # and one that is changed in place
         op(None, extra=[1])
-        assert op.python_calls == 21
+        assert op.python_calls == 22
         setattr(op, attribute, collections.OrderedDict(i=1))     # whose changes leave no trace
         for _ in range(2):
             op(None, extra=[1])
-        assert op.python_calls == 23
+        assert op.python_calls == 24
     delattr(op, attribute)
     assert getattr(op, attribute) is None
 
@@ -288,13 +292,13 @@ def test_calls_under_a_dispatch_mode_or_with_filled_memory_are_not_replayed():
         def __torch_dispatch__(self, func, types, args=(), kwargs=None):
             return func(*args, **(kwargs or {}))
     op = Recording('I')
-    op(None, extra=[1])
-    op(None, extra=[2])
-    assert op.python_calls == 1
+    for i in (0, 1, 2):
+        op(None, extra=[i])
+    assert op.python_calls == 2
     with Mode():
         op(None, extra=[3])
         op(None, extra=[4])
-    assert op.python_calls == 3
+    assert op.python_calls == 4
     before = torch.are_deterministic_algorithms_enabled()
     try:
         torch.use_deterministic_algorithms(True)
@@ -302,6 +306,24 @@ def test_calls_under_a_dispatch_mode_or_with_filled_memory_are_not_replayed():
         op(None, extra=[6])
     finally:
         torch.use_deterministic_algorithms(before)
-    assert op.python_calls == 5
+    assert op.python_calls == 6
     op(None, extra=[7])
-    assert op.python_calls == 5 and op.seen == [1, 2, 3, 4, 5, 6, 7]
+    assert op.python_calls == 6 and op.seen == [0, 1, 2, 3, 4, 5, 6, 7]
+
+
+def test_a_recipe_is_made_when_a_signature_is_met_again():
+    """Making one costs as much as a call: a call whose signature is another one every time leaves none."""
+    class Sized(calls.Operator):
+        def __init__(self):
+            self.pending = 0
+            self._bind(('x', 'size'), ())
+
+        def _call(self, pending, x=None, size=None):
+            self.pending += pending is not None
+    op = Sized()
+    for size in range(1000):
+        op(None, size)
+    assert op.pending < 10                               # the marks are 32 bits of a hash
+    for size in range(1000):
+        op(None, size)
+    assert op.pending > 800                              # two signatures in one place take it from each other

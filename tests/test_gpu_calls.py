@@ -104,7 +104,7 @@ def test_a_position_may_be_any_number(name, positions):
     print(f'[case] {name} {positions}', flush=True)
     dev = autort.device()
     x, inv = torch.randn(2, 2, 64, device=dev), torch.rand(128, device=dev)
-    for pos in positions:
+    for pos in positions * 3:
         angle = float(int(pos)) * inv[:64]
         if name == 'rotary_f32':
             want = torch.cat([x[:, 0] * angle.cos() - x[:, 1] * angle.sin(), x[:, 1] * angle.cos() + x[:, 0] * angle.sin()], 1)
@@ -138,7 +138,7 @@ def test_a_tensor_of_positions_in_the_place_of_the_list():
     import autort
     dev = autort.device()
     x, inv = torch.randn(2, 2, 64, device=dev), torch.rand(128, device=dev)
-    for pos in (3, 4):
+    for pos in (3, 4, 5, 6):
         got = autort.ops.rotary_f32(x, inv, torch.empty(2, 128, device=dev), extra=torch.tensor([pos], dtype=torch.int32, device=dev))
         assert torch.equal(got, autort.ops.rotary_f32(x, inv, torch.empty(2, 128, device=dev), extra=[pos]))
 
@@ -147,8 +147,8 @@ def test_errors_of_torch_are_python_exceptions_in_replayed_calls_too(op):
     import autort
     dev = autort.device()
     big = torch.zeros(32 << 20, device=dev)
-    op(big, big)
-    op(big, big)
+    for _ in range(3):
+        op(big, big)
     for transform in (lambda f: torch.vmap(f)(torch.zeros(2, 64, device=dev)), lambda f: torch.func.functionalize(f)(torch.zeros(64, device=dev)),
                       lambda f: torch.func.grad(lambda x: f(x).sum())(torch.zeros(64, device=dev))):
         with pytest.raises(RuntimeError):
@@ -192,7 +192,7 @@ def test_a_convolution_over_its_image_and_one_apart_from_it_do_not_depend_on_eac
         image = memory[:x.numel()].view_as(x).copy_(x)
         at = {'over': 0, 'apart': None, 'behind': x.numel()}[where]        # behind: the first element past the image
         check(op(image, w.to(dev), out=None if at is None else memory[at:at + x.numel()].view_as(x)))
-    assert sorted(taken) == [False, True, True]          # one recipe each: by hand where the memory is apart
+    assert sorted(taken) == [False] * 2 + [True] * 4     # a recipe each, made at the second call: by hand where the memory is apart
 
 
 def test_which_tensors_share_memory_is_part_of_the_signature():
@@ -205,8 +205,11 @@ def test_which_tensors_share_memory_is_part_of_the_signature():
             self._bind(('a', 'b', 'c', 'extra'), ())
 
         def _call(self, pending, *args, **kwargs):
-            return pending[0]
-    key = Keys()
+            return pending and pending[0]
+    op = Keys()
+
+    def key(*args, **kwargs):
+        return op(*args, **kwargs) or op(*args, **kwargs)          # pending when the signature is met again
     m = torch.zeros(64, device=dev)
     a, b, c = m[0:16], m[16:32], m[32:48]
     base = key(a, b, c)
@@ -237,8 +240,28 @@ def test_a_lazy_copy_is_written_apart_from_its_original(op):
     import autort
     dev = autort.device()
     a, b, kept = torch.randn(1000, device=dev), torch.randn(1000, device=dev), torch.zeros(1000, device=dev)
-    for _ in range(3):
+    for _ in range(4):
         out = torch._lazy_clone(kept)
         assert torch.equal(op(a, b, out=out), a + b) and not kept.any()
         both = torch._lazy_clone(kept)
         assert torch.equal(op(torch._lazy_clone(a), b, out=both), a + b) and not kept.any()
+
+
+def test_a_growing_cache_and_a_first_position_that_moves_on():
+    """Attention over a row more every time (another signature), and rows stored at another position (a number of `extra`)."""
+    import autort
+    dev = autort.device()
+    q, k, v, f = torch.randn(2, 128, device=dev), torch.randn(20, 2, 128, device=dev), torch.randn(20, 2, 128, device=dev), torch.tensor([0.1], device=dev)
+    qkv, inv = torch.randn(3, 3 * 256, device=dev).half(), torch.rand(128, device=dev).half()
+    qo, kc, vc = torch.zeros(3, 2, 128, device=dev).half(), torch.zeros(20, 256, device=dev).half(), torch.zeros(20, 256, device=dev).half()
+    for _ in range(3):
+        for s in range(1, 21):
+            want = torch.einsum('hs,shd->hd', torch.softmax(torch.einsum('hd,shd->hs', q, k[:s]) * 0.1, -1), v[:s])
+            assert torch.allclose(autort.ops.attention_f32(q, k[:s], v[:s], f), want, rtol=1e-4, atol=1e-5)
+        for first in (0, 5, 17, 2.0):
+            vc.zero_()
+            autort.ops.rope_qkv_store_rows_f16(qkv, inv, qo, kc, vc, extra=[first])
+            assert torch.equal(vc[int(first):int(first) + 3], qkv[:, 512:]) and vc.any(1).sum() == 3
+        for outside in (18, -1):
+            with pytest.raises(RuntimeError):
+                autort.ops.rope_qkv_store_rows_f16(qkv, inv, qo, kc, vc, extra=[outside])
