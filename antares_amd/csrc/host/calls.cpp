@@ -161,9 +161,10 @@ bool describe_overlaps(Key& key, const Slots& s) {
 bool describe(PyObject* o, bool dynamic, bool nested, Key& key, Slots& s) {
   if (s.n == kMaxSlots) return false;
   s.obj[s.n++] = o;
-  if (o == nullptr || o == Py_None) return key.put(0);
+  if (o == nullptr) return key.put(0);                   // not given: another call than with None, maybe one argument short
+  if (o == Py_None) return key.put(8);
   if (is_tensor(o)) return describe_tensor(o, key, s);
-  if (PyBool_Check(o)) return key.put(2 | (int64_t)(o == Py_True) << 8);
+  if (PyBool_Check(o)) return key.put(dynamic ? 2 : 2 | (int64_t)(o == Py_True) << 8);
   if (PyLong_CheckExact(o)) {
     if (dynamic) return key.put(3);
     int overflow = 0;

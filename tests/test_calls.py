@@ -327,3 +327,30 @@ def test_a_recipe_is_made_when_a_signature_is_met_again():
     for size in range(1000):
         op(None, size)
     assert op.pending > 800                              # two signatures in one place take it from each other
+
+
+def test_an_argument_that_is_missing_is_not_one_that_is_none():
+    entry = ctypes.CFUNCTYPE(ctypes.c_int)(lambda: 0)
+
+    class Two(calls.Operator):
+        def __init__(self):
+            self._bind(('a', 'b', 'c'), ())
+
+        def _call(self, pending, a, b, c=None):
+            call = calls.Call(0)
+            call.library(entry)
+            call.keep(self, pending, [], device_stream=False)
+    op = Two()
+    for _ in range(4):
+        op(None, None)
+        op(b=None, a=None)
+        with pytest.raises(TypeError):
+            op(None)
+        with pytest.raises(TypeError):
+            op(b=None)
+        with pytest.raises(TypeError):
+            op(None, None, None, None)
+        with pytest.raises(TypeError):
+            op(None, None, a=None)
+        with pytest.raises(TypeError):
+            op(None, None, d=None)
