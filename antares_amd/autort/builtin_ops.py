@@ -43,7 +43,7 @@ class PartitionEvenFirst(calls.Operator):
     def __init__(self):
         self.tuned = {}                                 # str(n) -> {'value': cap on blocks, 'us': ...}
         self._loaded = False
-        self._bind(('x', 'out', 'extra'), ())
+        self._bind(('x', 'out', 'extra'), ('extra',))
 
     def _saved(self):
         """Winners of earlier tuning runs, kept in the operator store as `partition_even_first_i32.tuned.json`."""
@@ -207,7 +207,7 @@ class DecodeAttention(calls.Operator):
 
     def __init__(self, name: str):
         self.name = name
-        self._bind(('q', 'k', 'v', 'att_f', 'out', 'extra'), ())
+        self._bind(('q', 'k', 'v', 'att_f', 'out', 'extra'), ('extra',))
 
     def _call(self, pending, q, k, v, att_f, out=None, extra=None):
         if q.dim() != 2 or k.dim() != 3 or k.shape != v.shape or k.shape[1:] != q.shape:
@@ -233,7 +233,7 @@ class CausalAttention(calls.Operator):
     name = 'attention_causal_f16'
 
     def __init__(self):
-        self._bind(('q', 'k', 'v', 'att_f', 'out', 'extra'), ())
+        self._bind(('q', 'k', 'v', 'att_f', 'out', 'extra'), ('extra',))
 
     def _call(self, pending, q, k, v, att_f, out=None, extra=None):
         if q.dim() != 3 or k.dim() != 3 or k.shape != v.shape or k.shape[1:] != q.shape[1:] or k.shape[0] < q.shape[0]:
@@ -282,7 +282,7 @@ class GemvW4Fused(calls.Operator):
 
     def __init__(self):
         self._bind(('x', 'qweight', 'scales', 'qzeros', 'out', 'norm_weight', 'residual', 'eps', 'swiglu', 'extra', 'sumsq_in', 'sumsq_out',
-                    'sumsq_clear'), ())
+                    'sumsq_clear'), ('extra',))
 
     def _call(self, pending, x, qweight, scales, qzeros, out=None, norm_weight=None, residual=None, eps=RMS_EPS, swiglu=False,
                  extra=None, sumsq_in=None, sumsq_out=None, sumsq_clear=None):
@@ -350,7 +350,7 @@ class GemvW4Packed(calls.Operator):
     name = 'gemv_w4p'
 
     def __init__(self):
-        self._bind(('x', 'packed', 'out', 'norm_weight', 'residual', 'eps', 'swiglu_out', 'shape', 'extra'), ())
+        self._bind(('x', 'packed', 'out', 'norm_weight', 'residual', 'eps', 'swiglu_out', 'shape', 'extra'), ('extra',))
 
     def _call(self, pending, x, packed, out=None, norm_weight=None, residual=None, eps=RMS_EPS, swiglu_out=False, shape=None, extra=None):
         K, N = shape if shape is not None else getattr(packed, 'w4_shape', (None, None))
@@ -399,7 +399,7 @@ class AttentionRope(calls.Operator):
     name = 'attention_rope_f16'
 
     def __init__(self):
-        self._bind(('qkv', 'inv_freq', 'key_cache', 'val_cache', 'att_f', 'out', 'extra'), ())
+        self._bind(('qkv', 'inv_freq', 'key_cache', 'val_cache', 'att_f', 'out', 'extra'), ('extra',))
 
     def _call(self, pending, qkv, inv_freq, key_cache, val_cache, att_f, out, extra=None):
         heads, head_dim = out.shape
@@ -425,7 +425,7 @@ class AttentionRopeSplit(calls.Operator):
     name = 'attention_rope_split_f16'
 
     def __init__(self):
-        self._bind(('qkv', 'inv_freq', 'key_cache', 'val_cache', 'att_f', 'partial', 'extra'), ())
+        self._bind(('qkv', 'inv_freq', 'key_cache', 'val_cache', 'att_f', 'partial', 'extra'), ('extra',))
 
     def _call(self, pending, qkv, inv_freq, key_cache, val_cache, att_f, partial, extra=None):
         if partial.dim() != 3 or partial.shape[2] != 132 or partial.dtype != torch.float32:
@@ -549,7 +549,7 @@ class RopeQkvStore(calls.Operator):
 
     def __init__(self, name):
         self.name = name
-        self._bind(('qkv', 'inv_freq', 'q_out', 'key_cache', 'val_cache', 'extra'), ())
+        self._bind(('qkv', 'inv_freq', 'q_out', 'key_cache', 'val_cache', 'extra'), ('extra',))
 
     def _call(self, pending, qkv, inv_freq, q_out, key_cache, val_cache, extra=None):
         heads, head_dim = q_out.shape
