@@ -119,7 +119,7 @@ class Call:
         return a.value if a.__class__ is Number else a
 
     def kernel(self, func, grid: int, block: int, args):
-        values = [a if a.__class__ is int else a.data_ptr() or address(a) for a in args]
+        values = [a if a.__class__ is int else (a.data_ptr() or address(a)) if a.__class__ is _Tensor else self._value(a) for a in args]
         self.steps.append((func, (grid, 1, 1), (block, 1, 1), args))
         capi.launch(func, (grid, 1, 1), (block, 1, 1), self.stream, values)
 
