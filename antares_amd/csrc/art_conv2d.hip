@@ -21,7 +21,7 @@
 //     per 64 bytes of channels (18 to 72 matrix instructions per wavefront and barrier for a 3 x 3 filter, not 2 to 8);
 //   * 2 x 2 wavefronts of MT x NT tiles of 32 features x 32 points; blocks of one run of points are neighbours on one XCD.
 // Measured, padding 1, both launches, against the generic lowering (a padded copy, then a gathering product): float16
-// 32 x 128 x 28 x 28 -> 128 41.4 -> 21.1 us, 24 x 200 x 33 x 33 -> 48 89 -> 23 us, 2 x 160 x 18 x 18 -> 64 57 -> 14 us;
+// 32 x 128 x 28 x 28 -> 128 40.2 -> 20.1 us, 24 x 200 x 33 x 33 -> 48 89 -> 23 us, 2 x 160 x 18 x 18 -> 64 57 -> 14 us;
 // float32 32 x 128 x 28 x 28 -> 128 113 -> 81 us (the matrix instructions alone take 47), 23 x 128 x 30 x 30 -> 176 119 -> 86.
 // The first of these spends 7 us of the matrix cores' time in 18.6 us: one block per compute unit and only 4 chunks, so the
 // first image fetch, the waits between chunks and the stores of 12.8 MB stay in sight; packing the filter takes 2.3 us.

@@ -10,7 +10,7 @@
 //     groups.  Wavefront (c, h) multiplies 32 columns by the k half h of every group, so every weight is unpacked once per
 //     block; the two k halves meet in LDS after the loop.  What bounds the loop is the issue of instructions, not the
 //     matrix cores (with the MFMAs taken out a group takes as long): a wavefront issues one per 7 cycles or so, and a
-//     group is 140 / 160 / 205 of them at MT = 1 / 2 / 4, two thirds of them unpacking - 1090 / 1200 / 1460 cycles.
+//     group is 137 / 158 / 201 of them at MT = 1 / 2 / 4, 84 of them vector instructions that unpack - 1090 / 1200 / 1460 cycles.
 //     Sixteen wavefronts with half the work each were slower (the LDS meeting doubles), and so were four column quarters
 //     replaced by two (same loop, longer meeting), blocks that start at groups of their own, and branches around the
 //     loads of the last groups;
@@ -25,9 +25,10 @@
 //   * split-K without atomics (5.6 M float atomics cost 75 us on this chip): each K-split writes its fp32 tile to the
 //     library workspace and a second small kernel adds the splits in a fixed order and rounds once to fp16 - results
 //     do not depend on timing.
-// Before (blocks of 256 columns, a k half of 64 columns per wavefront, x operands permuted instead of weights): 64 rows over
-// 4096 x 4096 / 4096 x 22016 / 11008 x 4096 took 13.6 / 28.9 / 17.2 us, now 11.9 / 22.9 / 16.2; 128 rows over 4096 x 12288 / 22016
-// 27.4 / 40.2, now 21.9 / 32; 16 rows over 1024 x 3072 8.3, now 6.9.
+// Before (blocks of 256 columns, a k half of 64 columns per wavefront, x operands permuted instead of weights) and now, on one
+// card, weights from memory: 64 rows over 4096 x 4096 / 4096 x 22016 / 11008 x 4096 13.6 / 28.6 / 18.2 us -> 11.2 / 22.4 / 16.9;
+// 50 rows over 11008 x 4096 17.9 -> 16.2; 128 rows over 4096 x 12288 / 22016 28.1 / 40.0 -> 22.3 / 31.2; 16 rows over
+// 1024 x 3072 7.4 -> 6.8.
 #include "art_w4_mfma.h"
 
 #include <type_traits>
@@ -308,7 +309,7 @@ __global__ __launch_bounds__(256) void gemm_w4a16_combine_kernel(const float* __
 // The same with the RMSNorm that follows (norm_out = fp16(y / rms(y) * weight), from the rounded y): a block owns a row, whose
 // elements stay in registers, 8 per thread and turn (N % 8 == 0, N <= 8192; as many threads as a row of up to 4096 has
 // pieces of 8).  Bound by the launch: instead of two launches of 2 us and more, one; a layer of the 32-layer model's prompt pass has
-// two of them: 8 layers 611 -> 596 us at 8 tokens, 938 -> 911 at 100, 1318 -> 1311 at 200 (fewer K-splits meet).
+// two of them: 8 layers 608 -> 594 us at 8 tokens, 776 -> 750 at 50, 962 -> 925 at 100, 1345 -> 1337 at 200 (fewer K-splits meet).
 constexpr int kNormThreads = 512, kNormTurns = 2;
 __global__ __launch_bounds__(kNormThreads) void gemm_w4a16_combine_norm_kernel(const float* __restrict__ partial, _Float16* y, int N,
                                                                                 long long split_stride, int splits, const _Float16* residual,
@@ -450,7 +451,7 @@ int run_rows(const _Float16* xs, const unsigned char* qweight, const _Float16* s
   Plan p;
   ART_REQUIRE(choose(p, M, K, N, swiglu, scratch_bytes, art::compute_units(), code, splits), "art_gemm_w4a16: K=%d N=%d are too large", K, N);
   // Where K-splits meet in a pass of their own, the norm is part of that pass, up to 256 rows: beyond them
-  // nothing is gained (8 layers of 4096 columns: 966 -> 944 us at 100 rows, 1881 -> 1879 at 300).
+  // nothing is gained (8 layers of the same pass: 1384 -> 1368 us at 256 tokens, 1861 and 1854 at 300, 2178 and 2183 at 500).
   const bool norm_there = norm && p.splits > 1 && M <= 256 && N % 8 == 0 && N <= 8 * kNormThreads * kNormTurns &&
                           (((uintptr_t)ys | (uintptr_t)res | (uintptr_t)norm->weight | (uintptr_t)norm->out) % 16) == 0;
   if (p.wide) {

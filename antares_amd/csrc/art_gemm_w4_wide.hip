@@ -8,19 +8,21 @@
 //     unit, MT = 8: 256 and one wavefront per SIMD).  No two wavefronts unpack the same weight.  What bounds the loop is
 //     the issue of vector instructions beside the MFMAs: one wavefront alone gets four of them into the shadow of an
 //     MFMA (32 cycles) and pays 7 cycles for every further one, two wavefronts get six each.  Hence pairs of k in
-//     natural order (one v_perm more per pair of weights) instead of a permutation of every x operand: 2.9 vector
-//     instructions per MFMA at MT = 8 against 4.6 (90 us against 103 for 1003 rows over 4096 x 4096);
+//     natural order (one v_perm more per pair of weights) instead of a permutation of every x operand: the loop has 2.3
+//     vector instructions per MFMA at MT = 8 and 4.7 at MT = 4 (counted over a launch 2.6 and 5.6 to 6.3);
 //   * per 64 values of k a block needs 8 KiB of packed weights, 4 MT KiB of x and the group's scales and zero points;
 //     they go from global memory straight into LDS (global_load_lds, no registers in flight), a ring of three slots.
 //     The weights run a stage ahead of x, so that the first operands of a stage can be unpacked in the stage before;
 //   * the chunk positions are swizzled so that every 16 lanes of a 16-byte read of x (rows 128 bytes apart), and of a
-//     transposing byte read of the weights, touch every bank once (SQ_LDS_BANK_CONFLICT 5.9 M -> 0.3 M per launch);
+//     transposing byte read of the weights, touch every bank once (SQ_LDS_BANK_CONFLICT 0.5 M cycles in a launch of 33 M
+//     wavefront cycles, 1003 rows over 4096 x 12288);
 //   * one round = 16 values of k per lane half = 2 MT MFMAs.  The operands of round e + 1 are read and unpacked between
 //     the MFMAs of round e, in four chunks fenced against the scheduler; each chunk also issues at most one load.  Left
-//     together the loads of a stage blocked every wavefront of the compute unit at once (about 700 cycles per stage:
-//     90 -> 71 us).
-// Measured (MI355X, 1003 rows): 4096 x 12288 93 us = 1.09 PFLOP/s, 4096 x 22016 166 us, 11008 x 4096 96 us, 4096 x 4096
-// 46 us with two K-splits; the 64-row blocks of art_gemm_w4.hip: 156, 248, 130 and 62 us.
+//     together the loads of a stage blocked every wavefront of the compute unit at once, about 700 cycles per stage.
+// Measured (MI355X, 1003 rows, weights from memory): 4096 x 12288 93 us = 1.08 PFLOP/s (matrix cores busy 0.77 of the time),
+// 4096 x 22016 166 us; the 64-row blocks of art_gemm_w4.hip take 131 and 233 us, its 128-row blocks 112 and 211, and the
+// kernel there was before this one (64 rows x 256 columns) took 157 and 246.  4096 columns are too few for blocks of 256:
+// 4096 x 4096 takes 45 us here and 37.5 with 128 x 128 blocks, 11008 x 4096 97 and 92.
 #include "art_w4_mfma.h"
 
 #include <type_traits>

@@ -137,7 +137,8 @@ int art_gemv_w4a16(const void* x_dev, const void* qweight_dev, const void* scale
  *                  plus 256 for blocks of 32 rows, 512 for 64, 1280 for 128 (all over 128 columns), 1024 for 128 or 2048 for
  *                  256 rows over 256 columns (none: the library picks): more rows per block unpack a weight for more
  *                  row tiles, fewer make more blocks, which need fewer K-splits, i.e. fewer fp32 copies of the output
- *                  written and read back;
+ *                  written and read back.  Blocks that cannot number or address the columns (65536 tiles of 128) are
+ *                  replaced by ones that can;
  *   max_blocks:    cap on the blocks of the partition, 64..16384 (each walks its span tile by tile). */
 int art_gemv_w4a16_tuned(const void* x_dev, const void* qweight_dev, const void* scales_dev, const void* qzeros_dev,
                          void* y_dev, int M, int K, int N, int k_per_block, void* stream);

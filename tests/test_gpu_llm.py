@@ -315,7 +315,7 @@ def test_fused_decode_attention_against_the_oracle(parts, pos):
 @pytest.mark.usefixtures('oracle_built')
 @pytest.mark.parametrize('T,H', [(1, 4), (5, 4), (31, 4), (32, 32), (33, 4), (100, 32), (128, 32), (200, 4), (384, 32)])
 def test_causal_attention_over_a_prompt_against_the_oracle(T, H):
-    """attention_causal_f16 (matrix cores, one wavefront per 32 queries) against the oracle's attention applied position by
+    """attention_causal_f16 (matrix cores, a block of 32 queries) against the oracle's attention applied position by
     position: query t sees rows 0..t of cache views that have more rows than the prompt."""
     import autort
     from oracle import hot_ops
