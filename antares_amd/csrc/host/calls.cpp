@@ -477,7 +477,10 @@ PyObject* operator_commit(PyObject* self, PyObject* args) {
     if (v >= tensors) { PyErr_SetString(PyExc_IndexError, "commit: a result that does not exist"); return nullptr; }
     r->results.push_back(v);
   }
-  if (op->table->size() >= kMaxRecipes) op->table->clear();
+  if (op->table->size() >= kMaxRecipes) {
+    op->table->clear();
+    op->met->clear();
+  }
   std::string k(key, (size_t)key_size);
   (*op->table)[k] = r;
   *op->last_key = std::move(k);

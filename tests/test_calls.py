@@ -354,3 +354,29 @@ def test_an_argument_that_is_missing_is_not_one_that_is_none():
             op(None, None, a=None)
         with pytest.raises(TypeError):
             op(None, None, d=None)
+
+
+def test_the_table_is_emptied_when_it_is_full():
+    entry = ctypes.CFUNCTYPE(ctypes.c_int, ctypes.c_int)(lambda n: seen.append(n) or 0)
+
+    class Sized(calls.Operator):
+        def __init__(self):
+            self.python_calls = 0
+            self._bind(('size',), ())
+
+        def _call(self, pending, size):
+            self.python_calls += 1
+            call = calls.Call(0)
+            call.library(entry, size)
+            call.keep(self, pending, [], device_stream=False)
+    op, seen = Sized(), []
+    for size in range(9000):
+        for _ in range(3):
+            op(size)
+    assert seen == [size for size in range(9000) for _ in range(3)] and op.python_calls == 18000
+    op(8999)                                             # made after the table was emptied
+    assert op.python_calls == 18000
+    op(0)
+    op(0)
+    op(0)
+    assert op.python_calls == 18002
