@@ -373,10 +373,11 @@ struct Plan {
   bool wide;
   int row_tiles, splits;
 };
-// What a launch takes, in microseconds: a fixed part, one or two co-resident blocks' time per group and round, and for
-// K-splits the second launch and the fp32 tiles.  Fitted to 1500 launches of 4 to 1003 rows over eight weight shapes
-// (1024 x 3072 to 4096 x 22016, 11008 x 4096, 8704 x 704) on MI355X: 8 % off in the mean, and the form it picks is within
-// 1 % of the fastest one in the mean.
+// What a launch takes, in microseconds: a fixed part, one or two co-resident blocks' time per group and round, the ramp and
+// the meeting of the k halves again for every further round of blocks of 128 columns (4 rows over 4096 x 12288: 13.3 us with
+// 480 blocks, i.e. 5 K-splits in one round, 14.6 with 768), and for K-splits the second launch and the fp32 tiles.  Against
+// 7200 launches of 4 to 1003 rows over 18 weight shapes (512 x 512 to 11008 x 12288, 4096 x 22016, 8704 x 704) on MI355X it
+// is 7 % off in the mean, and the form it picks 1.2 % slower than the fastest one.
 double estimate(int M, int K, int N, const Plan& p, int compute_units) {
   struct Cost { double fixed, one, two; int per_cu; };
   const Cost c = p.wide ? (p.row_tiles == 8 ? Cost{6.5, 2.06, 2.08, 1} : Cost{4.3, 1.37, 2.23, 2})
@@ -387,7 +388,8 @@ double estimate(int M, int K, int N, const Plan& p, int compute_units) {
   double per_group = blocks / round * c.two;
   if (rest > compute_units) per_group += c.two;
   else if (rest > 0) per_group += c.per_cu == 2 || blocks > round ? c.one : c.one + (c.two - c.one) * rest / compute_units;
-  return c.fixed + groups * per_group + (p.splits > 1 ? 2.4 + (8.0 * p.splits + 2.0) * M * N / 4.4e6 : 0.0);
+  const double again = p.wide ? 0.0 : 1.5 * ((blocks - 1) / round);
+  return c.fixed + again + groups * per_group + (p.splits > 1 ? 2.4 + (8.0 * p.splits + 2.0) * M * N / 4.4e6 : 0.0);
 }
 // What a form's 32-bit offsets (a block's rows of x and of the packed weights) and its division by the number of column
 // tiles hold.
