@@ -295,26 +295,40 @@ long long blocks_of(const Geometry& g, int form) {
   return (long long)((g.columns + points_of(form) - 1) / points_of(form)) * ((g.F + features_of(form) - 1) / features_of(form));
 }
 
-// The form for these sizes, or 0: the generic kernels are faster or sum more exactly there.  Lines from sweeps of 90 sizes
-// (C 16-256, F 16-256, images of 7-56 squared, batches 1-32), times in us generic / here.
+// What a launch of a form takes, in microseconds, up to a part that is the same for all of them: blocks go to the compute
+// units in rounds that last as long full or not (the blocks of a unit share its matrix cores), and a round is a ramp and its
+// chunks.  Fitted to 250 sizes (C 16-256, F 16-256, images of 7-56 squared, batches 1-32): float32 1.7 % off,
+// float16 3.7 %; the form it picks is 0.1 % (float32) and 0.5 % slower than the fastest one in the mean.  Float32: 23 x 128 ->
+// 80, 38 x 38 takes 111 / 124 / 150 us in 1038 / 520 / 260 blocks (5, 3, 2 rounds), 11 x 144 -> 232, 28 x 28 79 / 95 / 90 us in
+// 540 / 272 / 136 (3, 2, 1); float16: 32 x 128 -> 128, 28 x 28 27.1 / 21.7 / 21.1 us in 784 / 392 / 196.
+constexpr int kUnits = 256;                      // compute units of an MI355X
+double launch_time(const Geometry& g, int f16, int form) {
+  struct Cost { double fixed, chunk, round; };
+  static const Cost cost[2][3] = {{{6.9, 2.74, -0.65}, {8.3, 5.11, -1.82}, {8.7, 9.09, -1.55}},
+                                  {{7.4, 1.36, -0.46}, {8.2, 2.14, -0.98}, {9.3, 2.79, -1.08}}};
+  const Cost& c = cost[f16 != 0][form - 1];
+  return c.fixed + (double)((blocks_of(g, form) + kUnits - 1) / kUnits) * (g.chunks * c.chunk + c.round);
+}
+
+// The form for these sizes, or 0: the generic kernels are faster or sum more exactly there.  Lines from sweeps of the sizes
+// above, times in us generic / here.
 //  * fewer than 32 features, or fewer than 16 blocks of 64 x 64: the generic path sums on the vector units in short
 //    chains.  In float32 that error (0.8e-7 against 64 bits) is below the matrix instructions' (1.3e-7): left alone.  In
 //    float16 it is the same (0.7-1.1e-7 both) from 64 channels on, and the times are 62 / 16 (1 x 224 -> 24, 35 x 35) and
 //    120 / 14 (2 x 128 -> 24, 46 x 46); below 8192 results the generic path wins (7 / 9 for 7 x 40 -> 16, 7 x 7).
 //  * from 1024 terms per result on the generic path slices the sum over an idle chip: 13 / 18 (float16, 5 x 216 -> 40,
-//    14 x 14, 16 blocks), 22 / 14 at 144 blocks; float32 23 / 43 at 40 blocks, 80 / 55 at 475.
-//  * 64 x 128 from 128 such blocks on (float16, 150 blocks: 28.8 with 64 x 64, 27.1; 92 blocks: 18.7, 21.0), 128 x 128
-//    from 192 on where it pads no more features (32 x 128 -> 128, 28 x 28: 27.1, 21.7, 21.1).
+//    14 x 14, 16 blocks), 22 / 14 at 144 blocks; float32 23 / 43 at 40 blocks, 62 / 51 at 204.  (Just past
+//    one round it is faster again, 73 / 84 at 300 blocks, 74 / 67 at 381, with twice the error: not left to it.)
+//  * below 32 features only 64 x 64, whose rows of taps are summed by themselves: the larger blocks' error is 1.2e-7.
 int choose(const Geometry& g, int f16) {
-  const long long small = blocks_of(g, 1);
+  const long long small = blocks_of(g, 1), results = (long long)g.columns * g.F;
   const bool vector_units = g.F < 32 || small < 16;
-  if (vector_units && (!f16 || (long long)g.columns * g.F < 8192 || (g.F < 32 && g.C < 64))) return 0;
+  if (vector_units && (!f16 || results < 8192 || (g.F < 32 && g.C < 64))) return 0;
   if (!vector_units && 9LL * g.C >= 1024 && small < (f16 ? 64 : 192)) return 0;
-  if (g.F >= 32) {
-    if ((g.F + 127) / 128 * 2 == (g.F + 63) / 64 && blocks_of(g, 3) >= 192 && fits(g, 3)) return 3;
-    if (blocks_of(g, 2) >= 128 && fits(g, 2)) return 2;
-  }
-  return fits(g, 1) ? 1 : 0;
+  int best = 0;
+  for (int form = 1; form <= (g.F < 32 ? 1 : 3); ++form)
+    if (fits(g, form) && (!best || launch_time(g, f16, form) < launch_time(g, f16, best))) best = form;
+  return best;
 }
 
 template <typename T, int MT, int NT>
