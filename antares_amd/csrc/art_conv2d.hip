@@ -19,6 +19,8 @@
 //     operand is one contiguous kilobyte that comes from L2 straight into registers, a tap ahead of its use;
 //   * the next 64 bytes of channels travel to registers while these are multiplied, two LDS buffers, one LDS-only barrier
 //     per 64 bytes of channels (18 to 72 matrix instructions per wavefront and barrier for a 3 x 3 filter, not 2 to 8);
+//   * a last chunk of which only the lower half exists is multiplied without the upper half (64-feature blocks): float32
+//     20 x 24 -> 64, 20 x 20 12.0 -> 10.5 us (generic 11.4), float16 19 x 19 of 16 channels 8.8 -> 7.3 (7.7 to 8.4);
 //   * 2 x 2 wavefronts of MT x NT tiles of 32 features x 32 points; blocks of one run of points are neighbours on one XCD.
 // Measured, padding 1, both launches, against the generic lowering (a padded copy, then a gathering product): float16
 // 32 x 128 x 28 x 28 -> 128 40.2 -> 20.1 us, 24 x 200 x 33 x 33 -> 48 89 -> 23 us, 2 x 160 x 18 x 18 -> 64 57 -> 14 us;
@@ -196,19 +198,22 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 4))
     for (int j = 0; j < NT; ++j)
 #pragma unroll
       for (int e = 0; e < 16; ++e) total[i][j][e] = 0.f;
-  auto chunk = [&](int q, auto last_chunk) {
+  // `half`: only the lower half of the (last) chunk's channels exist, the upper half's products are left out
+  auto chunk = [&](int q, auto last_chunk, auto half) {
     constexpr bool kMore = !decltype(last_chunk)::value;
+    constexpr int kHalves = decltype(half)::value ? 1 : 2;
     const T* tile = image + (size_t)(q & 1) * g.span * kPitch;
     // a chunk is summed by itself and then added to the total (where registers allow, a row of taps by itself before
     // that): the error of a sum grows with the length of its chain
     f32x16 acc[MT][NT], row[MT][NT];
     vec b[2][NT];
-    auto look = [&](int h, int t) {
+    auto look = [&](int step) {                       // the points of half `step % kHalves` of a tap
+      const int t = step / kHalves, h = step % kHalves;
       const T* from = tile + ((t / 3) * wide + t % 3) * kPitch;
 #pragma unroll
-      for (int j = 0; j < NT; ++j) b[h][j] = *reinterpret_cast<const vec*>(from + at[j] + h * 2 * V);
+      for (int j = 0; j < NT; ++j) b[step & 1][j] = *reinterpret_cast<const vec*>(from + at[j] + h * 2 * V);
     };
-    look(0, 0);
+    look(0);
 #pragma unroll
     for (int t = 0; t < kTaps; ++t) {
       if (kMore) {
@@ -218,13 +223,14 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 4))
       if (kMore || t + kAhead < kTaps) fetch_filter((t + kAhead) % kSets, q * kTaps + t + kAhead);
       __builtin_amdgcn_sched_barrier(0);              // left to the scheduler, the loads sink to their use
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        if (h == 0 || t + 1 < kTaps) look(h ^ 1, t + h);        // the other half, or the next tap's first
+      for (int h = 0; h < kHalves; ++h) {
+        const int step = t * kHalves + h;
+        if (step + 1 < kTaps * kHalves) look(step + 1);
 #pragma unroll
         for (int i = 0; i < MT; ++i)
 #pragma unroll
           for (int j = 0; j < NT; ++j)
-            row[i][j] = Elem<T>::multiply(a[t % kSets][i][h], b[h][j], h == 0 && t % kSum == 0 ? f32x16(0) : row[i][j]);
+            row[i][j] = Elem<T>::multiply(a[t % kSets][i][h], b[step & 1][j], h == 0 && t % kSum == 0 ? f32x16(0) : row[i][j]);
       }
       if (t % kSum != kSum - 1) continue;
 #pragma unroll
@@ -243,8 +249,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 4))
       art_lds_barrier();      // the other buffer is written, this one is free
     }
   };
-  for (int q = 0; q + 1 < g.chunks; ++q) chunk(q, std::false_type{});
-  chunk(g.chunks - 1, std::true_type{});
+  for (int q = 0; q + 1 < g.chunks; ++q) chunk(q, std::false_type{}, std::false_type{});
+  if (MT == 1 && g.C - (g.chunks - 1) * 4 * V <= 2 * V) chunk(g.chunks - 1, std::true_type{}, std::true_type{});   // MT = 2 has no registers left for it
+  else chunk(g.chunks - 1, std::true_type{}, std::false_type{});
 
   // accumulator element e: feature (e / 4) * 8 + (lane / 32) * 4 + e % 4 of the tile, point lane % 32
 #pragma unroll
@@ -307,7 +314,9 @@ double launch_time(const Geometry& g, int f16, int form) {
   static const Cost cost[2][3] = {{{6.9, 2.74, -0.65}, {8.3, 5.11, -1.82}, {8.7, 9.09, -1.55}},
                                   {{7.4, 1.36, -0.46}, {8.2, 2.14, -0.98}, {9.3, 2.79, -1.08}}};
   const Cost& c = cost[f16 != 0][form - 1];
-  return c.fixed + (double)((blocks_of(g, form) + kUnits - 1) / kUnits) * (g.chunks * c.chunk + c.round);
+  const int per_chunk = f16 ? 32 : 16;
+  const double chunks = g.chunks - (form < 3 && g.C - (g.chunks - 1) * per_chunk <= per_chunk / 2 ? 0.5 : 0.0);
+  return c.fixed + (double)((blocks_of(g, form) + kUnits - 1) / kUnits) * (chunks * c.chunk + c.round);
 }
 
 // The form for these sizes, or 0: the generic kernels are faster or sum more exactly there.  Lines from sweeps of the sizes
