@@ -303,20 +303,24 @@ long long blocks_of(const Geometry& g, int form) {
 }
 
 // What a launch of a form takes, in microseconds, up to a part that is the same for all of them: blocks go to the compute
-// units in rounds that last as long full or not (the blocks of a unit share its matrix cores), and a round is a ramp and its
-// chunks.  Fitted to 250 sizes (C 16-256, F 16-256, images of 7-56 squared, batches 1-32): float32 1.7 % off,
-// float16 3.7 %; the form it picks is 0.1 % (float32) and 0.5 % slower than the fastest one in the mean.  Float32: 23 x 128 ->
-// 80, 38 x 38 takes 111 / 124 / 150 us in 1038 / 520 / 260 blocks (5, 3, 2 rounds), 11 x 144 -> 232, 28 x 28 79 / 95 / 90 us in
-// 540 / 272 / 136 (3, 2, 1); float16: 32 x 128 -> 128, 28 x 28 27.1 / 21.7 / 21.1 us in 784 / 392 / 196.
+// units in rounds, and a round is a ramp and its chunks.  In float32 a round lasts as long full or not (the blocks of a unit
+// share its matrix cores); in float16, where they mostly wait, half of the last round is paid by its blocks.  Fitted to 350
+// sizes in float32 and 260 in float16 (C 16-256, F 16-256, images of 7-56 squared, batches 1-32): 2.4 and 4.1 % off, and the
+// form it picks is 0.2 and 0.3 % slower than the fastest one in the mean.  Float32: 23 x 128 -> 80, 38 x 38 takes 111 / 124 /
+// 150 us in 1038 / 520 / 260 blocks (5, 3, 2 rounds), 11 x 144 -> 232, 28 x 28 79 / 95 / 90 us in 540 / 272 / 136 (3, 2, 1);
+// float16: 32 x 128 -> 128, 28 x 28 27.1 / 21.7 / 21.1 us in 784 / 392 / 196, 13 x 24 -> 88, 39 x 39 11.9 / 10.7 / 11.7 in
+// 618 / 310 / 155.
 constexpr int kUnits = 256;                      // compute units of an MI355X
 double launch_time(const Geometry& g, int f16, int form) {
   struct Cost { double fixed, chunk, round; };
   static const Cost cost[2][3] = {{{6.9, 2.74, -0.65}, {8.3, 5.11, -1.82}, {8.7, 9.09, -1.55}},
-                                  {{7.4, 1.36, -0.46}, {8.2, 2.14, -0.98}, {9.3, 2.79, -1.08}}};
+                                  {{7.1, 1.43, -0.31}, {8.35, 2.12, -1.15}, {8.9, 2.80, -0.80}}};
   const Cost& c = cost[f16 != 0][form - 1];
   const int per_chunk = f16 ? 32 : 16;
   const double chunks = g.chunks - (form < 3 && g.C - (g.chunks - 1) * per_chunk <= per_chunk / 2 ? 0.5 : 0.0);
-  return c.fixed + (double)((blocks_of(g, form) + kUnits - 1) / kUnits) * (chunks * c.chunk + c.round);
+  const long long blocks = blocks_of(g, form), whole = (blocks + kUnits - 1) / kUnits;
+  const double rounds = f16 && whole > 1 ? 0.5 * ((double)blocks / kUnits + whole) : (double)whole;
+  return c.fixed + rounds * (chunks * c.chunk + c.round);
 }
 
 // The form for these sizes, or 0: the generic kernels are faster or sum more exactly there.  Lines from sweeps of the sizes
