@@ -23,11 +23,15 @@ def _require_cuda(*tensors):
 
 def _run(op, pending, result, fn, *args):
     """Calls a library entry point on the current stream and leaves the recipe of the call with the operator."""
-    call = calls.Call(current_stream_handle())
+    stream = current_stream_handle()
+    if pending is None:
+        capi.check(fn(*calls.values(args, stream), stream))
+        return result
+    call = calls.Call(stream)
     call.library(fn, *args, STREAM)
     # a tensor that the entry point does not take may have had its value read here (a number given as a tensor), which is
     # another one in the next call: no recipe
-    if pending is not None and not any(isinstance(t, torch.Tensor) and t.numel() and t is not result and all(t is not a for a in args) for t in pending[1]):
+    if not any(isinstance(t, torch.Tensor) and t.numel() and t is not result and all(t is not a for a in args) for t in pending[1]):
         call.keep(op, pending, [result], device_stream=False)
     return result
 

@@ -4,10 +4,10 @@
 // allocation through torch.empty, ctypes conversions), more than most of the kernels it launches.  What a call does
 // depends only on the dtypes, shapes, devices, contiguity and 16-byte alignment of its tensors, on which of them share
 // memory and on which arguments are given, so the Python side works it out once per such signature - a recipe: outputs and
-// intermediates to allocate, kernels and library entry points to call, and where each argument comes from - when the
-// signature is met for the second time, and this file replays it: signature, look-up, allocation, launches.  Anything
-// unusual (an argument that is no plain tensor, a new signature) goes to the operator's Python method, which checks
-// everything and raises the errors; a recipe holds no data and no result, only how to compute it.
+// intermediates to allocate, kernels and library entry points to call, and where each argument comes from - and this file
+// replays it: signature, look-up, allocation, launches.  Anything unusual (an argument that is no plain tensor, a new
+// signature) goes to the operator's Python method, which checks everything and raises the errors; a recipe holds no data
+// and no result, only how to compute it.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
@@ -31,9 +31,11 @@ namespace {
 constexpr int kMaxSlots = 24;            // flattened arguments of a call
 constexpr int kMaxInts = 20;             // integer and pointer arguments of a library entry point
 constexpr int kMaxFloats = 4;
-// A recipe costs as much to make as a call without one (attention over a cache that grows: 10 us of host time a call, 17 with a
-// recipe made each time, 4 replayed): it is made when a signature is met again.  The table holds the positions of a long
-// sequence; it is emptied when it is full.
+// A recipe costs as much to make as a call without one (attention over a cache that grows: 9 us of host time a call, 17 with a
+// recipe made each time, 4 replayed).  An operator whose last kCredit recipes have not been used is called with another
+// signature every time: it gets one only when a signature is met again.  The table holds the positions of a long sequence;
+// it is emptied when it is full.
+constexpr int kCredit = 8;
 constexpr size_t kMaxRecipes = 8192;     // per operator
 constexpr size_t kMet = 8192;            // signatures that are remembered, by a part of their hash
 
@@ -69,7 +71,7 @@ struct Recipe {
   std::vector<Launch> launches;
   std::vector<std::pair<int, bool>> numbers;             // slots whose numbers are passed on; true: as a float
   std::vector<int> results;
-  bool uses_stream;
+  bool uses_stream, used;
 };
 
 struct Operator {
@@ -78,6 +80,7 @@ struct Operator {
   std::vector<PyObject*>* params;                        // interned names of the parameters
   std::vector<char>* dynamic;                            // list parameter whose numbers are not part of the signature
   std::unordered_map<std::string, std::shared_ptr<Recipe>>* table;
+  int credit;                                            // recipes that may still be made on first sight: one less each, one more with its use
   std::vector<uint32_t>* met;
   std::string* last_key;
   std::shared_ptr<Recipe>* last;
@@ -103,6 +106,13 @@ bool met_before(Operator* op, const char* bytes, size_t size) {
   if (place == mark) return true;
   place = mark;
   return false;
+}
+
+void renew(Operator* op) {                               // nothing is known about the operator's calls
+  op->table->clear();
+  op->last->reset();
+  op->met->clear();
+  op->credit = kCredit;
 }
 
 struct Slots {
@@ -344,6 +354,11 @@ bool plain_allocations() {
   return !c10::impl::TorchDispatchModeTLS::any_modes_set() && !(context.deterministicAlgorithms() && context.deterministicFillUninitializedMemory());
 }
 
+void use(Operator* op, Recipe& r) {
+  if (!r.used && op->credit < kCredit) ++op->credit;
+  r.used = true;
+}
+
 // C++ exceptions of torch (no storage, out of memory, no device) leave as the Python exceptions that torch makes of them.
 PyObject* operator_call(PyObject* self, PyObject* args, PyObject* kwargs) {
   HANDLE_TH_ERRORS
@@ -356,6 +371,7 @@ PyObject* operator_call(PyObject* self, PyObject* args, PyObject* kwargs) {
     const size_t size = (size_t)key.n * sizeof(int64_t);
     if (*op->last && op->last_key->size() == size && memcmp(op->last_key->data(), bytes, size) == 0 && current(op, **op->last)) {
       std::shared_ptr<Recipe> r = *op->last;
+      use(op, *r);
       return execute(r, s);
     }
     auto it = op->table->find(std::string(bytes, size));
@@ -363,11 +379,15 @@ PyObject* operator_call(PyObject* self, PyObject* args, PyObject* kwargs) {
       std::shared_ptr<Recipe> r = it->second;
       *op->last_key = it->first;
       *op->last = r;
+      use(op, *r);
       return execute(r, s);
     }
-    known = it != op->table->end() || met_before(op, bytes, size);
+    if (it == op->table->end() && !met_before(op, bytes, size)) {
+      known = op->credit > 0;
+      if (known) --op->credit;
+    }
   }
-  // not seen before: the Python method runs the call and, where it can, leaves a recipe (commit) for this signature
+  // no recipe: the Python method runs the call and, where it can and is asked to (`known`), leaves one (commit)
   static PyObject* name = PyUnicode_InternFromString("_call");
   PyObject* pending;
   if (known) {
@@ -418,7 +438,7 @@ PyObject* operator_commit(PyObject* self, PyObject* args) {
   r->config_version = version_of(op->config);
   r->device = device;
   r->device_stream = device_stream != 0;
-  r->uses_stream = false;
+  r->uses_stream = r->used = false;
   r->slots = slots;
   if (!PyList_Check(allocs) || !PyList_Check(launches) || !PyList_Check(results) || PyList_GET_SIZE(allocs) > kMaxSlots) {
     PyErr_SetString(PyExc_TypeError, "commit: allocs (at most 24), launches and results are lists");
@@ -477,10 +497,7 @@ PyObject* operator_commit(PyObject* self, PyObject* args) {
     if (v >= tensors) { PyErr_SetString(PyExc_IndexError, "commit: a result that does not exist"); return nullptr; }
     r->results.push_back(v);
   }
-  if (op->table->size() >= kMaxRecipes) {
-    op->table->clear();
-    op->met->clear();
-  }
+  if (op->table->size() >= kMaxRecipes) renew(op);
   std::string k(key, (size_t)key_size);
   (*op->table)[k] = r;
   *op->last_key = std::move(k);
@@ -497,8 +514,7 @@ PyObject* operator_bind(PyObject* self, PyObject* args) {
   for (PyObject* p : *op->params) Py_DECREF(p);
   op->params->clear();
   op->dynamic->clear();
-  op->table->clear();
-  op->last->reset();
+  renew(op);
   for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(names); ++i) {
     PyObject* n = PyTuple_GET_ITEM(names, i);
     if (!PyUnicode_Check(n)) { PyErr_SetString(PyExc_TypeError, "bind: names are strings"); return nullptr; }
@@ -519,6 +535,7 @@ PyObject* operator_new(PyTypeObject* type, PyObject*, PyObject*) {
   op->dynamic = new std::vector<char>();
   op->table = new std::unordered_map<std::string, std::shared_ptr<Recipe>>();
   op->met = new std::vector<uint32_t>();
+  op->credit = kCredit;
   op->last_key = new std::string();
   op->last = new std::shared_ptr<Recipe>();
   return (PyObject*)op;
@@ -563,8 +580,7 @@ PyObject* attribute_get(PyObject* self, void* offset) {
 
 int attribute_set(PyObject* self, PyObject* value, void* offset) {
   Operator* op = (Operator*)self;
-  op->table->clear();
-  op->last->reset();
+  renew(op);
   Py_XINCREF(value);
   PyObject** field = (PyObject**)((char*)self + (size_t)offset);
   PyObject* old = *field;

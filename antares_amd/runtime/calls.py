@@ -3,8 +3,8 @@
 ``Operator`` (``csrc/host/calls.cpp``) is the base class of everything callable in ``autort.ops``.  A call whose
 signature - dtypes, shapes, devices, contiguity and 16-byte alignment of the tensors, which of them share memory, which
 arguments are given - has a recipe is replayed from it without entering Python; any other call reaches the subclass's
-``_call(pending, ...)``, which checks the arguments, runs the operator and leaves the recipe with ``pending`` (None when the
-signature is met for the first time or the arguments are nothing a recipe can be kept for).
+``_call(pending, ...)``, which checks the arguments, runs the operator and leaves the recipe with ``pending`` (None when none
+is wanted, or the arguments are nothing a recipe can be kept for).
 """
 from __future__ import annotations
 
@@ -94,6 +94,19 @@ def address(t: torch.Tensor) -> int:
     return at
 
 
+def _value(a, stream: int):
+    if a is STREAM:
+        return stream
+    if isinstance(a, _Tensor):
+        return address(a)
+    return a.value if a.__class__ is Number else a
+
+
+def values(args, stream: int) -> list:
+    """Arguments as ctypes takes them: tensors by their address, STREAM as the handle, a Number as its value."""
+    return [a if a.__class__ is int else (a.data_ptr() or address(a)) if a.__class__ is _Tensor else _value(a, stream) for a in args]
+
+
 class Call:
     """What one call of an operator launches, in order: kernels and entry points of the library, with tensors as
     tensors, the stream as STREAM, list numbers as Number, and constants."""
@@ -105,23 +118,14 @@ class Call:
         self.steps = []
 
     def library(self, fn, *args):
-        values = [a if a.__class__ is int else (a.data_ptr() or address(a)) if a.__class__ is _Tensor else self._value(a) for a in args]
+        given = values(args, self.stream)
         self.steps.append((fn, None, None, args))
-        rc = fn(*values)
-        if rc:
-            capi.check(rc)
-
-    def _value(self, a):
-        if a is STREAM:
-            return self.stream
-        if isinstance(a, _Tensor):
-            return address(a)
-        return a.value if a.__class__ is Number else a
+        capi.check(fn(*given))
 
     def kernel(self, func, grid: int, block: int, args):
-        values = [a if a.__class__ is int else (a.data_ptr() or address(a)) if a.__class__ is _Tensor else self._value(a) for a in args]
+        given = values(args, self.stream)
         self.steps.append((func, (grid, 1, 1), (block, 1, 1), args))
-        capi.launch(func, (grid, 1, 1), (block, 1, 1), self.stream, values)
+        capi.launch(func, (grid, 1, 1), (block, 1, 1), self.stream, given)
 
     def keep(self, op: Operator, pending, results, device_stream: bool):
         """Leaves the recipe of this call with the operator.  Tensors that are not among the call's arguments are

@@ -44,7 +44,7 @@ def test_a_whole_number_is_passed_on_whatever_kind_of_number_it_is(values):
     for v in values * 2:
         op(None, extra=[v])
         op(extra=(v,))
-    assert op.seen == [int(v) for v in values * 2 for _ in range(2)] and op.python_calls <= 4
+    assert op.seen == [int(v) for v in values * 2 for _ in range(2)] and op.python_calls == 2
 
 
 def test_a_position_that_changes_its_kind():
@@ -59,7 +59,7 @@ def test_a_float_is_passed_on_whatever_kind_of_number_it_is():
     values = (0.5, 0.25, 3, 4, 1e30) * 3
     for v in values:
         op(None, extra=[v])
-    assert op.seen == [ctypes.c_float(float(v)).value for v in values] and op.python_calls == 4
+    assert op.seen == [ctypes.c_float(float(v)).value for v in values] and op.python_calls == 2
 
 
 def test_a_number_that_is_none_raises_what_it_raises_at_the_first_call():
@@ -176,7 +176,6 @@ def test_an_error_of_torch_in_a_replayed_call_is_a_python_exception():
             call.keep(self, pending, [], device_stream=False)
     op = Streaming()
     op(None)
-    op(None)
     for _ in range(3):
         with pytest.raises(RuntimeError):               # no device, hence no current stream
             op(None)
@@ -206,16 +205,15 @@ def test_arguments_live_until_the_call_is_over(as_list):
     extra = [value] if as_list else (value,)
 
     def during():
-        if op.seen[2:] and as_list:
+        if op.seen[1:] and as_list:
             extra.clear()
         counts.append(sys.getrefcount(value))
     op = Recording('F', during)
-    op(None, extra=[value])
     op(None, extra=[value])                              # leaves the recipe
     counts.clear()
     before = sys.getrefcount(value)
     op(None, extra=extra)
-    assert op.seen == [1234.5] * 3 and op.python_calls == 2
+    assert op.seen == [1234.5] * 2 and op.python_calls == 1
     assert counts == [before + (0 if as_list else 1)]           # the list's reference is gone, the call's is there
     assert sys.getrefcount(value) == before - as_list
 
@@ -256,7 +254,7 @@ def test_a_copy_is_called_like_the_operator_it_is_a_copy_of():
         twin(None, extra=[i])
     twin(extra=[6], x=None)
     op(None, extra=[7])
-    assert op.seen == [1, 2, 3, 4, 5, 6, 7] and (op.python_calls, twin.python_calls) == (2, 4)
+    assert op.seen == [1, 2, 3, 4, 5, 6, 7] and (op.python_calls, twin.python_calls) == (1, 2)
 
 
 def test_built_in_operators_can_be_pickled():
@@ -274,15 +272,15 @@ def test_an_attribute_that_is_replaced_ends_the_recipes(attribute):
         setattr(op, attribute, (lambda: i) if attribute == 'fast_path' else {'i': i})
         for _ in range(3):
             op(None, extra=[i])
-        assert op.python_calls == i + 2
+        assert op.python_calls == i + 1
     if attribute != 'fast_path':
         getattr(op, attribute)['i'] = 'changed'              # and one that is changed in place
         op(None, extra=[1])
-        assert op.python_calls == 22
+        assert op.python_calls == 21
         setattr(op, attribute, collections.OrderedDict(i=1))     # whose changes leave no trace
         for _ in range(2):
             op(None, extra=[1])
-        assert op.python_calls == 24
+        assert op.python_calls == 23
     delattr(op, attribute)
     assert getattr(op, attribute) is None
 
@@ -294,11 +292,11 @@ def test_calls_under_a_dispatch_mode_or_with_filled_memory_are_not_replayed():
     op = Recording('I')
     for i in (0, 1, 2):
         op(None, extra=[i])
-    assert op.python_calls == 2
+    assert op.python_calls == 1
     with Mode():
         op(None, extra=[3])
         op(None, extra=[4])
-    assert op.python_calls == 4
+    assert op.python_calls == 3
     before = torch.are_deterministic_algorithms_enabled()
     try:
         torch.use_deterministic_algorithms(True)
@@ -306,27 +304,53 @@ def test_calls_under_a_dispatch_mode_or_with_filled_memory_are_not_replayed():
         op(None, extra=[6])
     finally:
         torch.use_deterministic_algorithms(before)
-    assert op.python_calls == 6
+    assert op.python_calls == 5
     op(None, extra=[7])
-    assert op.python_calls == 6 and op.seen == [0, 1, 2, 3, 4, 5, 6, 7]
+    assert op.python_calls == 5 and op.seen == [0, 1, 2, 3, 4, 5, 6, 7]
 
 
-def test_a_recipe_is_made_when_a_signature_is_met_again():
-    """Making one costs as much as a call: a call whose signature is another one every time leaves none."""
-    class Sized(calls.Operator):
-        def __init__(self):
-            self.pending = 0
-            self._bind(('x', 'size'), ())
+class Sized(calls.Operator):
+    """Its signature is the size: every size has a recipe of its own."""
 
-        def _call(self, pending, x=None, size=None):
-            self.pending += pending is not None
+    def __init__(self):
+        self.python_calls, self.pending, self.seen = 0, 0, []
+        self.entry = ctypes.CFUNCTYPE(ctypes.c_int, ctypes.c_int)(lambda n: self.seen.append(n) or 0)
+        self._bind(('size',), ())
+
+    def _call(self, pending, size):
+        self.python_calls += 1
+        self.pending += pending is not None
+        call = calls.Call(0)
+        call.library(self.entry, size)
+        call.keep(self, pending, [], device_stream=False)
+
+
+def test_recipes_that_are_not_used_are_made_only_for_signatures_met_again():
+    """Making one costs as much as a call: where every call has another signature, it is not worth it."""
     op = Sized()
     for size in range(1000):
-        op(None, size)
-    assert op.pending < 10                               # the marks are 32 bits of a hash
+        op(size)
+    assert 8 <= op.pending < 16                          # the credit; and the marks are 32 bits of a hash
     for size in range(1000):
-        op(None, size)
-    assert op.pending > 800                              # two signatures in one place take it from each other
+        op(size)
+    made = op.pending
+    assert made > 800                                    # two signatures in one place of the marks take it from each other
+    for size in range(1000):
+        op(size)
+    assert op.pending - made < 200 and op.seen == [size for _ in range(3) for size in range(1000)]
+
+
+def test_recipes_that_are_used_are_made_at_the_first_call():
+    op = Sized()
+    for size in range(1000):
+        for _ in range(3):
+            op(size)
+    assert op.python_calls == 1000
+    for size in range(2000, 2008):                       # eight of them may wait for their use
+        op(size)
+    for size in range(2000, 2008):
+        op(size)
+    assert op.python_calls == 1008
 
 
 def test_an_argument_that_is_missing_is_not_one_that_is_none():
@@ -357,26 +381,13 @@ def test_an_argument_that_is_missing_is_not_one_that_is_none():
 
 
 def test_the_table_is_emptied_when_it_is_full():
-    entry = ctypes.CFUNCTYPE(ctypes.c_int, ctypes.c_int)(lambda n: seen.append(n) or 0)
-
-    class Sized(calls.Operator):
-        def __init__(self):
-            self.python_calls = 0
-            self._bind(('size',), ())
-
-        def _call(self, pending, size):
-            self.python_calls += 1
-            call = calls.Call(0)
-            call.library(entry, size)
-            call.keep(self, pending, [], device_stream=False)
-    op, seen = Sized(), []
+    op = Sized()
     for size in range(9000):
         for _ in range(3):
             op(size)
-    assert seen == [size for size in range(9000) for _ in range(3)] and op.python_calls == 18000
+    assert op.seen == [size for size in range(9000) for _ in range(3)] and op.python_calls == 9000
     op(8999)                                             # made after the table was emptied
-    assert op.python_calls == 18000
+    assert op.python_calls == 9000
     op(0)
     op(0)
-    op(0)
-    assert op.python_calls == 18002
+    assert op.python_calls == 9001
