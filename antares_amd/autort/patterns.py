@@ -187,6 +187,62 @@ register(W4A16_IR, W4A16_INPUTS, _w4a16_handler)
 
 
 # ---------------------------------------------------------------------------
+# Products of small and odd sizes (art_gemm_tile): float16 and float32 below, int8 A[M,K] @ B[N,K]^T
+# ---------------------------------------------------------------------------
+_TILE_SLICES = (1, 2, 3, 4, 6, 8, 12, 16, 24)
+
+
+def _tile_product(op, call, kind: int, a, b, c, M: int, N: int, K: int, large: bool, rival=None) -> bool:
+    """Runs the product with ``art_gemm_tile`` if that is the faster kernel for these sizes.  ``rival``: what a tuning run keeps
+    of the kernel for large products; the faster of the two runs, and one that was kept alone stays."""
+    lib = capi.lib()
+    if max(M, N, K) >= 1 << 31 or any(t.data_ptr() < c.data_ptr() + c.element_size() * c.numel() and c.data_ptr() < t.data_ptr() + t.element_size() * t.numel()
+                                      for t in (a, b)):
+        return False                              # a result over an operand: left to the kernels that always took it
+    code = lib.art_gemm_tile_form(kind, M, N, K, int(large), 0, 0)
+    key = f'gemm_tile.form|{kind},{M},{K},{N}'
+    saved = op.tuned.get(key)
+    trials = op.config.get('tune')
+    if saved is None and rival is not None and not (isinstance(trials, int) and trials > 0):
+        return False
+    if not code and saved is None:
+        return False
+
+    def partial(value):
+        return torch.empty((value & 255) * M * N, dtype=torch.int32 if kind == 2 else torch.float32, device=a.device) if value & 255 > 1 else None
+
+    if saved is None and isinstance(trials, int) and trials > 0 and not torch.cuda.is_current_stream_capturing():
+        codes = [code] + [v for v in (lib.art_gemm_tile_form(kind, M, N, K, 0, form, s) for form in (1, 2, 3, 4) for s in _TILE_SLICES)
+                          if v and v != code and (v >> 8 == 4) == (code >> 8 == 4) and (v & 255) * M * N <= 1 << 26]
+        codes = codes[:trials]
+        scratch = partial(max(codes, key=lambda v: v & 255))
+
+        def run(value, t):
+            capi.check(lib.art_gemm_tile(c_void_p(t[0].data_ptr()), c_void_p(t[1].data_ptr()), c_void_p(t[2].data_ptr()),
+                                         c_void_p(scratch.data_ptr() if scratch is not None else 0), kind, M, N, K, value >> 8, value & 255,
+                                         c_void_p(torch.cuda.current_stream().cuda_stream)))
+        saved = tune_hand_kernel(op, key, codes, run, len(codes), [(a, b, torch.empty_like(c))])
+    if saved is not None:
+        if rival is not None and rival['us'] <= saved['us']:
+            return False
+        value = int(saved['value'])
+        if lib.art_gemm_tile_form(kind, M, N, K, int(large), value >> 8, value & 255) == value and value >> 8:
+            code = value
+    if not code:
+        return False
+    call.library(lib.art_gemm_tile, a, b, c, partial(code), kind, M, N, K, code >> 8, code & 255, STREAM)
+    return True
+
+
+def _gemm_i8_handler(op, bound, env, call) -> bool:
+    a, b, c = (bound[op.fast_roles[n]] for n in 'abc')
+    return _tile_product(op, call, 2, a, b, c, a.shape[0], b.shape[0], a.shape[1], False)
+
+
+register('c[M, N] +=! a[M, K].cast(`int32`) * b[N, K].cast(`int32`)', ['a=int8[M:4096, K:4096]', 'b=int8[N:4096, K:4096]'], _gemm_i8_handler)
+
+
+# ---------------------------------------------------------------------------
 # fp16 GEMM with fp32 accumulation: C[M,N] = A[M,K] @ B[K,N] (AntaresIR.md:115 with the casts that
 # make the accumulator fp32)
 # ---------------------------------------------------------------------------
@@ -203,7 +259,7 @@ def _gemm_f16_handler(op, bound, env, call) -> bool:
     M, K = a.shape
     N = b.shape[1]
     if N % 8 or K % 64 or a.data_ptr() % 16 or b.data_ptr() % 16 or c.data_ptr() % 16:
-        return False
+        return _tile_product(op, call, 0, a, b, c, M, N, K, False)
 
     def run(value, t):
         capi.check(capi.lib().art_gemm_f16_tuned(c_void_p(t[0].data_ptr()), c_void_p(t[1].data_ptr()), c_void_p(t[2].data_ptr()), M, N, K,
@@ -215,6 +271,8 @@ def _gemm_f16_handler(op, bound, env, call) -> bool:
     if saved is None and isinstance(trials, int) and trials > 0 and not torch.cuda.is_current_stream_capturing():
         saved = tune_hand_kernel(op, key, [256, 512], run, trials,
                                  [(a, b, torch.empty_like(c))])
+    if _tile_product(op, call, 0, a, b, c, M, N, K, True, saved):
+        return True
     call.library(capi.lib().art_gemm_f16_tuned, a, b, c, M, N, K, int(saved['value'] if saved is not None else 0), STREAM)
     return True
 
@@ -234,9 +292,9 @@ def _gemm_f32_handler(op, bound, env, call) -> bool:
     a, b, c = bound[r['a']], bound[r['b']], bound[r['c']]
     M, K = a.shape
     N = b.shape[1]
-    # small products are left to the generic lowering: a launch of the tiled kernel needs a few hundred tiles to pay
+    # a launch of the kernel for large products needs a few hundred tiles to pay
     if N % 4 or K % 32 or N < 4 or M * N < 128 * 128 * 32 or a.data_ptr() % 16 or b.data_ptr() % 16:
-        return False
+        return _tile_product(op, call, 1, a, b, c, M, N, K, False)
 
     def run(_, t):
         capi.check(capi.lib().art_gemm_f32(c_void_p(t[0].data_ptr()), c_void_p(t[1].data_ptr()), c_void_p(t[2].data_ptr()), M, N, K,
@@ -246,6 +304,8 @@ def _gemm_f32_handler(op, bound, env, call) -> bool:
     trials = op.config.get('tune')
     if key not in op.tuned and isinstance(trials, int) and trials > 0 and not torch.cuda.is_current_stream_capturing():
         tune_hand_kernel(op, key, [0], run, 1, [(a, b, torch.empty_like(c))])
+    if _tile_product(op, call, 1, a, b, c, M, N, K, True, op.tuned.get(key)):
+        return True
     call.library(capi.lib().art_gemm_f32, a, b, c, M, N, K, STREAM)
     return True
 

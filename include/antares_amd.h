@@ -244,6 +244,17 @@ int art_gemv_w4p(const void* x_dev, const void* packed_dev, void* y_dev, int K, 
 int art_gemv_gptq(const void* x_dev, const void* qweight_dev, const void* scales_dev, void* y_dev,
                   int K, int N, int x_f16, int scales_f16, void* stream);
 
+/* Matrix products of small and odd sizes: C[M,N] = A[M,K] @ B[K,N] in float16 (type 0; float32 sums) or float32 (type 1), and
+ * C[M,N] = A[M,K] @ B[N,K]^T from int8 to int32 (type 2), all row-major, any alignment of the elements' own, K and (types
+ * 0 and 1) N of at least 16 bytes of elements (AntaresIR.md:115).
+ *   art_gemm_tile_form: 256 * form + slices of k.  form == 0 asks for the library's choice (`large` != 0: art_gemm_f16 /
+ *     art_gemm_f32 take these operands); 0 means that another kernel is faster, or that the sizes are not taken.  Otherwise
+ *     the same code if art_gemm_tile takes it, else 0.  Forms: 1 = blocks of 64 x 64, 2 = 64 x 128, 3 = 128 x 128 (not float32),
+ *     4 = 64 x 64 with short sums (float32 only).
+ *   art_gemm_tile: partial_dev holds slices * M * N float32 (int32) values of any content, 16-byte aligned; it may be NULL for one slice. */
+int art_gemm_tile_form(int type, int M, int N, int K, int large, int form, int slices);
+int art_gemm_tile(const void* a_dev, const void* b_dev, void* c_dev, void* partial_dev, int type, int M, int N, int K, int form, int slices,
+                  void* stream);
 /* fp16 GEMM on the matrix cores: C[M,N] = A[M,K] @ B[K,N], all row-major, fp32
  * accumulation, fp16 output.  Any M; N % 8 == 0, K % 64 == 0 (tiles of 256 x 256; edge tiles are clamped).
  * Replaces the kernel the reference generates for `C[N,M] +=! A[N,K] * B[K,M]`

@@ -120,3 +120,93 @@ def test_8192_cubed_through_a_random_projection(gemm):
     i, j = 1234, 4321
     assert abs(float(c[i, j]) - float(a[i].double() @ b[:, j].double())) < 1e-2 * max(1.0, abs(float(c[i, j])))
     assert abs(float(c[n - 1, 0]) - float(a[n - 1].double() @ b[:, 0].double())) < 1e-2 * max(1.0, abs(float(c[n - 1, 0])))
+
+
+TILE_TYPES = {'float16': (0, 64), 'float32': (1, 32), 'int8': (2, 128)}      # dtype -> (kind, values of k in a chunk)
+
+
+def _tile_operands(dtype, M, N, K, dev, offset):
+    """Operands at an address that is aligned to nothing but the element (offset odd), and the float64 / int64 product with
+    the sum of the products' magnitudes."""
+    g = torch.Generator().manual_seed(M + N + K)
+    if dtype == 'int8':
+        a, b = torch.randint(-128, 128, (M, K), generator=g, dtype=torch.int8), torch.randint(-128, 128, (N, K), generator=g, dtype=torch.int8)
+        want, size = a.double() @ b.double().t(), None
+    else:
+        t = getattr(torch, dtype)
+        a, b = torch.randn(M, K, generator=g).to(t), torch.randn(K, N, generator=g).to(t)
+        want, size = a.double() @ b.double(), a.double().abs() @ b.double().abs()
+
+    def put(x):
+        room = torch.empty(x.numel() + offset, dtype=x.dtype, device=dev)[offset:].view(x.shape)
+        room.copy_(x)
+        return room
+    return put(a), put(b), want, size
+
+
+@pytest.mark.parametrize('dtype', list(TILE_TYPES))
+# one tile, a row / column / value of k more or less than a tile, the shortest k, the narrowest N, several chunks and slices
+@pytest.mark.parametrize('M,N,chunks,rest', [(64, 64, 1, 0), (65, 63, 1, 1), (63, 129, 2, -1), (1, 17, 0, 16), (130, 129, 5, 3), (257, 66, 7, 0), (128, 128, 4, 17),
+                                             (200, 1000, 3, 9)])
+def test_tile_products_of_every_form(dtype, M, N, chunks, rest):
+    """`art_gemm_tile`: every form and several numbers of slices against the 64-bit product.  Bounds: int8 exact; float32 sums of
+    at most 32 + chunks + slices terms in a row, each addition off by 2^-24 of the magnitudes; float16 the same over all of K,
+    and the result's own rounding (2^-11)."""
+    import autort
+    from ctypes import c_void_p
+    from antares_amd.runtime import capi
+    kind, per = TILE_TYPES[dtype]
+    K = chunks * per + rest
+    dev = autort.device()
+    capi.init(dev.index or 0)
+    lib = capi.lib()
+    a, b, want, size = _tile_operands(dtype, M, N, K, dev, 1)
+    total = (K + per - 1) // per
+    for form in (1, 2, 3, 4):
+        for slices in sorted({1, 2, 3, total}):
+            if not lib.art_gemm_tile_form(kind, M, N, K, 0, form, slices):
+                assert form == (3 if kind == 1 else 4) or slices > total
+                continue
+            print(f'[case] art_gemm_tile {dtype} {M}x{N}x{K} form {form} slices {slices}', flush=True)
+            c = torch.zeros(M, N, dtype=torch.int32 if kind == 2 else getattr(torch, dtype), device=dev)
+            partial = torch.full((slices * M * N,), -7, dtype=torch.int32, device=dev)      # NaN as float32: nothing is read before it is written
+            capi.check(lib.art_gemm_tile(*(c_void_p(t.data_ptr()) for t in (a, b, c, partial)), kind, M, N, K, form, slices,
+                                         c_void_p(torch.cuda.current_stream().cuda_stream)))
+            got = c.cpu().double()
+            if kind == 2:
+                assert torch.equal(got, want)
+            elif kind == 1:
+                assert bool(((got - want).abs() <= (32 + total + slices) * 2.0 ** -24 * size).all())
+            else:
+                assert bool(((got - want).abs() <= (K + slices) * 2.0 ** -24 * size + 2.0 ** -11 * want.abs() + 2.0 ** -24).all())
+
+
+@pytest.mark.parametrize('dtype,M,N,K', [('float16', 78, 207, 582), ('float16', 448, 704, 2368), ('float16', 144, 160, 104), ('float32', 248, 120, 1616),
+                                         ('float32', 192, 576, 192), ('float32', 70, 420, 268), ('int8', 232, 120, 1448), ('int8', 112, 3568, 72)])
+def test_small_products_take_the_tile_kernel_and_agree_with_the_generic_kernels(dtype, M, N, K):
+    """The route of an exported program: the call goes to `art_gemm_tile`, agrees with the generic kernels (int8 bit for bit), and
+    in float32 is no further from the 64-bit product than they are."""
+    import autort
+    from antares_amd.autort import patterns
+    from antares_amd.runtime import capi
+    dev = autort.device()
+    print(f'[case] tile route {dtype} {M}x{N}x{K}', flush=True)
+    ir, inputs = {'float16': (patterns.GEMM_F16_IR, patterns.GEMM_F16_INPUTS), 'float32': (patterns.GEMM_F32_IR, patterns.GEMM_F32_INPUTS),
+                  'int8': ('o[N, M] +=! x[N, K].cast(`int32`) * y[M, K].cast(`int32`)', ['x=int8[N:64, K:64]', 'y=int8[M:64, K:64]'])}[dtype]
+    a, b, want, _ = _tile_operands(dtype, M, N, K, dev, 0)
+    kind = TILE_TYPES[dtype][0]
+    assert capi.lib().art_gemm_tile_form(kind, M, N, K, 0, 0, 0)
+    results = []
+    for generic in (False, True):
+        op = autort.export(ir=ir, inputs=inputs, name=f'tile_{dtype}_{int(generic)}')
+        if generic:
+            op.fast_path = None
+        else:
+            assert op.fast_path is not None
+        results.append(op(a, b).cpu().double())
+    got, old = results
+    if kind == 2:
+        assert torch.equal(got, old) and torch.equal(got, want)
+    else:
+        off = [float((r - want).norm() / want.norm()) for r in results]
+        assert off[0] <= (1e-3 if kind == 0 else 1.05 * off[1]), off
