@@ -474,10 +474,12 @@ def _conv2d_handler(st, axes, window):
                  window['h'][0], window['w'][0])
         if max(abs(v) for v in shape) >= 1 << 31:
             return False
-        form = lib.art_conv2d_form(*shape, 0)
+        form = lib.art_conv2d_choose(*shape)
         if not form:
             return False
-        packed = torch.empty(lib.art_conv2d_packed_bytes(shape[0], e['c'], e['f']), dtype=torch.uint8, device=x.device)
+
+        def scratch(forms):
+            return torch.empty(max(lib.art_conv2d_scratch_bytes(*shape, v) for v in forms), dtype=torch.uint8, device=x.device)
 
         def run(value, t):
             capi.check(lib.art_conv2d(*(c_void_p(v.data_ptr()) for v in t), *shape, int(value), c_void_p(torch.cuda.current_stream().cuda_stream)))
@@ -486,10 +488,13 @@ def _conv2d_handler(st, axes, window):
         saved = op.tuned.get(key)
         trials = op.config.get('tune')
         if saved is None and isinstance(trials, int) and trials > 0 and not torch.cuda.is_current_stream_capturing():
-            forms = [form] + [v for v in (1, 2, 3) if v != form and lib.art_conv2d_form(*shape, v)]
-            saved = tune_hand_kernel(op, key, forms, run, trials, [(x, w, packed, torch.empty_like(y))])
+            # a float32 form with longer sums than the library's choice is not tried
+            others = [v for v in (1, 2, 3, 4, 5, 6) + tuple(k + 256 * s for k in (4, 5, 6, 7) for s in (2, 3, 4, 6, 8)) if (form & 255 == 7) == (v & 255 == 7)]
+            forms = [form] + [v for v in others if v != form and lib.art_conv2d_form(*shape, v)]
+            forms = forms[:trials]
+            saved = tune_hand_kernel(op, key, forms, run, len(forms), [(x, w, scratch(forms), torch.empty_like(y))])
         if saved is not None and lib.art_conv2d_form(*shape, int(saved['value'])):
             form = int(saved['value'])
-        call.library(lib.art_conv2d, x, w, packed, y, *shape, form, STREAM)
+        call.library(lib.art_conv2d, x, w, scratch([form]), y, *shape, form, STREAM)
         return True
     return handler

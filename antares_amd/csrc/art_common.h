@@ -48,6 +48,27 @@ constexpr size_t kExchangeBytes = 64 * 1024;
 constexpr size_t kSlotOffset = 64 * 1024;                // 64-bit split-K accumulators (zero between launches)
 constexpr size_t kScratchOffset = 4 * 1024 * 1024;       // partial sums, tile counts (any content)
 
+// 64 lanes x 16 (4) bytes from base + lane offset straight into LDS at lds_dst + 16 (4) * lane.  The instruction takes
+// the LDS address from m0, which nothing else here uses (the compiler warns that it does not preserve a reserved register
+// that is named as clobbered; nothing has to be preserved).  The waits are written by hand: the compiler does not see
+// these loads.
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+__device__ __forceinline__ void load_lds_x4(const void* base, unsigned int off, unsigned int lds_dst) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds_dst) : "m0");
+}
+__device__ __forceinline__ void load_lds_x1(const void* base, unsigned int off, unsigned int lds_dst) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" ::"v"(off), "s"(base), "s"(lds_dst) : "m0");
+}
+#pragma clang diagnostic pop
+
+// A base address that is the same for every lane, in scalar registers whatever surrounds the load.
+__device__ __forceinline__ const void* uniform(const void* p) {
+  const unsigned long long v = (unsigned long long)p;
+  return (const void*)((unsigned long long)(unsigned int)__builtin_amdgcn_readfirstlane((int)v) |
+                       (unsigned long long)(unsigned int)__builtin_amdgcn_readfirstlane((int)(v >> 32)) << 32);
+}
+
 }  // namespace art
 
 // Workgroup barrier that orders LDS traffic only.  __syncthreads() also waits for every outstanding

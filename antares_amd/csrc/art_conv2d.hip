@@ -27,53 +27,18 @@
 // float32 32 x 128 x 28 x 28 -> 128 113 -> 81 us (the matrix instructions alone take 47), 23 x 128 x 30 x 30 -> 176 119 -> 86.
 // The first of these spends 7 us of the matrix cores' time in 18.6 us: one block per compute unit and only 4 chunks, so the
 // first image fetch, the waits between chunks and the stores of 12.8 MB stay in sight; packing the filter takes 2.3 us.
+// Today it is taken for large images with little to multiply (`choose`); art_conv2d_staged.hip stages the image first.
 #include <type_traits>
 
-#include "art_common.h"
+#include "art_conv2d.h"
 
 namespace {
 
-constexpr int kThreads = 256;
-constexpr int kTaps = 9;                        // 3 x 3
-constexpr int kChunkBytes = 64;                 // channels of a point that are staged at a time
+using namespace art::conv;
+
 constexpr int kPitchBytes = kChunkBytes + 16;   // from one point to the next in LDS
 constexpr unsigned kOutside = 0xffffffffu;
 constexpr size_t kMaxLds = 64 * 1024;
-
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-
-template <typename T> struct Elem;
-template <> struct Elem<_Float16> {
-  typedef _Float16 vec __attribute__((ext_vector_type(8)));
-  typedef unsigned short raw;
-  static __device__ __forceinline__ f32x16 multiply(vec a, vec b, f32x16 c) { return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0); }
-};
-template <> struct Elem<float> {
-  typedef float vec __attribute__((ext_vector_type(4)));
-  typedef float raw;
-  // instruction m multiplies k = m (lanes 0-31) and k = 4 + m (lanes 32-63) of 8
-  static __device__ __forceinline__ f32x16 multiply(vec a, vec b, f32x16 c) {
-#pragma unroll
-    for (int m = 0; m < 4; ++m) c = __builtin_amdgcn_mfma_f32_32x32x2f32(a[m], b[m], c, 0, 0, 0);
-    return c;
-  }
-};
-
-struct Geometry {
-  int N, C, H, W, F, HO, WO, ph, pw;
-  int columns;          // output points: N * HO * WO
-  int chunks;           // runs of 64 bytes of channels
-  int row_tiles;        // 32-feature tiles of the packed filter
-  int row_blocks;       // blocks along the features
-  int span;             // points the LDS buffers hold
-};
-
-// Output point -> its place in the padded image (where tap (0, 0) reads).
-__device__ __forceinline__ int place_of(int column, const Geometry& g) {
-  const unsigned hw = (unsigned)(g.HO * g.WO), n = (unsigned)column / hw, r = (unsigned)column % hw;
-  const unsigned ho = r / (unsigned)g.WO, wo = r % (unsigned)g.WO;
-  return (int)((n * (unsigned)(g.HO + 2) + ho) * (unsigned)(g.WO + 2) + wo);
-}
 
 // Filter [F][C][taps] -> [chunk][tap][32 features][half][lane][16 bytes], zeros past F and C.  A thread gathers the 16
 // bytes of one lane; bound by latency (about 2 us).
@@ -279,9 +244,12 @@ int span_of(const Geometry& g, int columns) {
 
 size_t lds_of(int span) { return (size_t)span * (2 * kPitchBytes + 4); }
 
-// Forms: 1 = 64 features x 64 points per block, 2 = 64 x 128, 3 = 128 x 128.
-int features_of(int form) { return form == 3 ? 128 : 64; }
-int points_of(int form) { return form == 1 ? 64 : 128; }
+// Forms: 1 = 64 features x 64 points per block, 2 = 64 x 128, 3 = 128 x 128; 4, 5, 6 the same over the staged image, 7 = 64 x 64
+// there with short sums (float32), plus 256 x slices of the channels (0: one).
+int shape_of(int form) { return (form & 255) % 3; }
+int features_of(int form) { return shape_of(form) == 0 ? 128 : 64; }
+int points_of(int form) { return shape_of(form) == 1 ? 64 : 128; }
+int slices_of(int form) { return form >> 8 ? form >> 8 : 1; }
 
 bool geometry(Geometry& g, int f16, int N, int C, int H, int W, int F, int HO, int WO, int ph, int pw) {
   g = Geometry{N, C, H, W, F, HO, WO, ph, pw, 0, 0, 0, 0, 0};
@@ -296,7 +264,13 @@ bool geometry(Geometry& g, int f16, int N, int C, int H, int W, int F, int HO, i
   return (long long)g.chunks * kTaps * ((F + 127) / 128) * 4 < (1 << 22);      // packed filter below 4 GiB
 }
 
-bool fits(const Geometry& g, int form) { return form >= 1 && form <= 3 && lds_of(span_of(g, points_of(form))) <= kMaxLds; }
+bool fits(Geometry g, int f16, int form) {
+  const int kind = form & 255;
+  if (form < 1 || kind < 1 || kind > (f16 ? 6 : 7)) return false;
+  g.span = span_of(g, points_of(form));
+  if (kind <= 3) return form == kind && lds_of(g.span) <= kMaxLds;
+  return slices_of(form) <= 64 && slices_of(form) <= g.chunks && staged_lds(g) <= 160 * 1024;
+}
 
 long long blocks_of(const Geometry& g, int form) {
   return (long long)((g.columns + points_of(form) - 1) / points_of(form)) * ((g.F + features_of(form) - 1) / features_of(form));
@@ -323,24 +297,68 @@ double launch_time(const Geometry& g, int f16, int form) {
   return c.fixed + rounds * (chunks * c.chunk + c.round);
 }
 
+// The same for the staged forms (the launch that stages the image included): a fixed part, per chunk of a block's slice a time
+// that grows with the blocks that share a compute unit and with how unevenly they do, the copy, the stores, and for slices the
+// third launch.  Fitted to 116 sizes in float16 and 214 in float32 of the same ranges: 3.1 and 1.9 % off, and what it picks is 0.05 and
+// 0.25 % slower than the fastest in the mean.
+double staged_time(const Geometry& g, int f16, int form, int slices) {
+  struct Cost { double fixed, alone, shared, uneven; };
+  struct Rest { double sum, sum_bytes, copy, store; };
+  static const Cost cost[2][4] = {{{6.30, 2.657, 2.526, 2.445}, {6.97, 4.661, 4.081, 4.561}, {8.15, 8.396, 7.815, 8.575}, {6.25, 4.809, 5.443, 5.217}},
+                                  {{6.52, 0.998, 0.861, 0.730}, {7.14, 1.309, 0.900, 0.661}, {8.03, 1.836, 1.636, 1.386}, {}}};
+  static const Rest rest[2] = {{2.64, 0.384, 0.580, 0.271}, {2.62, 0.342, 0.510, 0.242}};
+  const Cost& c = cost[f16 != 0][form - 4];
+  const Rest& r = rest[f16 != 0];
+  const int per_chunk = f16 ? 32 : 16;
+  const double half = form != 6 && g.C - (g.chunks - 1) * per_chunk <= per_chunk / 2 ? 0.5 : 0.0;
+  const double rounds = (double)blocks_of(g, form) * slices / kUnits, full = rounds > 1 ? rounds : 1, megabytes = 4e-6 * g.columns * g.F;
+  const double chunks = slices > 1 ? (g.chunks + slices - 1) / slices : g.chunks - half;
+  const double t = c.fixed + chunks * (c.alone + c.shared * (full - 1) + c.uneven * (ceil(rounds) > full ? ceil(rounds) - full : 0)) +
+                   r.copy * 64e-6 * g.chunks * g.N * (g.HO + 2) * (g.WO + 2);
+  return slices == 1 ? t + r.store * megabytes : t + r.sum + r.sum_bytes * (slices + 1) * megabytes;
+}
+
 // The form for these sizes, or 0: the generic kernels are faster or sum more exactly there.  Lines from sweeps of the sizes
 // above, times in us generic / here.
 //  * fewer than 32 features, or fewer than 16 blocks of 64 x 64: the generic path sums on the vector units in short
-//    chains.  In float32 that error (0.8e-7 against 64 bits) is below the matrix instructions' (1.3e-7): left alone.  In
-//    float16 it is the same (0.7-1.1e-7 both) from 64 channels on, and the times are 62 / 16 (1 x 224 -> 24, 35 x 35) and
-//    120 / 14 (2 x 128 -> 24, 46 x 46); below 8192 results the generic path wins (7 / 9 for 7 x 40 -> 16, 7 x 7).
-//  * from 1024 terms per result on the generic path slices the sum over an idle chip: 13 / 18 (float16, 5 x 216 -> 40,
-//    14 x 14, 16 blocks), 22 / 14 at 144 blocks; float32 23 / 43 at 40 blocks, 62 / 51 at 204.  (Just past
-//    one round it is faster again, 73 / 84 at 300 blocks, 74 / 67 at 381, with twice the error: not left to it.)
+//    chains.  In float32 that error (0.73e-7 to 1.26e-7 against 64 bits) is below the matrix instructions' (1.2e-7 to 1.5e-7), not
+//    below that of the short sums (0.69e-7 to 0.76e-7): form 7, where it is faster than 5.5 us + 1.1 ps per product there:
+//    375 / 37 (2 x 232 -> 24, 52 x 52), 57 / 16 (3 x 184 -> 48, 14 x 14), 7.6 / 13.7 (1 x 24 -> 32, 15 x 15).  In
+//    float16 the error is the same (0.7-1.1e-7 both) from 64 channels on; below 8192 results the generic path wins (5.6 / 7.0 for
+//    1 x 16 -> 40, 7 x 7).
+//  * elsewhere one of the forms wins, with the channels sliced where there are few blocks: float32 23 / 20 (9 x 216 -> 64,
+//    17 x 17, 46 without slices), float16 19 / 13.8 (9 x 240 -> 104, 13 x 13).  The image is staged unless it is large and
+//    there is little to multiply: float16 18 x 64 -> 48, 51 x 51 15.3 gathered, 16.8 staged, 1 x 40 -> 152, 42 x 42 10.0 and 9.0.
 //  * below 32 features only 64 x 64, whose rows of taps are summed by themselves: the larger blocks' error is 1.2e-7.
 int choose(const Geometry& g, int f16) {
+  const long long small = blocks_of(g, 1), results = (long long)g.columns * g.F;
+  const bool vector_units = g.F < 32 || small < 16;
+  if (f16 && vector_units && (results < 8192 || (g.F < 32 && g.C < 64))) return 0;
+  int best = 0;
+  double t_best = f16 || !vector_units ? 1e30 : 5.5 + 1.1e-6 * results * 9 * g.C;
+  auto consider = [&](int form, double t) {
+    if (t < t_best && fits(g, f16, form)) { best = form; t_best = t; }
+  };
+  for (int form = 1; form <= 7; ++form) {
+    if (form == 7 ? f16 || !vector_units : !f16 && vector_units) continue;
+    if (shape_of(form) != 1 && g.F < 32) continue;
+    if (form <= 3) consider(form, launch_time(g, f16, form));
+    for (int slices : {1, 2, 3, 4, 5, 6, 8, 12})
+      if (form > 3 && slices <= g.chunks && (slices == 1 || slices * blocks_of(g, form) <= 4 * kUnits)) consider(form + (slices > 1 ? 256 * slices : 0), staged_time(g, f16, form, slices));
+  }
+  return best;
+}
+
+// Among the forms that need no more scratch than the packed filter, for callers that have no more; beyond these lines, too, the
+// generic kernels were faster: from 1024 terms per result on they slice the sum over an idle chip.
+int choose_gathered(const Geometry& g, int f16) {
   const long long small = blocks_of(g, 1), results = (long long)g.columns * g.F;
   const bool vector_units = g.F < 32 || small < 16;
   if (vector_units && (!f16 || results < 8192 || (g.F < 32 && g.C < 64))) return 0;
   if (!vector_units && 9LL * g.C >= 1024 && small < (f16 ? 64 : 192)) return 0;
   int best = 0;
   for (int form = 1; form <= (g.F < 32 ? 1 : 3); ++form)
-    if (fits(g, form) && (!best || launch_time(g, f16, form) < launch_time(g, f16, best))) best = form;
+    if (fits(g, f16, form) && (!best || launch_time(g, f16, form) < launch_time(g, f16, best))) best = form;
   return best;
 }
 
@@ -367,7 +385,12 @@ int run(const void* x, const void* w, void* packed, void* y, const Geometry& g, 
 extern "C" int art_conv2d_form(int f16, int N, int C, int H, int W, int F, int HO, int WO, int ph, int pw, int form) {
   Geometry g;
   if (!geometry(g, f16, N, C, H, W, F, HO, WO, ph, pw)) return 0;
-  return form ? (fits(g, form) ? form : 0) : choose(g, f16);
+  return form ? (fits(g, f16, form) ? form : 0) : choose_gathered(g, f16);
+}
+
+extern "C" int art_conv2d_choose(int f16, int N, int C, int H, int W, int F, int HO, int WO, int ph, int pw) {
+  Geometry g;
+  return geometry(g, f16, N, C, H, W, F, HO, WO, ph, pw) ? choose(g, f16) : 0;
 }
 
 extern "C" size_t art_conv2d_packed_bytes(int f16, int C, int F) {
@@ -375,10 +398,16 @@ extern "C" size_t art_conv2d_packed_bytes(int f16, int C, int F) {
   return chunks * kTaps * (((size_t)F + 127) / 128) * 4 * 2048;
 }
 
+extern "C" size_t art_conv2d_scratch_bytes(int f16, int N, int C, int H, int W, int F, int HO, int WO, int ph, int pw, int form) {
+  Geometry g;
+  if (!geometry(g, f16, N, C, H, W, F, HO, WO, ph, pw) || !fits(g, f16, form)) return 0;
+  return (form & 255) <= 3 ? art_conv2d_packed_bytes(f16, C, F) : staged_bytes(g, slices_of(form));
+}
+
 extern "C" int art_conv2d(const void* x_dev, const void* w_dev, void* packed_dev, void* y_dev, int f16, int N, int C, int H, int W, int F, int HO,
                           int WO, int ph, int pw, int form, void* stream) {
   Geometry g;
-  ART_REQUIRE(geometry(g, f16, N, C, H, W, F, HO, WO, ph, pw) && fits(g, form), "art_conv2d: sizes the kernel does not take (form %d)", form);
+  ART_REQUIRE(geometry(g, f16, N, C, H, W, F, HO, WO, ph, pw) && fits(g, f16, form), "art_conv2d: sizes the kernel does not take (form %d)", form);
   ART_REQUIRE(x_dev && w_dev && packed_dev && y_dev, "art_conv2d: null pointer");
   const uintptr_t size = f16 ? 2 : 4;
   ART_REQUIRE((uintptr_t)x_dev % size == 0 && (uintptr_t)w_dev % size == 0 && (uintptr_t)packed_dev % 16 == 0 && (uintptr_t)y_dev % 4 == 0,
@@ -389,6 +418,8 @@ extern "C" int art_conv2d(const void* x_dev, const void* w_dev, void* packed_dev
   g.row_blocks = (F + features_of(form) - 1) / features_of(form);
   g.row_tiles = g.row_blocks * (features_of(form) / 32);
   g.span = span_of(g, points_of(form));
+  if ((form & 255) > 3)
+    return run_staged(x_dev, w_dev, packed_dev, y_dev, g, f16, form & 255, slices_of(form), (int)blocks_of(g, form), (hipStream_t)stream);
   return f16 ? run<_Float16>(x_dev, w_dev, packed_dev, y_dev, g, form, (hipStream_t)stream)
              : run<float>(x_dev, w_dev, packed_dev, y_dev, g, form, (hipStream_t)stream);
 }

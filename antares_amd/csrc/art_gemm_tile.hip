@@ -32,7 +32,7 @@
 // times as fast.
 #include <type_traits>
 
-#include "art_common.h"
+#include "art_conv2d.h"
 
 namespace {
 
@@ -445,6 +445,12 @@ int run(const void* a, const void* b, void* c, void* partial, const Sizes& z, in
 }
 
 }  // namespace
+
+int art::sum_slices(const float* partial, float* y, long long count, int slices, hipStream_t stream) {
+  gemm_tile_sum_kernel<float, double, float><<<dim3((unsigned)((count + 1023) / 1024)), dim3(256), 0, stream>>>(partial, y, count, slices);
+  ART_LAUNCH_CHECK();
+  return 0;
+}
 
 extern "C" int art_gemm_tile_form(int type, int M, int N, int K, int large, int form, int splits) {
   if (form == 0) return choose(type, M, N, K, large != 0);

@@ -5,6 +5,10 @@
 namespace art {
 namespace w4 {
 
+using ::art::load_lds_x1;
+using ::art::load_lds_x4;
+using ::art::uniform;
+
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 typedef _Float16 h4 __attribute__((ext_vector_type(4)));
 typedef _Float16 h2 __attribute__((ext_vector_type(2)));
@@ -23,27 +27,6 @@ __device__ __forceinline__ h2 as_h2(unsigned int v) { return __builtin_bit_cast(
 // (w & mask) | bias in one v_bitop3_b32 (truth table 0xEA = (a & b) | c).
 __device__ __forceinline__ unsigned int and_or(unsigned int w, unsigned int mask, unsigned int bias) {
   return __builtin_amdgcn_bitop3_b32(w, mask, bias, 0xEA);
-}
-
-// 64 lanes x 16 (4) bytes from base + lane offset straight into LDS at lds_dst + 16 (4) * lane.  The instruction takes
-// the LDS address from m0, which nothing else here uses (the compiler warns that it does not preserve a reserved register
-// that is named as clobbered; nothing has to be preserved).  The waits are written by hand: the compiler does not see
-// these loads.
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"
-__device__ __forceinline__ void load_lds_x4(const void* base, unsigned int off, unsigned int lds_dst) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds_dst) : "m0");
-}
-__device__ __forceinline__ void load_lds_x1(const void* base, unsigned int off, unsigned int lds_dst) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" ::"v"(off), "s"(base), "s"(lds_dst) : "m0");
-}
-#pragma clang diagnostic pop
-
-// A base address that is the same for every lane, in scalar registers whatever surrounds the load.
-__device__ __forceinline__ const void* uniform(const void* p) {
-  const unsigned long long v = (unsigned long long)p;
-  return (const void*)((unsigned long long)(unsigned int)__builtin_amdgcn_readfirstlane((int)v) |
-                       (unsigned long long)(unsigned int)__builtin_amdgcn_readfirstlane((int)(v >> 32)) << 32);
 }
 
 constexpr Magic kMagic{0x000F000Fu, 0x00F000F0u, 0x64006400u, 0x54005400u};

@@ -91,7 +91,9 @@ _SIGNATURES = {
     'art_gemm_f32_batched': (c_int, [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p]),
     'art_gemm_f32_ex': (c_int, [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p]),
     'art_conv2d_form': (c_int, [c_int] * 11),
+    'art_conv2d_choose': (c_int, [c_int] * 10),
     'art_conv2d_packed_bytes': (c_size_t, [c_int] * 3),
+    'art_conv2d_scratch_bytes': (c_size_t, [c_int] * 11),
     'art_conv2d': (c_int, [c_void_p] * 4 + [c_int] * 11 + [c_void_p]),
     'art_rmsnorm': (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_float, c_float, c_int, c_int, c_int, c_void_p]),
     'art_rotary': (c_int, [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p, c_int, c_longlong, c_int, c_int, c_int, c_int,

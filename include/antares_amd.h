@@ -283,11 +283,16 @@ int art_gemm_f32_ex(const void* a_dev, const void* b_dev, void* c_dev, int batch
 
 /* 3 x 3 convolution, stride 1, zero outside the image, float32 sums and results, on the matrix cores:
  * y[N,F,HO,WO] = sum over c, kh, kw of x[N,C,ho+kh-ph,wo+kw-pw] * w[F,C,3,3]; x and w both float16 (f16 = 1) or float32.
- * Programs written as AntaresIR.md:166 (reference: algo_tiling.py:35-98).  packed: scratch of art_conv2d_packed_bytes.
- * form: block shape, 1 = 64 features x 64 points, 2 = 64 x 128, 3 = 128 x 128; art_conv2d_form gives the library's choice
- * (form = 0 asks for it) and 0 where these sizes are not taken. */
+ * Programs written as AntaresIR.md:166 (reference: algo_tiling.py:35-98).
+ * form: block shape, 1 = 64 features x 64 points, 2 = 64 x 128, 3 = 128 x 128, with a packed_dev of art_conv2d_packed_bytes;
+ * 4, 5, 6 the same over a staged copy of the image, 7 = 64 x 64 there with shorter sums (float32), each plus 256 x slices of the
+ * channels (or plus 0: one), with a packed_dev of art_conv2d_scratch_bytes for that form.  art_conv2d_choose gives the library's
+ * choice among all of them, art_conv2d_form among the first three (form = 0 asks for it; any other form comes back if it
+ * takes these sizes); 0 where these sizes are not taken. */
 int art_conv2d_form(int f16, int N, int C, int H, int W, int F, int HO, int WO, int ph, int pw, int form);
+int art_conv2d_choose(int f16, int N, int C, int H, int W, int F, int HO, int WO, int ph, int pw);
 size_t art_conv2d_packed_bytes(int f16, int C, int F);
+size_t art_conv2d_scratch_bytes(int f16, int N, int C, int H, int W, int F, int HO, int WO, int ph, int pw, int form);
 int art_conv2d(const void* x_dev, const void* w_dev, void* packed_dev, void* y_dev, int f16, int N, int C, int H, int W, int F, int HO,
                int WO, int ph, int pw, int form, void* stream);
 

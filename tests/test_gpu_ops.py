@@ -1224,6 +1224,62 @@ def test_convolution_blocks_match_float64(autort, dtype, form, case):
     assert ((y.cpu().double() - want).abs() <= bound + 1e-30).all()
 
 
+@pytest.mark.parametrize('dtype', ['float16', 'float32'])
+@pytest.mark.parametrize('case', CONV_CASES + [(1, 100, (11, 57), 70, (1, 1), (11, 57), True),      # several chunks, a row longer than a block of 64
+                                               (2, 40, (120, 5), 200, (1, 1), (120, 5), True)])     # many rows to a block
+def test_staged_convolution_blocks_match_float64(autort, dtype, case):
+    """Every form over the staged image, whole and in slices of the channels, with scratch that holds NaN: nothing is read that
+    was not written.  The bound is that of the gathering forms, one addition per slice more; the short sums (form 7) are held
+    to 2^-24 for each of a chain of 7 and two roundings."""
+    from ctypes import c_void_p
+    from antares_amd.runtime import capi
+    N, C, (H, W), F, (ph, pw), (HO, WO), _ = case
+    note(f'staged convolution {dtype} {case}')
+    g = torch.Generator().manual_seed(N * 1000 + C + W)
+    x, w = torch.randn(N, C, H, W, generator=g).to(getattr(torch, dtype)), torch.randn(F, C, 3, 3, generator=g).to(getattr(torch, dtype))
+    f16 = int(dtype == 'float16')
+    shape = (f16, N, C, H, W, F, HO, WO, ph, pw)
+    lib, dev = capi.lib(), autort.device()
+    xd, wd = x.to(dev), w.to(dev)
+    pad = max(ph, pw, 0) + 2
+
+    def reference(a, b):
+        return torch.nn.functional.conv2d(torch.nn.functional.pad(a, (pad, pad + 2, pad, pad + 2)), b)[:, :, pad - ph:pad - ph + HO, pad - pw:pad - pw + WO]
+    want, size = reference(x.double(), w.double()), reference(x.double().abs(), w.double().abs())
+    chunks = -(-C // (32 if f16 else 16))
+    for kind in (4, 5, 6) if f16 else (4, 5, 6, 7):
+        for slices in sorted({1, 2, 3, chunks}):
+            form = kind + 256 * slices
+            if slices > chunks:
+                assert lib.art_conv2d_form(*shape, form) == 0
+                continue
+            assert lib.art_conv2d_form(*shape, form) == form
+            y = torch.full((N, F, HO, WO), 7.0, device=dev)
+            scratch = torch.full((lib.art_conv2d_scratch_bytes(*shape, form),), 255, dtype=torch.uint8, device=dev)
+            capi.check(lib.art_conv2d(*(c_void_p(t.data_ptr()) for t in (xd, wd, scratch, y)), *shape, form, c_void_p(torch.cuda.current_stream().cuda_stream)))
+            bound = (9 * 2.0 ** -24 if kind == 7 else 2.0 ** -23 * 9 * C + slices * 2.0 ** -24) * size
+            assert bool(((y.cpu().double() - want).abs() <= bound + 1e-30).all()), (kind, slices)
+
+
+@pytest.mark.parametrize('dtype,n,c,f,hw', [('float16', 1, 216, 48, 35), ('float32', 2, 72, 56, 20), ('float32', 9, 216, 64, 17), ('float32', 12, 24, 24, 46),
+                                            ('float16', 6, 88, 40, 8)])
+def test_staged_convolutions_are_no_further_from_float64_than_the_generic_kernels(autort, dtype, n, c, f, hw):
+    from antares_amd.runtime import capi
+    note(f'staged convolution operator {dtype} {n}x{c}x{hw}x{hw} -> {f}')
+    dev, dt = autort.device(), getattr(torch, dtype)
+    assert capi.lib().art_conv2d_choose(int(dtype == 'float16'), n, c, hw, hw, f, hw, hw, 1, 1) & 255 > 3
+    x, w = torch.randn(n, c, hw, hw, device=dev).to(dt), torch.randn(f, c, 3, 3, device=dev).to(dt)
+    want = torch.nn.functional.conv2d(x.cpu().double(), w.cpu().double(), padding=1)
+    off = []
+    for generic in (False, True):
+        op = autort.export(ir=conv_program(dtype, (hw, hw), (hw, hw), (1, 1)),
+                           inputs=[f'input0={dtype}[N:{n}, C:{c}, H:{hw}, W:{hw}]', f'input1={dtype}[F:{f}, C:{c}, KH:3, KW:3]'], name=f'conv_st_{dtype}_{n}_{c}_{int(generic)}')
+        if generic:
+            op.fast_path = None
+        off.append(float((op(x, w).cpu().double() - want).norm() / want.norm()))
+    assert off[0] <= 1.05 * off[1], off
+
+
 @pytest.mark.parametrize('dtype,n,c,f,hw', [('float16', 4, 40, 72, 20), ('float16', 2, 64, 24, 23), ('float32', 5, 20, 72, 21), ('float16', 30, 16, 256, 28)])
 def test_convolution_operator_takes_the_kernel_and_agrees_with_the_generic_one(autort, dtype, n, c, f, hw):
     note(f'convolution operator {dtype} {n}x{c}x{hw}x{hw} -> {f}')
