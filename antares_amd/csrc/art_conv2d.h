@@ -28,6 +28,17 @@ template <> struct Elem<float> {
   }
 };
 
+// x / d for x below 2^30: x * mul >> shift with mul = ceil(2^shift / d), shift = 30 + ceil(log2 d).
+struct Div {
+  unsigned int mul, shift, by;
+};
+inline Div make_div(unsigned int d) {
+  unsigned int s = 0;
+  while ((1u << s) < d) ++s;
+  return Div{(unsigned int)(((1ull << (30 + s)) + d - 1) / d), 30 + s, d};
+}
+__device__ __forceinline__ unsigned int over(unsigned int x, const Div& d) { return (unsigned int)((unsigned long long)x * d.mul >> d.shift); }
+
 struct Geometry {
   int N, C, H, W, F, HO, WO, ph, pw;
   int columns;          // output points: N * HO * WO
@@ -35,13 +46,45 @@ struct Geometry {
   int row_tiles;        // 32-feature tiles of the packed filter
   int row_blocks;       // blocks along the features
   int span;             // points the LDS buffers hold
+  Div results, width;   // output points of an image, of a row
+  Div image, wide;      // padded points of an image, of a row
+  Div blocks_across;    // row_blocks
 };
 
 // Output point -> its place in the padded image (where tap (0, 0) reads).
 __device__ __forceinline__ int place_of(int column, const Geometry& g) {
-  const unsigned hw = (unsigned)(g.HO * g.WO), n = (unsigned)column / hw, r = (unsigned)column % hw;
-  const unsigned ho = r / (unsigned)g.WO, wo = r % (unsigned)g.WO;
-  return (int)((n * (unsigned)(g.HO + 2) + ho) * (unsigned)(g.WO + 2) + wo);
+  const unsigned n = over((unsigned)column, g.results), r = (unsigned)column - n * g.results.by, ho = over(r, g.width), wo = r - ho * g.width.by;
+  return (int)((n * (unsigned)(g.HO + 2) + ho) * g.wide.by + wo);
+}
+
+// A wavefront's tiles to memory: accumulator element e is feature f0 + (e / 4) * 8 + (lane / 32) * 4 + e % 4 of the tile, point
+// lane % 32 at to[j].  One addition per store: worked out anew each time, the addresses were a quarter of the kernels' code.
+template <int MT, int NT>
+__device__ __forceinline__ void store_results(const f32x16 (&total)[MT][NT], float* y, const size_t (&to)[NT], int column, int last, int f_first, const Geometry& g) {
+  const int hl = (threadIdx.x & 63) >> 5;
+  const size_t plane = g.results.by;
+#pragma unroll
+  for (int j = 0; j < NT; ++j) {
+    if (column + j * 32 > last) continue;
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+      const int f0 = f_first + i * 32;
+      float* p = y + to[j] + (size_t)(f0 + hl * 4) * plane;
+      if (f0 + 32 <= g.F) {
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          __builtin_nontemporal_store(total[i][j][e], p);
+          p += (e & 3) == 3 ? 5 * plane : plane;
+        }
+      } else {
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          if (f0 + (e >> 2) * 8 + hl * 4 + (e & 3) < g.F) __builtin_nontemporal_store(total[i][j][e], p);
+          p += (e & 3) == 3 ? 5 * plane : plane;
+        }
+      }
+    }
+  }
 }
 
 // Forms 4 to 7 (art_conv2d_staged.hip): blocks of 64 features x 64 points, 64 x 128, 128 x 128, and 64 x 64 with short sums (float32

@@ -23,7 +23,7 @@
 //     20 x 24 -> 64, 20 x 20 12.0 -> 10.5 us (generic 11.4), float16 19 x 19 of 16 channels 8.8 -> 7.3 (7.7 to 8.4);
 //   * 2 x 2 wavefronts of MT x NT tiles of 32 features x 32 points; blocks of one run of points are neighbours on one XCD.
 // Measured, padding 1, both launches, against the generic lowering (a padded copy, then a gathering product): float16
-// 32 x 128 x 28 x 28 -> 128 40.2 -> 20.1 us, 24 x 200 x 33 x 33 -> 48 89 -> 23 us, 2 x 160 x 18 x 18 -> 64 57 -> 14 us;
+// 32 x 128 x 28 x 28 -> 128 40.2 -> 18.4 us, 24 x 200 x 33 x 33 -> 48 89 -> 23 us, 2 x 160 x 18 x 18 -> 64 57 -> 14 us;
 // float32 32 x 128 x 28 x 28 -> 128 113 -> 81 us (the matrix instructions alone take 47), 23 x 128 x 30 x 30 -> 176 119 -> 86.
 // The first of these spends 7 us of the matrix cores' time in 18.6 us: one block per compute unit and only 4 chunks, so the
 // first image fetch, the waits between chunks and the stores of 12.8 MB stay in sight; packing the filter takes 2.3 us.
@@ -69,18 +69,18 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 4))
   unsigned* where = reinterpret_cast<unsigned*>(lds + 2 * (size_t)g.span * kPitchBytes);   // [span]: byte offset into x without the channel, or kOutside
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave >> 1, wn = wave & 1;
-  const int wide = g.WO + 2, high = g.HO + 2;
+  const int wide = g.WO + 2;
   // workgroups go to the eight XCDs round robin: an XCD gets a contiguous run of blocks
   const int per = gridDim.x >> 3, left = gridDim.x & 7, xcd = blockIdx.x & 7;
   const int block = xcd * per + (xcd < left ? xcd : left) + (blockIdx.x >> 3);
-  const int rb = block % g.row_blocks, column0 = (block / g.row_blocks) * TN;
+  const int run = (int)over((unsigned)block, g.blocks_across), rb = block - run * g.row_blocks, column0 = run * TN;
   const int last = (column0 + TN < g.columns ? column0 + TN : g.columns) - 1;
   const int place0 = place_of(column0, g);
   const int points = place_of(last, g) - place0 + 2 * wide + 3;            // <= span
 
   for (int i = tid; i < points; i += kThreads) {
-    const unsigned p = (unsigned)(place0 + i), n = p / (unsigned)(high * wide), r = p % (unsigned)(high * wide);
-    const int h = (int)(r / (unsigned)wide) - g.ph, w = (int)(r % (unsigned)wide) - g.pw;
+    const unsigned p = (unsigned)(place0 + i), n = over(p, g.image), r = p - n * g.image.by, row = over(r, g.wide);
+    const int h = (int)row - g.ph, w = (int)(r - row * g.wide.by) - g.pw;
     const bool in = h >= 0 && h < g.H && w >= 0 && w < g.W;
     where[i] = in ? ((n * (unsigned)g.C * (unsigned)g.H + (unsigned)h) * (unsigned)g.W + (unsigned)w) * (unsigned)sizeof(T) : kOutside;
   }
@@ -93,8 +93,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 4))
     int column = column0 + wn * 32 * NT + j * 32 + (lane & 31);
     if (column > last) column = last;
     at[j] = (place_of(column, g) - place0) * kPitch + (lane >> 5) * V;
-    const unsigned hw = (unsigned)(g.HO * g.WO);
-    to[j] = (size_t)((unsigned)column / hw) * g.F * hw + (unsigned)column % hw;
+    const unsigned hw = g.results.by, n = over((unsigned)column, g.results);
+    to[j] = (size_t)n * g.F * hw + ((unsigned)column - n * hw);
   }
   // Item i of a lane: point lane + 64 i, channels wave * V .. + V - 1 of the chunk.  Loads go out without a branch between
   // them (points and channels past the end re-read the last one) and stay as they came until they are put into LDS: a
@@ -218,18 +218,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 4))
   if (MT == 1 && g.C - (g.chunks - 1) * 4 * V <= 2 * V) chunk(g.chunks - 1, std::true_type{}, std::true_type{});   // MT = 2 has no registers left for it
   else chunk(g.chunks - 1, std::true_type{}, std::false_type{});
 
-  // accumulator element e: feature (e / 4) * 8 + (lane / 32) * 4 + e % 4 of the tile, point lane % 32
-#pragma unroll
-  for (int j = 0; j < NT; ++j) {
-    if (column0 + wn * 32 * NT + j * 32 + (lane & 31) > last) continue;
-#pragma unroll
-    for (int i = 0; i < MT; ++i)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        const int f = ((rb * 2 + wm) * MT + i) * 32 + (e >> 2) * 8 + (lane >> 5) * 4 + (e & 3);
-        if (f < g.F) __builtin_nontemporal_store(total[i][j][e], y + to[j] + (size_t)f * g.HO * g.WO);
-      }
-  }
+  store_results<MT, NT>(total, y, to, column0 + wn * 32 * NT + (lane & 31), last, ((rb * 2 + wm) * MT) * 32, g);
 }
 
 // The most points a block of `columns` output points can need: every step to the next row skips two points, every
@@ -252,7 +241,7 @@ int points_of(int form) { return shape_of(form) == 1 ? 64 : 128; }
 int slices_of(int form) { return form >> 8 ? form >> 8 : 1; }
 
 bool geometry(Geometry& g, int f16, int N, int C, int H, int W, int F, int HO, int WO, int ph, int pw) {
-  g = Geometry{N, C, H, W, F, HO, WO, ph, pw, 0, 0, 0, 0, 0};
+  g = Geometry{N, C, H, W, F, HO, WO, ph, pw};
   if (N < 1 || C < 1 || H < 1 || W < 1 || F < 1 || HO < 1 || WO < 1) return false;
   // byte offsets into x and places in the padded image are 32-bit
   if ((long long)HO > (1 << 20) || (long long)WO > (1 << 20)) return false;
@@ -260,6 +249,10 @@ bool geometry(Geometry& g, int f16, int N, int C, int H, int W, int F, int HO, i
   if (image > (1LL << 30) / N || (long long)H * W > (1LL << 30) / ((long long)N * C)) return false;
   if ((long long)N * C * H * W * (f16 ? 2 : 4) > (1LL << 31)) return false;
   g.columns = N * HO * WO;
+  g.results = make_div((unsigned)(HO * WO));
+  g.width = make_div((unsigned)WO);
+  g.image = make_div((unsigned)((HO + 2) * (WO + 2)));
+  g.wide = make_div((unsigned)(WO + 2));
   g.chunks = (C + (f16 ? 31 : 15)) / (f16 ? 32 : 16);
   return (long long)g.chunks * kTaps * ((F + 127) / 128) * 4 < (1 << 22);      // packed filter below 4 GiB
 }
@@ -276,25 +269,20 @@ long long blocks_of(const Geometry& g, int form) {
   return (long long)((g.columns + points_of(form) - 1) / points_of(form)) * ((g.F + features_of(form) - 1) / features_of(form));
 }
 
-// What a launch of a form takes, in microseconds, up to a part that is the same for all of them: blocks go to the compute
-// units in rounds, and a round is a ramp and its chunks.  In float32 a round lasts as long full or not (the blocks of a unit
-// share its matrix cores); in float16, where they mostly wait, half of the last round is paid by its blocks.  Fitted to 350
-// sizes in float32 and 260 in float16 (C 16-256, F 16-256, images of 7-56 squared, batches 1-32): 2.4 and 4.1 % off, and the
-// form it picks is 0.2 and 0.3 % slower than the fastest one in the mean.  Float32: 23 x 128 -> 80, 38 x 38 takes 111 / 124 /
-// 150 us in 1038 / 520 / 260 blocks (5, 3, 2 rounds), 11 x 144 -> 232, 28 x 28 79 / 95 / 90 us in 540 / 272 / 136 (3, 2, 1);
-// float16: 32 x 128 -> 128, 28 x 28 27.1 / 21.7 / 21.1 us in 784 / 392 / 196, 13 x 24 -> 88, 39 x 39 11.9 / 10.7 / 11.7 in
-// 618 / 310 / 155.
+// What a form takes, in microseconds, both launches: a fixed part, per chunk of a block a time that grows with the blocks that
+// share a compute unit and with how unevenly they do, a ramp per further round, and the stores.  Fitted to 157 sizes in float16
+// and 153 in float32 (C 16-256, F 16-256, images of 7-56 squared, batches 1-32): 4.4 and 2.1 % off.  Over 150 other sizes
+// the form picked among all, the staged ones below included, was 0.2 % slower than the fastest in the mean, 1.2 times at worst.
 constexpr int kUnits = 256;                      // compute units of an MI355X
 double launch_time(const Geometry& g, int f16, int form) {
-  struct Cost { double fixed, chunk, round; };
-  static const Cost cost[2][3] = {{{6.9, 2.74, -0.65}, {8.3, 5.11, -1.82}, {8.7, 9.09, -1.55}},
-                                  {{7.1, 1.43, -0.31}, {8.35, 2.12, -1.15}, {8.9, 2.80, -0.80}}};
+  struct Cost { double fixed, alone, shared, uneven, again; };
+  static const Cost cost[2][3] = {{{5.66, 3.189, 2.500, 2.260, 0.486}, {5.97, 5.350, 4.539, 4.369, 0.0}, {5.92, 9.003, 8.308, 8.981, 4.782}},
+                                  {{6.32, 1.718, 1.331, 0.781, 0.169}, {6.89, 2.324, 1.382, 0.819, 0.466}, {7.26, 2.992, 1.627, 2.012, 0.271}}};
   const Cost& c = cost[f16 != 0][form - 1];
   const int per_chunk = f16 ? 32 : 16;
   const double chunks = g.chunks - (form < 3 && g.C - (g.chunks - 1) * per_chunk <= per_chunk / 2 ? 0.5 : 0.0);
-  const long long blocks = blocks_of(g, form), whole = (blocks + kUnits - 1) / kUnits;
-  const double rounds = f16 && whole > 1 ? 0.5 * ((double)blocks / kUnits + whole) : (double)whole;
-  return c.fixed + rounds * (chunks * c.chunk + c.round);
+  const double rounds = (double)blocks_of(g, form) / kUnits, full = rounds > 1 ? rounds : 1, uneven = ceil(rounds) > full ? ceil(rounds) - full : 0;
+  return c.fixed + chunks * (c.alone + c.shared * (full - 1) + c.uneven * uneven) + c.again * (full - 1) + (f16 ? 0.207 : 0.357) * 4e-6 * g.columns * g.F;
 }
 
 // The same for the staged forms (the launch that stages the image included): a fixed part, per chunk of a block's slice a time
@@ -322,26 +310,25 @@ double staged_time(const Geometry& g, int f16, int form, int slices) {
 // above, times in us generic / here.
 //  * fewer than 32 features, or fewer than 16 blocks of 64 x 64: the generic path sums on the vector units in short
 //    chains.  In float32 that error (0.73e-7 to 1.26e-7 against 64 bits) is below the matrix instructions' (1.2e-7 to 1.5e-7), not
-//    below that of the short sums (0.69e-7 to 0.76e-7): form 7, where it is faster than 5.5 us + 1.1 ps per product there:
-//    375 / 37 (2 x 232 -> 24, 52 x 52), 57 / 16 (3 x 184 -> 48, 14 x 14), 7.6 / 13.7 (1 x 24 -> 32, 15 x 15).  In
-//    float16 the error is the same (0.7-1.1e-7 both) from 64 channels on; below 8192 results the generic path wins (5.6 / 7.0 for
-//    1 x 16 -> 40, 7 x 7).
+//    below that of the short sums (0.69e-7 to 0.76e-7): form 7 only.  In float16 it is that of the blocks of 64 x 64, whose rows of
+//    taps are summed by themselves (0.69e-7 to 1.1e-7 there, 0.62e-7 to 0.87e-7 here; the larger blocks have 1.2e-7).  Where it is
+//    faster than 5.5 us + 1.1 ps per product there (float16 5.3 us + 1.3 ps): float32 375 / 37 (2 x 232 -> 24, 52 x 52), 57 / 16
+//    (3 x 184 -> 48, 14 x 14), 7.6 / 13.7 (1 x 24 -> 32, 15 x 15); float16 319 / 19 (28 x 40 -> 16, 42 x 42), 16.7 / 8.1 (4 x 48 -> 16,
+//    20 x 20), 5.6 / 7.0 (1 x 16 -> 40, 7 x 7).
 //  * elsewhere one of the forms wins, with the channels sliced where there are few blocks: float32 23 / 20 (9 x 216 -> 64,
 //    17 x 17, 46 without slices), float16 19 / 13.8 (9 x 240 -> 104, 13 x 13).  The image is staged unless it is large and
 //    there is little to multiply: float16 18 x 64 -> 48, 51 x 51 15.3 gathered, 16.8 staged, 1 x 40 -> 152, 42 x 42 10.0 and 9.0.
-//  * below 32 features only 64 x 64, whose rows of taps are summed by themselves: the larger blocks' error is 1.2e-7.
 int choose(const Geometry& g, int f16) {
   const long long small = blocks_of(g, 1), results = (long long)g.columns * g.F;
   const bool vector_units = g.F < 32 || small < 16;
-  if (f16 && vector_units && (results < 8192 || (g.F < 32 && g.C < 64))) return 0;
   int best = 0;
-  double t_best = f16 || !vector_units ? 1e30 : 5.5 + 1.1e-6 * results * 9 * g.C;
+  double t_best = !vector_units ? 1e30 : (f16 ? 5.3 : 5.5) + (f16 ? 1.3e-6 : 1.1e-6) * results * 9 * g.C;
   auto consider = [&](int form, double t) {
     if (t < t_best && fits(g, f16, form)) { best = form; t_best = t; }
   };
   for (int form = 1; form <= 7; ++form) {
     if (form == 7 ? f16 || !vector_units : !f16 && vector_units) continue;
-    if (shape_of(form) != 1 && g.F < 32) continue;
+    if (shape_of(form) != 1 && vector_units) continue;
     if (form <= 3) consider(form, launch_time(g, f16, form));
     for (int slices : {1, 2, 3, 4, 5, 6, 8, 12})
       if (form > 3 && slices <= g.chunks && (slices == 1 || slices * blocks_of(g, form) <= 4 * kUnits)) consider(form + (slices > 1 ? 256 * slices : 0), staged_time(g, f16, form, slices));
@@ -417,6 +404,7 @@ extern "C" int art_conv2d(const void* x_dev, const void* w_dev, void* packed_dev
               "art_conv2d: the result must not overlap an operand");
   g.row_blocks = (F + features_of(form) - 1) / features_of(form);
   g.row_tiles = g.row_blocks * (features_of(form) / 32);
+  g.blocks_across = make_div((unsigned)g.row_blocks);
   g.span = span_of(g, points_of(form));
   if ((form & 255) > 3)
     return run_staged(x_dev, w_dev, packed_dev, y_dev, g, f16, form & 255, slices_of(form), (int)blocks_of(g, form), (hipStream_t)stream);

@@ -28,34 +28,16 @@ using namespace art::conv;
 using art::load_lds_x4;
 using art::uniform;
 
-// x / d for x below 2^30: x * mul >> shift with mul = ceil(2^shift / d), shift = 30 + ceil(log2 d).
-struct Div {
-  unsigned int mul, shift, by;
-};
-Div make_div(unsigned int d) {
-  unsigned int s = 0;
-  while ((1u << s) < d) ++s;
-  return Div{(unsigned int)(((1ull << (30 + s)) + d - 1) / d), 30 + s, d};
-}
-__device__ __forceinline__ unsigned int over(unsigned int x, const Div& d) { return (unsigned int)((unsigned long long)x * d.mul >> d.shift); }
-
 struct Staged {
   Geometry g;
-  Div results, width;        // output points of an image, of a row
-  Div image, wide;           // padded points of an image, of a row
   int places;                // padded points in all
   int filter_blocks, place_blocks;
   const char* image_copy;
-  Div blocks, row_blocks;    // blocks of a slice of the chunks, and along the features
+  Div blocks;                // blocks of a slice of the chunks
   int slices, slice_chunks, longer;      // chunks of a slice; the first `longer` slices have one more
   long long results_all;     // N * F * HO * WO
   int half_last;             // of the last chunk only the lower half of the channels exists
 };
-
-__device__ __forceinline__ int place_in(unsigned int column, const Staged& s) {
-  const unsigned int n = over(column, s.results), r = column - n * s.results.by, ho = over(r, s.width), wo = r - ho * s.width.by;
-  return (int)((n * (unsigned)(s.g.HO + 2) + ho) * s.wide.by + wo);
-}
 
 // Blocks in front: filter [F][C][taps] -> [chunk][tap][32 features][half][lane][16 bytes], zeros past F and C.  The others: 64 points of
 // a chunk of channels, a wavefront per 16 bytes of them.  Bound by latency for small images, by memory for large ones.
@@ -82,8 +64,8 @@ __global__ __launch_bounds__(kThreads) void conv2d_stage_kernel(const T* __restr
   __shared__ __align__(16) vec turned[64 * 4];          // the points' pieces meet here, so that the stores are whole lines
   const int b = blockIdx.x - s.filter_blocks, q = b / s.place_blocks, piece = threadIdx.x >> 6, local = threadIdx.x & 63;
   const unsigned place = (unsigned)(b - q * s.place_blocks) * 64 + local;
-  const unsigned n = over(place, s.image), r = place - n * s.image.by, ph = over(r, s.wide);
-  const int h = (int)ph - g.ph, wc = (int)(r - ph * s.wide.by) - g.pw, c0 = (q * 4 + piece) * V;
+  const unsigned n = over(place, g.image), r = place - n * g.image.by, ph = over(r, g.wide);
+  const int h = (int)ph - g.ph, wc = (int)(r - ph * g.wide.by) - g.pw, c0 = (q * 4 + piece) * V;
   const bool in = place < (unsigned)s.places && h >= 0 && h < g.H && wc >= 0 && wc < g.W;
   const size_t plane = (size_t)g.H * g.W;
   const T* from = x + (in ? ((size_t)n * g.C * g.H + h) * g.W + wc : 0);
@@ -117,12 +99,12 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, MT 
   // workgroups go to the eight XCDs round robin: an XCD gets a contiguous run of blocks
   const int per = gridDim.x >> 3, left = gridDim.x & 7, xcd = blockIdx.x & 7;
   const int block = xcd * per + (xcd < left ? xcd : left) + (blockIdx.x >> 3);
-  const int slice = (int)over((unsigned)block, s.blocks), in_slice = block - slice * (int)s.blocks.by, run = (int)over((unsigned)in_slice, s.row_blocks);
+  const int slice = (int)over((unsigned)block, s.blocks), in_slice = block - slice * (int)s.blocks.by, run = (int)over((unsigned)in_slice, g.blocks_across);
   const int chunk0 = slice * s.slice_chunks + (slice < s.longer ? slice : s.longer), chunks = s.slice_chunks + (slice < s.longer ? 1 : 0);
-  const int rb = in_slice - run * (int)s.row_blocks.by, column0 = run * TN;
+  const int rb = in_slice - run * (int)g.blocks_across.by, column0 = run * TN;
   const int last = (column0 + TN < g.columns ? column0 + TN : g.columns) - 1;
-  const int wide = (int)s.wide.by, place0 = place_in(column0, s);
-  const int units = (place_in(last, s) - place0 + 2 * wide + 3 + 15) >> 4;          // 16 points = 1 KiB of a chunk
+  const int wide = (int)g.wide.by, place0 = place_of(column0, g);
+  const int units = (place_of(last, g) - place0 + 2 * wide + 3 + 15) >> 4;          // 16 points = 1 KiB of a chunk
   const unsigned buffer = (unsigned)((g.span + 15) >> 4) << 10;                   // bytes of a chunk's points
   const size_t chunk_bytes = (size_t)s.places * kChunkBytes;
   const char* image = s.image_copy + (size_t)place0 * kChunkBytes + (size_t)chunk0 * chunk_bytes;
@@ -161,9 +143,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, MT 
   for (int j = 0; j < NT; ++j) {
     int column = column0 + wn * 32 * NT + j * 32 + (lane & 31);
     if (column > last) column = last;
-    at[j] = (unsigned)(place_in(column, s) - place0);
-    const unsigned n = over((unsigned)column, s.results);
-    to[j] = (size_t)n * g.F * s.results.by + ((unsigned)column - n * s.results.by);
+    at[j] = (unsigned)(place_of(column, g) - place0);
+    const unsigned n = over((unsigned)column, g.results);
+    to[j] = (size_t)n * g.F * g.results.by + ((unsigned)column - n * g.results.by);
   }
 
   double fine[FINE ? 16 : 1] = {};
@@ -244,31 +226,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, MT 
     for (int e = 0; e < 16; ++e) total[0][0][e] = (float)fine[e];
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");    // nothing of the ring is on its way when its space is given back
 
-  // accumulator element e: feature (e / 4) * 8 + (lane / 32) * 4 + e % 4 of the tile, point lane % 32
-  const size_t plane = s.results.by;
-  y += slice * s.results_all;
-#pragma unroll
-  for (int j = 0; j < NT; ++j) {
-    if (column0 + wn * 32 * NT + j * 32 + (lane & 31) > last) continue;
-#pragma unroll
-    for (int i = 0; i < MT; ++i) {
-      const int f0 = ((rb * 2 + wm) * MT + i) * 32;
-      float* p = y + to[j] + (size_t)(f0 + hl * 4) * plane;
-      if (f0 + 32 <= g.F) {
-#pragma unroll
-        for (int e = 0; e < 16; ++e) {
-          __builtin_nontemporal_store(total[i][j][e], p);
-          p += (e & 3) == 3 ? 5 * plane : plane;
-        }
-      } else {
-#pragma unroll
-        for (int e = 0; e < 16; ++e) {
-          if (f0 + (e >> 2) * 8 + hl * 4 + (e & 3) < g.F) __builtin_nontemporal_store(total[i][j][e], p);
-          p += (e & 3) == 3 ? 5 * plane : plane;
-        }
-      }
-    }
-  }
+  store_results<MT, NT>(total, y + slice * s.results_all, to, column0 + wn * 32 * NT + (lane & 31), last, ((rb * 2 + wm) * MT) * 32, g);
 }
 
 size_t filter_bytes(const Geometry& g) { return ((size_t)g.chunks * kTaps * ((g.F + 127) / 128) * 4 * 2048 + 255) & ~(size_t)255; }
@@ -314,15 +272,10 @@ size_t art::conv::staged_lds(const Geometry& g) { return (size_t)((g.span + 15) 
 int art::conv::run_staged(const void* x, const void* w, void* packed, void* y, const Geometry& g, int f16, int form, int slices, int blocks, hipStream_t stream) {
   Staged s{};
   s.g = g;
-  s.results = make_div((unsigned)(g.HO * g.WO));
-  s.width = make_div((unsigned)g.WO);
-  s.image = make_div((unsigned)((g.HO + 2) * (g.WO + 2)));
-  s.wide = make_div((unsigned)(g.WO + 2));
   s.places = (int)places_of(g);
   s.filter_blocks = (g.chunks * kTaps * g.row_tiles * 128 + kThreads - 1) / kThreads;
   s.place_blocks = (s.places + 63) / 64;
   s.blocks = make_div((unsigned)blocks);
-  s.row_blocks = make_div((unsigned)g.row_blocks);
   s.slices = slices;
   s.slice_chunks = g.chunks / slices;
   s.longer = g.chunks % slices;

@@ -1262,7 +1262,7 @@ def test_staged_convolution_blocks_match_float64(autort, dtype, case):
 
 
 @pytest.mark.parametrize('dtype,n,c,f,hw', [('float16', 1, 216, 48, 35), ('float32', 2, 72, 56, 20), ('float32', 9, 216, 64, 17), ('float32', 12, 24, 24, 46),
-                                            ('float16', 6, 88, 40, 8)])
+                                            ('float16', 6, 88, 40, 8), ('float16', 4, 48, 16, 20)])
 def test_staged_convolutions_are_no_further_from_float64_than_the_generic_kernels(autort, dtype, n, c, f, hw):
     from antares_amd.runtime import capi
     note(f'staged convolution operator {dtype} {n}x{c}x{hw}x{hw} -> {f}')
