@@ -69,6 +69,16 @@ __device__ __forceinline__ const void* uniform(const void* p) {
                        (unsigned long long)(unsigned int)__builtin_amdgcn_readfirstlane((int)(v >> 32)) << 32);
 }
 
+// g / (1 + e^-g) of a value that fp16 holds.  t, g times log2(e) cut to 13 bits, is exact; e^-g = 2^n 2^(t - n + the rest).
+// The quotient is corrected once; numerator and denominator are divided by 16, so that its reciprocal stays a normal
+// number.  Zeros, infinities and NaN come out as of the division itself (-infinity: NaN).
+__device__ __forceinline__ float silu(float g) {
+  const float at = __builtin_amdgcn_fmed3f(g, -96.0f, 96.0f), t = at * -1.442626953125f, n = rintf(t);
+  const float e = ldexpf(__builtin_amdgcn_exp2f(fmaf(at, -6.8087776e-5f, t - n)), (int)n);
+  const float num = g * 0.0625f, den = fmaf(e, 0.0625f, 0.0625f), r = __builtin_amdgcn_rcpf(den), q = num * r;
+  return __builtin_amdgcn_div_fixupf(fmaf(fmaf(0.0f - den, q, num), r, q), den, num);
+}
+
 }  // namespace art
 
 // Workgroup barrier that orders LDS traffic only.  __syncthreads() also waits for every outstanding

@@ -29,6 +29,10 @@
 // card, weights from memory: 64 rows over 4096 x 4096 / 4096 x 22016 / 11008 x 4096 13.6 / 28.6 / 18.2 us -> 11.2 / 22.4 / 16.9;
 // 50 rows over 11008 x 4096 17.9 -> 16.2; 128 rows over 4096 x 12288 / 22016 28.1 / 40.0 -> 22.3 / 31.2; 16 rows over
 // 1024 x 3072 7.4 -> 6.8.
+// The end of a block: the k halves exchange halves of their sums as they lie in the registers, the K-splits' sums leave from
+// there, SWIGLU pairs gate and up by lane exchange.  Against sums that meet as [row][column] by one half of the wavefronts and are
+// read back by fours, half of the lanes without work in SWIGLU, on one card: 128 rows over 4096 x 22016 34.9 -> 32.5 us, SWIGLU
+// 39.0 -> 35.3, 50 rows with SWIGLU 26.6 -> 25.2, six splits of 128 rows over 11008 x 4096 26.1 -> 25.5.
 #include "art_w4_mfma.h"
 
 #include <type_traits>
@@ -41,11 +45,10 @@ constexpr int kThreads = 512;                       // 8 wavefronts: 4 column qu
 constexpr int BN = 128, GK = 128;                   // columns of a block, k of a quantisation group
 constexpr int W_BYTES = (GK / 2) * BN;              // packed weights of a group: 64 byte-rows x 128 columns
 constexpr int Q_BYTES = 2048;                       // scales (256 B) at 0, zero points (64 B) at 256; the rest takes the idle lanes
-constexpr int RLD = BN + 4;                         // floats per row of a result tile in LDS
 constexpr int stage_bytes(int MT) { return W_BYTES + Q_BYTES + MT * 32 * GK * 2; }
 constexpr size_t lds_bytes(int MT) { return 3 * (size_t)stage_bytes(MT); }     // 55, 80 (two blocks per compute unit), 129 KB
-static_assert(32 * RLD * 4 <= 3 * stage_bytes(1) && 64 * RLD * 4 <= 3 * stage_bytes(2) && 128 * RLD * 4 <= 3 * stage_bytes(4),
-              "the result tile of the epilogue fits the ring");
+static_assert(16 * 1024 + 32 * (BN + 8) * 2 <= 3 * stage_bytes(1) && 32 * 1024 + 64 * (BN + 8) * 2 <= 3 * stage_bytes(2) &&
+                  64 * 1024 + 128 * (BN + 8) * 2 <= 3 * stage_bytes(4), "the sums that are handed over and the results fit the ring");
 
 // How the (column tile, K split) pairs are laid out; worked out on the host, so that a block starts without divisions.
 struct Work {
@@ -231,46 +234,66 @@ __global__ __launch_bounds__(kThreads, MT == 4 ? 2 : 4) void gemm_w4a16_kernel(
 
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // nothing of the ring is on its way when its space is reused or given back
 
-  // ---- the two k halves meet in LDS as [row][column]; then every thread owns four neighbouring columns.
-  // Accumulator element r of tile t is row t*32 + (r/4)*8 + (lane/32)*4 + r%4.
-  float* red = reinterpret_cast<float*>(smem);
-  auto at = [&](int t, int r) { return (t * 32 + (r >> 2) * 8 + h * 4 + (r & 3)) * RLD + colpos; };
+  // ---- the two k halves meet: wavefront (c, h) hands half of its sums to (c, 1 - h), by fours of rows, and keeps the other.
+  // Accumulator elements 4 (q % 4) .. + 3 of tile q / 4 are rows (q / 4) * 32 + (q % 4) * 8 + (lane / 32) * 4 .. + 3.
+  constexpr int KEEP = 2 * MT;
+  f32x4* const meet = reinterpret_cast<f32x4*>(smem) + cw * KEEP * 64 + lane;
+  auto quad = [&](int q) { return f32x4{acc[q >> 2][4 * (q & 3)], acc[q >> 2][4 * (q & 3) + 1], acc[q >> 2][4 * (q & 3) + 2], acc[q >> 2][4 * (q & 3) + 3]}; };
+  f32x4 sum[KEEP];
   __syncthreads();
-  if (kh == 1)
+  if (kh == 0) {
 #pragma unroll
-    for (int t = 0; t < MT; ++t)
+    for (int j = 0; j < KEEP; ++j) { meet[(4 * KEEP + j) * 64] = quad(KEEP + j); sum[j] = quad(j); }
+  } else {
 #pragma unroll
-      for (int r = 0; r < 16; ++r) red[at(t, r)] = acc[t][r];
+    for (int j = 0; j < KEEP; ++j) { meet[j * 64] = quad(j); sum[j] = quad(KEEP + j); }
+  }
   __syncthreads();
-  if (kh == 0)
 #pragma unroll
-    for (int t = 0; t < MT; ++t)
+  for (int j = 0; j < KEEP; ++j) sum[j] += meet[(4 * KEEP * kh + j) * 64];
+  auto row_of = [&](int j) { return ((kh * KEEP + j) >> 2) * 32 + ((kh * KEEP + j) & 3) * 8 + h * 4; };
+  if (work.splits > 1) {                            // 64 bytes and more of a row at a time
+    if (!cols.inside(colpos)) return;
+    float* const to = partial + ((size_t)split * M + m0) * N + cols.at(colpos);
 #pragma unroll
-      for (int r = 0; r < 16; ++r) red[at(t, r)] += acc[t][r];
-  __syncthreads();
-  constexpr int kQuads = BN / 4;
-#pragma unroll 1
-  for (int e = tid; e < BM * kQuads; e += kThreads) {
-    const int row = e / kQuads, c4 = (e % kQuads) * 4;
-    if (m0 + row >= M || !cols.inside(c4)) continue;
-    const size_t out = (size_t)(m0 + row) * N + cols.at(c4);
-    const f32x4 v = *reinterpret_cast<const f32x4*>(red + row * RLD + c4);
-    if (work.splits > 1) {
-      *reinterpret_cast<f32x4*>(partial + (size_t)split * M * N + out) = v;
-    } else if (SWIGLU) {                            // the gate half of the tile works, with the up half 64 columns further on
-      if (c4 >= BN / 2) continue;
-      const f32x4 u = *reinterpret_cast<const f32x4*>(red + row * RLD + BN / 2 + c4);
-      *reinterpret_cast<h4*>(y + (size_t)(m0 + row) * (N / 2) + cols.at(c4)) =
-          swiglu4(h4{(_Float16)v[0], (_Float16)v[1], (_Float16)v[2], (_Float16)v[3]}, h4{(_Float16)u[0], (_Float16)u[1], (_Float16)u[2], (_Float16)u[3]});
-    } else {
-      h4 o = h4{(_Float16)v[0], (_Float16)v[1], (_Float16)v[2], (_Float16)v[3]};
-      if (residual) {                               // y = fp16(fp16(product) + residual); may alias y: same elements
-        const h4 res = *reinterpret_cast<const h4*>(residual + out);
-        o = h4{(_Float16)((float)o[0] + (float)res[0]), (_Float16)((float)o[1] + (float)res[1]),
-               (_Float16)((float)o[2] + (float)res[2]), (_Float16)((float)o[3] + (float)res[3])};
+    for (int j = 0; j < KEEP; ++j)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (m0 + row_of(j) + i < M) to[(size_t)(row_of(j) + i) * N] = sum[j][i];
+    return;
+  }
+  // fp16 results to LDS as [row][column], out in pieces of eight columns.  SWIGLU: lanes 0-15 hold a gate column, lanes 16-31 its up
+  // column; exchanged, the lower ones have both of one row and the upper ones both of the next.
+  constexpr int COLS = SWIGLU ? BN / 2 : BN, C_LD = COLS + 8;
+  _Float16* const cs = reinterpret_cast<_Float16*>(smem + 8 * KEEP * 1024);
+#pragma unroll
+  for (int j = 0; j < KEEP; ++j) {
+    if constexpr (SWIGLU) {
+#pragma unroll
+      for (int i = 0; i < 4; i += 2) {
+        const float here = sum[j][i], next = sum[j][i + 1];      // (a bit cast of an element of a vector takes its first one)
+        const auto pair = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned int, here), __builtin_bit_cast(unsigned int, next), false, false);
+        const float g = (float)(_Float16)__builtin_bit_cast(float, (unsigned int)pair[0]), u = (float)(_Float16)__builtin_bit_cast(float, (unsigned int)pair[1]);
+        cs[(row_of(j) + i + hi16) * C_LD + cw * 16 + s16] = (_Float16)(art::silu(g) * u);
       }
-      *reinterpret_cast<h4*>(y + out) = o;
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) cs[(row_of(j) + i) * C_LD + colpos] = (_Float16)sum[j][i];
     }
+  }
+  __syncthreads();
+#pragma unroll 1
+  for (int e = tid; e < BM * (COLS / 8); e += kThreads) {
+    const int row = e / (COLS / 8), c8 = (e % (COLS / 8)) * 8;
+    if (m0 + row >= M || !cols.inside(c8)) continue;
+    const size_t out = (size_t)(m0 + row) * (SWIGLU ? N / 2 : N) + cols.at(c8);
+    h8 o = *reinterpret_cast<const h8*>(cs + row * C_LD + c8);
+    if (!SWIGLU && residual) {                      // y = fp16(fp16(product) + residual); may alias y: same elements
+      const h8 res = *reinterpret_cast<const h8_by_8*>(residual + out);
+#pragma unroll
+      for (int k = 0; k < 8; ++k) o[k] = (_Float16)((float)o[k] + (float)res[k]);
+    }
+    *reinterpret_cast<h8_by_8*>(y + out) = o;
   }
 }
 

@@ -283,9 +283,8 @@ __global__ __launch_bounds__(kThreads, MT == 8 ? 1 : 2) void gemm_w4a16_wide_ker
         const int row = c >> 4, col = (c & 15) * 8, grow = m0 + p * 128 + row;
         if (grow >= M || !cols.inside(col)) continue;
         const h8 g = *reinterpret_cast<const h8*>(cs + row * C_LD + col), u = *reinterpret_cast<const h8*>(cs + row * C_LD + 128 + col);
-        _Float16* dst = y + (size_t)grow * (N / 2) + cols.at(col);      // y is 8-byte aligned
-        *reinterpret_cast<h4*>(dst) = swiglu4(h4{g[0], g[1], g[2], g[3]}, h4{u[0], u[1], u[2], u[3]});
-        *reinterpret_cast<h4*>(dst + 4) = swiglu4(h4{g[4], g[5], g[6], g[7]}, h4{u[4], u[5], u[6], u[7]});
+        const h4 lo = swiglu4(h4{g[0], g[1], g[2], g[3]}, h4{u[0], u[1], u[2], u[3]}), hi = swiglu4(h4{g[4], g[5], g[6], g[7]}, h4{u[4], u[5], u[6], u[7]});
+        *reinterpret_cast<h8_by_8*>(y + (size_t)grow * (N / 2) + cols.at(col)) = h8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
       }
       continue;
     }
@@ -296,16 +295,11 @@ __global__ __launch_bounds__(kThreads, MT == 8 ? 1 : 2) void gemm_w4a16_wide_ker
       const size_t at = (size_t)grow * N + cols.at(col);
       h8 o = *reinterpret_cast<const h8*>(cs + row * C_LD + col);
       if (residual) {                               // y = fp16(fp16(product) + residual)
-        const h4 r0 = *reinterpret_cast<const h4*>(residual + at), r1 = *reinterpret_cast<const h4*>(residual + at + 4);
+        const h8 res = *reinterpret_cast<const h8_by_8*>(residual + at);
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          o[k] = (_Float16)((float)o[k] + (float)r0[k]);
-          o[k + 4] = (_Float16)((float)o[k + 4] + (float)r1[k]);
-        }
+        for (int k = 0; k < 8; ++k) o[k] = (_Float16)((float)o[k] + (float)res[k]);
       }
-      // y is 8-byte aligned
-      *reinterpret_cast<h4*>(y + at) = h4{o[0], o[1], o[2], o[3]};
-      *reinterpret_cast<h4*>(y + at + 4) = h4{o[4], o[5], o[6], o[7]};
+      *reinterpret_cast<h8_by_8*>(y + at) = o;
     }
   }
 }

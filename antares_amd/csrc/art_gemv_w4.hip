@@ -305,7 +305,7 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(1, 4))) 
     if (swiglu) {
       const half2_t gt = as_h2(gpair), u = as_h2(upair);
       const float g0f = (float)gt.x, g1f = (float)gt.y;
-      o = half2_t{(_Float16)(g0f / (1.0f + expf(0.0f - g0f)) * (float)u.x), (_Float16)(g1f / (1.0f + expf(0.0f - g1f)) * (float)u.y)};
+      o = half2_t{(_Float16)(art::silu(g0f) * (float)u.x), (_Float16)(art::silu(g1f) * (float)u.y)};
     } else {                  // softmax merge: out = sum_p e^(m_p - M) acc_p / sum_p e^(m_p - M) l_p, rounded once to fp16
       float mm = -INFINITY;
 #pragma unroll

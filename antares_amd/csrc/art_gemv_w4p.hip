@@ -230,7 +230,7 @@ __global__ __launch_bounds__(64 * kMaxWaves) void gemv_w4p_kernel(Args a, Magic 
       }
       if constexpr (EPI == 2) {
         const float gf = (float)(_Float16)s, uf = (float)(_Float16)u;
-        a.y[t * 8 + tid] = (_Float16)(gf / (1.0f + expf(0.0f - gf)) * uf);
+        a.y[t * 8 + tid] = (_Float16)(art::silu(gf) * uf);
       } else {
         const int n = t * kTileCols + tid;
         _Float16 o = (_Float16)s;
@@ -410,7 +410,7 @@ __global__ __launch_bounds__(256) void gemv_w4q_kernel(Args a, Magic magic) {
     const float up = ART_DPP_F(r, 0xB1);
     if (lane < 4 && !odd) {
       const float gf = (float)(_Float16)r, uf = (float)(_Float16)up;
-      a.y[tile * 8 + 2 * wave + (lane >> 1)] = (_Float16)(gf / (1.0f + expf(0.0f - gf)) * uf);
+      a.y[tile * 8 + 2 * wave + (lane >> 1)] = (_Float16)(art::silu(gf) * uf);
     }
   } else if (lane < 4) {
     _Float16 o = (_Float16)r;

@@ -572,6 +572,40 @@ def test_w4a16_gemm_with_swiglu_behind_it(autort, M, K, F):
     assert got.shape == (M, F) and np.allclose(got.float().cpu().numpy(), want, **FP16_TOL)
 
 
+# Every fp16 gate: one weight of a gate column is 1 (infinite gates: 2), one of its up column too.  The gate itself is exact; silu in float32
+# is less than 2^-22 off, the product with up and its rounding 2^-24 and 2^-11, or half of 2^-24 among the subnormal numbers.
+@pytest.mark.parametrize('code', [256 + 1, 512 + 1, 1280 + 1, 1024 + 1, 2048 + 1])
+def test_w4a16_gemm_with_swiglu_over_every_fp16_gate(autort, code):
+    from ctypes import c_void_p
+    from antares_amd.runtime import capi
+    dev = autort.device()
+    g = torch.arange(65536, dtype=torch.int32).to(torch.int16).view(torch.float16)
+    g = torch.cat([g[torch.isfinite(g)], torch.tensor([40000.0, -40000.0, 60000.0, -60000.0], dtype=torch.float16)])
+    F, M = 16, g.numel()
+    x = torch.zeros(M, 128, dtype=torch.float16)
+    x[:, 0], x[:, 1] = g, torch.tensor([1.0, -3.5, 1000.0], dtype=torch.float16).repeat(M // 3 + 1)[:M]
+    q = torch.full((128, 2 * F), 8, dtype=torch.uint8)
+    q[0, :F] = 9
+    q[1, F:] = 9
+    scales = torch.ones(1, 2 * F, dtype=torch.float16)
+    scales[0, 1] = 2.0                    # gate column 1: twice the value, infinite beyond 32752
+    d = [t.to(dev) for t in (x, q[0::2] | (q[1::2] << 4), scales, torch.full((1, F), 0x88, dtype=torch.uint8))]
+    out = torch.empty(M, F, dtype=torch.float16, device=dev)
+    note(f'every gate, code {code}')
+    capi.check(capi.lib().art_gemm_w4a16_swiglu(*(c_void_p(t.data_ptr()) for t in d), c_void_p(out.data_ptr()), M, 128, 2 * F, code,
+                                                c_void_p(torch.cuda.current_stream().cuda_stream)))
+    got = out.cpu()
+    for column, gate in ((0, g), (1, g * 2), (F - 1, g)):
+        exact = gate.double()
+        want = torch.where(exact < -700, -0.0, exact / (1 + torch.exp(-exact.clamp(min=-700)))) * x[:, 1].double()
+        want[exact == -float('inf')] = float('nan')
+        y, fits = got[:, column].double(), want.abs() < 65504
+        assert torch.equal(torch.isnan(y), torch.isnan(want))
+        bound = want[fits].abs() * (2.0 ** -11 + 2.0 ** -21) + 2.0 ** -25
+        assert bool(((y[fits] - want[fits]).abs() <= bound).all())
+        assert torch.equal(y[want.abs() > 65520], torch.sign(want[want.abs() > 65520]) * float('inf'))
+
+
 ROW_VECTOR_CASES = [
     # program, inputs, shapes of the inputs, does the row-vector variant apply to these extents
     ('output0[N, C] = input0[N, C] + input1[C]', ['input0=float32[N:300, C:1024]', 'input1=float32[C:1024]'], [(300, 1024), (1024,)], True),
