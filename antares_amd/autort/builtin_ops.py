@@ -593,6 +593,59 @@ class RopeQkvStoreRows(calls.Operator):
 builtin('rope_qkv_store_rows_f16')(lambda: RopeQkvStoreRows())
 
 
+class RopeAngles(calls.Operator):
+    """``rope_angles_f16(inv_freq[D], angles[T, D/2, 2], extra=[first_pos])``: sine and cosine of the rotary embedding's angles
+    at positions first_pos + t (a host integer, default 0), float32."""
+    name = 'rope_angles_f16'
+
+    def __init__(self):
+        self._bind(('inv_freq', 'angles', 'extra'), ('extra',))
+
+    def _call(self, pending, inv_freq, angles, extra=None):
+        if angles.dim() != 3 or angles.shape[2] != 2 or inv_freq.numel() < angles.shape[1]:
+            raise ValueError(f'{self.name}: shapes do not fit together')
+        if inv_freq.dtype != torch.float16 or angles.dtype != torch.float32:
+            raise TypeError(f'{self.name}: inv_freq must be float16, angles float32')
+        first = Number(int(extra[0]), 3, 'I') if extra else 0
+        _require_cuda(inv_freq, angles)
+        return _run(self, pending, angles, capi.lib().art_rope_angles, inv_freq, angles, angles.shape[0], angles.shape[1], first)
+
+
+builtin('rope_angles_f16')(lambda: RopeAngles())
+
+
+class GemmW4RopeStore(calls.Operator):
+    """``gemm_w4a16_rope_store(x[T,K], qweight[K/2, 3*H*128], scales, qzeros, angles[T,64,2], q_out[T,H,128], key_cache[S,H*128],
+    val_cache[S,H*128], extra=[first_pos], k_splits=0)``: the packed int4 product of the T tokens of a prompt with a q | k | v
+    matrix, and ``rope_qkv_store_rows_f16`` behind it with the angles of ``rope_angles_f16``.  ``k_splits``: the launch
+    parameter that tuning keeps for the product (0: the library's choice)."""
+    name = 'gemm_w4a16_rope_store'
+
+    def __init__(self):
+        self._bind(('x', 'qweight', 'scales', 'qzeros', 'angles', 'q_out', 'key_cache', 'val_cache', 'extra', 'k_splits'), ('extra',))
+
+    def _call(self, pending, x, qweight, scales, qzeros, angles, q_out, key_cache, val_cache, extra=None, k_splits=0):
+        T, K = x.shape
+        N = qweight.shape[1]
+        heads = q_out.shape[1]
+        if qweight.shape[0] * 2 != K or scales.shape != (K // 128, N) or qzeros.shape != (K // 128, N // 2) or q_out.shape != (T, heads, 128):
+            raise ValueError(f'{self.name}: operand shapes do not match T, K and the heads')
+        if N != 3 * heads * 128 or angles.shape != (T, 64, 2) or key_cache.shape[-1] != heads * 128 or val_cache.shape != key_cache.shape:
+            raise ValueError(f'{self.name}: shapes do not fit together')
+        for t in (x, scales, q_out, key_cache, val_cache):
+            if t.dtype != torch.float16:
+                raise TypeError(f'{self.name}: x, scales, q_out and the caches must be float16')
+        if angles.dtype != torch.float32:
+            raise TypeError(f'{self.name}: the angles must be float32')
+        first = Number(int(extra[0]), 10, 'I') if extra else 0
+        _require_cuda(x, qweight, scales, qzeros, angles, q_out, key_cache, val_cache)
+        return _run(self, pending, q_out, capi.lib().art_gemm_w4a16_rope_store, x, qweight, scales, qzeros, angles, q_out, key_cache, val_cache, T, K,
+                    heads, first, key_cache.numel() // (heads * 128), int(k_splits))
+
+
+builtin('gemm_w4a16_rope_store')(lambda: GemmW4RopeStore())
+
+
 class GreedyNext(calls.Operator):
     """``greedy_next_f16(logits[V], prompt[L] or None, token[1], pos[1], embed[V, D], x[D])``: the bookkeeping
     between two decode steps in one launch - pos += 1; token = prompt[pos] while the prompt lasts, else

@@ -33,6 +33,10 @@
 // there, SWIGLU pairs gate and up by lane exchange.  Against sums that meet as [row][column] by one half of the wavefronts and are
 // read back by fours, half of the lanes without work in SWIGLU, on one card: 128 rows over 4096 x 22016 34.9 -> 32.5 us, SWIGLU
 // 39.0 -> 35.3, 50 rows with SWIGLU 26.6 -> 25.2, six splits of 128 rows over 11008 x 4096 26.1 -> 25.5.
+// q | k | v (kRope): a block is a head, its rows are rotated on the way out, with angles that are fetched before the loop.  Against the
+// rotation in a launch of its own behind the product (4096 x 12288, both launches, one card): 16 rows 16.1 -> 15.0 us, 50 rows
+// 21.2 -> 18.9, 128 rows 26.1 -> 22.4; blocks of 256 columns: 300 rows 47.4 -> 44.1, 1003 rows 104.7 -> 99.3 (the product alone
+// 96.0).  A rotation of the sums in registers, its code unrolled, lost more in the wide blocks than the launch costs.
 #include "art_w4_mfma.h"
 
 #include <type_traits>
@@ -57,11 +61,12 @@ struct Work {
   int groups, longer;                               // groups of a K split; the first `longer` have one more
 };
 
-template <int MT, bool SWIGLU>
+template <int MT, Tail TAIL>
 __global__ __launch_bounds__(kThreads, MT == 4 ? 2 : 4) void gemm_w4a16_kernel(
     const _Float16* __restrict__ x, const unsigned char* __restrict__ qweight, const _Float16* __restrict__ scales,
     const unsigned char* __restrict__ qzeros, _Float16* y, float* __restrict__ partial, int M, int K, int N, Work work, Magic mg,
-    const _Float16* residual) {                     // residual may be y itself
+    const _Float16* residual, Rope rope) {          // residual may be y itself
+  constexpr bool SWIGLU = TAIL == kSwiglu, ROPE = TAIL == kRope;
   constexpr int STAGE = stage_bytes(MT), BM = 32 * MT;
   constexpr int L = 2 + MT;                         // LDS-direct loads per wavefront and group: weights, scales, MT x
   extern __shared__ __align__(1024) unsigned char smem[];
@@ -75,7 +80,7 @@ __global__ __launch_bounds__(kThreads, MT == 4 ? 2 : 4) void gemm_w4a16_kernel(
   const int m0 = (int)(blockIdx.x >> 3) * BM;
   if (unit >= work.units) return;
   const int split = work.inv_tiles ? (int)__umulhi(unit, work.inv_tiles) : unit;      // unit / col_tiles
-  const TileColumns<SWIGLU, BN> cols{(unit - split * work.col_tiles) * (SWIGLU ? BN / 2 : BN), N};
+  const TileColumns<TAIL, BN> cols{(unit - split * work.col_tiles) * (SWIGLU ? BN / 2 : BN), N};
   const int g_begin = split * work.groups + (split < work.longer ? split : work.longer), groups = work.groups + (split < work.longer ? 1 : 0);
   const unsigned int lds0 = (unsigned int)(size_t)(__attribute__((address_space(3))) unsigned char*)smem;
 
@@ -111,6 +116,18 @@ __global__ __launch_bounds__(kThreads, MT == 4 ? 2 : 4) void gemm_w4a16_kernel(
     if (fetched + 1 < groups) { wbase += (size_t)(GK / 2) * N; qbase += qstep; }
   };
   auto next_x = [&](int fetched) { if (fetched + 1 < groups) xbase += GK * 2; };
+
+  // ROPE: the block is one head.  The angles that this thread needs at the end are fetched first.
+  const int head = cols.n0 / BN;
+  const bool rotated = ROPE && work.splits == 1 && rope.rotated(head);
+  constexpr int PIECES = ROPE ? (BM * 8 + kThreads - 1) / kThreads : 1;
+  Angles<8> angles[PIECES];
+  if (rotated)
+#pragma unroll
+    for (int i = 0; i < PIECES; ++i) {
+      const int row = m0 + ((tid + i * kThreads) >> 3);
+      angles[i] = load_angles<8>(rope.angles + (size_t)(row < M ? row : M - 1) * 64 + (tid & 7) * 8);
+    }
 
   // ---- operand roles.  A transposing read takes 8 byte-rows x 16 columns per 16 lanes: lane s16 supplies the
   // 8-byte piece (row s16 / 2, half s16 % 2) and receives the 8 bytes of column s16.  Lanes 16-31 take the chunk four
@@ -240,6 +257,7 @@ __global__ __launch_bounds__(kThreads, MT == 4 ? 2 : 4) void gemm_w4a16_kernel(
   f32x4* const meet = reinterpret_cast<f32x4*>(smem) + cw * KEEP * 64 + lane;
   auto quad = [&](int q) { return f32x4{acc[q >> 2][4 * (q & 3)], acc[q >> 2][4 * (q & 3) + 1], acc[q >> 2][4 * (q & 3) + 2], acc[q >> 2][4 * (q & 3) + 3]}; };
   f32x4 sum[KEEP];
+  auto row_of = [&](int j) { return ((kh * KEEP + j) >> 2) * 32 + ((kh * KEEP + j) & 3) * 8 + h * 4; };
   __syncthreads();
   if (kh == 0) {
 #pragma unroll
@@ -251,7 +269,6 @@ __global__ __launch_bounds__(kThreads, MT == 4 ? 2 : 4) void gemm_w4a16_kernel(
   __syncthreads();
 #pragma unroll
   for (int j = 0; j < KEEP; ++j) sum[j] += meet[(4 * KEEP * kh + j) * 64];
-  auto row_of = [&](int j) { return ((kh * KEEP + j) >> 2) * 32 + ((kh * KEEP + j) & 3) * 8 + h * 4; };
   if (work.splits > 1) {                            // 64 bytes and more of a row at a time
     if (!cols.inside(colpos)) return;
     float* const to = partial + ((size_t)split * M + m0) * N + cols.at(colpos);
@@ -262,15 +279,14 @@ __global__ __launch_bounds__(kThreads, MT == 4 ? 2 : 4) void gemm_w4a16_kernel(
         if (m0 + row_of(j) + i < M) to[(size_t)(row_of(j) + i) * N] = sum[j][i];
     return;
   }
-  // fp16 results to LDS as [row][column], out in pieces of eight columns.  SWIGLU: lanes 0-15 hold a gate column, lanes 16-31 its up
-  // column; exchanged, the lower ones have both of one row and the upper ones both of the next.
+  // fp16 results to LDS as [row][column], out in pieces of eight columns.
   constexpr int COLS = SWIGLU ? BN / 2 : BN, C_LD = COLS + 8;
   _Float16* const cs = reinterpret_cast<_Float16*>(smem + 8 * KEEP * 1024);
 #pragma unroll
   for (int j = 0; j < KEEP; ++j) {
-    if constexpr (SWIGLU) {
+    if constexpr (SWIGLU) {                         // lanes 0-15 hold a gate column, lanes 16-31 its up column
 #pragma unroll
-      for (int i = 0; i < 4; i += 2) {
+      for (int i = 0; i < 4; i += 2) {              // exchanged: the former have both of one row, the latter both of the next
         const float here = sum[j][i], next = sum[j][i + 1];      // (a bit cast of an element of a vector takes its first one)
         const auto pair = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned int, here), __builtin_bit_cast(unsigned int, next), false, false);
         const float g = (float)(_Float16)__builtin_bit_cast(float, (unsigned int)pair[0]), u = (float)(_Float16)__builtin_bit_cast(float, (unsigned int)pair[1]);
@@ -282,13 +298,27 @@ __global__ __launch_bounds__(kThreads, MT == 4 ? 2 : 4) void gemm_w4a16_kernel(
     }
   }
   __syncthreads();
+  if constexpr (ROPE) {
+    _Float16* const to = rope.at(head);
+#pragma unroll
+    for (int i = 0; i < PIECES; ++i) {
+      const int row = (tid + i * kThreads) >> 3, c8 = (tid & 7) * 8;
+      if (row >= BM || m0 + row >= M) break;
+      h8 a = *reinterpret_cast<const h8*>(cs + row * C_LD + c8), b = *reinterpret_cast<const h8*>(cs + row * C_LD + c8 + 64);
+      if (rotated) rotate(a, b, angles[i]);
+      _Float16* const out = to + (size_t)(m0 + row) * (rope.heads * 128) + c8;
+      *reinterpret_cast<h8*>(out) = a;
+      *reinterpret_cast<h8*>(out + 64) = b;
+    }
+    return;
+  }
 #pragma unroll 1
   for (int e = tid; e < BM * (COLS / 8); e += kThreads) {
     const int row = e / (COLS / 8), c8 = (e % (COLS / 8)) * 8;
     if (m0 + row >= M || !cols.inside(c8)) continue;
     const size_t out = (size_t)(m0 + row) * (SWIGLU ? N / 2 : N) + cols.at(c8);
     h8 o = *reinterpret_cast<const h8*>(cs + row * C_LD + c8);
-    if (!SWIGLU && residual) {                      // y = fp16(fp16(product) + residual); may alias y: same elements
+    if (TAIL == kPlain && residual) {                      // y = fp16(fp16(product) + residual); may alias y: same elements
       const h8 res = *reinterpret_cast<const h8_by_8*>(residual + out);
 #pragma unroll
       for (int k = 0; k < 8; ++k) o[k] = (_Float16)((float)o[k] + (float)res[k]);
@@ -391,6 +421,23 @@ __global__ __launch_bounds__(256) void gemm_w4a16_combine_swiglu_kernel(const fl
                                                             h4{(_Float16)u[0], (_Float16)u[1], (_Float16)u[2], (_Float16)u[3]});
 }
 
+// The same for q | k | v: columns j .. j + 3 of a head and their partners 64 further on, rotated in q and k.
+__global__ __launch_bounds__(256) void gemm_w4a16_combine_rope_kernel(const float* __restrict__ partial, int rows, int splits, Rope rope) {
+  const int pieces = rope.heads * 48;               // of a row
+  const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
+  if (i >= (long long)rows * pieces) return;
+  const long long row = i / pieces, stride = (long long)rows * pieces * 8;
+  const int at = (int)(i - row * pieces), head = at >> 4, j = (at & 15) * 4;
+  const float* const from = partial + (row * pieces * 8 + head * 128 + j);
+  const f32x4 first = sum_splits(from, stride, splits), second = sum_splits(from + 64, stride, splits);
+  h4 a = h4{(_Float16)first[0], (_Float16)first[1], (_Float16)first[2], (_Float16)first[3]};
+  h4 b = h4{(_Float16)second[0], (_Float16)second[1], (_Float16)second[2], (_Float16)second[3]};
+  if (rope.rotated(head)) rotate(a, b, load_angles<4>(rope.angles + row * 64 + j));
+  _Float16* const to = rope.at(head) + row * rope.heads * 128 + j;
+  *reinterpret_cast<h4*>(to) = a;
+  *reinterpret_cast<h4*>(to + 64) = b;
+}
+
 // ---- Which kernel, rows per block and K-splits.
 struct Plan {
   bool wide;
@@ -449,8 +496,8 @@ struct Norm {
   float eps;
 };
 
-int combine(const float* partial, _Float16* y, int rows, int N, int splits, const _Float16* residual, bool swiglu, const Norm* norm,
-            hipStream_t stream) {
+int combine(const float* partial, _Float16* y, int rows, int N, int splits, const _Float16* residual, Tail tail, const Norm* norm,
+            const Rope& rope, hipStream_t stream) {
   if (norm) {
     const int threads = N < 8 * kNormThreads ? (N / 8 + 63) / 64 * 64 : kNormThreads;
     gemm_w4a16_combine_norm_kernel<<<dim3(rows), threads, 0, stream>>>(partial, y, N, (long long)rows * N, splits, residual,
@@ -458,7 +505,12 @@ int combine(const float* partial, _Float16* y, int rows, int N, int splits, cons
     ART_LAUNCH_CHECK();
     return 0;
   }
-  if (swiglu) {
+  if (tail == kRope) {
+    gemm_w4a16_combine_rope_kernel<<<dim3((unsigned)(((long long)rows * (N / 8) + 255) / 256)), 256, 0, stream>>>(partial, rows, splits, rope);
+    ART_LAUNCH_CHECK();
+    return 0;
+  }
+  if (tail == kSwiglu) {
     gemm_w4a16_combine_swiglu_kernel<<<dim3((unsigned)(((long long)rows * (N / 8) + 255) / 256)), 256, 0, stream>>>(partial, y, rows, N, splits);
     ART_LAUNCH_CHECK();
     return 0;
@@ -472,7 +524,8 @@ int combine(const float* partial, _Float16* y, int rows, int N, int splits, cons
 // One launch of the product (and of the pass behind it) over up to kMaxRows rows.
 constexpr int kMaxRows = 1 << 18;                   // 8192 blocks of 32 rows
 int run_rows(const _Float16* xs, const unsigned char* qweight, const _Float16* scales, const unsigned char* qzeros, _Float16* ys, const _Float16* res,
-             int M, int K, int N, int code, int splits, bool swiglu, const Norm* norm, float* scratch, size_t scratch_bytes, hipStream_t st) {
+             int M, int K, int N, int code, int splits, Tail tail, const Norm* norm, const Rope& rope, float* scratch, size_t scratch_bytes, hipStream_t st) {
+  const bool swiglu = tail == kSwiglu;
   Plan p;
   ART_REQUIRE(choose(p, M, K, N, swiglu, scratch_bytes, art::compute_units(), code, splits), "art_gemm_w4a16: K=%d N=%d are too large", K, N);
   // Where K-splits meet in a pass of their own, the norm is part of that pass, up to 256 rows: beyond them
@@ -480,35 +533,34 @@ int run_rows(const _Float16* xs, const unsigned char* qweight, const _Float16* s
   const bool norm_there = norm && p.splits > 1 && M <= 256 && N % 8 == 0 && N <= 8 * kNormThreads * kNormTurns &&
                           (((uintptr_t)ys | (uintptr_t)res | (uintptr_t)norm->weight | (uintptr_t)norm->out) % 16) == 0;
   if (p.wide) {
-    if (art::w4::gemm_wide(xs, qweight, scales, qzeros, ys, scratch, M, K, N, p.splits, p.row_tiles, res, swiglu, st)) return 1;
+    if (art::w4::gemm_wide(xs, qweight, scales, qzeros, ys, scratch, M, K, N, p.splits, p.row_tiles, res, tail, rope, st)) return 1;
   } else {
+    static const decltype(&gemm_w4a16_kernel<1, kPlain>) kernels[3][3] = {
+        {gemm_w4a16_kernel<1, kPlain>, gemm_w4a16_kernel<1, kSwiglu>, gemm_w4a16_kernel<1, kRope>},
+        {gemm_w4a16_kernel<2, kPlain>, gemm_w4a16_kernel<2, kSwiglu>, gemm_w4a16_kernel<2, kRope>},
+        {gemm_w4a16_kernel<4, kPlain>, gemm_w4a16_kernel<4, kSwiglu>, gemm_w4a16_kernel<4, kRope>}};
     static bool configured = false;
     if (!configured) {
-      const void* kernels[3][2] = {{(const void*)gemm_w4a16_kernel<1, false>, (const void*)gemm_w4a16_kernel<1, true>},
-                                   {(const void*)gemm_w4a16_kernel<2, false>, (const void*)gemm_w4a16_kernel<2, true>},
-                                   {(const void*)gemm_w4a16_kernel<4, false>, (const void*)gemm_w4a16_kernel<4, true>}};
       for (int i = 0; i < 3; ++i)
-        for (int j = 0; j < 2; ++j)
-          ART_HIP(hipFuncSetAttribute(kernels[i][j], hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes(1 << i)));
+        for (int j = 0; j < 3; ++j)
+          ART_HIP(hipFuncSetAttribute((const void*)kernels[i][j], hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes(1 << i)));
       configured = true;
     }
     const int col_tiles = tile_count(N, swiglu, BN), m_blocks = (M + 32 * p.row_tiles - 1) / (32 * p.row_tiles);
     const int units = col_tiles * p.splits, G = K / GK;
     const Work work{units, col_tiles, p.splits, (unsigned int)((0x100000000ull + col_tiles - 1) / col_tiles), G / p.splits, G % p.splits};
     const dim3 grid(8 * m_blocks, (units + 7) / 8);
-    const auto kernel = p.row_tiles == 1   ? (swiglu ? gemm_w4a16_kernel<1, true> : gemm_w4a16_kernel<1, false>)
-                        : p.row_tiles == 2 ? (swiglu ? gemm_w4a16_kernel<2, true> : gemm_w4a16_kernel<2, false>)
-                                           : (swiglu ? gemm_w4a16_kernel<4, true> : gemm_w4a16_kernel<4, false>);
-    kernel<<<grid, kThreads, lds_bytes(p.row_tiles), st>>>(xs, qweight, scales, qzeros, ys, scratch, M, K, N, work, kMagic, res);
+    const auto kernel = kernels[p.row_tiles == 4 ? 2 : p.row_tiles - 1][tail];
+    kernel<<<grid, kThreads, lds_bytes(p.row_tiles), st>>>(xs, qweight, scales, qzeros, ys, scratch, M, K, N, work, kMagic, res, rope);
     ART_LAUNCH_CHECK();
   }
-  if (p.splits > 1 && combine(scratch, ys, M, N, p.splits, res, swiglu, norm_there ? norm : nullptr, st)) return 1;
+  if (p.splits > 1 && combine(scratch, ys, M, N, p.splits, res, tail, norm_there ? norm : nullptr, rope, st)) return 1;
   return norm && !norm_there ? art_rmsnorm(ys, nullptr, norm->weight, norm->out, M, N, 1.0f / (float)N, norm->eps, 1, 1, 1, st) : 0;
 }
 
 int run(const void* x_dev, const void* qweight_dev, const void* scales_dev, const void* qzeros_dev, void* y_dev, const void* residual_dev,
-        int M, int K, int N, int k_splits, bool swiglu, const Norm* norm, void* stream) {
-  const int n_out = swiglu ? N / 2 : N;
+        int M, int K, int N, int k_splits, Tail tail, const Norm* norm, const Rope* rope, void* stream) {
+  const int n_out = tail == kSwiglu ? N / 2 : tail == kRope ? N / 3 : N;
   const int code = k_splits >> 8;                   // 0: library's choice; else rows of a block / 32, 5: 128 rows x 128 columns
   ART_REQUIRE(k_splits >= 0 && (code <= 2 || code == 4 || code == 5 || code == 8),
               "art_gemm_w4a16: k_splits must be 0 (library's choice) or 1..255, plus 256 x the rows-per-block code 1, 2, 4, 5 or 8 (got %d)", k_splits);
@@ -527,9 +579,11 @@ int run(const void* x_dev, const void* qweight_dev, const void* scales_dev, cons
   for (int m0 = 0; m0 < M; m0 += kMaxRows) {
     const size_t out = (size_t)m0 * n_out;
     const Norm rows_norm = norm ? Norm{norm->weight, (_Float16*)norm->out + out, norm->eps} : Norm{};
+    const size_t d = (size_t)N / 3 * m0;
+    const Rope rows_rope = rope ? Rope{rope->angles + 64 * (size_t)m0, rope->q + d, rope->k + d, rope->v + d, rope->heads} : Rope{};
     if (run_rows((const _Float16*)x_dev + (size_t)m0 * K, (const unsigned char*)qweight_dev, (const _Float16*)scales_dev, (const unsigned char*)qzeros_dev,
                  (_Float16*)y_dev + out, residual_dev ? (const _Float16*)residual_dev + out : nullptr, M - m0 < kMaxRows ? M - m0 : kMaxRows, K, N, code,
-                 k_splits & 0xff, swiglu, norm ? &rows_norm : nullptr, scratch, scratch_bytes, (hipStream_t)stream))
+                 k_splits & 0xff, tail, norm ? &rows_norm : nullptr, rows_rope, scratch, scratch_bytes, (hipStream_t)stream))
       return 1;
     if (M - m0 <= kMaxRows) break;                  // m0 does not pass the largest int
   }
@@ -550,13 +604,13 @@ extern "C" int art_gemm_w4a16_tuned(const void* x_dev, const void* qweight_dev, 
 
 extern "C" int art_gemm_w4a16_residual(const void* x_dev, const void* qweight_dev, const void* scales_dev, const void* qzeros_dev,
                                        void* y_dev, const void* residual_dev, int M, int K, int N, int k_splits, void* stream) {
-  return run(x_dev, qweight_dev, scales_dev, qzeros_dev, y_dev, residual_dev, M, K, N, k_splits, false, nullptr, stream);
+  return run(x_dev, qweight_dev, scales_dev, qzeros_dev, y_dev, residual_dev, M, K, N, k_splits, kPlain, nullptr, nullptr, stream);
 }
 
 extern "C" int art_gemm_w4a16_swiglu(const void* x_dev, const void* qweight_dev, const void* scales_dev, const void* qzeros_dev,
                                      void* y_dev, int M, int K, int N, int k_splits, void* stream) {
   ART_REQUIRE(N % 32 == 0, "art_gemm_w4a16_swiglu: the gate and up halves must be multiples of 16 columns (N=%d)", N);
-  return run(x_dev, qweight_dev, scales_dev, qzeros_dev, y_dev, nullptr, M, K, N, k_splits, true, nullptr, stream);
+  return run(x_dev, qweight_dev, scales_dev, qzeros_dev, y_dev, nullptr, M, K, N, k_splits, kSwiglu, nullptr, nullptr, stream);
 }
 
 extern "C" int art_gemm_w4a16_residual_norm(const void* x_dev, const void* qweight_dev, const void* scales_dev, const void* qzeros_dev,
@@ -570,5 +624,24 @@ extern "C" int art_gemm_w4a16_residual_norm(const void* x_dev, const void* qweig
                   !art::overlaps(norm_out_dev, (size_t)M * N * 2, x_dev, (size_t)M * K * 2),
               "art_gemm_w4a16_residual_norm: the normalised result must not overlap an operand or the result");
   const Norm norm{norm_weight_dev, norm_out_dev, eps};
-  return run(x_dev, qweight_dev, scales_dev, qzeros_dev, y_dev, residual_dev, M, K, N, k_splits, false, &norm, stream);
+  return run(x_dev, qweight_dev, scales_dev, qzeros_dev, y_dev, residual_dev, M, K, N, k_splits, kPlain, &norm, nullptr, stream);
+}
+
+extern "C" int art_gemm_w4a16_rope_store(const void* x_dev, const void* qweight_dev, const void* scales_dev, const void* qzeros_dev,
+                                         const void* angles_dev, void* q_out_dev, void* key_cache_dev, void* val_cache_dev, int M, int K, int heads,
+                                         int first_pos, int max_positions, int k_splits, void* stream) {
+  ART_REQUIRE(angles_dev && q_out_dev && key_cache_dev && val_cache_dev, "art_gemm_w4a16_rope_store: null pointer");
+  ART_REQUIRE(heads >= 1 && heads < 1 << 22, "art_gemm_w4a16_rope_store: bad shape");
+  ART_REQUIRE(M >= 1 && first_pos >= 0 && max_positions >= M && first_pos <= max_positions - M,
+              "art_gemm_w4a16_rope_store: positions %d.. of %d rows do not fit caches of %d", first_pos, M, max_positions);
+  ART_REQUIRE((((uintptr_t)q_out_dev | (uintptr_t)key_cache_dev | (uintptr_t)val_cache_dev | (uintptr_t)angles_dev) % 16) == 0,
+              "art_gemm_w4a16_rope_store: the angles, q and the caches must be 16-byte aligned");
+  const size_t row = (size_t)heads * 128, rows = (size_t)M * row * 2, first = (size_t)first_pos * row;
+  const Rope rope{(const float2*)angles_dev, (_Float16*)q_out_dev, (_Float16*)key_cache_dev + first, (_Float16*)val_cache_dev + first, heads};
+  const void* outs[3] = {rope.q, rope.k, rope.v};
+  for (int i = 0; i < 3; ++i)
+    ART_REQUIRE(!art::overlaps(x_dev, (size_t)M * K * 2, outs[i], rows) && !art::overlaps(angles_dev, (size_t)M * 512, outs[i], rows) &&
+                    !art::overlaps(outs[i], rows, outs[(i + 1) % 3], rows),
+                "art_gemm_w4a16_rope_store: q, keys and values must not overlap an operand or each other");
+  return run(x_dev, qweight_dev, scales_dev, qzeros_dev, q_out_dev, nullptr, M, K, 3 * heads * 128, k_splits, kRope, nullptr, &rope, stream);
 }

@@ -41,13 +41,14 @@ constexpr int stage_bytes(int MT) { return W_BYTES + Q_BYTES + MT * 32 * SK * 2;
 constexpr size_t lds_bytes(int MT) { return (size_t)NS * stage_bytes(MT); }
 static_assert(128 * C_LD * 2 <= NS * stage_bytes(4), "128 staged output rows fit the ring");
 
-// SWIGLU: the matrix is gate | up (N / 2 columns each); a block owns 128 gate columns and the matching 128 up columns and
+// kSwiglu: the matrix is gate | up (N / 2 columns each); a block owns 128 gate columns and the matching 128 up columns and
 // stores y[m, n] = fp16(silu(fp16(gate)) * fp16(up)), N / 2 columns.
-template <int MT, bool SWIGLU>
+template <int MT, Tail TAIL>
 __global__ __launch_bounds__(kThreads, MT == 8 ? 1 : 2) void gemm_w4a16_wide_kernel(
     const _Float16* __restrict__ x, const unsigned char* __restrict__ qweight, const _Float16* __restrict__ scales,
     const unsigned char* __restrict__ qzeros, _Float16* y, float* __restrict__ partial, int M, int K, int N, int splits,
-    int col_tiles, int m_blocks, Magic mg, const _Float16* residual) {       // residual may be y itself
+    int col_tiles, int m_blocks, Magic mg, const _Float16* residual, Rope rope) {       // residual may be y itself
+  constexpr bool SWIGLU = TAIL == kSwiglu;
   constexpr int STAGE = stage_bytes(MT), BM = 32 * MT;
   constexpr int L = 2 + MT + 1;                     // loads per wavefront and stage
   extern __shared__ __align__(1024) unsigned char smem[];
@@ -57,7 +58,7 @@ __global__ __launch_bounds__(kThreads, MT == 8 ? 1 : 2) void gemm_w4a16_wide_ker
   const int m_block = (int)(blockIdx.x % (8 * m_blocks)) / 8;
   if (unit >= col_tiles * splits) return;
   const int split = unit / col_tiles;
-  const TileColumns<SWIGLU, BN> cols{(unit % col_tiles) * (SWIGLU ? BN / 2 : BN), N};
+  const TileColumns<TAIL, BN> cols{(unit % col_tiles) * (SWIGLU ? BN / 2 : BN), N};
   const int m0 = m_block * BM;
   const int G = K / 128;
   const int g_begin = (int)((long long)G * split / splits), g_end = (int)((long long)G * (split + 1) / splits);
@@ -266,6 +267,14 @@ __global__ __launch_bounds__(kThreads, MT == 8 ? 1 : 2) void gemm_w4a16_wide_ker
     return;
   }
   _Float16* cs = reinterpret_cast<_Float16*>(smem);
+  // kRope: a block is two heads, whose angles are the same; a thread has columns 8 (tid % 8) .. + 7 and their partners of both in every
+  // 32nd row.  The angles of its next row are on their way while it rotates one.
+  const int head = cols.n0 >> 7;
+  const bool rotated[2] = {TAIL == kRope && rope.rotated(head), TAIL == kRope && rope.rotated(head + 1)};
+  _Float16* const to[2] = {TAIL == kRope ? rope.at(head) : nullptr, TAIL == kRope ? rope.at(head + 1) : nullptr};
+  Angles<8> angles;
+  auto fetch_angles = [&](int row) { angles = load_angles<8>(rope.angles + (size_t)(row < M ? row : M - 1) * 64 + (tid & 7) * 8); };
+  if (rotated[0]) fetch_angles(m0 + (tid >> 3));
 #pragma unroll
   for (int p = 0; p < MT / 4; ++p) {                // 128 rows at a time through LDS, out as 16-byte stores
     __syncthreads();
@@ -277,6 +286,25 @@ __global__ __launch_bounds__(kThreads, MT == 8 ? 1 : 2) void gemm_w4a16_wide_ker
         for (int r = 0; r < 16; ++r)
           cs[(t * 32 + (r >> 2) * 8 + h * 4 + (r & 3)) * C_LD + colpos[ct]] = (_Float16)acc[4 * p + t][ct][r];
     __syncthreads();
+    if constexpr (TAIL == kRope) {
+#pragma unroll 1
+      for (int row = tid >> 3; row < 128; row += kThreads / 8) {
+        const int grow = m0 + p * 128 + row, col = (tid & 7) * 8;
+        const Angles<8> now = angles;
+        if (rotated[0]) fetch_angles(grow + kThreads / 8);
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+          h8 a = *reinterpret_cast<const h8*>(cs + row * C_LD + k * 128 + col), b = *reinterpret_cast<const h8*>(cs + row * C_LD + k * 128 + col + 64);
+          if (rotated[k]) rotate(a, b, now);
+          _Float16* const out = to[k] + (size_t)grow * (rope.heads * 128) + col;
+          if (grow < M && (k == 0 || cols.inside(128))) {
+            *reinterpret_cast<h8*>(out) = a;
+            *reinterpret_cast<h8*>(out + 64) = b;
+          }
+        }
+      }
+      continue;
+    }
     if constexpr (SWIGLU) {
 #pragma unroll 1
       for (int c = tid; c < 128 * (BN / 16); c += kThreads) {
@@ -304,18 +332,18 @@ __global__ __launch_bounds__(kThreads, MT == 8 ? 1 : 2) void gemm_w4a16_wide_ker
   }
 }
 
-template <int MT, bool SWIGLU>
+template <int MT, Tail TAIL>
 int launch(const _Float16* x, const unsigned char* qweight, const _Float16* scales, const unsigned char* qzeros, _Float16* y,
-           float* partial, int M, int K, int N, int splits, const _Float16* residual, hipStream_t stream) {
+           float* partial, int M, int K, int N, int splits, const _Float16* residual, const Rope& rope, hipStream_t stream) {
   static bool configured = false;
   if (!configured) {
-    ART_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_w4a16_wide_kernel<MT, SWIGLU>), hipFuncAttributeMaxDynamicSharedMemorySize,
+    ART_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_w4a16_wide_kernel<MT, TAIL>), hipFuncAttributeMaxDynamicSharedMemorySize,
                                 (int)lds_bytes(MT)));
     configured = true;
   }
-  const int col_tiles = tile_count(N, SWIGLU, BN), m_blocks = (M + 32 * MT - 1) / (32 * MT);
-  gemm_w4a16_wide_kernel<MT, SWIGLU><<<dim3((unsigned)((col_tiles * splits + 7) / 8 * 8 * m_blocks)), kThreads, lds_bytes(MT), stream>>>(
-      x, qweight, scales, qzeros, y, partial, M, K, N, splits, col_tiles, m_blocks, kMagic, residual);
+  const int col_tiles = tile_count(N, TAIL == kSwiglu, BN), m_blocks = (M + 32 * MT - 1) / (32 * MT);
+  gemm_w4a16_wide_kernel<MT, TAIL><<<dim3((unsigned)((col_tiles * splits + 7) / 8 * 8 * m_blocks)), kThreads, lds_bytes(MT), stream>>>(
+      x, qweight, scales, qzeros, y, partial, M, K, N, splits, col_tiles, m_blocks, kMagic, residual, rope);
   ART_LAUNCH_CHECK();
   return 0;
 }
@@ -323,10 +351,9 @@ int launch(const _Float16* x, const unsigned char* qweight, const _Float16* scal
 }  // namespace
 
 int art::w4::gemm_wide(const _Float16* x, const unsigned char* qweight, const _Float16* scales, const unsigned char* qzeros, _Float16* y,
-                       float* partial, int M, int K, int N, int splits, int row_tiles, const _Float16* residual, bool swiglu, hipStream_t stream) {
-  if (swiglu)
-    return row_tiles == 8 ? launch<8, true>(x, qweight, scales, qzeros, y, partial, M, K, N, splits, nullptr, stream)
-                          : launch<4, true>(x, qweight, scales, qzeros, y, partial, M, K, N, splits, nullptr, stream);
-  return row_tiles == 8 ? launch<8, false>(x, qweight, scales, qzeros, y, partial, M, K, N, splits, residual, stream)
-                        : launch<4, false>(x, qweight, scales, qzeros, y, partial, M, K, N, splits, residual, stream);
+                       float* partial, int M, int K, int N, int splits, int row_tiles, const _Float16* residual, Tail tail, const Rope& rope,
+                       hipStream_t stream) {
+  static const decltype(&launch<4, kPlain>) by_rows[2][3] = {{launch<4, kPlain>, launch<4, kSwiglu>, launch<4, kRope>},
+                                                             {launch<8, kPlain>, launch<8, kSwiglu>, launch<8, kRope>}};
+  return by_rows[row_tiles == 8][tail](x, qweight, scales, qzeros, y, partial, M, K, N, splits, residual, rope, stream);
 }

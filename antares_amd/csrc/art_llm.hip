@@ -505,6 +505,16 @@ __global__ __launch_bounds__(256) void rope_qkv_store_rows_kernel(const _Float16
     store8(dst + at + half, rb);
   }
 }
+// Sine and cosine of the angles of rows first_pos .. of a rotary embedding, as art_gemm_w4a16_rope_store reads them.
+__global__ __launch_bounds__(256) void rope_angles_kernel(const _Float16* __restrict__ freq, float2* __restrict__ angles, int rows, int half,
+                                                           int first_pos) {
+  const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
+  if (i >= (long long)rows * half) return;
+  const int t = (int)(i / half);
+  float2 a;
+  sincosf((float)(first_pos + t) * (float)freq[i - (long long)t * half], &a.x, &a.y);
+  angles[i] = a;
+}
 // Any other shape: one pair per lane, grid.y = token.
 __global__ __launch_bounds__(256) void rope_qkv_store_rows_any_kernel(const _Float16* __restrict__ qkv, const _Float16* __restrict__ freq,
                                                                    _Float16* __restrict__ q_out, _Float16* __restrict__ key_cache,
@@ -622,6 +632,17 @@ extern "C" int art_rope_qkv_store(const void* qkv_dev, const void* freq_dev, voi
   if (dtype == 0) { if (freq_dtype == 0) ART_RQS(float, float); else ART_RQS(float, _Float16); }
   else { if (freq_dtype == 0) ART_RQS(_Float16, float); else ART_RQS(_Float16, _Float16); }
 #undef ART_RQS
+  ART_LAUNCH_CHECK();
+  return 0;
+}
+
+extern "C" int art_rope_angles(const void* freq_dev, void* angles_dev, int rows, int half, int first_pos, void* stream) {
+  ART_REQUIRE(freq_dev && angles_dev, "art_rope_angles: null pointer");
+  ART_REQUIRE(rows >= 1 && half >= 1 && first_pos >= 0 && first_pos <= 0x7fffffff - rows, "art_rope_angles: bad arguments");
+  ART_REQUIRE((uintptr_t)freq_dev % 2 == 0 && (uintptr_t)angles_dev % 8 == 0, "art_rope_angles: misaligned tensor");
+  const long long blocks = ((long long)rows * half + 255) / 256;
+  ART_REQUIRE(blocks <= 0x7fffffffLL, "art_rope_angles: too many angles");
+  rope_angles_kernel<<<dim3((unsigned)blocks), 256, 0, (hipStream_t)stream>>>((const _Float16*)freq_dev, (float2*)angles_dev, rows, half, first_pos);
   ART_LAUNCH_CHECK();
   return 0;
 }

@@ -32,16 +32,52 @@ __device__ __forceinline__ unsigned int and_or(unsigned int w, unsigned int mask
 
 constexpr Magic kMagic{0x000F000Fu, 0x00F000F0u, 0x64006400u, 0x54005400u};
 
-// The BN columns of a block: neighbours, or (SWIGLU, the matrix is gate | up) BN / 2 of the gate half and the matching ones of
-// the up half.  N % 16 == 0 (SWIGLU: N % 32), so a piece of 16 columns is inside or outside as a whole.
-template <bool SWIGLU, int BN>
+// What becomes of the product: stored (a residual added), SwiGLU of its gate | up halves, or, of q | k | v with heads of
+// 128 columns, q and k rotated and all three stored where the attention reads them.
+enum Tail { kPlain, kSwiglu, kRope };
+
+// The BN columns of a block: neighbours, or (kSwiglu) BN / 2 of the gate half and the matching ones of the up half.
+// N % 16 == 0 (kSwiglu: N % 32), so a piece of 16 columns is inside or outside as a whole.
+template <Tail TAIL, int BN>
 struct TileColumns {
   int n0, N;
+  static constexpr bool SWIGLU = TAIL == kSwiglu;
   __device__ __forceinline__ int at(int pos) const { return SWIGLU && pos >= BN / 2 ? N / 2 + n0 + pos - BN / 2 : n0 + pos; }
   __device__ __forceinline__ bool inside(int pos) const { return SWIGLU ? n0 + (pos & (BN / 2 - 1)) < N / 2 : n0 + pos < N; }
   __device__ __forceinline__ int safe(int pos) const { return inside(pos) ? at(pos) : 0; }
 };
 inline int tile_count(int N, bool swiglu, int bn) { return swiglu ? (N / 2 + bn / 2 - 1) / (bn / 2) : (N + bn - 1) / bn; }
+
+// kRope: sine and cosine of row m, column j < 64 of a head at angles[64 m + j]; row m of q, k and v holds `heads` heads of 128.
+struct Rope {
+  const float2* angles;
+  _Float16 *q, *k, *v;
+  int heads;
+  // where head h of q | k | v has its first row, and whether it is rotated
+  __device__ __forceinline__ _Float16* at(int h) const {
+    return h < heads ? q + h * 128 : h < 2 * heads ? k + (h - heads) * 128 : v + (h - 2 * heads) * 128;
+  }
+  __device__ __forceinline__ bool rotated(int h) const { return h < 2 * heads; }
+};
+// Neighbouring columns of the first half of a head and their partners 64 further on, with their angles (sine, cosine).
+template <int COUNT> struct Angles {
+  f32x4 of[COUNT / 2];
+};
+template <int COUNT> __device__ __forceinline__ Angles<COUNT> load_angles(const float2* from) {
+  Angles<COUNT> a;
+#pragma unroll
+  for (int k = 0; k < COUNT / 2; ++k) a.of[k] = reinterpret_cast<const f32x4*>(from)[k];
+  return a;
+}
+template <int COUNT, class V> __device__ __forceinline__ void rotate(V& a, V& b, const Angles<COUNT>& angles) {
+#pragma unroll
+  for (int k = 0; k < COUNT; ++k) {
+    const float sine = angles.of[k >> 1][2 * (k & 1)], cosine = angles.of[k >> 1][2 * (k & 1) + 1];
+    const float x = (float)a[k], y = (float)b[k];
+    a[k] = (_Float16)(x * cosine - y * sine);
+    b[k] = (_Float16)(y * cosine + x * sine);
+  }
+}
 
 // fp16(silu(gate) * up) of fp16 operands in fp32.  silu is half as many instructions as expf and a division (every fp16 gate gives
 // the same fp16 value): 1003 rows over 4096 x 22016 with SWIGLU 186.4 -> 184.1 us.
@@ -53,10 +89,9 @@ __device__ __forceinline__ h4 swiglu4(h4 g, h4 u) {
 }
 
 // Large batches (art_gemm_w4_wide.hip): one launch over blocks of 32 row_tiles rows x 256 columns, K cut into `splits`;
-// with splits > 1 the fp32 tiles go to `partial` [splits][M][N].  row_tiles is 4 or 8.  swiglu: y[M, N/2] from
-// gate | up, no residual.
+// with splits > 1 the fp32 tiles go to `partial` [splits][M][N].  row_tiles is 4 or 8.  No residual but with kPlain.
 int gemm_wide(const _Float16* x, const unsigned char* qweight, const _Float16* scales, const unsigned char* qzeros, _Float16* y,
-              float* partial, int M, int K, int N, int splits, int row_tiles, const _Float16* residual, bool swiglu, hipStream_t stream);
+              float* partial, int M, int K, int N, int splits, int row_tiles, const _Float16* residual, Tail tail, const Rope& rope, hipStream_t stream);
 
 }  // namespace w4
 }  // namespace art

@@ -293,11 +293,12 @@ class LlamaInt4Decoder:
 
     def prefill(self, tokens: torch.Tensor, graph: bool = True) -> torch.Tensor:
         """Ingests a whole prompt (int32 [T] on the device, T >= 4, positions 0..T-1) in one pass: the projections
-        run as batched int4 GEMMs on the matrix cores (`gemv_w4a16` with T rows), attention is causal over the
-        prompt (`attention_causal_f16`, matrix cores), keys and values land in cache rows 0..T-1.  Leaves the step
+        run as batched int4 GEMMs on the matrix cores, the q | k | v one with the rotary embedding behind it
+        (`gemm_w4a16_rope_store`), attention is causal over the prompt (`attention_causal_f16`, matrix cores), keys and
+        values land in cache rows 0..T-1.  Leaves the step
         state at the last prompt position (self.pos = T - 1, self.x = its hidden state, self.logits = its logits), so
         `advance()` and the recorded decode step continue from there.  Same operators and roundings as the one-token
-        step, applied to T rows.  With ``graph`` the pass is recorded once per prompt length in a HIP graph (about 360
+        step, applied to T rows.  With ``graph`` the pass is recorded once per prompt length in a HIP graph (about 230
         launches) and replayed on later calls with the new tokens copied into the recorded input."""
         T = int(tokens.numel())
         if not 4 <= T <= self.cfg.max_seq:
@@ -334,23 +335,23 @@ class LlamaInt4Decoder:
         ops = self._prefill_ops(T)
         f16 = dict(dtype=torch.float16, device=self.dev)
         x = ops['embed'](self.w['embed'], tokens.view(T))
-        qkv = torch.empty(T, 3 * d, **f16)
         hid = torch.empty(T, F, **f16)
         qr = torch.empty(T, H, D, **f16)
-
-        def linear(inp, lin, out):
-            self.gemv(inp, lin['qweight'], lin['scales'], lin['qzeros'], out=out)
+        angles = self.autort.ops.rope_angles_f16(self.inv_freq, torch.empty(T, D // 2, 2, dtype=torch.float32, device=self.dev))
 
         def gemm_res(inp, lin, acc, norm_weight):    # acc += inp @ W -> the RMSNorm in front of the next projection
             return self.autort.ops.gemm_w4a16_residual_norm(inp, lin['qweight'], lin['scales'], lin['qzeros'], acc, norm_weight, residual=acc,
                                                             eps=cfg.rms_eps)
 
+        saved = self.gemv.tuned.get(f'gemm_w4a16.k_splits|{T},{d},{3 * d}')       # of a tuning run over this product
+        k_splits = int(saved['value']) if saved is not None else 0
         layers = self.w['layers']
         # the built-in operator takes rows: one launch for the T positions
         xb = self.autort.ops.rmsnorm_f16(x, None, layers[0]['att_norm'], extra=[1.0 / d, cfg.rms_eps])
         for l, lw in enumerate(layers):
-            linear(xb, lw['qkv'], qkv)
-            self.autort.ops.rope_qkv_store_rows_f16(qkv, self.inv_freq, qr, self.key_cache[l], self.val_cache[l])
+            qkv = lw['qkv']
+            self.autort.ops.gemm_w4a16_rope_store(xb, qkv['qweight'], qkv['scales'], qkv['qzeros'], angles, qr, self.key_cache[l], self.val_cache[l],
+                                                   k_splits=k_splits)
             att = self.autort.ops.attention_causal_f16(qr, self.key_cache[l].view(cfg.max_seq, H, D),
                                                        self.val_cache[l].view(cfg.max_seq, H, D), self.att_f)
             xb = gemm_res(att.view(T, d), lw['o'], x, lw['ffn_norm'])

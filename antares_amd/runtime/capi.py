@@ -62,6 +62,8 @@ _SIGNATURES = {
     'art_gemm_w4a16_residual': (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p]),
     'art_gemm_w4a16_residual_norm': (c_int, [c_void_p] * 8 + [c_int, c_int, c_int, c_float, c_int, c_void_p]),
     'art_gemm_w4a16_swiglu': (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p]),
+    'art_gemm_w4a16_rope_store': (c_int, [c_void_p] * 8 + [c_int] * 6 + [c_void_p]),
+    'art_rope_angles': (c_int, [c_void_p, c_void_p, c_int, c_int, c_int, c_void_p]),
     'art_partition_even_first_i32_tuned': (c_int, [c_void_p, c_void_p, c_longlong, c_int, c_void_p]),
     'art_gemv_w4a16_noalloc': (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p]),
     'art_decode_attention_rope_split': (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_void_p, c_int, c_int, c_void_p]),

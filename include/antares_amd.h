@@ -164,6 +164,16 @@ int art_gemm_w4a16_residual_norm(const void* x_dev, const void* qweight_dev, con
 int art_gemm_w4a16_swiglu(const void* x_dev, const void* qweight_dev, const void* scales_dev, const void* qzeros_dev,
                           void* y_dev, int M, int K, int N, int k_splits, void* stream);
 
+/* The same product with a q | k | v matrix (3 * heads * 128 columns) and what stands between it and the attention (:151-158): row m is
+ * position first_pos + m, rotated q goes to q_out [M, heads, 128], rotated k and v into cache rows first_pos + m (of
+ * max_positions).  angles_dev: fp32 [M, 64, 2], sine and cosine of the rotation of columns j and j + 64 of a head in row m,
+ * as art_rope_angles leaves them.  The angles, q_out and the caches are 16-byte aligned; no output overlaps an operand or another one. */
+int art_gemm_w4a16_rope_store(const void* x_dev, const void* qweight_dev, const void* scales_dev, const void* qzeros_dev,
+                              const void* angles_dev, void* q_out_dev, void* key_cache_dev, void* val_cache_dev, int M, int K, int heads,
+                              int first_pos, int max_positions, int k_splits, void* stream);
+/* Sine and cosine of (first_pos + t) * inv_freq[j] for t < rows, j < half: fp32 [rows, half, 2] from fp16 frequencies. */
+int art_rope_angles(const void* inv_freq_dev, void* angles_dev, int rows, int half, int first_pos, void* stream);
+
 /* art_gemv_w4a16 for callers that cannot allocate device memory or let a library do it (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc).  It has no counterpart in the reference.  Same
  * operands, constraints and results (bit for bit) as art_gemv_w4a16, with M in 1..4 and M * N <= 131072: the

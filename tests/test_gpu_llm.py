@@ -441,6 +441,49 @@ def test_rope_qkv_store_rows_against_the_oracle():
         autort.ops.rope_qkv_store_rows_f16(qkv.to(dev), inv_freq.to(dev), q_out, kd, vd, extra=[S - T + 1])
 
 
+# both kernels with and without K-splits, heads that end inside a block of 256 columns, rows that end inside a block; against the product
+# by itself with the same launch parameters and the rotation behind it: v and the sums of a product are the same bits, a rotated value is one
+# rounding of fp32 arithmetic whose terms may be contracted differently: within half of an fp16 step and 2^-22 of its terms.
+@pytest.mark.parametrize('T,K,H', [(5, 256, 1), (33, 512, 3), (129, 384, 2), (257, 256, 5)])
+def test_the_q_k_v_product_that_rotates_and_stores(T, K, H):
+    import autort
+    from ctypes import c_void_p
+    from antares_amd import workloads
+    from antares_amd.runtime import capi
+    dev, N, first = autort.device(), 3 * H * 128, 4
+    p = workloads.w4_problem(T + K + H, T, K, N)
+    d = [p[k].to(dev) for k in ('x', 'qweight', 'scales', 'qzeros')]
+    half = (1.0 / (10000 ** (torch.arange(0, 128, 2).float() / 128))).half()
+    inv = torch.cat([half, half]).to(dev)
+    angles = autort.ops.rope_angles_f16(inv, torch.empty(T, 64, 2, device=dev), extra=[first])
+    at = torch.arange(first, first + T).double().view(T, 1) * half.double().view(1, 64)
+    assert (angles.cpu().double() - torch.stack([at.sin(), at.cos()], -1)).abs().max() < 2.0 ** -24 * (T + first) + 2.0 ** -22
+
+    def outputs():
+        return [torch.full((T, H, 128), 7.0, dtype=torch.float16, device=dev)] + [torch.full((T + 9, H * 128), 7.0, dtype=torch.float16, device=dev) for _ in range(2)]
+    for code in (0, 256 + 1, 256 + 2, 512 + 1, 512 + 2, 1280 + 1, 1280 + 2, 1024 + 1, 1024 + 2, 2048 + 1, 2048 + 2):
+        note(f'q k v product T={T} K={K} H={H} code {code}')
+        qkv = torch.empty(T, N, dtype=torch.float16, device=dev)
+        capi.check(capi.lib().art_gemm_w4a16_tuned(*(c_void_p(t.data_ptr()) for t in d + [qkv]), T, K, N, code, c_void_p(torch.cuda.current_stream().cuda_stream)))
+        got, want = outputs(), outputs()
+        autort.ops.gemm_w4a16_rope_store(*d, angles, *got, extra=[first], k_splits=code)
+        autort.ops.rope_qkv_store_rows_f16(qkv, inv, *want, extra=[first])
+        assert torch.equal(got[2], want[2])
+        for part, (a, b) in enumerate(zip(got[:2], want[:2])):
+            if part:
+                assert (a[:first] == 7.0).all() and (a[first + T:] == 7.0).all()
+                a, b = a[first:first + T], b[first:first + T]
+            x = qkv[:, part * H * 128:(part + 1) * H * 128].view(T, H, 2, 64).double().abs()
+            terms = x.sum(2, keepdim=True).expand(T, H, 2, 64).reshape(T, H, 128)
+            a, b = a.view(T, H, 128).double(), b.view(T, H, 128).double()
+            assert ((a - b).abs() <= torch.maximum(a.abs(), b.abs()) * 2.0 ** -10 + terms * 2.0 ** -22 + 2.0 ** -24).all()
+    with pytest.raises(Exception, match='do not fit'):
+        autort.ops.gemm_w4a16_rope_store(*d, angles, *outputs(), extra=[10])
+    with pytest.raises(Exception, match='overlap'):
+        q, kc, _ = outputs()
+        autort.ops.gemm_w4a16_rope_store(*d, angles, q, kc, kc)
+
+
 def _tile_sums_of_squares(y: torch.Tensor) -> np.ndarray:
     """What a projection leaves in its sum-of-squares buffer for the fp16 outputs y: per tile of 128 columns the sum of
     floor(y^2 * 2^30), each square capped at 2^25 (integer arithmetic)."""
