@@ -244,7 +244,10 @@ class ExportedOp(calls.Operator):
                 for n in group.args:
                     if n not in bound:
                         bound[n] = torch.empty(g.shape_of(n, env), dtype=TORCH_DTYPE[g.tensors[n].dtype], device=dev)
-                sym, grid = group.choose(env, {n: bound[n].data_ptr() for n in group.args})
+                pointers = {n: bound[n].data_ptr() for n in group.args}
+                sym, grid = group.choose(env, pointers)
+                if not grid:
+                    sym, grid = group.choose_short(env, pointers)
                 if grid:
                     call.kernel(module.function(sym), grid, 256, [bound[n] for n in group.args] + dims)
                     skip = group.count - 1

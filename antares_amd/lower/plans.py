@@ -39,6 +39,8 @@ class RowGroup(_Rule):
     cached: List[Tuple[int, int, int, str]] = field(default_factory=list)
     vec_tensors: List[str] = field(default_factory=list)   # tensors that must be 16-byte aligned for the vector kernels
     pure: bool = False             # reductions only, no map behind them
+    # kernels with a row in the registers of 16 lanes: (elements per vector, vectors per lane, symbol)
+    short: List[Tuple[int, int, str]] = field(default_factory=list)
 
     def _extents(self, env: Dict[str, int]) -> Tuple[int, int]:
         e = self.red_axis[1]
@@ -77,6 +79,23 @@ class RowGroup(_Rule):
             pick = min(blocks, key=lambda f: f[2])
         per_block = BLOCK // pick[0]
         return pick[3], min((rows + per_block - 1) // per_block, MAX_GRID)
+
+    def choose_short(self, env: Dict[str, int], pointers: Dict[str, int]) -> Tuple[str, int]:
+        """The same for rows of 16 to 127 elements, four of them in a wavefront; grid 0 when the per-statement kernels do
+        better (below 16 most lanes would idle) or there are no such kernels.  Vectors where every lane gets one: with fewer,
+        the lanes without work cost more than the loads (2^20 rows of 16: 81 us in vectors, 40 one by one).
+        Softmax and layer normalisation in float32, statements / this (us): few rows 9.0 / 3.9, where the launches
+        bound; 65536 rows of 20 9.5 / 4.8, of 64 26 / 8.7, of 120 37 / 15; 2^20 rows of 16 54 / 40, of 32 294 / 62, of 120
+        563 / 199.  Error of the softmax against 64 bits 5.7e-8 to 1.2e-7 / 5.4e-8 to 5.9e-8."""
+        rows, n = self._extents(env)
+        if not 16 <= n < 128:
+            return self.symbol, 0
+        aligned = all(pointers[t] % 16 == 0 for t in self.vec_tensors)
+        fits = [(v, e, sym) for v, e, sym in self.short if n <= 16 * v * e and (v == 1 or (aligned and n % v == 0 and n >= 16 * v))]
+        if not fits:
+            return self.symbol, 0
+        _, _, sym = max(fits, key=lambda f: (f[0], -f[1]))
+        return sym, min((rows + 15) // 16, MAX_GRID)
 
 
 @dataclass

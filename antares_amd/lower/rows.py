@@ -91,9 +91,27 @@ def _row_run(n: Expr, r_ax: str):
     return None
 
 
+# A reduction over the 16 lanes of a row of lanes (a quarter of a wavefront): every one of them ends with the same value.
+_ROW16 = """#ifndef ART_ROW16
+#define ART_ROW16
+template <class T, class Op> ART_DEV T art_row16_reduce(T v, Op op) {
+  typedef typename art_carrier<T>::type C;
+  if constexpr (sizeof(C) == 4) {
+    struct Wrapped { Op op; ART_MEM C operator()(C a, C b) const { return (C)op((T)a, (T)b); } };
+    C c = (C)v;
+    for (int i = 0; i < 4; ++i) c = art_row_step<C>(c, Wrapped{op}, i);
+    return (T)c;
+  } else {
+    for (int m = 1; m < 16; m <<= 1) v = op(v, __shfl_xor(v, m, 64));
+    return v;
+  }
+}
+#endif"""
+
+
 def _lower_row_group(graph, i: int, count: int, sym: str) -> Tuple[str, RowGroup]:
     """Kernels that compute the whole run row by row.  Every reduction meets in the row's team of lanes (a block of
-    256 or one wavefront) and its result stays in a register for the statements that follow; reduce results are
+    256, one wavefront or, for rows shorter than two wavefronts, 16 lanes) and its result stays in a register for the statements that follow; reduce results are
     also stored, as the per-statement kernels would.  Where a row fits, it is read once, all loads in flight
     together, and kept in registers (4 or 16 vectors of 1 or 16 bytes per lane); longer rows are walked once per
     statement by a block (the first walk brings the row from memory, the later ones find it in cache)."""
@@ -141,7 +159,7 @@ def _lower_row_group(graph, i: int, count: int, sym: str) -> Tuple[str, RowGroup
                 return f'{sl[2]}[__e]' + ('[__k]' if V > 1 else '')
             return None
         em = ExprEmitter(tensors, load_override=override)
-        lane = 'threadIdx.x' if team == BLOCK else '(threadIdx.x & 63)'
+        lane = 'threadIdx.x' if team == BLOCK else f'(threadIdx.x & {team - 1})'
 
         def over_row(per_chunk_before, per_element, per_chunk_after):
             """Loop over this lane's share of the row: chunk-level lines, then element-level lines inside."""
@@ -176,7 +194,7 @@ def _lower_row_group(graph, i: int, count: int, sym: str) -> Tuple[str, RowGroup
             body.append('  for (long long __o = blockIdx.x; __o < __rows; __o += gridDim.x) {')
         else:
             per_block = BLOCK // team
-            body.append(f'  for (long long __o = (long long)blockIdx.x * {per_block} + (threadIdx.x >> 6); __o < __rows; '
+            body.append(f'  for (long long __o = (long long)blockIdx.x * {per_block} + (threadIdx.x / {team}); __o < __rows; '
                         f'__o += (long long)gridDim.x * {per_block}) {{')
         body += _decompose('__o', D, '    ')
         if E and slots:
@@ -194,7 +212,7 @@ def _lower_row_group(graph, i: int, count: int, sym: str) -> Tuple[str, RowGroup
             body.append(f'    {act} __acc_{st.output} = {reduce_identity(st.reduce, st.root.dtype)};')
             body += over_row([], [f'__acc_{st.output} = {op}(__acc_{st.output}, ({act})({em.expr(st.root)}));'], [])
             meet = (f'art_block_reduce(__acc_{st.output}, {op}, __smem_{st.output})' if team == BLOCK
-                    else f'art_wave_reduce(__acc_{st.output}, {op})')
+                    else f'{"art_wave_reduce" if team == 64 else "art_row16_reduce"}(__acc_{st.output}, {op})')
             body += [f'    const {oct_} __t_{st.output} = ({oct_}){meet};',
                      f'    if ({lane} == 0) {st.output}[{plain.offset(st.output, [plain.expr(ix) for ix in st.out_index])}] = __t_{st.output};']
         if m is not None and V > 1:
@@ -214,4 +232,11 @@ def _lower_row_group(graph, i: int, count: int, sym: str) -> Tuple[str, RowGroup
                 name = f'{sym}_{"w" if team == 64 else "b"}{E}' + (f'v{V}' if V > 1 else '')
                 group.cached.append((team, V, E, name))
                 code.append(emit(name, team, V, E))
+        if m is not None and (not isinstance(r_ext, int) or 16 <= r_ext < 128):
+            for V, E in ((1, 2), (1, 4), (1, 8)) + (((min(vmax, 4), 8 // min(vmax, 4)),) if vector_ok else ()):
+                name = f'{sym}_q{E}' + (f'v{V}' if V > 1 else '')
+                group.short.append((V, E, name))
+                code.append(emit(name, 16, V, E))
+        if group.short:
+            code.insert(0, _ROW16)
     return '\n\n'.join(code), group
