@@ -19,6 +19,9 @@
 //              even -> out[evens_before + rank]
 //              odd  -> out[total_even + odds_before + rank]
 //
+// Up to 65536 values the two launches are what takes the time: one launch, in which every block counts the evens of all
+// values by itself (partition_short_kernel).
+//
 // The order inside both halves is the input order, and the result is
 // bit-identical to the reference pipeline for non-negative inputs (for negative
 // odd values the reference's `data % 2` is -1 and indexes out of bounds; here
@@ -37,10 +40,9 @@ __device__ __forceinline__ int even_count4(i32x4 v) {
   return 4 - ((v.x & 1) + (v.y & 1) + (v.z & 1) + (v.w & 1));
 }
 
-// Loads vector `j` of this thread (elements 4*(j*256+tid) .. +3 of the tile); elements past n read as odd (1).
+// The vector of elements e0 .. e0 + 3; elements past n read as odd (1).
 template <bool LAST_USE = false>
-__device__ __forceinline__ i32x4 load_vec(const int* __restrict__ in, long long base, int j, long long n) {
-  const long long e0 = base + 4LL * (j * kThreads + threadIdx.x);
+__device__ __forceinline__ i32x4 load_at(const int* __restrict__ in, long long e0, long long n) {
   if (e0 + 3 < n) {
     if (LAST_USE) return __builtin_nontemporal_load(reinterpret_cast<const i32x4*>(in + e0));   // the scatter pass is the last reader
     return *reinterpret_cast<const i32x4*>(in + e0);
@@ -50,6 +52,28 @@ __device__ __forceinline__ i32x4 load_vec(const int* __restrict__ in, long long 
   if (e0 + 1 < n) v.y = in[e0 + 1];
   if (e0 + 2 < n) v.z = in[e0 + 2];
   return v;
+}
+// Vector `j` of this thread of a tile.
+template <bool LAST_USE = false>
+__device__ __forceinline__ i32x4 load_vec(const int* __restrict__ in, long long base, int j, long long n) {
+  return load_at<LAST_USE>(in, base + 4LL * (j * kThreads + threadIdx.x), n);
+}
+
+// Both runs leave as 16-byte non-temporal stores (written once, read by nobody here): up to three elements bring the destination to
+// a 16-byte boundary, whole vectors follow, up to three elements finish the run.
+template <int THREADS>
+__device__ __forceinline__ void flush_run(int* __restrict__ out, const int* s_items, long long dst0, unsigned int src0, unsigned int count) {
+  const unsigned int tid = threadIdx.x;
+  const unsigned int to_boundary = (4u - (unsigned int)((reinterpret_cast<uintptr_t>(out + dst0) >> 2) & 3)) & 3u;
+  const unsigned int head = to_boundary < count ? to_boundary : count;
+  const unsigned int vecs = (count - head) >> 2, tail = (count - head) & 3;
+  if (tid < head) __builtin_nontemporal_store(s_items[src0 + tid], &out[dst0 + tid]);
+  for (unsigned int q = tid; q < vecs; q += THREADS) {
+    const unsigned int s = src0 + head + 4 * q;
+    const i32x4 pack = {s_items[s], s_items[s + 1], s_items[s + 2], s_items[s + 3]};
+    __builtin_nontemporal_store(pack, reinterpret_cast<i32x4*>(out + dst0 + head + 4 * (long long)q));
+  }
+  if (tid < tail) __builtin_nontemporal_store(s_items[src0 + head + 4 * vecs + tid], &out[dst0 + head + 4 * (long long)vecs + tid]);
 }
 
 __global__ __launch_bounds__(kThreads) void partition_count_kernel(const int* __restrict__ in, long long n, int tiles_per_block,
@@ -164,22 +188,8 @@ __global__ __launch_bounds__(kThreads) void partition_scatter_kernel(const int* 
     art_lds_barrier();
     const long long odd_base = total_even + (base - even_before);
     const unsigned int tile_odd = (unsigned int)valid - tile_even;     // padding was counted as odd and sits last
-    // Both runs leave as 16-byte non-temporal stores (written once, read by nobody here): up to three elements
-    // bring the destination to a 16-byte boundary, whole vectors follow, up to three elements finish the run.
-    auto flush_run = [&](long long dst0, unsigned int src0, unsigned int count) {
-      const unsigned int to_boundary = (4u - (unsigned int)((reinterpret_cast<uintptr_t>(out + dst0) >> 2) & 3)) & 3u;
-      const unsigned int head = to_boundary < count ? to_boundary : count;
-      const unsigned int vecs = (count - head) >> 2, tail = (count - head) & 3;
-      if (tid < head) __builtin_nontemporal_store(s_items[src0 + tid], &out[dst0 + tid]);
-      for (unsigned int q = tid; q < vecs; q += kThreads) {
-        const unsigned int s = src0 + head + 4 * q;
-        const i32x4 pack = {s_items[s], s_items[s + 1], s_items[s + 2], s_items[s + 3]};
-        __builtin_nontemporal_store(pack, reinterpret_cast<i32x4*>(out + dst0 + head + 4 * (long long)q));
-      }
-      if (tid < tail) __builtin_nontemporal_store(s_items[src0 + head + 4 * vecs + tid], &out[dst0 + head + 4 * (long long)vecs + tid]);
-    };
-    flush_run(even_before, 0, tile_even);
-    flush_run(odd_base, tile_even, tile_odd);
+    flush_run<kThreads>(out, s_items, even_before, 0, tile_even);
+    flush_run<kThreads>(out, s_items, odd_base, tile_even, tile_odd);
     even_before += tile_even;
     if (more) {
 #pragma unroll
@@ -187,6 +197,69 @@ __global__ __launch_bounds__(kThreads) void partition_scatter_kernel(const int* 
     }
     art_lds_barrier();                                            // s_items / s_wave are reused by the next tile
   }
+}
+
+// Up to kShortTiles tiles, one per block of 1024 threads with one vector each.  A block reads all values, at most 16 vectors per
+// thread and eight of them in flight at a time, to know the evens in front of its tile and in total.  Two launches / this one:
+// 1000 values 6.0 / 4.1 us, 32768 6.7 / 4.6, 65536 6.8 / 5.9, 131072 6.9 / 9.9: with more blocks that all read the same
+// addresses the second launch is cheaper, and sixteen vectors in flight make it no faster (65536: 6.2).
+constexpr int kShortThreads = 1024, kShortTiles = 16;
+static_assert(kShortThreads * 4 == kTile && kShortTiles * 64 * 4 < 1 << 16, "one vector per thread; a wavefront's counts fit 16 bits");
+__global__ __launch_bounds__(kShortThreads) void partition_short_kernel(const int* __restrict__ in, int* __restrict__ out, int n) {
+  __shared__ int s_items[kTile];
+  __shared__ unsigned int s_before[16], s_total[16], s_wave[16];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, b = blockIdx.x, tiles = gridDim.x;
+  unsigned int before = 0, total = 0;               // evens of this thread's vectors: in tiles in front of this one, in all
+  i32x4 mine = {1, 1, 1, 1};
+#pragma unroll
+  for (int t0 = 0; t0 < kShortTiles; t0 += 8) {
+    if (t0 >= tiles) break;
+    i32x4 v[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = load_at(in, (long long)(t0 + j) * kTile + 4 * tid, n);        // past n: reads as odd, counts 0
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const unsigned int c = even_count4(v[j]);
+      total += c;
+      if (t0 + j < b) before += c;
+      if (t0 + j == b) mine = v[j];
+    }
+  }
+  unsigned int both = before << 16 | total;         // at most 4096 each in a wavefront
+#pragma unroll
+  for (int m = 1; m < 64; m <<= 1) both += __shfl_xor(both, m, 64);
+  const int items[4] = {mine.x, mine.y, mine.z, mine.w};
+  unsigned int below = 0, in_wave = 0;              // evens of the tile in the lanes below this one, in the wavefront
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const unsigned long long m = __ballot((items[e] & 1) == 0);
+    below = __builtin_amdgcn_mbcnt_hi((unsigned int)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned int)m, below));
+    in_wave += (unsigned int)__popcll(m);
+  }
+  if (lane == 0) {
+    s_before[wave] = both >> 16;
+    s_total[wave] = both & 0xffffu;
+    s_wave[wave] = in_wave;
+  }
+  art_lds_barrier();
+  unsigned int even_before = 0, total_even = 0, tile_even = 0, ev = below;
+#pragma unroll
+  for (int w = 0; w < 16; ++w) {
+    even_before += s_before[w];
+    total_even += s_total[w];
+    if (w < wave) ev += s_wave[w];
+    tile_even += s_wave[w];
+  }
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {                     // evens to [0, tile_even), odds behind them
+    const bool is_even = (items[e] & 1) == 0;
+    s_items[is_even ? ev : tile_even + (4u * tid + e - ev)] = items[e];
+    ev += is_even ? 1u : 0u;
+  }
+  art_lds_barrier();
+  const int base = b * kTile, valid = n - base < kTile ? n - base : kTile;
+  flush_run<kShortThreads>(out, s_items, even_before, 0, tile_even);
+  flush_run<kShortThreads>(out, s_items, total_even + (base - even_before), tile_even, valid - tile_even);
 }
 
 }  // namespace
@@ -205,6 +278,11 @@ extern "C" int art_partition_even_first_i32_tuned(const void* in_dev, void* out_
   ART_REQUIRE(((uintptr_t)out_dev % 4) == 0, "art_partition_even_first_i32: output must be 4-byte aligned");
   art::Workspace* wsp = art::workspace((hipStream_t)stream);
   if (!wsp) return 1;
+  if (max_blocks == 0 && n <= (long long)kShortTiles * kTile) {
+    partition_short_kernel<<<dim3((unsigned)((n + kTile - 1) / kTile)), dim3(kShortThreads), 0, (hipStream_t)stream>>>((const int*)in_dev, (int*)out_dev, (int)n);
+    ART_LAUNCH_CHECK();
+    return 0;
+  }
   art::Workspace& ws = *wsp;
   const long long tiles = (n + kTile - 1) / kTile;
   const long long kMaxBlocks = max_blocks ? max_blocks : 1024;  // bounds the counts every block adds up (4 KiB from L2 at 1024)

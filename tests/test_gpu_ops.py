@@ -114,6 +114,27 @@ def test_partition_empty_and_degenerate(autort):
         assert (backing[:shift] == -7).all() and (backing[shift + 10_007:] == -7).all()
 
 
+# one launch up to 65536 values: edges of a wavefront's vectors, of tiles, of the eight tiles that are read at a time, of the range
+@pytest.mark.parametrize('n', [1, 2, 5, 255, 257, 4095, 4096, 4097, 32767, 32769, 65533, 65536, 65537])
+@pytest.mark.parametrize('shift', [0, 1])
+def test_partition_of_few_values_in_one_launch_and_in_two(autort, n, shift):
+    from ctypes import c_void_p
+    from antares_amd.runtime import capi
+    note(f'partition N={n} shift={shift}')
+    dev = autort.device()
+    autort.ops.partition_even_first_i32(torch.zeros(8, dtype=torch.int32, device=dev))
+    x = torch.randint(-2 ** 31, 2 ** 31, (n,), generator=torch.Generator().manual_seed(n), dtype=torch.int64).to(torch.int32)
+    xd = x.to(dev)
+    for values in (xd, xd & ~1, xd | 1):
+        want = torch.cat([values[(values & 1) == 0], values[(values & 1) == 1]]).cpu()
+        for blocks in (0, 1024):                 # the library's choice; two launches
+            out = torch.full((n + 8,), 7, dtype=torch.int32, device=dev)
+            capi.check(capi.lib().art_partition_even_first_i32_tuned(c_void_p(values.data_ptr()), c_void_p(out.data_ptr() + 4 * shift), n, blocks,
+                                                                     c_void_p(torch.cuda.current_stream().cuda_stream)))
+            got = out.cpu()
+            assert torch.equal(got[shift:shift + n], want) and (got[:shift] == 7).all() and (got[shift + n:] == 7).all()
+
+
 def test_partition_full_size_properties(autort):
     note('partition N=16777216 (size-independent properties)')
     x = workloads.partition_input(2, 16_777_216).to(autort.device())
