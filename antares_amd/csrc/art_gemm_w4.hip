@@ -56,7 +56,8 @@ static_assert(16 * 1024 + 32 * (BN + 8) * 2 <= 3 * stage_bytes(1) && 32 * 1024 +
 
 // How the (column tile, K split) pairs are laid out; worked out on the host, so that a block starts without divisions.
 struct Work {
-  int units, col_tiles, splits;
+  Deal deal;
+  int col_tiles, splits;
   unsigned int inv_tiles;                           // ceil(2^32 / col_tiles), 0 for one tile: unit / col_tiles = mulhi(unit, inv_tiles) for units below 2^16
   int groups, longer;                               // groups of a K split; the first `longer` have one more
 };
@@ -73,12 +74,9 @@ __global__ __launch_bounds__(kThreads, MT == 4 ? 2 : 4) void gemm_w4a16_kernel(
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int cw = wave & 3, kh = wave >> 2;          // 32-column quarter of the tile, k half of every group
 
-  // block -> (column tile, K split, block of rows).  The row blocks of one (tile, split) stream the same weights: they
-  // get block ids that are 8 apart, which the dispatcher places on the same XCD at the same time, so that the weights
-  // come from HBM once and from that XCD's L2 for the others.
-  const int unit = blockIdx.y * 8 + (blockIdx.x & 7);                  // (tile, split) pair
-  const int m0 = (int)(blockIdx.x >> 3) * BM;
-  if (unit >= work.units) return;
+  int unit, m_block;                                // (tile, split) pair, block of rows
+  if (!work.deal.take(unit, m_block)) return;
+  const int m0 = m_block * BM;
   const int split = work.inv_tiles ? (int)__umulhi(unit, work.inv_tiles) : unit;      // unit / col_tiles
   const TileColumns<TAIL, BN> cols{(unit - split * work.col_tiles) * (SWIGLU ? BN / 2 : BN), N};
   const int g_begin = split * work.groups + (split < work.longer ? split : work.longer), groups = work.groups + (split < work.longer ? 1 : 0);
@@ -461,10 +459,11 @@ double estimate(int M, int K, int N, const Plan& p, int compute_units) {
   const double again = p.wide ? 0.0 : 1.5 * ((blocks - 1) / round);
   return c.fixed + again + groups * per_group + (p.splits > 1 ? 2.4 + (8.0 * p.splits + 2.0) * M * N / 4.4e6 : 0.0);
 }
-// What a form's 32-bit offsets (a block's rows of x and of the packed weights) and its division by the number of column
-// tiles hold.
+// What a form's 32-bit offsets (a block's rows of x and of the packed weights), its division by the number of column
+// tiles and its grid hold.
 bool holds(const Plan& p, int K, int N, bool swiglu) {
-  return 64LL * p.row_tiles * K <= 1LL << 32 && 64LL * N <= 1LL << 32 && (p.wide || (long long)tile_count(N, swiglu, BN) * p.splits < 65536);
+  const long long units = (long long)tile_count(N, swiglu, p.wide ? 256 : BN) * p.splits;
+  return 64LL * p.row_tiles * K <= 1LL << 32 && 64LL * N <= 1LL << 32 && units < (p.wide ? 1 << 19 : 1 << 16);
 }
 // False: no form takes these sizes.  `code` and `splits` are the caller's wishes (0: none); a form that does not hold the
 // sizes is replaced by one that does.
@@ -548,8 +547,8 @@ int run_rows(const _Float16* xs, const unsigned char* qweight, const _Float16* s
     }
     const int col_tiles = tile_count(N, swiglu, BN), m_blocks = (M + 32 * p.row_tiles - 1) / (32 * p.row_tiles);
     const int units = col_tiles * p.splits, G = K / GK;
-    const Work work{units, col_tiles, p.splits, (unsigned int)((0x100000000ull + col_tiles - 1) / col_tiles), G / p.splits, G % p.splits};
-    const dim3 grid(8 * m_blocks, (units + 7) / 8);
+    dim3 grid;
+    const Work work{deal(units, m_blocks, grid), col_tiles, p.splits, (unsigned int)((0x100000000ull + col_tiles - 1) / col_tiles), G / p.splits, G % p.splits};
     const auto kernel = kernels[p.row_tiles == 4 ? 2 : p.row_tiles - 1][tail];
     kernel<<<grid, kThreads, lds_bytes(p.row_tiles), st>>>(xs, qweight, scales, qzeros, ys, scratch, M, K, N, work, kMagic, res, rope);
     ART_LAUNCH_CHECK();

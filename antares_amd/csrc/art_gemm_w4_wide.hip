@@ -47,16 +47,14 @@ template <int MT, Tail TAIL>
 __global__ __launch_bounds__(kThreads, MT == 8 ? 1 : 2) void gemm_w4a16_wide_kernel(
     const _Float16* __restrict__ x, const unsigned char* __restrict__ qweight, const _Float16* __restrict__ scales,
     const unsigned char* __restrict__ qzeros, _Float16* y, float* __restrict__ partial, int M, int K, int N, int splits,
-    int col_tiles, int m_blocks, Magic mg, const _Float16* residual, Rope rope) {       // residual may be y itself
+    int col_tiles, Deal deal, Magic mg, const _Float16* residual, Rope rope) {       // residual may be y itself
   constexpr bool SWIGLU = TAIL == kSwiglu;
   constexpr int STAGE = stage_bytes(MT), BM = 32 * MT;
   constexpr int L = 2 + MT + 1;                     // loads per wavefront and stage
   extern __shared__ __align__(1024) unsigned char smem[];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  // the row blocks of one (column tile, K split) have block ids 8 apart: the same XCD, whose L2 then serves the weights
-  const int unit = (int)(blockIdx.x / (8 * m_blocks)) * 8 + (int)(blockIdx.x % 8);
-  const int m_block = (int)(blockIdx.x % (8 * m_blocks)) / 8;
-  if (unit >= col_tiles * splits) return;
+  int unit, m_block;                                // (column tile, K split) pair, block of rows
+  if (!deal.take(unit, m_block)) return;
   const int split = unit / col_tiles;
   const TileColumns<TAIL, BN> cols{(unit % col_tiles) * (SWIGLU ? BN / 2 : BN), N};
   const int m0 = m_block * BM;
@@ -342,8 +340,10 @@ int launch(const _Float16* x, const unsigned char* qweight, const _Float16* scal
     configured = true;
   }
   const int col_tiles = tile_count(N, TAIL == kSwiglu, BN), m_blocks = (M + 32 * MT - 1) / (32 * MT);
-  gemm_w4a16_wide_kernel<MT, TAIL><<<dim3((unsigned)((col_tiles * splits + 7) / 8 * 8 * m_blocks)), kThreads, lds_bytes(MT), stream>>>(
-      x, qweight, scales, qzeros, y, partial, M, K, N, splits, col_tiles, m_blocks, kMagic, residual, rope);
+  dim3 grid;
+  const Deal dealt = deal(col_tiles * splits, m_blocks, grid);
+  gemm_w4a16_wide_kernel<MT, TAIL><<<grid, kThreads, lds_bytes(MT), stream>>>(
+      x, qweight, scales, qzeros, y, partial, M, K, N, splits, col_tiles, dealt, kMagic, residual, rope);
   ART_LAUNCH_CHECK();
   return 0;
 }
