@@ -10,7 +10,7 @@
 //     groups.  Wavefront (c, h) multiplies 32 columns by the k half h of every group, so every weight is unpacked once per
 //     block; the two k halves meet in LDS after the loop.  What bounds the loop is the issue of instructions, not the
 //     matrix cores (with the MFMAs taken out a group takes as long): a wavefront issues one per 7 cycles or so, and a
-//     group is 137 / 158 / 201 of them at MT = 1 / 2 / 4, 84 of them vector instructions that unpack - 1090 / 1200 / 1460 cycles.
+//     group is 136 / 149 / 193 of them at MT = 1 / 2 / 4, 64 of them vector instructions that unpack - 1090 / 1170 / 1420 cycles.
 //     Sixteen wavefronts with half the work each were slower (the LDS meeting doubles), and so were four column quarters
 //     replaced by two (same loop, longer meeting), blocks that start at groups of their own, and branches around the
 //     loads of the last groups;
@@ -148,7 +148,7 @@ __global__ __launch_bounds__(kThreads, MT == 4 ? 2 : 4) void gemm_w4a16_kernel(
   i32x2 pk[2], pk_next[2];                          // packed weights of the group and of the next one: [q]
   _Float16 raw_s;
   unsigned int raw_z;
-  h2 s2, zz2;                                       // scale, 1024 + zero point of this lane's column
+  h2 s2, zz2;                                       // scale, 1024 and 64 + zero point of this lane's column
   h8 fa[2][MT];                                     // operands of a round, double buffered: x
   h2 fb[2][4];                                      // ... weights, in pairs of k
   auto read_weights = [&](unsigned int slot, i32x2 (&to)[2], int q) {
@@ -163,16 +163,14 @@ __global__ __launch_bounds__(kThreads, MT == 4 ? 2 : 4) void gemm_w4a16_kernel(
     const unsigned int z = (raw_z >> ((colpos & 1) * 4)) & 15u;
     const _Float16 s = cols.inside(colpos) ? raw_s : (_Float16)0.f;
     s2 = h2{s, s};
-    zz2 = as_h2(z | (z << 16) | mg.bias_lo);
+    zz2 = as_h2(z | (z << 20) | mg.bias);
   };
   auto read_x = [&](unsigned int slot, int e, int t) {
     fa[e & 1][t] = *reinterpret_cast<const h8*>(smem + slot + a_off[e] + t * 8192);
   };
   // pair j for round e = 2 q + dword.  Byte j of the word holds k = 2 j (low nibble) and 2 j + 1 (high nibble).
   auto unpack = [&](const i32x2 (&from)[2], int e, int j) {
-    const unsigned int w = (unsigned int)from[e >> 1][e & 1], u = w >> 4;
-    const unsigned int q = __builtin_amdgcn_perm(u, w, 0x0c040c00u + 0x00010001u * j);
-    fb[e & 1][j] = (as_h2(and_or(q, mg.mask_lo, mg.bias_lo)) - zz2) * s2;
+    fb[e & 1][j] = (as_h2(and_or(nibble_pair<(MT > 1)>((unsigned int)from[e >> 1][e & 1], j), mg.mask, mg.bias)) - zz2) * s2;
   };
   auto multiply = [&](int slot, int t) {
     const h2* p = fb[slot];

@@ -8,8 +8,8 @@
 //     unit, MT = 8: 256 and one wavefront per SIMD).  No two wavefronts unpack the same weight.  What bounds the loop is
 //     the issue of vector instructions beside the MFMAs: one wavefront alone gets four of them into the shadow of an
 //     MFMA (32 cycles) and pays 7 cycles for every further one, two wavefronts get six each.  Hence pairs of k in
-//     natural order (one v_perm more per pair of weights) instead of a permutation of every x operand: the loop has 2.3
-//     vector instructions per MFMA at MT = 8 and 4.7 at MT = 4 (counted over a launch 2.6 and 5.6 to 6.3);
+//     natural order (half a v_perm and half a shift more per pair of weights) instead of a permutation of every x
+//     operand: the loop has 2.1 vector instructions per MFMA at MT = 8 and 4.3 at MT = 4;
 //   * per 64 values of k a block needs 8 KiB of packed weights, 4 MT KiB of x and the group's scales and zero points;
 //     they go from global memory straight into LDS (global_load_lds, no registers in flight), a ring of three slots.
 //     The weights run a stage ahead of x, so that the first operands of a stage can be unpacked in the stage before;
@@ -128,7 +128,7 @@ __global__ __launch_bounds__(kThreads, MT == 8 ? 1 : 2) void gemm_w4a16_wide_ker
   i32x2 pk[2][2][2];                                // packed weights: [stage parity][q][column tile]
   _Float16 raw_s[2];
   unsigned int raw_z[2];
-  h2 s2[2], zz2[2];                                 // scale, 1024 + zero point of this lane's two columns
+  h2 s2[2], zz2[2];                                 // scale, 1024 and 64 + zero point of this lane's two columns
   h8 fa[2][MT];                                     // operands of a round, double buffered: x
   h2 fb[2][2][4];                                   // ... weights, in pairs of k
   auto read_weights = [&](unsigned int slot, int par, int part) {
@@ -144,16 +144,14 @@ __global__ __launch_bounds__(kThreads, MT == 8 ? 1 : 2) void gemm_w4a16_wide_ker
     const unsigned int z = (raw_z[ct] >> ((colpos[ct] & 1) * 4)) & 15u;
     const _Float16 s = cols.inside(colpos[ct]) ? raw_s[ct] : (_Float16)0.f;
     s2[ct] = h2{s, s};
-    zz2[ct] = as_h2(z | (z << 16) | mg.bias_lo);
+    zz2[ct] = as_h2(z | (z << 20) | mg.bias);
   };
   auto read_x = [&](unsigned int slot, int e, int t) {
     fa[e & 1][t] = *reinterpret_cast<const h8*>(smem + slot + a_off[e] + t * 4096);
   };
   // pair j of column tile ct for round e.  Byte j of the word holds k = 2 j (low nibble) and 2 j + 1 (high nibble).
   auto unpack = [&](int par, int e, int ct, int j) {
-    const unsigned int w = (unsigned int)pk[par][e >> 1][ct][e & 1], u = w >> 4;
-    const unsigned int q = __builtin_amdgcn_perm(u, w, 0x0c040c00u + 0x00010001u * j);
-    fb[e & 1][ct][j] = (as_h2(and_or(q, mg.mask_lo, mg.bias_lo)) - zz2[ct]) * s2[ct];
+    fb[e & 1][ct][j] = (as_h2(and_or(nibble_pair<true>((unsigned int)pk[par][e >> 1][ct][e & 1], j), mg.mask, mg.bias)) - zz2[ct]) * s2[ct];
   };
   auto multiply = [&](int slot, int t) {
 #pragma unroll

@@ -20,7 +20,7 @@ typedef int i32x2 __attribute__((ext_vector_type(2)));
 typedef __attribute__((address_space(3))) i32x2 lds_i32x2;
 
 struct Magic {
-  unsigned int mask_lo, mask_hi, bias_lo, bias_hi;   // 0x000F000F 0x00F000F0 0x64006400 0x54005400
+  unsigned int mask, bias;
 };
 
 __device__ __forceinline__ h2 as_h2(unsigned int v) { return __builtin_bit_cast(h2, v); }
@@ -30,7 +30,18 @@ __device__ __forceinline__ unsigned int and_or(unsigned int w, unsigned int mask
   return __builtin_amdgcn_bitop3_b32(w, mask, bias, 0xEA);
 }
 
-constexpr Magic kMagic{0x000F000Fu, 0x00F000F0u, 0x64006400u, 0x54005400u};
+constexpr Magic kMagic{0x00F0000Fu, 0x54006400u};
+
+// Byte j of a word holds k = 2 j (low nibble) and 2 j + 1 (high nibble).  Masked and biased as kMagic, the result is fp16 (1024 + the
+// first, 64 + the second): the low nibble is the last bits of 1024 + q, the high one those of 64 + q where it lies.  SHIFT: two of
+// four byte permutations are shifts, which issue faster but wait for the first ones: blocks of 32 rows, with little between the
+// pairs, are 2 to 4 % slower so, larger ones 1 to 3 % faster (one card, against a shift and four permutations per word: 128
+// rows over 4096 x 22016 30.1 -> 29.4 us, over 11008 x 4096 22.9 -> 22.5, 1003 rows over 4096 x 22016 161.0 -> 158.8).
+template <bool SHIFT> __device__ __forceinline__ unsigned int nibble_pair(unsigned int w, int j) {
+  if (!SHIFT) return __builtin_amdgcn_perm(w, w, 0x0c000c00u + 0x00010001u * j);
+  const unsigned int twice = __builtin_amdgcn_perm(w, w, j < 2 ? 0x01000100u : 0x03020302u);      // a half word in both halves
+  return j & 1 ? twice >> 8 : twice;
+}
 
 // What becomes of the product: stored (a residual added), SwiGLU of its gate | up halves, or, of q | k | v with heads of
 // 128 columns, q and k rotated and all three stored where the attention reads them.
