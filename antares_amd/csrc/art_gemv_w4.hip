@@ -202,6 +202,8 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(1, 4))) 
   const int cl = tid % CL, kl = tid / CL;
   const int tile = blockIdx.x, split = blockIdx.y;
   const int n0 = tile * CT + cl * 16;
+  // every argument that a load needs, in one trip: left to itself the compiler fetches those of the weights behind the loads of x
+  asm volatile("" ::"s"(qweight), "s"(scales), "s"(qzeros), "s"(fused.residual), "s"(fused.att_partial), "s"(fused.att_parts), "s"(K), "s"(N));
   const int rows = K >> 1;
   const int r0 = split * kRowsPerBlock + kl * R;          // first packed row of this lane
   const bool k_ok = r0 < rows;                            // rows % 64 == 0, so a lane is all in or all out
@@ -221,7 +223,6 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(1, 4))) 
   if constexpr (MODE == 4) {                              // one word per lane: K / 128 <= 64
     if (lane < (K >> 7)) ss_word = fused.sumsq_in[lane];
   }
-  if (M == 1 && fused.sumsq_clear != nullptr && blockIdx.x == 0 && blockIdx.y == 0 && tid < kSumsqWords) fused.sumsq_clear[tid] = 0ull;
   if constexpr (norm_own) {
 #pragma unroll
     for (int i = 0; i < kSq; ++i) {
@@ -300,6 +301,8 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(1, 4))) 
   const unsigned int sc2 = *reinterpret_cast<const unsigned int*>(scales + (size_t)gc * N + pcolc);
   const unsigned char zb = qzeros[(size_t)gc * (N >> 1) + (pcolc >> 1)];
   __builtin_amdgcn_sched_barrier(0);                      // nothing below may move above the loads, no load below them
+  // (in front of the loads it would put a second trip for the arguments of the kernel before them)
+  if (M == 1 && fused.sumsq_clear != nullptr && blockIdx.x == 0 && blockIdx.y == 0 && tid < kSumsqWords) fused.sumsq_clear[tid] = 0ull;
   if constexpr (swiglu || attn) {       // part 2: pair -> LDS -> all 16 values of the k lane (same wavefront: no block barrier needed)
     half2_t o;
     if (swiglu) {

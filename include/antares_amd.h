@@ -353,7 +353,7 @@ int art_rope_qkv_store_rows(const void* qkv_dev, const void* freq_dev, void* q_o
                             int rows, int heads, int head_dim, int first_pos, int max_positions, void* stream);
 /* art_rope_qkv_store and art_decode_attention in one launch (fp16): block h rotates its head's q and k,
  * writes k and v into cache row *pos_dev and attends over rows 0..*pos_dev.  The caches have max_positions rows:
- * a position outside 0..max_positions-1 (a recorded graph replayed once too often) touches no cache row and
+ * a position outside 0..max_positions-1 (a recorded graph replayed once too often) reads no cache row but the first, writes none and
  * returns NaN. */
 int art_decode_attention_rope(const void* qkv_dev, const void* inv_freq_dev, void* key_cache_dev, void* val_cache_dev,
                               const void* att_f_dev, void* out_dev, int heads, int head_dim, const void* pos_dev,
