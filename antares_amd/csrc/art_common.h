@@ -69,6 +69,16 @@ __device__ __forceinline__ const void* uniform(const void* p) {
                        (unsigned long long)(unsigned int)__builtin_amdgcn_readfirstlane((int)(v >> 32)) << 32);
 }
 
+// x / d for x below 2^30: x * mul >> shift with mul = ceil(2^shift / d), shift = 30 + ceil(log2 d).
+struct Div {
+  unsigned int mul, shift, by;
+};
+inline Div make_div(unsigned int d) {
+  const unsigned int s = d > 1 ? 32 - __builtin_clz(d - 1) : 0;
+  return Div{(unsigned int)(((1ull << (30 + s)) + d - 1) / d), 30 + s, d};
+}
+__device__ __forceinline__ unsigned int over(unsigned int x, const Div& d) { return (unsigned int)((unsigned long long)x * d.mul >> d.shift); }
+
 // g / (1 + e^-g) of a value that fp16 holds.  t, g times log2(e) cut to 13 bits, is exact; e^-g = 2^n 2^(t - n + the rest).
 // The quotient is corrected once; numerator and denominator are divided by 16, so that its reciprocal stays a normal
 // number.  Zeros, infinities and NaN come out as of the division itself (-infinity: NaN).

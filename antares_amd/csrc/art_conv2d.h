@@ -5,6 +5,10 @@
 namespace art {
 namespace conv {
 
+using ::art::Div;
+using ::art::make_div;
+using ::art::over;
+
 constexpr int kThreads = 256;
 constexpr int kTaps = 9;                        // 3 x 3
 constexpr int kChunkBytes = 64;                 // channels of a point that are staged at a time
@@ -27,17 +31,6 @@ template <> struct Elem<float> {
     return c;
   }
 };
-
-// x / d for x below 2^30: x * mul >> shift with mul = ceil(2^shift / d), shift = 30 + ceil(log2 d).
-struct Div {
-  unsigned int mul, shift, by;
-};
-inline Div make_div(unsigned int d) {
-  unsigned int s = 0;
-  while ((1u << s) < d) ++s;
-  return Div{(unsigned int)(((1ull << (30 + s)) + d - 1) / d), 30 + s, d};
-}
-__device__ __forceinline__ unsigned int over(unsigned int x, const Div& d) { return (unsigned int)((unsigned long long)x * d.mul >> d.shift); }
 
 struct Geometry {
   int N, C, H, W, F, HO, WO, ph, pw;

@@ -407,23 +407,22 @@ __global__ __launch_bounds__(kNormThreads) void gemm_w4a16_combine_norm_kernel(c
 
 // The same for gate | up: y[m, n] of N / 2 columns from the sums of columns n and N / 2 + n.
 __global__ __launch_bounds__(256) void gemm_w4a16_combine_swiglu_kernel(const float* __restrict__ partial, _Float16* y, int rows, int N,
-                                                                         int splits) {
-  const int quads = N / 8;           // groups of four output columns
-  const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
-  if (i >= (long long)rows * quads) return;
-  const long long row = i / quads, col = (i % quads) * 4, stride = (long long)rows * N;
+                                                                         int splits, Div quads) {      // groups of four output columns of a row
+  const unsigned i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= rows * quads.by) return;
+  const long long row = over(i, quads), col = (i - (unsigned)row * quads.by) * 4, stride = (long long)rows * N;
   const f32x4 g = sum_splits(partial + row * N + col, stride, splits), u = sum_splits(partial + row * N + N / 2 + col, stride, splits);
   *reinterpret_cast<h4*>(y + row * (N / 2) + col) = swiglu4(h4{(_Float16)g[0], (_Float16)g[1], (_Float16)g[2], (_Float16)g[3]},
                                                             h4{(_Float16)u[0], (_Float16)u[1], (_Float16)u[2], (_Float16)u[3]});
 }
 
 // The same for q | k | v: columns j .. j + 3 of a head and their partners 64 further on, rotated in q and k.
-__global__ __launch_bounds__(256) void gemm_w4a16_combine_rope_kernel(const float* __restrict__ partial, int rows, int splits, Rope rope) {
-  const int pieces = rope.heads * 48;               // of a row
-  const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
-  if (i >= (long long)rows * pieces) return;
-  const long long row = i / pieces, stride = (long long)rows * pieces * 8;
-  const int at = (int)(i - row * pieces), head = at >> 4, j = (at & 15) * 4;
+__global__ __launch_bounds__(256) void gemm_w4a16_combine_rope_kernel(const float* __restrict__ partial, int rows, int splits, Rope rope, Div of_row) {
+  const int pieces = of_row.by;                     // 48 heads
+  const unsigned i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= rows * of_row.by) return;
+  const long long row = over(i, of_row), stride = (long long)rows * pieces * 8;
+  const int at = (int)(i - (unsigned)row * of_row.by), head = at >> 4, j = (at & 15) * 4;
   const float* const from = partial + (row * pieces * 8 + head * 128 + j);
   const f32x4 first = sum_splits(from, stride, splits), second = sum_splits(from + 64, stride, splits);
   h4 a = h4{(_Float16)first[0], (_Float16)first[1], (_Float16)first[2], (_Float16)first[3]};
@@ -503,12 +502,12 @@ int combine(const float* partial, _Float16* y, int rows, int N, int splits, cons
     return 0;
   }
   if (tail == kRope) {
-    gemm_w4a16_combine_rope_kernel<<<dim3((unsigned)(((long long)rows * (N / 8) + 255) / 256)), 256, 0, stream>>>(partial, rows, splits, rope);
+    gemm_w4a16_combine_rope_kernel<<<dim3((unsigned)(((long long)rows * (N / 8) + 255) / 256)), 256, 0, stream>>>(partial, rows, splits, rope, make_div(N / 8));
     ART_LAUNCH_CHECK();
     return 0;
   }
   if (tail == kSwiglu) {
-    gemm_w4a16_combine_swiglu_kernel<<<dim3((unsigned)(((long long)rows * (N / 8) + 255) / 256)), 256, 0, stream>>>(partial, y, rows, N, splits);
+    gemm_w4a16_combine_swiglu_kernel<<<dim3((unsigned)(((long long)rows * (N / 8) + 255) / 256)), 256, 0, stream>>>(partial, y, rows, N, splits, make_div(N / 8));
     ART_LAUNCH_CHECK();
     return 0;
   }

@@ -5,6 +5,10 @@
 namespace art {
 namespace w4 {
 
+using ::art::Div;
+using ::art::make_div;
+using ::art::over;
+
 using ::art::load_lds_x1;
 using ::art::load_lds_x4;
 using ::art::uniform;
