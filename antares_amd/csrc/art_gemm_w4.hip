@@ -323,11 +323,21 @@ __global__ __launch_bounds__(kThreads, MT == 4 ? 2 : 4) void gemm_w4a16_kernel(
   }
 }
 
-// Four neighbouring sums over the K-splits, in split order: eight splits at a time, all eight loads issued before the
-// first is added (a loop of load-then-add runs one memory round trip per split).  Past the last split a load repeats
-// split 0 and is not added.
+// Four neighbouring sums over the K-splits, in split order, all loads issued before the first is added (a loop of load-then-add
+// runs one memory round trip per split).  SPLITS: their number, up to eight; 0: eight at a time, where past the last one a load
+// repeats split 0 and is not added.  With the number known, product and pass together: 128 rows over 4096 x 4096 in three splits
+// 15.0 -> 14.7 us, 50 rows in four 10.9 -> 10.7, 16 rows over 4096 x 12288 in two 13.6 -> 13.4.
+template <int SPLITS>
 __device__ __forceinline__ f32x4 sum_splits(const float* partial, long long split_stride, int splits) {
   f32x4 t = *reinterpret_cast<const f32x4*>(partial);
+  if constexpr (SPLITS > 0) {
+    f32x4 v[SPLITS];
+#pragma unroll
+    for (int j = 1; j < SPLITS; ++j) v[j] = *reinterpret_cast<const f32x4*>(partial + j * split_stride);
+#pragma unroll
+    for (int j = 1; j < SPLITS; ++j) t += v[j];
+    return t;
+  }
   for (int s0 = 1; s0 < splits; s0 += 8) {
     f32x4 v[8];
 #pragma unroll
@@ -340,12 +350,12 @@ __device__ __forceinline__ f32x4 sum_splits(const float* partial, long long spli
 }
 
 // y[m,n] = fp16(sum over splits); four columns per thread (N % 4 == 0).
-__global__ __launch_bounds__(256) void gemm_w4a16_combine_kernel(const float* __restrict__ partial, _Float16* y,
+template <int SPLITS> __global__ __launch_bounds__(256) void gemm_w4a16_combine_kernel(const float* __restrict__ partial, _Float16* y,
                                                                   long long count4, long long split_stride, int splits,
                                                                   const _Float16* residual) {
   const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
   if (i >= count4) return;
-  const f32x4 t = sum_splits(partial + i * 4, split_stride, splits);
+  const f32x4 t = sum_splits<SPLITS>(partial + i * 4, split_stride, splits);
   h4 out = h4{(_Float16)t[0], (_Float16)t[1], (_Float16)t[2], (_Float16)t[3]};
   if (residual) {                    // y = fp16(fp16(product) + residual); residual may be y itself
     const h4 res = *reinterpret_cast<const h4*>(residual + i * 4);
@@ -360,7 +370,7 @@ __global__ __launch_bounds__(256) void gemm_w4a16_combine_kernel(const float* __
 // pieces of 8).  Bound by the launch: instead of two launches of 2 us and more, one; a layer of the 32-layer model's prompt pass has
 // two of them: 8 layers 608 -> 594 us at 8 tokens, 776 -> 750 at 50, 962 -> 925 at 100, 1345 -> 1337 at 200 (fewer K-splits meet).
 constexpr int kNormThreads = 512, kNormTurns = 2;
-__global__ __launch_bounds__(kNormThreads) void gemm_w4a16_combine_norm_kernel(const float* __restrict__ partial, _Float16* y, int N,
+template <int SPLITS> __global__ __launch_bounds__(kNormThreads) void gemm_w4a16_combine_norm_kernel(const float* __restrict__ partial, _Float16* y, int N,
                                                                                 long long split_stride, int splits, const _Float16* residual,
                                                                                 const _Float16* __restrict__ weight, _Float16* __restrict__ norm_out, float eps) {
   typedef _Float16 h8 __attribute__((ext_vector_type(8)));
@@ -374,7 +384,7 @@ __global__ __launch_bounds__(kNormThreads) void gemm_w4a16_combine_norm_kernel(c
     const int c = tid + i * threads;
     if (c >= chunks) break;
     const size_t at = row + 8 * (size_t)c;
-    const f32x4 lo = sum_splits(partial + at, split_stride, splits), hi = sum_splits(partial + at + 4, split_stride, splits);
+    const f32x4 lo = sum_splits<SPLITS>(partial + at, split_stride, splits), hi = sum_splits<SPLITS>(partial + at + 4, split_stride, splits);
 #pragma unroll
     for (int k = 0; k < 8; ++k) v[i][k] = (_Float16)(k < 4 ? lo[k] : hi[k - 4]);
     if (residual) {
@@ -406,25 +416,25 @@ __global__ __launch_bounds__(kNormThreads) void gemm_w4a16_combine_norm_kernel(c
 }
 
 // The same for gate | up: y[m, n] of N / 2 columns from the sums of columns n and N / 2 + n.
-__global__ __launch_bounds__(256) void gemm_w4a16_combine_swiglu_kernel(const float* __restrict__ partial, _Float16* y, int rows, int N,
+template <int SPLITS> __global__ __launch_bounds__(256) void gemm_w4a16_combine_swiglu_kernel(const float* __restrict__ partial, _Float16* y, int rows, int N,
                                                                          int splits, Div quads) {      // groups of four output columns of a row
   const unsigned i = blockIdx.x * 256 + threadIdx.x;
   if (i >= rows * quads.by) return;
   const long long row = over(i, quads), col = (i - (unsigned)row * quads.by) * 4, stride = (long long)rows * N;
-  const f32x4 g = sum_splits(partial + row * N + col, stride, splits), u = sum_splits(partial + row * N + N / 2 + col, stride, splits);
+  const f32x4 g = sum_splits<SPLITS>(partial + row * N + col, stride, splits), u = sum_splits<SPLITS>(partial + row * N + N / 2 + col, stride, splits);
   *reinterpret_cast<h4*>(y + row * (N / 2) + col) = swiglu4(h4{(_Float16)g[0], (_Float16)g[1], (_Float16)g[2], (_Float16)g[3]},
                                                             h4{(_Float16)u[0], (_Float16)u[1], (_Float16)u[2], (_Float16)u[3]});
 }
 
 // The same for q | k | v: columns j .. j + 3 of a head and their partners 64 further on, rotated in q and k.
-__global__ __launch_bounds__(256) void gemm_w4a16_combine_rope_kernel(const float* __restrict__ partial, int rows, int splits, Rope rope, Div of_row) {
+template <int SPLITS> __global__ __launch_bounds__(256) void gemm_w4a16_combine_rope_kernel(const float* __restrict__ partial, int rows, int splits, Rope rope, Div of_row) {
   const int pieces = of_row.by;                     // 48 heads
   const unsigned i = blockIdx.x * 256 + threadIdx.x;
   if (i >= rows * of_row.by) return;
   const long long row = over(i, of_row), stride = (long long)rows * pieces * 8;
   const int at = (int)(i - (unsigned)row * of_row.by), head = at >> 4, j = (at & 15) * 4;
   const float* const from = partial + (row * pieces * 8 + head * 128 + j);
-  const f32x4 first = sum_splits(from, stride, splits), second = sum_splits(from + 64, stride, splits);
+  const f32x4 first = sum_splits<SPLITS>(from, stride, splits), second = sum_splits<SPLITS>(from + 64, stride, splits);
   h4 a = h4{(_Float16)first[0], (_Float16)first[1], (_Float16)first[2], (_Float16)first[3]};
   h4 b = h4{(_Float16)second[0], (_Float16)second[1], (_Float16)second[2], (_Float16)second[3]};
   if (rope.rotated(head)) rotate(a, b, load_angles<4>(rope.angles + row * 64 + j));
@@ -492,27 +502,28 @@ struct Norm {
   float eps;
 };
 
-int combine(const float* partial, _Float16* y, int rows, int N, int splits, const _Float16* residual, Tail tail, const Norm* norm,
-            const Rope& rope, hipStream_t stream) {
+template <int SPLITS>
+void launch_combine(const float* partial, _Float16* y, int rows, int N, int splits, const _Float16* residual, Tail tail, const Norm* norm,
+                    const Rope& rope, hipStream_t stream) {
+  const dim3 by_eight((unsigned)(((long long)rows * (N / 8) + 255) / 256));
   if (norm) {
     const int threads = N < 8 * kNormThreads ? (N / 8 + 63) / 64 * 64 : kNormThreads;
-    gemm_w4a16_combine_norm_kernel<<<dim3(rows), threads, 0, stream>>>(partial, y, N, (long long)rows * N, splits, residual,
-                                                                            (const _Float16*)norm->weight, (_Float16*)norm->out, norm->eps);
-    ART_LAUNCH_CHECK();
-    return 0;
+    gemm_w4a16_combine_norm_kernel<SPLITS><<<dim3(rows), threads, 0, stream>>>(partial, y, N, (long long)rows * N, splits, residual, (const _Float16*)norm->weight,
+                                                                                  (_Float16*)norm->out, norm->eps);
+  } else if (tail == kRope) {
+    gemm_w4a16_combine_rope_kernel<SPLITS><<<by_eight, 256, 0, stream>>>(partial, rows, splits, rope, make_div(N / 8));
+  } else if (tail == kSwiglu) {
+    gemm_w4a16_combine_swiglu_kernel<SPLITS><<<by_eight, 256, 0, stream>>>(partial, y, rows, N, splits, make_div(N / 8));
+  } else {
+    const long long count4 = (long long)rows * N / 4;
+    gemm_w4a16_combine_kernel<SPLITS><<<dim3((unsigned)((count4 + 255) / 256)), 256, 0, stream>>>(partial, y, count4, (long long)rows * N, splits, residual);
   }
-  if (tail == kRope) {
-    gemm_w4a16_combine_rope_kernel<<<dim3((unsigned)(((long long)rows * (N / 8) + 255) / 256)), 256, 0, stream>>>(partial, rows, splits, rope, make_div(N / 8));
-    ART_LAUNCH_CHECK();
-    return 0;
-  }
-  if (tail == kSwiglu) {
-    gemm_w4a16_combine_swiglu_kernel<<<dim3((unsigned)(((long long)rows * (N / 8) + 255) / 256)), 256, 0, stream>>>(partial, y, rows, N, splits, make_div(N / 8));
-    ART_LAUNCH_CHECK();
-    return 0;
-  }
-  const long long count4 = (long long)rows * N / 4;
-  gemm_w4a16_combine_kernel<<<dim3((unsigned)((count4 + 255) / 256)), 256, 0, stream>>>(partial, y, count4, (long long)rows * N, splits, residual);
+}
+int combine(const float* partial, _Float16* y, int rows, int N, int splits, const _Float16* residual, Tail tail, const Norm* norm, const Rope& rope,
+            hipStream_t stream) {
+  static const decltype(&launch_combine<0>) by_splits[9] = {launch_combine<0>, launch_combine<0>, launch_combine<2>, launch_combine<3>, launch_combine<4>,
+                                                            launch_combine<5>, launch_combine<6>, launch_combine<7>, launch_combine<8>};
+  by_splits[splits <= 8 ? splits : 0](partial, y, rows, N, splits, residual, tail, norm, rope, stream);
   ART_LAUNCH_CHECK();
   return 0;
 }

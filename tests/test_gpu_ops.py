@@ -593,6 +593,27 @@ def test_w4a16_gemm_with_swiglu_behind_it(autort, M, K, F):
     assert got.shape == (M, F) and np.allclose(got.float().cpu().numpy(), want, **FP16_TOL)
 
 
+# column tiles whose number is no multiple of eight times one, a few and more row blocks than XCDs; K-splits of every count that the pass behind
+# the product knows and one more
+@pytest.mark.parametrize('M,K,N', [(20, 384, 128 * 9), (300, 256, 128 * 15 + 16), (33 * 8 + 1, 128, 256 * 9 + 48), (70, 1280, 256 * 3)])
+def test_w4a16_gemm_blocks_that_are_dealt_to_all_xcds(autort, M, K, N):
+    from ctypes import c_void_p
+    from antares_amd.runtime import capi
+    from oracle import hot_ops
+    dev = autort.device()
+    p = workloads.w4_problem(K + N + M, M, K, N)
+    want = hot_ops.gemm_w4a16(p['x'].numpy(), p['qweight'].numpy(), p['scales'].numpy(), p['qzeros'].numpy()).astype(np.float32)
+    d = [p[k].to(dev) for k in ('x', 'qweight', 'scales', 'qzeros')]
+    for form in (1, 2, 5, 4, 8):
+        for splits in range(1, min(K // 128, 9) + 1):
+            note(f'w4a16 gemm M={M} K={K} N={N} form {form}, {splits} splits')
+            y = torch.full((M + 1, N), 7.0, dtype=torch.float16, device=dev)
+            capi.check(capi.lib().art_gemm_w4a16_tuned(*(c_void_p(t.data_ptr()) for t in d), c_void_p(y.data_ptr()), M, K, N, form * 256 + splits,
+                                                       c_void_p(torch.cuda.current_stream().cuda_stream)))
+            got = y.float().cpu().numpy()
+            assert np.allclose(got[:M], want, **FP16_TOL) and (got[M] == 7.0).all()
+
+
 # Every fp16 gate: one weight of a gate column is 1 (infinite gates: 2), one of its up column too.  The gate itself is exact; silu in float32
 # is less than 2^-22 off, the product with up and its rounding 2^-24 and 2^-11, or half of 2^-24 among the subnormal numbers.
 @pytest.mark.parametrize('code', [256 + 1, 512 + 1, 1280 + 1, 1024 + 1, 2048 + 1])
