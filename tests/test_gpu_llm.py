@@ -451,6 +451,7 @@ def test_the_q_k_v_product_that_rotates_and_stores(T, K, H):
     from antares_amd import workloads
     from antares_amd.runtime import capi
     dev, N, first = autort.device(), 3 * H * 128, 4
+    capi.init(0)
     p = workloads.w4_problem(T + K + H, T, K, N)
     d = [p[k].to(dev) for k in ('x', 'qweight', 'scales', 'qzeros')]
     half = (1.0 / (10000 ** (torch.arange(0, 128, 2).float() / 128))).half()

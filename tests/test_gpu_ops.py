@@ -601,6 +601,7 @@ def test_w4a16_gemm_blocks_that_are_dealt_to_all_xcds(autort, M, K, N):
     from antares_amd.runtime import capi
     from oracle import hot_ops
     dev = autort.device()
+    capi.init(0)
     p = workloads.w4_problem(K + N + M, M, K, N)
     want = hot_ops.gemm_w4a16(p['x'].numpy(), p['qweight'].numpy(), p['scales'].numpy(), p['qzeros'].numpy()).astype(np.float32)
     d = [p[k].to(dev) for k in ('x', 'qweight', 'scales', 'qzeros')]
@@ -621,6 +622,7 @@ def test_w4a16_gemm_with_swiglu_over_every_fp16_gate(autort, code):
     from ctypes import c_void_p
     from antares_amd.runtime import capi
     dev = autort.device()
+    capi.init(0)
     g = torch.arange(65536, dtype=torch.int32).to(torch.int16).view(torch.float16)
     g = torch.cat([g[torch.isfinite(g)], torch.tensor([40000.0, -40000.0, 60000.0, -60000.0], dtype=torch.float16)])
     F, M = 16, g.numel()
