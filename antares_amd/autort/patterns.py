@@ -226,7 +226,9 @@ def _tile_product(op, call, kind: int, a, b, c, M: int, N: int, K: int, large: b
         if rival is not None and rival['us'] <= saved['us']:
             return False
         value = int(saved['value'])
-        if lib.art_gemm_tile_form(kind, M, N, K, int(large), value >> 8, value & 255) == value and value >> 8:
+        # kept by another version of the library, it may have longer sums than are taken now
+        short_sums = lib.art_gemm_tile_form(kind, M, N, K, int(large), 0, 1) >> 8 == 4
+        if lib.art_gemm_tile_form(kind, M, N, K, int(large), value >> 8, value & 255) == value and value >> 8 and (value >> 8 == 4) == short_sums:
             code = value
     if not code:
         return False

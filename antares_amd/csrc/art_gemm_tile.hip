@@ -392,25 +392,31 @@ double large_time(int type, int M, int N, int K) {
   const double side = type == 0 ? 256 : 128, rounds = ceil(ceil(M / side) * ceil(N / side) / kUnits), million = 1e-6 * M * N;
   return type == 0 ? 5.26 + rounds * (0.0184 * K + 2.54) + 0.719 * million : 5.15 + rounds * 0.0601 * K + 0.655 * million;
 }
-// float32 products of few tiles, which the generic lowering sums on the vector units in short slices.
-bool fine(int type, int M, int N) { return type == 1 && (long long)((M + 63) / 64) * ((N + 63) / 64) < 16; }
+// Where the generic lowering has no matrix instructions for the product: it sums on the vector units.
+bool on_vector_units(int M, int N, int K) { return M < 32 || N < 32 || K < 32 || (long long)((M + 63) / 64) * ((N + 63) / 64) < 16; }
+// float32 there: short slices, 0.7e-7 to 1.6e-7 from 64 bits over 1100 sizes (M or N down to 1).  The chunk sums have 1.05e-7 to
+// 1.9e-7, above it for K of 64 to some 900 (7104 x 128 x 4 0.74e-7 and 1.14e-7, 1 x 637 x 10453 0.91 and 1.36); FINE is below it from
+// five values of k on (0.48e-7 to 0.73e-7; with four 0.41e-7, 3 % above).  Elsewhere the chunk sums are at or below it at all 1750.
+bool fine(int type, int M, int N, int K, bool large) { return type == 1 && !large && on_vector_units(M, N, K); }
 
-// 256 * form + slices for these sizes, or 0: another kernel is faster.  `large`: the kernel for large products takes them.
-int choose(int type, int M, int N, int K, bool large) {
-  if (!takes(type, M, N, K)) return 0;
+// 256 * form + slices for these sizes, or 0: another kernel is faster, or more exact.  `large`: the kernel for large products takes
+// them.  `own`: the best of the forms here, whatever the others take.
+int choose(int type, int M, int N, int K, bool large, bool own) {
+  if (!takes(type, M, N, K) || (type == 1 && K < 5)) return 0;
   const long long results = (long long)M * N;
   // The generic lowering keeps (times in us, generic / here): float16 from four rounds of 128 x 128 on (4000 x 4000 x 1000 62 / 69,
   // 4064 x 3856 x 400 42 / 38); float32 of a few thousand results and a short k, one launch without slices (66 x 87 x 70
   // 3.9 / 6.7, 64 x 192 x 192 7.6 / 7.3); int8 with aligned rows where the stores are most of it (2616 x 2048 x 64
   // 8.4 / 9.7, 4096 x 4096 x 512 27.4 / 28.0; 4096 x 4096 x 4096 106 / 98).
-  if (type == 0 && !large && (long long)((M + 127) / 128) * ((N + 127) / 128) >= 4 * kUnits) return 0;
-  if (type == 1 && results <= 8192 && K <= 256) return 0;
-  if (type == 2 && K % 16 == 0 && results * K >= 1LL << 26 && (K <= 64 || (K <= 512 && results >= 1LL << 24))) return 0;
+  if (type == 0 && !large && !own && (long long)((M + 127) / 128) * ((N + 127) / 128) >= 4 * kUnits) return 0;
+  if (type == 1 && !own && results <= 8192 && K <= 256) return 0;
+  if (type == 2 && !own && K % 16 == 0 && results * K >= 1LL << 26 && (K <= 64 || (K <= 512 && results >= 1LL << 24))) return 0;
   const int chunks = chunks_of(type, K);
-  double best = large ? large_time(type, M, N, K) : 1e30;
+  const bool short_sums = fine(type, M, N, K, large);
+  double best = large && !own ? large_time(type, M, N, K) : 1e30;
   int code = 0;
   for (int form = 1; form <= 4; ++form) {
-    if (!has(type, form) || (type == 1 && (form == 4) != fine(type, M, N))) continue;
+    if (!has(type, form) || (type == 1 && (form == 4) != short_sums)) continue;
     for (int splits : {1, 2, 3, 4, 5, 6, 8, 10, 12, 16, 24}) {
       if (splits > chunks || (splits > 1 && splits * results > 1LL << 26)) break;
       const double t = launch_time(type, M, N, K, form, splits);
@@ -461,7 +467,7 @@ int art::sum_slices(const float* partial, float* y, long long count, int slices,
 }
 
 extern "C" int art_gemm_tile_form(int type, int M, int N, int K, int large, int form, int splits) {
-  if (form == 0) return choose(type, M, N, K, large != 0);
+  if (form == 0) return choose(type, M, N, K, large != 0, splits != 0);
   return takes(type, M, N, K) && has(type, form) && splits >= 1 && splits <= 64 && splits <= chunks_of(type, K) ? 256 * form + splits : 0;
 }
 

@@ -258,7 +258,8 @@ int art_gemv_gptq(const void* x_dev, const void* qweight_dev, const void* scales
  * C[M,N] = A[M,K] @ B[N,K]^T from int8 to int32 (type 2), all row-major, any alignment of the elements' own, K and (types
  * 0 and 1) N of at least 16 bytes of elements (AntaresIR.md:115).
  *   art_gemm_tile_form: 256 * form + slices of k.  form == 0 asks for the library's choice (`large` != 0: art_gemm_f16 /
- *     art_gemm_f32 take these operands); 0 means that another kernel is faster, or that the sizes are not taken.  Otherwise
+ *     art_gemm_f32 take these operands); 0 means that another kernel is faster or more exact, or that the sizes are not taken.
+ *     form == 0 and slices == 1: the best form of this kernel, whatever the others take.  Otherwise
  *     the same code if art_gemm_tile takes it, else 0.  Forms: 1 = blocks of 64 x 64, 2 = 64 x 128, 3 = 128 x 128 (not float32),
  *     4 = 64 x 64 with short sums (float32 only).
  *   art_gemm_tile: partial_dev holds slices * M * N float32 (int32) values of any content, 16-byte aligned; it may be NULL for one slice. */

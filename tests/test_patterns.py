@@ -2,6 +2,7 @@
 import pytest
 import torch
 
+from antares_amd.autort import patterns
 from antares_amd.autort.op import ExportedOp
 from antares_amd.runtime import capi
 
@@ -66,3 +67,30 @@ def test_a_declared_result_too_small_for_the_program_is_refused(monkeypatch, spe
     op = ExportedOp(CONV, CONV_INPUTS + [spec], name='conv_room')
     with pytest.raises(Checked if fits else ValueError):
         op._call(None, *(GpuShaped(s) for s in ((4, 64, 28, 28), (64, 64, 3, 3), shape)))
+
+
+@pytest.mark.parametrize('K', [4, 5, 31, 32, 64, 512])
+def test_float32_products_on_the_vector_units_keep_short_sums(K):
+    """Where the generic lowering has no matrix instructions (its launch plan says so), its sums are short: the tile kernel takes such
+    a product with its short sums (form 4) or not at all, whatever an older module file has kept; elsewhere without them."""
+    lib = capi.lib()
+    op = ExportedOp(patterns.GEMM_F32_IR, patterns.GEMM_F32_INPUTS, name='gemm_thin')
+    plan, sizes = op.plans[0], (1, 8, 31, 32, 33, 63, 64, 65, 255, 1000, 4096, 16384)
+
+    class Codes(Launches):
+        def library(self, fn, *args):
+            self.taken.append(256 * args[-3] + args[-2])
+    for M in sizes:
+        for N in sizes[1:]:
+            own, code = lib.art_gemm_tile_form(1, M, N, K, 0, 0, 1), lib.art_gemm_tile_form(1, M, N, K, 0, 0, 0)
+            if K == 4:                                    # two products by themselves are no better than a chain of four
+                assert not own and not code
+                continue
+            short = plan._matrix_choice({'M': M, 'N': N, 'K': K})[0] is None
+            assert (own >> 8 == 4) == short and own >> 8 and code in (0, own), (M, N, K, own, code)
+            if M * N > 1 << 16:
+                continue
+            op.tuned = {f'gemm_tile.form|1,{M},{K},{N}': {'value': 256 * (1 if short else 4) + 1, 'us': 0.0}}
+            call = Codes()
+            op.fast_path(op, dict(a=torch.zeros(M, K), b=torch.zeros(K, N), c=torch.zeros(M, N)), {}, call)
+            assert call.taken == ([code] if code else []), (M, N, K)
