@@ -366,8 +366,9 @@ bool takes(int type, int M, int N, int K) {
 
 // What a launch takes, in microseconds: a fixed part; per chunk of a block's slice a time that grows with the blocks that
 // share a compute unit and with how unevenly they do; the stores; and for slices the second launch and the tiles between.
-// Fitted to 7000 launches (387 sizes of 64 to 4096 in M, N, K, odd ones among them): 5 % off, and the form and slices it
-// picks are 1.3 (float16), 1.0 (float32) and 0.7 % (int8) slower than the fastest ones in the mean.
+// Fitted to 7000 launches (387 sizes of 64 to 4096 in M, N, K, odd ones among them), 5 % off.  Over 1270 other sizes of that range the
+// form and slices it picks are 1.2 (float16), 0.5 (float32) and 0.4 % (int8) slower than the fastest ones in the mean, over 4260 outside
+// of it (M or N down to 1 and up to 16384, K of 4 to 16384) 1.4, 1.0 and 1.6 %.
 struct Cost { double fixed, alone, shared, uneven; };
 struct Rest { double sum, sum_bytes, store; };
 constexpr Cost kCost[3][3] = {{{3.67, 0.321, 0.210, 0.195}, {4.81, 0.494, 0.361, 0.272}, {6.17, 0.753, 0.439, 0.310}},
@@ -399,17 +400,51 @@ bool on_vector_units(int M, int N, int K) { return M < 32 || N < 32 || K < 32 ||
 // five values of k on (0.48e-7 to 0.73e-7; with four 0.41e-7, 3 % above).  Elsewhere the chunk sums are at or below it at all 1750.
 bool fine(int type, int M, int N, int K, bool large) { return type == 1 && !large && on_vector_units(M, N, K); }
 
+// The generic lowering's time on the vector units; elsewhere a time that nothing reaches (see `choose`).  Fitted to 3900
+// sizes, M and N of 1 to 16384, K of 4 to 16384, odd ones among them: where the two are within a factor of two of each other 6 to 17 %
+// off (25 % for float32 of 65536 and more results).  The kernel picked is 0.4 to 4.5 % slower than the faster one in the mean of a kind.
+double generic_time(int type, int M, int N, int K) {
+  const double million = 1e-6 * M * N, kk = K / 64.0;
+  if (on_vector_units(M, N, K)) {
+    // a thread per result, or per 4 x 4 of them; a wavefront per result, its k across the lanes; sums in two launches; a thread per
+    // result again.  Per launch, 64 values of k, million products, and million results (wavefronts: products, where a row of B is
+    // not one line: neighbouring k are then lines of their own).  us, generic / here:
+    // float16 24 x 61 x 446 3.9 / 6.2, 1088 x 24 x 192 8.5 / 4.3, 1440 x 56 x 24 3.3 / 4.0, 8 x 3968 x 1024 113 / 6.4; float32
+    // 64 x 6 x 832 3.5 / 8.9, 45 x 704 x 192 15.5 / 7.7, 5 x 9920 x 5376 1870 / 68; int8 920 x 1 x 370 3.1 / 4.6, 23 x 963 x 105 6.9 / 4.1.
+    struct Units { double fixed, k, products, rest; };
+    constexpr Units kShort[3] = {{2.459, 1.542, 0.212, 0.7}, {2.439, 1.6, 0.18, 1.307}, {2.412, 1.098, 0.205, 1.026}};
+    constexpr Units kPatch[2] = {{1.064, 9.852, 0.048, 0.728}, {2.099, 7.648, 0.058, 1.219}};
+    constexpr Units kWave[3] = {{2.928, 0.042, 0.91, 0.911}, {2.753, 0.053, 0.874, 1.287}, {3.024, 0.0, 0.869, 0.025}};
+    constexpr Units kSliced[3] = {{6.354, 0.0, 0.701, 1.325}, {3.698, 0.039, 0.605, 2.055}, {5.306, 0.016, 0.248, 0.0}};
+    constexpr Units kThread[2] = {{1.47, 1.61, 0.113, 8.452}, {0.345, 2.65, 0.191, 5.087}};
+    const double results = (double)M * N, line = (double)N * size_of(type) / 128, apart = million * K * (line < 1 ? line : 1);
+    auto time = [&](const Units& u, double rest) { return u.fixed + u.k * kk + u.products * million * K + u.rest * rest; };
+    if (K < 64) return type != 2 && results >= 131072 * 16 && M % 4 == 0 && N % 4 == 0 && K >= 8 ? time(kPatch[type], million) : time(kShort[type], million);
+    if (type != 2 && results >= 65536) return time(kThread[type], million);
+    if (K < 1024 || results > 8192) return time(kWave[type], apart);
+    // a long k and hardly any results: float32 72 x 8 x 16352 23 / 31, int8 31 x 2 x 6301 4.2 / 8.8, in the mean 1.9 and 1.2 times as fast
+    // there; float16 here where the estimate, 17 % off, is a fifth below: 8 x 128 x 7904 31 / 7.6, 47 x 9 x 4106 4.3 / 11.7
+    if (results > 1024) return time(kSliced[type], apart);
+    return type == 0 ? time({4.345, 0.006, 0.619, 1.204}, apart) : 0.0;
+  }
+  return 1e30;
+}
+
+// What a block's columns past a row's last whole vector cost, per chunk: they are shifted on their way into LDS.  For all columns of a
+// thin product, 0.18 us between rows of whole vectors and others in float16, 0.19 in float32.  Not part of the choice of slices.
+double ragged_time(int type, int N, int K, int splits) {
+  return type == 2 || N % (16 / size_of(type)) == 0 ? 0.0 : 0.12 * ((chunks_of(type, K) + splits - 1) / splits);
+}
+
 // 256 * form + slices for these sizes, or 0: another kernel is faster, or more exact.  `large`: the kernel for large products takes
 // them.  `own`: the best of the forms here, whatever the others take.
 int choose(int type, int M, int N, int K, bool large, bool own) {
   if (!takes(type, M, N, K) || (type == 1 && K < 5)) return 0;
   const long long results = (long long)M * N;
   // The generic lowering keeps (times in us, generic / here): float16 from four rounds of 128 x 128 on (4000 x 4000 x 1000 62 / 69,
-  // 4064 x 3856 x 400 42 / 38); float32 of a few thousand results and a short k, one launch without slices (66 x 87 x 70
-  // 3.9 / 6.7, 64 x 192 x 192 7.6 / 7.3); int8 with aligned rows where the stores are most of it (2616 x 2048 x 64
+  // 4064 x 3856 x 400 42 / 38); int8 with aligned rows where the stores are most of it (2616 x 2048 x 64
   // 8.4 / 9.7, 4096 x 4096 x 512 27.4 / 28.0; 4096 x 4096 x 4096 106 / 98).
   if (type == 0 && !large && !own && (long long)((M + 127) / 128) * ((N + 127) / 128) >= 4 * kUnits) return 0;
-  if (type == 1 && !own && results <= 8192 && K <= 256) return 0;
   if (type == 2 && !own && K % 16 == 0 && results * K >= 1LL << 26 && (K <= 64 || (K <= 512 && results >= 1LL << 24))) return 0;
   const int chunks = chunks_of(type, K);
   const bool short_sums = fine(type, M, N, K, large);
@@ -423,7 +458,7 @@ int choose(int type, int M, int N, int K, bool large, bool own) {
       if (t < best) { best = t; code = 256 * form + splits; }
     }
   }
-  return code;
+  return own || large || best + ragged_time(type, N, K, code & 255) < generic_time(type, M, N, K) ? code : 0;
 }
 
 template <typename T, bool BT, int TM, int TN, bool FINE = false>

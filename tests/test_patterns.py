@@ -94,3 +94,12 @@ def test_float32_products_on_the_vector_units_keep_short_sums(K):
             call = Codes()
             op.fast_path(op, dict(a=torch.zeros(M, K), b=torch.zeros(K, N), c=torch.zeros(M, N)), {}, call)
             assert call.taken == ([code] if code else []), (M, N, K)
+
+
+@pytest.mark.parametrize('kind,M,N,K,generic,here', [
+    (0, 24, 61, 446, 3.9, 6.2), (0, 1440, 56, 24, 3.3, 4.0), (0, 47, 9, 4106, 4.3, 11.7), (0, 1088, 24, 192, 8.5, 4.3), (0, 8, 3968, 1024, 113, 6.4),
+    (0, 8, 128, 7904, 31, 7.6), (1, 64, 6, 832, 3.5, 8.9), (1, 72, 8, 16352, 23, 31), (1, 1216, 4992, 8, 8.5, 12.9), (1, 45, 704, 192, 15.5, 7.7),
+    (1, 5, 9920, 5376, 1870, 68), (2, 920, 1, 370, 3.1, 4.6), (2, 31, 2, 6301, 4.2, 8.8), (2, 23, 963, 105, 6.9, 4.1)])
+def test_thin_products_go_to_the_kernel_that_was_measured_to_be_faster(kind, M, N, K, generic, here):
+    """One of each kind of kernel that the generic lowering has without matrix instructions; times in us on an MI355X."""
+    assert bool(capi.lib().art_gemm_tile_form(kind, M, N, K, 0, 0, 0)) == (here < generic)
