@@ -400,9 +400,10 @@ bool on_vector_units(int M, int N, int K) { return M < 32 || N < 32 || K < 32 ||
 // five values of k on (0.48e-7 to 0.73e-7; with four 0.41e-7, 3 % above).  Elsewhere the chunk sums are at or below it at all 1750.
 bool fine(int type, int M, int N, int K, bool large) { return type == 1 && !large && on_vector_units(M, N, K); }
 
-// The generic lowering's time on the vector units; elsewhere a time that nothing reaches (see `choose`).  Fitted to 3900
-// sizes, M and N of 1 to 16384, K of 4 to 16384, odd ones among them: where the two are within a factor of two of each other 6 to 17 %
-// off (25 % for float32 of 65536 and more results).  The kernel picked is 0.4 to 4.5 % slower than the faster one in the mean of a kind.
+// The generic lowering's time, on the vector units and on the matrix instructions, or a time that nothing reaches where it was not
+// the faster one.  Fitted to 4400 sizes, M and N of 1 to 16384, K of 4 to 16384, odd ones among them: where the two are within a factor of
+// two of each other 6 to 17 % off (25 % for float32 of 65536 and more results).  The kernel picked is 0.4 to 4.5 % slower than the
+// faster one in the mean of a kind.
 double generic_time(int type, int M, int N, int K) {
   const double million = 1e-6 * M * N, kk = K / 64.0;
   if (on_vector_units(M, N, K)) {
@@ -427,7 +428,20 @@ double generic_time(int type, int M, int N, int K) {
     if (results > 1024) return time(kSliced[type], apart);
     return type == 0 ? time({4.345, 0.006, 0.619, 1.204}, apart) : 0.0;
   }
-  return 1e30;
+  // Operands that the matrix kernels fetch in whole vectors and results that leave in whole lines; elsewhere, and in float32, they are 5 %
+  // faster at the most (int8 1472 x 1216 x 41: 10) and up to 2.9 times slower (int8 5369 x 3613 x 80 55 / 19, float16 7212 x 8134 x 615 390 / 175).
+  if (type == 1 || K % (16 / size_of(type)) != 0 || N % (type == 0 ? 8 : 16) != 0) return 1e30;
+  // Blocks of 128 x 128 or 64 x 64 as it chooses them (plans.py); taken where it is a tenth faster by this estimate, 9 % off.  us,
+  // generic / here: float16 4672 x 4992 x 32 20.4 / 24.9, 2216 x 7464 x 216 41.1 / 33.6; int8 4608 x 15168 x 64 56 / 66, 2176 x 2880 x 32
+  // 8.3 / 9.4, 3392 x 1664 x 192 9.8 / 10.0, 4096 x 4096 x 4096 106 / 98.  0.5 to 2.3 % off the faster one in the mean, at single sizes up to
+  // 16 % slower than it (int8 5952 x 1088 x 320 10.6 / 12.2).
+  constexpr Cost kMatrix[2][2] = {{{3.9, 0.588, 0.091, 0.34}, {5.562, 0.895, 0.945, 0.332}}, {{4.236, 0.209, 0.169, 0.264}, {4.462, 0.507, 0.449, 0.15}}};
+  constexpr double kStore[2][2] = {{0.443, 0.694}, {0.395, 0.701}};
+  const long long big = (long long)((M + 127) / 128) * ((N + 127) / 128), small = (long long)((M + 63) / 64) * ((N + 63) / 64);
+  const int side = small < 700 * ((big + 511) / 512) ? 0 : 1;
+  const Cost& c = kMatrix[type / 2][side];
+  const double rounds = (double)(side ? big : small) / kUnits, full = rounds > 1 ? rounds : 1;
+  return 1.1 * (c.fixed + kk * (c.alone + c.shared * (full - 1) + c.uneven * (ceil(rounds) - full)) + kStore[type / 2][side] * million);
 }
 
 // What a block's columns past a row's last whole vector cost, per chunk: they are shifted on their way into LDS.  For all columns of a
@@ -441,14 +455,9 @@ double ragged_time(int type, int N, int K, int splits) {
 int choose(int type, int M, int N, int K, bool large, bool own) {
   if (!takes(type, M, N, K) || (type == 1 && K < 5)) return 0;
   const long long results = (long long)M * N;
-  // The generic lowering keeps (times in us, generic / here): float16 from four rounds of 128 x 128 on (4000 x 4000 x 1000 62 / 69,
-  // 4064 x 3856 x 400 42 / 38); int8 with aligned rows where the stores are most of it (2616 x 2048 x 64
-  // 8.4 / 9.7, 4096 x 4096 x 512 27.4 / 28.0; 4096 x 4096 x 4096 106 / 98).
-  if (type == 0 && !large && !own && (long long)((M + 127) / 128) * ((N + 127) / 128) >= 4 * kUnits) return 0;
-  if (type == 2 && !own && K % 16 == 0 && results * K >= 1LL << 26 && (K <= 64 || (K <= 512 && results >= 1LL << 24))) return 0;
   const int chunks = chunks_of(type, K);
   const bool short_sums = fine(type, M, N, K, large);
-  double best = large && !own ? large_time(type, M, N, K) : 1e30;
+  double best = 1e30;
   int code = 0;
   for (int form = 1; form <= 4; ++form) {
     if (!has(type, form) || (type == 1 && (form == 4) != short_sums)) continue;
@@ -458,7 +467,9 @@ int choose(int type, int M, int N, int K, bool large, bool own) {
       if (t < best) { best = t; code = 256 * form + splits; }
     }
   }
-  return own || large || best + ragged_time(type, N, K, code & 255) < generic_time(type, M, N, K) ? code : 0;
+  if (own) return code;
+  if (large) return best < large_time(type, M, N, K) ? code : 0;
+  return best + ragged_time(type, N, K, code & 255) < generic_time(type, M, N, K) ? code : 0;
 }
 
 template <typename T, bool BT, int TM, int TN, bool FINE = false>

@@ -185,7 +185,9 @@ def test_tile_products_of_every_form(dtype, M, N, chunks, rest):
                                          ('float32', 192, 576, 192), ('float32', 70, 420, 268), ('int8', 232, 120, 1448), ('int8', 112, 3568, 72),
                                          # thin or short: the generic kernels sum on the vector units however many tiles there are
                                          ('float32', 16, 2048, 512), ('float32', 8, 4096, 256), ('float32', 3, 4096, 512), ('float32', 20000, 24, 130),
-                                         ('float32', 900, 1200, 28)])
+                                         ('float32', 900, 1200, 28),
+                                         # large, with rows that are not whole vectors
+                                         ('float16', 2100, 8001, 70), ('int8', 4097, 4099, 80)])
 def test_small_products_take_the_tile_kernel_and_agree_with_the_generic_kernels(dtype, M, N, K):
     """The route of an exported program: the call goes to `art_gemm_tile`, agrees with the generic kernels (int8 bit for bit), and
     in float32 is no further from the 64-bit product than they are."""

@@ -103,3 +103,11 @@ def test_float32_products_on_the_vector_units_keep_short_sums(K):
 def test_thin_products_go_to_the_kernel_that_was_measured_to_be_faster(kind, M, N, K, generic, here):
     """One of each kind of kernel that the generic lowering has without matrix instructions; times in us on an MI355X."""
     assert bool(capi.lib().art_gemm_tile_form(kind, M, N, K, 0, 0, 0)) == (here < generic)
+
+
+@pytest.mark.parametrize('kind,M,N,K,generic,here', [
+    (0, 4672, 4992, 32, 20.4, 24.9), (0, 2216, 7464, 216, 41.1, 33.6), (0, 7212, 8134, 615, 390, 175), (0, 2028, 15937, 171, 102, 53),
+    (2, 4608, 15168, 64, 56, 66), (2, 1856, 3456, 48, 8.2, 9.8), (2, 5369, 3613, 80, 55, 19), (2, 3592, 15416, 48, 114, 42), (2, 4096, 4096, 4096, 106, 98)])
+def test_products_that_are_mostly_stores_go_to_the_kernel_that_was_measured_to_be_faster(kind, M, N, K, generic, here):
+    """Whole vectors of k and whole lines of results: the generic kernels on the matrix instructions; odd ones: the tile kernel."""
+    assert bool(capi.lib().art_gemm_tile_form(kind, M, N, K, 0, 0, 0)) == (here < generic)
