@@ -490,12 +490,11 @@ def _conv2d_handler(st, axes, window):
         saved = op.tuned.get(key)
         trials = op.config.get('tune')
         if saved is None and isinstance(trials, int) and trials > 0 and not torch.cuda.is_current_stream_capturing():
-            # a float32 form with longer sums than the library's choice is not tried
-            others = [v for v in (1, 2, 3, 4, 5, 6) + tuple(k + 256 * s for k in (4, 5, 6, 7) for s in (2, 3, 4, 6, 8)) if (form & 255 == 7) == (v & 255 == 7)]
-            forms = [form] + [v for v in others if v != form and lib.art_conv2d_form(*shape, v)]
+            others = (1, 2, 3, 4, 5, 6) + tuple(k + 256 * s for k in (4, 5, 6, 7) for s in (2, 3, 4, 6, 8))
+            forms = [form] + [v for v in others if v != form and lib.art_conv2d_exact_enough(*shape, v)]
             forms = forms[:trials]
             saved = tune_hand_kernel(op, key, forms, run, len(forms), [(x, w, scratch(forms), torch.empty_like(y))])
-        if saved is not None and lib.art_conv2d_form(*shape, int(saved['value'])):
+        if saved is not None and lib.art_conv2d_exact_enough(*shape, int(saved['value'])):
             form = int(saved['value'])
         call.library(lib.art_conv2d, x, w, scratch([form]), y, *shape, form, STREAM)
         return True

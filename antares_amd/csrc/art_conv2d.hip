@@ -306,6 +306,19 @@ double staged_time(const Geometry& g, int f16, int form, int slices) {
   return slices == 1 ? t + r.store * megabytes : t + r.sum + r.sum_bytes * (slices + 1) * megabytes;
 }
 
+// Where the generic lowering has no matrix instructions for the convolution: it sums on the vector units.
+bool on_vector_units(const Geometry& g) { return g.F < 32 || g.columns < 32 || 9 * g.C < 32 || blocks_of(g, 1) < 16; }
+
+// Whether a form's sums are no longer than those of the generic kernels that it takes the place of.  On the vector units those are
+// short: float32 form 7 only, float16 the blocks of 64 x 64, whose rows of taps are summed by themselves;
+// one channel is a chain of nine there.  Elsewhere float16 with fewer than 32 channels that are not 8 or 16 and so on: the larger blocks sum 18 instructions in a row where
+// the generic kernels need 9 C / 16 (5 to 31 channels 1.02 to 1.22 times their error, the blocks of 64 x 64 0.66 to 1.01
+// times; with four channels both are above it).
+bool exact_enough(const Geometry& g, int f16, int form) {
+  if (on_vector_units(g)) return g.C > 1 && (f16 ? shape_of(form) == 1 : (form & 255) == 7);
+  return !f16 || (g.C > 4 && shape_of(form) == 1) || g.C >= 32 || g.C % 8 == 0;
+}
+
 // The form for these sizes, or 0: the generic kernels are faster or sum more exactly there.  Lines from sweeps of the sizes
 // above, times in us generic / here.
 //  * fewer than 32 features, or fewer than 16 blocks of 64 x 64: the generic path sums on the vector units in short
@@ -319,16 +332,15 @@ double staged_time(const Geometry& g, int f16, int form, int slices) {
 //    17 x 17, 46 without slices), float16 19 / 13.8 (9 x 240 -> 104, 13 x 13).  The image is staged unless it is large and
 //    there is little to multiply: float16 18 x 64 -> 48, 51 x 51 15.3 gathered, 16.8 staged, 1 x 40 -> 152, 42 x 42 10.0 and 9.0.
 int choose(const Geometry& g, int f16) {
-  const long long small = blocks_of(g, 1), results = (long long)g.columns * g.F;
-  const bool vector_units = g.F < 32 || small < 16;
+  const long long results = (long long)g.columns * g.F;
+  const bool vector_units = on_vector_units(g);
   int best = 0;
   double t_best = !vector_units ? 1e30 : (f16 ? 5.3 : 5.5) + (f16 ? 1.3e-6 : 1.1e-6) * results * 9 * g.C;
   auto consider = [&](int form, double t) {
     if (t < t_best && fits(g, f16, form)) { best = form; t_best = t; }
   };
   for (int form = 1; form <= 7; ++form) {
-    if (form == 7 ? f16 || !vector_units : !f16 && vector_units) continue;
-    if (shape_of(form) != 1 && vector_units) continue;
+    if (!exact_enough(g, f16, form) || (form == 7 && (f16 || !vector_units))) continue;
     if (form <= 3) consider(form, launch_time(g, f16, form));
     for (int slices : {1, 2, 3, 4, 5, 6, 8, 12})
       if (form > 3 && slices <= g.chunks && (slices == 1 || slices * blocks_of(g, form) <= 4 * kUnits)) consider(form + (slices > 1 ? 256 * slices : 0), staged_time(g, f16, form, slices));
@@ -373,6 +385,11 @@ extern "C" int art_conv2d_form(int f16, int N, int C, int H, int W, int F, int H
   Geometry g;
   if (!geometry(g, f16, N, C, H, W, F, HO, WO, ph, pw)) return 0;
   return form ? (fits(g, f16, form) ? form : 0) : choose_gathered(g, f16);
+}
+
+extern "C" int art_conv2d_exact_enough(int f16, int N, int C, int H, int W, int F, int HO, int WO, int ph, int pw, int form) {
+  Geometry g;
+  return geometry(g, f16, N, C, H, W, F, HO, WO, ph, pw) && fits(g, f16, form) && exact_enough(g, f16, form);
 }
 
 extern "C" int art_conv2d_choose(int f16, int N, int C, int H, int W, int F, int HO, int WO, int ph, int pw) {

@@ -1406,6 +1406,25 @@ def test_staged_convolutions_are_no_further_from_float64_than_the_generic_kernel
     assert off[0] <= 1.05 * off[1], off
 
 
+@pytest.mark.parametrize('dtype,n,c,f,hw', [('float16', 9, 9, 200, 49), ('float16', 17, 25, 88, 29), ('float16', 4, 4, 96, 40), ('float32', 5, 24, 2424, 2),
+                                            ('float32', 1, 208, 1160, 4), ('float32', 8, 3, 64, 40)])
+def test_convolutions_of_few_channels_or_points_are_no_further_from_float64_than_the_generic_kernels(autort, dtype, n, c, f, hw):
+    """Whichever kernel takes them: the generic sums are short here, on the vector units or over less than a chunk of channels."""
+    note(f'convolution of few channels or points {dtype} {n}x{c}x{hw}x{hw} -> {f}')
+    dev, dt = autort.device(), getattr(torch, dtype)
+    g = torch.Generator().manual_seed(n * c + f)
+    x, w = torch.randn(n, c, hw, hw, generator=g).to(dt), torch.randn(f, c, 3, 3, generator=g).to(dt)
+    want = torch.nn.functional.conv2d(x.double(), w.double(), padding=1)
+    off = []
+    for generic in (False, True):
+        op = autort.export(ir=conv_program(dtype, (hw, hw), (hw, hw), (1, 1)),
+                           inputs=[f'input0={dtype}[N:{n}, C:{c}, H:{hw}, W:{hw}]', f'input1={dtype}[F:{f}, C:{c}, KH:3, KW:3]'], name=f'conv_few_{dtype}_{n}_{c}_{int(generic)}')
+        if generic:
+            op.fast_path = None
+        off.append(float((op(x.to(dev), w.to(dev)).cpu().double() - want).norm() / want.norm()))
+    assert off[0] <= 1.05 * off[1], off
+
+
 @pytest.mark.parametrize('dtype,n,c,f,hw', [('float16', 4, 40, 72, 20), ('float16', 2, 64, 24, 23), ('float32', 5, 20, 72, 21), ('float16', 30, 16, 256, 28)])
 def test_convolution_operator_takes_the_kernel_and_agrees_with_the_generic_one(autort, dtype, n, c, f, hw):
     note(f'convolution operator {dtype} {n}x{c}x{hw}x{hw} -> {f}')

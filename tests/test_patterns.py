@@ -111,3 +111,45 @@ def test_thin_products_go_to_the_kernel_that_was_measured_to_be_faster(kind, M, 
 def test_products_that_are_mostly_stores_go_to_the_kernel_that_was_measured_to_be_faster(kind, M, N, K, generic, here):
     """Whole vectors of k and whole lines of results: the generic kernels on the matrix instructions; odd ones: the tile kernel."""
     assert bool(capi.lib().art_gemm_tile_form(kind, M, N, K, 0, 0, 0)) == (here < generic)
+
+
+@pytest.mark.parametrize('f16', [0, 1])
+def test_convolutions_are_taken_by_forms_whose_sums_are_no_longer_than_the_generic_ones(f16):
+    """Where the generic lowering has no matrix instructions (its launch plan says so): float32 form 7, float16 blocks of 64 x 64.
+    Elsewhere float16 with less than a chunk of channels, not whole eighths of them: blocks of 64 x 64.  Also for a form that a module
+    file has kept."""
+    lib, dtype = capi.lib(), 'float16' if f16 else 'float32'
+    cast = '.to(`float32`)' if f16 else ''
+    for n, c, hw, f in ((1, 16, 40, 31), (2, 1, 20, 64), (8, 3, 40, 64), (5, 24, 2, 2424), (1, 208, 4, 1160), (3, 32, 7, 32), (9, 9, 28, 200), (4, 4, 30, 96),
+                        (10, 11, 51, 146), (17, 25, 29, 88), (6, 24, 28, 96), (4, 16, 30, 64), (32, 128, 28, 128), (3, 40, 3, 1040)):
+        shape = (f16, n, c, hw, hw, f, hw, hw, 1, 1)
+        op = ExportedOp(f'o[N, F, HO, WO] +=! x[N, C, HO + KH, WO + KW]{cast} * w[F, C, KH, KW]{cast} where HO in {hw}, WO in {hw}',
+                        [f'x={dtype}[N:{n}, C:{c}, H:{hw + 2}, W:{hw + 2}]', f'w={dtype}[F:{f}, C:{c}, KH:3, KW:3]'], name=f'conv_sums_{f16}')
+        env = op.fused.bind_dims({'x': (n, c, hw + 2, hw + 2), 'w': (f, c, 3, 3)})
+        vector = op.plans[0]._matrix_choice(env)[0] is None
+        allowed = [v for v in range(1, 8) if lib.art_conv2d_exact_enough(*shape, v)]
+        if vector:
+            assert allowed == ([] if c == 1 else [1, 4] if f16 else [7]), (shape, allowed)
+        elif f16 and c < 32 and c % 8:
+            assert allowed == ([1, 4] if c > 4 else []), (shape, allowed)
+        else:
+            assert set(allowed) >= {1, 2, 3, 4, 5, 6}, (shape, allowed)
+        choice = lib.art_conv2d_choose(*shape)
+        assert not choice or (choice & 255) in allowed, (shape, choice, allowed)
+
+
+def test_a_kept_convolution_form_with_longer_sums_is_not_used():
+    class Codes(Launches):
+        def library(self, fn, *args):
+            self.taken.append(args[-2])
+    n, c, hw, f = 17, 25, 29, 88
+    ir = CONV.replace('28', str(hw)).replace('input0[N, C, HO + KH - 1, WO + KW - 1]', 'input0[N, C, HO + KH - 1, WO + KW - 1].to(`float32`)') \
+        .replace('input1[F, C, KH, KW]', 'input1[F, C, KH, KW].to(`float32`)')
+    op = ExportedOp(ir, [f'input0=float16[N:{n}, C:{c}, H:{hw}, W:{hw}]', f'input1=float16[F:{f}, C:{c}, KH:3, KW:3]'], name='conv_kept')
+    bound = {'input0': torch.zeros(n, c, hw, hw).half(), 'input1': torch.zeros(f, c, 3, 3).half(), 'output0': torch.zeros(n, f, hw, hw)}
+    env = op.fused.bind_dims({k: tuple(v.shape) for k, v in bound.items()})
+    choice = capi.lib().art_conv2d_choose(1, n, c, hw, hw, f, hw, hw, 1, 1)
+    for kept, used in ((5, choice), (1, 1)):
+        op.tuned = {f'conv2d.form|1,{n},{c},{hw},{hw},{f},{hw},{hw},1,1': {'value': kept, 'us': 0.0}}
+        call = Codes()
+        assert op.fast_path(op, bound, env, call) and call.taken == [used]
