@@ -309,13 +309,14 @@ double staged_time(const Geometry& g, int f16, int form, int slices) {
 // Where the generic lowering has no matrix instructions for the convolution: it sums on the vector units.
 bool on_vector_units(const Geometry& g) { return g.F < 32 || g.columns < 32 || 9 * g.C < 32 || blocks_of(g, 1) < 16; }
 
-// Whether a form's sums are no longer than those of the generic kernels that it takes the place of.  On the vector units those are
-// short: float32 form 7 only, float16 the blocks of 64 x 64, whose rows of taps are summed by themselves;
-// one channel is a chain of nine there.  Elsewhere float16 with fewer than 32 channels that are not 8 or 16 and so on: the larger blocks sum 18 instructions in a row where
+// Whether a form's sums are no longer than those of the generic kernels that it takes the place of.  On the vector units 64 terms and
+// more are spread over a wavefront: float32 form 7 only, float16 the blocks of 64 x 64, whose rows of taps are summed by themselves.
+// Fewer terms are a chain there: these blocks have 0.42 to 0.93 times its error.
+// Elsewhere float16 with fewer than 32 channels that are not 8 or 16 and so on: the larger blocks sum 18 instructions in a row where
 // the generic kernels need 9 C / 16 (5 to 31 channels 1.02 to 1.22 times their error, the blocks of 64 x 64 0.66 to 1.01
 // times; with four channels both are above it).
 bool exact_enough(const Geometry& g, int f16, int form) {
-  if (on_vector_units(g)) return g.C > 1 && (f16 ? shape_of(form) == 1 : (form & 255) == 7);
+  if (on_vector_units(g)) return f16 || 9 * g.C < 64 ? shape_of(form) == 1 : (form & 255) == 7;
   return !f16 || (g.C > 4 && shape_of(form) == 1) || g.C >= 32 || g.C % 8 == 0;
 }
 

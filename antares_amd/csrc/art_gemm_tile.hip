@@ -395,10 +395,12 @@ double large_time(int type, int M, int N, int K) {
 }
 // Where the generic lowering has no matrix instructions for the product: it sums on the vector units.
 bool on_vector_units(int M, int N, int K) { return M < 32 || N < 32 || K < 32 || (long long)((M + 63) / 64) * ((N + 63) / 64) < 16; }
-// float32 there: short slices, 0.7e-7 to 1.6e-7 from 64 bits over 1100 sizes (M or N down to 1).  The chunk sums have 1.05e-7 to
-// 1.9e-7, above it for K of 64 to some 900 (7104 x 128 x 4 0.74e-7 and 1.14e-7, 1 x 637 x 10453 0.91 and 1.36); FINE is below it from
-// five values of k on (0.48e-7 to 0.73e-7; with four 0.41e-7, 3 % above).  Elsewhere the chunk sums are at or below it at all 1750.
-bool fine(int type, int M, int N, int K, bool large) { return type == 1 && !large && on_vector_units(M, N, K); }
+// Float32 products whose k is spread over a wavefront or a block there: from 64 values of k on, below 65536 results.  Their sums are
+// 0.7e-7 to 1.6e-7 from 64 bits over 1100 sizes (M or N down to 1); the chunk sums have 1.05e-7 to 1.9e-7, above it for K of 64 to some 900
+// (7104 x 4 x 128 0.74e-7 and 1.14e-7, 1 x 10453 x 637 0.91 and 1.36), FINE 0.64e-7 to 0.73e-7.  A thread for each result is a chain over k:
+// the chunk sums have its error up to 32 values of k and less from there on (0.44 times with 65536 and more results).  On the matrix
+// instructions they are at or below it at all 1750 sizes.
+bool fine(int type, int M, int N, int K, bool large) { return type == 1 && !large && on_vector_units(M, N, K) && K >= 64 && (long long)M * N < 65536; }
 
 // The generic lowering's time, on the vector units and on the matrix instructions, or a time that nothing reaches where it was not
 // the faster one.  Fitted to 4400 sizes, M and N of 1 to 16384, K of 4 to 16384, odd ones among them: where the two are within a factor of
@@ -450,10 +452,10 @@ double ragged_time(int type, int N, int K, int splits) {
   return type == 2 || N % (16 / size_of(type)) == 0 ? 0.0 : 0.12 * ((chunks_of(type, K) + splits - 1) / splits);
 }
 
-// 256 * form + slices for these sizes, or 0: another kernel is faster, or more exact.  `large`: the kernel for large products takes
+// 256 * form + slices for these sizes, or 0: another kernel is faster.  `large`: the kernel for large products takes
 // them.  `own`: the best of the forms here, whatever the others take.
 int choose(int type, int M, int N, int K, bool large, bool own) {
-  if (!takes(type, M, N, K) || (type == 1 && K < 5)) return 0;
+  if (!takes(type, M, N, K)) return 0;
   const long long results = (long long)M * N;
   const int chunks = chunks_of(type, K);
   const bool short_sums = fine(type, M, N, K, large);
