@@ -320,23 +320,60 @@ bool exact_enough(const Geometry& g, int f16, int form) {
   return !f16 || (g.C > 4 && shape_of(form) == 1) || g.C >= 32 || g.C % 8 == 0;
 }
 
-// The form for these sizes, or 0: the generic kernels are faster or sum more exactly there.  Lines from sweeps of the sizes
-// above, times in us generic / here.
-//  * fewer than 32 features, or fewer than 16 blocks of 64 x 64: the generic path sums on the vector units in short
-//    chains.  In float32 that error (0.73e-7 to 1.26e-7 against 64 bits) is below the matrix instructions' (1.2e-7 to 1.5e-7), not
-//    below that of the short sums (0.69e-7 to 0.76e-7): form 7 only.  In float16 it is that of the blocks of 64 x 64, whose rows of
-//    taps are summed by themselves (0.69e-7 to 1.1e-7 there, 0.62e-7 to 0.87e-7 here; the larger blocks have 1.2e-7).  Where it is
-//    faster than 5.5 us + 1.1 ps per product there (float16 5.3 us + 1.3 ps): float32 375 / 37 (2 x 232 -> 24, 52 x 52), 57 / 16
-//    (3 x 184 -> 48, 14 x 14), 7.6 / 13.7 (1 x 24 -> 32, 15 x 15); float16 319 / 19 (28 x 40 -> 16, 42 x 42), 16.7 / 8.1 (4 x 48 -> 16,
-//    20 x 20), 5.6 / 7.0 (1 x 16 -> 40, 7 x 7).
-//  * elsewhere one of the forms wins, with the channels sliced where there are few blocks: float32 23 / 20 (9 x 216 -> 64,
-//    17 x 17, 46 without slices), float16 19 / 13.8 (9 x 240 -> 104, 13 x 13).  The image is staged unless it is large and
-//    there is little to multiply: float16 18 x 64 -> 48, 51 x 51 15.3 gathered, 16.8 staged, 1 x 40 -> 152, 42 x 42 10.0 and 9.0.
+// What comes on top of these times outside of the sizes they were fitted to: a filter of more than 256 x 256 is packed for longer, and
+// each further round of blocks over the staged image has a ramp of its own.  With it they are 6 (float32) and 10 % (float16) off over 530
+// such sizes (10 and 21 without); the forms picked are 0.2 to 1.5 % slower than the fastest either way, so it is no part of the picking.
+double outside_time(const Geometry& g, int f16, int form) {
+  const double filter = 1e-6 * art_conv2d_packed_bytes(f16, g.C, g.F), most = f16 ? 1.2 : 2.4, rounds = (double)blocks_of(g, form) * slices_of(form) / kUnits;
+  return (filter > most ? (f16 ? 2.547 : 1.749) * (filter - most) : 0.0) + ((form & 255) > 3 && rounds > 1 ? (f16 ? 1.584 : 0.811) * (rounds - 1) : 0.0);
+}
+
+// What the generic kernels take, in microseconds, 6 to 16 % off where the two are close.  On the vector units a thread or a wavefront per
+// result, or, for many results, a thread per 4 x 4 or 4 x 2 of them.  On the matrix instructions a padded copy of the image and blocks of
+// 128 x 128 or 64 x 64 as it chooses them (plans.py), from 1024 terms on in slices where they are few.  us, generic / here:
+//   float32 2 x 232 -> 24, 52 x 52 375 / 37; 1 x 24 -> 32, 15 x 15 7.6 / 13.7; 58 x 12 -> 4, 158 x 158 82 / 621; 205 x 40 -> 24, 33 x 33
+//   6457 / 213; 7 x 34 -> 4058, 6 x 6 17 / 25; 6 x 9 -> 294, 76 x 76 39 / 50; 9 x 216 -> 64, 17 x 17 23 / 20;
+//   float16 28 x 40 -> 16, 42 x 42 319 / 19; 1 x 16 -> 40, 7 x 7 5.6 / 7.0; 63 x 20 -> 4, 90 x 90 59 / 107; 2 x 65 -> 2887, 8 x 8 13.5 / 17.7;
+//   9 x 240 -> 104, 13 x 13 19 / 13.8.
+double generic_time(const Geometry& g, int f16) {
+  const double results = 1e-6 * g.columns * g.F, products = results * 9 * g.C, image = 1e-6 * g.N * g.C * g.H * g.W;
+  if (on_vector_units(g)) {
+    const bool patches = g.F % 4 == 0 && g.WO % 2 == 0 && (double)g.columns * g.F >= 131072.0 * (g.WO % 4 == 0 ? 16 : 8);
+    return patches ? (f16 ? 11.36 + 0.094 * products + 1.507 * image : 11.63 + 0.064 * products + 1.611 * image)
+                   : (f16 ? 5.3 + 1.3 * products : 5.5 + 1.1 * products);
+  }
+  struct Cost { double fixed, alone, shared, uneven, store, copy, sum; };
+  static const Cost cost[2][2] = {{{6.211, 1.813, 1.628, 1.308, 1.193, 2.021, 4.178}, {7.35, 5.891, 6.289, 1.18, 1.539, 2.211, 3.0}},
+                                  {{6.297, 0.851, 0.99, 0.347, 0.727, 0.0, 3.926}, {7.821, 1.47, 2.894, 1.055, 1.447, 1.719, 3.0}}};
+  const long long big = blocks_of(g, 3), small = blocks_of(g, 1);
+  const int side = big < 16 || small < (f16 ? 700 : 900) * ((big + (f16 ? 511 : 255)) / (f16 ? 512 : 256)) ? 0 : 1;
+  const Cost& c = cost[f16 != 0][side];
+  long long slices = 1;
+  if (small < 512 && 9 * g.C >= 1024) {
+    slices = 9 * g.C / 256 < (1024 + small - 1) / small ? 9 * g.C / 256 : (1024 + small - 1) / small;
+    slices = slices > 8 ? 8 : slices;
+  }
+  const double rounds = (double)(side ? big : small) * slices / kUnits, full = rounds > 1 ? rounds : 1, per = 9 * g.C / 64.0 / slices;
+  return c.fixed + per * (c.alone + c.shared * (full - 1) + c.uneven * (ceil(rounds) > full ? ceil(rounds) - full : 0)) + c.store * results * slices +
+         c.copy * image + (slices > 1 ? c.sum : 0.0);
+}
+
+// The form for these sizes, or 0: the generic kernels are faster or sum more exactly there.
+//  * One of the forms that are exact enough, by the estimates: the channels sliced where there are few blocks (float32 9 x 216 -> 64, 17 x 17
+//    20 us, 46 without slices), the image staged unless it is large and there is little to multiply (float16 18 x 64 -> 48, 51 x 51 15.3
+//    gathered, 16.8 staged, 1 x 40 -> 152, 42 x 42 10.0 and 9.0).
+//  * It is taken where the estimate is below the generic kernels' (on the matrix instructions, 5 % above): over 530 sizes outside of 16 to
+//    256 channels and features and 7 to 56 squared, 1.2 (float32) and 1.6 % (float16) off the faster one in the mean; within them 0.1 to 0.6 %.
+//  * Fewer than 8 channels: a chunk is mostly zeros.  Over 200 sizes the generic kernels were 1.14 (float32) and 1.10 times as fast in the
+//    mean, up to 5.6 and 7.5 (float16 10 x 3 -> 2, 151 x 151 7.6 / 58).  Faster here at all 19 sizes: two or three channels with 32 features and
+//    half a million results on in float16 (9 x 3 -> 105, 26 x 26 10.1 / 8.1, 40 x 3 -> 50, 87 x 87 159 / 74), 64 and a million in float32
+//    (14 x 2 -> 109, 38 x 38 15.6 / 14.1, 8 x 3 -> 105, 42 x 42 14.9 / 10.7).
 int choose(const Geometry& g, int f16) {
-  const long long results = (long long)g.columns * g.F;
+  const bool image_like = (g.C == 2 || g.C == 3) && g.F >= (f16 ? 32 : 64) && (long long)g.columns * g.F >= (f16 ? 1 << 19 : 1 << 20);
+  if (g.C < 8 && !image_like) return 0;
   const bool vector_units = on_vector_units(g);
   int best = 0;
-  double t_best = !vector_units ? 1e30 : (f16 ? 5.3 : 5.5) + (f16 ? 1.3e-6 : 1.1e-6) * results * 9 * g.C;
+  double t_best = 1e30;
   auto consider = [&](int form, double t) {
     if (t < t_best && fits(g, f16, form)) { best = form; t_best = t; }
   };
@@ -346,7 +383,7 @@ int choose(const Geometry& g, int f16) {
     for (int slices : {1, 2, 3, 4, 5, 6, 8, 12})
       if (form > 3 && slices <= g.chunks && (slices == 1 || slices * blocks_of(g, form) <= 4 * kUnits)) consider(form + (slices > 1 ? 256 * slices : 0), staged_time(g, f16, form, slices));
   }
-  return best;
+  return best && (image_like || t_best + outside_time(g, f16, best) < (vector_units ? 1.0 : 1.05) * generic_time(g, f16)) ? best : 0;
 }
 
 // Among the forms that need no more scratch than the packed filter, for callers that have no more; beyond these lines, too, the
