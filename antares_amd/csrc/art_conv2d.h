@@ -82,9 +82,12 @@ __device__ __forceinline__ void store_results(const f32x16 (&total)[MT][NT], flo
 
 // Forms 4 to 7 (art_conv2d_staged.hip): blocks of 64 features x 64 points, 64 x 128, 128 x 128, and 64 x 64 with short sums (float32
 // only), over a copy of the image that is laid out for them.  `packed` takes the filter, behind it the image, and behind that the results of the slices of channels.
+// The copy holds the images of a pass, kMostCopy bytes of them (or one image).
+constexpr size_t kMostCopy = 128 << 20;
+int images_of_pass(const Geometry& g);
 size_t staged_bytes(const Geometry& g, int slices);
 size_t staged_lds(const Geometry& g);
-int run_staged(const void* x, const void* w, void* packed, void* y, const Geometry& g, int f16, int form, int slices, int blocks, hipStream_t stream);
+int run_staged(const void* x, const void* w, void* packed, void* y, const Geometry& g, int f16, int form, int slices, hipStream_t stream);
 
 }  // namespace conv
 

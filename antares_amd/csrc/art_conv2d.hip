@@ -303,7 +303,8 @@ double staged_time(const Geometry& g, int f16, int form, int slices) {
   const double chunks = slices > 1 ? (g.chunks + slices - 1) / slices : g.chunks - half;
   const double t = c.fixed + chunks * (c.alone + c.shared * (full - 1) + c.uneven * (ceil(rounds) > full ? ceil(rounds) - full : 0)) +
                    r.copy * 64e-6 * g.chunks * g.N * (g.HO + 2) * (g.WO + 2);
-  return slices == 1 ? t + r.store * megabytes : t + r.sum + r.sum_bytes * (slices + 1) * megabytes;
+  const double passes = (g.N + images_of_pass(g) - 1) / images_of_pass(g);
+  return c.fixed * (passes - 1) + (slices == 1 ? t + r.store * megabytes : t + r.sum + r.sum_bytes * (slices + 1) * megabytes);
 }
 
 // Where the generic lowering has no matrix instructions for the convolution: it sums on the vector units.
@@ -368,9 +369,13 @@ double generic_time(const Geometry& g, int f16) {
 //    mean, up to 5.6 and 7.5 (float16 10 x 3 -> 2, 151 x 151 7.6 / 58).  Faster here at all 19 sizes: two or three channels with 32 features and
 //    half a million results on in float16 (9 x 3 -> 105, 26 x 26 10.1 / 8.1, 40 x 3 -> 50, 87 x 87 159 / 74), 64 and a million in float32
 //    (14 x 2 -> 109, 38 x 38 15.6 / 14.1, 8 x 3 -> 105, 42 x 42 14.9 / 10.7).
-int choose(const Geometry& g, int f16) {
+//  * A copy of more than 128 MiB for one image is not made: the image is gathered.  Beside the packed filter a call takes 192 MiB at the
+//    most, 128 for the copy and 64 for slices (4 kUnits blocks of 128 x 128).
+// `gathered`: the best of the forms that need no more than the packed filter, for callers that have no more.
+int choose(const Geometry& g, int f16, bool gathered) {
   const bool image_like = (g.C == 2 || g.C == 3) && g.F >= (f16 ? 32 : 64) && (long long)g.columns * g.F >= (f16 ? 1 << 19 : 1 << 20);
-  if (g.C < 8 && !image_like) return 0;
+  if (g.C < 8 && !image_like && !gathered) return 0;
+  const bool staged = !gathered && (size_t)g.chunks * (g.HO + 2) * (g.WO + 2) * kChunkBytes <= kMostCopy;
   const bool vector_units = on_vector_units(g);
   int best = 0;
   double t_best = 1e30;
@@ -381,22 +386,9 @@ int choose(const Geometry& g, int f16) {
     if (!exact_enough(g, f16, form) || (form == 7 && (f16 || !vector_units))) continue;
     if (form <= 3) consider(form, launch_time(g, f16, form));
     for (int slices : {1, 2, 3, 4, 5, 6, 8, 12})
-      if (form > 3 && slices <= g.chunks && (slices == 1 || slices * blocks_of(g, form) <= 4 * kUnits)) consider(form + (slices > 1 ? 256 * slices : 0), staged_time(g, f16, form, slices));
+      if (form > 3 && staged && slices <= g.chunks && (slices == 1 || slices * blocks_of(g, form) <= 4 * kUnits)) consider(form + (slices > 1 ? 256 * slices : 0), staged_time(g, f16, form, slices));
   }
-  return best && (image_like || t_best + outside_time(g, f16, best) < (vector_units ? 1.0 : 1.05) * generic_time(g, f16)) ? best : 0;
-}
-
-// Among the forms that need no more scratch than the packed filter, for callers that have no more; beyond these lines, too, the
-// generic kernels were faster: from 1024 terms per result on they slice the sum over an idle chip.
-int choose_gathered(const Geometry& g, int f16) {
-  const long long small = blocks_of(g, 1), results = (long long)g.columns * g.F;
-  const bool vector_units = g.F < 32 || small < 16;
-  if (vector_units && (!f16 || results < 8192 || (g.F < 32 && g.C < 64))) return 0;
-  if (!vector_units && 9LL * g.C >= 1024 && small < (f16 ? 64 : 192)) return 0;
-  int best = 0;
-  for (int form = 1; form <= (g.F < 32 ? 1 : 3); ++form)
-    if (fits(g, f16, form) && (!best || launch_time(g, f16, form) < launch_time(g, f16, best))) best = form;
-  return best;
+  return best && (gathered || image_like || t_best + outside_time(g, f16, best) < (vector_units ? 1.0 : 1.05) * generic_time(g, f16)) ? best : 0;
 }
 
 template <typename T, int MT, int NT>
@@ -422,7 +414,7 @@ int run(const void* x, const void* w, void* packed, void* y, const Geometry& g, 
 extern "C" int art_conv2d_form(int f16, int N, int C, int H, int W, int F, int HO, int WO, int ph, int pw, int form) {
   Geometry g;
   if (!geometry(g, f16, N, C, H, W, F, HO, WO, ph, pw)) return 0;
-  return form ? (fits(g, f16, form) ? form : 0) : choose_gathered(g, f16);
+  return form ? (fits(g, f16, form) ? form : 0) : choose(g, f16, true);
 }
 
 extern "C" int art_conv2d_exact_enough(int f16, int N, int C, int H, int W, int F, int HO, int WO, int ph, int pw, int form) {
@@ -432,7 +424,7 @@ extern "C" int art_conv2d_exact_enough(int f16, int N, int C, int H, int W, int 
 
 extern "C" int art_conv2d_choose(int f16, int N, int C, int H, int W, int F, int HO, int WO, int ph, int pw) {
   Geometry g;
-  return geometry(g, f16, N, C, H, W, F, HO, WO, ph, pw) ? choose(g, f16) : 0;
+  return geometry(g, f16, N, C, H, W, F, HO, WO, ph, pw) ? choose(g, f16, false) : 0;
 }
 
 extern "C" size_t art_conv2d_packed_bytes(int f16, int C, int F) {
@@ -462,7 +454,7 @@ extern "C" int art_conv2d(const void* x_dev, const void* w_dev, void* packed_dev
   g.blocks_across = make_div((unsigned)g.row_blocks);
   g.span = span_of(g, points_of(form));
   if ((form & 255) > 3)
-    return run_staged(x_dev, w_dev, packed_dev, y_dev, g, f16, form & 255, slices_of(form), (int)blocks_of(g, form), (hipStream_t)stream);
+    return run_staged(x_dev, w_dev, packed_dev, y_dev, g, f16, form & 255, slices_of(form), (hipStream_t)stream);
   return f16 ? run<_Float16>(x_dev, w_dev, packed_dev, y_dev, g, form, (hipStream_t)stream)
              : run<float>(x_dev, w_dev, packed_dev, y_dev, g, form, (hipStream_t)stream);
 }

@@ -13,7 +13,8 @@
 //   * a tap is a constant number of points added to a lane's point; the filter comes from L2 straight into registers, several
 //     taps ahead;
 //   * stores run over the features with one addition each;
-//   * few blocks: the chunks of channels are cut into slices, whose results a third launch adds.
+//   * few blocks: the chunks of channels are cut into slices, whose results a third launch adds;
+//   * the copy takes 128 MiB at the most: larger batches go in passes of as many images as fit.
 // Measured, all launches, against what ran before (the gathering kernel or the generic lowering), us: float16 1 x 40 x 42 x 42 -> 152
 // 10.1 -> 9.0, 2 x 40 x 12 x 12 -> 64 9.6 -> 7.9, 9 x 240 x 13 x 13 -> 104 19.4 -> 13.8, 3 x 184 x 51 x 51 -> 184 23.6 -> 19,
 // 32 x 128 x 28 x 28 -> 128 22.7 -> 21.7 (6 to 7 of them the copy of 7 MB, 13 the products: four chunks of 1.3 us, code, first
@@ -230,9 +231,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, MT 
 }
 
 size_t filter_bytes(const Geometry& g) { return ((size_t)g.chunks * kTaps * ((g.F + 127) / 128) * 4 * 2048 + 255) & ~(size_t)255; }
-size_t places_of(const Geometry& g) { return (size_t)g.N * (g.HO + 2) * (g.WO + 2); }
+size_t places_of(const Geometry& g, int images) { return (size_t)images * (g.HO + 2) * (g.WO + 2); }
 // the last unit of 16 points may reach 15 points past the copy
-size_t copy_bytes(const Geometry& g) { return ((size_t)g.chunks * places_of(g) * kChunkBytes + 1024 + 255) & ~(size_t)255; }
+size_t copy_bytes(const Geometry& g, int images) { return ((size_t)g.chunks * places_of(g, images) * kChunkBytes + 1024 + 255) & ~(size_t)255; }
 
 template <typename T, int MT, int NT, bool FINE = false>
 int launch(const void* packed, void* y, const Staged& s, hipStream_t st) {
@@ -247,14 +248,15 @@ int launch(const void* packed, void* y, const Staged& s, hipStream_t st) {
   return 0;
 }
 
+// One pass over s.g.N images, the first ones of x and y; `images`: the most of a pass, which the copy has room for.
 template <typename T>
-int run(const void* x, const void* w, void* packed, void* y, Staged& s, int form, hipStream_t st) {
+int run(const void* x, const void* w, void* packed, void* y, Staged& s, int form, int images, hipStream_t st) {
   const Geometry& g = s.g;
   T* copy = reinterpret_cast<T*>((char*)packed + filter_bytes(g));
   s.image_copy = (const char*)copy;
   conv2d_stage_kernel<T><<<dim3((unsigned)(s.filter_blocks + s.place_blocks * g.chunks)), dim3(kThreads), 0, st>>>((const T*)x, (const T*)w, (T*)packed, copy, s);
   ART_LAUNCH_CHECK();
-  float* partial = reinterpret_cast<float*>((char*)packed + filter_bytes(g) + copy_bytes(g));
+  float* partial = reinterpret_cast<float*>((char*)packed + filter_bytes(g) + copy_bytes(g, images));
   void* to = s.slices > 1 ? partial : y;
   if (form == 4 ? launch<T, 1, 1>(packed, to, s, st) : form == 5 ? launch<T, 1, 2>(packed, to, s, st)
       : form == 6 ? launch<T, 2, 2>(packed, to, s, st) : launch<T, 1, 1, sizeof(T) == 4>(packed, to, s, st))
@@ -264,23 +266,37 @@ int run(const void* x, const void* w, void* packed, void* y, Staged& s, int form
 
 }  // namespace
 
+int art::conv::images_of_pass(const Geometry& g) {
+  const size_t images = kMostCopy / ((size_t)g.chunks * places_of(g, 1) * kChunkBytes);
+  return images < 1 ? 1 : images < (size_t)g.N ? (int)images : g.N;
+}
 size_t art::conv::staged_bytes(const Geometry& g, int slices) {
-  return filter_bytes(g) + copy_bytes(g) + (slices > 1 ? (size_t)slices * g.columns * g.F * sizeof(float) : 0);
+  const int images = images_of_pass(g);
+  return filter_bytes(g) + copy_bytes(g, images) + (slices > 1 ? (size_t)slices * images * g.results.by * g.F * sizeof(float) : 0);
 }
 size_t art::conv::staged_lds(const Geometry& g) { return (size_t)((g.span + 15) / 16) * 3 * 1024; }
 
-int art::conv::run_staged(const void* x, const void* w, void* packed, void* y, const Geometry& g, int f16, int form, int slices, int blocks, hipStream_t stream) {
+int art::conv::run_staged(const void* x, const void* w, void* packed, void* y, const Geometry& g, int f16, int form, int slices, hipStream_t stream) {
   Staged s{};
   s.g = g;
-  s.places = (int)places_of(g);
   s.filter_blocks = (g.chunks * kTaps * g.row_tiles * 128 + kThreads - 1) / kThreads;
-  s.place_blocks = (s.places + 63) / 64;
-  s.blocks = make_div((unsigned)blocks);
   s.slices = slices;
   s.slice_chunks = g.chunks / slices;
   s.longer = g.chunks % slices;
-  s.results_all = (long long)g.columns * g.F;
-  const int per_chunk = f16 ? 32 : 16;
+  const int per_chunk = f16 ? 32 : 16, points = form == 4 || form == 7 ? 64 : 128, images = images_of_pass(g);
   s.half_last = g.C - (g.chunks - 1) * per_chunk <= per_chunk / 2;
-  return f16 ? run<_Float16>(x, w, packed, y, s, form, stream) : run<float>(x, w, packed, y, s, form, stream);
+  // Passes follow each other on the stream: each overwrites the copy (and the slices' results) of the one before it.
+  for (int n = 0; n < g.N; n += images) {
+    s.g.N = g.N - n < images ? g.N - n : images;
+    s.g.columns = s.g.N * (int)g.results.by;
+    s.places = (int)places_of(g, s.g.N);
+    s.place_blocks = (s.places + 63) / 64;
+    s.blocks = make_div((unsigned)((s.g.columns + points - 1) / points * g.row_blocks));
+    s.results_all = (long long)s.g.columns * g.F;
+    const void* from = (const char*)x + (size_t)n * g.C * g.H * g.W * (f16 ? 2 : 4);
+    void* to = (float*)y + (size_t)n * g.results.by * g.F;
+    if (f16 ? run<_Float16>(from, w, packed, to, s, form, images, stream) : run<float>(from, w, packed, to, s, form, images, stream)) return 1;
+    s.filter_blocks = 0;                              // it stays where the first pass packed it
+  }
+  return 0;
 }

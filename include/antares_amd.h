@@ -298,8 +298,9 @@ int art_gemm_f32_ex(const void* a_dev, const void* b_dev, void* c_dev, int batch
  * form: block shape, 1 = 64 features x 64 points, 2 = 64 x 128, 3 = 128 x 128, with a packed_dev of art_conv2d_packed_bytes;
  * 4, 5, 6 the same over a staged copy of the image, 7 = 64 x 64 there with shorter sums (float32), each plus 256 x slices of the
  * channels (or plus 0: one), with a packed_dev of art_conv2d_scratch_bytes for that form.  art_conv2d_choose gives the library's
- * choice among all of them, art_conv2d_form among the first three (form = 0 asks for it; any other form comes back if it
- * takes these sizes); 0 where these sizes are not taken.  art_conv2d_exact_enough: 1 if the form's sums are no longer than those of
+ * choice among all of them (128 MiB for the copy at the most: larger batches go in passes), art_conv2d_form with form = 0 the best of
+ * the first three for callers that have no room for a copy; any other form comes back if it takes these sizes; 0 where these sizes
+ * are not taken.  art_conv2d_exact_enough: 1 if the form's sums are no longer than those of
  * the generic kernels at these sizes (the choice always is). */
 int art_conv2d_form(int f16, int N, int C, int H, int W, int F, int HO, int WO, int ph, int pw, int form);
 int art_conv2d_choose(int f16, int N, int C, int H, int W, int F, int HO, int WO, int ph, int pw);

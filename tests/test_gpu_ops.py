@@ -1406,6 +1406,30 @@ def test_staged_convolutions_are_no_further_from_float64_than_the_generic_kernel
     assert off[0] <= 1.05 * off[1], off
 
 
+@pytest.mark.parametrize('dtype,n,c,f,h,w', [('float32', 3, 17, 8, 3000, 160), ('float16', 5, 40, 33, 2100, 150)])      # two (three) images to a pass, one (two) left
+def test_staged_convolutions_of_large_batches_in_passes(autort, dtype, n, c, f, h, w):
+    """A copy of 128 MiB at the most: the images go in passes.  The bounds are those of one pass."""
+    from ctypes import c_void_p
+    from antares_amd.runtime import capi
+    note(f'staged convolution in passes {dtype} {n}x{c}x{h}x{w} -> {f}')
+    g = torch.Generator().manual_seed(h)
+    x, wt = torch.randn(n, c, h, w, generator=g).to(getattr(torch, dtype)), torch.randn(f, c, 3, 3, generator=g).to(getattr(torch, dtype))
+    f16 = int(dtype == 'float16')
+    shape = (f16, n, c, h, w, f, h, w, 1, 1)
+    lib, dev = capi.lib(), autort.device()
+    xd, wd = x.to(dev), wt.to(dev)
+    # rows at both ends of every image and in its middle
+    rows = [0, 1, h // 2, h // 2 + 1, h - 2, h - 1]
+    pads = torch.nn.functional.pad(x.double(), (1, 1, 1, 1))
+    want, size = (torch.cat([torch.nn.functional.conv2d(a[:, :, r:r + 3], b) for r in rows], 2) for a, b in ((pads, wt.double()), (pads.abs(), wt.double().abs())))
+    for form in (4, 5, 4 + 512) if f16 else (4, 5, 7, 4 + 512):
+        y = torch.full((n, f, h, w), 7.0, device=dev)
+        scratch = torch.full((lib.art_conv2d_scratch_bytes(*shape, form),), 255, dtype=torch.uint8, device=dev)
+        assert 0 < scratch.numel() < (130 << 20) + (2 * 3 * f * h * w * 4 if form > 255 else 0)
+        capi.check(lib.art_conv2d(*(c_void_p(t.data_ptr()) for t in (xd, wd, scratch, y)), *shape, form, c_void_p(torch.cuda.current_stream().cuda_stream)))
+        assert bool(((y[:, :, rows].cpu().double() - want).abs() <= 2.0 ** -23 * 9 * c * size + 1e-30).all()), form
+
+
 @pytest.mark.parametrize('dtype,n,c,f,hw', [('float16', 9, 9, 200, 49), ('float16', 17, 25, 88, 29), ('float16', 4, 4, 96, 40), ('float32', 5, 24, 2424, 2),
                                             ('float32', 1, 208, 1160, 4), ('float32', 8, 3, 64, 40)])
 def test_convolutions_of_few_channels_or_points_are_no_further_from_float64_than_the_generic_kernels(autort, dtype, n, c, f, hw):

@@ -160,3 +160,17 @@ def test_a_kept_convolution_form_with_longer_sums_is_not_used():
 def test_convolutions_go_to_the_kernel_that_was_measured_to_be_faster(f16, n, c, f, hw, generic, here):
     """Few channels, features or points and very many of them; times in us on an MI355X."""
     assert bool(capi.lib().art_conv2d_choose(f16, n, c, hw, hw, f, hw, hw, 1, 1)) == (here < generic)
+
+
+@pytest.mark.parametrize('f16,n,c,h,w,f', [(1, 64, 512, 128, 128, 512), (0, 64, 64, 100, 100, 17), (1, 256, 64, 112, 112, 64), (0, 32, 256, 56, 56, 256),
+                                           (1, 2, 2048, 14, 14, 2048), (0, 1, 40, 12000, 60, 48), (0, 9, 216, 17, 17, 64)])
+def test_convolutions_take_a_bounded_copy_of_the_image(f16, n, c, h, w, f):
+    """128 MiB for the copy, whatever the batch (64 more for slices), beside the filter; one image of more is gathered."""
+    lib, shape = capi.lib(), (f16, n, c, h, w, f, h, w, 1, 1)
+    form = lib.art_conv2d_choose(*shape)
+    assert form
+    beside = lib.art_conv2d_scratch_bytes(*shape, form) - lib.art_conv2d_packed_bytes(f16, c, f)
+    assert beside <= (128 << 20) + (64 << 20 if form >> 8 else 0) + 4096
+    assert form <= 3 or -(-c // (32 if f16 else 16)) * (h + 2) * (w + 2) * 64 <= 128 << 20
+    gathered = lib.art_conv2d_form(*shape, 0)               # for callers that have no room for a copy
+    assert gathered <= 3 and (not gathered or lib.art_conv2d_exact_enough(*shape, gathered)) and (gathered or w > 80 or f < 32)
