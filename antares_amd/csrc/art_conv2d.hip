@@ -312,12 +312,12 @@ bool on_vector_units(const Geometry& g) { return g.F < 32 || g.columns < 32 || 9
 
 // Whether a form's sums are no longer than those of the generic kernels that it takes the place of.  On the vector units 64 terms and
 // more are spread over a wavefront: float32 form 7 only, float16 the blocks of 64 x 64, whose rows of taps are summed by themselves.
-// Fewer terms are a chain there: these blocks have 0.42 to 0.93 times its error.
+// Fewer terms are a chain there: 0.42 to 0.93 times its error in these blocks, 0.46 to 1.0 in the larger ones.
 // Elsewhere float16 with fewer than 32 channels that are not 8 or 16 and so on: the larger blocks sum 18 instructions in a row where
 // the generic kernels need 9 C / 16 (5 to 31 channels 1.02 to 1.22 times their error, the blocks of 64 x 64 0.66 to 1.01
 // times; with four channels both are above it).
 bool exact_enough(const Geometry& g, int f16, int form) {
-  if (on_vector_units(g)) return f16 || 9 * g.C < 64 ? shape_of(form) == 1 : (form & 255) == 7;
+  if (on_vector_units(g)) return 9 * g.C < 64 || (f16 ? shape_of(form) == 1 : (form & 255) == 7);
   return !f16 || (g.C > 4 && shape_of(form) == 1) || g.C >= 32 || g.C % 8 == 0;
 }
 

@@ -112,8 +112,8 @@ def test_products_that_are_mostly_stores_go_to_the_kernel_that_was_measured_to_b
 
 @pytest.mark.parametrize('f16', [0, 1])
 def test_convolutions_are_taken_by_forms_whose_sums_are_no_longer_than_the_generic_ones(f16):
-    """Where the generic lowering has no matrix instructions (its launch plan says so): float32 form 7 (any block of 64 x 64 below 64
-    terms, which are a chain there), float16 blocks of 64 x 64.  Elsewhere float16 with less than a chunk of channels, not whole eighths of them: blocks of 64 x 64.  Also for a form that a module
+    """Where the generic lowering has no matrix instructions (its launch plan says so): float32 form 7, float16 blocks of 64 x 64 (any
+    block below 64 terms, which are a chain there).  Elsewhere float16 with less than a chunk of channels, not whole eighths of them: blocks of 64 x 64.  Also for a form that a module
     file has kept."""
     lib, dtype = capi.lib(), 'float16' if f16 else 'float32'
     cast = '.to(`float32`)' if f16 else ''
@@ -126,7 +126,7 @@ def test_convolutions_are_taken_by_forms_whose_sums_are_no_longer_than_the_gener
         vector = op.plans[0]._matrix_choice(env)[0] is None
         allowed = [v for v in range(1, 8) if lib.art_conv2d_exact_enough(*shape, v)]
         if vector:
-            assert allowed == ([1, 4] if f16 else [7] if c >= 8 else [1, 4, 7]), (shape, allowed)
+            assert allowed == (list(range(1, 8 - f16)) if c < 8 else [1, 4] if f16 else [7]), (shape, allowed)
         elif f16 and c < 32 and c % 8:
             assert allowed == ([1, 4] if c > 4 else []), (shape, allowed)
         else:
