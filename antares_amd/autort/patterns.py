@@ -190,6 +190,7 @@ register(W4A16_IR, W4A16_INPUTS, _w4a16_handler)
 # Products of small and odd sizes (art_gemm_tile): float16 and float32 below, int8 A[M,K] @ B[N,K]^T
 # ---------------------------------------------------------------------------
 _TILE_SLICES = (1, 2, 3, 4, 6, 8, 12, 16, 24)
+_TILE_SLICES_ROOM = 1 << 25                  # values that the slices of a product take at the most (the library's own bound)
 
 
 def _tile_product(op, call, kind: int, a, b, c, M: int, N: int, K: int, large: bool, rival=None) -> bool:
@@ -213,7 +214,7 @@ def _tile_product(op, call, kind: int, a, b, c, M: int, N: int, K: int, large: b
 
     if saved is None and isinstance(trials, int) and trials > 0 and not torch.cuda.is_current_stream_capturing():
         codes = [code] + [v for v in (lib.art_gemm_tile_form(kind, M, N, K, 0, form, s) for form in (1, 2, 3, 4) for s in _TILE_SLICES)
-                          if v and v != code and (v >> 8 == 4) == (code >> 8 == 4) and (v & 255) * M * N <= 1 << 26]
+                          if v and v != code and (v >> 8 == 4) == (code >> 8 == 4) and ((v & 255) == 1 or (v & 255) * M * N <= _TILE_SLICES_ROOM)]
         codes = codes[:trials]
         scratch = partial(max(codes, key=lambda v: v & 255))
 
@@ -228,7 +229,8 @@ def _tile_product(op, call, kind: int, a, b, c, M: int, N: int, K: int, large: b
         value = int(saved['value'])
         # kept by another version of the library, it may have longer sums than are taken now
         short_sums = lib.art_gemm_tile_form(kind, M, N, K, int(large), 0, 1) >> 8 == 4
-        if lib.art_gemm_tile_form(kind, M, N, K, int(large), value >> 8, value & 255) == value and value >> 8 and (value >> 8 == 4) == short_sums:
+        if lib.art_gemm_tile_form(kind, M, N, K, int(large), value >> 8, value & 255) == value and value >> 8 and (value >> 8 == 4) == short_sums \
+                and (value & 255 == 1 or (value & 255) * M * N <= _TILE_SLICES_ROOM):
             code = value
     if not code:
         return False

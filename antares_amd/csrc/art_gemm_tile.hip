@@ -453,7 +453,9 @@ double ragged_time(int type, int N, int K, int splits) {
 }
 
 // 256 * form + slices for these sizes, or 0: another kernel is faster.  `large`: the kernel for large products takes
-// them.  `own`: the best of the forms here, whatever the others take.
+// them.  `own`: the best of the forms here, whatever the others take.  Slices take 128 MiB at the most: of 6000 float32 products of 1000 to
+// 4096 two would take more, and lose 1 % by the estimate (with 64 MiB 6 % of them up to 5 %).
+constexpr long long kMostSlices = 1LL << 25;                 // float32 (int32) values
 int choose(int type, int M, int N, int K, bool large, bool own) {
   if (!takes(type, M, N, K)) return 0;
   const long long results = (long long)M * N;
@@ -464,7 +466,7 @@ int choose(int type, int M, int N, int K, bool large, bool own) {
   for (int form = 1; form <= 4; ++form) {
     if (!has(type, form) || (type == 1 && (form == 4) != short_sums)) continue;
     for (int splits : {1, 2, 3, 4, 5, 6, 8, 10, 12, 16, 24}) {
-      if (splits > chunks || (splits > 1 && splits * results > 1LL << 26)) break;
+      if (splits > chunks || (splits > 1 && splits * results > kMostSlices)) break;
       const double t = launch_time(type, M, N, K, form, splits);
       if (t < best) { best = t; code = 256 * form + splits; }
     }

@@ -174,3 +174,23 @@ def test_convolutions_take_a_bounded_copy_of_the_image(f16, n, c, h, w, f):
     assert form <= 3 or -(-c // (32 if f16 else 16)) * (h + 2) * (w + 2) * 64 <= 128 << 20
     gathered = lib.art_conv2d_form(*shape, 0)               # for callers that have no room for a copy
     assert gathered <= 3 and (not gathered or lib.art_conv2d_exact_enough(*shape, gathered)) and (gathered or w > 80 or f < 32)
+
+
+def test_slices_of_a_product_take_a_bounded_part_of_the_memory():
+    """128 MiB at the most, also for a number of slices that a module file has kept."""
+    lib = capi.lib()
+    for kind, M, N, K in ((0, 2723, 9534, 15561), (1, 7351, 3031, 12535), (1, 3568, 3460, 3723), (2, 3173, 2863, 14926)):
+        slices = lib.art_gemm_tile_form(kind, M, N, K, 0, 0, 1) & 255
+        assert slices == 1 or slices * M * N * 4 <= 128 << 20
+
+    class Codes(Launches):
+        def library(self, fn, *args):
+            self.taken.append(256 * args[-3] + args[-2])
+    M, N, K = 1200, 1300, 700
+    op = ExportedOp(patterns.GEMM_F32_IR, patterns.GEMM_F32_INPUTS, name='gemm_kept')
+    bound, choice = dict(a=torch.zeros(M, K), b=torch.zeros(K, N), c=torch.zeros(M, N)), lib.art_gemm_tile_form(1, M, N, K, 0, 0, 0)
+    for kept, used in ((256 + 22, choice), (256 + 21, 256 + 21)):
+        op.tuned = {f'gemm_tile.form|1,{M},{K},{N}': {'value': kept, 'us': 0.0}}
+        call = Codes()
+        op.fast_path(op, bound, {}, call)
+        assert call.taken == [used]
