@@ -110,6 +110,15 @@ W4A16_INPUTS = ['x=float16[M:1, K:4096]', 'qweight=int8[KH:2048, N:11008]', 'sca
                 'qzeros=int8[G:32, NH:5504]']
 
 
+def scratch_memory(count: int, dtype, device):
+    """Memory that a kernel works in, None when there is not that much: the handler then takes a form that needs less, or leaves the
+    call to the generic kernels."""
+    try:
+        return torch.empty(count, dtype=dtype, device=device)
+    except torch.OutOfMemoryError:
+        return None
+
+
 def tune_hand_kernel(op, key: str, candidates, run, trials: int, clones):
     """``config="tune:N"`` for a hand-written kernel: times up to N values of its launch parameter for the shape of
     this call (the reference's tuner walks the knob space of the schedule that runs, tuner/OpEvo/main.py:467-616; a
@@ -210,13 +219,15 @@ def _tile_product(op, call, kind: int, a, b, c, M: int, N: int, K: int, large: b
         return False
 
     def partial(value):
-        return torch.empty((value & 255) * M * N, dtype=torch.int32 if kind == 2 else torch.float32, device=a.device) if value & 255 > 1 else None
+        return scratch_memory((value & 255) * M * N, torch.int32 if kind == 2 else torch.float32, a.device) if value & 255 > 1 else None
 
     if saved is None and isinstance(trials, int) and trials > 0 and not torch.cuda.is_current_stream_capturing():
         codes = [code] + [v for v in (lib.art_gemm_tile_form(kind, M, N, K, 0, form, s) for form in (1, 2, 3, 4) for s in _TILE_SLICES)
                           if v and v != code and (v >> 8 == 4) == (code >> 8 == 4) and ((v & 255) == 1 or (v & 255) * M * N <= _TILE_SLICES_ROOM)]
         codes = codes[:trials]
         scratch = partial(max(codes, key=lambda v: v & 255))
+        if scratch is None:
+            codes = [v for v in codes if v & 255 == 1] or [code >> 8 << 8 | 1]
 
         def run(value, t):
             capi.check(lib.art_gemm_tile(c_void_p(t[0].data_ptr()), c_void_p(t[1].data_ptr()), c_void_p(t[2].data_ptr()),
@@ -234,7 +245,10 @@ def _tile_product(op, call, kind: int, a, b, c, M: int, N: int, K: int, large: b
             code = value
     if not code:
         return False
-    call.library(lib.art_gemm_tile, a, b, c, partial(code), kind, M, N, K, code >> 8, code & 255, STREAM)
+    room = partial(code)
+    if room is None and code & 255 > 1:
+        code, call.replay = code >> 8 << 8 | 1, False
+    call.library(lib.art_gemm_tile, a, b, c, room, kind, M, N, K, code >> 8, code & 255, STREAM)
     return True
 
 
@@ -483,7 +497,7 @@ def _conv2d_handler(st, axes, window):
             return False
 
         def scratch(forms):
-            return torch.empty(max(lib.art_conv2d_scratch_bytes(*shape, v) for v in forms), dtype=torch.uint8, device=x.device)
+            return scratch_memory(max(lib.art_conv2d_scratch_bytes(*shape, v) for v in forms), torch.uint8, x.device)
 
         def run(value, t):
             capi.check(lib.art_conv2d(*(c_void_p(v.data_ptr()) for v in t), *shape, int(value), c_void_p(torch.cuda.current_stream().cuda_stream)))
@@ -495,9 +509,18 @@ def _conv2d_handler(st, axes, window):
             others = (1, 2, 3, 4, 5, 6) + tuple(k + 256 * s for k in (4, 5, 6, 7) for s in (2, 3, 4, 6, 8))
             forms = [form] + [v for v in others if v != form and lib.art_conv2d_exact_enough(*shape, v)]
             forms = forms[:trials]
-            saved = tune_hand_kernel(op, key, forms, run, len(forms), [(x, w, scratch(forms), torch.empty_like(y))])
+            room = scratch(forms)
+            if room is not None:
+                saved = tune_hand_kernel(op, key, forms, run, len(forms), [(x, w, room, torch.empty_like(y))])
         if saved is not None and lib.art_conv2d_exact_enough(*shape, int(saved['value'])):
             form = int(saved['value'])
-        call.library(lib.art_conv2d, x, w, scratch([form]), y, *shape, form, STREAM)
+        room = scratch([form])
+        if room is None:                          # no copy of the image then: gathered, or left to the generic kernels
+            call.replay = False
+            form = lib.art_conv2d_form(*shape, 0)
+            room = scratch([form]) if form else None
+            if room is None:
+                return False
+        call.library(lib.art_conv2d, x, w, room, y, *shape, form, STREAM)
         return True
     return handler

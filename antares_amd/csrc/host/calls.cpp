@@ -306,7 +306,8 @@ int launch_all(const Recipe& r, const uint64_t* pointer, const uint64_t* slot_in
   return 0;
 }
 
-PyObject* execute(const std::shared_ptr<Recipe>& keep, const Slots& s) {
+// `no_room`: nothing was launched, there was no memory for what the recipe allocates (nullptr, no error set).
+PyObject* execute(const std::shared_ptr<Recipe>& keep, const Slots& s, bool& no_room) {
   const Recipe& r = *keep;
   const Held held(s);
   at::Tensor fresh[kMaxSlots];
@@ -320,9 +321,14 @@ PyObject* execute(const std::shared_ptr<Recipe>& keep, const Slots& s) {
   }
   for (const auto& n : r.numbers)
     if (!pass_number(s.obj[n.first], n.second, slot_int[n.first], slot_float[n.first])) return nullptr;
-  for (size_t i = 0; i < r.allocs.size(); ++i) {
-    fresh[i] = at::Tensor(at::detail::empty_cuda(r.allocs[i].sizes, r.allocs[i].dtype, at::Device(at::kCUDA, (c10::DeviceIndex)r.device), std::nullopt));
-    pointer[s.n + i] = (uint64_t)(uintptr_t)fresh[i].const_data_ptr();
+  try {
+    for (size_t i = 0; i < r.allocs.size(); ++i) {
+      fresh[i] = at::Tensor(at::detail::empty_cuda(r.allocs[i].sizes, r.allocs[i].dtype, at::Device(at::kCUDA, (c10::DeviceIndex)r.device), std::nullopt));
+      pointer[s.n + i] = (uint64_t)(uintptr_t)fresh[i].const_data_ptr();
+    }
+  } catch (const c10::OutOfMemoryError&) {
+    no_room = true;
+    return nullptr;
   }
   const uint64_t stream = !r.uses_stream ? 0 : (uint64_t)(uintptr_t)c10::hip::getCurrentHIPStream(r.device_stream ? (c10::DeviceIndex)r.device : (c10::DeviceIndex)-1).stream();
   const int rc = launch_all(r, pointer, slot_int, slot_float, stream);
@@ -365,24 +371,28 @@ PyObject* operator_call(PyObject* self, PyObject* args, PyObject* kwargs) {
   Operator* op = (Operator*)self;
   Key key;
   Slots s;
-  bool known = plain_allocations() && signature(op, args, kwargs, key, s);
+  bool known = plain_allocations() && signature(op, args, kwargs, key, s), no_room = false;
   if (known) {
     const char* bytes = (const char*)key.word;
     const size_t size = (size_t)key.n * sizeof(int64_t);
     if (*op->last && op->last_key->size() == size && memcmp(op->last_key->data(), bytes, size) == 0 && current(op, **op->last)) {
       std::shared_ptr<Recipe> r = *op->last;
       use(op, *r);
-      return execute(r, s);
+      PyObject* result = execute(r, s, no_room);
+      if (!no_room) return result;
     }
     auto it = op->table->find(std::string(bytes, size));
-    if (it != op->table->end() && current(op, *it->second)) {
+    if (!no_room && it != op->table->end() && current(op, *it->second)) {
       std::shared_ptr<Recipe> r = it->second;
       *op->last_key = it->first;
       *op->last = r;
       use(op, *r);
-      return execute(r, s);
+      PyObject* result = execute(r, s, no_room);
+      if (!no_room) return result;
     }
-    if (it == op->table->end() && !met_before(op, bytes, size)) {
+    if (no_room) {
+      known = false;                                     // this call is run another way, or raises; the recipe stays for the next one
+    } else if (it == op->table->end() && !met_before(op, bytes, size)) {
       known = op->credit > 0;
       if (known) --op->credit;
     }

@@ -109,13 +109,15 @@ def values(args, stream: int) -> list:
 
 class Call:
     """What one call of an operator launches, in order: kernels and entry points of the library, with tensors as
-    tensors, the stream as STREAM, list numbers as Number, and constants."""
+    tensors, the stream as STREAM, list numbers as Number, and constants.  ``replay``: False when the next call of the same
+    signature may go another way (there was no memory for the usual one)."""
 
-    __slots__ = ('stream', 'steps')
+    __slots__ = ('stream', 'steps', 'replay')
 
     def __init__(self, stream: int):
         self.stream = stream
         self.steps = []
+        self.replay = True
 
     def library(self, fn, *args):
         given = values(args, self.stream)
@@ -130,7 +132,7 @@ class Call:
     def keep(self, op: Operator, pending, results, device_stream: bool):
         """Leaves the recipe of this call with the operator.  Tensors that are not among the call's arguments are
         allocated afresh by every later call; a view of an argument is neither, and a call that uses one leaves no recipe."""
-        if pending is None:
+        if pending is None or not self.replay:
             return
         setup()
         key, slots, device = pending

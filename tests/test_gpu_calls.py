@@ -265,3 +265,52 @@ def test_a_growing_cache_and_a_first_position_that_moves_on():
         for outside in (18, -1):
             with pytest.raises(RuntimeError):
                 autort.ops.rope_qkv_store_rows_f16(qkv, inv, qo, kc, vc, extra=[outside])
+
+
+@pytest.mark.parametrize('first', [True, False])
+def test_calls_run_without_room_for_their_scratch_memory(first):
+    """Memory runs out (a limit on what torch may take): a first call and a replayed one take a kernel that needs less, and once there
+    is room again the call is as before."""
+    import autort
+    from antares_amd.runtime import capi
+    dev = autort.device()
+    print(f'[case] calls without room, first={first}', flush=True)
+    n, c, hw, f = 30, 246, 20, 32
+    ir = (f'output0[N, F, HO, WO] +=! input0[N, C, HO + KH - 1, WO + KW - 1].when([HO + KH - 1 >= 0, HO + KH - 1 < {hw}, WO + KW - 1 >= 0, WO + KW - 1 < {hw}], 0.0) '
+          f'* input1[F, C, KH, KW] where HO in {hw}, WO in {hw}')
+    op = autort.export(ir=ir, inputs=[f'input0=float32[N:{n}, C:{c}, H:{hw}, W:{hw}]', f'input1=float32[F:{f}, C:{c}, KH:3, KW:3]'], name=f'conv_room_{int(first)}')
+    shape = (0, n, c, hw, hw, f, hw, hw, 1, 1)
+    lib = capi.lib()
+    form = lib.art_conv2d_choose(*shape)
+    assert form & 255 > 3 and lib.art_conv2d_scratch_bytes(*shape, form) > 24 << 20 and lib.art_conv2d_form(*shape, 0)
+    g = torch.Generator().manual_seed(3)
+    x, w = torch.randn(n, c, hw, hw, generator=g), torch.randn(f, c, 3, 3, generator=g)
+    want = torch.nn.functional.conv2d(x[:2].double(), w.double(), padding=1)
+    xd, wd, y = x.to(dev), w.to(dev), torch.empty(n, f, hw, hw, device=dev)
+
+    def off():
+        got = y[:2].cpu().double()
+        y.zero_()
+        return float((got - want).norm() / want.norm())
+    if not first:
+        for _ in range(2):
+            op(xd, wd, out=y)
+        assert off() < 1e-6
+    try:
+        torch.cuda.synchronize()
+        torch.cuda.empty_cache()
+        # room for the filter (a block of 2 MiB) and no copy of the image
+        torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (8 << 20)) / torch.cuda.get_device_properties(dev).total_memory)
+        held = []
+        with pytest.raises(torch.OutOfMemoryError):            # what is left in blocks of 24 MiB is taken
+            while len(held) < 1000:
+                held.append(torch.empty(24 << 20, dtype=torch.uint8, device=dev))
+        for _ in range(2):
+            op(xd, wd, out=y)
+            assert off() < 1e-6
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    op(xd, wd, out=y)
+    usual = y.clone()
+    op(xd, wd, out=y)
+    assert torch.equal(y, usual) and off() < 1e-6

@@ -194,3 +194,45 @@ def test_slices_of_a_product_take_a_bounded_part_of_the_memory():
         call = Codes()
         op.fast_path(op, bound, {}, call)
         assert call.taken == [used]
+
+
+def test_calls_without_room_for_their_scratch_memory_take_a_form_that_needs_less(monkeypatch):
+    """Where memory runs out: a product in one slice, a convolution that gathers its image, then the generic kernels; none of them
+    leaves a recipe for later calls."""
+    lib, room = capi.lib(), [1 << 40]
+    empty = torch.empty
+
+    def limited(count, **kw):
+        if count * kw['dtype'].itemsize > room[0]:
+            raise torch.OutOfMemoryError('no room')
+        return empty(count, **kw)
+    monkeypatch.setattr(torch, 'empty', limited)
+
+    class Codes(Launches):
+        replay = True
+
+        def library(self, fn, *args):
+            self.taken.append(args[-2] if fn.__name__ == 'art_conv2d' else 256 * args[-3] + args[-2])
+
+    def taken(op, bound, env):
+        call = Codes()
+        return op.fast_path(op, bound, env, call), call.taken, call.replay
+    M, N, K = 300, 300, 3000
+    code = lib.art_gemm_tile_form(1, M, N, K, 0, 0, 0)
+    assert code & 255 > 1
+    op, bound = ExportedOp(patterns.GEMM_F32_IR, patterns.GEMM_F32_INPUTS, name='gemm_room'), dict(a=torch.zeros(M, K), b=torch.zeros(K, N), c=torch.zeros(M, N))
+    assert taken(op, bound, {}) == (True, [code], True)
+    room[0] = 1000
+    assert taken(op, bound, {}) == (True, [code & ~255 | 1], False)
+    room[0] = 1 << 40
+    shape = (0, 4, 64, 28, 28, 64, 28, 28, 1, 1)
+    op = ExportedOp(CONV, CONV_INPUTS, name='conv_scratch')
+    bound = dict(zip(op.declared + op.fresh_outputs, (torch.zeros(4, 64, 28, 28), torch.zeros(64, 64, 3, 3), torch.zeros(4, 64, 28, 28))))
+    env = op.fused.bind_dims({k: tuple(v.shape) for k, v in bound.items()})
+    form, gathered = lib.art_conv2d_choose(*shape), lib.art_conv2d_form(*shape, 0)
+    assert form & 255 > 3 and 1 <= gathered <= 3
+    assert taken(op, bound, env) == (True, [form], True)
+    room[0] = lib.art_conv2d_packed_bytes(0, 64, 64)
+    assert taken(op, bound, env) == (True, [gathered], False)
+    room[0] -= 1
+    assert taken(op, bound, env) == (False, [], False)
