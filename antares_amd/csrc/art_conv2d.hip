@@ -135,6 +135,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 4))
   const vec* filter = reinterpret_cast<const vec*>(packed) + ((size_t)rb * 2 + wm) * MT * 128 + lane;
   const size_t filter_step = (size_t)g.row_tiles * 128;
   constexpr int kSum = MT == 1 && NT == 1 ? 3 : kTaps;            // taps summed by themselves
+  constexpr int kRows = sizeof(T) == 2 && kSum == 3 ? 2 : 1;      // float16: and the halves of the channels
   constexpr int kPerTap = MT == 1 ? kHeld : 2;        // points per lane asked for with a tap
   vec a[kSets][MT][2];
   auto fetch_filter = [&](int set, int tap) {
@@ -168,9 +169,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 4))
     constexpr bool kMore = !decltype(last_chunk)::value;
     constexpr int kHalves = decltype(half)::value ? 1 : 2;
     const T* tile = image + (size_t)(q & 1) * g.span * kPitch;
-    // a chunk is summed by itself and then added to the total (where registers allow, a row of taps by itself before
-    // that): the error of a sum grows with the length of its chain
-    f32x16 acc[MT][NT], row[MT][NT];
+    // a chunk is summed by itself and then added to the total (where registers allow, a row of taps by itself before that, in
+    // float16 for each half of the channels: 1 % of the time, 10 % of the error): the error of a sum grows with the length of its chain
+    f32x16 acc[MT][NT], row[kRows][MT][NT];
     vec b[2][NT];
     auto look = [&](int step) {                       // the points of half `step % kHalves` of a tap
       const int t = step / kHalves, h = step % kHalves;
@@ -195,13 +196,16 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 4))
         for (int i = 0; i < MT; ++i)
 #pragma unroll
           for (int j = 0; j < NT; ++j)
-            row[i][j] = Elem<T>::multiply(a[t % kSets][i][h], b[step & 1][j], h == 0 && t % kSum == 0 ? f32x16(0) : row[i][j]);
+            row[h % kRows][i][j] = Elem<T>::multiply(a[t % kSets][i][h], b[step & 1][j], h < kRows && t % kSum == 0 ? f32x16(0) : row[h % kRows][i][j]);
       }
       if (t % kSum != kSum - 1) continue;
 #pragma unroll
       for (int i = 0; i < MT; ++i)
 #pragma unroll
-        for (int j = 0; j < NT; ++j) acc[i][j] = t < kSum ? row[i][j] : acc[i][j] + row[i][j];
+        for (int j = 0; j < NT; ++j) {
+          const f32x16 sum = kRows == 2 && kHalves == 2 ? row[0][i][j] + row[kRows - 1][i][j] : row[0][i][j];
+          acc[i][j] = t < kSum ? sum : acc[i][j] + sum;
+        }
     }
 #pragma unroll
     for (int i = 0; i < MT; ++i)
@@ -311,14 +315,18 @@ double staged_time(const Geometry& g, int f16, int form, int slices) {
 bool on_vector_units(const Geometry& g) { return g.F < 32 || g.columns < 32 || 9 * g.C < 32 || blocks_of(g, 1) < 16; }
 
 // Whether a form's sums are no longer than those of the generic kernels that it takes the place of.  On the vector units 64 terms and
-// more are spread over a wavefront: float32 form 7 only, float16 the blocks of 64 x 64, whose rows of taps are summed by themselves.
+// more are spread over a wavefront: float32 form 7 only, float16 the blocks of 64 x 64, whose rows of taps are summed by themselves - the
+// gathering one by halves of the channels, too: 0.64 to 0.99 times the generic kernels' error; the staged one is 1.00 to 1.07 times from
+// 17 to 47 channels but 24 and is left out there (32 and 40, 1.00 to 1.02, only where the image is too wide to be gathered).
 // Fewer terms are a chain there: 0.42 to 0.93 times its error in these blocks, 0.46 to 1.0 in the larger ones.
 // Elsewhere float16 with fewer than 32 channels that are not 8 or 16 and so on: the larger blocks sum 18 instructions in a row where
 // the generic kernels need 9 C / 16 (5 to 31 channels 1.02 to 1.22 times their error, the blocks of 64 x 64 0.66 to 1.01
 // times; with four channels both are above it).
 bool exact_enough(const Geometry& g, int f16, int form) {
-  if (on_vector_units(g)) return 9 * g.C < 64 || (f16 ? shape_of(form) == 1 : (form & 255) == 7);
-  return !f16 || (g.C > 4 && shape_of(form) == 1) || g.C >= 32 || g.C % 8 == 0;
+  if (!on_vector_units(g)) return !f16 || (g.C > 4 && shape_of(form) == 1) || g.C >= 32 || g.C % 8 == 0;
+  if (9 * g.C < 64) return true;
+  if (!f16) return (form & 255) == 7;
+  return form == 1 || ((form & 255) == 4 && (g.C <= 16 || g.C == 24 || g.C >= 48 || (g.C % 8 == 0 && !fits(g, f16, 1))));
 }
 
 // What comes on top of these times outside of the sizes they were fitted to: a filter of more than 256 x 256 is packed for longer, and

@@ -1430,7 +1430,7 @@ def test_staged_convolutions_of_large_batches_in_passes(autort, dtype, n, c, f, 
         assert bool(((y[:, :, rows].cpu().double() - want).abs() <= 2.0 ** -23 * 9 * c * size + 1e-30).all()), form
 
 
-@pytest.mark.parametrize('dtype,n,c,f,hw', [('float16', 9, 9, 200, 49), ('float16', 17, 25, 88, 29), ('float16', 4, 4, 96, 40), ('float32', 5, 24, 2424, 2),
+@pytest.mark.parametrize('dtype,n,c,f,hw', [('float16', 9, 9, 200, 49), ('float16', 16, 25, 25, 40), ('float16', 4, 33, 17, 56), ('float16', 17, 25, 88, 29), ('float16', 4, 4, 96, 40), ('float32', 5, 24, 2424, 2),
                                             ('float32', 1, 208, 1160, 4), ('float32', 8, 3, 64, 40)])
 def test_convolutions_of_few_channels_or_points_are_no_further_from_float64_than_the_generic_kernels(autort, dtype, n, c, f, hw):
     """Whichever kernel takes them: the generic sums are short here, on the vector units or over less than a chunk of channels."""
@@ -1446,7 +1446,7 @@ def test_convolutions_of_few_channels_or_points_are_no_further_from_float64_than
         if generic:
             op.fast_path = None
         off.append(float((op(x.to(dev), w.to(dev)).cpu().double() - want).norm() / want.norm()))
-    assert off[0] <= 1.05 * off[1], off
+    assert off[0] <= 1.02 * off[1], off
 
 
 @pytest.mark.parametrize('dtype,n,c,f,hw', [('float16', 4, 40, 72, 20), ('float16', 2, 64, 24, 23), ('float32', 5, 20, 72, 21), ('float16', 30, 16, 256, 28)])
