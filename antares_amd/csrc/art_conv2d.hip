@@ -38,7 +38,7 @@ using namespace art::conv;
 
 constexpr int kPitchBytes = kChunkBytes + 16;   // from one point to the next in LDS
 constexpr unsigned kOutside = 0xffffffffu;
-constexpr size_t kMaxLds = 64 * 1024;
+constexpr size_t kMaxLds = 64 * 1024, kWideLds = 160 * 1024;     // with more than the first a compute unit holds one block
 
 // Filter [F][C][taps] -> [chunk][tap][32 features][half][lane][16 bytes], zeros past F and C.  A thread gathers the 16
 // bytes of one lane; bound by latency (about 2 us).
@@ -265,7 +265,7 @@ bool fits(Geometry g, int f16, int form) {
   const int kind = form & 255;
   if (form < 1 || kind < 1 || kind > (f16 ? 6 : 7)) return false;
   g.span = span_of(g, points_of(form));
-  if (kind <= 3) return form == kind && lds_of(g.span) <= kMaxLds;
+  if (kind <= 3) return form == kind && lds_of(g.span) <= (f16 && form == 1 ? kWideLds : kMaxLds);
   return slices_of(form) <= 64 && slices_of(form) <= g.chunks && staged_lds(g) <= 160 * 1024;
 }
 
@@ -286,7 +286,10 @@ double launch_time(const Geometry& g, int f16, int form) {
   const int per_chunk = f16 ? 32 : 16;
   const double chunks = g.chunks - (form < 3 && g.C - (g.chunks - 1) * per_chunk <= per_chunk / 2 ? 0.5 : 0.0);
   const double rounds = (double)blocks_of(g, form) / kUnits, full = rounds > 1 ? rounds : 1, uneven = ceil(rounds) > full ? ceil(rounds) - full : 0;
-  return c.fixed + chunks * (c.alone + c.shared * (full - 1) + c.uneven * uneven) + c.again * (full - 1) + (f16 ? 0.207 : 0.357) * 4e-6 * g.columns * g.F;
+  // an image so wide that a compute unit holds two blocks or one (float16 64 x 64): 2.0 and 3.8 a chunk and round over ten sizes, 10 % off
+  const size_t lds = lds_of(span_of(g, points_of(form)));
+  const double shared = lds <= kMaxLds ? c.shared : lds <= kWideLds / 2 ? 2.0 : 3.8;
+  return c.fixed + chunks * (c.alone + shared * (full - 1) + (lds <= kMaxLds ? c.uneven : shared) * uneven) + c.again * (full - 1) + (f16 ? 0.207 : 0.357) * 4e-6 * g.columns * g.F;
 }
 
 // The same for the staged forms (the launch that stages the image included): a fixed part, per chunk of a block's slice a time
@@ -316,8 +319,8 @@ bool on_vector_units(const Geometry& g) { return g.F < 32 || g.columns < 32 || 9
 
 // Whether a form's sums are no longer than those of the generic kernels that it takes the place of.  On the vector units 64 terms and
 // more are spread over a wavefront: float32 form 7 only, float16 the blocks of 64 x 64, whose rows of taps are summed by themselves - the
-// gathering one by halves of the channels, too: 0.64 to 0.99 times the generic kernels' error; the staged one is 1.00 to 1.07 times from
-// 17 to 47 channels but 24 and is left out there (32 and 40, 1.00 to 1.02, only where the image is too wide to be gathered).
+// gathering one by halves of the channels, too: 0.64 to 0.99 times the generic kernels' error; the staged one (0.6 to 1.02) is 1.00 to 1.07
+// times from 17 to 47 channels that are not 24, 32 or 40 and is left out there.
 // Fewer terms are a chain there: 0.42 to 0.93 times its error in these blocks, 0.46 to 1.0 in the larger ones.
 // Elsewhere float16 with fewer than 32 channels that are not 8 or 16 and so on: the larger blocks sum 18 instructions in a row where
 // the generic kernels need 9 C / 16 (5 to 31 channels 1.02 to 1.22 times their error, the blocks of 64 x 64 0.66 to 1.01
@@ -326,7 +329,7 @@ bool exact_enough(const Geometry& g, int f16, int form) {
   if (!on_vector_units(g)) return !f16 || (g.C > 4 && shape_of(form) == 1) || g.C >= 32 || g.C % 8 == 0;
   if (9 * g.C < 64) return true;
   if (!f16) return (form & 255) == 7;
-  return form == 1 || ((form & 255) == 4 && (g.C <= 16 || g.C == 24 || g.C >= 48 || (g.C % 8 == 0 && !fits(g, f16, 1))));
+  return form == 1 || ((form & 255) == 4 && (g.C <= 16 || g.C % 8 == 0 || g.C >= 48));
 }
 
 // What comes on top of these times outside of the sizes they were fitted to: a filter of more than 256 x 256 is packed for longer, and
@@ -377,6 +380,8 @@ double generic_time(const Geometry& g, int f16) {
 //    mean, up to 5.6 and 7.5 (float16 10 x 3 -> 2, 151 x 151 7.6 / 58).  Faster here at all 19 sizes: two or three channels with 32 features and
 //    half a million results on in float16 (9 x 3 -> 105, 26 x 26 10.1 / 8.1, 40 x 3 -> 50, 87 x 87 159 / 74), 64 and a million in float32
 //    (14 x 2 -> 109, 38 x 38 15.6 / 14.1, 8 x 3 -> 105, 42 x 42 14.9 / 10.7).
+//  * Images too wide for 64 KiB of LDS are staged, or gathered by blocks with 160 KiB where only these sum exactly enough (float16, 17 to 47
+//    channels on the vector units' ground): 18 x 44 -> 29, 120 x 120 102 us, 3 x 33 -> 21, 147 x 147 32 (staged 79 and 25, generic 8347 and 558).
 //  * A copy of more than 128 MiB for one image is not made: the image is gathered.  Beside the packed filter a call takes 192 MiB at the
 //    most, 128 for the copy and 64 for slices (4 kUnits blocks of 128 x 128).
 // `gathered`: the best of the forms that need no more than the packed filter, for callers that have no more.
@@ -392,7 +397,7 @@ int choose(const Geometry& g, int f16, bool gathered) {
   };
   for (int form = 1; form <= 7; ++form) {
     if (!exact_enough(g, f16, form) || (form == 7 && (f16 || !vector_units))) continue;
-    if (form <= 3) consider(form, launch_time(g, f16, form));
+    if (form <= 3 && (lds_of(span_of(g, points_of(form))) <= kMaxLds || (vector_units && !exact_enough(g, f16, 4)))) consider(form, launch_time(g, f16, form));
     for (int slices : {1, 2, 3, 4, 5, 6, 8, 12})
       if (form > 3 && staged && slices <= g.chunks && (slices == 1 || slices * blocks_of(g, form) <= 4 * kUnits)) consider(form + (slices > 1 ? 256 * slices : 0), staged_time(g, f16, form, slices));
   }
@@ -400,8 +405,15 @@ int choose(const Geometry& g, int f16, bool gathered) {
 }
 
 template <typename T, int MT, int NT>
-void launch(const void* x, const void* packed, void* y, const Geometry& g, unsigned blocks, hipStream_t st) {
+int launch(const void* x, const void* packed, void* y, const Geometry& g, unsigned blocks, hipStream_t st) {
+  static bool configured = false;
+  if (lds_of(g.span) > kMaxLds && !configured) {
+    ART_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(conv2d_kernel<T, MT, NT>), hipFuncAttributeMaxDynamicSharedMemorySize, kWideLds));
+    configured = true;
+  }
   conv2d_kernel<T, MT, NT><<<dim3(blocks), dim3(kThreads), lds_of(g.span), st>>>((const T*)x, (const T*)packed, (float*)y, g);
+  ART_LAUNCH_CHECK();
+  return 0;
 }
 
 template <typename T>
@@ -410,11 +422,8 @@ int run(const void* x, const void* w, void* packed, void* y, const Geometry& g, 
   conv2d_pack_kernel<T><<<dim3((unsigned)((lanes + kThreads - 1) / kThreads)), dim3(kThreads), 0, st>>>((const T*)w, (T*)packed, g);
   ART_LAUNCH_CHECK();
   const unsigned blocks = (unsigned)blocks_of(g, form);
-  if (form == 1) launch<T, 1, 1>(x, packed, y, g, blocks, st);
-  else if (form == 2) launch<T, 1, 2>(x, packed, y, g, blocks, st);
-  else launch<T, 2, 2>(x, packed, y, g, blocks, st);
-  ART_LAUNCH_CHECK();
-  return 0;
+  return form == 1 ? launch<T, 1, 1>(x, packed, y, g, blocks, st) : form == 2 ? launch<T, 1, 2>(x, packed, y, g, blocks, st)
+                                                                             : launch<T, 2, 2>(x, packed, y, g, blocks, st);
 }
 
 }  // namespace

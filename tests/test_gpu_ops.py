@@ -1318,11 +1318,10 @@ CONV_CASES = [  # N, C, (H, W), F, (ph, pw), (HO, WO), guarded
     (1, 16, (1, 1), 32, (1, 1), (1, 1), True),             # one point
     (4, 8, (30, 31), 20, (-1, 1), (27, 31), True),         # taps that start inside
 ]
+CONV_WIDE = (2, 33, (5, 200), 21, (1, 1), (5, 200), True)  # gathered by a block that has a compute unit's LDS to itself (float16 64 x 64)
 
 
-@pytest.mark.parametrize('dtype', ['float16', 'float32'])
-@pytest.mark.parametrize('form', [1, 2, 3])
-@pytest.mark.parametrize('case', CONV_CASES)
+@pytest.mark.parametrize('dtype,form,case', [(d, f, c) for c in CONV_CASES for f in (1, 2, 3) for d in ('float16', 'float32')] + [('float16', 1, CONV_WIDE)])
 def test_convolution_blocks_match_float64(autort, dtype, form, case):
     """Each block shape of the convolution kernel against the same sum in 64 bits: products of float16 are exact in
     float32, so the error is that of float32 sums of 9 C terms in any order."""

@@ -126,7 +126,7 @@ def test_convolutions_are_taken_by_forms_whose_sums_are_no_longer_than_the_gener
         vector = op.plans[0]._matrix_choice(env)[0] is None
         allowed = [v for v in range(1, 8) if lib.art_conv2d_exact_enough(*shape, v)]
         if vector:
-            assert allowed == (list(range(1, 8 - f16)) if c < 8 else [7] if not f16 else [1, 4] if c <= 16 or c == 24 or c >= 48 else [1]), (shape, allowed)
+            assert allowed == (list(range(1, 8 - f16)) if c < 8 else [7] if not f16 else [1, 4] if c <= 16 or c % 8 == 0 or c >= 48 else [1]), (shape, allowed)
         elif f16 and c < 32 and c % 8:
             assert allowed == ([1, 4] if c > 4 else []), (shape, allowed)
         else:
