@@ -374,8 +374,10 @@ double generic_time(const Geometry& g, int f16) {
 //  * One of the forms that are exact enough, by the estimates: the channels sliced where there are few blocks (float32 9 x 216 -> 64, 17 x 17
 //    20 us, 46 without slices), the image staged unless it is large and there is little to multiply (float16 18 x 64 -> 48, 51 x 51 15.3
 //    gathered, 16.8 staged, 1 x 40 -> 152, 42 x 42 10.0 and 9.0).
-//  * It is taken where the estimate is below the generic kernels' (on the matrix instructions, 5 % above): over 530 sizes outside of 16 to
-//    256 channels and features and 7 to 56 squared, 1.2 (float32) and 1.6 % (float16) off the faster one in the mean; within them 0.1 to 0.6 %.
+//  * It is taken where one of them is estimated below the generic kernels (on the matrix instructions, 5 % above): over 1100 sizes a type outside of
+//    16 to 256 channels and features and 7 to 56 squared (770 to fit it and 335 new ones), 0.7 to 1.3 (float32) and 1.5 to 1.7 %
+//    (float16) off the faster one in the mean; within them 0.1 to 0.9 %.  One of them, whichever it is: for many rounds the staged pick may be
+//    estimated above the generic kernels where a gathered form is not (float16 197 x 19 -> 80, 24 x 24 51 us, 36 staged, 32 gathered).
 //  * Fewer than 8 channels: a chunk is mostly zeros.  Over 200 sizes the generic kernels were 1.14 (float32) and 1.10 times as fast in the
 //    mean, up to 5.6 and 7.5 (float16 10 x 3 -> 2, 151 x 151 7.6 / 58).  Faster here at all 19 sizes: two or three channels with 32 features and
 //    half a million results on in float16 (9 x 3 -> 105, 26 x 26 10.1 / 8.1, 40 x 3 -> 50, 87 x 87 159 / 74), 64 and a million in float32
@@ -391,9 +393,11 @@ int choose(const Geometry& g, int f16, bool gathered) {
   const bool staged = !gathered && (size_t)g.chunks * (g.HO + 2) * (g.WO + 2) * kChunkBytes <= kMostCopy;
   const bool vector_units = on_vector_units(g);
   int best = 0;
-  double t_best = 1e30;
+  double t_best = 1e30, t_outside = 1e30;
   auto consider = [&](int form, double t) {
-    if (t < t_best && fits(g, f16, form)) { best = form; t_best = t; }
+    if (!fits(g, f16, form)) return;
+    if (t < t_best) { best = form; t_best = t; }
+    if (t + outside_time(g, f16, form) < t_outside) t_outside = t + outside_time(g, f16, form);
   };
   for (int form = 1; form <= 7; ++form) {
     if (!exact_enough(g, f16, form) || (form == 7 && (f16 || !vector_units))) continue;
@@ -401,7 +405,7 @@ int choose(const Geometry& g, int f16, bool gathered) {
     for (int slices : {1, 2, 3, 4, 5, 6, 8, 12})
       if (form > 3 && staged && slices <= g.chunks && (slices == 1 || slices * blocks_of(g, form) <= 4 * kUnits)) consider(form + (slices > 1 ? 256 * slices : 0), staged_time(g, f16, form, slices));
   }
-  return best && (gathered || image_like || t_best + outside_time(g, f16, best) < (vector_units ? 1.0 : 1.05) * generic_time(g, f16)) ? best : 0;
+  return best && (gathered || image_like || t_outside < (vector_units ? 1.0 : 1.05) * generic_time(g, f16)) ? best : 0;
 }
 
 template <typename T, int MT, int NT>

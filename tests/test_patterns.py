@@ -156,7 +156,7 @@ def test_a_kept_convolution_form_with_longer_sums_is_not_used():
     (0, 1, 24, 32, 15, 7.6, 13.7), (0, 58, 12, 4, 158, 82, 621), (0, 30, 9, 8, 104, 28, 144), (0, 7, 34, 4058, 6, 17, 25), (0, 6, 9, 294, 76, 39, 50),
     (0, 4, 3, 14, 159, 14, 42), (0, 1, 257, 1658, 1, 8.1, 34), (1, 63, 20, 4, 90, 59, 107), (1, 2, 65, 2887, 8, 13.5, 17.7), (1, 10, 3, 2, 151, 7.6, 58),
     (0, 2, 232, 24, 52, 375, 37), (0, 205, 40, 24, 33, 6457, 213), (0, 9, 216, 64, 17, 23, 20), (0, 8, 3, 105, 42, 14.9, 10.7), (1, 28, 40, 16, 42, 319, 19),
-    (1, 9, 240, 104, 13, 19, 13.8), (1, 40, 3, 50, 87, 159, 74), (1, 32, 128, 128, 28, 40, 18.5)])
+    (1, 9, 240, 104, 13, 19, 13.8), (1, 197, 19, 80, 24, 51, 36), (1, 40, 3, 50, 87, 159, 74), (1, 32, 128, 128, 28, 40, 18.5)])
 def test_convolutions_go_to_the_kernel_that_was_measured_to_be_faster(f16, n, c, f, hw, generic, here):
     """Few channels, features or points and very many of them; times in us on an MI355X."""
     assert bool(capi.lib().art_conv2d_choose(f16, n, c, hw, hw, f, hw, hw, 1, 1)) == (here < generic)
