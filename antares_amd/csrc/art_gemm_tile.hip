@@ -403,7 +403,7 @@ bool on_vector_units(int M, int N, int K) { return M < 32 || N < 32 || K < 32 ||
 bool fine(int type, int M, int N, int K, bool large) { return type == 1 && !large && on_vector_units(M, N, K) && K >= 64 && (long long)M * N < 65536; }
 
 // The generic lowering's time, on the vector units and on the matrix instructions, or a time that nothing reaches where it was not
-// the faster one.  Fitted to 4400 sizes, M and N of 1 to 16384, K of 4 to 16384, odd ones among them: where the two are within a factor of
+// the faster one.  Fitted to 4100 sizes, M and N of 1 to 16384, K of 4 to 16384, odd ones among them: where the two are within a factor of
 // two of each other 6 to 17 % off (25 % for float32 of 65536 and more results).  The kernel picked is 0.4 to 4.5 % slower than the
 // faster one in the mean of a kind.
 double generic_time(int type, int M, int N, int K) {
