@@ -19,17 +19,17 @@
 //   * rows of A (and of B in the transposed form) are 144 bytes apart in LDS, so that 16 lanes read 16-byte vectors from
 //     all banks; B as it lies in memory, [k][n], is read with ds_read_b64_tr_b16 (float16) or 4 bytes at a time (float32);
 //   * float32: a chunk of 32 values of k is summed by itself and then added to the total; where the generic lowering would
-//     sum on the vector units in short slices (FINE, see `choose`), four values of k by themselves, these sums in pairs, and
+//     sum on the vector units in short slices (FINE, see `fine`), four values of k by themselves, these sums in pairs, and
 //     the chunks and slices in float64.  One chain over k has 1.4e-7 (64 terms) to 1.1e-6 (4090) against 64 bits, the
-//     generic kernels 1.4e-7 to 1e-6 and, in short slices, 0.7e-7 to 1.6e-7; this 1.1e-7 to 2.3e-7 and, FINE, 0.66e-7 to 0.73e-7;
+//     generic kernels 1.4e-7 to 1e-6 and, in short slices, 0.7e-7 to 1.6e-7; this 1.1e-7 to 2.3e-7 and, FINE, 0.64e-7 to 0.73e-7;
 //   * blocks on one XCD are a contiguous run of (slice, tile), its L2 holds what they share.
 // Bound by latency below some 10 us - a launch, a chain of chunks whose loads L2 answers after several hundred
 // nanoseconds, a second launch for slices -, then by the matrix instructions (float32) or the loads (64 x 64 blocks of float16
 // fetch a byte per 32 operations).  Measured against what ran before (the generic lowering's tiles, padded copies and sliced
 // sums, or the kernels for large products), us: float16 145 x 223 x 869 87 -> 8, 169 x 1158 x 2507 54 -> 12, 1792 x 128 x 3584
 // 72 -> 12, 1024 x 2048 x 1024 27 -> 13, 136 x 448 x 104 4.5 -> 4.5; float32 320 x 192 x 512 94 -> 10, 391 x 239 x 503 19 -> 10,
-// 1109 x 238 x 829 28 -> 16; int8 984 x 1904 x 1520 82 -> 11, 448 x 128 x 576 24 -> 5.  Geometric mean over 387 sizes: 2.2, 1.5, 2.1
-// times as fast.
+// 1109 x 238 x 829 28 -> 16; int8 984 x 1904 x 1520 82 -> 11, 448 x 128 x 576 24 -> 5.  Geometric mean over 1260 sizes of 64 to 4096: 2.1,
+// 1.5 and 1.6 times as fast; over 4200 with M, N or K below 64 or odd large ones: 2.0, 1.34 and 1.64.
 #include <type_traits>
 
 #include "art_conv2d.h"
