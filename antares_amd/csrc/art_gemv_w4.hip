@@ -181,14 +181,18 @@ __device__ __forceinline__ unsigned int wave_sum_all_u32(unsigned int v) {
          ((unsigned int)__builtin_amdgcn_readlane((int)v, 32) + (unsigned int)__builtin_amdgcn_readlane((int)v, 48));
 }
 
+// The arguments up to `splits` are in registers when the kernel starts: with x and the weights' addresses fetched from memory
+// first the launch took 6.46 instead of 6.25 us at 4096 x 11008.
+// in: x, gate_up with MODE 2, att_partial with MODE 3.
 // The register allocator is told that four wavefronts per SIMD are plenty (a launch has three): with the default
 // target of eight it postpones two of the eight weight loads until registers free up, a second memory round trip.
 template <int M, int MODE, int R, int W>   // MODE 0: plain product, 1: RMSNorm of x fused, 2: x = SwiGLU(gate | up) fused, 3: x = merged split attention,
                                            // 4: RMSNorm of x fused, its sum of squares handed in (sumsq_in)
 __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(1, 4))) void gemv_w4a16_kernel(
-    const _Float16* __restrict__ x, const unsigned char* __restrict__ qweight, const _Float16* __restrict__ scales,
-    const unsigned char* __restrict__ qzeros, _Float16* __restrict__ y, int K, int N, int splits,
+    const void* __restrict__ in, const unsigned char* __restrict__ qweight, const _Float16* __restrict__ scales,
+    const unsigned char* __restrict__ qzeros, const _Float16* residual, int K, int N, int att_parts, int splits, _Float16* __restrict__ y,
     unsigned long long* __restrict__ slots, Magic magic, Fused fused) {
+  const _Float16* const x = static_cast<const _Float16*>(in);
   static_assert(R == 8 || (R == 4 && MODE == 0), "the fused prologues are written for 8 rows per lane");
   static_assert(MODE != 4 || W == 4, "the handed-in sum of squares comes with four wavefronts");
   static_assert(W == 4 || W == 8, "four or eight wavefronts per block");
@@ -202,8 +206,6 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(1, 4))) 
   const int cl = tid % CL, kl = tid / CL;
   const int tile = blockIdx.x, split = blockIdx.y;
   const int n0 = tile * CT + cl * 16;
-  // every argument that a load needs, in one trip: left to itself the compiler fetches those of the weights behind the loads of x
-  asm volatile("" ::"s"(qweight), "s"(scales), "s"(qzeros), "s"(fused.residual), "s"(fused.att_partial), "s"(fused.att_parts), "s"(K), "s"(N));
   const int rows = K >> 1;
   const int r0 = split * kRowsPerBlock + kl * R;          // first packed row of this lane
   const bool k_ok = r0 < rows;                            // rows % 64 == 0, so a lane is all in or all out
@@ -237,8 +239,8 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(1, 4))) 
   unsigned int gpair = 0, upair = 0;
   if constexpr (swiglu) {
     const int k = 2 * r0c + 2 * cl;
-    gpair = *reinterpret_cast<const unsigned int*>(fused.gate_up + k);
-    upair = *reinterpret_cast<const unsigned int*>(fused.gate_up + K + k);
+    gpair = *reinterpret_cast<const unsigned int*>(x + k);
+    upair = *reinterpret_cast<const unsigned int*>(x + K + k);
   }
 
   // ---- fused attention merge, part 1: x is the output of a decode attention that ran as `att_parts` blocks per
@@ -249,10 +251,10 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(1, 4))) 
   f32x2 pacc[kMaxParts], pml[kMaxParts];
   if constexpr (attn) {
     const int k = 2 * r0c + 2 * cl, head = k >> 7, d = k & 127;
-    const float* rec = fused.att_partial + (size_t)head * fused.att_parts * kPartStride;
+    const float* rec = static_cast<const float*>(in) + (size_t)head * att_parts * kPartStride;
 #pragma unroll
     for (int p = 0; p < kMaxParts; ++p) {
-      const int pc = p < fused.att_parts ? p : 0;         // unused parts re-read part 0 and get weight 0 below
+      const int pc = p < att_parts ? p : 0;         // unused parts re-read part 0 and get weight 0 below
       pacc[p] = *reinterpret_cast<const f32x2*>(rec + pc * kPartStride + d);
       pml[p] = *reinterpret_cast<const f32x2*>(rec + pc * kPartStride + 128);
     }
@@ -273,9 +275,9 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(1, 4))) 
   // (y may be the residual itself: only the block that arrives last at a column writes it, after every block of the
   // tile has issued its atomics, i.e. after every one of these loads has completed.)
   half2_t res2 = {(_Float16)0, (_Float16)0};
-  if (M == 1 && fused.residual != nullptr && tid < 64) {
+  if (M == 1 && residual != nullptr && tid < 64) {
     const int rc = tile * CT + 2 * tid;
-    if (rc < N) res2 = *reinterpret_cast<const half2_t*>(fused.residual + rc);
+    if (rc < N) res2 = *reinterpret_cast<const half2_t*>(residual + rc);
   }
   // fused RMSNorm: the norm weights of this lane's slice of x go out ahead of the weight stream too - loads return in
   // order, so behind it they would hold the first multiply-accumulate back until the whole patch has arrived
@@ -301,7 +303,7 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(1, 4))) 
   const unsigned int sc2 = *reinterpret_cast<const unsigned int*>(scales + (size_t)gc * N + pcolc);
   const unsigned char zb = qzeros[(size_t)gc * (N >> 1) + (pcolc >> 1)];
   __builtin_amdgcn_sched_barrier(0);                      // nothing below may move above the loads, no load below them
-  // (in front of the loads it would put a second trip for the arguments of the kernel before them)
+  // (in front of the loads it would put a trip for the arguments of the kernel before them)
   if (M == 1 && fused.sumsq_clear != nullptr && blockIdx.x == 0 && blockIdx.y == 0 && tid < kSumsqWords) fused.sumsq_clear[tid] = 0ull;
   if constexpr (swiglu || attn) {       // part 2: pair -> LDS -> all 16 values of the k lane (same wavefront: no block barrier needed)
     half2_t o;
@@ -313,11 +315,11 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(1, 4))) 
       float mm = -INFINITY;
 #pragma unroll
       for (int p = 0; p < kMaxParts; ++p)
-        if (p < fused.att_parts) mm = fmaxf(mm, pml[p][0]);
+        if (p < att_parts) mm = fmaxf(mm, pml[p][0]);
       float n0f = 0.f, n1f = 0.f, den = 0.f;
 #pragma unroll
       for (int p = 0; p < kMaxParts; ++p) {
-        const float wgt = (p < fused.att_parts && pml[p][0] != -INFINITY) ? __expf(pml[p][0] - mm) : 0.f;
+        const float wgt = (p < att_parts && pml[p][0] != -INFINITY) ? __expf(pml[p][0] - mm) : 0.f;
         n0f = fmaf(pacc[p][0], wgt, n0f);
         n1f = fmaf(pacc[p][1], wgt, n1f);
         den = fmaf(pml[p][1], wgt, den);
@@ -458,7 +460,7 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(1, 4))) 
 #pragma unroll
       for (int m = 0; m < M; ++m) {
         half2_t o = {(_Float16)r[m][0], (_Float16)r[m][1]};
-        if (M == 1 && fused.residual != nullptr) o = half2_t{(_Float16)((float)o.x + (float)res2.x), (_Float16)((float)o.y + (float)res2.y)};
+        if (M == 1 && residual != nullptr) o = half2_t{(_Float16)((float)o.x + (float)res2.x), (_Float16)((float)o.y + (float)res2.y)};
         *reinterpret_cast<half2_t*>(y + (size_t)m * N + col) = o;
         if (hand_on) sq_mine = sumsq_fixed((float)o.x) + sumsq_fixed((float)o.y);
       }
@@ -487,7 +489,7 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(1, 4))) 
           if (((old[m][j] + (1LL << 55)) >> 56) == (long long)(splits - 1)) {
             const long long total = old[m][j] + mine[m][j] - ((long long)splits << 56);
             _Float16 o = (_Float16)from_fixed(total);
-            if (M == 1 && fused.residual != nullptr) o = (_Float16)((float)o + (float)(j == 0 ? res2.x : res2.y));
+            if (M == 1 && residual != nullptr) o = (_Float16)((float)o + (float)(j == 0 ? res2.x : res2.y));
             y[(size_t)m * N + col + j] = o;
             slots[(size_t)m * N + col + j] = 0ull;            // ready for the next launch (stream order makes this visible)
             if (hand_on) sq_mine += sumsq_fixed((float)o);
@@ -535,9 +537,10 @@ int launch(const void* x, const void* qw, const void* sc, const void* qz, void* 
   }
   const Magic magic{0x000F000Fu, 0x00F000F0u, 0x64006400u, 0x54005400u};
   const dim3 grid(tiles, splits), block(64 * waves);
+  const void* const in = fused.norm_w ? x : fused.gate_up ? (const void*)fused.gate_up : fused.att_partial ? (const void*)fused.att_partial : x;
 #define ART_GEMV_LAUNCH(MODE, R, W)                                                                                          \
-  gemv_w4a16_kernel<M, MODE, R, W><<<grid, block, 0, stream>>>((const _Float16*)x, (const unsigned char*)qw, (const _Float16*)sc, \
-                                                               (const unsigned char*)qz, (_Float16*)y, K, N, splits, slots, magic, fused)
+  gemv_w4a16_kernel<M, MODE, R, W><<<grid, block, 0, stream>>>(in, (const unsigned char*)qw, (const _Float16*)sc, (const unsigned char*)qz, \
+                                                               fused.residual, K, N, fused.att_parts, splits, (_Float16*)y, slots, magic, fused)
   // the plain product is its own instantiation: it carries none of the fused prologues; rows of x beyond the first
   // and four rows per lane come with four wavefronts only
   if constexpr (M == 1) {

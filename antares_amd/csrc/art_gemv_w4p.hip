@@ -96,44 +96,41 @@ __device__ __forceinline__ float wave_sum_all(float v) {
          (__builtin_bit_cast(float, __builtin_amdgcn_readlane(b, 32)) + __builtin_bit_cast(float, __builtin_amdgcn_readlane(b, 48)));
 }
 
-struct Args {
-  const _Float16* x;
-  const unsigned char* packed;
-  _Float16* y;
-  const _Float16* norm_w;        // NORM: x is replaced by fp16(x * rsqrt(sum(x^2) * inv_n + eps) * norm_w)
-  const _Float16* residual;      // EPI 1: y = fp16(fp16(product) + residual)
-  float inv_n, eps;
-  int K, N, tiles;
-  unsigned int tile_stride;      // bytes between tiles
-};
+// What the first loads need comes first: these 14 words are in registers when the kernel starts.
+// norm_w    NORM: x is replaced by fp16(x * rsqrt(sum(x^2) * inv_n + eps) * norm_w)
+// residual  EPI 1: y = fp16(fp16(product) + residual)
+// tile_stride  bytes between tiles
+#define ART_W4P_PARAMS                                                                                                        \
+  const _Float16 *x, const unsigned char *packed, const _Float16 *norm_w, const _Float16 *residual, unsigned int tile_stride, \
+      int K, _Float16 *y, float inv_n, float eps, Magic magic
 
 // EPI 0: y[n] = fp16(product);  1: + residual;  2: columns 0..7 of a tile are a gate, 8..15 the matching up
 // projection: y[tile * 8 + j] = fp16(silu(fp16(gate_j)) * fp16(up_j)) (line :171 of the sample; N/2 outputs).
 template <bool NORM, int EPI>
-__global__ __launch_bounds__(64 * kMaxWaves) void gemv_w4p_kernel(Args a, Magic magic) {
+__global__ __launch_bounds__(64 * kMaxWaves) void gemv_w4p_kernel(ART_W4P_PARAMS) {
   __shared__ __align__(16) float part[kMaxWaves][kTileCols];     // per wavefront: scaled sums of the tile's columns
   __shared__ float s_ss[kMaxWaves];
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, waves = blockDim.x >> 6;
   const int gi = lane & 7, sb = lane >> 3;
   const int g = wave * 8 + gi;                              // quantisation group of this lane
-  const bool k_ok = g < (a.K >> 7);                         // groups past the end of K: x = 0 (their weights are zeros too)
+  const bool k_ok = g < (K >> 7);                         // groups past the end of K: x = 0 (their weights are zeros too)
   const int kbase = (k_ok ? g : 0) * 128 + sb * 16;
 
   // ---- loads that do not depend on the tile: x and the norm weights of this lane's 16 values of k
-  const u32x4* xp = reinterpret_cast<const u32x4*>(a.x + kbase);
+  const u32x4* xp = reinterpret_cast<const u32x4*>(x + kbase);
   u32x4 xv0 = xp[0], xv1 = xp[1];
   u32x4 n0v = {0, 0, 0, 0}, n1v = {0, 0, 0, 0};
   if constexpr (NORM) {
-    const u32x4* np = reinterpret_cast<const u32x4*>(a.norm_w + kbase);
+    const u32x4* np = reinterpret_cast<const u32x4*>(norm_w + kbase);
     n0v = np[0];
     n1v = np[1];
   }
 
-  const unsigned char* lane_base = a.packed + (size_t)wave * kChunkBytes;
+  const unsigned char* lane_base = packed + (size_t)wave * kChunkBytes;
   auto issue = [&](int tile, u32x4 (&w)[8], unsigned int& sc2, unsigned int& zb, _Float16& res) {
-    const unsigned char* wp = lane_base + (size_t)tile * a.tile_stride;
-    if constexpr (EPI == 1) res = a.residual[tile * kTileCols + (tid & 15)];      // fetched with the tile, not behind its reduction (by every lane: no divergent branch around a load)
+    const unsigned char* wp = lane_base + (size_t)tile * tile_stride;
+    if constexpr (EPI == 1) res = residual[tile * kTileCols + (tid & 15)];      // fetched with the tile, not behind its reduction (by every lane: no divergent branch around a load)
 #pragma unroll
     for (int i = 0; i < 8; ++i) w[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(wp + i * 1024 + lane * 16));
     sc2 = __builtin_nontemporal_load(reinterpret_cast<const unsigned int*>(wp + kScaleOff + (gi * 16 + 2 * sb) * 2));
@@ -167,7 +164,7 @@ __global__ __launch_bounds__(64 * kMaxWaves) void gemv_w4p_kernel(Args a, Magic 
     ss_all = (lane & 15) < waves ? ss_all : 0.f;
     ss_all = sum_over_lane_bits_012(ss_all);
     ss_all += ART_DPP_F(ss_all, 0x140);                     // row_mirror: all 16 lanes of the row
-    const float r = __builtin_amdgcn_rsqf(ss_all * a.inv_n + a.eps);       // v_rsq_f32: within 1 ulp of 1 / sqrt
+    const float r = __builtin_amdgcn_rsqf(ss_all * inv_n + eps);       // v_rsq_f32: within 1 ulp of 1 / sqrt
     const unsigned int nw[8] = {n0v[0], n0v[1], n0v[2], n0v[3], n1v[0], n1v[1], n1v[2], n1v[3]};
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
@@ -230,12 +227,12 @@ __global__ __launch_bounds__(64 * kMaxWaves) void gemv_w4p_kernel(Args a, Magic 
       }
       if constexpr (EPI == 2) {
         const float gf = (float)(_Float16)s, uf = (float)(_Float16)u;
-        a.y[t * 8 + tid] = (_Float16)(art::silu(gf) * uf);
+        y[t * 8 + tid] = (_Float16)(art::silu(gf) * uf);
       } else {
         const int n = t * kTileCols + tid;
         _Float16 o = (_Float16)s;
         if constexpr (EPI == 1) o = (_Float16)((float)o + (float)res);
-        a.y[n] = o;
+        y[n] = o;
       }
     }
   };
@@ -304,25 +301,25 @@ constexpr int kQuadMaxK = 4096, kQuadRecords = 4, kXChunkBytes = 144;   // 64 va
 __device__ __forceinline__ int quad_column(int wave, int c) { return (c >> 1) * 8 + 2 * wave + (c & 1); }
 
 template <bool NORM, int EPI>
-__global__ __launch_bounds__(256) void gemv_w4q_kernel(Args a, Magic magic) {
+__global__ __launch_bounds__(256) void gemv_w4q_kernel(ART_W4P_PARAMS) {
   __shared__ __align__(16) unsigned char xs[64 * kXChunkBytes];
   __shared__ __align__(8) float corr[64][2];                // per 64 values of k: 1024 * sum(low positions) + 64 * sum(high positions), sum(x)
   __shared__ float s_ss[4];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
 
   // ---- x: thread t prepares x[16t .. 16t+15]; past the end of K it is zero (the weights there are zeros too)
-  const bool k_ok = 16 * tid < a.K;
+  const bool k_ok = 16 * tid < K;
   const int k0 = k_ok ? 16 * tid : 0;
-  const u32x4* xp = reinterpret_cast<const u32x4*>(a.x + k0);
+  const u32x4* xp = reinterpret_cast<const u32x4*>(x + k0);
   u32x4 xv0 = xp[0], xv1 = xp[1];
   u32x4 n0v = {0, 0, 0, 0}, n1v = {0, 0, 0, 0};
   if constexpr (NORM) {
-    const u32x4* np = reinterpret_cast<const u32x4*>(a.norm_w + k0);
+    const u32x4* np = reinterpret_cast<const u32x4*>(norm_w + k0);
     n0v = np[0];
     n1v = np[1];
   }
   const int tile = blockIdx.x;
-  const unsigned char* wp = a.packed + (size_t)tile * a.tile_stride + (size_t)wave * kChunkBytes;
+  const unsigned char* wp = packed + (size_t)tile * tile_stride + (size_t)wave * kChunkBytes;
   u32x4 w[8];
 #pragma unroll
   for (int i = 0; i < 8; ++i) w[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(wp + i * 1024 + lane * 16));
@@ -333,7 +330,7 @@ __global__ __launch_bounds__(256) void gemv_w4q_kernel(Args a, Magic magic) {
   // (every lane loads it - the column repeats every four lanes: a load inside a divergent branch makes the compiler
   // wait there for every load in flight)
   _Float16 res = (_Float16)0;
-  if constexpr (EPI == 1) res = a.residual[tile * kTileCols + out_col];
+  if constexpr (EPI == 1) res = residual[tile * kTileCols + out_col];
   __builtin_amdgcn_sched_barrier(0);                        // nothing below moves above the loads
 
   if (!k_ok) { xv0 = u32x4{0, 0, 0, 0}; xv1 = u32x4{0, 0, 0, 0}; }
@@ -349,7 +346,7 @@ __global__ __launch_bounds__(256) void gemv_w4q_kernel(Args a, Magic magic) {
     ss = wave_sum_all(ss);
     if (lane == 0) s_ss[wave] = ss;
     art_lds_barrier();                                      // LDS only: the weight loads stay in flight
-    const float r = __builtin_amdgcn_rsqf(((s_ss[0] + s_ss[1]) + (s_ss[2] + s_ss[3])) * a.inv_n + a.eps);
+    const float r = __builtin_amdgcn_rsqf(((s_ss[0] + s_ss[1]) + (s_ss[2] + s_ss[3])) * inv_n + eps);
     const unsigned int nw[8] = {n0v[0], n0v[1], n0v[2], n0v[3], n1v[0], n1v[1], n1v[2], n1v[3]};
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
@@ -410,12 +407,12 @@ __global__ __launch_bounds__(256) void gemv_w4q_kernel(Args a, Magic magic) {
     const float up = ART_DPP_F(r, 0xB1);
     if (lane < 4 && !odd) {
       const float gf = (float)(_Float16)r, uf = (float)(_Float16)up;
-      a.y[tile * 8 + 2 * wave + (lane >> 1)] = (_Float16)(art::silu(gf) * uf);
+      y[tile * 8 + 2 * wave + (lane >> 1)] = (_Float16)(art::silu(gf) * uf);
     }
   } else if (lane < 4) {
     _Float16 o = (_Float16)r;
     if constexpr (EPI == 1) o = (_Float16)((float)o + (float)res);
-    a.y[tile * kTileCols + out_col] = o;
+    y[tile * kTileCols + out_col] = o;
   }
 }
 
@@ -516,15 +513,16 @@ extern "C" int art_gemv_w4p(const void* x_dev, const void* packed_dev, void* y_d
   ART_REQUIRE(!art::overlaps(x_dev, (size_t)K * 2, y_dev, y_bytes), "art_gemv_w4p: y must not overlap x (it may alias the residual)");
   const int tiles = N / kTileCols, waves = chunks_of(K);
   const int blocks = tiles;
-  Args a{(const _Float16*)x_dev, (const unsigned char*)packed_dev, (_Float16*)y_dev, (const _Float16*)norm_weight_dev,
-         (const _Float16*)residual_dev, 1.0f / (float)K, eps, K, N, tiles, (unsigned int)tile_stride_of(K)};
   const Magic magic{0x000F000Fu, 0x00F000F0u, 0x64006400u, 0x54005400u};
   const dim3 grid(blocks), block(64 * waves);
   hipStream_t st = (hipStream_t)stream;
+#define ART_W4P_ARGS                                                                                                          \
+  (const _Float16*)x_dev, (const unsigned char*)packed_dev, (const _Float16*)norm_weight_dev, (const _Float16*)residual_dev, \
+      (unsigned int)tile_stride_of(K), K, (_Float16*)y_dev, 1.0f / (float)K, eps, magic
 #define ART_W4P_LAUNCH(NORM, EPI)                                                          \
   do {                                                                                    \
-    if (quad_form(K)) gemv_w4q_kernel<NORM, EPI><<<grid, dim3(256), 0, st>>>(a, magic);    \
-    else gemv_w4p_kernel<NORM, EPI><<<grid, block, 0, st>>>(a, magic);                     \
+    if (quad_form(K)) gemv_w4q_kernel<NORM, EPI><<<grid, dim3(256), 0, st>>>(ART_W4P_ARGS);    \
+    else gemv_w4p_kernel<NORM, EPI><<<grid, block, 0, st>>>(ART_W4P_ARGS);                     \
   } while (0)
   if (norm_weight_dev != nullptr) {
     if (swiglu_out) ART_W4P_LAUNCH(true, 2);
@@ -536,6 +534,7 @@ extern "C" int art_gemv_w4p(const void* x_dev, const void* packed_dev, void* y_d
     else ART_W4P_LAUNCH(false, 0);
   }
 #undef ART_W4P_LAUNCH
+#undef ART_W4P_ARGS
   ART_LAUNCH_CHECK();
   return 0;
 }

@@ -232,14 +232,15 @@ template <class F> __device__ __forceinline__ float att_over_groups(float v, F o
   return att_swap32(v, v, op);
 }
 
+// The arguments up to len_host are in registers when the kernel starts.
 // ROPE = true: the block first rotates its head's q and k (rotate-half form) from the token's q|k|v vector,
 // writes k and v into cache row `pos` and attends over rows 0..pos; q_or_qkv then points at q|k|v.
 template <class QT, class KT, class OT, bool ROPE>
 __global__ __launch_bounds__(kAttThreads) void attention_kernel(const QT* __restrict__ q_or_qkv, KT* __restrict__ k, KT* __restrict__ v,
-                                                                 const float* __restrict__ att_f, OT* __restrict__ out, int heads,
-                                                                 const int* __restrict__ len_dev, int len_host,
-                                                                 const _Float16* __restrict__ inv_freq,
-                                                                 float* __restrict__ partial, int parts, unsigned long long inv_parts) {
+                                                                 const int* __restrict__ len_dev, const _Float16* __restrict__ inv_freq,
+                                                                 const float* __restrict__ att_f, int heads, int len_host,
+                                                                 unsigned long long inv_parts, OT* __restrict__ out,
+                                                                 float* __restrict__ partial, int parts) {
   // parts > 1: `parts` blocks share a head, each attends over a contiguous range of the cached positions and
   // leaves its unnormalised state in partial[head][part][kAttPartialStride] = { acc[128], max, sum, -, - };
   // whoever consumes the result merges them (the o-projection does it while it loads x).
@@ -250,7 +251,7 @@ __global__ __launch_bounds__(kAttThreads) void attention_kernel(const QT* __rest
   __shared__ float s_k[D], s_v[D];
   // x / parts for x below 2^30: inv_parts = ceil(2^32 / parts)
   auto over_parts = [&](unsigned int x) { return (int)(__umulhi(x, (unsigned int)inv_parts) + x * (unsigned int)(inv_parts >> 32)); };
-  const int h = over_parts(blockIdx.x), part = blockIdx.x - h * parts, tid = threadIdx.x;
+  const int h = blockIdx.x, part = blockIdx.y, tid = threadIdx.x;
   const int sub = tid & 7, group = tid >> 3, wave = tid >> 6, lane = tid & 63;
   const size_t row = (size_t)heads * D;
   // From here to the first use of a cache row the code is one straight line for every lane: all loads are issued
@@ -610,7 +611,7 @@ extern "C" int art_decode_attention(const void* q_dev, const void* k_dev, const 
   hipStream_t st = (hipStream_t)stream;
   const int* pd = (const int*)pos_dev;
   const float* af = (const float*)att_f_dev;
-#define ART_ATT(QT, KT) attention_kernel<QT, KT, QT, false><<<dim3(heads), dim3(kAttThreads), 0, st>>>((const QT*)q_dev, (KT*)k_dev, (KT*)v_dev, af, (QT*)out_dev, heads, pd, seq_len, nullptr, nullptr, 1, 1ull << 32)
+#define ART_ATT(QT, KT) attention_kernel<QT, KT, QT, false><<<dim3(heads), dim3(kAttThreads), 0, st>>>((const QT*)q_dev, (KT*)k_dev, (KT*)v_dev, pd, nullptr, af, heads, seq_len, 1ull << 32, (QT*)out_dev, nullptr, 1)
   if (q_dtype == 0) { if (kv_dtype == 0) ART_ATT(float, float); else ART_ATT(float, _Float16); }
   else { if (kv_dtype == 0) ART_ATT(_Float16, float); else ART_ATT(_Float16, _Float16); }
 #undef ART_ATT
@@ -688,10 +689,10 @@ extern "C" int art_decode_attention_rope_split(const void* qkv_dev, const void* 
   ART_REQUIRE(max_positions >= 1, "art_decode_attention_rope: the caches have no rows");
   ART_REQUIRE(((uintptr_t)key_cache_dev % 16) == 0 && ((uintptr_t)val_cache_dev % 16) == 0 && ((uintptr_t)out_dev % 16) == 0,
               "art_decode_attention_rope: caches and output must be 16-byte aligned");
-  attention_kernel<_Float16, _Float16, _Float16, true><<<dim3(heads * parts), dim3(kAttThreads), 0, (hipStream_t)stream>>>(
-      (const _Float16*)qkv_dev, (_Float16*)key_cache_dev, (_Float16*)val_cache_dev, (const float*)att_f_dev,
-      parts == 1 ? (_Float16*)out_dev : nullptr, heads, (const int*)pos_dev, max_positions, (const _Float16*)inv_freq_dev,
-      parts == 1 ? nullptr : (float*)out_dev, parts, (0x100000000ull + parts - 1) / parts);
+  attention_kernel<_Float16, _Float16, _Float16, true><<<dim3(heads, parts), dim3(kAttThreads), 0, (hipStream_t)stream>>>(
+      (const _Float16*)qkv_dev, (_Float16*)key_cache_dev, (_Float16*)val_cache_dev, (const int*)pos_dev, (const _Float16*)inv_freq_dev,
+      (const float*)att_f_dev, heads, max_positions, (0x100000000ull + parts - 1) / parts, parts == 1 ? (_Float16*)out_dev : nullptr,
+      parts == 1 ? nullptr : (float*)out_dev, parts);
   ART_LAUNCH_CHECK();
   return 0;
 }

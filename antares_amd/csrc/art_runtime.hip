@@ -191,9 +191,9 @@ int art_module_compile(const char* hip_source, const char* arch, void** blob, si
   hiprtcResult r = hiprtcCreateProgram(&prog, hip_source, "autort_kernel.hip", 0, nullptr, nullptr);
   ART_REQUIRE(r == HIPRTC_SUCCESS, "hiprtcCreateProgram: %s", hiprtcGetErrorString(r));
   std::string arch_opt = std::string("--offload-arch=") + ((arch && *arch) ? arch : "gfx950");
-  // Packed-FP32 instruction selection is switched off for every kernel of this library.
+  // Packed-FP32 instruction selection is switched off for every kernel of this library; the first arguments start in registers.
   const char* opts[] = {arch_opt.c_str(), "-O3", "-std=c++17", "-Wno-ignored-attributes",
-                        "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"};
+                        "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "-mllvm", "-amdgpu-kernarg-preload-count=14"};
   r = hiprtcCompileProgram(prog, (int)(sizeof(opts) / sizeof(opts[0])), opts);
   size_t log_size = 0;
   hiprtcGetProgramLogSize(prog, &log_size);

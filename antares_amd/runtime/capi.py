@@ -146,6 +146,10 @@ def device_props() -> dict:
     return {f: (getattr(p, f).decode() if isinstance(getattr(p, f), bytes) else getattr(p, f)) for f, _ in p._fields_}
 
 
+# What the library's compiler options change in a code object (part of the cache's key): arguments in registers at the start of a kernel.
+COMPILE_OPTIONS = 'kernarg-preload-14\n'
+
+
 def compile_hip(source: str, arch: str = 'gfx950') -> bytes:
     """HIP source -> code object bytes (in-process, no GPU needed)."""
     blob, size = c_void_p(), c_size_t()
