@@ -352,6 +352,9 @@ class LlamaInt4Decoder:
             qkv = lw['qkv']
             self.autort.ops.gemm_w4a16_rope_store(xb, qkv['qweight'], qkv['scales'], qkv['qzeros'], angles, qr, self.key_cache[l], self.val_cache[l],
                                                    k_splits=k_splits)
+            if l + 1 == len(layers) and self.packed:
+                self._prefill_last(l, x[T - 1], qr[T - 1], T)
+                break
             att = self.autort.ops.attention_causal_f16(qr, self.key_cache[l].view(cfg.max_seq, H, D),
                                                        self.val_cache[l].view(cfg.max_seq, H, D), self.att_f)
             xb = gemm_res(att.view(T, d), lw['o'], x, lw['ffn_norm'])
@@ -361,13 +364,25 @@ class LlamaInt4Decoder:
                 xb = gemm_res(hid, down, x, layers[l + 1]['att_norm'])
             else:                       # the final norm is folded into the last projection
                 self.autort.ops.gemm_w4a16_residual(hid, down['qweight'], down['scales'], down['qzeros'], x, residual=x)
-        self.x.copy_(x[T - 1])
+                self.x.copy_(x[T - 1])
+                h = self.w['lm_head']
+                self.autort.ops.gemv_w4a16_fused(self.x, h['qweight'], h['scales'], h['qzeros'], self.logits,
+                                                 norm_weight=self.w['final_norm'], eps=cfg.rms_eps)
         self.pos.fill_(T - 1)
         self.token.copy_(tokens.view(T)[T - 1:T])
-        h = self.w['lm_head']
-        self.autort.ops.gemv_w4a16_fused(self.x, h['qweight'], h['scales'], h['qzeros'], self.logits,
-                                         norm_weight=self.w['final_norm'], eps=cfg.rms_eps)
         return self.logits
+
+    def _prefill_last(self, l: int, x: torch.Tensor, q: torch.Tensor, T: int):
+        """The last layer behind its keys and values, and the logits.  Nothing reads that layer's other rows, so the last
+        position goes through it alone, with the operators of the one-token step over the repacked weights: a prompt of
+        1003 tokens through 32 layers 13.70 -> 13.38 ms, of 128 tokens 1.4 % less; the fewer layers, the more."""
+        cfg, gemv, pw = self.cfg, self.autort.ops.gemv_w4p, self.pw['layers'][l]
+        d, H, D, F = cfg.dim, cfg.n_heads, cfg.head_dim, cfg.ffn
+        self.autort.ops.attention_f16(q, self.key_cache[l, :T].view(T, H, D), self.val_cache[l, :T].view(T, H, D), self.att_f, self.att)
+        gemv(self.att.view(-1), pw['o'], self.x, residual=x, shape=(d, d))
+        gemv(self.x, pw['gate_up'], self.hb, norm_weight=self.w['layers'][l]['ffn_norm'], eps=cfg.rms_eps, swiglu_out=True, shape=(d, 2 * F))
+        gemv(self.hb, pw['down'], self.x, residual=self.x, shape=(F, d))
+        gemv(self.x, self.pw['lm_head'], self.logits, norm_weight=self.w['final_norm'], eps=cfg.rms_eps, shape=(d, cfg.vocab))
 
     def tune_att_parts(self, pos: int, candidates=(8, 4, 2, 1), runs: int = 20) -> Dict[str, object]:
         """The decode attention's launch parameter - blocks per head - for a cache filled up to `pos`: times the

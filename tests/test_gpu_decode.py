@@ -143,6 +143,24 @@ def test_prefill_of_a_whole_prompt_matches_the_oracle_token_by_token(T):
         dec.prefill(prompt[:3].to(dec.dev))
 
 
+@pytest.mark.parametrize('layers,T', [(1, 4), (1, 33), (2, 65)])
+def test_the_last_position_alone_through_the_last_layer_matches_all_rows_through_it(layers, T):
+    """Over repacked weights `prefill` takes only the last position through the last layer behind its keys and values; the
+    decoder without them takes every row: the same caches bit for bit, and logits within LOGIT_TOL of each other."""
+    from antares_amd.llama import LlamaInt4Decoder, random_weights
+    cfg = small_config(max_seq=80)
+    cfg.n_layers = layers
+    w = random_weights(cfg, seed=11)
+    prompt = torch.randint(0, cfg.vocab, (T,), generator=torch.Generator().manual_seed(T), dtype=torch.int32)
+    print(f'[case] layers={layers} T={T}', flush=True)
+    one, all_rows = LlamaInt4Decoder(cfg, w), LlamaInt4Decoder(cfg, w, packed=False)
+    got, want = one.prefill(prompt.to(one.dev)).float().cpu().numpy(), all_rows.prefill(prompt.to(one.dev)).float().cpu().numpy()
+    assert torch.equal(one.key_cache, all_rows.key_cache) and torch.equal(one.val_cache, all_rows.val_cache)
+    assert np.allclose(got, want, **LOGIT_TOL), np.abs(got - want).max()
+    assert np.allclose(one.x.float().cpu().numpy(), all_rows.x.float().cpu().numpy(), **LOGIT_TOL)
+    assert int(one.pos.item()) == T - 1 and int(one.token.item()) == int(prompt[-1])
+
+
 @pytest.mark.parametrize('graph,packed', [(False, True), (True, True), (True, False)])
 def test_full_width_decode_matches_the_oracle(graph, packed):
     """The benchmark model's widths (dim 4096, 32 heads, ffn 11008, vocab 32000, cache of 384 rows, attention over
