@@ -9,8 +9,13 @@
 //   * a block of eight wavefronts owns 128 columns, 32 MT rows (MT = 1, 2, 4) and a contiguous range of quantisation
 //     groups.  Wavefront (c, h) multiplies 32 columns by the k half h of every group, so every weight is unpacked once per
 //     block; the two k halves meet in LDS after the loop.  What bounds the loop is the issue of instructions, not the
-//     matrix cores (with the MFMAs taken out a group takes as long): a wavefront issues one per 7 cycles or so, and a
-//     group is 136 / 149 / 193 of them at MT = 1 / 2 / 4, 64 of them vector instructions that unpack - 1090 / 1170 / 1420 cycles.
+//     matrix cores (with the MFMAs taken out a group takes as long): a wavefront by itself issues a vector instruction every 8
+//     cycles, two of a SIMD one every 4 (the differences and products of halves and the byte permutations; shifts and
+//     v_bitop3 2), and a group is 114 / 126 / 169 instructions at MT = 1 / 2 / 4, 64 of them vector instructions that
+//     unpack.  Hence ring slots that are constants (the loop is three groups long) and loads from buffer descriptors, where one
+//     scalar offset moves on.  With slots and addresses in registers a group was 138 / 149 / 193 instructions, and each store of a
+//     K-split's sums ten (a comparison, a branch, 64-bit addresses) instead of two: 16 rows over 1024 x 3072 6.6 -> 6.2 us, over
+//     11008 x 4096 12.6 -> 12.0; 50 rows over 4096 x 12288 19.9 -> 18.3; 128 rows over 4096 x 4096 16.0 -> 14.9, 4096 x 22016 32.9 -> 31.4.
 //     Sixteen wavefronts with half the work each were slower (the LDS meeting doubles), and so were four column quarters
 //     replaced by two (same loop, longer meeting), blocks that start at groups of their own, and branches around the
 //     loads of the last groups;
@@ -21,7 +26,6 @@
 //     (rows of 256 bytes): every 16 lanes of a read touch every bank once;
 //   * the packed bytes stay packed in LDS.  ds_read_b64_tr_b8 hands a lane the 8 bytes = 16 values of k of ONE column,
 //     i.e. the B operand of two v_mfma_f32_32x32x16_f16;
-//   * the loop is rolled (one group per iteration): a launch fetches its code cold, about 0.3 us per KiB executed;
 //   * split-K without atomics (5.6 M float atomics cost 75 us on this chip): each K-split writes its fp32 tile to the
 //     library workspace and a second small kernel adds the splits in a fixed order and rounds once to fp16 - results
 //     do not depend on timing.
@@ -44,6 +48,8 @@
 namespace {
 
 using namespace art::w4;
+
+template <int V> using Int = std::integral_constant<int, V>;
 
 constexpr int kThreads = 512;                       // 8 wavefronts: 4 column quarters x 2 k halves
 constexpr int BN = 128, GK = 128;                   // columns of a block, k of a quantisation group
@@ -95,25 +101,33 @@ __global__ __launch_bounds__(kThreads, MT == 4 ? 2 : 4) void gemm_w4a16_kernel(
   }
   if (wave == 0) qoff = 2u * cols.safe(2 * lane);                        // scales of columns 2 lane, 2 lane + 1
   if (wave == 1 && lane < 16) qoff = (unsigned int)cols.safe(8 * lane) >> 1;      // zero points of 8 columns; idle lanes re-read the first
-  const unsigned char* wbase = qweight + (size_t)g_begin * (GK / 2) * N;
-  const unsigned char* xbase = reinterpret_cast<const unsigned char*>(x + (size_t)m0 * K + (size_t)g_begin * GK);
-  const unsigned char* qbase = wave == 1 ? qzeros + (size_t)g_begin * (N / 2) : reinterpret_cast<const unsigned char*>(scales + (size_t)g_begin * N);
-  const unsigned int qstep = wave == 1 ? N / 2 : 2 * N;
-  // Load j for ring slot `slot`: 0 packed weights, 1 scales and zero points, 2 .. MT + 1 x.  The slot of group i holds x of
+  const unsigned int wstep = (GK / 2) * N, qstep = wave == 1 ? N / 2 : 2 * N;
+  const art::u32x4_t wbuf = art::buffer_of(qweight + (size_t)g_begin * wstep), xbuf = art::buffer_of(x + (size_t)m0 * K + (size_t)g_begin * GK),
+                     qbuf = art::buffer_of(wave == 1 ? (const void*)(qzeros + (size_t)g_begin * qstep) : (const void*)(scales + (size_t)g_begin * N));
+  const unsigned int wlast = (groups - 1) * wstep, qlast = (groups - 1) * qstep, xlast = (groups - 1) * (GK * 2);
+  const unsigned int lds_w = lds0 + wave * 1024, lds_q = lds0 + wave * 256;
+  unsigned int wat = 0, qat = 0, xat = 0;           // the group whose loads go out next
+  // Load j for ring slot S: 0 packed weights, 1 scales and zero points, 2 .. MT + 1 x.  The slot of group i holds x of
   // group i and the weights of group i + 1.
-  auto issue = [&](unsigned int slot, int j) {
-    const unsigned int st = lds0 + slot;
-    if (j == 0) load_lds_x4(uniform(wbase), woff, st + wave * 1024);
-    else if (j == 1) load_lds_x1(uniform(qbase), qoff, st + W_BYTES + wave * 256);
-    else load_lds_x4(uniform(xbase), xoff[j - 2], st + W_BYTES + Q_BYTES + (wave + 8 * (j - 2)) * 1024);
+  auto issue = [&](auto s_tag, auto j_tag) {
+    constexpr unsigned int ST = decltype(s_tag)::value * STAGE;
+    constexpr int J = decltype(j_tag)::value;
+    if constexpr (J == 0) art::buffer_lds_x4<ST>(wbuf, woff, wat, lds_w);
+    else if constexpr (J == 1) art::buffer_lds_x1<ST + W_BYTES>(qbuf, qoff, qat, lds_q);
+    else art::buffer_lds_x4<ST + W_BYTES + Q_BYTES + 8 * (J - 2) * 1024>(xbuf, xoff[J - 2], xat, lds_w);
   };
-  // The bases move on behind the loads of a group.  At the end they stay at the last one: it is fetched again, into
-  // slots that nobody reads, and the loop needs neither branches (a handful of them cost a tenth of a group's time) nor a
-  // varying count of loads.
-  auto next_weights = [&](int fetched) {
-    if (fetched + 1 < groups) { wbase += (size_t)(GK / 2) * N; qbase += qstep; }
+  auto issue_x = [&](auto s_tag) {
+    issue(s_tag, Int<2>{});
+    if constexpr (MT >= 2) issue(s_tag, Int<3>{});
+    if constexpr (MT >= 4) { issue(s_tag, Int<4>{}); issue(s_tag, Int<5>{}); }
   };
-  auto next_x = [&](int fetched) { if (fetched + 1 < groups) xbase += GK * 2; };
+  // At the end they stay at the last group: it is fetched again, into slots that nobody reads, and the loop needs neither
+  // branches (a handful of them cost a tenth of a group's time) nor a varying count of loads.
+  auto next_weights = [&]() {
+    wat = wat + wstep < wlast ? wat + wstep : wlast;
+    qat = qat + qstep < qlast ? qat + qstep : qlast;
+  };
+  auto next_x = [&]() { xat = xat + GK * 2 < xlast ? xat + GK * 2 : xlast; };
 
   // ROPE: the block is one head.  The angles that this thread needs at the end are fetched first.
   const int head = cols.n0 / BN;
@@ -179,16 +193,19 @@ __global__ __launch_bounds__(kThreads, MT == 4 ? 2 : 4) void gemm_w4a16_kernel(
   };
 
   // ---- prologue: weights of group 0 into slot 2, then slots 0 and 1
-  issue(2 * STAGE, 0);
-  issue(2 * STAGE, 1);
-  next_weights(0);
-#pragma unroll
-  for (int g = 0; g < 2; ++g) {
-#pragma unroll
-    for (int j = 0; j < L; ++j) issue(g * STAGE, j);
-    next_weights(g + 1);
-    next_x(g);
-  }
+  issue(Int<2>{}, Int<0>{});
+  issue(Int<2>{}, Int<1>{});
+  next_weights();
+  issue(Int<0>{}, Int<0>{});
+  issue(Int<0>{}, Int<1>{});
+  issue_x(Int<0>{});
+  next_weights();
+  next_x();
+  issue(Int<1>{}, Int<0>{});
+  issue(Int<1>{}, Int<1>{});
+  issue_x(Int<1>{});
+  next_weights();
+  next_x();
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(L) : "memory");       // loads return in order
   art_lds_barrier();
   read_weights(2 * STAGE, pk, 0);
@@ -200,49 +217,55 @@ __global__ __launch_bounds__(kThreads, MT == 4 ? 2 : 4) void gemm_w4a16_kernel(
 #pragma unroll
   for (int j = 0; j < 4; ++j) unpack(pk, 0, j);
   art_lds_barrier();                                // slot 2 is free again: it takes the weights of group 3 first
-  unsigned int s_cur = 0, s_next = STAGE, s_fill = 2 * STAGE;
-  issue(s_fill, 0);
-  issue(s_fill, 1);
-  next_weights(3);
+  issue(Int<2>{}, Int<0>{});
+  issue(Int<2>{}, Int<1>{});
+  next_weights();
 
   // A round multiplies 16 values of k per lane half and prepares the operands of the round behind it, in MT chunks: one
-  // MFMA, one read of x, 4 / MT unpacked pairs, at most two loads for the group two ahead.
-  auto round = [&](auto e_tag) {
-    constexpr int E = decltype(e_tag)::value;
+  // MFMA, one read of x, 4 / MT unpacked pairs, at most two loads.  S: the slot of the group.
+  auto chunk_of = [&](auto s_tag, auto e_tag, auto c_tag) {
+    constexpr int S = decltype(s_tag)::value, E = decltype(e_tag)::value, c = decltype(c_tag)::value;
     constexpr int kPairs = 4 / MT;
+    constexpr unsigned int s_cur = S * STAGE, s_next = (S + 1) % 3 * STAGE;
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (E == 0) issue(Int<(S + 2) % 3>{}, Int<2 + c>{});         // x of the group two ahead
+    if constexpr (E == 3 && c == 0) issue(s_tag, Int<0>{});                // weights of the group four ahead
+    if constexpr (E == 3 && c == MT - 1) issue(s_tag, Int<1>{});
+    if (E == 2 && c == 0) { read_weights(s_cur, pk_next, 0); read_scales(s_cur); }     // the weights of the next group came with x of this one
+    if (E == 2 && c == MT - 1) read_weights(s_cur, pk_next, 1);
+    if (E == 3 && c == 0) decode_scales();
+    E == 3 ? read_x(s_next, 0, c) : read_x(s_cur, (E + 1) & 3, c);
 #pragma unroll
-    for (int c = 0; c < MT; ++c) {
-      __builtin_amdgcn_sched_barrier(0);
-      if (E == 0) issue(s_fill, 2 + c);             // x of the group two ahead
-      if (E == 3 && c == 0) issue(s_fill, 0);       // weights of the group four ahead
-      if (E == 3 && c == MT - 1) issue(s_fill, 1);
-      if (E == 2 && c == 0) { read_weights(s_cur, pk_next, 0); read_scales(s_cur); }     // the weights of the next group came with x of this one
-      if (E == 2 && c == MT - 1) read_weights(s_cur, pk_next, 1);
-      if (E == 3 && c == 0) decode_scales();
-      E == 3 ? read_x(s_next, 0, c) : read_x(s_cur, (E + 1) & 3, c);
-#pragma unroll
-      for (int p = c * kPairs; p < (c + 1) * kPairs; ++p) unpack(E == 3 ? pk_next : pk, (E + 1) & 3, p);
-      multiply(E & 1, c);
-    }
+    for (int p = c * kPairs; p < (c + 1) * kPairs; ++p) unpack(E == 3 ? pk_next : pk, (E + 1) & 3, p);
+    multiply(E & 1, c);
+  };
+  auto round = [&](auto s_tag, auto e_tag) {
+    chunk_of(s_tag, e_tag, Int<0>{});
+    if constexpr (MT >= 2) chunk_of(s_tag, e_tag, Int<1>{});
+    if constexpr (MT >= 4) { chunk_of(s_tag, e_tag, Int<2>{}); chunk_of(s_tag, e_tag, Int<3>{}); }
     __builtin_amdgcn_sched_barrier(0);
   };
-#pragma unroll 1
-  for (int i = 0; i < groups; ++i) {
-    round(std::integral_constant<int, 0>{});
-    next_x(i + 2);
-    round(std::integral_constant<int, 1>{});
-    round(std::integral_constant<int, 2>{});
+  auto group = [&](auto s_tag) {
+    round(s_tag, Int<0>{});
+    next_x();
+    round(s_tag, Int<1>{});
+    round(s_tag, Int<2>{});
     // The next slot is complete once only the loads of the slot behind it (weights, x) are outstanding, and everybody has read all of
     // this one, which then takes group i + 3.  Behind the last group the reads return old bytes; nothing uses them.
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(L) : "memory");
     art_lds_barrier();
-    s_fill = s_cur;
-    round(std::integral_constant<int, 3>{});
-    next_weights(i + 4);
-    s_cur = s_next;
-    s_next = 3 * STAGE - s_cur - s_fill;
+    round(s_tag, Int<3>{});
+    next_weights();
     pk[0] = pk_next[0];
     pk[1] = pk_next[1];
+  };
+  for (int left = groups;;) {                       // the slots are constants
+    group(Int<0>{});
+    if (--left == 0) break;
+    group(Int<1>{});
+    if (--left == 0) break;
+    group(Int<2>{});
+    if (--left == 0) break;
   }
 
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // nothing of the ring is on its way when its space is reused or given back
@@ -267,12 +290,12 @@ __global__ __launch_bounds__(kThreads, MT == 4 ? 2 : 4) void gemm_w4a16_kernel(
   for (int j = 0; j < KEEP; ++j) sum[j] += meet[(4 * KEEP * kh + j) * 64];
   if (work.splits > 1) {                            // 64 bytes and more of a row at a time
     if (!cols.inside(colpos)) return;
-    float* const to = partial + ((size_t)split * M + m0) * N + cols.at(colpos);
+    const PartialTile to(partial, split, M, N);
+    const unsigned int at = to.at(m0 + row_of(0), cols.at(colpos));
 #pragma unroll
     for (int j = 0; j < KEEP; ++j)
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-        if (m0 + row_of(j) + i < M) to[(size_t)(row_of(j) + i) * N] = sum[j][i];
+      for (int i = 0; i < 4; ++i) to.store(at, (j >> 2) * 32 + (j & 3) * 8 + i, sum[j][i]);
     return;
   }
   // fp16 results to LDS as [row][column], out in pieces of eight columns.
@@ -466,11 +489,11 @@ double estimate(int M, int K, int N, const Plan& p, int compute_units) {
   const double again = p.wide ? 0.0 : 1.5 * ((blocks - 1) / round);
   return c.fixed + again + groups * per_group + (p.splits > 1 ? 2.4 + (8.0 * p.splits + 2.0) * M * N / 4.4e6 : 0.0);
 }
-// What a form's 32-bit offsets (a block's rows of x and of the packed weights), its division by the number of column
+// What a form's 32-bit offsets (a block's rows of x and its packed weights), its division by the number of column
 // tiles and its grid hold.
 bool holds(const Plan& p, int K, int N, bool swiglu) {
-  const long long units = (long long)tile_count(N, swiglu, p.wide ? 256 : BN) * p.splits;
-  return 64LL * p.row_tiles * K <= 1LL << 32 && 64LL * N <= 1LL << 32 && units < (p.wide ? 1 << 19 : 1 << 16);
+  const long long units = (long long)tile_count(N, swiglu, p.wide ? 256 : BN) * p.splits, groups = (K / GK + p.splits - 1) / p.splits;
+  return 64LL * p.row_tiles * K <= 1LL << 32 && 64 * groups * N <= 1LL << 32 && units < (p.wide ? 1 << 19 : 1 << 16);
 }
 // False: no form takes these sizes.  `code` and `splits` are the caller's wishes (0: none); a form that does not hold the
 // sizes is replaced by one that does.

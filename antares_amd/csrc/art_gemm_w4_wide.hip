@@ -16,6 +16,11 @@
 //   * the chunk positions are swizzled so that every 16 lanes of a 16-byte read of x (rows 128 bytes apart), and of a
 //     transposing byte read of the weights, touch every bank once (SQ_LDS_BANK_CONFLICT 0.5 M cycles in a launch of 33 M
 //     wavefront cycles, 1003 rows over 4096 x 12288);
+//   * loads come from buffer descriptors, one scalar offset moves on from stage to stage; with four row tiles the ring slots are
+//     constants (the loop is three groups long; with eight the compiler spills in such a loop).  A group is 647 instructions with eight
+//     row tiles, 470 with four; with 64-bit addresses that stop at the last stage, and differences directly in front of their products (a
+//     wait state each), it was 711 and 549, and a K-split's sums left by ten instructions a store instead of two: 200 rows over
+//     11008 x 4096 38.7 -> 34.9 us, 1003 rows over 4096 x 12288 101.2 -> 99.1, 8192 x 2048 50.8 -> 47.7;
 //   * one round = 16 values of k per lane half = 2 MT MFMAs.  The operands of round e + 1 are read and unpacked between
 //     the MFMAs of round e, in four chunks fenced against the scheduler; each chunk also issues at most one load.  Left
 //     together the loads of a stage blocked every wavefront of the compute unit at once, about 700 cycles per stage.
@@ -30,6 +35,8 @@
 namespace {
 
 using namespace art::w4;
+
+template <int V> using Int = std::integral_constant<int, V>;
 
 constexpr int kThreads = 256;
 constexpr int BN = 256, SK = 64;                    // columns of a block, k of a stage
@@ -74,32 +81,37 @@ __global__ __launch_bounds__(kThreads, MT == 8 ? 1 : 2) void gemm_w4a16_wide_ker
     const int r = 8 * (wave + 4 * u) + (lane >> 3), row = m0 + r < M ? m0 + r : M - 1;
     xoff[u] = (unsigned int)(row - m0) * (2 * K) + (((lane & 7) ^ ((r >> 1) & 7)) * 16);
   }
-  const unsigned char* wbase = qweight + (size_t)g_begin * 64 * N;
-  const unsigned char* xbase = reinterpret_cast<const unsigned char*>(x + (size_t)m0 * K + (size_t)g_begin * 128);
   // scales and zero points share one load: wavefronts 0 and 1 fetch the scales of columns 2 d, 2 d + 1, half of
   // wavefront 2 the zero points of columns 8 (d - 128) .. + 7, the others repeat the first scales
   const bool is_zero = tid >= 128 && tid < 160;
   qoff = is_zero ? (unsigned int)cols.safe(8 * (tid - 128)) >> 1 : (tid < 128 ? 2u * cols.safe(2 * tid) : 0u);
-  const unsigned char* qbase = wave == 2 ? qzeros + (size_t)g_begin * (N / 2) : reinterpret_cast<const unsigned char*>(scales + (size_t)g_begin * N);
-  const unsigned int qstep = wave == 2 ? N / 2 : 2 * N;
+  const unsigned int wstep = 32u * N, qstep = wave == 2 ? N / 2 : 2 * N;
+  const art::u32x4_t wbuf = art::buffer_of(qweight + (size_t)g_begin * 64 * N), xbuf = art::buffer_of(x + (size_t)m0 * K + (size_t)g_begin * 128),
+                     qbuf = art::buffer_of(wave == 2 ? (const void*)(qzeros + (size_t)g_begin * qstep) : (const void*)(scales + (size_t)g_begin * N));
+  const unsigned int wlast = (steps - 1) * wstep, qlast = (g_count - 1) * qstep, xlast = (steps - 1) * (SK * 2);
+  const unsigned int lds_w = lds0 + wave * 1024, lds_q = lds0 + wave * 256;
+  unsigned int wat = 0, qat = 0, xat = 0;           // the stage whose loads go out next
 
-  // Load j of ring slot `slot`: 0, 1 packed weights, 2 scales and zero points, 3 .. MT + 2 x.  The weights run one
+  // Load j of ring slot `slot` (its offset): 0, 1 packed weights, 2 scales and zero points, 3 .. MT + 2 x.  The weights run one
   // stage ahead of x: slot of stage i holds x of stage i and the weights of stage i + 1.
-  auto issue = [&](unsigned int slot, int j) {
-    const unsigned int st = lds0 + slot;
-    if (j < 2) load_lds_x4(uniform(wbase), woff[j], st + (wave + 4 * j) * 1024);
-    else if (j == 2) load_lds_x1(uniform(qbase), qoff, st + W_BYTES + wave * 256);
-    else load_lds_x4(uniform(xbase), xoff[j - 3], st + W_BYTES + Q_BYTES + (wave + 4 * (j - 3)) * 1024);
+  auto issue = [&](unsigned int slot, auto j_tag) {
+    constexpr int J = decltype(j_tag)::value;
+    if constexpr (J < 2) art::buffer_lds_x4<4 * J * 1024>(wbuf, woff[J], wat, lds_w + slot);
+    else if constexpr (J == 2) art::buffer_lds_x1<W_BYTES>(qbuf, qoff, qat, lds_q + slot);
+    else art::buffer_lds_x4<W_BYTES + Q_BYTES + 4 * (J - 3) * 1024>(xbuf, xoff[J - 3], xat, lds_w + slot);
   };
-  // The bases move on behind the loads of a stage.  At the end they stay at the last one: it is fetched again, into
-  // slots that nobody reads, and the loop needs neither branches nor a varying count of loads.
-  auto next_weights = [&](int fetched) {            // stage whose weights were just fetched
-    if (fetched + 1 < steps) {
-      wbase += (size_t)32 * N;
-      if (fetched & 1) qbase += qstep;
-    }
+  auto issue_weights = [&](unsigned int slot) { issue(slot, Int<0>{}); issue(slot, Int<1>{}); issue(slot, Int<2>{}); };
+  auto issue_x = [&](unsigned int slot) {
+    issue(slot, Int<3>{}); issue(slot, Int<4>{}); issue(slot, Int<5>{}); issue(slot, Int<6>{});
+    if constexpr (MT == 8) { issue(slot, Int<7>{}); issue(slot, Int<8>{}); issue(slot, Int<9>{}); issue(slot, Int<10>{}); }
   };
-  auto next_x = [&](int fetched) { if (fetched + 1 < steps) xbase += SK * 2; };
+  // At the end they stay at the last stage: it is fetched again, into slots that nobody reads, and the loop needs neither
+  // branches nor a varying count of loads.  A group is two stages.
+  auto next_weights = [&](auto odd_tag) {           // of the stage whose weights were just fetched
+    wat = wat + wstep < wlast ? wat + wstep : wlast;
+    if constexpr (decltype(odd_tag)::value == 1) qat = qat + qstep < qlast ? qat + qstep : qlast;
+  };
+  auto next_x = [&]() { xat = xat + SK * 2 < xlast ? xat + SK * 2 : xlast; };
 
   // ---- operand roles.  A transposing read takes 8 byte-rows x 16 columns per 16 lanes: lane s16 supplies the 8-byte
   // piece (row s16 / 2, half s16 % 2) and receives the 8 bytes (16 values of k) of column s16.  Lanes 16-31 take the
@@ -148,9 +160,14 @@ __global__ __launch_bounds__(kThreads, MT == 8 ? 1 : 2) void gemm_w4a16_wide_ker
   auto read_x = [&](unsigned int slot, int e, int t) {
     fa[e & 1][t] = *reinterpret_cast<const h8*>(smem + slot + a_off[e] + t * 4096);
   };
-  // pair j of column tile ct for round e.  Byte j of the word holds k = 2 j (low nibble) and 2 j + 1 (high nibble).
-  auto unpack = [&](int par, int e, int ct, int j) {
-    fb[e & 1][ct][j] = (as_h2(and_or(nibble_pair<true>((unsigned int)pk[par][e >> 1][ct][e & 1], j), mg.mask, mg.bias)) - zz2[ct]) * s2[ct];
+  // pairs j and j + 1 (j even) of column tile ct for round e.  Byte j of the word holds k = 2 j (low nibble) and 2 j + 1 (high
+  // nibble).  Step by step for both: a difference directly in front of its product costs a wait state.
+  auto unpack_two = [&](int par, int e, int ct, int j) {
+    const unsigned int w = (unsigned int)pk[par][e >> 1][ct][e & 1];
+    const h2 a = as_h2(and_or(nibble_pair<true>(w, j), mg.mask, mg.bias)), b = as_h2(and_or(nibble_pair<true>(w, j + 1), mg.mask, mg.bias));
+    const h2 da = a - zz2[ct], db = b - zz2[ct];
+    fb[e & 1][ct][j] = da * s2[ct];
+    fb[e & 1][ct][j + 1] = db * s2[ct];
   };
   auto multiply = [&](int slot, int t) {
 #pragma unroll
@@ -162,17 +179,16 @@ __global__ __launch_bounds__(kThreads, MT == 8 ? 1 : 2) void gemm_w4a16_wide_ker
   };
 
   // ---- prologue: weights of stage 0 into slot 2, then slots 0 and 1
-#pragma unroll
-  for (int j = 0; j < 3; ++j) issue(2 * STAGE, j);
-  next_weights(0);
-#pragma unroll
-  for (int j = 0; j < L; ++j) issue(0, j);
-  next_weights(1);
-  next_x(0);
-#pragma unroll
-  for (int j = 0; j < L; ++j) issue(STAGE, j);
-  next_weights(2);
-  next_x(1);
+  issue_weights(2 * STAGE);
+  next_weights(Int<0>{});
+  issue_weights(0);
+  issue_x(0);
+  next_weights(Int<1>{});
+  next_x();
+  issue_weights(STAGE);
+  issue_x(STAGE);
+  next_weights(Int<0>{});
+  next_x();
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(L) : "memory");       // loads return in order
   art_lds_barrier();
 #pragma unroll
@@ -184,81 +200,94 @@ __global__ __launch_bounds__(kThreads, MT == 8 ? 1 : 2) void gemm_w4a16_wide_ker
 #pragma unroll
   for (int ct = 0; ct < 2; ++ct)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) unpack(0, 0, ct, j);
+    for (int j = 0; j < 4; j += 2) unpack_two(0, 0, ct, j);
   art_lds_barrier();                                // slot 2 is free again
-  unsigned int s_cur = 0, s_next = STAGE, s_fill = 2 * STAGE;
 
   // A round multiplies 16 values of k per lane half and prepares the operands of the round behind it, in four chunks:
-  // MT / 2 MFMAs, MT / 4 reads of x, two unpacked pairs and one load for the stage two ahead.
+  // MT / 2 MFMAs, MT / 4 reads of x, two unpacked pairs and one load for the stage two ahead.  PAR: which half of its group the
+  // stage is.
   constexpr int CT_ = MT / 4;                       // row tiles per chunk
-  auto round = [&](int i, auto par_tag, auto e_tag) {
-    constexpr int PAR = decltype(par_tag)::value, E = decltype(e_tag)::value;
+  auto chunk_of = [&](unsigned int s_cur, unsigned int s_next, unsigned int s_fill, auto par_tag, auto e_tag, auto c_tag) {
+    constexpr int PAR = decltype(par_tag)::value, E = decltype(e_tag)::value, c = decltype(c_tag)::value;
+    __builtin_amdgcn_sched_barrier(0);
+    constexpr int kFirst[4] = {3, 7, 11, 0};        // loads of rounds 0, 1, 2; round 3 starts the next stage's
+    constexpr int j = kFirst[E] + c;
+    if constexpr (E == 3 ? c < 3 : j < L) issue(E == 3 ? s_cur : s_fill, Int<j>{});
+    if (E == 2) read_weights(s_cur, PAR ^ 1, c);    // the weights of stage i + 1 came with x of stage i
+    if (E == 2 && PAR == 1 && c < 2) read_scales(s_cur, c);
+    if (E == 3 && PAR == 1 && c == 0) { decode_scales(0); decode_scales(1); }
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      __builtin_amdgcn_sched_barrier(0);
-      constexpr int kFirst[4] = {3, 7, 11, 0};      // loads of rounds 0, 1, 2; round 3 starts the next stage's
-      const int j = kFirst[E] + c;
-      if (E == 3 ? c < 3 : j < L) issue(s_fill, j);
-      if (E == 2) read_weights(s_cur, PAR ^ 1, c);  // the weights of stage i + 1 came with x of stage i
-      if (E == 2 && PAR == 1 && c < 2) read_scales(s_cur, c);
-      if (E == 3 && PAR == 1 && c == 0) { decode_scales(0); decode_scales(1); }
+    for (int t = c * CT_; t < (c + 1) * CT_; ++t) E == 3 ? read_x(s_next, 0, t) : read_x(s_cur, (E + 1) & 3, t);
+    unpack_two(E == 3 ? PAR ^ 1 : PAR, (E + 1) & 3, c >> 1, 2 * (c & 1));
 #pragma unroll
-      for (int t = c * CT_; t < (c + 1) * CT_; ++t) E == 3 ? read_x(s_next, 0, t) : read_x(s_cur, (E + 1) & 3, t);
+    for (int t = c * CT_; t < (c + 1) * CT_; ++t) multiply(E & 1, t);
 #pragma unroll
-      for (int p = 2 * c; p < 2 * c + 2; ++p) unpack(E == 3 ? PAR ^ 1 : PAR, (E + 1) & 3, p >> 2, p & 3);
-#pragma unroll
-      for (int t = c * CT_; t < (c + 1) * CT_; ++t) multiply(E & 1, t);
-#pragma unroll
-      for (int m = 0; m < 2 * CT_; ++m) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-        __builtin_amdgcn_sched_group_barrier(0x002, MT == 8 ? 3 : 5, 0);
-      }
+    for (int m = 0; m < 2 * CT_; ++m) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x002, MT == 8 ? 3 : 5, 0);
     }
+  };
+  auto round = [&](unsigned int s_cur, unsigned int s_next, unsigned int s_fill, auto par_tag, auto e_tag) {
+    chunk_of(s_cur, s_next, s_fill, par_tag, e_tag, Int<0>{});
+    chunk_of(s_cur, s_next, s_fill, par_tag, e_tag, Int<1>{});
+    chunk_of(s_cur, s_next, s_fill, par_tag, e_tag, Int<2>{});
+    chunk_of(s_cur, s_next, s_fill, par_tag, e_tag, Int<3>{});
     __builtin_amdgcn_sched_barrier(0);
   };
-  auto stage = [&](int i, auto par_tag) {
-    using E0 = std::integral_constant<int, 0>;
-    using E1 = std::integral_constant<int, 1>;
-    using E2 = std::integral_constant<int, 2>;
-    using E3 = std::integral_constant<int, 3>;
-    round(i, par_tag, E0{});
-    round(i, par_tag, E1{});
-    round(i, par_tag, E2{});
-    next_x(i + 2);
+  auto stage = [&](unsigned int s_cur, unsigned int s_next, unsigned int s_fill, auto par_tag) {
+    round(s_cur, s_next, s_fill, par_tag, Int<0>{});
+    round(s_cur, s_next, s_fill, par_tag, Int<1>{});
+    round(s_cur, s_next, s_fill, par_tag, Int<2>{});
+    next_x();
     // The next slot is complete once only the x loads of stage i + 2 are outstanding ... and everybody has read all of
     // this one, which then takes stage i + 3.  Behind the last stage the reads return old bytes; nothing uses them.
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(L) : "memory");
     art_lds_barrier();
-    const unsigned int free_slot = s_cur;
-    s_fill = free_slot;
-    round(i, par_tag, E3{});
-    next_weights(i + 4);
-    s_cur = s_next;
-    s_next = 3 * STAGE - s_cur - s_fill;
+    round(s_cur, s_next, s_fill, par_tag, Int<3>{});
+    next_weights(par_tag);                          // of stage i + 4, the same half of its group
   };
   // the weights of slot 2 (stage 3) open the pattern: from here on every round 3 fetches the weights of the next slot
-#pragma unroll
-  for (int j = 0; j < 3; ++j) issue(s_fill, j);
-  next_weights(3);
+  issue_weights(2 * STAGE);
+  next_weights(Int<1>{});
+  if constexpr (MT == 8) {                          // (with constants as below the compiler spills in the loop)
+    unsigned int s_cur = 0, s_next = STAGE, s_fill = 2 * STAGE;
 #pragma unroll 1
-  for (int i = 0; i < steps; i += 2) {
-    stage(i, std::integral_constant<int, 0>{});
-    stage(i + 1, std::integral_constant<int, 1>{});
+    for (int left = g_count; left > 0; --left) {
+      stage(s_cur, s_next, s_fill, Int<0>{});
+      stage(s_next, s_fill, s_cur, Int<1>{});
+      const unsigned int first = s_cur;
+      s_cur = s_fill;
+      s_fill = s_next;
+      s_next = first;
+    }
+  } else {
+    for (int left = g_count;;) {                    // the slots are constants
+      stage(0, STAGE, 2 * STAGE, Int<0>{});
+      stage(STAGE, 2 * STAGE, 0, Int<1>{});
+      if (--left == 0) break;
+      stage(2 * STAGE, 0, STAGE, Int<0>{});
+      stage(0, STAGE, 2 * STAGE, Int<1>{});
+      if (--left == 0) break;
+      stage(STAGE, 2 * STAGE, 0, Int<0>{});
+      stage(2 * STAGE, 0, STAGE, Int<1>{});
+      if (--left == 0) break;
+    }
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // nothing of the ring is on its way when its space is reused or given back
 
   // Accumulator element r of row tile t is row t * 32 + (r / 4) * 8 + 4 h + r % 4.
   if (splits > 1) {
+    const PartialTile to(partial, split, M, N);
 #pragma unroll
-    for (int t = 0; t < MT; ++t)
+    for (int ct = 0; ct < 2; ++ct) {
+      if (!cols.inside(colpos[ct])) continue;
+      const unsigned int at = to.at(m0 + 4 * h, cols.at(colpos[ct]));
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int row = m0 + t * 32 + (r >> 2) * 8 + h * 4 + (r & 3);
+      for (int t = 0; t < MT; ++t)
 #pragma unroll
-        for (int ct = 0; ct < 2; ++ct)
-          if (row < M && cols.inside(colpos[ct])) partial[((size_t)split * M + row) * N + cols.at(colpos[ct])] = acc[t][ct][r];
-      }
+        for (int r = 0; r < 16; ++r) to.store(at, t * 32 + (r >> 2) * 8 + (r & 3), acc[t][ct][r]);
+    }
     return;
   }
   _Float16* cs = reinterpret_cast<_Float16*>(smem);

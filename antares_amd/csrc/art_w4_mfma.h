@@ -63,6 +63,19 @@ struct TileColumns {
 };
 inline int tile_count(int N, bool swiglu, int bn) { return swiglu ? (N / 2 + bn / 2 - 1) / (bn / 2) : (N + bn - 1) / bn; }
 
+// The M x N sums of a K split on their way to the pass that adds them: a buffer of exactly that many bytes, so that what is stored to
+// rows past M is dropped on the way out, without a comparison and a branch for each store.
+struct PartialTile {
+  __amdgpu_buffer_rsrc_t buffer;
+  unsigned int row;                                 // bytes
+  __device__ __forceinline__ PartialTile(float* partial, int split, int M, int N)
+      : buffer(__builtin_amdgcn_make_buffer_rsrc(partial + (size_t)split * M * N, 0, M * N * 4, art::kBufferFlags)), row(4u * N) {}
+  __device__ __forceinline__ unsigned int at(int m, int n) const { return m * row + 4u * n; }
+  __device__ __forceinline__ void store(unsigned int at, int rows_on, float v) const {
+    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned int, v), buffer, (int)(at + rows_on * row), 0, 0);
+  }
+};
+
 // kRope: sine and cosine of row m, column j < 64 of a head at angles[64 m + j]; row m of q, k and v holds `heads` heads of 128.
 struct Rope {
   const float2* angles;
