@@ -68,7 +68,7 @@ struct Work {
   int groups, longer;                               // groups of a K split; the first `longer` have one more
 };
 
-template <int MT, Tail TAIL>
+template <int MT, Tail TAIL, bool FAR = false>
 __global__ __launch_bounds__(kThreads, MT == 4 ? 2 : 4) void gemm_w4a16_kernel(
     const _Float16* __restrict__ x, const unsigned char* __restrict__ qweight, const _Float16* __restrict__ scales,
     const unsigned char* __restrict__ qzeros, _Float16* y, float* __restrict__ partial, int M, int K, int N, Work work, Magic mg,
@@ -101,33 +101,29 @@ __global__ __launch_bounds__(kThreads, MT == 4 ? 2 : 4) void gemm_w4a16_kernel(
   }
   if (wave == 0) qoff = 2u * cols.safe(2 * lane);                        // scales of columns 2 lane, 2 lane + 1
   if (wave == 1 && lane < 16) qoff = (unsigned int)cols.safe(8 * lane) >> 1;      // zero points of 8 columns; idle lanes re-read the first
-  const unsigned int wstep = (GK / 2) * N, qstep = wave == 1 ? N / 2 : 2 * N;
-  const art::u32x4_t wbuf = art::buffer_of(qweight + (size_t)g_begin * wstep), xbuf = art::buffer_of(x + (size_t)m0 * K + (size_t)g_begin * GK),
-                     qbuf = art::buffer_of(wave == 1 ? (const void*)(qzeros + (size_t)g_begin * qstep) : (const void*)(scales + (size_t)g_begin * N));
-  const unsigned int wlast = (groups - 1) * wstep, qlast = (groups - 1) * qstep, xlast = (groups - 1) * (GK * 2);
+  const unsigned int qstep = wave == 1 ? N / 2 : 2 * N;
+  Rows<FAR> w_rows(qweight + (size_t)g_begin * (GK / 2) * N, (GK / 2) * N, groups), x_rows(x + (size_t)m0 * K + (size_t)g_begin * GK, GK * 2, groups),
+      q_rows(wave == 1 ? (const void*)(qzeros + (size_t)g_begin * qstep) : (const void*)(scales + (size_t)g_begin * N), qstep, groups);
   const unsigned int lds_w = lds0 + wave * 1024, lds_q = lds0 + wave * 256;
-  unsigned int wat = 0, qat = 0, xat = 0;           // the group whose loads go out next
   // Load j for ring slot S: 0 packed weights, 1 scales and zero points, 2 .. MT + 1 x.  The slot of group i holds x of
   // group i and the weights of group i + 1.
   auto issue = [&](auto s_tag, auto j_tag) {
     constexpr unsigned int ST = decltype(s_tag)::value * STAGE;
     constexpr int J = decltype(j_tag)::value;
-    if constexpr (J == 0) art::buffer_lds_x4<ST>(wbuf, woff, wat, lds_w);
-    else if constexpr (J == 1) art::buffer_lds_x1<ST + W_BYTES>(qbuf, qoff, qat, lds_q);
-    else art::buffer_lds_x4<ST + W_BYTES + Q_BYTES + 8 * (J - 2) * 1024>(xbuf, xoff[J - 2], xat, lds_w);
+    if constexpr (J == 0) buffer_lds_x4<ST>(w_rows.buffer, woff, w_rows.at, lds_w);
+    else if constexpr (J == 1) buffer_lds_x1<ST + W_BYTES>(q_rows.buffer, qoff, q_rows.at, lds_q);
+    else buffer_lds_x4<ST + W_BYTES + Q_BYTES + 8 * (J - 2) * 1024>(x_rows.buffer, xoff[J - 2], x_rows.at, lds_w);
   };
   auto issue_x = [&](auto s_tag) {
     issue(s_tag, Int<2>{});
     if constexpr (MT >= 2) issue(s_tag, Int<3>{});
     if constexpr (MT >= 4) { issue(s_tag, Int<4>{}); issue(s_tag, Int<5>{}); }
   };
-  // At the end they stay at the last group: it is fetched again, into slots that nobody reads, and the loop needs neither
-  // branches (a handful of them cost a tenth of a group's time) nor a varying count of loads.
   auto next_weights = [&]() {
-    wat = wat + wstep < wlast ? wat + wstep : wlast;
-    qat = qat + qstep < qlast ? qat + qstep : qlast;
+    w_rows.next();
+    q_rows.next();
+    if (w_rows.far()) { w_rows.rebase(); q_rows.rebase(); }
   };
-  auto next_x = [&]() { xat = xat + GK * 2 < xlast ? xat + GK * 2 : xlast; };
 
   // ROPE: the block is one head.  The angles that this thread needs at the end are fetched first.
   const int head = cols.n0 / BN;
@@ -200,12 +196,12 @@ __global__ __launch_bounds__(kThreads, MT == 4 ? 2 : 4) void gemm_w4a16_kernel(
   issue(Int<0>{}, Int<1>{});
   issue_x(Int<0>{});
   next_weights();
-  next_x();
+  x_rows.next();
   issue(Int<1>{}, Int<0>{});
   issue(Int<1>{}, Int<1>{});
   issue_x(Int<1>{});
   next_weights();
-  next_x();
+  x_rows.next();
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(L) : "memory");       // loads return in order
   art_lds_barrier();
   read_weights(2 * STAGE, pk, 0);
@@ -247,7 +243,7 @@ __global__ __launch_bounds__(kThreads, MT == 4 ? 2 : 4) void gemm_w4a16_kernel(
   };
   auto group = [&](auto s_tag) {
     round(s_tag, Int<0>{});
-    next_x();
+    x_rows.next();
     round(s_tag, Int<1>{});
     round(s_tag, Int<2>{});
     // The next slot is complete once only the loads of the slot behind it (weights, x) are outstanding, and everybody has read all of
@@ -489,11 +485,13 @@ double estimate(int M, int K, int N, const Plan& p, int compute_units) {
   const double again = p.wide ? 0.0 : 1.5 * ((blocks - 1) / round);
   return c.fixed + again + groups * per_group + (p.splits > 1 ? 2.4 + (8.0 * p.splits + 2.0) * M * N / 4.4e6 : 0.0);
 }
-// What a form's 32-bit offsets (a block's rows of x and its packed weights), its division by the number of column
-// tiles and its grid hold.
+// What a form's 32-bit offsets (a block's rows of x and of the packed weights), its division by the number of column
+// tiles and its grid hold.  Where the packed weights of a split do not fit 32 bits, two of the forms are left.
+bool far(const Plan& p, int K, int N) { return 64LL * N * ((K / GK + p.splits - 1) / p.splits) > 1LL << 32; }
 bool holds(const Plan& p, int K, int N, bool swiglu) {
-  const long long units = (long long)tile_count(N, swiglu, p.wide ? 256 : BN) * p.splits, groups = (K / GK + p.splits - 1) / p.splits;
-  return 64LL * p.row_tiles * K <= 1LL << 32 && 64 * groups * N <= 1LL << 32 && units < (p.wide ? 1 << 19 : 1 << 16);
+  const long long units = (long long)tile_count(N, swiglu, p.wide ? 256 : BN) * p.splits;
+  return 64LL * p.row_tiles * K <= 1LL << 32 && 64LL * N <= 1LL << 32 && units < (p.wide ? 1 << 19 : 1 << 16) &&
+         (!far(p, K, N) || p.row_tiles == (p.wide ? 4 : 1));
 }
 // False: no form takes these sizes.  `code` and `splits` are the caller's wishes (0: none); a form that does not hold the
 // sizes is replaced by one that does.
@@ -563,24 +561,25 @@ int run_rows(const _Float16* xs, const unsigned char* qweight, const _Float16* s
   const bool norm_there = norm && p.splits > 1 && M <= 256 && N % 8 == 0 && N <= 8 * kNormThreads * kNormTurns &&
                           (((uintptr_t)ys | (uintptr_t)res | (uintptr_t)norm->weight | (uintptr_t)norm->out) % 16) == 0;
   if (p.wide) {
-    if (art::w4::gemm_wide(xs, qweight, scales, qzeros, ys, scratch, M, K, N, p.splits, p.row_tiles, res, tail, rope, st)) return 1;
+    if (art::w4::gemm_wide(xs, qweight, scales, qzeros, ys, scratch, M, K, N, p.splits, p.row_tiles, far(p, K, N), res, tail, rope, st)) return 1;
   } else {
-    static const decltype(&gemm_w4a16_kernel<1, kPlain>) kernels[3][3] = {
+    static const decltype(&gemm_w4a16_kernel<1, kPlain>) kernels[4][3] = {
         {gemm_w4a16_kernel<1, kPlain>, gemm_w4a16_kernel<1, kSwiglu>, gemm_w4a16_kernel<1, kRope>},
         {gemm_w4a16_kernel<2, kPlain>, gemm_w4a16_kernel<2, kSwiglu>, gemm_w4a16_kernel<2, kRope>},
-        {gemm_w4a16_kernel<4, kPlain>, gemm_w4a16_kernel<4, kSwiglu>, gemm_w4a16_kernel<4, kRope>}};
+        {gemm_w4a16_kernel<4, kPlain>, gemm_w4a16_kernel<4, kSwiglu>, gemm_w4a16_kernel<4, kRope>},
+        {gemm_w4a16_kernel<1, kPlain, true>, gemm_w4a16_kernel<1, kSwiglu, true>, gemm_w4a16_kernel<1, kRope, true>}};
     static bool configured = false;
     if (!configured) {
-      for (int i = 0; i < 3; ++i)
+      for (int i = 0; i < 4; ++i)
         for (int j = 0; j < 3; ++j)
-          ART_HIP(hipFuncSetAttribute((const void*)kernels[i][j], hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes(1 << i)));
+          ART_HIP(hipFuncSetAttribute((const void*)kernels[i][j], hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes(i == 3 ? 1 : 1 << i)));
       configured = true;
     }
     const int col_tiles = tile_count(N, swiglu, BN), m_blocks = (M + 32 * p.row_tiles - 1) / (32 * p.row_tiles);
     const int units = col_tiles * p.splits, G = K / GK;
     dim3 grid;
     const Work work{deal(units, m_blocks, grid), col_tiles, p.splits, (unsigned int)((0x100000000ull + col_tiles - 1) / col_tiles), G / p.splits, G % p.splits};
-    const auto kernel = kernels[p.row_tiles == 4 ? 2 : p.row_tiles - 1][tail];
+    const auto kernel = kernels[far(p, K, N) ? 3 : p.row_tiles == 4 ? 2 : p.row_tiles - 1][tail];
     kernel<<<grid, kThreads, lds_bytes(p.row_tiles), st>>>(xs, qweight, scales, qzeros, ys, scratch, M, K, N, work, kMagic, res, rope);
     ART_LAUNCH_CHECK();
   }

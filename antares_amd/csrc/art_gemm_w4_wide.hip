@@ -50,7 +50,7 @@ static_assert(128 * C_LD * 2 <= NS * stage_bytes(4), "128 staged output rows fit
 
 // kSwiglu: the matrix is gate | up (N / 2 columns each); a block owns 128 gate columns and the matching 128 up columns and
 // stores y[m, n] = fp16(silu(fp16(gate)) * fp16(up)), N / 2 columns.
-template <int MT, Tail TAIL>
+template <int MT, Tail TAIL, bool FAR>
 __global__ __launch_bounds__(kThreads, MT == 8 ? 1 : 2) void gemm_w4a16_wide_kernel(
     const _Float16* __restrict__ x, const unsigned char* __restrict__ qweight, const _Float16* __restrict__ scales,
     const unsigned char* __restrict__ qzeros, _Float16* y, float* __restrict__ partial, int M, int K, int N, int splits,
@@ -85,33 +85,31 @@ __global__ __launch_bounds__(kThreads, MT == 8 ? 1 : 2) void gemm_w4a16_wide_ker
   // wavefront 2 the zero points of columns 8 (d - 128) .. + 7, the others repeat the first scales
   const bool is_zero = tid >= 128 && tid < 160;
   qoff = is_zero ? (unsigned int)cols.safe(8 * (tid - 128)) >> 1 : (tid < 128 ? 2u * cols.safe(2 * tid) : 0u);
-  const unsigned int wstep = 32u * N, qstep = wave == 2 ? N / 2 : 2 * N;
-  const art::u32x4_t wbuf = art::buffer_of(qweight + (size_t)g_begin * 64 * N), xbuf = art::buffer_of(x + (size_t)m0 * K + (size_t)g_begin * 128),
-                     qbuf = art::buffer_of(wave == 2 ? (const void*)(qzeros + (size_t)g_begin * qstep) : (const void*)(scales + (size_t)g_begin * N));
-  const unsigned int wlast = (steps - 1) * wstep, qlast = (g_count - 1) * qstep, xlast = (steps - 1) * (SK * 2);
+  const unsigned int qstep = wave == 2 ? N / 2 : 2 * N;
+  Rows<FAR> w_rows(qweight + (size_t)g_begin * 64 * N, 32u * N, steps), x_rows(x + (size_t)m0 * K + (size_t)g_begin * 128, SK * 2, steps),
+      q_rows(wave == 2 ? (const void*)(qzeros + (size_t)g_begin * qstep) : (const void*)(scales + (size_t)g_begin * N), qstep, g_count);
   const unsigned int lds_w = lds0 + wave * 1024, lds_q = lds0 + wave * 256;
-  unsigned int wat = 0, qat = 0, xat = 0;           // the stage whose loads go out next
 
   // Load j of ring slot `slot` (its offset): 0, 1 packed weights, 2 scales and zero points, 3 .. MT + 2 x.  The weights run one
   // stage ahead of x: slot of stage i holds x of stage i and the weights of stage i + 1.
   auto issue = [&](unsigned int slot, auto j_tag) {
     constexpr int J = decltype(j_tag)::value;
-    if constexpr (J < 2) art::buffer_lds_x4<4 * J * 1024>(wbuf, woff[J], wat, lds_w + slot);
-    else if constexpr (J == 2) art::buffer_lds_x1<W_BYTES>(qbuf, qoff, qat, lds_q + slot);
-    else art::buffer_lds_x4<W_BYTES + Q_BYTES + 4 * (J - 3) * 1024>(xbuf, xoff[J - 3], xat, lds_w + slot);
+    if constexpr (J < 2) buffer_lds_x4<4 * J * 1024>(w_rows.buffer, woff[J], w_rows.at, lds_w + slot);
+    else if constexpr (J == 2) buffer_lds_x1<W_BYTES>(q_rows.buffer, qoff, q_rows.at, lds_q + slot);
+    else buffer_lds_x4<W_BYTES + Q_BYTES + 4 * (J - 3) * 1024>(x_rows.buffer, xoff[J - 3], x_rows.at, lds_w + slot);
   };
   auto issue_weights = [&](unsigned int slot) { issue(slot, Int<0>{}); issue(slot, Int<1>{}); issue(slot, Int<2>{}); };
   auto issue_x = [&](unsigned int slot) {
     issue(slot, Int<3>{}); issue(slot, Int<4>{}); issue(slot, Int<5>{}); issue(slot, Int<6>{});
     if constexpr (MT == 8) { issue(slot, Int<7>{}); issue(slot, Int<8>{}); issue(slot, Int<9>{}); issue(slot, Int<10>{}); }
   };
-  // At the end they stay at the last stage: it is fetched again, into slots that nobody reads, and the loop needs neither
-  // branches nor a varying count of loads.  A group is two stages.
-  auto next_weights = [&](auto odd_tag) {           // of the stage whose weights were just fetched
-    wat = wat + wstep < wlast ? wat + wstep : wlast;
-    if constexpr (decltype(odd_tag)::value == 1) qat = qat + qstep < qlast ? qat + qstep : qlast;
+  auto next_weights = [&](auto odd_tag) {           // of the stage whose weights were just fetched; a group is two stages
+    w_rows.next();
+    if constexpr (decltype(odd_tag)::value == 1) {
+      q_rows.next();
+      if (w_rows.far()) { w_rows.rebase(); q_rows.rebase(); }
+    }
   };
-  auto next_x = [&]() { xat = xat + SK * 2 < xlast ? xat + SK * 2 : xlast; };
 
   // ---- operand roles.  A transposing read takes 8 byte-rows x 16 columns per 16 lanes: lane s16 supplies the 8-byte
   // piece (row s16 / 2, half s16 % 2) and receives the 8 bytes (16 values of k) of column s16.  Lanes 16-31 take the
@@ -184,11 +182,11 @@ __global__ __launch_bounds__(kThreads, MT == 8 ? 1 : 2) void gemm_w4a16_wide_ker
   issue_weights(0);
   issue_x(0);
   next_weights(Int<1>{});
-  next_x();
+  x_rows.next();
   issue_weights(STAGE);
   issue_x(STAGE);
   next_weights(Int<0>{});
-  next_x();
+  x_rows.next();
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(L) : "memory");       // loads return in order
   art_lds_barrier();
 #pragma unroll
@@ -239,7 +237,7 @@ __global__ __launch_bounds__(kThreads, MT == 8 ? 1 : 2) void gemm_w4a16_wide_ker
     round(s_cur, s_next, s_fill, par_tag, Int<0>{});
     round(s_cur, s_next, s_fill, par_tag, Int<1>{});
     round(s_cur, s_next, s_fill, par_tag, Int<2>{});
-    next_x();
+    x_rows.next();
     // The next slot is complete once only the x loads of stage i + 2 are outstanding ... and everybody has read all of
     // this one, which then takes stage i + 3.  Behind the last stage the reads return old bytes; nothing uses them.
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(L) : "memory");
@@ -356,19 +354,19 @@ __global__ __launch_bounds__(kThreads, MT == 8 ? 1 : 2) void gemm_w4a16_wide_ker
   }
 }
 
-template <int MT, Tail TAIL>
+template <int MT, Tail TAIL, bool FAR = false>
 int launch(const _Float16* x, const unsigned char* qweight, const _Float16* scales, const unsigned char* qzeros, _Float16* y,
            float* partial, int M, int K, int N, int splits, const _Float16* residual, const Rope& rope, hipStream_t stream) {
   static bool configured = false;
   if (!configured) {
-    ART_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_w4a16_wide_kernel<MT, TAIL>), hipFuncAttributeMaxDynamicSharedMemorySize,
+    ART_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_w4a16_wide_kernel<MT, TAIL, FAR>), hipFuncAttributeMaxDynamicSharedMemorySize,
                                 (int)lds_bytes(MT)));
     configured = true;
   }
   const int col_tiles = tile_count(N, TAIL == kSwiglu, BN), m_blocks = (M + 32 * MT - 1) / (32 * MT);
   dim3 grid;
   const Deal dealt = deal(col_tiles * splits, m_blocks, grid);
-  gemm_w4a16_wide_kernel<MT, TAIL><<<grid, kThreads, lds_bytes(MT), stream>>>(
+  gemm_w4a16_wide_kernel<MT, TAIL, FAR><<<grid, kThreads, lds_bytes(MT), stream>>>(
       x, qweight, scales, qzeros, y, partial, M, K, N, splits, dealt, make_div((unsigned)col_tiles), K / 128 / splits, K / 128 % splits,
       kMagic, residual, rope);
   ART_LAUNCH_CHECK();
@@ -378,9 +376,10 @@ int launch(const _Float16* x, const unsigned char* qweight, const _Float16* scal
 }  // namespace
 
 int art::w4::gemm_wide(const _Float16* x, const unsigned char* qweight, const _Float16* scales, const unsigned char* qzeros, _Float16* y,
-                       float* partial, int M, int K, int N, int splits, int row_tiles, const _Float16* residual, Tail tail, const Rope& rope,
+                       float* partial, int M, int K, int N, int splits, int row_tiles, bool far, const _Float16* residual, Tail tail, const Rope& rope,
                        hipStream_t stream) {
-  static const decltype(&launch<4, kPlain>) by_rows[2][3] = {{launch<4, kPlain>, launch<4, kSwiglu>, launch<4, kRope>},
-                                                             {launch<8, kPlain>, launch<8, kSwiglu>, launch<8, kRope>}};
-  return by_rows[row_tiles == 8][tail](x, qweight, scales, qzeros, y, partial, M, K, N, splits, residual, rope, stream);
+  static const decltype(&launch<4, kPlain>) by_rows[3][3] = {{launch<4, kPlain>, launch<4, kSwiglu>, launch<4, kRope>},
+                                                             {launch<8, kPlain>, launch<8, kSwiglu>, launch<8, kRope>},
+                                                             {launch<4, kPlain, true>, launch<4, kSwiglu, true>, launch<4, kRope, true>}};
+  return by_rows[far ? 2 : row_tiles == 8][tail](x, qweight, scales, qzeros, y, partial, M, K, N, splits, residual, rope, stream);
 }

@@ -9,9 +9,10 @@ using ::art::Div;
 using ::art::make_div;
 using ::art::over;
 
-using ::art::load_lds_x1;
-using ::art::load_lds_x4;
-using ::art::uniform;
+using ::art::buffer_lds_x1;
+using ::art::buffer_lds_x4;
+using ::art::buffer_of;
+using ::art::u32x4_t;
 
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 typedef h8 h8_by_8 __attribute__((aligned(8)));      // rows that are 8-byte aligned
@@ -62,6 +63,33 @@ struct TileColumns {
   __device__ __forceinline__ int safe(int pos) const { return inside(pos) ? at(pos) : 0; }
 };
 inline int tile_count(int N, bool swiglu, int bn) { return swiglu ? (N / 2 + bn / 2 - 1) / (bn / 2) : (N + bn - 1) / bn; }
+
+// Rows of memory that a block fetches one after another, `step` bytes apart: a descriptor and the offset of the next.  Behind the last
+// row it stays there: that one is fetched again, into slots that nobody reads, and the loop needs neither branches nor a varying
+// count of loads.  Offsets are 32 bits; FAR, for more than that: wherever one has passed 2 GiB, the descriptor moves on (rebase; in
+// every kernel it would cost 2 to 3 %).
+template <bool FAR> struct Rows {
+  u32x4_t buffer;
+  unsigned int at, step, last;
+  unsigned long long end;                           // FAR: from the descriptor's base to the last row
+  __device__ __forceinline__ Rows(const void* base, unsigned int bytes, int count) : buffer(buffer_of(base)), at(0), step(bytes), last(bytes * (count - 1)) {
+    if constexpr (FAR) {
+      end = (unsigned long long)bytes * (unsigned int)(count - 1);
+      set_last();
+    }
+  }
+  __device__ __forceinline__ void set_last() { last = end > 0xffffffffull ? 0xffffffffu : (unsigned int)end; }
+  __device__ __forceinline__ void next() { at = at + step < last ? at + step : last; }
+  __device__ __forceinline__ bool far() const { return FAR && (int)at < 0; }
+  __device__ __forceinline__ void rebase() {
+    const unsigned long long base = ((unsigned long long)buffer[1] << 32 | buffer[0]) + at;
+    buffer[0] = (unsigned int)base;
+    buffer[1] = (unsigned int)(base >> 32);
+    end -= at;
+    at = 0;
+    set_last();
+  }
+};
 
 // The M x N sums of a K split on their way to the pass that adds them: a buffer of exactly that many bytes, so that what is stored to
 // rows past M is dropped on the way out, without a comparison and a branch for each store.
@@ -144,9 +172,10 @@ __device__ __forceinline__ h4 swiglu4(h4 g, h4 u) {
 }
 
 // Large batches (art_gemm_w4_wide.hip): one launch over blocks of 32 row_tiles rows x 256 columns, K cut into `splits`;
-// with splits > 1 the fp32 tiles go to `partial` [splits][M][N].  row_tiles is 4 or 8.  No residual but with kPlain.
+// with splits > 1 the fp32 tiles go to `partial` [splits][M][N].  row_tiles is 4 or 8; far (the packed weights of a split are 4 GiB and
+// more): 4.  No residual but with kPlain.
 int gemm_wide(const _Float16* x, const unsigned char* qweight, const _Float16* scales, const unsigned char* qzeros, _Float16* y,
-              float* partial, int M, int K, int N, int splits, int row_tiles, const _Float16* residual, Tail tail, const Rope& rope, hipStream_t stream);
+              float* partial, int M, int K, int N, int splits, int row_tiles, bool far, const _Float16* residual, Tail tail, const Rope& rope, hipStream_t stream);
 
 }  // namespace w4
 }  // namespace art

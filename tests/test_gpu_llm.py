@@ -580,3 +580,29 @@ def test_sum_of_squares_buffers_are_checked(autort):
         autort.ops.gemv_w4a16_fused(x, qw, sc, qz, sumsq_out=a, sumsq_clear=a)
     with pytest.raises(TypeError, match='sum-of-squares buffer'):
         autort.ops.gemv_w4a16_fused(x, qw, sc, qz, sumsq_out=torch.zeros(8, dtype=torch.int64, device=dev))
+
+
+@pytest.mark.parametrize('M,code', [(5, 256 + 1), (5, 1024 + 1), (130, 2048 + 1), (5, 1024 + 2)])
+def test_int4_products_of_more_than_4_gib_of_packed_weights(autort, M, code):
+    """K x N of 257 groups x 262144 columns: the offsets of a block's weights pass 2 GiB and 4 GiB (in two K-splits: 2 GiB).  Columns
+    at both ends and in the middle against float64 sums of the same float16 weights: float16 rounding (2^-11) and float32 sums
+    of 32896 terms (their error is at most 2^-24 times some hundred partial sums)."""
+    from ctypes import c_void_p
+    from antares_amd.runtime import capi
+    note(f'more than 4 GiB M={M} code={code}')
+    dev, K, N = autort.device(), 257 * 128, 262144
+    g = torch.Generator(device=dev).manual_seed(M)
+    q = torch.randint(0, 256, (K // 2, N), generator=g, device=dev, dtype=torch.uint8)
+    z = torch.randint(0, 256, (K // 128, N // 2), generator=g, device=dev, dtype=torch.uint8)
+    s = (torch.rand(K // 128, N, generator=g, device=dev) * 0.019 + 0.001).half()
+    x = torch.randn(M, K, generator=g, device=dev).half()
+    y = torch.full((M, N), float('nan'), dtype=torch.float16, device=dev)
+    capi.check(capi.lib().art_gemm_w4a16_tuned(*(c_void_p(t.data_ptr()) for t in (x, q, s, z, y)), M, K, N, code, c_void_p(torch.cuda.current_stream().cuda_stream)))
+    cols = torch.cat([torch.arange(0, 16), torch.arange(N // 2 - 8, N // 2 + 8), torch.arange(N - 16, N)]).to(dev)
+    qc, zc = q[:, cols], z[:, cols // 2]
+    w = torch.stack([qc & 15, qc >> 4], 1).reshape(K, -1).half()
+    zero = torch.where(cols % 2 == 0, zc & 15, zc >> 4).half().repeat_interleave(128, 0)
+    w = (w - zero) * s[:, cols].repeat_interleave(128, 0)
+    want, got = (x.double() @ w.double()), y[:, cols].double()
+    assert ((got - want).abs() <= want.abs() * 2.0 ** -10 + 2e-3).all(), (got - want).abs().max()
+    assert not torch.isnan(y).any()
