@@ -388,48 +388,73 @@ template <int SPLITS> __global__ __launch_bounds__(256) void gemm_w4a16_combine_
 // elements stay in registers, 8 per thread and turn (N % 8 == 0, N <= 8192; as many threads as a row of up to 4096 has
 // pieces of 8).  Bound by the launch: instead of two launches of 2 us and more, one; a layer of the 32-layer model's prompt pass has
 // two of them: 8 layers 608 -> 594 us at 8 tokens, 776 -> 750 at 50, 962 -> 925 at 100, 1345 -> 1337 at 200 (fewer K-splits meet).
+// The sum over a row is bound by its steps: by DPP instead of six trips through LDS, the wavefronts' sums read at once, product and pass
+// 9.1 -> 8.9 us at 8 rows over 4096 x 4096, 14.3 -> 14.0 at 128 rows, 2048 x 2048 6.5 -> 6.2 and 9.2 -> 8.9.
 constexpr int kNormThreads = 512, kNormTurns = 2;
-template <int SPLITS> __global__ __launch_bounds__(kNormThreads) void gemm_w4a16_combine_norm_kernel(const float* __restrict__ partial, _Float16* y, int N,
-                                                                                long long split_stride, int splits, const _Float16* residual,
-                                                                                const _Float16* __restrict__ weight, _Float16* __restrict__ norm_out, float eps) {
-  typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+// Sum over the 64 lanes of a wavefront; every lane gets it.
+__device__ __forceinline__ float wave_sum(float v) {
+#define ART_DPP_ADD(ctrl) v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), ctrl, 0xf, 0xf, false))
+  ART_DPP_ADD(0xB1);                                // quad_perm [1,0,3,2]
+  ART_DPP_ADD(0x4E);                                // quad_perm [2,3,0,1]
+  ART_DPP_ADD(0x141);                               // row_half_mirror
+  ART_DPP_ADD(0x140);                               // row_mirror
+#undef ART_DPP_ADD
+  const int b = __builtin_bit_cast(int, v);
+  return (__builtin_bit_cast(float, __builtin_amdgcn_readlane(b, 0)) + __builtin_bit_cast(float, __builtin_amdgcn_readlane(b, 16))) +
+         (__builtin_bit_cast(float, __builtin_amdgcn_readlane(b, 32)) + __builtin_bit_cast(float, __builtin_amdgcn_readlane(b, 48)));
+}
+template <int SPLITS> __global__ __launch_bounds__(kNormThreads) void gemm_w4a16_combine_norm_kernel(const float* __restrict__ partial, const _Float16* residual,
+                                                                                const _Float16* __restrict__ weight, _Float16* y, long long split_stride, int N,
+                                                                                int splits, int threads, float eps, _Float16* __restrict__ norm_out) {
   __shared__ float s_part[kNormThreads / 64];
-  const int tid = threadIdx.x, threads = blockDim.x, chunks = N >> 3;
+  const int tid = threadIdx.x, chunks = N >> 3;
   const size_t row = (size_t)blockIdx.x * N;
-  h8 v[kNormTurns];
+  // the norm's weights and the residual are asked for with the sums, not behind them (every lane asks: no branch around a load)
+  h8 v[kNormTurns], w[kNormTurns], res[kNormTurns];
+  f32x4 lo[kNormTurns], hi[kNormTurns];
+  const bool second = chunks > threads;             // the same for the whole launch
+#pragma unroll
+  for (int i = 0; i < kNormTurns; ++i) {
+    if (i > 0 && !second) break;
+    const int c = tid + i * threads, at = 8 * (c < chunks ? c : chunks - 1);
+    w[i] = *reinterpret_cast<const h8*>(weight + at);
+    if (residual) res[i] = *reinterpret_cast<const h8*>(residual + row + at);
+    lo[i] = sum_splits<SPLITS>(partial + row + at, split_stride, splits);
+    hi[i] = sum_splits<SPLITS>(partial + row + at + 4, split_stride, splits);
+  }
   float a = 0.f;
 #pragma unroll
   for (int i = 0; i < kNormTurns; ++i) {
     const int c = tid + i * threads;
     if (c >= chunks) break;
-    const size_t at = row + 8 * (size_t)c;
-    const f32x4 lo = sum_splits<SPLITS>(partial + at, split_stride, splits), hi = sum_splits<SPLITS>(partial + at + 4, split_stride, splits);
 #pragma unroll
-    for (int k = 0; k < 8; ++k) v[i][k] = (_Float16)(k < 4 ? lo[k] : hi[k - 4]);
+    for (int k = 0; k < 8; ++k) v[i][k] = (_Float16)(k < 4 ? lo[i][k] : hi[i][k - 4]);
     if (residual) {
-      const h8 res = *reinterpret_cast<const h8*>(residual + at);
 #pragma unroll
-      for (int k = 0; k < 8; ++k) v[i][k] = (_Float16)((float)v[i][k] + (float)res[k]);
+      for (int k = 0; k < 8; ++k) v[i][k] = (_Float16)((float)v[i][k] + (float)res[i][k]);
     }
-    *reinterpret_cast<h8*>(y + at) = v[i];
+    *reinterpret_cast<h8*>(y + row + 8 * (size_t)c) = v[i];
 #pragma unroll
     for (int k = 0; k < 8; ++k) a = fmaf((float)v[i][k], (float)v[i][k], a);
   }
-#pragma unroll
-  for (int m = 1; m < 64; m <<= 1) a += __shfl_xor(a, m, 64);
+  a = wave_sum(a);
   if ((tid & 63) == 0) s_part[tid >> 6] = a;
-  __syncthreads();
-  float ss = 0.f;
-  for (int k = 0; k < threads >> 6; ++k) ss += s_part[k];
+  art_lds_barrier();                                // LDS only: y need not have landed
+  const int waves = threads >> 6;
+  float ss = 0.f;                                   // fixed length: one trip to LDS, not one for each wavefront
+#pragma unroll
+  for (int k = 0; k < kNormThreads / 64; ++k) {
+    const float part = s_part[k];
+    ss += k < waves ? part : 0.f;
+  }
   const float r = 1.0f / sqrtf(ss * (1.0f / (float)N) + eps);
 #pragma unroll
   for (int i = 0; i < kNormTurns; ++i) {
     const int c = tid + i * threads;
     if (c >= chunks) break;
-    const h8 w = *reinterpret_cast<const h8*>(weight + 8 * (size_t)c);
     h8 o;
 #pragma unroll
-    for (int k = 0; k < 8; ++k) o[k] = (_Float16)((float)v[i][k] * r * (float)w[k]);
+    for (int k = 0; k < 8; ++k) o[k] = (_Float16)((float)v[i][k] * r * (float)w[i][k]);
     *reinterpret_cast<h8*>(norm_out + row + 8 * (size_t)c) = o;
   }
 }
@@ -529,8 +554,8 @@ void launch_combine(const float* partial, _Float16* y, int rows, int N, int spli
   const dim3 by_eight((unsigned)(((long long)rows * (N / 8) + 255) / 256));
   if (norm) {
     const int threads = N < 8 * kNormThreads ? (N / 8 + 63) / 64 * 64 : kNormThreads;
-    gemm_w4a16_combine_norm_kernel<SPLITS><<<dim3(rows), threads, 0, stream>>>(partial, y, N, (long long)rows * N, splits, residual, (const _Float16*)norm->weight,
-                                                                                  (_Float16*)norm->out, norm->eps);
+    gemm_w4a16_combine_norm_kernel<SPLITS><<<dim3(rows), threads, 0, stream>>>(partial, residual, (const _Float16*)norm->weight, y, (long long)rows * N, N, splits,
+                                                                               threads, norm->eps, (_Float16*)norm->out);
   } else if (tail == kRope) {
     gemm_w4a16_combine_rope_kernel<SPLITS><<<by_eight, 256, 0, stream>>>(partial, rows, splits, rope, make_div(N / 8));
   } else if (tail == kSwiglu) {
