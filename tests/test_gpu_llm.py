@@ -606,3 +606,37 @@ def test_int4_products_of_more_than_4_gib_of_packed_weights(autort, M, code):
     want, got = (x.double() @ w.double()), y[:, cols].double()
     assert ((got - want).abs() <= want.abs() * 2.0 ** -10 + 2e-3).all(), (got - want).abs().max()
     assert not torch.isnan(y).any()
+
+
+@pytest.mark.parametrize('M', [4, 16, 17, 32, 33, 64])
+@pytest.mark.parametrize('K,N', [(128, 16), (1152, 48), (640, 208), (4224, 96), (1024, 1056), (2176, 9008)])
+def test_int4_products_of_a_few_rows_over_blocks_of_32_and_64_columns(autort, M, K, N):
+    """Up to 64 rows over narrow or shallow matrices are taken by blocks of 32 or 64 columns whose wavefronts divide K among them:
+    fewer groups than wavefronts, a last block half or a quarter inside the matrix, both rows-of-x forms' edges.  Against float64
+    sums of the same float16 weights: the result's rounding (2^-11) and float32 sums of K terms (K 2^-24 of the sum of absolute values)."""
+    note(f'few rows M={M} K={K} N={N}')
+    dev = autort.device()
+    g = torch.Generator(device=dev).manual_seed(M * 7 + K + N)
+    q = torch.randint(0, 256, (K // 2, N), generator=g, device=dev, dtype=torch.uint8)
+    z = torch.randint(0, 256, (K // 128, N // 2), generator=g, device=dev, dtype=torch.uint8)
+    s = (torch.rand(K // 128, N, generator=g, device=dev) * 0.019 + 0.001).half()
+    x, res = torch.randn(M, K, generator=g, device=dev).half(), torch.randn(M, N, generator=g, device=dev).half()
+    zero = torch.stack([z & 15, z >> 4], 2).reshape(K // 128, N).half().repeat_interleave(128, 0)
+    w = ((torch.stack([q & 15, q >> 4], 1).reshape(K, N).half() - zero) * s.repeat_interleave(128, 0)).double()
+    want, room = x.double() @ w, (x.double().abs() @ w.abs()) * K * 2.0 ** -24
+
+    def near(got, want, room):
+        assert ((got.double() - want).abs() <= want.abs() * 2.0 ** -11 + room + 2.0 ** -25).all(), ((got.double() - want).abs() - room).max()
+    out = torch.full((M, N), float('nan'), dtype=torch.float16, device=dev)
+    autort.ops.gemm_w4a16_residual(x, q, s, z, out)
+    near(out, want, room)
+    y = res.clone()                                 # the result over the residual: fp16(fp16(product) + residual)
+    autort.ops.gemm_w4a16_residual(x, q, s, z, y, residual=y)
+    near(y, want + res.double(), room + want.abs() * 2.0 ** -11)
+    if N % 32 == 0:                                 # gate | up; silu's slope is at most 1.1, its rounding that of the gate
+        hid = torch.full((M, N // 2), float('nan'), dtype=torch.float16, device=dev)
+        autort.ops.gemm_w4a16_swiglu(x, q, s, z, hid)
+        gate, up = want[:, :N // 2], want[:, N // 2:]
+        rg, ru = room[:, :N // 2] + gate.abs() * 2.0 ** -11, room[:, N // 2:] + up.abs() * 2.0 ** -11
+        silu = torch.nn.functional.silu(gate)
+        near(hid, silu * up, 1.1 * rg * up.abs() + silu.abs() * ru + 1.1 * rg * ru + (silu * up).abs() * 2.0 ** -20)
