@@ -3,7 +3,7 @@
 // on the matrix cores with fp32 accumulation; w is rounded exactly as the reference's dequant + matmul program
 // does (samples/05_llama2_7b_int4.py:135-144 exported with a batch axis).  This file holds the entry points, the kernel
 // for batches that do not fill blocks of 256 columns x 128 or 256 rows (art_gemm_w4_wide.hip takes those), the pass that
-// adds K-splits, and the rule that chooses among it, art_gemm_w4_wide.hip and, for up to 64 rows, art_gemm_w4_deep.hip.
+// adds K-splits, and the rule that chooses among it, art_gemm_w4_wide.hip and art_gemm_w4_deep.hip.
 //
 // Design for MI355X:
 //   * a block of eight wavefronts owns 128 columns, 32 MT rows (MT = 1, 2, 4) and a contiguous range of quantisation
@@ -495,36 +495,43 @@ struct Plan {
 };
 // What a launch takes, in microseconds.  K-splits: the second launch and the fp32 tiles on top.
 double splits_estimate(int M, int N, int splits) { return splits > 1 ? 1.8 + (8.0 * splits + 2.0) * M * N / 4.2e6 : 0.0; }
-// A fixed part, one or two co-resident blocks' time per group and round, the ramp and
-// the meeting of the k halves again for every further round of blocks of 128 columns (4 rows over 4096 x 12288: 13.3 us with
-// 480 blocks, i.e. 5 K-splits in one round, 14.6 with 768).  Constants from 31000 launches of
-// 4 to 1003 rows over matrices of 512 x 512 to 11008 x 14700 on MI355X: the estimate is 4 to 6 % off in the mean, the form it picks 0.3 to 0.9 %
-// slower than the fastest one (the constants before it, of the kernels before these: 0.9 to 1.7 %).
+// Where K-splits meet in a pass of their own, a norm is part of that pass, up to 256 rows: beyond them nothing is
+// gained (8 layers of the same pass: 1384 -> 1368 us at 256 tokens, 1861 and 1854 at 300, 2178 and 2183 at 500).
+bool norm_fits(int M, int N) { return M <= 256 && N % 8 == 0 && N <= 8 * kNormThreads * kNormTurns; }
+// Else it is a launch of its own.
+double norm_estimate(int M, int N, int splits) { return splits == 1 ? 2.4 + 2.0e-6 * M * N : 0.0; }
+// A fixed part, one or two co-resident blocks' time per group and round (one's: more with more of the compute units at work), the
+// ramp and the meeting of the k halves again for every further round of blocks of 128 columns (4 rows over 4096 x 12288: 13.3 us with
+// 480 blocks, i.e. 5 K-splits in one round, 14.6 with 768).  Constants of both estimates from all
+// forms over 6200 sizes of 4 to 1003 rows, 512 x 512 to 11008 x 14700, on MI355X, a quarter with weights that stay in the last-level cache, the
+// others with weights from HBM, as a model's are (up to 1.4 times the time): the pick is 1 to 2 % slower than the fastest form in both.  From
+// the former alone prompts lost: a layer of 32 heads at 8 and 64 tokens 71 and 82 us, now 62 and 78; of 8 heads 27 and 32, now 23 and 28.
 double estimate(int M, int K, int N, const Plan& p, int compute_units) {
-  struct Cost { double fixed, one, two; int per_cu; };
-  const Cost c = p.wide ? (p.row_tiles == 8 ? Cost{8.5, 2.16, 1.94, 1} : Cost{5.2, 1.2, 2.3, 2})
-                        : p.row_tiles == 4 ? Cost{4.8, 0.52, 0.82, 1} : p.row_tiles == 2 ? Cost{4.7, 0.44, 0.82, 2} : Cost{4.4, 0.39, 0.88, 2};
+  struct Cost { double fixed, one, two; int per_cu; double busy; };
+  const Cost c = p.wide ? (p.row_tiles == 8 ? Cost{8.5, 2.16, 1.94, 1, 0} : Cost{5.2, 1.2, 2.3, 2, 0})
+                        : p.row_tiles == 4 ? Cost{4.8, 0.52, 0.82, 1, 0} : p.row_tiles == 2 ? Cost{4.75, 0.410, 0.985, 2, 0.12} : Cost{3.75, 0.348, 0.848, 2, 0};
   const int groups = (K / GK + p.splits - 1) / p.splits, m_blocks = (M + 32 * p.row_tiles - 1) / (32 * p.row_tiles);
   const int blocks = tile_count(N, false, p.wide ? 256 : BN) * m_blocks * p.splits, round = c.per_cu * compute_units;
   const int rest = blocks % round;
+  const double one = c.one * (1 + c.busy * (blocks < compute_units ? (double)blocks / compute_units : 1.0));
   double per_group = blocks / round * c.two;
   if (rest > compute_units) per_group += c.two;
-  else if (rest > 0) per_group += c.per_cu == 2 || blocks > round ? c.one : c.one + (c.two - c.one) * rest / compute_units;
+  else if (rest > 0) per_group += c.per_cu == 2 || blocks > round ? one : one + (c.two - one) * rest / compute_units;
   const double again = p.wide ? 0.0 : 0.73 * ((blocks - 1) / round);
   return c.fixed + again + groups * per_group + splits_estimate(M, N, p.splits);
 }
-// The deep kernel: a fixed part and, for each group, what the load path of a compute unit needs for it (all eight wavefronts share it,
-// so groups count, not rounds of them), more with more of the compute units at work and with each further block on one.  17000 launches
-// of 4 to 64 rows: 3 to 4 % off in the mean; with these forms the pick is 0.6 to 1.0 % slower than the fastest one.
+// art_gemm_w4_deep.hip: a fixed part and, for each group, what the load path of a compute unit needs for it (all eight wavefronts share it,
+// so groups count, not rounds of them), more with more of the compute units at work and with each further block on one.
 double deep_estimate(int M, int K, int N, const Plan& p, Tail tail, int compute_units) {
   struct Cost { double fixed, group, busy, further, again; };
-  const Cost c = p.deep == 2 ? (M <= 16 ? Cost{3.52, 0.160, 0.46, 0.92, 0.93} : Cost{3.26, 0.200, 0.54, 1.14, 1.54})
-                             : M <= 16 ? Cost{3.02, 0.096, 0.51, 1.10, 0.62} : M <= 32 ? Cost{2.95, 0.142, 0.47, 1.17, 1.40} : Cost{3.33, 0.204, 0.41, 1.11, 1.38};
-  const int groups = (K / GK + p.splits - 1) / p.splits, blocks = deep_tiles(N, tail, p.deep) * p.splits, more = (blocks - 1) / compute_units;
+  const Cost c = p.deep == 2 ? (M <= 16 ? Cost{3.26, 0.155, 0.418, 2.13, 0.44} : Cost{3.50, 0.178, 0.263, 1.63, 1.20})
+                 : p.row_tiles == 2 ? Cost{3.18, 0.201, 0.391, 1.34, 1.23} : M <= 16 ? Cost{3.04, 0.103, 0.332, 2.10, 0.36} : Cost{3.22, 0.151, 0.066, 1.38, 1.11};
+  const int groups = (K / GK + p.splits - 1) / p.splits, m_blocks = (M + 32 * p.row_tiles - 1) / (32 * p.row_tiles);
+  const int blocks = deep_tiles(N, tail, p.deep) * m_blocks * p.splits, more = (blocks - 1) / compute_units;
   const double busy = blocks < compute_units ? (double)blocks / compute_units : 1.0;
   return c.fixed + c.group * groups * (1 + c.busy * busy + c.further * more) + c.again * more + splits_estimate(M, N, p.splits);
 }
-constexpr int kDeepRows = 64;
+constexpr int kDeepBlocks = 8;                      // of rows
 // What a form's 32-bit offsets (a block's rows of x and of the packed weights), its division by the number of column
 // tiles and its grid hold.  Where the packed weights of a split do not fit 32 bits, two of the forms are left.
 bool far(const Plan& p, int K, int N) { return 64LL * N * ((K / GK + p.splits - 1) / p.splits) > 1LL << 32; }
@@ -535,14 +542,16 @@ bool holds(const Plan& p, int K, int N, Tail tail) {
   return offsets && units < (p.wide ? 1 << 19 : 1 << 16) && (!far(p, K, N) || p.row_tiles == (p.wide ? 4 : 1));
 }
 // False: no form takes these sizes.  `code` and `splits` are the caller's wishes (0: none; the deep kernel comes with none); a form that
-// does not hold the sizes is replaced by one that does.  What becomes of the product has
-// no part in it: its bits are the same with a residual, a norm or neither behind it.
-bool choose(Plan& best, int M, int K, int N, Tail tail, size_t scratch_bytes, int compute_units, int code, int splits) {
+// does not hold the sizes is replaced by one that does.  A product with a
+// residual counts as one with a norm behind it, in its own call or the next: the bits of y are the same in both.
+bool choose(Plan& best, int M, int K, int N, Tail tail, bool residual, size_t scratch_bytes, int compute_units, int code, int splits) {
   const int G = K / GK;
   const size_t per_split = (size_t)M * N * sizeof(float);
   const int cap = (int)(scratch_bytes / per_split), most = G < cap ? G : (cap < 1 ? 1 : cap);
   double t_best = 1e30;
+  const bool norm_in_pass = residual && norm_fits(M, N);
   auto consider = [&](const Plan& p, double t) {
+    if (norm_in_pass) t += norm_estimate(M, N, p.splits);
     if (t < t_best) { t_best = t; best = p; }
   };
   for (int pass = 0; pass < 2 && t_best == 1e30; ++pass) {
@@ -558,12 +567,14 @@ bool choose(Plan& best, int M, int K, int N, Tail tail, size_t scratch_bytes, in
     }
     if (t_best == 1e30) splits = 1;
   }
-  if (code == 0 && splits == 0 && M <= kDeepRows)
-    for (int deep = 1; deep <= (M <= 32 ? 2 : 1); ++deep)
+  if (code == 0 && splits == 0)
+    for (const Plan form : {Plan{false, 1, 1, 1}, Plan{false, 1, 1, 2}, Plan{false, 2, 1, 1}}) {
+      if (M > 32 * form.row_tiles * kDeepBlocks || 16 * form.row_tiles >= M && form.row_tiles > 1) continue;
       for (int s = 1; s <= 16 && (s == 1 || (s <= most && 2 * s <= G + 1)); ++s) {
-        const Plan p{false, 2, s, deep};
+        const Plan p{false, form.row_tiles, s, form.deep};
         if (holds(p, K, N, tail)) consider(p, deep_estimate(M, K, N, p, tail, compute_units));
       }
+    }
   return t_best < 1e30;
 }
 // An RMSNorm of the result: out = fp16(y / rms(y) * weight).
@@ -605,13 +616,11 @@ int run_rows(const _Float16* xs, const unsigned char* qweight, const _Float16* s
              int M, int K, int N, int code, int splits, Tail tail, const Norm* norm, const Rope& rope, float* scratch, size_t scratch_bytes, hipStream_t st) {
   const bool swiglu = tail == kSwiglu;
   Plan p;
-  ART_REQUIRE(choose(p, M, K, N, tail, scratch_bytes, art::compute_units(), code, splits), "art_gemm_w4a16: K=%d N=%d are too large", K, N);
-  // Where K-splits meet in a pass of their own, the norm is part of that pass, up to 256 rows: beyond them
-  // nothing is gained (8 layers of the same pass: 1384 -> 1368 us at 256 tokens, 1861 and 1854 at 300, 2178 and 2183 at 500).
-  const bool norm_there = norm && p.splits > 1 && M <= 256 && N % 8 == 0 && N <= 8 * kNormThreads * kNormTurns &&
+  ART_REQUIRE(choose(p, M, K, N, tail, res != nullptr, scratch_bytes, art::compute_units(), code, splits), "art_gemm_w4a16: K=%d N=%d are too large", K, N);
+  const bool norm_there = norm && p.splits > 1 && norm_fits(M, N) &&
                           (((uintptr_t)ys | (uintptr_t)res | (uintptr_t)norm->weight | (uintptr_t)norm->out) % 16) == 0;
   if (p.deep) {
-    if (art::w4::gemm_deep(xs, qweight, scales, qzeros, ys, scratch, M, K, N, p.splits, p.deep, res, tail, rope, st)) return 1;
+    if (art::w4::gemm_deep(xs, qweight, scales, qzeros, ys, scratch, M, K, N, p.splits, p.row_tiles, p.deep, res, tail, rope, st)) return 1;
   } else if (p.wide) {
     if (art::w4::gemm_wide(xs, qweight, scales, qzeros, ys, scratch, M, K, N, p.splits, p.row_tiles, far(p, K, N), res, tail, rope, st)) return 1;
   } else {

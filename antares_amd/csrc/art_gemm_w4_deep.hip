@@ -1,23 +1,26 @@
-// Weight-only int4 GEMM for a few rows (4 to 64): the arithmetic of art_gemm_w4.hip,
+// Weight-only int4 GEMM for small products (4 to 512 rows): the arithmetic of art_gemm_w4.hip,
 //     y[m,n] = sum_k x[m,k] * w[k,n],   w[k,n] = fp16(s[g,n] * fp16(q[k,n] - z[g,n])),   group g = k / 128,
 // on the matrix cores with fp32 accumulation, for sizes where that kernel's blocks of 128 columns either leave most of the chip
 // without work or need K-splits, whose sums a second launch adds: a chain of groups one after another, or two launches.
 //
-//   * a block owns 32 columns (or 64, with up to 32 rows) and all of K (or of a K split); its eight wavefronts take the quantisation groups in
+//   * a block owns 16, 32 or 64 rows, 32 columns (or 64, with up to 32 rows) and all of K (or of a K split); its eight wavefronts
+//     take the quantisation groups in
 //     turn, so that K is worked on eight-fold in parallel without a second launch, and meet once, at the end, in LDS;
 //   * a wavefront works by itself: what its next group needs - 2 or 4 KiB of packed weights, their scales and zero points, 4 to 16 KiB of x -
 //     goes from global memory into LDS of its own (no barrier in the loop), into the place that the group before has just been read
 //     from.  Fetching weights two or three groups ahead was slower (16 rows over 4096 x 4096 7.5 -> 8.4 and 9.0 us): the loads that are
 //     needed first queue behind them;
-//   * neighbouring blocks share the lines of the packed weights (32 or 64 of 128 bytes a row) and run on one XCD, at the same time.
+//   * the blocks of a tile's rows share its weights, neighbouring tiles the lines of the packed weights (32 or 64 of 128 bytes a row): they run
+//     on one XCD, at the same time.
 //
 // What bounds it: the launch and one trip to memory (3.0 us) at the smallest sizes; beyond them the load path of a compute unit, 0.1 to 0.2 us a
 // group for all eight wavefronts - every block takes in all of x, and a row's 32 bytes of weights cost it as much as 64.  64 columns halve both,
-// with half as many blocks: better from some 150 of them on.  More than 64 rows of x do not fit LDS.
+// with half as many blocks: better from some 150 of them on.  64 rows of x and 64 columns do not fit LDS.
 // Measured (MI355X, weights from memory; the best form of the kernels before -> this one): 16 rows over 1024 x 1024 6.0 -> 3.7 us, 1024 x 5376
 // 6.9 -> 4.5, 2048 x 6144 8.4 -> 6.0, 4096 x 4096 8.6 -> 7.5, 4096 x 12288 13.1 -> 10.9; 32 rows over 2048 x 2048 7.2 -> 5.2, 2048 x 10752
-// 10.2 -> 7.6; 64 rows over 1024 x 5376 7.1 -> 5.9, 2048 x 6144 10.5 -> 8.1, and not better over 4096 x 12288 (16.2 and 21.8).  1020 sizes of 4 to 64
-// rows, 512 to 11008 x 512 to 14700, geometric mean: 1.31 times up to 16 rows, 1.27 up to 32, 1.12 up to 64 (art_gemm_w4.hip chooses).
+// 10.2 -> 7.6; 64 rows over 1024 x 5376 7.1 -> 5.9, 2048 x 6144 10.5 -> 8.1, and not better over 4096 x 12288 (16.2 and 21.8).  Sizes of 512 to
+// 11008 x 512 to 14700, geometric mean where the better of both is taken (art_gemm_w4.hip chooses): 1.31 times up to 16 rows, 1.25 up to 32, 1.16 up to
+// 128, 1.08 up to 256, 1.05 up to 512.
 #include "art_w4_mfma.h"
 
 #include <type_traits>
@@ -39,14 +42,20 @@ constexpr size_t lds_bytes(int XR, int CT) { return (size_t)kWaves * wave_bytes(
 template <int XR, int CT, Tail TAIL>
 __global__ __launch_bounds__(kThreads, XR == 16 ? 4 : 2) void gemm_w4a16_deep_kernel(
     const _Float16* __restrict__ x, const unsigned char* __restrict__ qweight, const _Float16* __restrict__ scales,
-    const unsigned char* __restrict__ qzeros, int K, int N, int M, int tiles, unsigned int inv_tiles, int each, _Float16* y, float* __restrict__ partial,
+    const unsigned char* __restrict__ qzeros, int K, int N, int M, int tiles, unsigned int inv_tiles, int each, int m_blocks, unsigned int inv_blocks, _Float16* y, float* __restrict__ partial,
     int splits, int groups_of_split, int longer, Magic mg, const _Float16* residual, Rope rope) {
   constexpr int MT = XR == 64 ? 2 : 1, BN = 32 * CT, W_BYTES = w_bytes(CT);
   constexpr int XL = XR / 4, WL = W_BYTES / 1024;   // loads of x and of the packed weights per group
   extern __shared__ __align__(1024) unsigned char smem[];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int unit = (blockIdx.x & 7) * each + (blockIdx.x >> 3);      // (tile, K split); neighbours on one XCD
-  if (unit >= tiles * splits) return;
+  int unit = (blockIdx.x & 7) * each + (blockIdx.x >> 3);            // (tile, K split, block of rows); neighbours on one XCD
+  if (unit >= tiles * splits * m_blocks) return;
+  int m0 = 0;
+  if (m_blocks > 1) {
+    const int block = unit;
+    unit = (int)__umulhi(block, inv_blocks);        // block / m_blocks
+    m0 = (block - unit * m_blocks) * XR;
+  }
   const int split = inv_tiles ? (int)__umulhi(unit, inv_tiles) : unit, tile = unit - split * tiles;
   const int g_begin = split * groups_of_split + (split < longer ? split : longer), g_count = groups_of_split + (split < longer ? 1 : 0);
   const int mine = (g_count - wave + kWaves - 1) / kWaves;           // groups wave, wave + 8, ... of the split
@@ -78,7 +87,7 @@ __global__ __launch_bounds__(kThreads, XR == 16 ? 4 : 2) void gemm_w4a16_deep_ke
 
   if (mine > 0) {
     const int g0 = g_begin + wave;
-    Rows<false> w_rows(qweight + (size_t)g0 * (GK / 2) * N, kWaves * (GK / 2) * N, mine), x_rows(x + (size_t)g0 * GK, kWaves * GK * 2, mine),
+    Rows<false> w_rows(qweight + (size_t)g0 * (GK / 2) * N, kWaves * (GK / 2) * N, mine), x_rows(x + (size_t)m0 * K + (size_t)g0 * GK, kWaves * GK * 2, mine),
         s_rows(scales + (size_t)g0 * N, kWaves * 2 * N, mine), z_rows(qzeros + (size_t)g0 * (N / 2), kWaves * (N / 2), mine);
     // Position (row, piece p) of the packed weights holds piece p, with two tiles p ^ (2 in every other four rows): the 32 lanes of a
     // transposing read, 8 rows of two pieces, touch every bank once.
@@ -94,7 +103,7 @@ __global__ __launch_bounds__(kThreads, XR == 16 ? 4 : 2) void gemm_w4a16_deep_ke
 #pragma unroll
     for (int u = 0; u < XL; ++u) {
       const int r = 4 * u + (lane >> 4);
-      xoff[u] = (unsigned int)(r < M ? r : M - 1) * (2 * K) + (((lane & 15) ^ (r & 15)) * 16);
+      xoff[u] = (unsigned int)(m0 + r < M ? r : M - 1 - m0) * (2 * K) + (((lane & 15) ^ (r & 15)) * 16);
     }
     auto fetch_x4 = [&](auto u_tag) {
       constexpr int U = decltype(u_tag)::value;
@@ -194,7 +203,7 @@ __global__ __launch_bounds__(kThreads, XR == 16 ? 4 : 2) void gemm_w4a16_deep_ke
 #pragma unroll
     for (int w = 1; w < kWaves; ++w) sum += of[w];
   }
-  const int t = (quad >> 2) % MT, ct = (quad >> 2) / MT, piece = 2 * ct + hi16, row0 = t * 32 + (quad & 3) * 8 + h * 4 + part;
+  const int t = (quad >> 2) % MT, ct = (quad >> 2) / MT, piece = 2 * ct + hi16, row0 = m0 + t * 32 + (quad & 3) * 8 + h * 4 + part;
   if (!inside(piece)) return;                       // both of a pair or neither, but for kPlain
   const int col = piece_at(piece) + s16;
   if (splits > 1) {
@@ -243,7 +252,7 @@ __global__ __launch_bounds__(kThreads, XR == 16 ? 4 : 2) void gemm_w4a16_deep_ke
 }  // namespace
 
 int art::w4::gemm_deep(const _Float16* x, const unsigned char* qweight, const _Float16* scales, const unsigned char* qzeros, _Float16* y,
-                       float* partial, int M, int K, int N, int splits, int col_tiles, const _Float16* residual, Tail tail, const Rope& rope, hipStream_t stream) {
+                       float* partial, int M, int K, int N, int splits, int row_tiles, int col_tiles, const _Float16* residual, Tail tail, const Rope& rope, hipStream_t stream) {
 #define ART_DEEP(XR, CT) {gemm_w4a16_deep_kernel<XR, CT, kPlain>, gemm_w4a16_deep_kernel<XR, CT, kSwiglu>, gemm_w4a16_deep_kernel<XR, CT, kRope>}
   static const decltype(&gemm_w4a16_deep_kernel<16, 1, kPlain>) kernels[5][3] = {ART_DEEP(16, 1), ART_DEEP(32, 1), ART_DEEP(64, 1), ART_DEEP(16, 2), ART_DEEP(32, 2)};
 #undef ART_DEEP
@@ -255,12 +264,12 @@ int art::w4::gemm_deep(const _Float16* x, const unsigned char* qweight, const _F
         ART_HIP(hipFuncSetAttribute((const void*)kernels[i][j], hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds[i]));
     configured = true;
   }
-  const bool two = col_tiles == 2;
-  const int form = M <= 16 ? (two ? 3 : 0) : M <= 32 ? (two ? 4 : 1) : 2;
-  const int tiles = deep_tiles(N, tail, two ? 2 : 1), units = tiles * splits, each = (units + 7) / 8, G = K / GK;
+  const int rows = M <= 16 ? 16 : 32 * row_tiles, m_blocks = (M + rows - 1) / rows, form = (rows == 16 ? 0 : rows == 32 ? 1 : 2) + (col_tiles == 2 ? 3 : 0);
+  const int tiles = deep_tiles(N, tail, col_tiles), units = tiles * splits * m_blocks, each = (units + 7) / 8, G = K / GK;
   kernels[form][tail]<<<dim3(8 * each), kThreads, lds[form], stream>>>(
-      x, qweight, scales, qzeros, K, N, M, tiles, (unsigned int)((0x100000000ull + tiles - 1) / tiles), each, y, partial, splits, G / splits, G % splits,
-      kMagic, residual, rope);
+      x, qweight, scales, qzeros, K, N, M, tiles, (unsigned int)((0x100000000ull + tiles - 1) / tiles), each, m_blocks,
+      (unsigned int)((0x100000000ull + m_blocks - 1) / m_blocks), y, partial, splits, G / splits,
+      G % splits, kMagic, residual, rope);
   ART_LAUNCH_CHECK();
   return 0;
 }

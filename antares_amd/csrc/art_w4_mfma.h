@@ -177,11 +177,12 @@ __device__ __forceinline__ h4 swiglu4(h4 g, h4 u) {
 int gemm_wide(const _Float16* x, const unsigned char* qweight, const _Float16* scales, const unsigned char* qzeros, _Float16* y,
               float* partial, int M, int K, int N, int splits, int row_tiles, bool far, const _Float16* residual, Tail tail, const Rope& rope, hipStream_t stream);
 
-// A few rows (art_gemm_w4_deep.hip): one launch over blocks of 32 columns and up to 64 rows, or 64 columns and up to 32 rows (col_tiles 1, 2).
+// Small products (art_gemm_w4_deep.hip): one launch over blocks of 32 row_tiles rows (1 or 2; 16 where there are no more) and 32 col_tiles columns (1, or
+// 2 with one row tile).
 // Partial sums as above; tiles x splits below 2^16, the packed weights of a split below 4 GiB.
 inline int deep_tiles(int N, Tail tail, int col_tiles) { return tail == kPlain ? (N + 32 * col_tiles - 1) / (32 * col_tiles) : (N / 2 + 16 * col_tiles - 1) / (16 * col_tiles); }
 int gemm_deep(const _Float16* x, const unsigned char* qweight, const _Float16* scales, const unsigned char* qzeros, _Float16* y,
-              float* partial, int M, int K, int N, int splits, int col_tiles, const _Float16* residual, Tail tail, const Rope& rope, hipStream_t stream);
+              float* partial, int M, int K, int N, int splits, int row_tiles, int col_tiles, const _Float16* residual, Tail tail, const Rope& rope, hipStream_t stream);
 
 }  // namespace w4
 }  // namespace art
