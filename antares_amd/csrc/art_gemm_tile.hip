@@ -22,6 +22,7 @@
 //     sum on the vector units in short slices (FINE, see `fine`), four values of k by themselves, these sums in pairs, and
 //     the chunks and slices in float64.  One chain over k has 1.4e-7 (64 terms) to 1.1e-6 (4090) against 64 bits, the
 //     generic kernels 1.4e-7 to 1e-6 and, in short slices, 0.7e-7 to 1.6e-7; this 1.1e-7 to 2.3e-7 and, FINE, 0.64e-7 to 0.73e-7;
+//   * a chunk goes to LDS behind the products of the one before, float16 with a block per compute unit in front of them (see the loop);
 //   * blocks on one XCD are a contiguous run of (slice, tile), its L2 holds what they share.
 // Bound by latency below some 10 us - a launch, a chain of chunks whose loads L2 answers after several hundred
 // nanoseconds, a second launch for slices -, then by the matrix instructions (float32) or the loads (64 x 64 blocks of float16
@@ -48,6 +49,7 @@ typedef unsigned int u32x4_any __attribute__((ext_vector_type(4), aligned(1))); 
 typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
 
 constexpr int kThreads = 256;
+constexpr int kUnits = 256;                  // compute units of an MI355X
 constexpr int kChunk = 128;                  // bytes of k of a row that are staged at a time
 constexpr int kRow = kChunk + 16;            // bytes from row to row in LDS where k is contiguous
 
@@ -283,17 +285,48 @@ __global__ __launch_bounds__(kThreads, TM * TN == 4 || (sizeof(T) == 4 && (TN ==
   fetch(S0{});
   art_lds_barrier();
   // Chunk t is in LDS buffer t % 2, chunk t + 1 in the other register stage, chunk t + 2 on its way.
-  for (int t = 0; t < count; t += 2) {
+  if constexpr (FINE) {                               // (its registers do not hold a loop with code behind it)
+    for (int t = 0; t < count; t += 2) {
+      multiply_chunk(t);
+      if (t + 1 == count) break;
+      put(first + t + 1, S1{});
+      fetch(S1{});
+      art_lds_barrier();
+      multiply_chunk(t + 1);
+      if (t + 2 == count) break;
+      put(first + t + 2, S0{});
+      fetch(S0{});
+      art_lds_barrier();
+    }
+  } else {
+    // No exit in the middle of the loop: one that leaves behind an odd chunk makes the compiler wait for chunk t + 2's loads where
+    // chunk t + 1 goes to LDS (2 to 4 % over 300 sizes).  EARLY: the next chunk goes to LDS in front of the products, not behind
+    // them; with a block of its own on each compute unit nothing else hides that (float16 192 x 3656 x 2944 19.9 -> 16.9 us, 968 x
+    // 1880 x 3928 40.5 -> 34.8), with two to three it is slower (1472 x 1920 x 3136 39.8 -> 44.1); float32 and int8 gain nothing.
+    auto loop = [&](auto early) {
+      constexpr bool EARLY = decltype(early)::value;
+      auto step = [&](int chunk, auto buffer, auto stage) {
+        using Four = std::integral_constant<int, 4>;
+        if constexpr (!EARLY) multiply(decltype(buffer)::value, Four{});
+        put(chunk, stage);
+        fetch(stage);
+        if constexpr (EARLY) multiply(decltype(buffer)::value, Four{});
+        art_lds_barrier();
+      };
+      int t = 0;
+      for (; t + 2 < count; t += 2) {
+        step(first + t + 1, S0{}, S1{});
+        step(first + t + 2, S1{}, S0{});
+      }
+      return t;
+    };
+    const int t = S == 2 && z.blocks <= kUnits ? loop(std::true_type{}) : loop(std::false_type{});
     multiply_chunk(t);
-    if (t + 1 == count) break;
-    put(first + t + 1, S1{});
-    fetch(S1{});
-    art_lds_barrier();
-    multiply_chunk(t + 1);
-    if (t + 2 == count) break;
-    put(first + t + 2, S0{});
-    fetch(S0{});
-    art_lds_barrier();
+    if (t + 1 < count) {
+      put(first + t + 1, S1{});
+      art_lds_barrier();
+      multiply_chunk(t + 1);
+    }
   }
 
   if constexpr (FINE)
@@ -375,7 +408,6 @@ constexpr Cost kCost[3][3] = {{{3.67, 0.321, 0.210, 0.195}, {4.81, 0.494, 0.361,
                               {{3.24, 0.816, 0.514, 0.574}, {4.22, 1.360, 1.031, 1.048}, {3.35, 1.114, 0.736, 0.628}},
                               {{3.55, 0.309, 0.217, 0.294}, {4.57, 0.452, 0.432, 0.370}, {5.83, 0.731, 0.502, 0.501}}};
 constexpr Rest kRest[3] = {{2.31, 0.408, 0.425}, {2.73, 0.388, 0.242}, {2.09, 0.403, 0.208}};       // per million floats, per million bytes
-constexpr int kUnits = 256;                  // compute units of an MI355X
 double launch_time(int type, int M, int N, int K, int form, int splits) {
   const Cost& c = kCost[type][form > 2 ? 2 : form - 1];
   const Rest& r = kRest[type];

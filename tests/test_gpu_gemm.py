@@ -181,6 +181,27 @@ def test_tile_products_of_every_form(dtype, M, N, chunks, rest):
                 assert bool(((got - want).abs() <= (K + slices) * 2.0 ** -24 * size + 2.0 ** -11 * want.abs() + 2.0 ** -24).all())
 
 
+@pytest.mark.parametrize('chunks,rest', [(1, 0), (2, 3), (3, 0), (4, -1), (7, 5)])
+def test_tile_products_of_more_blocks_than_compute_units(chunks, rest):
+    """float16 puts the next chunk into LDS in front of the products with up to 256 blocks, behind them with more: the same sums in
+    the same order, so the rows that 16 x 16 and 18 x 16 tiles share are the same bit for bit, and within the bound of the other forms
+    (every addition off by 2^-24 of the magnitudes, one rounding to float16)."""
+    from ctypes import c_void_p
+    from antares_amd.runtime import capi
+    capi.init(0)
+    dev, N, K = torch.device('cuda', 0), 1000, 64 * chunks + rest
+    a, b, want, size = _tile_operands('float16', 1100, N, K, dev, 1)
+    results = []
+    for M in (1000, 1100):
+        print(f'[case] art_gemm_tile float16 {M}x{N}x{K} form 1', flush=True)
+        c = torch.full((M, N), float('nan'), dtype=torch.float16, device=dev)
+        capi.check(capi.lib().art_gemm_tile(c_void_p(a.data_ptr()), c_void_p(b.data_ptr()), c_void_p(c.data_ptr()), None, 0, M, N, K, 1, 1,
+                                            c_void_p(torch.cuda.current_stream().cuda_stream)))
+        results.append(c.cpu())
+    assert torch.equal(results[0], results[1][:1000])
+    assert ((results[1].double() - want).abs() <= size * (K * 2.0 ** -24) + want.abs() * 2.0 ** -11 + 2.0 ** -24).all()
+
+
 @pytest.mark.parametrize('dtype,M,N,K', [('float16', 78, 207, 582), ('float16', 448, 704, 2368), ('float16', 144, 160, 104), ('float32', 248, 120, 1616),
                                          ('float32', 192, 576, 192), ('float32', 70, 420, 268), ('int8', 232, 120, 1448), ('int8', 112, 3568, 72),
                                          # thin or short: the generic kernels sum on the vector units however many tiles there are
