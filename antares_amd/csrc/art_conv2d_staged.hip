@@ -2,7 +2,7 @@
 // filter and copies the image with the channels of a point side by side, the second one multiplies.
 //
 // Why: the kernel that gathers the image as it lies in memory spends most of its time before its first product - its code is
-// 12 to 20 KiB (fetched cold, about 0.3 us per KiB), every staged point takes divisions, comparisons and 2- or 4-byte loads.
+// 12 to 20 KiB, run once, and every staged point takes divisions, comparisons and 2- or 4-byte loads.
 // With nothing but the products left in its loop it still took 16.2 of 21.8 us at float16 32 x 128 x 28 x 28 -> 128.  Here
 //   * the copy holds the image padded to HO + 2 rows of WO + 2 points, [64 bytes of channels][point][64 bytes], zeros where the
 //     image or its channels end.  It is made by the launch that packs the filter anyway;

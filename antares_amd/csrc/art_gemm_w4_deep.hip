@@ -4,8 +4,8 @@
 // without work or need K-splits, whose sums a second launch adds: a chain of groups one after another, or two launches.
 //
 //   * a block owns 16, 32 or 64 rows, 32 columns (or 64, with up to 32 rows) and all of K (or of a K split); its eight wavefronts
-//     take the quantisation groups in
-//     turn, so that K is worked on eight-fold in parallel without a second launch, and meet once, at the end, in LDS;
+//     take the quantisation groups in turn, so that K is worked on eight-fold in parallel without a second launch, and meet once, at the
+//     end, in LDS;
 //   * a wavefront works by itself: what its next group needs - 2 or 4 KiB of packed weights, their scales and zero points, 4 to 16 KiB of x -
 //     goes from global memory into LDS of its own (no barrier in the loop), into the place that the group before has just been read
 //     from.  Fetching weights two or three groups ahead was slower (16 rows over 4096 x 4096 7.5 -> 8.4 and 9.0 us): the loads that are
@@ -16,7 +16,7 @@
 // What bounds it: the launch and one trip to memory (3.0 us) at the smallest sizes; beyond them the load path of a compute unit, 0.1 to 0.2 us a
 // group for all eight wavefronts - every block takes in all of x, and a row's 32 bytes of weights cost it as much as 64.  64 columns halve both,
 // with half as many blocks: better from some 150 of them on.  64 rows of x and 64 columns do not fit LDS.
-// Measured (MI355X, weights from memory; the best form of the kernels before -> this one): 16 rows over 1024 x 1024 6.0 -> 3.7 us, 1024 x 5376
+// Measured (MI355X, weights from the last-level cache; the best form of the kernels before -> this one): 16 rows over 1024 x 1024 6.0 -> 3.7 us, 1024 x 5376
 // 6.9 -> 4.5, 2048 x 6144 8.4 -> 6.0, 4096 x 4096 8.6 -> 7.5, 4096 x 12288 13.1 -> 10.9; 32 rows over 2048 x 2048 7.2 -> 5.2, 2048 x 10752
 // 10.2 -> 7.6; 64 rows over 1024 x 5376 7.1 -> 5.9, 2048 x 6144 10.5 -> 8.1, and not better over 4096 x 12288 (16.2 and 21.8).  Sizes of 512 to
 // 11008 x 512 to 14700, geometric mean where the better of both is taken (art_gemm_w4.hip chooses): 1.31 times up to 16 rows, 1.25 up to 32, 1.16 up to
