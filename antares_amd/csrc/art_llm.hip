@@ -96,25 +96,28 @@ __device__ __forceinline__ void store8(float* p, const float (&v)[8]) {
 
 // Rows of up to 8192 elements, a multiple of 8, on 16-byte boundaries: the row is read once, 16 bytes per lane, and kept
 // in registers between the sum and the product (the element-wise form reads it twice, two bytes per lane: 1003 rows of
-// 4096 halves took 8.5 us, 16.4 MB at 1.9 TB/s).
+// 4096 halves took 8.5 us, 16.4 MB at 1.9 TB/s).  TURNS chunks of 8 per thread: all of the row's and the weights' loads go out together,
+// where loads behind a test of the row's length were each waited for before the next (halves, 1003 rows of 4096 6.05 -> 5.26 us, 400
+// of 4096 3.86 -> 3.27, 512 of 8192 7.35 -> 5.81; up to 128 rows the launch).  One, two or four turns: with four, rows of up to 2048 read their
+// first chunk three times more.
 constexpr int kRmsVecThreads = 256, kRmsVecMax = 4;
-template <class XT, class WT, class OT>
+template <class XT, class WT, class OT, int TURNS>
 __global__ __launch_bounds__(kRmsVecThreads) void rmsnorm_vec_kernel(const XT* __restrict__ x, const float* __restrict__ vsum,
                                                                       const WT* __restrict__ w, OT* out, int n, float inv_n, float eps) {
   __shared__ float s_part[kRmsVecThreads / 64];
   const int tid = threadIdx.x, chunks = n >> 3;
   const XT* xr = x + (size_t)blockIdx.x * n;
   OT* orow = out + (size_t)blockIdx.x * n;
-  float v[kRmsVecMax][8], wv[kRmsVecMax][8];
+  float v[TURNS][8], wv[TURNS][8];
 #pragma unroll
-  for (int i = 0; i < kRmsVecMax; ++i) {
+  for (int i = 0; i < TURNS; ++i) {
     const int c = tid + i * kRmsVecThreads;
-    if (i * kRmsVecThreads < chunks) load8(xr + 8 * (size_t)(c < chunks ? c : 0), v[i]);
+    load8(xr + 8 * (size_t)(c < chunks ? c : 0), v[i]);
   }
 #pragma unroll
-  for (int i = 0; i < kRmsVecMax; ++i) {
+  for (int i = 0; i < TURNS; ++i) {
     const int c = tid + i * kRmsVecThreads;
-    if (i * kRmsVecThreads < chunks) load8(w + 8 * (size_t)(c < chunks ? c : 0), wv[i]);
+    load8(w + 8 * (size_t)(c < chunks ? c : 0), wv[i]);
   }
   float ss;
   if (vsum != nullptr) {
@@ -122,7 +125,7 @@ __global__ __launch_bounds__(kRmsVecThreads) void rmsnorm_vec_kernel(const XT* _
   } else {
     float a = 0.f;
 #pragma unroll
-    for (int i = 0; i < kRmsVecMax; ++i)
+    for (int i = 0; i < TURNS; ++i)
       if (tid + i * kRmsVecThreads < chunks)
 #pragma unroll
         for (int k = 0; k < 8; ++k) a = fmaf(v[i][k], v[i][k], a);
@@ -133,7 +136,7 @@ __global__ __launch_bounds__(kRmsVecThreads) void rmsnorm_vec_kernel(const XT* _
   }
   const float r = 1.0f / sqrtf(ss * inv_n + eps);
 #pragma unroll
-  for (int i = 0; i < kRmsVecMax; ++i) {
+  for (int i = 0; i < TURNS; ++i) {
     const int c = tid + i * kRmsVecThreads;
     if (c >= chunks) break;
     float o[8];
@@ -556,8 +559,12 @@ extern "C" int art_rmsnorm(const void* x_dev, const void* vsum_dev, const void* 
   hipStream_t st = (hipStream_t)stream;
   const float* vs = (const float*)vsum_dev;
   const bool vec = n % 8 == 0 && n <= 8 * kRmsVecThreads * kRmsVecMax && (((uintptr_t)x_dev | (uintptr_t)w_dev | (uintptr_t)out_dev) % 16) == 0;
+#define ART_RMS_VEC(XT, WT, OT, TURNS) \
+  rmsnorm_vec_kernel<XT, WT, OT, TURNS><<<dim3(rows), dim3(kRmsVecThreads), 0, st>>>((const XT*)x_dev, vs, (const WT*)w_dev, (OT*)out_dev, n, inv_n, eps)
 #define ART_RMS(XT, WT, OT)                                                                                                                  \
-  if (vec) rmsnorm_vec_kernel<XT, WT, OT><<<dim3(rows), dim3(kRmsVecThreads), 0, st>>>((const XT*)x_dev, vs, (const WT*)w_dev, (OT*)out_dev, n, inv_n, eps); \
+  if (vec && n <= 8 * kRmsVecThreads) ART_RMS_VEC(XT, WT, OT, 1);                                                                            \
+  else if (vec && n <= 2 * 8 * kRmsVecThreads) ART_RMS_VEC(XT, WT, OT, 2);                                                                   \
+  else if (vec) ART_RMS_VEC(XT, WT, OT, kRmsVecMax);                                                                                         \
   else rmsnorm_kernel<XT, WT, OT><<<dim3(rows), dim3(1024), 0, st>>>((const XT*)x_dev, vs, (const WT*)w_dev, (OT*)out_dev, n, inv_n, eps)
   const int key = x_dtype * 4 + w_dtype * 2 + out_dtype;
   switch (key) {
@@ -571,6 +578,7 @@ extern "C" int art_rmsnorm(const void* x_dev, const void* vsum_dev, const void* 
     default: ART_RMS(_Float16, _Float16, _Float16); break;
   }
 #undef ART_RMS
+#undef ART_RMS_VEC
   ART_LAUNCH_CHECK();
   return 0;
 }

@@ -1470,6 +1470,30 @@ def test_convolution_operator_takes_the_kernel_and_agrees_with_the_generic_one(a
     assert ((got - want)[fin].norm() / want[fin].norm()).item() < 2.0 ** -23 * 9 * c       # float32 sums of 9 c terms, another order
 
 
+# one, two and four chunks of 8 per thread, at the ends of each, and a length that is not whole chunks
+@pytest.mark.parametrize('dtype', ['float16', 'float32'])
+@pytest.mark.parametrize('n', [8, 2048, 2056, 4096, 4104, 8192, 1001])
+def test_rmsnorm_rows_of_every_length(autort, dtype, n):
+    """art_rmsnorm against float64: a float32 sum of n squares in some order (n 2^-24 of it at most, half of that in the root), three
+    roundings to float32 and one to the result's type; nothing behind the rows is written."""
+    from ctypes import c_void_p
+    from antares_amd.runtime import capi
+    dev, t = autort.device(), getattr(torch, dtype)
+    capi.init(0)
+    g = torch.Generator().manual_seed(n)
+    x, w = torch.randn(3, n, generator=g).to(t), torch.randn(n, generator=g).to(t)
+    xd, wd, out = x.to(dev), w.to(dev), torch.full((4, n), 7.0, dtype=t, device=dev)
+    kind = int(dtype == 'float16')
+    note(f'rmsnorm {dtype} 3 rows of {n}')
+    capi.check(capi.lib().art_rmsnorm(c_void_p(xd.data_ptr()), None, c_void_p(wd.data_ptr()), c_void_p(out.data_ptr()), 3, n, 1.0 / n, 1e-5, kind, kind, kind,
+                                      c_void_p(torch.cuda.current_stream().cuda_stream)))
+    y = x.double()
+    exact = y / torch.sqrt((y * y).mean(1, keepdim=True) + 1e-5) * w.double()
+    got = out.cpu().double()
+    assert ((got[:3] - exact).abs() <= exact.abs() * ((n / 2 + 8) * 2.0 ** -24 + (2.0 ** -11 if kind else 0)) + 2.0 ** -24).all()
+    assert (got[3] == 7.0).all()
+
+
 # with and without K-splits, one and two turns of a block, a row that is not whole 16-byte pieces of 8 (two launches)
 @pytest.mark.parametrize('M,K,N', [(1, 256, 16), (5, 512, 272), (33, 1024, 4096), (130, 640, 8192), (20, 512, 8208), (300, 256, 144)])
 def test_w4a16_gemm_with_residual_and_rmsnorm_behind_it(autort, M, K, N):
