@@ -105,10 +105,8 @@ __global__ __launch_bounds__(kThreads, MT == 8 ? 1 : 2) void gemm_w4a16_wide_ker
   };
   auto next_weights = [&](auto odd_tag) {           // of the stage whose weights were just fetched; a group is two stages
     w_rows.next();
-    if constexpr (decltype(odd_tag)::value == 1) {
-      q_rows.next();
-      if (w_rows.far()) { w_rows.rebase(); q_rows.rebase(); }
-    }
+    if constexpr (decltype(odd_tag)::value == 1) q_rows.next();
+    if (w_rows.far()) { w_rows.rebase(); q_rows.rebase(); }
   };
 
   // ---- operand roles.  A transposing read takes 8 byte-rows x 16 columns per 16 lanes: lane s16 supplies the 8-byte

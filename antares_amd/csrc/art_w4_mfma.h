@@ -67,7 +67,8 @@ inline int tile_count(int N, bool swiglu, int bn) { return swiglu ? (N / 2 + bn 
 // Rows of memory that a block fetches one after another, `step` bytes apart: a descriptor and the offset of the next.  Behind the last
 // row it stays there: that one is fetched again, into slots that nobody reads, and the loop needs neither branches nor a varying
 // count of loads.  Offsets are 32 bits; FAR, for more than that: wherever one has passed 2 GiB, the descriptor moves on (rebase; in
-// every kernel it would cost 2 to 3 %).
+// every kernel it would cost 2 to 3 %).  A step is at most 2 GiB (67108864 columns of a stage of the wide kernel) and far() is asked
+// behind every next(): an offset of less than 2 GiB and a step stay below 4 GiB, two steps need not.
 template <bool FAR> struct Rows {
   u32x4_t buffer;
   unsigned int at, step, last;

@@ -589,6 +589,7 @@ def test_int4_products_of_more_than_4_gib_of_packed_weights(autort, M, code):
     of 32896 terms (their error is at most 2^-24 times some hundred partial sums)."""
     from ctypes import c_void_p
     from antares_amd.runtime import capi
+    capi.init(0)
     note(f'more than 4 GiB M={M} code={code}')
     dev, K, N = autort.device(), 257 * 128, 262144
     g = torch.Generator(device=dev).manual_seed(M)
@@ -605,6 +606,33 @@ def test_int4_products_of_more_than_4_gib_of_packed_weights(autort, M, code):
     w = (w - zero) * s[:, cols].repeat_interleave(128, 0)
     want, got = (x.double() @ w.double()), y[:, cols].double()
     assert ((got - want).abs() <= want.abs() * 2.0 ** -10 + 2e-3).all(), (got - want).abs().max()
+    assert not torch.isnan(y).any()
+
+
+def test_int4_products_of_the_most_columns(autort):
+    """67108864 columns, the most that a kernel takes: a stage of 32 byte-rows of the packed weights is 2 GiB, so an offset passes 4 GiB
+    with every second one.  Six stages; columns at both ends and in the middle against float64 sums of the same float16 weights:
+    float16 rounding (2^-11), float32 sums of 384 terms."""
+    from ctypes import c_void_p
+    from antares_amd.runtime import capi
+    dev, M, K, N = autort.device(), 4, 384, 1 << 26
+    capi.init(0)
+    note(f'the most columns M={M} K={K} N={N}')
+    g = torch.Generator(device=dev).manual_seed(26)
+    q = torch.randint(0, 256, (K // 2, N), generator=g, device=dev, dtype=torch.uint8)
+    z = torch.randint(0, 256, (K // 128, N // 2), generator=g, device=dev, dtype=torch.uint8)
+    s = (torch.rand(K // 128, N, generator=g, device=dev) * 0.019 + 0.001).half()
+    x = torch.randn(M, K, generator=g, device=dev).half()
+    y = torch.full((M, N), float('nan'), dtype=torch.float16, device=dev)
+    capi.check(capi.lib().art_gemm_w4a16(*(c_void_p(t.data_ptr()) for t in (x, q, s, z, y)), M, K, N, c_void_p(torch.cuda.current_stream().cuda_stream)))
+    cols = torch.cat([torch.arange(0, 16), torch.arange(N // 2 - 8, N // 2 + 8), torch.arange(N - 16, N)]).to(dev)
+    qc, zc = q[:, cols], z[:, cols // 2]
+    w = torch.stack([qc & 15, qc >> 4], 1).reshape(K, -1).half()
+    zero = torch.where(cols % 2 == 0, zc & 15, zc >> 4).half().repeat_interleave(128, 0)
+    w = ((w - zero) * s[:, cols].repeat_interleave(128, 0)).double()
+    want, got = x.double() @ w, y[:, cols].double()
+    room = (x.double().abs() @ w.abs()) * K * 2.0 ** -24
+    assert ((got - want).abs() <= want.abs() * 2.0 ** -11 + room + 2.0 ** -25).all(), (got - want).abs().max()
     assert not torch.isnan(y).any()
 
 
