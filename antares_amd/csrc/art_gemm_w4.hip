@@ -533,10 +533,13 @@ double deep_estimate(int M, int K, int N, const Plan& p, Tail tail, int compute_
 }
 constexpr int kDeepBlocks = 8;                      // of rows
 // What a form's 32-bit offsets (a block's rows of x and of the packed weights), its division by the number of column
-// tiles and its grid hold.  Where the packed weights of a split do not fit 32 bits, two of the forms are left.
-bool far(const Plan& p, int K, int N) { return 64LL * N * ((K / GK + p.splits - 1) / p.splits) > 1LL << 32; }
-bool holds(const Plan& p, int K, int N, Tail tail) {
-  const bool offsets = 64LL * p.row_tiles * K <= 1LL << 32 && 64LL * N <= 1LL << 32;
+// tiles and its grid hold.  Where the packed weights of a split do not fit 32 bits, two of the forms are left.  Offsets end below 4 GiB - 1,
+// the limit of a descriptor: of a load that ends at it the last word comes back as zero.  (x: with K-splits a block's rows end before that.)
+int groups_of(const Plan& p, int K) { return (K / GK + p.splits - 1) / p.splits; }
+bool far(const Plan& p, int K, int N) { return 64LL * N * groups_of(p, K) >= 1LL << 32; }
+bool holds(const Plan& p, int M, int K, int N, Tail tail) {
+  const int rows = M < 32 * p.row_tiles ? M : 32 * p.row_tiles;
+  const bool offsets = 64LL * p.row_tiles * K <= 1LL << 32 && 2LL * K * (rows - 1) + 256LL * groups_of(p, K) < 1LL << 32 && 64LL * N <= 1LL << 32;
   if (p.deep) return offsets && !far(p, K, N) && (long long)deep_tiles(N, tail, p.deep) * p.splits < 1 << 16;
   const long long units = (long long)tile_count(N, tail == kSwiglu, p.wide ? 256 : BN) * p.splits;
   return offsets && units < (p.wide ? 1 << 19 : 1 << 16) && (!far(p, K, N) || p.row_tiles == (p.wide ? 4 : 1));
@@ -554,25 +557,24 @@ bool choose(Plan& best, int M, int K, int N, Tail tail, bool residual, size_t sc
     if (norm_in_pass) t += norm_estimate(M, N, p.splits);
     if (t < t_best) { t_best = t; best = p; }
   };
-  for (int pass = 0; pass < 2 && t_best == 1e30; ++pass) {
+  for (int pass = 0; pass < 3 && t_best == 1e30; ++pass) {        // the wishes; without the form; without the splits
     for (const Plan form : {Plan{false, 1, 1, 0}, Plan{false, 2, 1, 0}, Plan{false, 4, 1, 0}, Plan{true, 4, 1, 0}, Plan{true, 8, 1, 0}}) {
       const int form_code = form.wide ? form.row_tiles : form.row_tiles == 4 ? 5 : form.row_tiles;
       if (pass == 0 && (code != 0 ? code != form_code : 16 * form.row_tiles >= M && form.row_tiles > 1)) continue;     // not over twice the rows
       for (int s = splits > 0 ? splits : 1; s <= (splits > 0 ? splits : 32); ++s) {
         if (splits == 0 && s > 1 && (s > most || 2 * s > G + 1)) break;
         const Plan p{form.wide, form.row_tiles, s > most ? most : s, 0};
-        if (!holds(p, K, N, tail)) break;
-        consider(p, estimate(M, K, N, p, compute_units));
+        if (holds(p, M, K, N, tail)) consider(p, estimate(M, K, N, p, compute_units));
       }
     }
-    if (t_best == 1e30) splits = 1;
+    if (t_best == 1e30) splits = pass == 0 ? 1 : 0;
   }
   if (code == 0 && splits == 0)
     for (const Plan form : {Plan{false, 1, 1, 1}, Plan{false, 1, 1, 2}, Plan{false, 2, 1, 1}}) {
       if (M > 32 * form.row_tiles * kDeepBlocks || 16 * form.row_tiles >= M && form.row_tiles > 1) continue;
       for (int s = 1; s <= 16 && (s == 1 || (s <= most && 2 * s <= G + 1)); ++s) {
         const Plan p{false, form.row_tiles, s, form.deep};
-        if (holds(p, K, N, tail)) consider(p, deep_estimate(M, K, N, p, tail, compute_units));
+        if (holds(p, M, K, N, tail)) consider(p, deep_estimate(M, K, N, p, tail, compute_units));
       }
     }
   return t_best < 1e30;

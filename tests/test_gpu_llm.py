@@ -636,6 +636,33 @@ def test_int4_products_of_the_most_columns(autort):
     assert not torch.isnan(y).any()
 
 
+@pytest.mark.parametrize('M,K,N,code', [(32, 1 << 26, 16, 0), (32, 1 << 26, 16, 256 + 1), (64, 1 << 25, 16, 512 + 1), (128, 1 << 24, 16, 1280 + 1),
+                                        (5, 256 * 128, 262144, 256 + 1), (130, 256 * 128, 262144, 1024 + 1)])
+def test_int4_products_whose_offsets_end_at_4_gib(autort, M, K, N, code):
+    """A block's rows of x, or its packed weights, are 4 GiB to the byte.  Only the last group's values of x are not zero, so that
+    its last bytes count; against float64 sums of the same float16 weights: float16 rounding (2^-11), float32 sums of 128 terms."""
+    from ctypes import c_void_p
+    from antares_amd.runtime import capi
+    capi.init(0)
+    note(f'offsets that end at 4 GiB M={M} K={K} N={N} code={code}')
+    dev = autort.device()
+    g = torch.Generator(device=dev).manual_seed(M)
+    q = torch.randint(0, 256, (K // 2, N), generator=g, device=dev, dtype=torch.uint8)
+    z = torch.randint(0, 256, (K // 128, N // 2), generator=g, device=dev, dtype=torch.uint8)
+    s = (torch.rand(K // 128, N, generator=g, device=dev) * 0.019 + 0.001).half()
+    x = torch.zeros(M, K, dtype=torch.float16, device=dev)
+    x[:, K - 128:] = torch.randn(M, 128, generator=g, device=dev).half()
+    y = torch.full((M, N), float('nan'), dtype=torch.float16, device=dev)
+    capi.check(capi.lib().art_gemm_w4a16_tuned(*(c_void_p(t.data_ptr()) for t in (x, q, s, z, y)), M, K, N, code, c_void_p(torch.cuda.current_stream().cuda_stream)))
+    cols = torch.arange(N - 16, N, device=dev)
+    qc, zc = q[K // 2 - 64:, cols], z[K // 128 - 1, cols // 2]
+    w = torch.stack([qc & 15, qc >> 4], 1).reshape(128, -1).half() - torch.where(cols % 2 == 0, zc & 15, zc >> 4).half()
+    w = (w * s[K // 128 - 1, cols]).double()
+    last, got = x[:, K - 128:].double(), y[:, cols].double()
+    want, room = last @ w, (last.abs() @ w.abs()) * 128 * 2.0 ** -24
+    assert ((got - want).abs() <= want.abs() * 2.0 ** -11 + room + 2.0 ** -25).all(), (got - want).abs().max()
+
+
 @pytest.mark.parametrize('M', [4, 16, 17, 32, 33, 64, 65, 131, 250])
 @pytest.mark.parametrize('K,N', [(128, 16), (1152, 48), (640, 208), (4224, 96), (1024, 1056), (2176, 9008)])
 def test_int4_products_of_a_few_rows_over_blocks_of_32_and_64_columns(autort, M, K, N):
