@@ -539,6 +539,8 @@ int groups_of(const Plan& p, int K) { return (K / GK + p.splits - 1) / p.splits;
 bool far(const Plan& p, int K, int N) { return 64LL * N * groups_of(p, K) >= 1LL << 32; }
 bool holds(const Plan& p, int M, int K, int N, Tail tail) {
   const int rows = M < 32 * p.row_tiles ? M : 32 * p.row_tiles;
+  const long long padded = (M + 32LL * p.row_tiles - 1) / (32 * p.row_tiles) * (32 * p.row_tiles);
+  if (p.splits > 1 && 4LL * N * padded > 1LL << 32) return false;       // PartialTile
   const bool offsets = 64LL * p.row_tiles * K <= 1LL << 32 && 2LL * K * (rows - 1) + 256LL * groups_of(p, K) < 1LL << 32 && 64LL * N <= 1LL << 32;
   if (p.deep) return offsets && !far(p, K, N) && (long long)deep_tiles(N, tail, p.deep) * p.splits < 1 << 16;
   const long long units = (long long)tile_count(N, tail == kSwiglu, p.wide ? 256 : BN) * p.splits;

@@ -93,7 +93,8 @@ template <bool FAR> struct Rows {
 };
 
 // The M x N sums of a K split on their way to the pass that adds them: a buffer of exactly that many bytes, so that what is stored to
-// rows past M is dropped on the way out, without a comparison and a branch for each store.
+// rows past M is dropped on the way out, without a comparison and a branch for each store.  Offsets are 32 bits: 4 N times the rows of
+// all blocks is at most 4 GiB, or what is past M comes round to the first rows.
 struct PartialTile {
   __amdgpu_buffer_rsrc_t buffer;
   unsigned int row;                                 // bytes

@@ -663,6 +663,32 @@ def test_int4_products_whose_offsets_end_at_4_gib(autort, M, K, N, code):
     assert ((got - want).abs() <= want.abs() * 2.0 ** -11 + room + 2.0 ** -25).all(), (got - want).abs().max()
 
 
+@pytest.mark.parametrize('N', [(1 << 22) - 16, (1 << 22) + 16, 4718592])
+def test_one_row_in_blocks_of_256_rows_and_two_splits_of_k(autort, N):
+    """A block of 256 rows over N columns of float32 sums spans 4 GiB: what belongs to rows past M must not come round to the first
+    row.  Against float64 sums of the same float16 weights: float16 rounding (2^-11), float32 sums of 256 terms."""
+    from ctypes import c_void_p
+    from antares_amd.runtime import capi
+    capi.init(0)
+    note(f'one row in blocks of 256, two splits, N={N}')
+    dev, M, K = autort.device(), 1, 256
+    g = torch.Generator(device=dev).manual_seed(22)
+    q = torch.randint(0, 256, (K // 2, N), generator=g, device=dev, dtype=torch.uint8)
+    z = torch.randint(0, 256, (K // 128, N // 2), generator=g, device=dev, dtype=torch.uint8)
+    s = (torch.rand(K // 128, N, generator=g, device=dev) * 0.019 + 0.001).half()
+    x = torch.randn(M, K, generator=g, device=dev).half()
+    y = torch.full((M, N), float('nan'), dtype=torch.float16, device=dev)
+    capi.check(capi.lib().art_gemm_w4a16_tuned(*(c_void_p(t.data_ptr()) for t in (x, q, s, z, y)), M, K, N, 2048 + 2, c_void_p(torch.cuda.current_stream().cuda_stream)))
+    for first in range(0, N, 1 << 18):
+        cols = torch.arange(first, min(first + (1 << 18), N), device=dev)
+        qc, zc = q[:, cols], z[:, cols // 2]
+        zero = torch.where(cols % 2 == 0, zc & 15, zc >> 4).half().repeat_interleave(128, 0)
+        w = ((torch.stack([qc & 15, qc >> 4], 1).reshape(K, -1).half() - zero) * s[:, cols].repeat_interleave(128, 0)).double()
+        want, got = x.double() @ w, y[:, cols].double()
+        room = (x.double().abs() @ w.abs()) * K * 2.0 ** -24
+        assert ((got - want).abs() <= want.abs() * 2.0 ** -11 + room + 2.0 ** -25).all(), (got - want).abs().max()
+
+
 @pytest.mark.parametrize('M', [4, 16, 17, 32, 33, 64, 65, 131, 250])
 @pytest.mark.parametrize('K,N', [(128, 16), (1152, 48), (640, 208), (4224, 96), (1024, 1056), (2176, 9008)])
 def test_int4_products_of_a_few_rows_over_blocks_of_32_and_64_columns(autort, M, K, N):
