@@ -186,6 +186,8 @@ def _w4a16_handler(op, bound, env, call) -> bool:
             # 1280 + v: over blocks of 128 rows; 1024 + v, 2048 + v: of 128 and 256 rows and twice the columns
             cands = [0] + [512 + v for v in counts] + ([256 + v for v in counts] if M > 32 else [])
             cands += [rows + v for rows in (1280, 1024, 2048) for v in counts if v <= 16] if M > 64 else []
+            # 2304, 2560 + v: blocks of 32 rows whose wavefronts divide K, over 32 and 64 columns; 2816 + v: of 64 rows over 32 columns
+            cands += [form + v for form, rows in ((2304, 256), (2560, 256), (2816, 512)) for v in counts if v <= 16 and M <= rows]
         saved = tune_hand_kernel(op, key, cands, run, trials, clones)
         del clones
     call.library(entry, x, q, s, z, y, M, K, N, *knobs(saved['value'] if saved is not None else 0), STREAM)

@@ -542,11 +542,14 @@ bool holds(const Plan& p, int M, int K, int N, Tail tail) {
   const long long padded = (M + 32LL * p.row_tiles - 1) / (32 * p.row_tiles) * (32 * p.row_tiles);
   if (p.splits > 1 && 4LL * N * padded > 1LL << 32) return false;       // PartialTile
   const bool offsets = 64LL * p.row_tiles * K <= 1LL << 32 && 2LL * K * (rows - 1) + 256LL * groups_of(p, K) < 1LL << 32 && 64LL * N <= 1LL << 32;
-  if (p.deep) return offsets && !far(p, K, N) && (long long)deep_tiles(N, tail, p.deep) * p.splits < 1 << 16;
+  if (p.deep) return offsets && !far(p, K, N) && (long long)deep_tiles(N, tail, p.deep) * p.splits < 1 << 16 && M <= 32 * p.row_tiles * kDeepBlocks;
   const long long units = (long long)tile_count(N, tail == kSwiglu, p.wide ? 256 : BN) * p.splits;
   return offsets && units < (p.wide ? 1 << 19 : 1 << 16) && (!far(p, K, N) || p.row_tiles == (p.wide ? 4 : 1));
 }
-// False: no form takes these sizes.  `code` and `splits` are the caller's wishes (0: none; the deep kernel comes with none); a form that
+// What a caller's k_splits calls a form: rows of a block / 32, 5: 128 rows x 128 columns, 9, 10, 11: art_gemm_w4_deep.hip with 32 x 32, 32 x 64,
+// 64 rows x 32 columns.
+int code_of(const Plan& p) { return p.deep ? 7 + 2 * p.row_tiles + (p.deep == 2 ? 1 : 0) : !p.wide && p.row_tiles == 4 ? 5 : p.row_tiles; }
+// False: no form takes these sizes.  `code` and `splits` are the caller's wishes (0: none; splits alone: not the deep kernel); a form that
 // does not hold the sizes is replaced by one that does.  A product with a
 // residual counts as one with a norm behind it, in its own call or the next: the bits of y are the same in both.
 bool choose(Plan& best, int M, int K, int N, Tail tail, bool residual, size_t scratch_bytes, int compute_units, int code, int splits) {
@@ -560,25 +563,18 @@ bool choose(Plan& best, int M, int K, int N, Tail tail, bool residual, size_t sc
     if (t < t_best) { t_best = t; best = p; }
   };
   for (int pass = 0; pass < 3 && t_best == 1e30; ++pass) {        // the wishes; without the form; without the splits
-    for (const Plan form : {Plan{false, 1, 1, 0}, Plan{false, 2, 1, 0}, Plan{false, 4, 1, 0}, Plan{true, 4, 1, 0}, Plan{true, 8, 1, 0}}) {
-      const int form_code = form.wide ? form.row_tiles : form.row_tiles == 4 ? 5 : form.row_tiles;
-      if (pass == 0 && (code != 0 ? code != form_code : 16 * form.row_tiles >= M && form.row_tiles > 1)) continue;     // not over twice the rows
-      for (int s = splits > 0 ? splits : 1; s <= (splits > 0 ? splits : 32); ++s) {
+    for (const Plan form : {Plan{false, 1, 1, 0}, Plan{false, 2, 1, 0}, Plan{false, 4, 1, 0}, Plan{true, 4, 1, 0}, Plan{true, 8, 1, 0},
+                            Plan{false, 1, 1, 1}, Plan{false, 1, 1, 2}, Plan{false, 2, 1, 1}}) {
+      if (form.deep && (pass > 0 || code == 0 && splits > 0)) continue;
+      if (pass == 0 && (code != 0 ? code != code_of(form) : 16 * form.row_tiles >= M && form.row_tiles > 1)) continue;      // not over twice the rows
+      for (int s = splits > 0 ? splits : 1; s <= (splits > 0 ? splits : form.deep ? 16 : 32); ++s) {
         if (splits == 0 && s > 1 && (s > most || 2 * s > G + 1)) break;
-        const Plan p{form.wide, form.row_tiles, s > most ? most : s, 0};
-        if (holds(p, M, K, N, tail)) consider(p, estimate(M, K, N, p, compute_units));
+        const Plan p{form.wide, form.row_tiles, s > most ? most : s, form.deep};
+        if (holds(p, M, K, N, tail)) consider(p, p.deep ? deep_estimate(M, K, N, p, tail, compute_units) : estimate(M, K, N, p, compute_units));
       }
     }
     if (t_best == 1e30) splits = pass == 0 ? 1 : 0;
   }
-  if (code == 0 && splits == 0)
-    for (const Plan form : {Plan{false, 1, 1, 1}, Plan{false, 1, 1, 2}, Plan{false, 2, 1, 1}}) {
-      if (M > 32 * form.row_tiles * kDeepBlocks || 16 * form.row_tiles >= M && form.row_tiles > 1) continue;
-      for (int s = 1; s <= 16 && (s == 1 || (s <= most && 2 * s <= G + 1)); ++s) {
-        const Plan p{false, form.row_tiles, s, form.deep};
-        if (holds(p, M, K, N, tail)) consider(p, deep_estimate(M, K, N, p, tail, compute_units));
-      }
-    }
   return t_best < 1e30;
 }
 // An RMSNorm of the result: out = fp16(y / rms(y) * weight).
@@ -652,12 +648,17 @@ int run_rows(const _Float16* xs, const unsigned char* qweight, const _Float16* s
   return norm && !norm_there ? art_rmsnorm(ys, nullptr, norm->weight, norm->out, M, N, 1.0f / (float)N, norm->eps, 1, 1, 1, st) : 0;
 }
 
+bool code_taken(int k_splits) {
+  const int code = k_splits >> 8;
+  return k_splits >= 0 && (code <= 2 || code == 4 || code == 5 || code >= 8 && code <= 11);
+}
+
 int run(const void* x_dev, const void* qweight_dev, const void* scales_dev, const void* qzeros_dev, void* y_dev, const void* residual_dev,
         int M, int K, int N, int k_splits, Tail tail, const Norm* norm, const Rope* rope, void* stream) {
   const int n_out = tail == kSwiglu ? N / 2 : tail == kRope ? N / 3 : N;
-  const int code = k_splits >> 8;                   // 0: library's choice; else rows of a block / 32, 5: 128 rows x 128 columns
-  ART_REQUIRE(k_splits >= 0 && (code <= 2 || code == 4 || code == 5 || code == 8),
-              "art_gemm_w4a16: k_splits must be 0 (library's choice) or 1..255, plus 256 x the rows-per-block code 1, 2, 4, 5 or 8 (got %d)", k_splits);
+  const int code = k_splits >> 8;                   // 0: library's choice; else code_of
+  ART_REQUIRE(code_taken(k_splits),
+              "art_gemm_w4a16: k_splits must be 0 (library's choice) or 1..255, plus 256 x the rows-per-block code 1, 2, 4, 5 or 8 to 11 (got %d)", k_splits);
   ART_REQUIRE(((uintptr_t)residual_dev % 8) == 0, "art_gemm_w4a16: the residual must be 8-byte aligned");
   ART_REQUIRE(!art::overlaps(x_dev, (size_t)M * K * 2, y_dev, (size_t)M * n_out * 2), "art_gemm_w4a16: y must not overlap x");
   ART_REQUIRE(x_dev && qweight_dev && scales_dev && qzeros_dev && y_dev, "art_gemm_w4a16: null pointer");
@@ -685,6 +686,13 @@ int run(const void* x_dev, const void* qweight_dev, const void* scales_dev, cons
 }
 
 }  // namespace
+
+extern "C" int art_gemm_w4a16_form(int M, int K, int N, int tail, int residual, int k_splits) {
+  Plan p;
+  if (M < 1 || K < 1 || N < 1 || K % GK != 0 || N % 16 != 0 || tail < kPlain || tail > kRope || !code_taken(k_splits)) return 0;
+  if (!choose(p, M < kMaxRows ? M : kMaxRows, K, N, (Tail)tail, residual != 0, art_workspace_bytes() - art::kScratchOffset, 256, k_splits >> 8, k_splits & 0xff)) return 0;
+  return 256 * code_of(p) + p.splits;
+}
 
 extern "C" int art_gemm_w4a16(const void* x_dev, const void* qweight_dev, const void* scales_dev, const void* qzeros_dev,
                               void* y_dev, int M, int K, int N, void* stream) {

@@ -85,6 +85,7 @@ _SIGNATURES = {
                                            c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_void_p]),
     'art_decode_attention_rope': (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_void_p, c_int, c_void_p]),
     'art_rope_qkv_store': (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_void_p, c_int, c_int, c_int, c_void_p]),
+    'art_gemm_w4a16_form': (c_int, [c_int, c_int, c_int, c_int, c_int, c_int]),
     'art_gemm_tile_form': (c_int, [c_int, c_int, c_int, c_int, c_int, c_int, c_int]),
     'art_gemm_tile': (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p]),
     'art_gemm_f16': (c_int, [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p]),

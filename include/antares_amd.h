@@ -137,8 +137,10 @@ int art_gemv_w4a16(const void* x_dev, const void* qweight_dev, const void* scale
  *                  plus 256 for blocks of 32 rows, 512 for 64, 1280 for 128 (all over 128 columns), 1024 for 128 or 2048 for
  *                  256 rows over 256 columns (none: the library picks): more rows per block unpack a weight for more
  *                  row tiles, fewer make more blocks, which need fewer K-splits, i.e. fewer fp32 copies of the output
- *                  written and read back.  Blocks that cannot number or address the columns (65536 tiles of 128) are
- *                  replaced by ones that can;
+ *                  written and read back.  2304, 2560, 2816: small blocks of 32 rows x 32 columns, 32 x 64, 64 x 32 whose wavefronts
+ *                  divide K, for up to 8 blocks of rows.  Blocks that cannot number or address the rows or columns (65536 tiles of 128)
+ *                  are replaced by ones that can (art_gemm_w4a16_form: 256 * form + splits as a product of these sizes runs, on 256 compute
+ *                  units; 0: not taken.  tail 0 plain, 1 SwiGLU, 2 rotation and store);
  *   max_blocks:    cap on the blocks of the partition, 64..16384 (each walks its span tile by tile). */
 int art_gemv_w4a16_tuned(const void* x_dev, const void* qweight_dev, const void* scales_dev, const void* qzeros_dev,
                          void* y_dev, int M, int K, int N, int k_per_block, void* stream);
@@ -149,6 +151,7 @@ int art_gemv_w4a16_knobs(const void* x_dev, const void* qweight_dev, const void*
                          void* y_dev, int M, int K, int N, int rows_per_lane, int waves_per_block, void* stream);
 int art_gemm_w4a16_tuned(const void* x_dev, const void* qweight_dev, const void* scales_dev, const void* qzeros_dev,
                          void* y_dev, int M, int K, int N, int k_splits, void* stream);
+int art_gemm_w4a16_form(int M, int K, int N, int tail, int residual, int k_splits);
 int art_partition_even_first_i32_tuned(const void* in_dev, void* out_dev, long long n, int max_blocks, void* stream);
 /* art_gemm_w4a16_tuned with the residual add that follows a projection (samples/05_llama2_7b_int4.py:168,173) folded
  * into the last pass: y = fp16(fp16(product) + residual).  residual_dev: fp16 [M,N], may be y itself, may be NULL. */

@@ -485,6 +485,42 @@ def test_the_q_k_v_product_that_rotates_and_stores(T, K, H):
         autort.ops.gemm_w4a16_rope_store(*d, angles, q, kc, kc)
 
 
+@pytest.mark.parametrize('T,K,H', [(5, 256, 1), (16, 1152, 2), (20, 640, 3), (33, 512, 3), (129, 384, 2), (250, 256, 5)])
+def test_the_q_k_v_product_that_rotates_and_stores_in_small_blocks(T, K, H):
+    """As above, blocks of 32 x 32, 32 x 64 and 64 x 32 by their launch parameter, one and more K-splits."""
+    import autort
+    from ctypes import c_void_p
+    from antares_amd import workloads
+    from antares_amd.runtime import capi
+    dev, N, first = autort.device(), 3 * H * 128, 4
+    capi.init(0)
+    p = workloads.w4_problem(T + K + H, T, K, N)
+    d = [p[k].to(dev) for k in ('x', 'qweight', 'scales', 'qzeros')]
+    half = (1.0 / (10000 ** (torch.arange(0, 128, 2).float() / 128))).half()
+    inv = torch.cat([half, half]).to(dev)
+    angles = autort.ops.rope_angles_f16(inv, torch.empty(T, 64, 2, device=dev), extra=[first])
+
+    def outputs():
+        return [torch.full((T, H, 128), 7.0, dtype=torch.float16, device=dev)] + [torch.full((T + 9, H * 128), 7.0, dtype=torch.float16, device=dev) for _ in range(2)]
+    for code in [256 * form + splits for form in (9, 10, 11) for splits in (1, 2, 3) if splits <= K // 128]:
+        note(f'q k v product T={T} K={K} H={H} code {code}')
+        assert capi.lib().art_gemm_w4a16_form(T, K, N, 2, 0, code) == code
+        qkv = torch.empty(T, N, dtype=torch.float16, device=dev)
+        capi.check(capi.lib().art_gemm_w4a16_tuned(*(c_void_p(t.data_ptr()) for t in d + [qkv]), T, K, N, code, c_void_p(torch.cuda.current_stream().cuda_stream)))
+        got, want = outputs(), outputs()
+        autort.ops.gemm_w4a16_rope_store(*d, angles, *got, extra=[first], k_splits=code)
+        autort.ops.rope_qkv_store_rows_f16(qkv, inv, *want, extra=[first])
+        assert torch.equal(got[2], want[2])
+        for part, (a, b) in enumerate(zip(got[:2], want[:2])):
+            if part:
+                assert (a[:first] == 7.0).all() and (a[first + T:] == 7.0).all()
+                a, b = a[first:first + T], b[first:first + T]
+            x = qkv[:, part * H * 128:(part + 1) * H * 128].view(T, H, 2, 64).double().abs()
+            terms = x.sum(2, keepdim=True).expand(T, H, 2, 64).reshape(T, H, 128)
+            a, b = a.view(T, H, 128).double(), b.view(T, H, 128).double()
+            assert ((a - b).abs() <= torch.maximum(a.abs(), b.abs()) * 2.0 ** -10 + terms * 2.0 ** -22 + 2.0 ** -24).all()
+
+
 def _tile_sums_of_squares(y: torch.Tensor) -> np.ndarray:
     """What a projection leaves in its sum-of-squares buffer for the fp16 outputs y: per tile of 128 columns the sum of
     floor(y^2 * 2^30), each square capped at 2^25 (integer arithmetic)."""
@@ -721,3 +757,54 @@ def test_int4_products_of_a_few_rows_over_blocks_of_32_and_64_columns(autort, M,
         rg, ru = room[:, :N // 2] + gate.abs() * 2.0 ** -11, room[:, N // 2:] + up.abs() * 2.0 ** -11
         silu = torch.nn.functional.silu(gate)
         near(hid, silu * up, 1.1 * rg * up.abs() + silu.abs() * ru + 1.1 * rg * ru + (silu * up).abs() * 2.0 ** -20)
+
+
+@pytest.mark.parametrize('form', [9, 10, 11])
+@pytest.mark.parametrize('M', [1, 4, 16, 17, 32, 33, 64, 65, 131, 250])
+def test_int4_products_in_small_blocks_by_their_launch_parameter(autort, M, form):
+    """Blocks of 32 x 32, 32 x 64 and 64 x 32, one and more K-splits: plain with and without a residual, SwiGLU, RMSNorm behind it;
+    matrices that end a half and a quarter inside a block.  Bounds as in the test above; the norm's: its own arithmetic over the float16
+    result that it is given, and that result's bits are those of the product by itself."""
+    from ctypes import c_void_p
+    from antares_amd.runtime import capi
+    capi.init(0)
+    dev, lib, stream = autort.device(), capi.lib(), c_void_p(torch.cuda.current_stream().cuda_stream)
+
+    def ptr(*tensors):
+        return [c_void_p(t.data_ptr()) for t in tensors]
+
+    def near(got, want, room):
+        assert ((got.double() - want).abs() <= want.abs() * 2.0 ** -11 + room + 2.0 ** -25).all(), ((got.double() - want).abs() - room).max()
+    for K, N in ((128, 16), (1152, 96), (640, 208), (2176, 224), (1024, 1056)):
+        g = torch.Generator(device=dev).manual_seed(M * 7 + K + N)
+        q = torch.randint(0, 256, (K // 2, N), generator=g, device=dev, dtype=torch.uint8)
+        z = torch.randint(0, 256, (K // 128, N // 2), generator=g, device=dev, dtype=torch.uint8)
+        s = (torch.rand(K // 128, N, generator=g, device=dev) * 0.019 + 0.001).half()
+        x, res, norm = torch.randn(M, K, generator=g, device=dev).half(), torch.randn(M, N, generator=g, device=dev).half(), torch.randn(N, generator=g, device=dev).half()
+        zero = torch.stack([z & 15, z >> 4], 2).reshape(K // 128, N).half().repeat_interleave(128, 0)
+        w = ((torch.stack([q & 15, q >> 4], 1).reshape(K, N).half() - zero) * s.repeat_interleave(128, 0)).double()
+        want, room = x.double() @ w, (x.double().abs() @ w.abs()) * K * 2.0 ** -24
+        for splits in sorted({1, min(2, K // 128), min(3, K // 128), K // 128}):
+            code = 256 * form + splits
+            note(f'small blocks M={M} K={K} N={N} code={code}')
+            assert all(lib.art_gemm_w4a16_form(M, K, N, 0, residual, code) == code for residual in (0, 1))
+            out = torch.full((M, N), float('nan'), dtype=torch.float16, device=dev)
+            capi.check(lib.art_gemm_w4a16_tuned(*ptr(x, q, s, z, out), M, K, N, code, stream))
+            near(out, want, room)
+            y, normed = res.clone(), torch.full((M, N), float('nan'), dtype=torch.float16, device=dev)
+            capi.check(lib.art_gemm_w4a16_residual(*ptr(x, q, s, z, y, y), M, K, N, code, stream))
+            near(y, want + res.double(), room + want.abs() * 2.0 ** -11)
+            y2 = res.clone()
+            capi.check(lib.art_gemm_w4a16_residual_norm(*ptr(x, q, s, z, y2, y2, norm, normed), M, K, N, 1e-5, code, stream))
+            assert torch.equal(y2, y)
+            yd = y.double()
+            exact = yd / torch.sqrt((yd * yd).mean(1, keepdim=True) + 1e-5) * norm.double()
+            near(normed, exact, exact.abs() * (N / 2 + 8) * 2.0 ** -24)
+            if N % 32 == 0:
+                assert lib.art_gemm_w4a16_form(M, K, N, 1, 0, code) == code
+                hid = torch.full((M, N // 2), float('nan'), dtype=torch.float16, device=dev)
+                capi.check(lib.art_gemm_w4a16_swiglu(*ptr(x, q, s, z, hid), M, K, N, code, stream))
+                gate, up = want[:, :N // 2], want[:, N // 2:]
+                rg, ru = room[:, :N // 2] + gate.abs() * 2.0 ** -11, room[:, N // 2:] + up.abs() * 2.0 ** -11
+                silu = torch.nn.functional.silu(gate)
+                near(hid, silu * up, 1.1 * rg * up.abs() + silu.abs() * ru + 1.1 * rg * ru + (silu * up).abs() * 2.0 ** -20)

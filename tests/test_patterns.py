@@ -236,3 +236,27 @@ def test_calls_without_room_for_their_scratch_memory_take_a_form_that_needs_less
     assert taken(op, bound, env) == (True, [gathered], False)
     room[0] -= 1
     assert taken(op, bound, env) == (False, [], False)
+
+
+def test_forms_of_the_int4_product():
+    """Every form runs where it is asked for; one that cannot number or address its rows and columns is replaced, and what
+    no form takes is refused: offsets of a block's x and of its sums of a K split end below 4 GiB, weights of 4 GiB and more come with two forms."""
+    form = capi.lib().art_gemm_w4a16_form
+    for code in (1, 2, 4, 5, 8, 9, 10, 11):
+        for splits in (1, 3):
+            assert form(250, 1024, 1056, 0, 0, 256 * code + splits) == 256 * code + splits
+    assert form(64, 4096, 4096, 0, 0, 3) & 255 == 3 and form(64, 4096, 4096, 0, 0, 3) >> 8 in (1, 2)
+    assert form(64, 256, 4096, 0, 0, 2304 + 9) == 2304 + 2                                # no more splits than groups
+    for code in (3, 6, 7, 12, 255):
+        assert form(64, 4096, 4096, 0, 0, 256 * code) == 0
+    assert form(64, 4096, 4104, 0, 0, 0) == 0 and form(64, 4160, 4096, 0, 0, 0) == 0 and form(0, 4096, 4096, 0, 0, 0) == 0
+    assert form(257, 1024, 1056, 0, 0, 2304 + 1) >> 8 not in (0, 9) and form(512, 1024, 1056, 0, 0, 2816 + 1) == 2816 + 1
+    assert form(4, 384, 1 << 26, 0, 0, 0) == 1024 + 1 and form(4, 384, (1 << 26) + 16, 0, 0, 0) == 0
+    assert form(32, (1 << 26) - 128, 16, 0, 0, 256 + 1) == 256 + 1
+    assert form(32, 1 << 26, 16, 0, 0, 256 + 1) & 255 > 1 and form(64, 1 << 25, 16, 0, 0, 512 + 1) not in (0, 512 + 1) and form(4, (1 << 26) + 128, 16, 0, 0, 0) == 0
+    for code, taken in ((1, 1), (2, None), (5, None), (4, 4), (8, None), (9, None)):
+        got = form(200, 256 * 128, 262144, 0, 0, 256 * code + 1)
+        assert got and (got == 256 * code + 1) == (taken is not None)
+        assert form(200, 255 * 128, 262144, 0, 0, 256 * code + 1) == 256 * code + 1
+    assert form(1, 256, 1 << 22, 0, 0, 2048 + 2) == 2048 + 2
+    assert form(1, 256, (1 << 22) + 16, 0, 0, 2048 + 2) not in (0, 2048 + 2)
