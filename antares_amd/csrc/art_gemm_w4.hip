@@ -493,43 +493,56 @@ struct Plan {
   int row_tiles, splits;
   int deep;                                         // column tiles of a block of art_gemm_w4_deep.hip, 0: not that kernel
 };
-// What a launch takes, in microseconds.  K-splits: the second launch and the fp32 tiles on top.
-double splits_estimate(int M, int N, int splits) { return splits > 1 ? 1.8 + (8.0 * splits + 2.0) * M * N / 4.2e6 : 0.0; }
+// What a launch takes, in microseconds.  K-splits: the second launch and the fp32 tiles on top; of more than eight the pass that also turns or
+// gates waits twice (q | k | v of one head, 8 rows, K = 3712: 5.8 us in seven splits, 9.3 in fifteen).
+double splits_estimate(int M, int N, int splits, Tail tail) {
+  return splits > 1 ? 1.8 + (8.0 * splits + 2.0) * M * N / 4.2e6 + (splits > 8 && tail != kPlain ? 2.65 : 0.0) : 0.0;
+}
 // Where K-splits meet in a pass of their own, a norm is part of that pass, up to 256 rows: beyond them nothing is
 // gained (8 layers of the same pass: 1384 -> 1368 us at 256 tokens, 1861 and 1854 at 300, 2178 and 2183 at 500).
 bool norm_fits(int M, int N) { return M <= 256 && N % 8 == 0 && N <= 8 * kNormThreads * kNormTurns; }
 // Else it is a launch of its own.
 double norm_estimate(int M, int N, int splits) { return splits == 1 ? 2.4 + 2.0e-6 * M * N : 0.0; }
-// A fixed part, one or two co-resident blocks' time per group and round (one's: more with more of the compute units at work), the
-// ramp and the meeting of the k halves again for every further round of blocks of 128 columns (4 rows over 4096 x 12288: 13.3 us with
-// 480 blocks, i.e. 5 K-splits in one round, 14.6 with 768).  Constants of both estimates from all
-// forms over 6200 sizes of 4 to 1003 rows, 512 x 512 to 11008 x 14700, on MI355X, a quarter with weights that stay in the last-level cache, the
-// others with weights from HBM, as a model's are (up to 1.4 times the time): the pick is 1 to 2 % slower than the fastest form in both.  From
-// the former alone prompts lost: a layer of 32 heads at 8 and 64 tokens 71 and 82 us, now 62 and 78; of 8 heads 27 and 32, now 23 and 28.
-double estimate(int M, int K, int N, const Plan& p, int compute_units) {
-  struct Cost { double fixed, one, two; int per_cu; double busy; };
-  const Cost c = p.wide ? (p.row_tiles == 8 ? Cost{8.5, 2.16, 1.94, 1, 0} : Cost{5.2, 1.2, 2.3, 2, 0})
-                        : p.row_tiles == 4 ? Cost{4.8, 0.52, 0.82, 1, 0} : p.row_tiles == 2 ? Cost{4.75, 0.410, 0.985, 2, 0.12} : Cost{3.75, 0.348, 0.848, 2, 0};
+// A fixed part, one or two co-resident blocks' time per group and round (one's: more with more of the compute units at work; either: more where
+// several blocks of rows unpack the same weights), the ramp and the meeting of the k halves again for every further round of blocks of 128
+// columns (4 rows over 4096 x 12288: 13.3 us with 480 blocks, i.e. 5 K-splits in one round, 14.6 with 768).  Constants of 128 columns x 128 rows and
+// of 256 columns from all forms over 6200 sizes of 4 to 1003 rows on MI355X, a quarter with weights that stay in the last-level cache; the others, and
+// those of deep_estimate, from 4065 sizes of 4 to 512 rows, 512 x 512 to 8192 x 24576, each with weights from HBM, as a model's are, and from the
+// cache, the former counting 70 %: the pick is 0.9 and 1.2 % slower than the fastest form.  Without the terms for blocks of rows,
+// rows whole KiB apart and halves it was 2.1 and 1.7 % slower, and lost 20 to 40 % at square matrices of 4096 and more (weights from HBM, us: 8 rows over
+// 4096 x 4096 10.1, now 7.8; 5120 x 5120 14.0, 9.2; 64 rows over 11008 x 4096 18.5, 15.9; 256 rows 34.4, 32.1; 64 rows over 4096 x 12288 18.6, 17.7).
+// Where a product from the cache would rather have the narrow blocks it loses (8 rows over 5120 x 5120 6.9, now 7.9).
+double estimate(int M, int K, int N, const Plan& p, Tail tail, int compute_units) {
+  struct Cost { double fixed, one, two; int per_cu; double busy, rows; };
+  const Cost c = p.wide ? (p.row_tiles == 8 ? Cost{8.5, 2.16, 1.94, 1, 0, 0} : Cost{5.2, 1.2, 2.3, 2, 0, 0})
+                        : p.row_tiles == 4 ? Cost{4.8, 0.52, 0.82, 1, 0, 0} : p.row_tiles == 2 ? Cost{4.373, 0.422, 0.924, 2, 0.073, 0.037} : Cost{3.83, 0.401, 0.863, 2, 0.001, 0.044};
   const int groups = (K / GK + p.splits - 1) / p.splits, m_blocks = (M + 32 * p.row_tiles - 1) / (32 * p.row_tiles);
-  const int blocks = tile_count(N, false, p.wide ? 256 : BN) * m_blocks * p.splits, round = c.per_cu * compute_units;
-  const int rest = blocks % round;
-  const double one = c.one * (1 + c.busy * (blocks < compute_units ? (double)blocks / compute_units : 1.0));
-  double per_group = blocks / round * c.two;
-  if (rest > compute_units) per_group += c.two;
-  else if (rest > 0) per_group += c.per_cu == 2 || blocks > round ? one : one + (c.two - one) * rest / compute_units;
+  const int blocks = tile_count(N, false, p.wide ? 256 : BN) * m_blocks * p.splits, round = c.per_cu * compute_units, rest = blocks % round;
+  const double busy = blocks < compute_units ? (double)blocks / compute_units : 1.0;
+  double one = 0.0, two = blocks / round;           // rounds of each kind
+  if (rest > compute_units) two += 1.0;
+  else if (rest > 0) {
+    one = c.per_cu == 2 || blocks > round ? 1.0 : 1.0 - (double)rest / compute_units;
+    two += 1.0 - one;
+  }
+  const double per_group = (c.one + c.busy * busy) * one + c.two * two + c.rows * busy * (1.0 - 1.0 / m_blocks) * (one + two);
   const double again = p.wide ? 0.0 : 0.73 * ((blocks - 1) / round);
-  return c.fixed + again + groups * per_group + splits_estimate(M, N, p.splits);
+  return c.fixed + again + groups * per_group + splits_estimate(M, N, p.splits, tail);
 }
 // art_gemm_w4_deep.hip: a fixed part and, for each group, what the load path of a compute unit needs for it (all eight wavefronts share it,
-// so groups count, not rounds of them), more with more of the compute units at work and with each further block on one.
+// so groups count, not rounds of them), more with more of the compute units at work and with each further block on one.  Narrow blocks
+// have few bytes on their way to HBM, and wait longest where rows are whole KiB apart (4992 x 3808, one split: 9.5 us; 5120 x 5120: 13.9, from the
+// cache 6.8) and for pieces of 16 columns of two halves (gate | up).
 double deep_estimate(int M, int K, int N, const Plan& p, Tail tail, int compute_units) {
-  struct Cost { double fixed, group, busy, further, again; };
-  const Cost c = p.deep == 2 ? (M <= 16 ? Cost{3.26, 0.155, 0.418, 2.13, 0.44} : Cost{3.50, 0.178, 0.263, 1.63, 1.20})
-                 : p.row_tiles == 2 ? Cost{3.18, 0.201, 0.391, 1.34, 1.23} : M <= 16 ? Cost{3.04, 0.103, 0.332, 2.10, 0.36} : Cost{3.22, 0.151, 0.066, 1.38, 1.11};
+  struct Cost { double fixed, group, busy, further, again, whole_kib, halves; };
+  const Cost c = p.deep == 2 ? (M <= 16 ? Cost{3.569, 0.172, 0.047, 0.270, 0.408, 0.030, 0.014} : Cost{3.314, 0.215, 0.057, 0.224, 1.622, 0.029, 0.037})
+                 : p.row_tiles == 2 ? Cost{3.187, 0.213, 0.113, 0.229, 1.483, 0.021, 0.026}
+                 : M <= 16 ? Cost{3.035, 0.104, 0.059, 0.159, 0.370, 0.034, 0.024} : Cost{3.073, 0.144, 0.051, 0.179, 1.320, 0.027, 0.028};
   const int groups = (K / GK + p.splits - 1) / p.splits, m_blocks = (M + 32 * p.row_tiles - 1) / (32 * p.row_tiles);
   const int blocks = deep_tiles(N, tail, p.deep) * m_blocks * p.splits, more = (blocks - 1) / compute_units;
   const double busy = blocks < compute_units ? (double)blocks / compute_units : 1.0;
-  return c.fixed + c.group * groups * (1 + c.busy * busy + c.further * more) + c.again * more + splits_estimate(M, N, p.splits);
+  const double waits = (N % 1024 == 0 ? c.whole_kib : 0.0) + (tail == kSwiglu ? c.halves : 0.0);
+  return c.fixed + groups * (c.group + c.busy * busy + c.further * more + waits * (1 + more)) + c.again * more + splits_estimate(M, N, p.splits, tail);
 }
 constexpr int kDeepBlocks = 8;                      // of rows
 // What a form's 32-bit offsets (a block's rows of x and of the packed weights), its division by the number of column
@@ -570,7 +583,7 @@ bool choose(Plan& best, int M, int K, int N, Tail tail, bool residual, size_t sc
       for (int s = splits > 0 ? splits : 1; s <= (splits > 0 ? splits : form.deep ? 16 : 32); ++s) {
         if (splits == 0 && s > 1 && (s > most || 2 * s > G + 1)) break;
         const Plan p{form.wide, form.row_tiles, s > most ? most : s, form.deep};
-        if (holds(p, M, K, N, tail)) consider(p, p.deep ? deep_estimate(M, K, N, p, tail, compute_units) : estimate(M, K, N, p, compute_units));
+        if (holds(p, M, K, N, tail)) consider(p, p.deep ? deep_estimate(M, K, N, p, tail, compute_units) : estimate(M, K, N, p, tail, compute_units));
       }
     }
     if (t_best == 1e30) splits = pass == 0 ? 1 : 0;
