@@ -46,7 +46,7 @@ def compile_cached(source: str) -> bytes:
     """HIP source -> code object.  Code objects are cached on disk by the hash
     of their source and of the options that the library adds, so a process only
     compiles what no earlier process has compiled.  Needs no GPU."""
-    key = hashlib.sha256((capi.COMPILE_OPTIONS + source).encode()).hexdigest()[:24]
+    key = hashlib.sha256((capi.compile_options() + '\n' + source).encode()).hexdigest()[:24]
     path = os.path.join(_CACHE_DIR, key + '.hsaco')
     if os.path.exists(path):
         with open(path, 'rb') as f:

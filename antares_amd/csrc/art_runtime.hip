@@ -184,6 +184,14 @@ int art_device_props(art_props* out) {
   return 0;
 }
 
+// Of every kernel that art_module_compile makes: packed-FP32 instruction selection is switched off, the first arguments start in registers.
+#define ART_COMPILE_OPTIONS(X)                                                                                                       \
+  X("-O3") X("-std=c++17") X("-Wno-ignored-attributes") X("-Xclang") X("-target-feature") X("-Xclang") X("-packed-fp32-ops") X("-mllvm") \
+  X("-amdgpu-kernarg-preload-count=14")
+#define ART_OPTION_TEXT(option) option " "
+#define ART_OPTION_ITEM(option) , option
+const char* art_compile_options(void) { return ART_COMPILE_OPTIONS(ART_OPTION_TEXT); }
+
 int art_module_compile(const char* hip_source, const char* arch, void** blob, size_t* size) {
   ART_REQUIRE(hip_source && blob && size, "art_module_compile: null argument");
   art::compile_log().clear();
@@ -191,9 +199,7 @@ int art_module_compile(const char* hip_source, const char* arch, void** blob, si
   hiprtcResult r = hiprtcCreateProgram(&prog, hip_source, "autort_kernel.hip", 0, nullptr, nullptr);
   ART_REQUIRE(r == HIPRTC_SUCCESS, "hiprtcCreateProgram: %s", hiprtcGetErrorString(r));
   std::string arch_opt = std::string("--offload-arch=") + ((arch && *arch) ? arch : "gfx950");
-  // Packed-FP32 instruction selection is switched off for every kernel of this library; the first arguments start in registers.
-  const char* opts[] = {arch_opt.c_str(), "-O3", "-std=c++17", "-Wno-ignored-attributes",
-                        "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "-mllvm", "-amdgpu-kernarg-preload-count=14"};
+  const char* opts[] = {arch_opt.c_str() ART_COMPILE_OPTIONS(ART_OPTION_ITEM)};
   r = hiprtcCompileProgram(prog, (int)(sizeof(opts) / sizeof(opts[0])), opts);
   size_t log_size = 0;
   hiprtcGetProgramLogSize(prog, &log_size);

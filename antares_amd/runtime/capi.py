@@ -30,6 +30,7 @@ _SIGNATURES = {
     'art_init': (c_int, [c_int]),
     'art_last_error': (c_char_p, []),
     'art_compile_log': (c_char_p, []),
+    'art_compile_options': (c_char_p, []),
     'art_device_props': (c_int, [POINTER(ArtProps)]),
     'art_module_compile': (c_int, [c_char_p, c_char_p, POINTER(c_void_p), POINTER(c_size_t)]),
     'art_blob_free': (None, [c_void_p]),
@@ -147,8 +148,9 @@ def device_props() -> dict:
     return {f: (getattr(p, f).decode() if isinstance(getattr(p, f), bytes) else getattr(p, f)) for f, _ in p._fields_}
 
 
-# What the library's compiler options change in a code object (part of the cache's key): arguments in registers at the start of a kernel.
-COMPILE_OPTIONS = 'kernarg-preload-14\n'
+def compile_options() -> str:
+    """The options that the library adds to a compilation."""
+    return lib().art_compile_options().decode()
 
 
 def compile_hip(source: str, arch: str = 'gfx950') -> bytes:

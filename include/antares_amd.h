@@ -73,6 +73,9 @@ int art_device_props(art_props* out);
  * which forks `hipcc --genco`; this one compiles in-process. */
 int art_module_compile(const char* hip_source, const char* arch, void** blob, size_t* size);
 void art_blob_free(void* blob);
+/* The compiler options that art_module_compile adds, separated by blanks: with the source and `arch` they make up a code object, so
+ * they belong into the key of a cache of them. */
+const char* art_compile_options(void);
 /* Text of the compiler log of the last art_module_compile on this thread. */
 const char* art_compile_log(void);
 

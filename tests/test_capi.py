@@ -41,6 +41,22 @@ def test_compile_without_gpu_and_error_reporting(lib):
     assert 'error' in lib.lib().art_compile_log().decode()
 
 
+def test_cached_code_objects_are_those_of_the_options_they_were_compiled_with(lib, tmp_path, monkeypatch):
+    """The key of the cache holds the very options that the library compiles with: other options, another code object."""
+    from antares_amd.autort import op
+    options = lib.compile_options().split()
+    assert '-packed-fp32-ops' in options and '-amdgpu-kernarg-preload-count=14' in options and '-O3' in options
+    monkeypatch.setattr(op, '_CACHE_DIR', str(tmp_path))
+    compiled = []
+    monkeypatch.setattr(lib, 'compile_hip', lambda source: compiled.append(source) or source.encode())
+    for text, count in (('a', 1), ('a', 1), ('b', 2)):
+        op.compile_cached(text)
+        assert len(compiled) == count
+    monkeypatch.setattr(lib, 'compile_options', lambda: '-O3 -another')
+    op.compile_cached('a')
+    assert len(compiled) == 3 and len(list(tmp_path.glob('*.hsaco'))) == 3
+
+
 def test_bad_arguments_return_errors(lib):
     l = lib.lib()
     assert l.art_launch(None, 1, 1, 1, 64, 1, 1, 0, None, None, 0) != 0
