@@ -51,7 +51,7 @@ constexpr size_t kScratchOffset = 4 * 1024 * 1024;       // partial sums, tile c
 typedef unsigned int u32x4_t __attribute__((ext_vector_type(4)));
 constexpr unsigned int kBufferFlags = 0x00020000u;       // word 3 of a buffer descriptor: 32-bit data
 
-// 64 lanes x 16 (4) bytes from base + lane offset straight into LDS at lds_dst + 16 (4) * lane.  The instruction takes
+// 64 lanes x 16 bytes from base + lane offset straight into LDS at lds_dst + 16 * lane.  The instruction takes
 // the LDS address from m0, which nothing else here uses (the compiler warns that it does not preserve a reserved register
 // that is named as clobbered; nothing has to be preserved).  The waits are written by hand: the compiler does not see
 // these loads.
@@ -60,10 +60,7 @@ constexpr unsigned int kBufferFlags = 0x00020000u;       // word 3 of a buffer d
 __device__ __forceinline__ void load_lds_x4(const void* base, unsigned int off, unsigned int lds_dst) {
   asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds_dst) : "m0");
 }
-__device__ __forceinline__ void load_lds_x1(const void* base, unsigned int off, unsigned int lds_dst) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" ::"v"(off), "s"(base), "s"(lds_dst) : "m0");
-}
-// The same from base + scalar offset + lane offset, the base in a buffer descriptor (buffer_of); LDS address: a scalar plus a constant.
+// The same, 16 or 4 bytes a lane, from base + scalar offset + lane offset, the base in a buffer descriptor (buffer_of); LDS address: a scalar plus a constant.
 // Nothing but the scalar offset has to move on from one load to the next.
 template <unsigned LDS> __device__ __forceinline__ void buffer_lds_x4(u32x4_t buffer, unsigned int off, unsigned int scalar_off, unsigned int lds) {
   asm volatile("s_add_u32 m0, %2, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %4 offen lds" ::"v"(off), "s"(buffer), "s"(lds), "n"(LDS), "s"(scalar_off) : "m0", "scc");

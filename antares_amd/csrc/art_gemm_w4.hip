@@ -20,7 +20,7 @@
 //     replaced by two (same loop, longer meeting), blocks that start at groups of their own, and branches around the
 //     loads of the last groups;
 //   * everything a group needs - 8 KiB of packed weights, 8 MT KiB of x, 256 B of scales, 64 B of zero points - goes from
-//     global memory straight into LDS (global_load_lds: no registers hold data in flight), into a ring of three slots.
+//     global memory straight into LDS (buffer loads: no registers hold data in flight), into a ring of three slots.
 //     The weights run a group ahead of x, so that the first operands of a group are unpacked in the one before;
 //   * LDS position (row r, chunk p) holds chunk p ^ ((r / 2) & 7) of the weights (rows of 128 bytes) and p ^ (r & 15) of x
 //     (rows of 256 bytes): every 16 lanes of a read touch every bank once;

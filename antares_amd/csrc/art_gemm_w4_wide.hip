@@ -11,7 +11,7 @@
 //     natural order (half a v_perm and half a shift more per pair of weights) instead of a permutation of every x
 //     operand: the loop has 2.1 vector instructions per MFMA at MT = 8 and 4.3 at MT = 4;
 //   * per 64 values of k a block needs 8 KiB of packed weights, 4 MT KiB of x and the group's scales and zero points;
-//     they go from global memory straight into LDS (global_load_lds, no registers in flight), a ring of three slots.
+//     they go from global memory straight into LDS (buffer loads, no registers in flight), a ring of three slots.
 //     The weights run a stage ahead of x, so that the first operands of a stage can be unpacked in the stage before;
 //   * the chunk positions are swizzled so that every 16 lanes of a 16-byte read of x (rows 128 bytes apart), and of a
 //     transposing byte read of the weights, touch every bank once (SQ_LDS_BANK_CONFLICT 0.5 M cycles in a launch of 33 M

@@ -162,7 +162,7 @@ class LlamaInt4Decoder:
             up = {'qweight': gu['qweight'][:, F:].contiguous(), 'scales': gu['scales'][:, F:].contiguous(),
                   'qzeros': gu['qzeros'][:, F // 2:].contiguous()}
             layers.append({'qkv': packed(lw['qkv']), 'gate_up': packed(interleave_gate_up(gate, up)), 'down': packed(lw['down']),
-                           'o': packed(lw['o'])})      # used when the attention runs as one block per head
+                           'o': packed(lw['o'])})      # used when the attention runs as one block per head, and by a prompt's last layer
         self.pw = {'layers': layers, 'lm_head': packed(self.w['lm_head'])}
 
     def _ops(self):
@@ -297,8 +297,10 @@ class LlamaInt4Decoder:
         (`gemm_w4a16_rope_store`), attention is causal over the prompt (`attention_causal_f16`, matrix cores), keys and
         values land in cache rows 0..T-1.  Leaves the step
         state at the last prompt position (self.pos = T - 1, self.x = its hidden state, self.logits = its logits), so
-        `advance()` and the recorded decode step continue from there.  Same operators and roundings as the one-token
-        step, applied to T rows.  With ``graph`` the pass is recorded once per prompt length in a HIP graph (about 230
+        `advance()` and the recorded decode step continue from there.  The operators are those of the one-token step, applied
+        to T rows; the int4 products round a weight to float16 before they multiply.  Over repacked weights the last position alone
+        goes through the last layer behind its keys and values, with the one-token step's operators themselves
+        (`_prefill_last`: decode attention, `gemv_w4p`), which sum quantised values and scale the sums.  With ``graph`` the pass is recorded once per prompt length in a HIP graph (about 230
         launches) and replayed on later calls with the new tokens copied into the recorded input."""
         T = int(tokens.numel())
         if not 4 <= T <= self.cfg.max_seq:
@@ -335,7 +337,7 @@ class LlamaInt4Decoder:
         ops = self._prefill_ops(T)
         f16 = dict(dtype=torch.float16, device=self.dev)
         x = ops['embed'](self.w['embed'], tokens.view(T))
-        hid = torch.empty(T, F, **f16)
+        hid = torch.empty(T, F, **f16) if not self.packed or cfg.n_layers > 1 else None      # a prompt's last layer has rows of its own
         qr = torch.empty(T, H, D, **f16)
         angles = self.autort.ops.rope_angles_f16(self.inv_freq, torch.empty(T, D // 2, 2, dtype=torch.float32, device=self.dev))
 
