@@ -493,29 +493,32 @@ struct Plan {
   int row_tiles, splits;
   int deep;                                         // column tiles of a block of art_gemm_w4_deep.hip, 0: not that kernel
 };
-// What a launch takes, in microseconds.  K-splits: the second launch and the fp32 tiles on top; of more than eight the pass that also turns or
-// gates waits twice (q | k | v of one head, 8 rows, K = 3712: 5.8 us in seven splits, 9.3 in fifteen).
+// What a launch takes, in microseconds.  K-splits: the second launch and the fp32 tiles on top.  A pass that also turns or gates costs a
+// prompt more than it costs alone (q | k | v of 64 rows over 4096 x 12288, in a prompt's trace: one launch 18.8, two splits 16.1 and the pass 5.0; in a loop
+// of its own 18.6 and 17.7), and waits twice for more than eight (8 rows, K = 3712, one head: 5.8 in seven splits, 9.3 in fifteen).
 double splits_estimate(int M, int N, int splits, Tail tail) {
-  return splits > 1 ? 1.8 + (8.0 * splits + 2.0) * M * N / 4.2e6 + (splits > 8 && tail != kPlain ? 2.65 : 0.0) : 0.0;
+  return splits > 1 ? 1.8 + (8.0 * splits + 2.0) * M * N / 4.2e6 + (tail == kPlain ? 0.0 : splits > 8 ? 3.5 : 0.849) : 0.0;
 }
 // Where K-splits meet in a pass of their own, a norm is part of that pass, up to 256 rows: beyond them nothing is
 // gained (8 layers of the same pass: 1384 -> 1368 us at 256 tokens, 1861 and 1854 at 300, 2178 and 2183 at 500).
 bool norm_fits(int M, int N) { return M <= 256 && N % 8 == 0 && N <= 8 * kNormThreads * kNormTurns; }
-// Else it is a launch of its own.
-double norm_estimate(int M, int N, int splits) { return splits == 1 ? 2.4 + 2.0e-6 * M * N : 0.0; }
+// Else it is a launch of its own.  (Of more than eight splits the pass waits twice.)
+double norm_estimate(int M, int N, int splits) { return splits == 1 ? 3.046 + 2.178e-6 * M * N : splits > 8 ? 1.0 : 0.0; }
 // A fixed part, one or two co-resident blocks' time per group and round (one's: more with more of the compute units at work; either: more where
-// several blocks of rows unpack the same weights), the ramp and the meeting of the k halves again for every further round of blocks of 128
-// columns (4 rows over 4096 x 12288: 13.3 us with 480 blocks, i.e. 5 K-splits in one round, 14.6 with 768).  Constants of 128 columns x 128 rows and
-// of 256 columns from all forms over 6200 sizes of 4 to 1003 rows on MI355X, a quarter with weights that stay in the last-level cache; the others, and
-// those of deep_estimate, from 4065 sizes of 4 to 512 rows, 512 x 512 to 8192 x 24576, each with weights from HBM, as a model's are, and from the
-// cache, the former counting 70 %: the pick is 0.9 and 1.2 % slower than the fastest form.  Without the terms for blocks of rows,
-// rows whole KiB apart and halves it was 2.1 and 1.7 % slower, and lost 20 to 40 % at square matrices of 4096 and more (weights from HBM, us: 8 rows over
-// 4096 x 4096 10.1, now 7.8; 5120 x 5120 14.0, 9.2; 64 rows over 11008 x 4096 18.5, 15.9; 256 rows 34.4, 32.1; 64 rows over 4096 x 12288 18.6, 17.7).
-// Where a product from the cache would rather have the narrow blocks it loses (8 rows over 5120 x 5120 6.9, now 7.9).
+// several blocks of rows unpack the same weights; two's: more where rows are whole KiB apart, and for the halves of gate | up), the ramp and
+// the meeting of the k halves again for every further round of blocks of 128 columns (4 rows over 4096 x 12288: 13.3 us with 480 blocks, i.e. 5 K-splits
+// in one round, 14.6 with 768).  Constants of 128 columns x 128 rows and of 256 columns are from all forms over 6200 sizes of 4 to 1003 rows on MI355X, a
+// quarter with weights that stay in the last-level cache.  The others and deep_estimate's are from 2678 sizes of 4 to 512 rows, each with
+// weights from HBM and from the cache, the former counting 70 %, and from 3469 prompts of 4 to 620 tokens (models of 8 to 64 heads): for each product of a
+// layer, what another form does to the layer's time.  The pick is 0.9 % (HBM) and 1.4 % (cache) slower than the fastest
+// form, a layer of a prompt 0.8 %.  Before there were terms for blocks of rows, rows whole KiB apart and halves: 2.1, 1.6 and 1.4 %, and 20 to 40 % at some
+// (weights from HBM, us: 8 rows over 4096 x 4096 10.1, now 7.8; 5120 x 5120 14.0, 9.2; 64 rows over 11008 x 4096 18.5, 15.9; 256 rows 34.4, 32.1).
+// Products from the cache would rather keep the narrow blocks there (8 rows over 5120 x 5120 6.9, now 7.9).
 double estimate(int M, int K, int N, const Plan& p, Tail tail, int compute_units) {
-  struct Cost { double fixed, one, two; int per_cu; double busy, rows; };
-  const Cost c = p.wide ? (p.row_tiles == 8 ? Cost{8.5, 2.16, 1.94, 1, 0, 0} : Cost{5.2, 1.2, 2.3, 2, 0, 0})
-                        : p.row_tiles == 4 ? Cost{4.8, 0.52, 0.82, 1, 0, 0} : p.row_tiles == 2 ? Cost{4.373, 0.422, 0.924, 2, 0.073, 0.037} : Cost{3.83, 0.401, 0.863, 2, 0.001, 0.044};
+  struct Cost { double fixed, one, two; int per_cu; double busy, rows, whole_kib, halves; };
+  const Cost c = p.wide ? (p.row_tiles == 8 ? Cost{8.5, 2.16, 1.94, 1, 0, 0, 0, 0} : Cost{5.2, 1.2, 2.3, 2, 0, 0, 0, 0})
+                 : p.row_tiles == 4 ? Cost{4.8, 0.52, 0.82, 1, 0, 0, 0, 0}
+                 : p.row_tiles == 2 ? Cost{4.419, 0.372, 0.915, 2, 0.1, 0.065, 0.005, 0.04} : Cost{3.697, 0.388, 0.831, 2, 0, 0.053, 0.011, 0};
   const int groups = (K / GK + p.splits - 1) / p.splits, m_blocks = (M + 32 * p.row_tiles - 1) / (32 * p.row_tiles);
   const int blocks = tile_count(N, false, p.wide ? 256 : BN) * m_blocks * p.splits, round = c.per_cu * compute_units, rest = blocks % round;
   const double busy = blocks < compute_units ? (double)blocks / compute_units : 1.0;
@@ -525,7 +528,8 @@ double estimate(int M, int K, int N, const Plan& p, Tail tail, int compute_units
     one = c.per_cu == 2 || blocks > round ? 1.0 : 1.0 - (double)rest / compute_units;
     two += 1.0 - one;
   }
-  const double per_group = (c.one + c.busy * busy) * one + c.two * two + c.rows * busy * (1.0 - 1.0 / m_blocks) * (one + two);
+  const double waits = ((N % 1024 == 0 ? c.whole_kib : 0.0) + (tail == kSwiglu ? c.halves : 0.0)) / m_blocks;       // (blocks of rows share weights)
+  const double per_group = (c.one + c.busy * busy) * one + (c.two + waits) * two + c.rows * busy * (1.0 - 1.0 / m_blocks) * (one + two);
   const double again = p.wide ? 0.0 : 0.73 * ((blocks - 1) / round);
   return c.fixed + again + groups * per_group + splits_estimate(M, N, p.splits, tail);
 }
@@ -535,9 +539,9 @@ double estimate(int M, int K, int N, const Plan& p, Tail tail, int compute_units
 // cache 6.8) and for pieces of 16 columns of two halves (gate | up).
 double deep_estimate(int M, int K, int N, const Plan& p, Tail tail, int compute_units) {
   struct Cost { double fixed, group, busy, further, again, whole_kib, halves; };
-  const Cost c = p.deep == 2 ? (M <= 16 ? Cost{3.569, 0.172, 0.047, 0.270, 0.408, 0.030, 0.014} : Cost{3.314, 0.215, 0.057, 0.224, 1.622, 0.029, 0.037})
-                 : p.row_tiles == 2 ? Cost{3.187, 0.213, 0.113, 0.229, 1.483, 0.021, 0.026}
-                 : M <= 16 ? Cost{3.035, 0.104, 0.059, 0.159, 0.370, 0.034, 0.024} : Cost{3.073, 0.144, 0.051, 0.179, 1.320, 0.027, 0.028};
+  const Cost c = p.deep == 2 ? (M <= 16 ? Cost{3.23, 0.178, 0.04, 0.257, 0.404, 0.036, 0.014} : Cost{3.21, 0.213, 0.064, 0.205, 1.88, 0.017, 0.035})
+                 : p.row_tiles == 2 ? Cost{3.449, 0.2, 0.101, 0.219, 1.577, 0.02, 0.028}
+                 : M <= 16 ? Cost{2.737, 0.102, 0.069, 0.148, 0.387, 0.04, 0.024} : Cost{2.943, 0.147, 0.051, 0.162, 1.471, 0.024, 0.028};
   const int groups = (K / GK + p.splits - 1) / p.splits, m_blocks = (M + 32 * p.row_tiles - 1) / (32 * p.row_tiles);
   const int blocks = deep_tiles(N, tail, p.deep) * m_blocks * p.splits, more = (blocks - 1) / compute_units;
   const double busy = blocks < compute_units ? (double)blocks / compute_units : 1.0;
