@@ -728,7 +728,7 @@ def test_one_row_in_blocks_of_256_rows_and_two_splits_of_k(autort, N):
 @pytest.mark.parametrize('M', [4, 16, 17, 32, 33, 64, 65, 131, 250])
 @pytest.mark.parametrize('K,N', [(128, 16), (1152, 48), (640, 208), (4224, 96), (1024, 1056), (2176, 9008)])
 def test_int4_products_of_a_few_rows_over_blocks_of_32_and_64_columns(autort, M, K, N):
-    """Narrow or shallow products are taken by blocks of 32 or 64 columns whose wavefronts divide K among them:
+    """Narrow or shallow products as the library chooses, most of them blocks of 32 or 64 columns whose wavefronts divide K among them:
     fewer groups than wavefronts, a last block half or a quarter inside the matrix, one and several blocks of rows and their edges.  Against float64
     sums of the same float16 weights: the result's rounding (2^-11) and float32 sums of K terms (K 2^-24 of the sum of absolute values)."""
     note(f'few rows M={M} K={K} N={N}')
