@@ -494,21 +494,22 @@ def _conv2d_handler(st, axes, window):
                  window['h'][0], window['w'][0])
         if max(abs(v) for v in shape) >= 1 << 31:
             return False
-        form = lib.art_conv2d_choose(*shape)
+        form = lib.art_conv2d_direct(*shape) or lib.art_conv2d_choose(*shape)
         if not form:
             return False
 
-        def scratch(forms):
-            return scratch_memory(max(lib.art_conv2d_scratch_bytes(*shape, v) for v in forms), torch.uint8, x.device)
+        def scratch(forms):                       # 0: none is needed
+            count = max(lib.art_conv2d_scratch_bytes(*shape, v) for v in forms)
+            return scratch_memory(count, torch.uint8, x.device) if count else 0
 
         def run(value, t):
-            capi.check(lib.art_conv2d(*(c_void_p(v.data_ptr()) for v in t), *shape, int(value), c_void_p(torch.cuda.current_stream().cuda_stream)))
+            capi.check(lib.art_conv2d(*(c_void_p(v.data_ptr() if isinstance(v, torch.Tensor) else v) for v in t), *shape, int(value), c_void_p(torch.cuda.current_stream().cuda_stream)))
         # the launch parameter: the shape of a block
         key = 'conv2d.form|' + ','.join(str(v) for v in shape)
         saved = op.tuned.get(key)
         trials = op.config.get('tune')
         if saved is None and isinstance(trials, int) and trials > 0 and not torch.cuda.is_current_stream_capturing():
-            others = (1, 2, 3, 4, 5, 6) + tuple(k + 256 * s for k in (4, 5, 6, 7) for s in (2, 3, 4, 6, 8))
+            others = (1, 2, 3, 4, 5, 6, 8, 9, 10) + tuple(k + 256 * s for k in (4, 5, 6, 7) for s in (2, 3, 4, 6, 8))
             forms = [form] + [v for v in others if v != form and lib.art_conv2d_exact_enough(*shape, v)]
             forms = forms[:trials]
             room = scratch(forms)

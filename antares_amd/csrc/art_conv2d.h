@@ -89,6 +89,11 @@ size_t staged_bytes(const Geometry& g, int slices);
 size_t staged_lds(const Geometry& g);
 int run_staged(const void* x, const void* w, void* packed, void* y, const Geometry& g, int f16, int form, int slices, hipStream_t stream);
 
+// Forms 8 to 10 (art_conv2d_direct.hip): blocks of 16 features x 16, 32 or 64 points over all channels, in one launch, without copies.
+bool direct_fits(const Geometry& g, int f16, int form);
+double direct_time(const Geometry& g, int f16, int form);
+int run_direct(const void* x, const void* w, void* y, const Geometry& g, int f16, int form, hipStream_t stream);
+
 }  // namespace conv
 
 // y[i] = sum over slices of partial[slice * count + i], in order and in float64 (art_gemm_tile.hip).

@@ -238,10 +238,11 @@ int span_of(const Geometry& g, int columns) {
 size_t lds_of(int span) { return (size_t)span * (2 * kPitchBytes + 4); }
 
 // Forms: 1 = 64 features x 64 points per block, 2 = 64 x 128, 3 = 128 x 128; 4, 5, 6 the same over the staged image, 7 = 64 x 64
-// there with short sums (float32), plus 256 x slices of the channels (0: one).
+// there with short sums (float32), plus 256 x slices of the channels (0: one); 8, 9, 10 = 16 features x 16, 32, 64 points (art_conv2d_direct.hip).
+bool direct(int form) { return (form & 255) > 7; }
 int shape_of(int form) { return (form & 255) % 3; }
-int features_of(int form) { return shape_of(form) == 0 ? 128 : 64; }
-int points_of(int form) { return shape_of(form) == 1 ? 64 : 128; }
+int features_of(int form) { return direct(form) ? 16 : shape_of(form) == 0 ? 128 : 64; }
+int points_of(int form) { return direct(form) ? 16 << ((form & 255) - 8) : shape_of(form) == 1 ? 64 : 128; }
 int slices_of(int form) { return form >> 8 ? form >> 8 : 1; }
 
 bool geometry(Geometry& g, int f16, int N, int C, int H, int W, int F, int HO, int WO, int ph, int pw) {
@@ -263,8 +264,9 @@ bool geometry(Geometry& g, int f16, int N, int C, int H, int W, int F, int HO, i
 
 bool fits(Geometry g, int f16, int form) {
   const int kind = form & 255;
-  if (form < 1 || kind < 1 || kind > (f16 ? 6 : 7)) return false;
+  if (form < 1 || kind < 1 || (kind > (f16 ? 6 : 7) && !direct(form))) return false;
   g.span = span_of(g, points_of(form));
+  if (direct(form)) return art::conv::direct_fits(g, f16, form);
   if (kind <= 3) return form == kind && lds_of(g.span) <= (f16 && form == 1 ? kWideLds : kMaxLds);
   return slices_of(form) <= 64 && slices_of(form) <= g.chunks && staged_lds(g) <= 160 * 1024;
 }
@@ -326,6 +328,7 @@ bool on_vector_units(const Geometry& g) { return g.F < 32 || g.columns < 32 || 9
 // the generic kernels need 9 C / 16 (5 to 31 channels 1.02 to 1.22 times their error, the blocks of 64 x 64 0.66 to 1.01
 // times; with four channels both are above it).
 bool exact_enough(const Geometry& g, int f16, int form) {
+  if (direct(form)) return true;
   if (!on_vector_units(g)) return !f16 || (g.C > 4 && shape_of(form) == 1) || g.C >= 32 || g.C % 8 == 0;
   if (9 * g.C < 64) return true;
   if (!f16) return (form & 255) == 7;
@@ -387,7 +390,7 @@ double generic_time(const Geometry& g, int f16) {
 //  * A copy of more than 128 MiB for one image is not made: the image is gathered.  Beside the packed filter a call takes 192 MiB at the
 //    most, 128 for the copy and 64 for slices (4 kUnits blocks of 128 x 128).
 // `gathered`: the best of the forms that need no more than the packed filter, for callers that have no more.
-int choose(const Geometry& g, int f16, bool gathered) {
+int choose(const Geometry& g, int f16, bool gathered, double* time = nullptr) {
   const bool image_like = (g.C == 2 || g.C == 3) && g.F >= (f16 ? 32 : 64) && (long long)g.columns * g.F >= (f16 ? 1 << 19 : 1 << 20);
   if (g.C < 8 && !image_like && !gathered) return 0;
   const bool staged = !gathered && (size_t)g.chunks * (g.HO + 2) * (g.WO + 2) * kChunkBytes <= kMostCopy;
@@ -405,7 +408,9 @@ int choose(const Geometry& g, int f16, bool gathered) {
     for (int slices : {1, 2, 3, 4, 5, 6, 8, 12})
       if (form > 3 && staged && slices <= g.chunks && (slices == 1 || slices * blocks_of(g, form) <= 4 * kUnits)) consider(form + (slices > 1 ? 256 * slices : 0), staged_time(g, f16, form, slices));
   }
-  return best && (gathered || image_like || t_outside < (vector_units ? 1.0 : 1.05) * generic_time(g, f16)) ? best : 0;
+  if (!best || !(gathered || image_like || t_outside < (vector_units ? 1.0 : 1.05) * generic_time(g, f16))) return 0;
+  if (time) *time = t_best + outside_time(g, f16, best);
+  return best;
 }
 
 template <typename T, int MT, int NT>
@@ -448,6 +453,31 @@ extern "C" int art_conv2d_choose(int f16, int N, int C, int H, int W, int F, int
   return geometry(g, f16, N, C, H, W, F, HO, WO, ph, pw) ? choose(g, f16, false) : 0;
 }
 
+// The form of art_conv2d_direct.hip for these sizes, or 0 where its time is estimated above that of what `choose` takes, or of the generic
+// kernels where that takes none.
+//  * Over 900 sizes (a third of them outside of 16 to 256 channels and features and 7 to 56 squared) what is taken then is 1.42 to 1.49 (float32) and 1.18 times
+//    as fast as before in the mean, on 6 of them more than 5 % slower (up to 1.28 times).
+//  * Not where the generic kernels have few terms or most taps are outside of the image (their estimate is twice their time there): fewer than 8
+//    channels (3 x 4 x 6 x 6 -> 108 2.9 us, 4.2 here), images of fewer than four points (13 x 8 x 1 x 1 -> 78 2.4 and 4.4).
+//  * Not for more than 100 million products on the matrix instructions' ground: the other forms' larger blocks catch up there, and half
+//    of all wrong picks were beyond it (9 x 48 x 34 x 34 -> 80 22.3 us, 27.6 here), for 1.5 % of the gain.
+extern "C" int art_conv2d_direct(int f16, int N, int C, int H, int W, int F, int HO, int WO, int ph, int pw) {
+  Geometry g;
+  if (!geometry(g, f16, N, C, H, W, F, HO, WO, ph, pw) || C < 8 || (long long)HO * WO < 4) return 0;
+  if (9.0 * g.columns * F * C > 1e8 && !on_vector_units(g)) return 0;
+  double least = 1e30;
+  int best = 0;
+  for (int form = 8; form <= 10; ++form) {
+    if (!fits(g, f16, form)) continue;
+    const double t = art::conv::direct_time(g, f16, form);
+    if (t < least) { least = t; best = form; }
+  }
+  if (!best) return 0;
+  double other = 0.0;
+  if (!choose(g, f16, false, &other)) other = generic_time(g, f16);
+  return least < other ? best : 0;
+}
+
 extern "C" size_t art_conv2d_packed_bytes(int f16, int C, int F) {
   const size_t chunks = ((size_t)C + (f16 ? 31 : 15)) / (f16 ? 32 : 16);
   return chunks * kTaps * (((size_t)F + 127) / 128) * 4 * 2048;
@@ -456,16 +486,16 @@ extern "C" size_t art_conv2d_packed_bytes(int f16, int C, int F) {
 extern "C" size_t art_conv2d_scratch_bytes(int f16, int N, int C, int H, int W, int F, int HO, int WO, int ph, int pw, int form) {
   Geometry g;
   if (!geometry(g, f16, N, C, H, W, F, HO, WO, ph, pw) || !fits(g, f16, form)) return 0;
-  return (form & 255) <= 3 ? art_conv2d_packed_bytes(f16, C, F) : staged_bytes(g, slices_of(form));
+  return direct(form) ? 0 : (form & 255) <= 3 ? art_conv2d_packed_bytes(f16, C, F) : staged_bytes(g, slices_of(form));
 }
 
 extern "C" int art_conv2d(const void* x_dev, const void* w_dev, void* packed_dev, void* y_dev, int f16, int N, int C, int H, int W, int F, int HO,
                           int WO, int ph, int pw, int form, void* stream) {
   Geometry g;
   ART_REQUIRE(geometry(g, f16, N, C, H, W, F, HO, WO, ph, pw) && fits(g, f16, form), "art_conv2d: sizes the kernel does not take (form %d)", form);
-  ART_REQUIRE(x_dev && w_dev && packed_dev && y_dev, "art_conv2d: null pointer");
+  ART_REQUIRE(x_dev && w_dev && (packed_dev || direct(form)) && y_dev, "art_conv2d: null pointer");
   const uintptr_t size = f16 ? 2 : 4;
-  ART_REQUIRE((uintptr_t)x_dev % size == 0 && (uintptr_t)w_dev % size == 0 && (uintptr_t)packed_dev % 16 == 0 && (uintptr_t)y_dev % 4 == 0,
+  ART_REQUIRE((uintptr_t)x_dev % size == 0 && (uintptr_t)w_dev % size == 0 && (direct(form) || (uintptr_t)packed_dev % 16 == 0) && (uintptr_t)y_dev % 4 == 0,
               "art_conv2d: misaligned tensor");
   ART_REQUIRE(!art::overlaps(y_dev, (size_t)N * F * HO * WO * 4, x_dev, (size_t)N * C * H * W * size) &&
                   !art::overlaps(y_dev, (size_t)N * F * HO * WO * 4, w_dev, (size_t)F * C * 9 * size),
@@ -474,6 +504,7 @@ extern "C" int art_conv2d(const void* x_dev, const void* w_dev, void* packed_dev
   g.row_tiles = g.row_blocks * (features_of(form) / 32);
   g.blocks_across = make_div((unsigned)g.row_blocks);
   g.span = span_of(g, points_of(form));
+  if (direct(form)) return art::conv::run_direct(x_dev, w_dev, y_dev, g, f16, form, (hipStream_t)stream);
   if ((form & 255) > 3)
     return run_staged(x_dev, w_dev, packed_dev, y_dev, g, f16, form & 255, slices_of(form), (hipStream_t)stream);
   return f16 ? run<_Float16>(x_dev, w_dev, packed_dev, y_dev, g, form, (hipStream_t)stream)

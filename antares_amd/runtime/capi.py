@@ -96,6 +96,7 @@ _SIGNATURES = {
     'art_gemm_f32_ex': (c_int, [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p]),
     'art_conv2d_form': (c_int, [c_int] * 11),
     'art_conv2d_choose': (c_int, [c_int] * 10),
+    'art_conv2d_direct': (c_int, [c_int] * 10),
     'art_conv2d_exact_enough': (c_int, [c_int] * 11),
     'art_conv2d_packed_bytes': (c_size_t, [c_int] * 3),
     'art_conv2d_scratch_bytes': (c_size_t, [c_int] * 11),

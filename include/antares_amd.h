@@ -306,8 +306,11 @@ int art_gemm_f32_ex(const void* a_dev, const void* b_dev, void* c_dev, int batch
  * channels (or plus 0: one), with a packed_dev of art_conv2d_scratch_bytes for that form.  art_conv2d_choose gives the library's
  * choice among all of them (128 MiB for the copy at the most: larger batches go in passes), art_conv2d_form with form = 0 the best of
  * the first three for callers that have no room for a copy; any other form comes back if it takes these sizes; 0 where these sizes
- * are not taken.  art_conv2d_exact_enough: 1 if the form's sums are no longer than those of
+ * are not taken.  Forms 8, 9 and 10 = 16 features x 16, 32 and 64 points run in one launch and need no memory (packed_dev may be null; C % 8 == 0
+ * in float16, C % 4 == 0 in float32): art_conv2d_direct gives the one that is faster than art_conv2d_choose's, or 0.
+ * art_conv2d_exact_enough: 1 if the form's sums are no longer than those of
  * the generic kernels at these sizes (the choice always is). */
+int art_conv2d_direct(int f16, int N, int C, int H, int W, int F, int HO, int WO, int ph, int pw);
 int art_conv2d_form(int f16, int N, int C, int H, int W, int F, int HO, int WO, int ph, int pw, int form);
 int art_conv2d_choose(int f16, int N, int C, int H, int W, int F, int HO, int WO, int ph, int pw);
 int art_conv2d_exact_enough(int f16, int N, int C, int H, int W, int F, int HO, int WO, int ph, int pw, int form);

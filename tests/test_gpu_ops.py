@@ -1386,6 +1386,67 @@ def test_staged_convolution_blocks_match_float64(autort, dtype, case):
             assert bool(((y.cpu().double() - want).abs() <= bound + 1e-30).all()), (kind, slices)
 
 
+@pytest.mark.parametrize('dtype', ['float16', 'float32'])
+@pytest.mark.parametrize('case', [
+    (2, 16, (9, 9), 33, (1, 1), (9, 9)),             # a block spans several images, one more feature than two tiles
+    (3, 8, (13, 17), 16, (1, 1), (13, 17)),          # one unit of channels (float16: half of one)
+    (1, 72, (40, 3), 130, (1, 1), (40, 3)),          # rows of three points
+    (5, 24, (8, 8), 48, (0, 0), (6, 6)),             # no padding
+    (2, 24, (12, 10), 40, (2, 0), (14, 7)),          # padded on one axis by two, results short of the other's end
+    (1, 16, (1, 1), 32, (1, 1), (1, 1)),             # one point
+    (4, 8, (30, 31), 20, (-1, 1), (27, 31)),         # taps that start inside, blocks that stay inside an image
+    (3, 264, (6, 30), 15, (1, 1), (6, 30)),          # wavefronts in several rounds, four points per lane
+    (1, 408, (24, 40), 17, (1, 1), (24, 40)),        # ... and more of them than the registers allow at once
+])
+@pytest.mark.parametrize('offset', [0, 1])           # values by which the filter misses a 16-byte boundary
+def test_one_launch_convolutions_match_float64(autort, dtype, case, offset):
+    """Sums in float64 of float32 sums of 8 products three times over (float16: of 48 products): a chain of 6 (48) roundings of 2^-24 and
+    the one of the result."""
+    from ctypes import c_void_p
+    from antares_amd.runtime import capi
+    N, C, (H, W), F, (ph, pw), (HO, WO) = case
+    note(f'one-launch convolution {dtype} {case} offset {offset}')
+    g = torch.Generator().manual_seed(N * 1000 + C + W)
+    x, w = torch.randn(N, C, H, W, generator=g).to(getattr(torch, dtype)), torch.randn(F, C, 3, 3, generator=g).to(getattr(torch, dtype))
+    f16 = int(dtype == 'float16')
+    shape = (f16, N, C, H, W, F, HO, WO, ph, pw)
+    lib, dev = capi.lib(), autort.device()
+    xd, memory = x.to(dev), torch.empty(w.numel() + 1, dtype=w.dtype, device=dev)
+    wd = memory[offset:offset + w.numel()].view(w.shape).copy_(w)
+    pad = max(ph, pw, 0) + 2
+
+    def reference(a, b):
+        return torch.nn.functional.conv2d(torch.nn.functional.pad(a, (pad, pad + 2, pad, pad + 2)), b)[:, :, pad - ph:pad - ph + HO, pad - pw:pad - pw + WO]
+    want, size = reference(x.double(), w.double()), reference(x.double().abs(), w.double().abs())
+    for form in (8, 9, 10):
+        assert lib.art_conv2d_form(*shape, form) == form and lib.art_conv2d_scratch_bytes(*shape, form) == 0
+        y = torch.full((N, F, HO, WO), 7.0, device=dev)
+        capi.check(lib.art_conv2d(c_void_p(xd.data_ptr()), c_void_p(wd.data_ptr()), None, c_void_p(y.data_ptr()), *shape, form,
+                                  c_void_p(torch.cuda.current_stream().cuda_stream)))
+        assert bool(((y.cpu().double() - want).abs() <= (49 if f16 else 7) * 2.0 ** -24 * size + 1e-30).all()), form
+
+
+@pytest.mark.parametrize('dtype,n,c,f,hw', [('float32', 4, 40, 104, 8), ('float32', 1, 24, 24, 39), ('float32', 62, 8, 7, 22), ('float32', 16, 48, 16, 20), ('float16', 1, 104, 176, 9),
+                                            ('float16', 3, 56, 232, 7)])
+def test_one_launch_convolutions_are_no_further_from_float64_than_those_with_copies(autort, dtype, n, c, f, hw):
+    from ctypes import c_void_p
+    from antares_amd.runtime import capi
+    note(f'one-launch convolution against copies {dtype} {n}x{c}x{hw}x{hw} -> {f}')
+    lib, dev, f16 = capi.lib(), autort.device(), int(dtype == 'float16')
+    shape = (f16, n, c, hw, hw, f, hw, hw, 1, 1)
+    forms = [lib.art_conv2d_direct(*shape), lib.art_conv2d_choose(*shape)]
+    assert forms[0] >= 8 and 0 < forms[1] & 255 < 8
+    g = torch.Generator().manual_seed(c)
+    x, w = torch.randn(n, c, hw, hw, generator=g).to(getattr(torch, dtype)), torch.randn(f, c, 3, 3, generator=g).to(getattr(torch, dtype))
+    want = torch.nn.functional.conv2d(x.double(), w.double(), padding=1)
+    xd, wd, off = x.to(dev), w.to(dev), []
+    for form in forms:
+        y, scratch = torch.empty(n, f, hw, hw, device=dev), torch.empty(lib.art_conv2d_scratch_bytes(*shape, form) + 16, dtype=torch.uint8, device=dev)
+        capi.check(lib.art_conv2d(*(c_void_p(t.data_ptr()) for t in (xd, wd, scratch, y)), *shape, form, c_void_p(torch.cuda.current_stream().cuda_stream)))
+        off.append(float((y.cpu().double() - want).norm() / want.norm()))
+    assert off[0] <= 1.02 * off[1], off          # (2 %: what single inputs scatter)
+
+
 @pytest.mark.parametrize('dtype,n,c,f,hw', [('float16', 1, 216, 48, 35), ('float32', 2, 72, 56, 20), ('float32', 9, 216, 64, 17), ('float32', 12, 24, 24, 46),
                                             ('float16', 6, 88, 40, 8), ('float16', 4, 48, 16, 20)])
 def test_staged_convolutions_are_no_further_from_float64_than_the_generic_kernels(autort, dtype, n, c, f, hw):

@@ -162,6 +162,21 @@ def test_convolutions_go_to_the_kernel_that_was_measured_to_be_faster(f16, n, c,
     assert bool(capi.lib().art_conv2d_choose(f16, n, c, hw, hw, f, hw, hw, 1, 1)) == (here < generic)
 
 
+@pytest.mark.parametrize('f16,n,c,f,hw,before,direct', [
+    (0, 4, 40, 104, 8, 12.9, 4.6), (0, 2, 232, 24, 52, 35.8, 20.9), (0, 1, 24, 32, 15, 7.6, 4.2), (1, 1, 104, 176, 9, 9.4, 5.4), (1, 32, 128, 128, 28, 18.4, 60),
+    (0, 11, 176, 104, 34, 63, 92), (1, 26, 120, 32, 37, 19, 36)])
+def test_convolutions_in_one_launch_where_that_was_measured_to_be_faster(f16, n, c, f, hw, before, direct):
+    """Few products; times in us on an MI355X."""
+    assert bool(capi.lib().art_conv2d_direct(f16, n, c, hw, hw, f, hw, hw, 1, 1)) == (direct < before)
+
+
+@pytest.mark.parametrize('f16,n,c,hw,forms', [(1, 2, 8, 9, [8, 9, 10]), (1, 2, 12, 9, []), (0, 2, 12, 9, [8, 9, 10]), (0, 2, 6, 9, []), (0, 2, 8, 100, [8, 9]), (0, 2, 8, 110, [8]),
+                                              (0, 2, 8, 120, []), (0, 1, 8, 15, [8, 9, 10])])
+def test_convolutions_in_one_launch_take_whole_pieces_of_the_filter_and_short_runs(f16, n, c, hw, forms):
+    """A feature's taps in 16-byte pieces; runs of four points per lane at the most: a block's own, two rows and a bit."""
+    assert [v for v in (8, 9, 10) if capi.lib().art_conv2d_form(f16, n, c, hw, hw, 32, hw, hw, 1, 1, v)] == forms
+
+
 @pytest.mark.parametrize('f16,n,c,h,w,f', [(1, 64, 512, 128, 128, 512), (0, 64, 64, 100, 100, 17), (1, 256, 64, 112, 112, 64), (0, 32, 256, 56, 56, 256),
                                            (1, 2, 2048, 14, 14, 2048), (0, 1, 40, 12000, 60, 48), (0, 9, 216, 17, 17, 64)])
 def test_convolutions_take_a_bounded_copy_of_the_image(f16, n, c, h, w, f):
