@@ -11,22 +11,28 @@
 //   * the output points of a block (64 or 128 in a row of n, ho, wo) need one CONTIGUOUS run of points of the image
 //     padded to HO + 2 rows of WO + 2: the run is staged in LDS once per 64 bytes of channels (32 float16 or
 //     16 float32), as [point][channel], and a tap is a constant number of points added to a lane's LDS address.  Global
-//     reads run along the points (a wavefront reads 64 of them from one channel), 16-byte LDS writes put a lane's 8 or 4
-//     channels side by side; 80 bytes from point to point keep reads and writes on distinct banks;
-//   * the offset of each staged point (or "outside") is worked out once per block;
+//     reads run along the points, two of them per lane (a wavefront reads 128 from one channel; rows of the padded image are of an even
+//     number, so that both are in one row): what bounds a chunk beside its products is the number of these loads and of the lines
+//     that each touches.  16-byte LDS writes put a lane's 8 or 4 channels side by side; 80 bytes from point to point keep reads
+//     and writes on distinct banks.  Against a point per load, padding read from the first point of the image, and all loads
+//     with the first three taps (one card, us): float16 32 x 128 x 28 x 28 -> 128 19.3 -> 17.7, 32 x 256 x 14 x 14 -> 256 28.1 -> 22.9, 16 x 256 x 28 x 28 -> 256
+//     31.5 -> 27.4, 26 x 120 x 37 x 37 -> 32 18.6 -> 16.7; float32 32 x 128 x 28 x 28 -> 128 79.7 -> 77.5;
+//   * the offset of each pair of points, and which of them are inside, is worked out once per block;
 //   * the filter is packed first, by a launch of its own, in the order in which wavefronts feed it to the matrix
 //     instructions: [64 bytes of channels][tap][32 features][half][lane] with 16 bytes per lane, so that a wavefront's
 //     operand is one contiguous kilobyte that comes from L2 straight into registers, a tap ahead of its use;
-//   * the next 64 bytes of channels travel to registers while these are multiplied, two LDS buffers, one LDS-only barrier
+//   * the next 64 bytes of channels travel to registers while these are multiplied, a few loads with every tap, two LDS buffers, one LDS-only barrier
 //     per 64 bytes of channels (18 to 72 matrix instructions per wavefront and barrier for a 3 x 3 filter, not 2 to 8);
 //   * a last chunk of which only the lower half exists is multiplied without the upper half (64-feature blocks): float32
 //     20 x 24 -> 64, 20 x 20 12.0 -> 10.5 us (generic 11.4), float16 19 x 19 of 16 channels 8.8 -> 7.3 (7.7 to 8.4);
 //   * 2 x 2 wavefronts of MT x NT tiles of 32 features x 32 points; blocks of one run of points are neighbours on one XCD.
 // Measured, padding 1, both launches, against the generic lowering (a padded copy, then a gathering product): float16
-// 32 x 128 x 28 x 28 -> 128 40.2 -> 18.4 us, 24 x 200 x 33 x 33 -> 48 89 -> 23 us, 2 x 160 x 18 x 18 -> 64 57 -> 14 us;
+// 32 x 128 x 28 x 28 -> 128 40.2 -> 17.3 us, 24 x 200 x 33 x 33 -> 48 89 -> 23 us, 2 x 160 x 18 x 18 -> 64 57 -> 14 us;
 // float32 32 x 128 x 28 x 28 -> 128 113 -> 81 us (the matrix instructions alone take 47), 23 x 128 x 30 x 30 -> 176 119 -> 86.
-// The first of these spends 7 us of the matrix cores' time in 18.6 us: one block per compute unit and only 4 chunks, so the
-// first image fetch, the waits between chunks and the stores of 12.8 MB stay in sight; packing the filter takes 2.3 us.
+// The first of these (clocks of a block, 27500 in all at 2.1 GHz; its products alone are 9200): 1150 for the places, 3700 until the first
+// image is in LDS, three chunks of 5150 and the last of 3400 (2600 without the filter's loads, which half fill the load path), 2900 for
+// the stores of 12.8 MB; packing the filter takes 2.3 us.  Without effect: the filter nine taps ahead, and blocks of four wavefronts
+// along the features, which load the filter once and read each point four times from LDS.
 // Today it is taken for large images with little to multiply (`choose`); art_conv2d_staged.hip stages the image first.
 #include <type_traits>
 
@@ -37,7 +43,7 @@ namespace {
 using namespace art::conv;
 
 constexpr int kPitchBytes = kChunkBytes + 16;   // from one point to the next in LDS
-constexpr unsigned kOutside = 0xffffffffu;
+constexpr unsigned kFirst = 1u, kSecond = 0x80000000u;         // flags beside an offset into x: below 2^31 and even
 constexpr size_t kMaxLds = 64 * 1024, kWideLds = 160 * 1024;     // with more than the first a compute unit holds one block
 
 // Filter [F][C][taps] -> [chunk][tap][32 features][half][lane][16 bytes], zeros past F and C.  A thread gathers the 16
@@ -59,30 +65,39 @@ __global__ __launch_bounds__(kThreads) void conv2d_pack_kernel(const T* __restri
   reinterpret_cast<typename Elem<T>::vec*>(packed)[id] = v;
 }
 
-template <typename T, int MT, int NT>
+// PAIRS: a lane brings two neighbouring points at a time (rows of an even number of padded points, so that both are in one row; W >= 2).
+template <typename T, int MT, int NT, bool PAIRS>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 4))) void conv2d_kernel(const T* __restrict__ x, const T* __restrict__ packed, float* __restrict__ y, Geometry g) {
   typedef typename Elem<T>::vec vec;
-  constexpr int kHeld = NT == 1 ? 3 : 5;              // points per lane that travel while the channels before them are multiplied (more: fetched behind them)
+  typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+  typedef u32x2 two_words __attribute__((aligned(4)));
+  typedef unsigned one_word __attribute__((aligned(2)));
+  constexpr bool F16 = sizeof(T) == 2;
+  constexpr int P = PAIRS ? 2 : 1;                    // points of an item
+  constexpr int kHeld = PAIRS ? (NT == 1 ? 2 : 3) : (NT == 1 ? 3 : 5);        // items per lane that travel while the channels before them are multiplied (more: fetched behind them)
   constexpr int V = 16 / sizeof(T), TN = 64 * NT, kPitch = kPitchBytes / sizeof(T);
   extern __shared__ __align__(16) char lds[];
   T* image = reinterpret_cast<T*>(lds);                                                 // [2][span][pitch]
-  unsigned* where = reinterpret_cast<unsigned*>(lds + 2 * (size_t)g.span * kPitchBytes);   // [span]: byte offset into x without the channel, or kOutside
+  unsigned* where = reinterpret_cast<unsigned*>(lds + 2 * (size_t)g.span * kPitchBytes);   // of an item: byte offset into x without the channel, and which of its points are inside
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave >> 1, wn = wave & 1;
-  const int wide = g.WO + 2;
+  const int wide = (int)g.wide.by;
   // workgroups go to the eight XCDs round robin: an XCD gets a contiguous run of blocks
   const int per = gridDim.x >> 3, left = gridDim.x & 7, xcd = blockIdx.x & 7;
   const int block = xcd * per + (xcd < left ? xcd : left) + (blockIdx.x >> 3);
   const int run = (int)over((unsigned)block, g.blocks_across), rb = block - run * g.row_blocks, column0 = run * TN;
   const int last = (column0 + TN < g.columns ? column0 + TN : g.columns) - 1;
-  const int place0 = place_of(column0, g);
-  const int points = place_of(last, g) - place0 + 2 * wide + 3;            // <= span
+  const int place0 = place_of(column0, g) & ~(P - 1);
+  const int count = (place_of(last, g) - place0 + 2 * wide + 3 + P - 1) / P;            // items; P times that <= span
 
-  for (int i = tid; i < points; i += kThreads) {
-    const unsigned p = (unsigned)(place0 + i), n = over(p, g.image), r = p - n * g.image.by, row = over(r, g.wide);
+  // A lane that has no use for a point reads the nearest one inside: the first point of x cost every load a line of its own
+  // (float16 32 x 256 x 14 x 14 -> 256 33.2 -> 29.8 us).
+  for (int i = tid; i < count; i += kThreads) {
+    const unsigned p = (unsigned)(place0 + P * i), n = over(p, g.image), r = p - n * g.image.by, row = over(r, g.wide);
     const int h = (int)row - g.ph, w = (int)(r - row * g.wide.by) - g.pw;
-    const bool in = h >= 0 && h < g.H && w >= 0 && w < g.W;
-    where[i] = in ? ((n * (unsigned)g.C * (unsigned)g.H + (unsigned)h) * (unsigned)g.W + (unsigned)w) * (unsigned)sizeof(T) : kOutside;
+    const int hc = h < 0 ? 0 : h < g.H ? h : g.H - 1, wc = w < 0 ? 0 : w <= g.W - P ? w : g.W - P;
+    const unsigned inside = hc != h ? 0u : ((unsigned)w < (unsigned)g.W ? kFirst : 0u) | (PAIRS && (unsigned)(w + 1) < (unsigned)g.W ? kSecond : 0u);
+    where[i] = ((n * (unsigned)g.C * (unsigned)g.H + (unsigned)hc) * (unsigned)g.W + (unsigned)wc) * (unsigned)sizeof(T) | inside;
   }
 
   // this lane's output points: LDS place of tap (0, 0), and where the result goes
@@ -96,37 +111,60 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 4))
     const unsigned hw = g.results.by, n = over((unsigned)column, g.results);
     to[j] = (size_t)n * g.F * hw + ((unsigned)column - n * hw);
   }
-  // Item i of a lane: point lane + 64 i, channels wave * V .. + V - 1 of the chunk.  Loads go out without a branch between
+  // Item i of a lane: points P (lane + 64 i) .. + P - 1, channels wave * V .. + V - 1 of the chunk.  Loads go out without a branch between
   // them (points and channels past the end re-read the last one) and stay as they came until they are put into LDS: a
   // branch or a conversion behind each load is a wait for it.
   const size_t plane = (size_t)g.H * g.W * sizeof(T);
-  const int items = (points + 63) >> 6;
-  struct Item { typename Elem<T>::raw v[V]; };
-  auto fetch = [&](int q, int i) {
-    const int point = lane + 64 * i, c0 = (q * 4 + wave) * V;
-    const unsigned o = where[point < points ? point : points - 1];
-    const unsigned from = o == kOutside ? 0u : o;
-    Item r;
-#pragma unroll
-    for (int j = 0; j < V; ++j) {
-      const int c = c0 + j < g.C ? c0 + j : g.C - 1;                                    // the same in all lanes
-      const char* base = reinterpret_cast<const char*>(x) + c * plane;
-      r.v[j] = *reinterpret_cast<const typename Elem<T>::raw*>(base + (size_t)from);
-    }
-    return r;
+  const int items = (count + 63) >> 6;
+  typedef typename std::conditional<F16, unsigned, typename std::conditional<PAIRS, u32x2, unsigned>::type>::type Word;      // of one channel
+  struct Item { Word v[V]; };
+  auto place = [&](int i) { return where[lane + 64 * i < count ? lane + 64 * i : count - 1]; };
+  auto fetch = [&](int q, unsigned from, int j, Item& r) {
+    const int c0 = (q * 4 + wave) * V, c = c0 + j < g.C ? c0 + j : g.C - 1;               // the same in all lanes
+    const char* p = reinterpret_cast<const char*>(x) + c * plane + (size_t)(from & ~(kFirst | kSecond));
+    if constexpr (F16 && PAIRS) r.v[j] = *reinterpret_cast<const one_word*>(p);
+    else if constexpr (F16) r.v[j] = *reinterpret_cast<const unsigned short*>(p);
+    else if constexpr (PAIRS) r.v[j] = *reinterpret_cast<const two_words*>(p);
+    else r.v[j] = *reinterpret_cast<const unsigned*>(p);
   };
-  auto put = [&](int q, int i, const Item& r) {
-    const int point = lane + 64 * i, c0 = (q * 4 + wave) * V;
-    vec v;
+  auto put = [&](int q, int i, unsigned from, const Item& r) {
+    const int point = P * (lane + 64 * i), c0 = (q * 4 + wave) * V;
+    vec v[P];
 #pragma unroll
-    for (int j = 0; j < V; ++j) v[j] = __builtin_bit_cast(T, r.v[j]);
-    if (c0 + V > g.C) {
+    for (int k = 0; k < P; ++k) {
+      // both inside: first and second; one of a pair inside: it is the one further in of the two that were read
+      const bool in = (from & (k ? kSecond : kFirst)) != 0, second = PAIRS && ((from & kSecond) ? k == 1 && (from & kFirst) : k == 0);
+      if constexpr (F16) {
+        const unsigned halves = !in ? 0x0c0c0c0cu : second ? 0x07060302u : 0x05040100u;
+        typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+        u32x4 packed_halves;
 #pragma unroll
-      for (int j = 0; j < V; ++j) if (c0 + j >= g.C) v[j] = (T)0;
+        for (int j = 0; j < 4; ++j) packed_halves[j] = __builtin_amdgcn_perm(r.v[2 * j + 1], r.v[2 * j], halves);
+        v[k] = __builtin_bit_cast(vec, packed_halves);
+      } else {
+#pragma unroll
+        for (int j = 0; j < V; ++j) {
+          unsigned word;
+          if constexpr (PAIRS) word = second ? r.v[j][1] : r.v[j][0];
+          else word = r.v[j];
+          v[k][j] = __builtin_bit_cast(T, in ? word : 0u);
+        }
+      }
+      if (c0 + V > g.C) {
+#pragma unroll
+        for (int j = 0; j < V; ++j) if (c0 + j >= g.C) v[k][j] = (T)0;
+      }
     }
-    if (point >= points) return;
-    if (where[point] == kOutside) v = vec(0);
-    *reinterpret_cast<vec*>(image + ((size_t)(q & 1) * g.span + point) * kPitch + wave * V) = v;
+    if (point >= P * count) return;
+#pragma unroll
+    for (int k = 0; k < P; ++k) *reinterpret_cast<vec*>(image + ((size_t)(q & 1) * g.span + point + k) * kPitch + wave * V) = v[k];
+  };
+  auto fetch_and_put = [&](int q, int i) {
+    Item r;
+    const unsigned from = place(i);
+#pragma unroll
+    for (int j = 0; j < V; ++j) fetch(q, from, j, r);
+    put(q, i, from, r);
   };
 
   // The filter: a wavefront's MT x 2 operands of a tap, 64 x 16 bytes each, asked for kAhead taps before their use (a
@@ -136,7 +174,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 4))
   const size_t filter_step = (size_t)g.row_tiles * 128;
   constexpr int kSum = MT == 1 && NT == 1 ? 3 : kTaps;            // taps summed by themselves
   constexpr int kRows = sizeof(T) == 2 && kSum == 3 ? 2 : 1;      // float16: and the halves of the channels
-  constexpr int kPerTap = MT == 1 ? kHeld : 2;        // points per lane asked for with a tap
+  constexpr int kPerTap = (kHeld * V + kTaps - 2) / (kTaps - 1);      // loads of the next chunk's image that go out with a tap
   vec a[kSets][MT][2];
   auto fetch_filter = [&](int set, int tap) {
     const vec* p = filter + (size_t)tap * filter_step;
@@ -148,14 +186,19 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 4))
 
   art_lds_barrier();                                  // `where` is written
   Item held[kHeld];
+  unsigned from[kHeld];
 #pragma unroll
-  for (int i = 0; i < kHeld; ++i) held[i] = fetch(0, i);
+  for (int i = 0; i < kHeld; ++i) from[i] = place(i);
+#pragma unroll
+  for (int i = 0; i < kHeld; ++i)
+#pragma unroll
+    for (int j = 0; j < V; ++j) fetch(0, from[i], j, held[i]);
 #pragma unroll
   for (int t = 0; t < kAhead; ++t) fetch_filter(t, t);      // asked for last: loads come back in order
   __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-  for (int i = 0; i < kHeld; ++i) put(0, i, held[i]);
-  for (int i = kHeld; i < items; ++i) put(0, i, fetch(0, i));
+  for (int i = 0; i < kHeld; ++i) put(0, i, from[i], held[i]);
+  for (int i = kHeld; i < items; ++i) fetch_and_put(0, i);
   art_lds_barrier();
   f32x16 total[MT][NT];
 #pragma unroll
@@ -184,7 +227,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 4))
     for (int t = 0; t < kTaps; ++t) {
       if (kMore) {
 #pragma unroll
-        for (int i = t * kPerTap; i < (t + 1) * kPerTap && i < kHeld; ++i) held[i] = fetch(q + 1, i);
+        for (int k = t * kPerTap; k < (t + 1) * kPerTap && k < kHeld * V; ++k) fetch(q + 1, from[k / V], k % V, held[k / V]);
       }
       if (kMore || t + kAhead < kTaps) fetch_filter((t + kAhead) % kSets, q * kTaps + t + kAhead);
       __builtin_amdgcn_sched_barrier(0);              // left to the scheduler, the loads sink to their use
@@ -213,8 +256,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 4))
       for (int j = 0; j < NT; ++j) total[i][j] += acc[i][j];
     if (kMore) {
 #pragma unroll
-      for (int i = 0; i < kHeld; ++i) put(q + 1, i, held[i]);
-      for (int i = kHeld; i < items; ++i) put(q + 1, i, fetch(q + 1, i));
+      for (int i = 0; i < kHeld; ++i) put(q + 1, i, from[i], held[i]);
+      for (int i = kHeld; i < items; ++i) fetch_and_put(q + 1, i);
       art_lds_barrier();      // the other buffer is written, this one is free
     }
   };
@@ -227,11 +270,11 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 4))
 
 // The most points a block of `columns` output points can need: every step to the next row skips two points, every
 // step to the next image two rows.
-int span_of(const Geometry& g, int columns) {
+int span_of(const Geometry& g, int columns, bool pairs = false) {
   if (columns > g.columns) columns = g.columns;
-  const long long wide = g.WO + 2, hw = (long long)g.HO * g.WO;
+  const long long wide = g.WO + 2 + (pairs && g.WO % 2), hw = (long long)g.HO * g.WO;
   const long long rows = (columns - 1 + g.WO - 1) / g.WO, images = (columns - 1 + hw - 1) / hw;
-  const long long span = columns - 1 + rows * 2 + images * 2 * wide + 2 * wide + 3;
+  const long long span = columns - 1 + rows * (wide - g.WO) + images * 2 * wide + 2 * wide + 3 + (pairs ? 2 : 0);
   return span > (1 << 20) ? 1 << 20 : (int)span;
 }
 
@@ -276,14 +319,14 @@ long long blocks_of(const Geometry& g, int form) {
 }
 
 // What a form takes, in microseconds, both launches: a fixed part, per chunk of a block a time that grows with the blocks that
-// share a compute unit and with how unevenly they do, a ramp per further round, and the stores.  Fitted to 157 sizes in float16
-// and 153 in float32 (C 16-256, F 16-256, images of 7-56 squared, batches 1-32): 4.4 and 2.1 % off.  Over 150 other sizes
-// the form picked among all, the staged ones below included, was 0.2 % slower than the fastest in the mean, 1.2 times at worst.
+// share a compute unit and with how unevenly they do, a ramp per further round, and the stores.  Fitted to 330 sizes a form in float16 and
+// 310 in float32, two thirds of them of 16 to 256 channels and features, images of 7 to 56 squared and batches of 1 to 32: 5 and 1 to 3 % off.
+// (float16 64 x 64: 0.45 above the fit; where it is that close, the staged form with its shorter first fetch stays.)
 constexpr int kUnits = 256;                      // compute units of an MI355X
 double launch_time(const Geometry& g, int f16, int form) {
-  struct Cost { double fixed, alone, shared, uneven, again; };
-  static const Cost cost[2][3] = {{{5.66, 3.189, 2.500, 2.260, 0.486}, {5.97, 5.350, 4.539, 4.369, 0.0}, {5.92, 9.003, 8.308, 8.981, 4.782}},
-                                  {{6.32, 1.718, 1.331, 0.781, 0.169}, {6.89, 2.324, 1.382, 0.819, 0.466}, {7.26, 2.992, 1.627, 2.012, 0.271}}};
+  struct Cost { double fixed, alone, shared, uneven, again, store; };
+  static const Cost cost[2][3] = {{{5.364, 2.772, 2.427, 2.502, 0.862, 0.193}, {5.916, 4.966, 4.242, 4.677, 1.743, 0.148}, {6.714, 8.862, 8.215, 9.696, 1.217, 0.148}},
+                                  {{5.950, 1.524, 1.065, 0.756, 0.404, 0.241}, {6.181, 1.748, 0.815, 0.889, 1.157, 0.234}, {6.879, 2.374, 1.306, 1.421, 1.398, 0.193}}};
   const Cost& c = cost[f16 != 0][form - 1];
   const int per_chunk = f16 ? 32 : 16;
   const double chunks = g.chunks - (form < 3 && g.C - (g.chunks - 1) * per_chunk <= per_chunk / 2 ? 0.5 : 0.0);
@@ -291,7 +334,7 @@ double launch_time(const Geometry& g, int f16, int form) {
   // an image so wide that a compute unit holds two blocks or one (float16 64 x 64): 2.0 and 3.8 a chunk and round over ten sizes, 10 % off
   const size_t lds = lds_of(span_of(g, points_of(form)));
   const double shared = lds <= kMaxLds ? c.shared : lds <= kWideLds / 2 ? 2.0 : 3.8;
-  return c.fixed + chunks * (c.alone + shared * (full - 1) + (lds <= kMaxLds ? c.uneven : shared) * uneven) + c.again * (full - 1) + (f16 ? 0.207 : 0.357) * 4e-6 * g.columns * g.F;
+  return c.fixed + chunks * (c.alone + shared * (full - 1) + (lds <= kMaxLds ? c.uneven : shared) * uneven) + c.again * (full - 1) + c.store * 4e-6 * g.columns * g.F;
 }
 
 // The same for the staged forms (the launch that stages the image included): a fixed part, per chunk of a block's slice a time
@@ -413,14 +456,14 @@ int choose(const Geometry& g, int f16, bool gathered, double* time = nullptr) {
   return best;
 }
 
-template <typename T, int MT, int NT>
+template <typename T, int MT, int NT, bool PAIRS>
 int launch(const void* x, const void* packed, void* y, const Geometry& g, unsigned blocks, hipStream_t st) {
   static bool configured = false;
   if (lds_of(g.span) > kMaxLds && !configured) {
-    ART_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(conv2d_kernel<T, MT, NT>), hipFuncAttributeMaxDynamicSharedMemorySize, kWideLds));
+    ART_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(conv2d_kernel<T, MT, NT, PAIRS>), hipFuncAttributeMaxDynamicSharedMemorySize, kWideLds));
     configured = true;
   }
-  conv2d_kernel<T, MT, NT><<<dim3(blocks), dim3(kThreads), lds_of(g.span), st>>>((const T*)x, (const T*)packed, (float*)y, g);
+  conv2d_kernel<T, MT, NT, PAIRS><<<dim3(blocks), dim3(kThreads), lds_of(g.span), st>>>((const T*)x, (const T*)packed, (float*)y, g);
   ART_LAUNCH_CHECK();
   return 0;
 }
@@ -431,8 +474,19 @@ int run(const void* x, const void* w, void* packed, void* y, const Geometry& g, 
   conv2d_pack_kernel<T><<<dim3((unsigned)((lanes + kThreads - 1) / kThreads)), dim3(kThreads), 0, st>>>((const T*)w, (T*)packed, g);
   ART_LAUNCH_CHECK();
   const unsigned blocks = (unsigned)blocks_of(g, form);
-  return form == 1 ? launch<T, 1, 1>(x, packed, y, g, blocks, st) : form == 2 ? launch<T, 1, 2>(x, packed, y, g, blocks, st)
-                                                                             : launch<T, 2, 2>(x, packed, y, g, blocks, st);
+  // Two points at a time, in rows of an even number, unless a row has one or the odd column does not fit into LDS any more.
+  const int span = span_of(g, points_of(form), true);
+  if (g.W >= 2 && (long long)(g.HO + 2) * (g.WO + 2 + g.WO % 2) <= (1 << 30) / g.N &&
+      lds_of(span) <= (lds_of(g.span) > kMaxLds ? kWideLds : kMaxLds)) {
+    Geometry even = g;
+    even.span = span;
+    even.wide = make_div((unsigned)(g.WO + 2 + g.WO % 2));
+    even.image = make_div((unsigned)(g.HO + 2) * even.wide.by);
+    return form == 1 ? launch<T, 1, 1, true>(x, packed, y, even, blocks, st) : form == 2 ? launch<T, 1, 2, true>(x, packed, y, even, blocks, st)
+                                                                                       : launch<T, 2, 2, true>(x, packed, y, even, blocks, st);
+  }
+  return form == 1 ? launch<T, 1, 1, false>(x, packed, y, g, blocks, st) : form == 2 ? launch<T, 1, 2, false>(x, packed, y, g, blocks, st)
+                                                                                    : launch<T, 2, 2, false>(x, packed, y, g, blocks, st);
 }
 
 }  // namespace

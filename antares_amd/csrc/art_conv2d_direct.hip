@@ -71,10 +71,10 @@ __global__ __launch_bounds__(64 * most_waves(sizeof(T), NT, KP)) void conv2d_dir
   bool in[KP];
 #pragma unroll
   for (int i = 0; i < KP; ++i) {
-    const unsigned p = (unsigned)(place0 + lane + 64 * i), n = over(p, g.image), r = p - n * g.image.by, row = over(r, g.wide);
-    const int h = (int)row - g.ph, c = (int)(r - row * g.wide.by) - g.pw;
-    in[i] = lane + 64 * i < points && h >= 0 && h < g.H && c >= 0 && c < g.W;
-    from[i] = in[i] ? ((n * (unsigned)g.C * (unsigned)g.H + (unsigned)h) * (unsigned)g.W + (unsigned)c) * (unsigned)sizeof(T) : 0u;
+    const unsigned p = (unsigned)(place0 + (lane + 64 * i < points ? lane + 64 * i : points - 1)), n = over(p, g.image), r = p - n * g.image.by, row = over(r, g.wide);
+    const int h = (int)row - g.ph, c = (int)(r - row * g.wide.by) - g.pw, near_h = h < 0 ? 0 : h < g.H ? h : g.H - 1, near_c = c < 0 ? 0 : c < g.W ? c : g.W - 1;
+    in[i] = lane + 64 * i < points && h == near_h && c == near_c;
+    from[i] = ((n * (unsigned)g.C * (unsigned)g.H + (unsigned)near_h) * (unsigned)g.W + (unsigned)near_c) * (unsigned)sizeof(T);      // outside: the nearest point inside
   }
   // this lane's output points: their place in the run
   int at[NT];

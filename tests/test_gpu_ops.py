@@ -1349,6 +1349,16 @@ def test_convolution_blocks_match_float64(autort, dtype, form, case):
     assert ((y.cpu().double() - want).abs() <= bound + 1e-30).all()
 
 
+@pytest.mark.parametrize('dtype,form,case', [(d, f, c) for c in (
+    (3, 40, (50, 1), 40, (1, 1), (50, 1), True),           # a point to a row: gathered one by one
+    (2, 24, (33, 2), 40, (1, 1), (33, 2), True),           # both points of a pair, and one of each of two
+    (2, 33, (7, 9), 70, (0, 0), (5, 7), False),            # odd rows without padding: no point outside between two rows
+    (1, 16, (6, 11), 33, (1, 3), (7, 13), True),           # pairs that begin two points outside
+) for f in (1, 2, 3) for d in ('float16', 'float32')])
+def test_convolutions_gathered_two_points_at_a_time_match_float64(autort, dtype, form, case):
+    test_convolution_blocks_match_float64(autort, dtype, form, case)
+
+
 @pytest.mark.parametrize('dtype', ['float16', 'float32'])
 @pytest.mark.parametrize('case', CONV_CASES + [(1, 100, (11, 57), 70, (1, 1), (11, 57), True),      # several chunks, a row longer than a block of 64
                                                (2, 40, (120, 5), 200, (1, 1), (120, 5), True)])     # many rows to a block
