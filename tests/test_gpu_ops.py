@@ -1350,7 +1350,7 @@ def test_convolution_blocks_match_float64(autort, dtype, form, case):
 
 
 @pytest.mark.parametrize('dtype,form,case', [(d, f, c) for c in (
-    (3, 40, (50, 1), 40, (1, 1), (50, 1), True),           # a point to a row: gathered one by one
+    (3, 40, (20, 1), 40, (1, 1), (20, 1), True),           # a point to a row: gathered one by one
     (2, 24, (33, 2), 40, (1, 1), (33, 2), True),           # both points of a pair, and one of each of two
     (2, 33, (7, 9), 70, (0, 0), (5, 7), False),            # odd rows without padding: no point outside between two rows
     (1, 16, (6, 11), 33, (1, 3), (7, 13), True),           # pairs that begin two points outside
