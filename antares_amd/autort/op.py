@@ -245,7 +245,9 @@ class ExportedOp(calls.Operator):
                     if n not in bound:
                         bound[n] = torch.empty(g.shape_of(n, env), dtype=TORCH_DTYPE[g.tensors[n].dtype], device=dev)
                 pointers = {n: bound[n].data_ptr() for n in group.args}
-                sym, grid = group.choose(env, pointers)
+                sym, grid = group.choose_ragged(env, pointers)
+                if not grid:
+                    sym, grid = group.choose(env, pointers)
                 if not grid:
                     sym, grid = group.choose_short(env, pointers)
                 if grid:

@@ -17,12 +17,12 @@ class _Rule:
 
     def __setattr__(self, name, value):
         object.__setattr__(self, name, value)
-        if name == 'choose':
+        if name.startswith('choose'):
             calls.forget()
 
     def __delattr__(self, name):
         object.__delattr__(self, name)
-        if name == 'choose':
+        if name.startswith('choose'):
             calls.forget()
 
 
@@ -41,6 +41,8 @@ class RowGroup(_Rule):
     pure: bool = False             # reductions only, no map behind them
     # kernels with a row in the registers of 16 lanes: (elements per vector, vectors per lane, symbol)
     short: List[Tuple[int, int, str]] = field(default_factory=list)
+    # kernels in vectors for rows of any length and address, like `cached`
+    ragged: List[Tuple[int, int, int, str]] = field(default_factory=list)
 
     def _extents(self, env: Dict[str, int]) -> Tuple[int, int]:
         e = self.red_axis[1]
@@ -79,6 +81,40 @@ class RowGroup(_Rule):
             pick = min(blocks, key=lambda f: f[2])
         per_block = BLOCK // pick[0]
         return pick[3], min((rows + per_block - 1) // per_block, MAX_GRID)
+
+    def choose_ragged(self, env: Dict[str, int], pointers: Dict[str, int]) -> Tuple[str, int]:
+        """The same among the kernels in vectors for rows of any length and address; grid 0 where those of `choose` are as fast.  With V
+        elements to 16 bytes, softmax and layer normalisation in float32, `choose` / this (us):
+          * up to 64 V, a wavefront per row: 4487 x 167 6.9 / 4.8, 912 x 152 3.9 / 3.1, 2 x 140 3.2 / 2.7; there is one in `choose` for 8192 rows
+            and more (10806 x 132 4.8 / 4.9, 56548 x 157 18.8 / 24.4);
+          * up to 128 V, with 256 rows and more (in whole vectors below 8192): 62446 x 339 65.7 / 43.3, 5045 x 435 6.7 / 5.4, 418 x 344 3.8 / 3.5; with
+            fewer rows a block has each of them sooner (60 x 470 3.3 / 3.6);
+          * up to 256 V, with 8192 rows and more that are not whole vectors: 30000 x 701 31 / 27, 10328 x 513 11.0 / 9.9; 2400 x 555 5.7 / 6.2;
+          * 256 to 512 V, not whole vectors, a block per row: 766 x 1113 5.5 / 4.8, 8814 x 1454 25.8 / 24.3;
+          * 1024 to 2048 V, eight vectors per lane: rows that are not whole vectors were walked (6012 x 4973 77 / 51, 70 x 7558 8.9 / 6.6); whole
+            ones had sixteen, so that half as many blocks shared a compute unit, with 1024 rows and more (6864 x 4460 72 / 50, 562 x 6448 6.0 / 7.6).
+        Elements of four bytes only: with eight or more of them per vector and lane a wavefront per row was as often slower (float16 12022 x 604 18.1 / 19.9).
+        Sums are no longer than in `choose`: an element of every vector's four after the other there, in pairs here."""
+        rows, n = self._extents(env)
+        if n < 128 or rows == 0 or not self.ragged:
+            return self.symbol, 0
+        V = self.ragged[0][1]
+        whole = n % V == 0 and all(pointers[t] % 16 == 0 for t in self.vec_tensors)
+        if n <= 64 * V:
+            form = (64, 1) if rows < 8192 else None
+        elif n <= 128 * V:
+            form = (64, 2) if rows >= 256 and (rows < 8192 or not whole) else None
+        elif n <= 256 * V:
+            form = (64, 4) if rows >= 8192 and not whole else None
+        elif n <= 512 * V:
+            form = (BLOCK, 2) if not whole else None
+        else:
+            form = (BLOCK, 8) if 1024 * V < n <= 2048 * V and (rows >= 1024 or not whole) else None
+        for team, _, E, sym in self.ragged:
+            if (team, E) == form:
+                per_block = BLOCK // team
+                return sym, min((rows + per_block - 1) // per_block, MAX_GRID)
+        return self.symbol, 0
 
     def choose_short(self, env: Dict[str, int], pointers: Dict[str, int]) -> Tuple[str, int]:
         """The same for rows of 16 to 127 elements, four of them in a wavefront; grid 0 when the per-statement kernels do

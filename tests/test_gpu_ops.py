@@ -1272,6 +1272,41 @@ def test_rows_of_fewer_than_two_wavefronts(autort, program, dtype, rows, n, offs
         assert bool(((got.double() - want)[fine].abs() <= want[fine] * (n + 60) * eps + torch.finfo(t).tiny).all())
 
 
+# vectors that start anywhere: the first and the last length of every form, rows of whole vectors at odd addresses, rows that end inside a block
+@pytest.mark.parametrize('program,dtype', [('softmax', 'float32'), ('sum', 'int32')])
+@pytest.mark.parametrize('rows,n,offset', [(3, 128, 0), (7, 129, 0), (5, 253, 1), (1001, 256, 0), (259, 257, 0), (258, 511, 0), (257, 512, 1), (8195, 513, 0), (8193, 1023, 0), (8193, 1024, 3),
+                                           (2, 1025, 0), (1, 2047, 2), (3, 4097, 0), (2, 8191, 0), (1025, 8192, 0)])
+def test_rows_in_vectors_that_start_anywhere(autort, program, dtype, rows, n, offset):
+    """One kernel, and the statements one by one: exact for whole numbers, else both within (n + 8) roundings of the sums, the exponentials and the
+    quotient of the float64 result.  Infinities, NaN and rows of the type's lowest value included."""
+    note(f'ragged rows {program} {dtype} {rows} x {n} at {offset}')
+    dev, t = autort.device(), getattr(torch, dtype)
+    op = autort.export(ir=SHORT_ROWS[program], inputs=[f'input0={dtype}[N:64, C:100]'], name=f'ragged_{program}_{dtype}')
+    g = torch.Generator().manual_seed(rows + n)
+    x = torch.randint(-1, 2, (rows, n), generator=g).to(t) if program == 'sum' else torch.randn(rows, n, generator=g)
+    if program == 'softmax' and rows > 8:
+        x[1, 3], x[2], x[3, 0], x[4], x[5, n - 1], x[6, n - 2] = float('-inf'), float('-inf'), float('nan'), torch.finfo(t).min, float('inf'), float('-inf')
+    xd = torch.zeros(rows * n + offset, dtype=t, device=dev)[offset:].view(rows, n).copy_(x)
+    group = op.plans[0].row_group
+    assert group.choose_ragged({'N': rows, 'C': n}, {a: (4 * offset if a == 'input0' else 0) for a in group.args})[1] > 0
+    together = op(xd).cpu()
+    try:
+        for p in op.plans:
+            p.row_group = None
+        apart = op(xd).cpu()
+    finally:
+        op.plans[0].row_group = group
+    if program == 'sum':
+        assert torch.equal(together, apart) and torch.equal(together.long(), x.long() - x.long().sum(1, keepdim=True) * n)
+        return
+    want = torch.softmax(x.double(), 1)
+    eps = torch.finfo(t).eps
+    for got in (together, apart):
+        assert torch.equal(got.isnan(), want.isnan())
+        fine = ~want.isnan()
+        assert bool(((got.double() - want)[fine].abs() <= want[fine] * (n + 60) * eps + torch.finfo(t).tiny).all())
+
+
 @pytest.mark.parametrize('ir,ta,tb,M,N,K', [
     ('out[M, N] +=! x[K, M] * w[K, N]', True, False, 1028, 512, 96),
     ('out[M, N] +=! x[M, K] * w[N, K]', False, True, 1000, 1030, 64),       # a linear layer: N need not be a multiple of 4

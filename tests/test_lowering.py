@@ -41,6 +41,19 @@ def test_softmax_is_one_row_group_with_kernels_for_short_and_long_rows():
         assert f'void {sym}(' in src
 
 
+@pytest.mark.parametrize('rows,n,offset,form', [
+    (32, 128, 0, 'rw1'), (32, 255, 4, 'rw1'), (8192, 255, 0, None), (255, 300, 0, None), (256, 300, 0, 'rw2'), (8192, 300, 0, None), (8192, 301, 0, 'rw2'), (8192, 300, 4, 'rw2'),
+    (8191, 600, 4, None), (8192, 601, 0, 'rw4'), (8192, 600, 0, None), (5, 1025, 0, 'rb2'), (5, 1028, 0, None), (5, 2049, 0, None), (5, 4097, 0, 'rb8'), (1023, 4100, 0, None),
+    (1024, 4100, 0, 'rb8'), (1024, 8193, 0, None), (32, 127, 0, None)])
+def test_rows_take_vectors_that_start_anywhere_where_they_are_faster(rows, n, offset, form):
+    src, plans = lowered(SOFTMAX, ['input0=float32[N:32, C:1024]'])
+    group = plans[0].row_group
+    sym, grid = group.choose_ragged({'N': rows, 'C': n}, {a: (offset if a == 'output0' else 0) for a in group.args})
+    assert (sym, grid) == (f'{group.symbol}_{form}', -(-rows // (4 if form[1] == 'w' else 1))) if form else grid == 0
+    assert f'void {sym}(' in src
+    assert not lowered(SOFTMAX, ['input0=float16[N:32, C:1024]'])[1][0].row_group.ragged
+
+
 @pytest.mark.parametrize('ir,inputs,covered', [
     # the map reads a result at another row's position: the reduction alone is a group
     ('t[N] +=! x[N, C]; y[N, C] = x[N, C] - t[(N + 1) % 8]', ['x=float32[N:8, C:256]'], 1),
