@@ -339,14 +339,15 @@ double launch_time(const Geometry& g, int f16, int form) {
 
 // The same for the staged forms (the launch that stages the image included): a fixed part, per chunk of a block's slice a time
 // that grows with the blocks that share a compute unit and with how unevenly they do, the copy, the stores, and for slices the
-// third launch.  Fitted to 116 sizes in float16 and 214 in float32 of the same ranges: 3.1 and 1.9 % off, and what it picks is 0.05 and
-// 0.25 % slower than the fastest in the mean.
+// third launch.  Fitted to 116 sizes in float16 and, float32, to the 2058 times of 320 sizes that are within 1.5 times the fastest: 3.1 and 3 % off.  What
+// is picked of all forms in float32 is 0.48 % slower than the fastest in the mean, 2.2 % of the sizes by more than 5 % (0.63 and 4.1 % with the
+// constants before the gathering forms loaded two points at a time: these came out 2 % below, the staged ones 3 % above what they take).
 double staged_time(const Geometry& g, int f16, int form, int slices) {
   struct Cost { double fixed, alone, shared, uneven; };
   struct Rest { double sum, sum_bytes, copy, store; };
-  static const Cost cost[2][4] = {{{6.30, 2.657, 2.526, 2.445}, {6.97, 4.661, 4.081, 4.561}, {8.15, 8.396, 7.815, 8.575}, {6.25, 4.809, 5.443, 5.217}},
+  static const Cost cost[2][4] = {{{5.82, 2.736, 2.642, 2.469}, {6.48, 4.700, 4.335, 4.628}, {8.11, 8.376, 8.365, 9.814}, {6.25, 4.809, 5.443, 5.217}},
                                   {{6.52, 0.998, 0.861, 0.730}, {7.14, 1.309, 0.900, 0.661}, {8.03, 1.836, 1.636, 1.386}, {}}};
-  static const Rest rest[2] = {{2.64, 0.384, 0.580, 0.271}, {2.62, 0.342, 0.510, 0.242}};
+  static const Rest rest[2] = {{2.55, 0.348, 0.440, 0.246}, {2.62, 0.342, 0.510, 0.242}};
   const Cost& c = cost[f16 != 0][form - 4];
   const Rest& r = rest[f16 != 0];
   const int per_chunk = f16 ? 32 : 16;
