@@ -63,8 +63,8 @@ static_assert(16 * 1024 + 32 * (BN + 8) * 2 <= 3 * stage_bytes(1) && 32 * 1024 +
 // How the (column tile, K split) pairs are laid out; worked out on the host, so that a block starts without divisions.
 struct Work {
   Deal deal;
-  int col_tiles, splits;
-  unsigned int inv_tiles;                           // ceil(2^32 / col_tiles), 0 for one tile: unit / col_tiles = mulhi(unit, inv_tiles) for units below 2^16
+  int splits;
+  unsigned int inv_splits;                          // ceil(2^32 / splits), 0 for one split: unit / splits = mulhi(unit, inv_splits) for units below 2^16
   int groups, longer;                               // groups of a K split; the first `longer` have one more
 };
 
@@ -83,8 +83,8 @@ __global__ __launch_bounds__(kThreads, MT == 4 ? 2 : 4) void gemm_w4a16_kernel(
   int unit, m_block;                                // (tile, split) pair, block of rows
   if (!work.deal.take(unit, m_block)) return;
   const int m0 = m_block * BM;
-  const int split = work.inv_tiles ? (int)__umulhi(unit, work.inv_tiles) : unit;      // unit / col_tiles
-  const TileColumns<TAIL, BN> cols{(unit - split * work.col_tiles) * (SWIGLU ? BN / 2 : BN), N};
+  const int tile = work.inv_splits ? (int)__umulhi(unit, work.inv_splits) : unit, split = unit - tile * work.splits;
+  const TileColumns<TAIL, BN> cols{tile * (SWIGLU ? BN / 2 : BN), N};
   const int g_begin = split * work.groups + (split < work.longer ? split : work.longer), groups = work.groups + (split < work.longer ? 1 : 0);
   const unsigned int lds0 = (unsigned int)(size_t)(__attribute__((address_space(3))) unsigned char*)smem;
 
@@ -656,7 +656,7 @@ int run_rows(const _Float16* xs, const unsigned char* qweight, const _Float16* s
     const int col_tiles = tile_count(N, swiglu, BN), m_blocks = (M + 32 * p.row_tiles - 1) / (32 * p.row_tiles);
     const int units = col_tiles * p.splits, G = K / GK;
     dim3 grid;
-    const Work work{deal(units, m_blocks, grid), col_tiles, p.splits, (unsigned int)((0x100000000ull + col_tiles - 1) / col_tiles), G / p.splits, G % p.splits};
+    const Work work{deal(units, m_blocks, grid), p.splits, (unsigned int)((0x100000000ull + p.splits - 1) / p.splits), G / p.splits, G % p.splits};
     const auto kernel = kernels[far(p, K, N) ? 3 : p.row_tiles == 4 ? 2 : p.row_tiles - 1][tail];
     kernel<<<grid, kThreads, lds_bytes(p.row_tiles), st>>>(xs, qweight, scales, qzeros, ys, scratch, M, K, N, work, kMagic, res, rope);
     ART_LAUNCH_CHECK();

@@ -54,7 +54,7 @@ template <int MT, Tail TAIL, bool FAR>
 __global__ __launch_bounds__(kThreads, MT == 8 ? 1 : 2) void gemm_w4a16_wide_kernel(
     const _Float16* __restrict__ x, const unsigned char* __restrict__ qweight, const _Float16* __restrict__ scales,
     const unsigned char* __restrict__ qzeros, _Float16* y, float* __restrict__ partial, int M, int K, int N, int splits,
-    Deal deal, Div col_tiles, int groups, int longer, Magic mg, const _Float16* residual, Rope rope) {       // residual may be y itself
+    Deal deal, Div by_splits, int groups, int longer, Magic mg, const _Float16* residual, Rope rope) {       // residual may be y itself
   constexpr bool SWIGLU = TAIL == kSwiglu;
   constexpr int STAGE = stage_bytes(MT), BM = 32 * MT;
   constexpr int L = 2 + MT + 1;                     // loads per wavefront and stage
@@ -62,8 +62,8 @@ __global__ __launch_bounds__(kThreads, MT == 8 ? 1 : 2) void gemm_w4a16_wide_ker
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   int unit, m_block;                                // (column tile, K split) pair, block of rows
   if (!deal.take(unit, m_block)) return;
-  const int split = (int)over((unsigned)unit, col_tiles);
-  const TileColumns<TAIL, BN> cols{(unit - split * (int)col_tiles.by) * (SWIGLU ? BN / 2 : BN), N};
+  const int tile = (int)over((unsigned)unit, by_splits), split = unit - tile * splits;
+  const TileColumns<TAIL, BN> cols{tile * (SWIGLU ? BN / 2 : BN), N};
   const int m0 = m_block * BM;
   const int g_begin = split * groups + (split < longer ? split : longer), g_count = groups + (split < longer ? 1 : 0);
   const int steps = 2 * g_count;          // splits <= G: at least two
@@ -365,7 +365,7 @@ int launch(const _Float16* x, const unsigned char* qweight, const _Float16* scal
   dim3 grid;
   const Deal dealt = deal(col_tiles * splits, m_blocks, grid);
   gemm_w4a16_wide_kernel<MT, TAIL, FAR><<<grid, kThreads, lds_bytes(MT), stream>>>(
-      x, qweight, scales, qzeros, y, partial, M, K, N, splits, dealt, make_div((unsigned)col_tiles), K / 128 / splits, K / 128 % splits,
+      x, qweight, scales, qzeros, y, partial, M, K, N, splits, dealt, make_div((unsigned)splits), K / 128 / splits, K / 128 % splits,
       kMagic, residual, rope);
   ART_LAUNCH_CHECK();
   return 0;
