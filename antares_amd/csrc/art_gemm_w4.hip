@@ -10,8 +10,8 @@
 //     groups.  Wavefront (c, h) multiplies 32 columns by the k half h of every group, so every weight is unpacked once per
 //     block; the two k halves meet in LDS after the loop.  What bounds the loop is the issue of instructions, not the
 //     matrix cores (with the MFMAs taken out a group takes as long): a wavefront by itself issues a vector instruction every 8
-//     cycles, two of a SIMD one every 4 (the differences and products of halves and the byte permutations; shifts and
-//     v_bitop3 2), and a group is 114 / 126 / 169 instructions at MT = 1 / 2 / 4, 64 of them vector instructions that
+//     cycles, two of a SIMD one every 4 (the differences and products of halves and byte permutations; shifts and
+//     v_bitop3 2), and a group is some 95 / 120 / 157 instructions at MT = 1 / 2 / 4, 56 of them vector instructions that
 //     unpack.  Hence ring slots that are constants (the loop is three groups long) and loads from buffer descriptors, where one
 //     scalar offset moves on.  With slots and addresses in registers a group was 138 / 149 / 193 instructions, and each store of a
 //     K-split's sums ten (a comparison, a branch, 64-bit addresses) instead of two: 16 rows over 1024 x 3072 6.6 -> 6.2 us, over
@@ -24,8 +24,11 @@
 //     The weights run a group ahead of x, so that the first operands of a group are unpacked in the one before;
 //   * LDS position (row r, chunk p) holds chunk p ^ ((r / 2) & 7) of the weights (rows of 128 bytes) and p ^ (r & 15) of x
 //     (rows of 256 bytes): every 16 lanes of a read touch every bank once;
-//   * the packed bytes stay packed in LDS.  ds_read_b64_tr_b8 hands a lane the 8 bytes = 16 values of k of ONE column,
-//     i.e. the B operand of two v_mfma_f32_32x32x16_f16;
+//   * the packed bytes stay packed in LDS.  ds_read_b64_tr_b8 hands a lane four bytes = 8 values of k of ONE column, each byte twice (the
+//     B operand of a v_mfma_f32_32x32x16_f16): a byte's nibbles are where the two halves of a pair want them without a permutation.  Against
+//     every byte once, eight of them a read, and permutations (64 instructions that unpack), HBM / cache, us: 16 rows of gate | up
+//     4096 x 22016 19.1 / 18.3 -> 18.5 / 16.8, 50 rows 22.7 / 20.7 -> 22.5 / 19.4, 128 rows over 4096 x 12288 21.5 / 19.4 -> 20.7 / 19.5, over 11008 x 4096 in
+//     four splits 23.3 / 21.7 -> 22.0 / 21.0; 17 products 1.022 / 1.029 times as fast;
 //   * split-K without atomics (5.6 M float atomics cost 75 us on this chip): each K-split writes its fp32 tile to the
 //     library workspace and a second small kernel adds the splits in a fixed order and rounds once to fp16 - results
 //     do not depend on timing.
@@ -142,10 +145,12 @@ __global__ __launch_bounds__(kThreads, MT == 4 ? 2 : 4) void gemm_w4a16_kernel(
   // further on, whose swizzled positions are the other four (and, with SWIGLU, the up columns of the lanes' gates).
   const int s16 = lane & 15, hi16 = (lane >> 4) & 1, h = lane >> 5;
   const int chunk = cw + 4 * hi16, colpos = chunk * 16 + s16;              // the column (within the tile) this lane accumulates
-  const int b_row = kh * 32 + h * 16 + (s16 >> 1);                         // + 8 q
-  int b_off[2], a_off[4];
+  int b_off[4], a_off[4];
 #pragma unroll
-  for (int q = 0; q < 2; ++q) b_off[q] = (b_row + 8 * q) * 128 + ((chunk ^ (((b_row + 8 * q) >> 1) & 7)) * 16) + (s16 & 1) * 8;
+  for (int e = 0; e < 4; ++e) {
+    const int r = kh * 32 + h * 16 + 4 * e + twice_row(s16 >> 1);
+    b_off[e] = r * 128 + ((chunk ^ ((r >> 1) & 7)) * 16) + (s16 & 1) * 8;
+  }
 #pragma unroll
   for (int e = 0; e < 4; ++e) a_off[e] = W_BYTES + Q_BYTES + (lane & 31) * 256 + (((kh * 8 + h * 4 + e) ^ s16) * 16);     // + 8192 per row tile
 
@@ -155,14 +160,14 @@ __global__ __launch_bounds__(kThreads, MT == 4 ? 2 : 4) void gemm_w4a16_kernel(
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[t][r] = 0.f;
 
-  i32x2 pk[2], pk_next[2];                          // packed weights of the group and of the next one: [q]
+  i32x2 pk[4], pk_next[4];                          // packed weights of the group and of the next one: [round]
   _Float16 raw_s;
   unsigned int raw_z;
   h2 s2, zz2;                                       // scale, 1024 and 64 + zero point of this lane's column
   h8 fa[2][MT];                                     // operands of a round, double buffered: x
   h2 fb[2][4];                                      // ... weights, in pairs of k
-  auto read_weights = [&](unsigned int slot, i32x2 (&to)[2], int q) {
-    to[q] = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_i32x2*)(smem + slot + b_off[q]));
+  auto read_weights = [&](unsigned int slot, i32x2 (&to)[4], int e) {
+    to[e] = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_i32x2*)(smem + slot + b_off[e]));
   };
   auto read_scales = [&](unsigned int slot) {
     const unsigned char* st = smem + slot + W_BYTES;
@@ -178,9 +183,8 @@ __global__ __launch_bounds__(kThreads, MT == 4 ? 2 : 4) void gemm_w4a16_kernel(
   auto read_x = [&](unsigned int slot, int e, int t) {
     fa[e & 1][t] = *reinterpret_cast<const h8*>(smem + slot + a_off[e] + t * 8192);
   };
-  // pair j for round e = 2 q + dword.  Byte j of the word holds k = 2 j (low nibble) and 2 j + 1 (high nibble).
-  auto unpack = [&](const i32x2 (&from)[2], int e, int j) {
-    fb[e & 1][j] = (as_h2(and_or(nibble_pair<(MT > 1)>((unsigned int)from[e >> 1][e & 1], j), mg.mask, mg.bias)) - zz2) * s2;
+  auto unpack = [&](const i32x2 (&from)[4], int e, int j) {       // k = 2 j, 2 j + 1 of round e
+    fb[e & 1][j] = (as_h2(and_or(nibbles_of_twice((unsigned int)from[e][j >> 1], j), mg.mask, mg.bias)) - zz2) * s2;
   };
   auto multiply = [&](int slot, int t) {
     const h2* p = fb[slot];
@@ -204,8 +208,8 @@ __global__ __launch_bounds__(kThreads, MT == 4 ? 2 : 4) void gemm_w4a16_kernel(
   x_rows.next();
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(L) : "memory");       // loads return in order
   art_lds_barrier();
-  read_weights(2 * STAGE, pk, 0);
-  read_weights(2 * STAGE, pk, 1);
+#pragma unroll
+  for (int e = 0; e < 4; ++e) read_weights(2 * STAGE, pk, e);
   read_scales(2 * STAGE);
   decode_scales();
 #pragma unroll
@@ -227,8 +231,9 @@ __global__ __launch_bounds__(kThreads, MT == 4 ? 2 : 4) void gemm_w4a16_kernel(
     if constexpr (E == 0) issue(Int<(S + 2) % 3>{}, Int<2 + c>{});         // x of the group two ahead
     if constexpr (E == 3 && c == 0) issue(s_tag, Int<0>{});                // weights of the group four ahead
     if constexpr (E == 3 && c == MT - 1) issue(s_tag, Int<1>{});
-    if (E == 2 && c == 0) { read_weights(s_cur, pk_next, 0); read_scales(s_cur); }     // the weights of the next group came with x of this one
-    if (E == 2 && c == MT - 1) read_weights(s_cur, pk_next, 1);
+    if (E < 3 && c == 0) read_weights(s_cur, pk_next, E);                  // the weights of the next group came with x of this one
+    if (E == 2 && c == 0) read_scales(s_cur);
+    if (E == 2 && c == MT - 1) read_weights(s_cur, pk_next, 3);
     if (E == 3 && c == 0) decode_scales();
     E == 3 ? read_x(s_next, 0, c) : read_x(s_cur, (E + 1) & 3, c);
 #pragma unroll
@@ -252,8 +257,8 @@ __global__ __launch_bounds__(kThreads, MT == 4 ? 2 : 4) void gemm_w4a16_kernel(
     art_lds_barrier();
     round(s_tag, Int<3>{});
     next_weights();
-    pk[0] = pk_next[0];
-    pk[1] = pk_next[1];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) pk[e] = pk_next[e];
   };
   for (int left = groups;;) {                       // the slots are constants
     group(Int<0>{});

@@ -172,7 +172,7 @@ __global__ __launch_bounds__(kThreads, XR == 16 ? 4 : 2) void gemm_w4a16_deep_ke
         for (int ct = 0; ct < CT; ++ct) {
           h2 p[4];
 #pragma unroll
-          for (int j = 0; j < 4; ++j) p[j] = as_h2(and_or(nibble_pair<true>((unsigned int)pk[ct][e >> 1][e & 1], j), mg.mask, mg.bias)) - zz2[ct];
+          for (int j = 0; j < 4; ++j) p[j] = as_h2(and_or(nibble_pair((unsigned int)pk[ct][e >> 1][e & 1], j), mg.mask, mg.bias)) - zz2[ct];
 #pragma unroll
           for (int j = 0; j < 4; ++j) p[j] = p[j] * s2[ct];
           const h8 b = h8{p[0][0], p[0][1], p[1][0], p[1][1], p[2][0], p[2][1], p[3][0], p[3][1]};

@@ -160,7 +160,7 @@ __global__ __launch_bounds__(kThreads, MT == 8 ? 1 : 2) void gemm_w4a16_wide_ker
   // nibble).  Step by step for both: a difference directly in front of its product costs a wait state.
   auto unpack_two = [&](int par, int e, int ct, int j) {
     const unsigned int w = (unsigned int)pk[par][e >> 1][ct][e & 1];
-    const h2 a = as_h2(and_or(nibble_pair<true>(w, j), mg.mask, mg.bias)), b = as_h2(and_or(nibble_pair<true>(w, j + 1), mg.mask, mg.bias));
+    const h2 a = as_h2(and_or(nibble_pair(w, j), mg.mask, mg.bias)), b = as_h2(and_or(nibble_pair(w, j + 1), mg.mask, mg.bias));
     const h2 da = a - zz2[ct], db = b - zz2[ct];
     fb[e & 1][ct][j] = da * s2[ct];
     fb[e & 1][ct][j + 1] = db * s2[ct];

@@ -38,15 +38,20 @@ __device__ __forceinline__ unsigned int and_or(unsigned int w, unsigned int mask
 constexpr Magic kMagic{0x00F0000Fu, 0x54006400u};
 
 // Byte j of a word holds k = 2 j (low nibble) and 2 j + 1 (high nibble).  Masked and biased as kMagic, the result is fp16 (1024 + the
-// first, 64 + the second): the low nibble is the last bits of 1024 + q, the high one those of 64 + q where it lies.  SHIFT: two of
-// four byte permutations are shifts, which issue faster but wait for the first ones: blocks of 32 rows, with little between the
-// pairs, are 2 to 4 % slower so, larger ones 1 to 3 % faster (one card, against a shift and four permutations per word: 128
-// rows over 4096 x 22016 30.1 -> 29.4 us, over 11008 x 4096 22.9 -> 22.5, 1003 rows over 4096 x 22016 161.0 -> 158.8).
-template <bool SHIFT> __device__ __forceinline__ unsigned int nibble_pair(unsigned int w, int j) {
-  if (!SHIFT) return __builtin_amdgcn_perm(w, w, 0x0c000c00u + 0x00010001u * j);
+// first, 64 + the second): the low nibble is the last bits of 1024 + q, the high one those of 64 + q where it lies.  Two of
+// four byte permutations are shifts, which issue faster (one card, against a shift and four permutations per word: 1003 rows over
+// 4096 x 22016 161.0 -> 158.8 us).
+__device__ __forceinline__ unsigned int nibble_pair(unsigned int w, int j) {
   const unsigned int twice = __builtin_amdgcn_perm(w, w, j < 2 ? 0x01000100u : 0x03020302u);      // a half word in both halves
   return j & 1 ? twice >> 8 : twice;
 }
+
+// No permutation is left where a transposing read brings every byte in both halves of a word: of the eight rows that it takes, row i is
+// twice_row(i) of four, and the words hold rows (0, 1, 0, 1) and (2, 3, 2, 3).  Twice the reads for a sixth less vector work; blocks of 128
+// columns take it (art_gemm_w4.hip).  The small blocks wait for their loads either way and spill in one form (16 rows over 4096 x 4096 7.8 -> 8.3 us),
+// the wide ones have the permutations in the shadow of their products (0 to 1 %).
+__device__ __forceinline__ int twice_row(int i) { return (i & 1) + ((i >> 2) & 1) * 2; }
+__device__ __forceinline__ unsigned int nibbles_of_twice(unsigned int w, int j) { return j & 1 ? w >> 8 : w; }
 
 // What becomes of the product: stored (a residual added), SwiGLU of its gate | up halves, or, of q | k | v with heads of
 // 128 columns, q and k rotated and all three stored where the attention reads them.
