@@ -77,6 +77,13 @@ __device__ __forceinline__ u32x4_t buffer_of(const void* p) {
                  kBufferFlags};
 }
 
+// The unit of block b when runs of 2^shift units go round the eight XCDs (block b runs on XCD b % 8), for a multiple of 8 << shift units;
+// shift 0: unit b.
+__device__ __forceinline__ int unit_of_runs(int b, int shift) {
+  const int i = b >> 3;
+  return (i >> shift << (shift + 3)) + ((b & 7) << shift) + (i & ((1 << shift) - 1));
+}
+
 // A base address that is the same for every lane, in scalar registers whatever surrounds the load.
 __device__ __forceinline__ const void* uniform(const void* p) {
   const unsigned long long v = (unsigned long long)p;

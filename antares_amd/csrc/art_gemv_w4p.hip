@@ -102,7 +102,7 @@ __device__ __forceinline__ float wave_sum_all(float v) {
 // tile_stride  bytes between tiles
 #define ART_W4P_PARAMS                                                                                                        \
   const _Float16 *x, const unsigned char *packed, const _Float16 *norm_w, const _Float16 *residual, unsigned int tile_stride, \
-      int K, _Float16 *y, float inv_n, float eps, Magic magic
+      int K, int run_shift, _Float16 *y, float inv_n, float eps, Magic magic
 
 // EPI 0: y[n] = fp16(product);  1: + residual;  2: columns 0..7 of a tile are a gate, 8..15 the matching up
 // projection: y[tile * 8 + j] = fp16(silu(fp16(gate_j)) * fp16(up_j)) (line :171 of the sample; N/2 outputs).
@@ -140,7 +140,7 @@ __global__ __launch_bounds__(64 * kMaxWaves) void gemv_w4p_kernel(ART_W4P_PARAMS
   u32x4 wa[8];
   unsigned int sca, za;
   _Float16 resa = (_Float16)0;
-  int tile = blockIdx.x;
+  const int tile = art::unit_of_runs(blockIdx.x, run_shift);
   issue(tile, wa, sca, za, resa);
   __builtin_amdgcn_sched_barrier(0);                        // nothing below moves above the loads
 
@@ -318,7 +318,7 @@ __global__ __launch_bounds__(256) void gemv_w4q_kernel(ART_W4P_PARAMS) {
     n0v = np[0];
     n1v = np[1];
   }
-  const int tile = blockIdx.x;
+  const int tile = art::unit_of_runs(blockIdx.x, run_shift);
   const unsigned char* wp = packed + (size_t)tile * tile_stride + (size_t)wave * kChunkBytes;
   u32x4 w[8];
 #pragma unroll
@@ -512,13 +512,16 @@ extern "C" int art_gemv_w4p(const void* x_dev, const void* packed_dev, void* y_d
   // blocks of one tile write y while blocks of other tiles still read x: only the residual may alias y
   ART_REQUIRE(!art::overlaps(x_dev, (size_t)K * 2, y_dev, y_bytes), "art_gemv_w4p: y must not overlap x (it may alias the residual)");
   const int tiles = N / kTileCols, waves = chunks_of(K);
-  const int blocks = tiles;
+  // Runs of up to 32 tiles go round the XCDs: of q | k | v with 8, 16, 24 or 32 heads the columns of 1, 2, 1 or 4 heads each of q, k and v, which the
+  // attention's blocks of these heads then read where they were written (art_llm.hip).
+  int run_shift = 0;
+  while (run_shift < 5 && tiles % (16 << run_shift) == 0) ++run_shift;
   const Magic magic{0x000F000Fu, 0x00F000F0u, 0x64006400u, 0x54005400u};
-  const dim3 grid(blocks), block(64 * waves);
+  const dim3 grid(tiles), block(64 * waves);
   hipStream_t st = (hipStream_t)stream;
 #define ART_W4P_ARGS                                                                                                          \
   (const _Float16*)x_dev, (const unsigned char*)packed_dev, (const _Float16*)norm_weight_dev, (const _Float16*)residual_dev, \
-      (unsigned int)tile_stride_of(K), K, (_Float16*)y_dev, 1.0f / (float)K, eps, magic
+      (unsigned int)tile_stride_of(K), K, run_shift, (_Float16*)y_dev, 1.0f / (float)K, eps, magic
 #define ART_W4P_LAUNCH(NORM, EPI)                                                          \
   do {                                                                                    \
     if (quad_form(K)) gemv_w4q_kernel<NORM, EPI><<<grid, dim3(256), 0, st>>>(ART_W4P_ARGS);    \

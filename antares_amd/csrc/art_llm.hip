@@ -254,7 +254,8 @@ __global__ __launch_bounds__(kAttThreads) void attention_kernel(const QT* __rest
   __shared__ float s_k[D], s_v[D];
   // x / parts for x below 2^30: inv_parts = ceil(2^32 / parts)
   auto over_parts = [&](unsigned int x) { return (int)(__umulhi(x, (unsigned int)inv_parts) + x * (unsigned int)(inv_parts >> 32)); };
-  const int h = blockIdx.x, part = blockIdx.y, tid = threadIdx.x;
+  // runs of 1, 2 or 4 heads go round the XCDs, as the tiles of q | k | v that hold them do (art_gemv_w4p.hip)
+  const int h = art::unit_of_runs(blockIdx.x, heads & 7 ? 0 : heads & 8 ? 0 : heads & 16 ? 1 : 2), part = blockIdx.y, tid = threadIdx.x;
   const int sub = tid & 7, group = tid >> 3, wave = tid >> 6, lane = tid & 63;
   const size_t row = (size_t)heads * D;
   // From here to the first use of a cache row the code is one straight line for every lane: all loads are issued
