@@ -103,7 +103,8 @@ struct Sizes {
   int chunks, splits;          // chunks of K, cut into `splits` slices
   int slice, longer;           // chunks of a slice; the first `longer` slices have one more
   int blocks;
-  art::Div tiles, shorter;     // row_tiles * col_tiles, the smaller of the two
+  int by_tile;                 // blocks are numbered by tile, then slice, not the other way round
+  art::Div inner, shorter;     // splits or tiles, the smaller of row_tiles and col_tiles
 };
 
 // BT: B is [N, K].  TM, TN: 32 x 32 tiles of a wavefront along rows and columns.
@@ -125,11 +126,12 @@ __global__ __launch_bounds__(kThreads, TM * TN == 4 || (sizeof(T) == 4 && (TN ==
   // trips and five divisions in front of the first load (float32 240 x 552 x 3200 19.8 -> 19.4 us, 336 x 320 x 1080 10.6 -> 9.8,
   // float16 159 x 776 x 2472 9.0 -> 8.6, 200 x 600 x 760 7.0 -> 6.6; int8 as before).
   asm volatile("" ::"s"(A), "s"(B), "s"(z.M), "s"(z.N), "s"(z.K), "s"(z.row_tiles), "s"(z.col_tiles), "s"(z.slice), "s"(z.longer), "s"(z.blocks),
-               "s"(z.tiles.mul), "s"(z.tiles.shift), "s"(z.tiles.by), "s"(z.shorter.mul), "s"(z.shorter.shift), "s"(z.shorter.by));
-  const int unit = xcd_unit(blockIdx.x, z.blocks), split = (int)art::over((unsigned)unit, z.tiles), tile = unit - split * (int)z.tiles.by;
+               "s"(z.inner.mul), "s"(z.inner.shift), "s"(z.inner.by), "s"(z.by_tile), "s"(z.shorter.mul), "s"(z.shorter.shift), "s"(z.shorter.by));
+  const int unit = xcd_unit(blockIdx.x, z.blocks), outer = (int)art::over((unsigned)unit, z.inner), rest = unit - outer * (int)z.inner.by;
+  const int split = z.by_tile ? rest : outer, tile = z.by_tile ? outer : rest;
   // neighbours along the shorter side of the grid of tiles
   const int along = (int)art::over((unsigned)tile, z.shorter), across = tile - along * (int)z.shorter.by;
-  const int tm = z.row_tiles <= z.col_tiles ? across : along, tn = z.row_tiles <= z.col_tiles ? along : across;
+  const int tm = z.row_tiles < z.col_tiles ? across : along, tn = z.row_tiles < z.col_tiles ? along : across;
   const int m0 = tm * BM, n0 = tn * BN;
   const int first = split * z.slice + (split < z.longer ? split : z.longer), count = z.slice + (split < z.longer ? 1 : 0);
 
@@ -351,12 +353,20 @@ __global__ __launch_bounds__(kThreads, TM * TN == 4 || (sizeof(T) == 4 && (TN ==
   }
 }
 
-// C = sum of the slices' tiles, in order.  Four neighbouring elements per thread, eight slices requested at a time.
+// C = sum of the slices' tiles, in order.  Block b takes the eighth b % 8 of the columns of `rows` rows of 4 `quads` elements (rows 1: of all
+// elements; 0: blocks in order).  Four neighbouring elements per thread, eight slices requested at a time.
 template <typename Sum, typename Total, typename Out>
-__global__ __launch_bounds__(256) void gemm_tile_sum_kernel(const Sum* __restrict__ partial, Out* __restrict__ C, long long count, int splits) {
+__global__ __launch_bounds__(256) void gemm_tile_sum_kernel(const Sum* __restrict__ partial, Out* __restrict__ C, long long count, int splits, int rows, int quads, art::Div eighth) {
   typedef Sum sum4 __attribute__((ext_vector_type(4), aligned(4)));
   typedef Total total4 __attribute__((ext_vector_type(4)));
-  const long long i = ((long long)blockIdx.x * 256 + threadIdx.x) * 4;
+  long long i = (long long)blockIdx.x * 256 + threadIdx.x;
+  if (rows > 0) {
+    const unsigned at = (blockIdx.x >> 3) * 256 + threadIdx.x, row = rows > 1 ? art::over(at, eighth) : at < eighth.by ? 0 : 1;
+    const unsigned quad = (blockIdx.x & 7) * eighth.by + at - row * eighth.by;
+    if ((int)row >= rows || (int)quad >= quads) return;
+    i = (long long)row * quads + quad;
+  }
+  i *= 4;
   if (i >= count) return;
   if (i + 4 <= count) {
     total4 t = __builtin_convertvector(*reinterpret_cast<const sum4*>(partial + i), total4);
@@ -377,6 +387,21 @@ __global__ __launch_bounds__(256) void gemm_tile_sum_kernel(const Sum* __restric
     for (int s = 1; s < splits; ++s) t += (Total)partial[s * count + k];
     C[k] = (Out)t;
   }
+}
+
+// Where the slices are added.  Blocks run on the XCDs in runs; numbered by tile, an XCD has all slices of an eighth of the tiles, which is an
+// eighth of the rows or, where there are more columns of tiles, of the columns, and the pass adds them on that XCD, from its L2.  Numbered by
+// slice, every XCD reads but its part of k of the operands, which is better for few tiles: with 8 to 15 of them 0.98 times as fast by tile, with
+// fewer 0.94.  From 16 on by tile, and columns only where an eighth of them is a line and more of partial sums: 248 such products of up to
+// 4096 x 4096 x 4096 are 1.05 times as fast, five of them more than 3 % slower (up to 9).  us: float16 448 x 512 x 1344 8.0 -> 7.2, 704 x 472 x 2128 11.9 -> 10.2, float32 128 x 1600 x 640
+// 10.1 -> 9.0, int8 3592 x 64 x 3048 8.5 -> 7.3; by slice it stays at 6.2 for int8 128 x 192 x 3328 (7.6 by tile).
+bool in_columns(int N, int row_tiles, int col_tiles) { return row_tiles < col_tiles && N % 4 == 0 && N >= 640; }
+
+template <typename Sum, typename Total, typename Out>
+void launch_sum(const Sum* partial, Out* C, long long count, int splits, int rows, hipStream_t stream) {
+  const long long quads = (count / (rows > 0 ? rows : 1) + 3) / 4, eighth = (quads + 7) / 8;
+  const unsigned blocks = rows > 0 ? 8u * (unsigned)((rows * eighth + 255) / 256) : (unsigned)((quads + 255) / 256);
+  gemm_tile_sum_kernel<Sum, Total, Out><<<dim3(blocks), dim3(256), 0, stream>>>(partial, C, count, splits, rows, (int)quads, art::make_div((unsigned)eighth));
 }
 
 // Forms: 1 = 64 x 64 per block, 2 = 64 x 128, 3 = 128 x 128 (not float32: no registers left for the chunk's sums), 4 = 64 x 64
@@ -534,8 +559,8 @@ int run(const void* a, const void* b, void* c, void* partial, const Sizes& z, in
   if (z.splits == 1) return 0;
   const long long count = (long long)z.M * z.N;
   typedef typename std::conditional<sizeof(T) == 4, double, typename Elem<T>::sum>::type total;
-  gemm_tile_sum_kernel<typename Elem<T>::sum, total, typename Elem<T>::out><<<dim3((unsigned)((count + 1023) / 1024)), dim3(256), 0, st>>>(
-      (const typename Elem<T>::sum*)partial, (typename Elem<T>::out*)c, count, z.splits);
+  launch_sum<typename Elem<T>::sum, total, typename Elem<T>::out>((const typename Elem<T>::sum*)partial, (typename Elem<T>::out*)c, count, z.splits,
+                                                                   z.by_tile ? (z.row_tiles < z.col_tiles ? z.M : 1) : 0, st);
   ART_LAUNCH_CHECK();
   return 0;
 }
@@ -543,7 +568,7 @@ int run(const void* a, const void* b, void* c, void* partial, const Sizes& z, in
 }  // namespace
 
 int art::sum_slices(const float* partial, float* y, long long count, int slices, hipStream_t stream) {
-  gemm_tile_sum_kernel<float, double, float><<<dim3((unsigned)((count + 1023) / 1024)), dim3(256), 0, stream>>>(partial, y, count, slices);
+  launch_sum<float, double, float>(partial, y, count, slices, 0, stream);
   ART_LAUNCH_CHECK();
   return 0;
 }
@@ -565,8 +590,9 @@ extern "C" int art_gemm_tile(const void* a_dev, const void* b_dev, void* c_dev, 
   ART_REQUIRE(!art::overlaps(c_dev, (size_t)M * N * out, a_dev, (size_t)M * K * s) && !art::overlaps(c_dev, (size_t)M * N * out, b_dev, (size_t)N * K * s),
               "art_gemm_tile: the result must not overlap an operand");
   const int row_tiles = (M + rows_of(form) - 1) / rows_of(form), col_tiles = (N + columns_of(form) - 1) / columns_of(form);
-  const Sizes z{M, N, K, row_tiles, col_tiles, chunks, splits, chunks / splits, chunks % splits, row_tiles * col_tiles * splits,
-                art::make_div((unsigned)(row_tiles * col_tiles)), art::make_div((unsigned)(row_tiles < col_tiles ? row_tiles : col_tiles))};
+  const int tiles = row_tiles * col_tiles, by_tile = splits > 1 && tiles >= 16 && (row_tiles >= col_tiles || in_columns(N, row_tiles, col_tiles));
+  const Sizes z{M, N, K, row_tiles, col_tiles, chunks, splits, chunks / splits, chunks % splits, tiles * splits,
+                by_tile, art::make_div((unsigned)(by_tile ? splits : tiles)), art::make_div((unsigned)(row_tiles < col_tiles ? row_tiles : col_tiles))};
   hipStream_t st = (hipStream_t)stream;
   return type == 0 ? run<_Float16, false>(a_dev, b_dev, c_dev, partial_dev, z, form, st)
        : type == 1 ? run<float, false>(a_dev, b_dev, c_dev, partial_dev, z, form, st)

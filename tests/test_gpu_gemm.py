@@ -181,6 +181,33 @@ def test_tile_products_of_every_form(dtype, M, N, chunks, rest):
                 assert bool(((got - want).abs() <= (K + slices) * 2.0 ** -24 * size + 2.0 ** -11 * want.abs() + 2.0 ** -24).all())
 
 
+# rows of tiles, as many columns as rows, columns whose eighths are and are not whole vectors; 16 tiles and numbers that are no multiple of eight
+@pytest.mark.parametrize('M,N', [(1100, 67), (1027, 64), (250, 255), (65, 1000), (130, 644), (64, 1021), (70, 4096)])
+@pytest.mark.parametrize('dtype', list(TILE_TYPES))
+def test_sliced_tile_products_of_sixteen_tiles_and_more(dtype, M, N):
+    """Slices that are numbered by tile and added by eighths of the rows or of the columns, as above: int8 exact, the others within their bounds."""
+    from ctypes import c_void_p
+    from antares_amd.runtime import capi
+    capi.init(0)
+    dev, lib = torch.device('cuda', 0), capi.lib()
+    kind, per = TILE_TYPES[dtype]
+    K = 7 * per + 16 // (2, 4, 1)[kind]
+    a, b, want, size = _tile_operands(dtype, M, N, K, dev, 1)
+    for form, slices in ((1, 2), (1, 8), (2, 3)):
+        print(f'[case] art_gemm_tile {dtype} {M}x{N}x{K} form {form} slices {slices}', flush=True)
+        c = torch.zeros(M, N, dtype=torch.int32 if kind == 2 else getattr(torch, dtype), device=dev)
+        partial = torch.full((slices * M * N,), -7, dtype=torch.int32, device=dev)          # NaN as float32
+        capi.check(lib.art_gemm_tile(*(c_void_p(t.data_ptr()) for t in (a, b, c, partial)), kind, M, N, K, form, slices,
+                                     c_void_p(torch.cuda.current_stream().cuda_stream)))
+        got = c.cpu().double()
+        if kind == 2:
+            assert torch.equal(got, want)
+        elif kind == 1:
+            assert bool(((got - want).abs() <= (32 + 8 + slices) * 2.0 ** -24 * size).all())
+        else:
+            assert bool(((got - want).abs() <= (K + slices) * 2.0 ** -24 * size + 2.0 ** -11 * want.abs() + 2.0 ** -24).all())
+
+
 @pytest.mark.parametrize('chunks,rest', [(1, 0), (2, 3), (3, 0), (4, -1), (7, 5)])
 def test_tile_products_of_more_blocks_than_compute_units(chunks, rest):
     """float16 puts the next chunk into LDS in front of the products with up to 256 blocks, behind them with more: the same sums in
