@@ -10,7 +10,7 @@
 // One block of four wavefronts per (head, tile of 32 queries).  The key tiles 0 .. the block's own are dealt out to the
 // wavefronts in turn, each keeps an online softmax of its share, and the four states are merged through LDS at the end:
 // nothing is computed above the diagonal, no barrier exists in the loop, and the longest chain of tiles - which bounds the
-// launch, 1.6 us a tile with one wavefront per SIMD - is a quarter of the tiles.  With four wavefronts the L2 has to serve the
+// launch, 1.0 us a tile with one wavefront per SIMD - is a quarter of the tiles.  With four wavefronts the L2 has to serve the
 // key tiles: the blocks of a head run on one XCD, those of the heads past a multiple of eight on all.  One wavefront per query
 // tile / four with the blocks of a head wherever they fall / four as here, us: 1003 tokens of 32 heads 50 / 63 / 26, of 31
 // heads 49 / 39 / 27; 4000 tokens of 31 heads 456 / 547 / 276, of 71 heads 917 / 1247 / 653; 128 tokens of 32 heads 8.0 / - / 5.2.
@@ -23,6 +23,11 @@
 //   * O^T += V^T P^T: the probabilities go from the accumulator layout straight into the B operand (the order of
 //     the summed index is free as long as both operands agree), V^T comes out of the row-major V tile through the
 //     transposing LDS read ds_read_b64_tr_b16, with the row quadruples chosen to match that order.
+//   * key tiles come through buffer descriptors: a lane's eight offsets into a tile never change, and rows past the prompt's end read as
+//     zeros.  What bounds a step is its vector instructions, and a comparison and a 64-bit product for each of eight rows were a quarter
+//     of their time: 32 heads, 400 tokens 9.6 -> 9.1 us, 1003 24.8 -> 23.2, 4000 256 -> 236; 8 heads 8.1 -> 7.5, 14.0 -> 12.4, 71 -> 65; up to 256
+//     tokens 1 to 2 %.  Not kept: 64 queries to a block, which share every key tile but leave one wavefront to a SIMD (1003 tokens 25 -> 37 us);
+//     maxima that stay until they have grown by 2^8 (another 4 %, but 3 to 14 % more error: the largest weight is no longer an exact 1);
 //   * the rescaling by 2^(m_old - m_new) is one multiplication per accumulator register, skipped where no maximum grew;
 //     exponentials are of base 2, log2(e) being folded into the scale; only the diagonal tile is masked.
 #include "art_common.h"
@@ -55,7 +60,8 @@ __device__ __forceinline__ float sum_with_lane_xor_32(float v) {
 }
 
 // q: [T, heads, 128]; k, v: rows of kv_stride halves, row s holding [heads, 128]; out: [T, heads, 128]
-template <int kWaves>
+// FAR: the 32 rows of a key tile take 4 GiB and more.
+template <int kWaves, bool FAR>
 __global__ __launch_bounds__(64 * kWaves, 2) void prefill_attention_kernel(const _Float16* __restrict__ q, const _Float16* __restrict__ k,
                                                                 const _Float16* __restrict__ v, _Float16* __restrict__ out, int T,
                                                                 int heads, long long kv_stride, const float* __restrict__ att_f,
@@ -91,13 +97,28 @@ __global__ __launch_bounds__(64 * kWaves, 2) void prefill_attention_kernel(const
   // staging of a K / V tile: 32 rows x 16 chunks of 16 bytes = 8 chunks per lane and matrix
   const int st_row = lane >> 4, st_col = (lane & 15) * 8;      // + 4 rows per i
   u32x4 kreg[8], vreg[8];
+  const unsigned row_bytes = (unsigned)kv_stride * 2u, lane_off = (unsigned)st_row * row_bytes + st_col * 2u;
   auto load_tile = [&](int kt) {
+    if constexpr (FAR) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int key = kt * KT + st_row + 4 * i;
-      const size_t off = (size_t)(key < T ? key : T - 1) * kv_stride + (size_t)h * D + st_col;
-      kreg[i] = *reinterpret_cast<const u32x4*>(k + off);
-      vreg[i] = *reinterpret_cast<const u32x4*>(v + off);
+      for (int i = 0; i < 8; ++i) {
+        const int key = kt * KT + st_row + 4 * i;
+        const size_t off = (size_t)(key < T ? key : T - 1) * kv_stride + (size_t)h * D + st_col;
+        kreg[i] = *reinterpret_cast<const u32x4*>(k + off);
+        vreg[i] = *reinterpret_cast<const u32x4*>(v + off);
+      }
+    } else {
+      // Buffers that end with the head's last row: what lies behind it reads as zeros.
+      const int rows = T - kt * KT < KT ? T - kt * KT : KT;
+      const size_t from = (size_t)(kt * KT) * kv_stride + (size_t)h * D;
+      const unsigned bytes = (unsigned)(rows - 1) * row_bytes + D * 2;
+      const auto kb = __builtin_amdgcn_make_buffer_rsrc(const_cast<_Float16*>(k + from), 0, (int)bytes, art::kBufferFlags);
+      const auto vb = __builtin_amdgcn_make_buffer_rsrc(const_cast<_Float16*>(v + from), 0, (int)bytes, art::kBufferFlags);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        kreg[i] = __builtin_amdgcn_raw_buffer_load_b128(kb, (int)(lane_off + 4u * i * row_bytes), 0, 0);
+        vreg[i] = __builtin_amdgcn_raw_buffer_load_b128(vb, (int)(lane_off + 4u * i * row_bytes), 0, 0);
+      }
     }
   };
   if (wave <= qt) load_tile(wave);
@@ -249,7 +270,9 @@ extern "C" int art_prefill_attention(const void* q_dev, const void* k_dev, const
   const unsigned chunks = (q_tiles + 7) / 8, rows = chunks < 32768 ? chunks : 32768;
   const unsigned a_chunk = chunks > 1 ? 8 * heads : (q_tiles * (heads & 7) + 7) / 8 * 8 + q_tiles * (heads & ~7);
   // one key tile: one wavefront, and no merge
-  const auto kernel = q_tiles == 1 ? prefill_attention_kernel<1> : prefill_attention_kernel<kMaxWaves>;
+  const bool far = kv_row_stride >= 1LL << 26;
+  const auto kernel = q_tiles == 1 ? (far ? prefill_attention_kernel<1, true> : prefill_attention_kernel<1, false>)
+                                   : (far ? prefill_attention_kernel<kMaxWaves, true> : prefill_attention_kernel<kMaxWaves, false>);
   kernel<<<dim3(a_chunk, rows, (chunks + rows - 1) / rows), dim3(q_tiles == 1 ? 64 : 64 * kMaxWaves), 0, (hipStream_t)stream>>>(
       (const _Float16*)q_dev, (const _Float16*)k_dev, (const _Float16*)v_dev, (_Float16*)out_dev, T, heads, kv_row_stride,
       (const float*)att_f_dev, q_tiles);

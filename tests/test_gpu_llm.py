@@ -313,6 +313,37 @@ def test_fused_decode_attention_against_the_oracle(parts, pos):
 
 
 @pytest.mark.usefixtures('oracle_built')
+@pytest.mark.parametrize('stride', [256, 264, (1 << 26) - 8, 1 << 26])       # halves from row to row; from the last on, a tile of them takes 4 GiB
+@pytest.mark.parametrize('T', [1, 31, 32, 33, 40])
+def test_causal_attention_reads_no_row_past_the_prompt(stride, T):
+    """The rows of the cache behind the prompt and beside its heads are NaN; the result is, bit for bit, that of dense rows."""
+    from ctypes import c_void_p
+    from antares_amd.runtime import capi
+    note(f'causal attention T={T} row stride {stride}')
+    capi.init(0)
+    dev, H, D = torch.device('cuda', 0), 2, 128
+    g = torch.Generator().manual_seed(T)
+    q, k, v = (torch.randn(T, H, D, generator=g).half().to(dev) for _ in range(3))
+    att_f = torch.tensor([1 / math.sqrt(D)], dtype=torch.float32, device=dev)
+
+    def call(keys, values, row_stride):
+        out = torch.full((T, H, D), 7.0, dtype=torch.float16, device=dev)
+        capi.check(capi.lib().art_prefill_attention(*(c_void_p(t.data_ptr()) for t in (q, keys, values, att_f, out)), T, H, D, row_stride,
+                                                    c_void_p(torch.cuda.current_stream().cuda_stream)))
+        return out
+
+    rows = [torch.empty((T + 1) * stride, dtype=torch.float16, device=dev).as_strided((T + 1, H, D), (stride, D, 1)) for _ in range(2)]
+    for to, t in zip(rows, (k, v)):
+        to[:T], to[T] = t, float('nan')
+    if stride > H * D:
+        for to in rows:
+            to.as_strided((T + 1, 8), (stride, 1), to.storage_offset() + H * D).fill_(float('nan'))
+    assert torch.equal(call(*rows, stride), call(k, v, H * D))
+    want = torch.softmax((torch.einsum('thd,shd->hts', q.double().cpu(), k.double().cpu()) * float(att_f)).masked_fill(torch.ones(T, T).triu(1).bool(), float('-inf')), 2)
+    want = torch.einsum('hts,shd->thd', want, v.double().cpu())
+    assert torch.allclose(call(k, v, H * D).double().cpu(), want, rtol=1e-2, atol=1e-2)
+
+
 @pytest.mark.parametrize('T,H', [(1, 4), (5, 4), (31, 4), (32, 32), (33, 4), (100, 32), (128, 32), (200, 4), (384, 32)])
 def test_causal_attention_over_a_prompt_against_the_oracle(T, H):
     """attention_causal_f16 (matrix cores, a block of 32 queries) against the oracle's attention applied position by
