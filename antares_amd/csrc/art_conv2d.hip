@@ -27,7 +27,7 @@
 //     20 x 24 -> 64, 20 x 20 12.0 -> 10.5 us (generic 11.4), float16 19 x 19 of 16 channels 8.8 -> 7.3 (7.7 to 8.4);
 //   * 2 x 2 wavefronts of MT x NT tiles of 32 features x 32 points; blocks of one run of points are neighbours on one XCD.
 // Measured, padding 1, both launches, against the generic lowering (a padded copy, then a gathering product): float16
-// 32 x 128 x 28 x 28 -> 128 40.2 -> 17.3 us, 24 x 200 x 33 x 33 -> 48 89 -> 23 us, 2 x 160 x 18 x 18 -> 64 57 -> 14 us;
+// 32 x 128 x 28 x 28 -> 128 40.2 -> 16.3 us, 24 x 200 x 33 x 33 -> 48 89 -> 23 us, 2 x 160 x 18 x 18 -> 64 57 -> 14 us;
 // float32 32 x 128 x 28 x 28 -> 128 113 -> 81 us (the matrix instructions alone take 47), 23 x 128 x 30 x 30 -> 176 119 -> 86.
 // The first of these (clocks of a block, 27500 in all at 2.1 GHz; its products alone are 9200): 1150 for the places, 3700 until the first
 // image is in LDS, three chunks of 5150 and the last of 3400 (2600 without the filter's loads, which half fill the load path), 2900 for
@@ -43,6 +43,7 @@ namespace {
 using namespace art::conv;
 
 constexpr int kPitchBytes = kChunkBytes + 16;   // from one point to the next in LDS
+#define ART_GLOBAL __attribute__((address_space(1)))
 constexpr unsigned kFirst = 1u, kSecond = 0x80000000u;         // flags beside an offset into x: below 2^31 and even
 constexpr size_t kMaxLds = 64 * 1024, kWideLds = 160 * 1024;     // with more than the first a compute unit holds one block
 
@@ -121,11 +122,20 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 4))
   auto place = [&](int i) { return where[lane + 64 * i < count ? lane + 64 * i : count - 1]; };
   auto fetch = [&](int q, unsigned from, int j, Item& r) {
     const int c0 = (q * 4 + wave) * V, c = c0 + j < g.C ? c0 + j : g.C - 1;               // the same in all lanes
-    const char* p = reinterpret_cast<const char*>(x) + c * plane + (size_t)(from & ~(kFirst | kSecond));
-    if constexpr (F16 && PAIRS) r.v[j] = *reinterpret_cast<const one_word*>(p);
-    else if constexpr (F16) r.v[j] = *reinterpret_cast<const unsigned short*>(p);
-    else if constexpr (PAIRS) r.v[j] = *reinterpret_cast<const two_words*>(p);
-    else r.v[j] = *reinterpret_cast<const unsigned*>(p);
+    const char* base = reinterpret_cast<const char*>(x) + c * plane;
+    unsigned off = from & ~(kFirst | kSecond);
+    if constexpr (F16) {
+      // Scalar base, 32-bit offset: the compiler would add in 64 bits in every lane for every load (34 sizes 1.019 times as fast as so, 32 x 128 x 28 x 28 -> 128
+      // 17.0 -> 16.3 us, 26 x 64 x 31 x 31 -> 112 13.3 -> 12.7; in float32 the products hide it, 0.98 to 1.03).
+      ART_GLOBAL const char* from_base = (ART_GLOBAL const char*)base;
+      asm("" : "+s"(from_base), "+v"(off));
+      if constexpr (PAIRS) r.v[j] = *(ART_GLOBAL const one_word*)(from_base + (size_t)off);
+      else r.v[j] = *(ART_GLOBAL const unsigned short*)(from_base + (size_t)off);
+    } else if constexpr (PAIRS) {
+      r.v[j] = *reinterpret_cast<const two_words*>(base + (size_t)off);
+    } else {
+      r.v[j] = *reinterpret_cast<const unsigned*>(base + (size_t)off);
+    }
   };
   auto put = [&](int q, int i, unsigned from, const Item& r) {
     const int point = P * (lane + 64 * i), c0 = (q * 4 + wave) * V;
