@@ -221,13 +221,16 @@ def _lower_row_group(graph, i: int, count: int, sym: str) -> Tuple[str, RowGroup
             act, oct_ = HIP_TYPE[st.root.dtype], HIP_TYPE[st.out_dtype]
             op = _REDUCE_OP[st.reduce] + '()'
             body.append(f'    {act} __acc_{st.output} = {reduce_identity(st.reduce, st.root.dtype)};')
-            if ragged:                  # the elements of a vector in pairs: the sums are no longer than those of a block with an element per lane
-                body += over_row([f'{act} __p[{V}];'], [f'__p[__k] = {r_ax} >= __s ? ({act})({em.expr(st.root)}) : {reduce_identity(st.reduce, st.root.dtype)};'],
+            value = f'({act})({em.expr(st.root)})'
+            if ragged:
+                value = f'({act})({r_ax} >= __s ? {value} : {reduce_identity(st.reduce, st.root.dtype)})'
+            if ragged and st.reduce not in '<>':      # the elements of a vector in pairs: the sums are no longer than those of a block with an element per lane
+                body += over_row([f'{act} __p[{V}];'], [f'__p[__k] = {value};'],
                                  ['#pragma unroll', f'for (int __w = {V // 2}; __w > 0; __w >>= 1)', '  #pragma unroll',
                                   f'  for (int __k = 0; __k < __w; ++__k) __p[__k] = {op}(__p[__k], __p[__k + __w]);',
                                   f'__acc_{st.output} = {op}(__acc_{st.output}, __p[0]);'])
-            else:
-                body += over_row([], [f'__acc_{st.output} = {op}(__acc_{st.output}, ({act})({em.expr(st.root)}));'], [])
+            else:                       # a NaN is skipped as the second operand of a maximum or minimum and kept as the first: it never becomes that
+                body += over_row([], [f'__acc_{st.output} = {op}(__acc_{st.output}, {value});'], [])
             meet = (f'art_block_reduce(__acc_{st.output}, {op}, __smem_{st.output})' if team == BLOCK
                     else f'{"art_wave_reduce" if team == 64 else "art_row16_reduce"}(__acc_{st.output}, {op})')
             body += [f'    const {oct_} __t_{st.output} = ({oct_}){meet};',

@@ -1307,6 +1307,33 @@ def test_rows_in_vectors_that_start_anywhere(autort, program, dtype, rows, n, of
         assert bool(((got.double() - want)[fine].abs() <= want[fine] * (n + 60) * eps + torch.finfo(t).tiny).all())
 
 
+@pytest.mark.parametrize('reduce', ['>', '<'])
+@pytest.mark.parametrize('rows,n,offset', [(36, 129, 0), (38, 254, 0), (37, 255, 1), (258, 511, 0), (8195, 601, 0), (36, 1026, 0), (41, 4099, 0), (1025, 4100, 0)])       # a form of these kernels each
+def test_extremes_of_rows_in_vectors_that_start_anywhere_skip_a_nan(autort, reduce, rows, n, offset):
+    """A NaN at each place of the first, an inner and the last vector of a row (which overlaps the one before), beside the row's extreme at each
+    other place: as the statements one by one, the row minus the extreme of its other values, to the bit."""
+    note(f'ragged rows {reduce} with NaN {rows} x {n} at {offset}')
+    dev, sign = autort.device(), 1.0 if reduce == '>' else -1.0
+    op = autort.export(ir=f't[N] {reduce}=! x[N, C]; y[N, C] = x[N, C] - t[N]', inputs=['x=float32[N:64, C:200]'], name=f'extreme_{"max" if sign > 0 else "min"}')
+    x = torch.randn(rows, n, generator=torch.Generator().manual_seed(n)) * sign
+    places = [(first, a, b) for first in (0, 64, n - 4) for a in range(4) for b in range(4) if a != b]
+    for row, (first, a, b) in enumerate(places):
+        x[row, first + a], x[row, first + b] = float('nan'), sign * (100 + row)
+    xd = torch.zeros(rows * n + offset, device=dev)[offset:].view(rows, n).copy_(x)
+    group = op.plans[0].row_group
+    assert group.choose_ragged({'N': rows, 'C': n}, {v: (4 * offset if v == 'x' else 0) for v in group.args})[1] > 0
+    together = op(xd).cpu()
+    try:
+        for p in op.plans:
+            p.row_group = None
+        apart = op(xd).cpu()
+    finally:
+        op.plans[0].row_group = group
+    want = x - x.nan_to_num(nan=-sign * 1e30).mul(sign).max(1, keepdim=True).values * sign
+    for got in (together, apart):
+        assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.nan_to_num(), want.nan_to_num())
+
+
 @pytest.mark.parametrize('ir,ta,tb,M,N,K', [
     ('out[M, N] +=! x[K, M] * w[K, N]', True, False, 1028, 512, 96),
     ('out[M, N] +=! x[M, K] * w[N, K]', False, True, 1000, 1030, 64),       # a linear layer: N need not be a multiple of 4

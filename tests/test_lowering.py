@@ -1,5 +1,7 @@
 """Decisions the generic lowering takes from the text of a program alone (no GPU): which statements one row kernel
 may cover, and that the generated source compiles for gfx950."""
+import re
+
 import pytest
 
 from antares_amd.ir import parse_program
@@ -52,6 +54,16 @@ def test_rows_take_vectors_that_start_anywhere_where_they_are_faster(rows, n, of
     assert (sym, grid) == (f'{group.symbol}_{form}', -(-rows // (4 if form[1] == 'w' else 1))) if form else grid == 0
     assert f'void {sym}(' in src
     assert not lowered(SOFTMAX, ['input0=float16[N:32, C:1024]'])[1][0].row_group.ragged
+
+
+@pytest.mark.parametrize('reduce', ['>', '<'])
+def test_no_kernel_over_rows_lets_a_value_be_the_first_operand_of_a_maximum(reduce):
+    """A NaN as second operand is skipped, as the first it stays and takes the other's place: within a lane the first is always what the
+    lane has so far, which starts at the identity."""
+    src, plans = lowered(f't[N] {reduce}=! x[N, C]; y[N, C] = x[N, C] - t[N]', ['x=float32[N:32, C:200]'])
+    assert plans[0].row_group.ragged
+    first = re.findall(r'Op(?:Max|Min)\(\)\((.+?), ', src)
+    assert len(first) > 10 and all(v.startswith('__acc') for v in first), sorted(set(first))
 
 
 @pytest.mark.parametrize('ir,inputs,covered', [
