@@ -373,35 +373,40 @@ __device__ __forceinline__ f32x4 sum_splits(const float* partial, long long spli
   return t;
 }
 
-// Which part of a row the pass adds where: block b runs on XCD b % 8 and takes that eighth of the columns.  The product deals its column
-// tiles, with all their K-splits, to the XCDs in the same order (Deal, art_gemm_w4_deep.hip), so that the sums are in the L2 that they were
-// written to unless the weights have pushed them out.  With rows dealt whole, product and pass, HBM / cache, us: 50 rows over 4096 x 4096 in four
-// splits 11.1 / 9.9, now 9.8 / 8.6, 64 over 8192 x 2048 in eight 11.2 / 10.3 and 10.0 / 9.0, 30 over 5504 x 2048 8.4 / 7.9 and 7.7 / 7.0; over 11008 x 4096
-// (3 MB of weights per XCD) 1 % either way.
-struct Eighth {
-  Div across;                                       // pieces of a row in an eighth
+// Which part of a row the pass adds where: block b runs on XCD b % 8 and takes that eighth of the columns (by_eighths; else whole rows in
+// order).  The product deals its column tiles, with all their K-splits, to the XCDs in the same order (Deal, art_gemm_w4_deep.hip), so that the
+// sums are in the L2 that they were written to unless the weights have pushed them out.  With rows dealt whole, product and pass, HBM / cache, us: 50 rows over
+// 4096 x 4096 in four splits 11.1 / 9.9, now 9.8 / 8.6, 64 over 8192 x 2048 in eight 11.2 / 10.3 and 10.0 / 9.0, 30 over 5504 x 2048 8.4 / 7.9 and 7.7 / 7.0; over
+// 11008 x 4096 (3 MB of weights per XCD) 1 % either way.
+struct Part {
+  Div across;                                       // pieces of a row in a part: an eighth of them, or all
   int pieces;                                       // of a row
   // false: nothing to do
   __device__ __forceinline__ bool take(int rows, unsigned& row, unsigned& piece) const {
-    const unsigned i = (blockIdx.x >> 3) * 256 + threadIdx.x;
+    const bool whole = (int)across.by == pieces;
+    const unsigned i = (whole ? blockIdx.x : blockIdx.x >> 3) * 256 + threadIdx.x;
     row = over(i, across);
-    piece = (blockIdx.x & 7) * across.by + i - row * across.by;
+    piece = i - row * across.by + (whole ? 0 : (blockIdx.x & 7) * across.by);
     return (int)row < rows && (int)piece < pieces;
   }
 };
-inline Eighth eighth(int rows, int pieces, dim3& grid) {
-  const unsigned across = (pieces + 7) / 8;
-  grid = dim3(8u * (unsigned)(((long long)rows * across + 255) / 256));
-  return Eighth{make_div(across), pieces};
-}
+
+// As numbers, which are in registers when a kernel starts; as a struct, which is not, 1 to 3 % slower.
+#define ART_PART_PARAMS unsigned mul, unsigned shift, unsigned across, int pieces
+#define ART_PART (Part{Div{mul, shift, across}, pieces})
 
 // y[m,n] = fp16(sum over splits); four columns per thread (N % 4 == 0).
 template <int SPLITS> __global__ __launch_bounds__(256) void gemm_w4a16_combine_kernel(const float* __restrict__ partial, _Float16* y,
-                                                                  int rows, Eighth quads, long long split_stride, int splits,
-                                                                  const _Float16* residual) {
-  unsigned row, quad;
-  if (!quads.take(rows, row, quad)) return;
-  const long long i = (long long)row * quads.pieces + quad;
+                                                                  const _Float16* residual, long long split_stride,
+                                                                  int splits, int rows, ART_PART_PARAMS) {
+  long long i = (long long)blockIdx.x * 256 + threadIdx.x;
+  if ((int)across == pieces) {
+    if (i >= (long long)rows * pieces) return;
+  } else {
+    unsigned row, quad;
+    if (!ART_PART.take(rows, row, quad)) return;
+    i = (long long)row * pieces + quad;
+  }
   const f32x4 t = sum_splits<SPLITS>(partial + i * 4, split_stride, splits);
   h4 out = h4{(_Float16)t[0], (_Float16)t[1], (_Float16)t[2], (_Float16)t[3]};
   if (residual) {                    // y = fp16(fp16(product) + residual); residual may be y itself
@@ -489,9 +494,9 @@ template <int SPLITS> __global__ __launch_bounds__(kNormThreads) void gemm_w4a16
 
 // The same for gate | up: y[m, n] of N / 2 columns from the sums of columns n and N / 2 + n.
 template <int SPLITS> __global__ __launch_bounds__(256) void gemm_w4a16_combine_swiglu_kernel(const float* __restrict__ partial, _Float16* y, int rows, int N,
-                                                                         int splits, Eighth quads) {   // groups of four output columns
+                                                                         int splits, ART_PART_PARAMS) {   // groups of four output columns
   unsigned m, quad;
-  if (!quads.take(rows, m, quad)) return;
+  if (!ART_PART.take(rows, m, quad)) return;
   const long long row = m, col = quad * 4, stride = (long long)rows * N;
   const f32x4 g = sum_splits<SPLITS>(partial + row * N + col, stride, splits), u = sum_splits<SPLITS>(partial + row * N + N / 2 + col, stride, splits);
   *reinterpret_cast<h4*>(y + row * (N / 2) + col) = swiglu4(h4{(_Float16)g[0], (_Float16)g[1], (_Float16)g[2], (_Float16)g[3]},
@@ -499,12 +504,12 @@ template <int SPLITS> __global__ __launch_bounds__(256) void gemm_w4a16_combine_
 }
 
 // The same for q | k | v: columns j .. j + 3 of a head and their partners 64 further on, rotated in q and k.
-template <int SPLITS> __global__ __launch_bounds__(256) void gemm_w4a16_combine_rope_kernel(const float* __restrict__ partial, int rows, int splits, Rope rope, Eighth pieces) {      // 48 heads of them
+template <int SPLITS> __global__ __launch_bounds__(256) void gemm_w4a16_combine_rope_kernel(const float* __restrict__ partial, int rows, int splits, ART_PART_PARAMS, Rope rope) {      // 48 heads of them
   unsigned m, at;
-  if (!pieces.take(rows, m, at)) return;
-  const long long row = m, stride = (long long)rows * pieces.pieces * 8;
+  if (!ART_PART.take(rows, m, at)) return;
+  const long long row = m, stride = (long long)rows * pieces * 8;
   const int head = at >> 4, j = (at & 15) * 4;
-  const float* const from = partial + (row * pieces.pieces * 8 + head * 128 + j);
+  const float* const from = partial + (row * pieces * 8 + head * 128 + j);
   const f32x4 first = sum_splits<SPLITS>(from, stride, splits), second = sum_splits<SPLITS>(from + 64, stride, splits);
   h4 a = h4{(_Float16)first[0], (_Float16)first[1], (_Float16)first[2], (_Float16)first[3]};
   h4 b = h4{(_Float16)second[0], (_Float16)second[1], (_Float16)second[2], (_Float16)second[3]};
@@ -631,20 +636,19 @@ struct Norm {
 template <int SPLITS>
 void launch_combine(const float* partial, _Float16* y, int rows, int N, int splits, const _Float16* residual, Tail tail, const Norm* norm,
                     const Rope& rope, hipStream_t stream) {
-  dim3 grid;
+  const int pieces = tail == kPlain ? N / 4 : N / 8;
+  const Div across = make_div((unsigned)(by_eighths(N, tail) ? (pieces + 7) / 8 : pieces));
+  const unsigned blocks = (unsigned)(((long long)rows * across.by + 255) / 256) * ((int)across.by == pieces ? 1 : 8);
   if (norm) {
     const int threads = N < 8 * kNormThreads ? (N / 8 + 63) / 64 * 64 : kNormThreads;
     gemm_w4a16_combine_norm_kernel<SPLITS><<<dim3(rows), threads, 0, stream>>>(partial, residual, (const _Float16*)norm->weight, y, (long long)rows * N, N, splits,
                                                                                threads, norm->eps, (_Float16*)norm->out);
   } else if (tail == kRope) {
-    const Eighth pieces = eighth(rows, N / 8, grid);
-    gemm_w4a16_combine_rope_kernel<SPLITS><<<grid, 256, 0, stream>>>(partial, rows, splits, rope, pieces);
+    gemm_w4a16_combine_rope_kernel<SPLITS><<<blocks, 256, 0, stream>>>(partial, rows, splits, across.mul, across.shift, across.by, pieces, rope);
   } else if (tail == kSwiglu) {
-    const Eighth quads = eighth(rows, N / 8, grid);
-    gemm_w4a16_combine_swiglu_kernel<SPLITS><<<grid, 256, 0, stream>>>(partial, y, rows, N, splits, quads);
+    gemm_w4a16_combine_swiglu_kernel<SPLITS><<<blocks, 256, 0, stream>>>(partial, y, rows, N, splits, across.mul, across.shift, across.by, pieces);
   } else {
-    const Eighth quads = eighth(rows, N / 4, grid);
-    gemm_w4a16_combine_kernel<SPLITS><<<grid, 256, 0, stream>>>(partial, y, rows, quads, (long long)rows * N, splits, residual);
+    gemm_w4a16_combine_kernel<SPLITS><<<blocks, 256, 0, stream>>>(partial, y, residual, (long long)rows * N, splits, rows, across.mul, across.shift, across.by, pieces);
   }
 }
 int combine(const float* partial, _Float16* y, int rows, int N, int splits, const _Float16* residual, Tail tail, const Norm* norm, const Rope& rope,

@@ -42,21 +42,23 @@ constexpr size_t lds_bytes(int XR, int CT) { return (size_t)kWaves * wave_bytes(
 template <int XR, int CT, Tail TAIL>
 __global__ __launch_bounds__(kThreads, XR == 16 ? 4 : 2) void gemm_w4a16_deep_kernel(
     const _Float16* __restrict__ x, const unsigned char* __restrict__ qweight, const _Float16* __restrict__ scales,
-    const unsigned char* __restrict__ qzeros, int K, int N, int M, int tiles, unsigned int inv_splits, int each, int m_blocks, unsigned int inv_blocks, _Float16* y, float* __restrict__ partial,
+    const unsigned char* __restrict__ qzeros, int K, int N, int M, int inner, unsigned int inv_inner, int each, int units, int m_blocks, unsigned int inv_blocks, _Float16* y, float* __restrict__ partial,
     int splits, int groups_of_split, int longer, Magic mg, const _Float16* residual, Rope rope) {
   constexpr int MT = XR == 64 ? 2 : 1, BN = 32 * CT, W_BYTES = w_bytes(CT);
   constexpr int XL = XR / 4, WL = W_BYTES / 1024;   // loads of x and of the packed weights per group
   extern __shared__ __align__(1024) unsigned char smem[];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  asm volatile("" ::"s"(units), "s"(m_blocks), "s"(inv_blocks), "s"(splits), "s"(groups_of_split), "s"(longer));      // all of them are asked for before the first branch
   int unit = (blockIdx.x & 7) * each + (blockIdx.x >> 3);            // (tile, K split, block of rows); neighbours on one XCD
-  if (unit >= tiles * splits * m_blocks) return;
+  if (unit >= units) return;
   int m0 = 0;
   if (m_blocks > 1) {
     const int block = unit;
     unit = (int)__umulhi(block, inv_blocks);        // block / m_blocks
     m0 = (block - unit * m_blocks) * XR;
   }
-  const int tile = inv_splits ? (int)__umulhi(unit, inv_splits) : unit, split = unit - tile * splits;      // unit / splits
+  const int across = inner < 0 ? -inner : inner, outer = inv_inner ? (int)__umulhi(unit, inv_inner) : unit, rest = unit - outer * across;      // unit / across
+  const int tile = inner < 0 ? rest : outer, split = inner < 0 ? outer : rest;
   const int g_begin = split * groups_of_split + (split < longer ? split : longer), g_count = groups_of_split + (split < longer ? 1 : 0);
   const int mine = (g_count - wave + kWaves - 1) / kWaves;           // groups wave, wave + 8, ... of the split
 
@@ -266,8 +268,10 @@ int art::w4::gemm_deep(const _Float16* x, const unsigned char* qweight, const _F
   }
   const int rows = M <= 16 ? 16 : 32 * row_tiles, m_blocks = (M + rows - 1) / rows, form = (rows == 16 ? 0 : rows == 32 ? 1 : 2) + (col_tiles == 2 ? 3 : 0);
   const int tiles = deep_tiles(N, tail, col_tiles), units = tiles * splits * m_blocks, each = (units + 7) / 8, G = K / GK;
+  const bool by_tile = by_eighths(N, tail);
+  const int across = by_tile ? splits : tiles;      // units next to each other: splits of a tile, or tiles of a split
   kernels[form][tail]<<<dim3(8 * each), kThreads, lds[form], stream>>>(
-      x, qweight, scales, qzeros, K, N, M, tiles, (unsigned int)((0x100000000ull + splits - 1) / splits), each, m_blocks,
+      x, qweight, scales, qzeros, K, N, M, by_tile ? across : -across, (unsigned int)((0x100000000ull + across - 1) / across), each, units, m_blocks,
       (unsigned int)((0x100000000ull + m_blocks - 1) / m_blocks), y, partial, splits, G / splits,
       G % splits, kMagic, residual, rope);
   ART_LAUNCH_CHECK();

@@ -173,6 +173,15 @@ inline Deal deal(int units, int m_blocks, dim3& grid) {
   return Deal{units / 8, m_blocks, left, (left + 7) / 8};
 }
 
+// Whether the pass that adds K-splits takes each row by eighths, on the XCDs that wrote them, and art_gemm_w4_deep.hip numbers its units by
+// column tile for that; else whole rows in order, and units by split: an XCD then reads one split's part of x, not all of them.  By eighths
+// from 2560 columns on, and below where an eighth of a row's sums (pieces of 16 bytes, two of them where a gate and its up
+// projection or the two halves of a head meet) is whole lines of memory: else two XCDs fetch the lines between.  Against rows dealt whole, in the mean over 4 to
+// 1000 rows and K of 2048 to 11008 (weights in the cache): 16 to 208 columns 0.87 to 0.95 times as fast (400 rows of 11008 over 64 columns 9.4 us, whole 7.2),
+// 256 1.07, 384 0.99, 512 1.04, 640 0.99, 1024 1.07, 1152 0.98, 1536 1.03, 2320 0.98, 2768 1.01, 3024 1.02, 4096 1.03, 5520 1.03; gate | up of 320 columns 0.89, 512 1.01,
+// 768 0.97, 1024 1.04, 1088 0.98, 2048 1.04, 4128 1.01, 4992 1.02; q | k | v of one head 0.92, 3 0.98, 4 1.02, 6 0.99, 8 1.01, 9 1.01, 11 1.03.
+inline bool by_eighths(int N, Tail tail) { return N >= 2560 || (tail == kPlain ? N / 4 : N / 8) % 64 == 0; }
+
 // fp16(silu(gate) * up) of fp16 operands in fp32.  silu is half as many instructions as expf and a division (every fp16 gate gives
 // the same fp16 value): 1003 rows over 4096 x 22016 with SWIGLU 186.4 -> 184.1 us.
 __device__ __forceinline__ h4 swiglu4(h4 g, h4 u) {

@@ -790,6 +790,43 @@ def test_int4_products_of_a_few_rows_over_blocks_of_32_and_64_columns(autort, M,
         near(hid, silu * up, 1.1 * rg * up.abs() + silu.abs() * ru + 1.1 * rg * ru + (silu * up).abs() * 2.0 ** -20)
 
 
+# widths on both sides of the rule that has a row's sums added by eighths: whole lines (gate | up: twice as many columns) or not, few and many columns
+@pytest.mark.parametrize('N', [32, 224, 256, 288, 512, 2528, 2544, 2560, 2592])
+@pytest.mark.parametrize('M', [5, 70, 300])
+def test_int4_products_whose_k_splits_are_added_by_eighths_or_by_rows(autort, M, N):
+    """Blocks of every kind, plain and SwiGLU.  Bounds as in the test above."""
+    from ctypes import c_void_p
+    from antares_amd.runtime import capi
+    capi.init(0)
+    dev, lib, stream, K = autort.device(), capi.lib(), c_void_p(torch.cuda.current_stream().cuda_stream), 1152
+
+    def near(got, want, room):
+        assert ((got.double() - want).abs() <= want.abs() * 2.0 ** -11 + room + 2.0 ** -25).all(), ((got.double() - want).abs() - room).max()
+    g = torch.Generator(device=dev).manual_seed(M + N)
+    q = torch.randint(0, 256, (K // 2, N), generator=g, device=dev, dtype=torch.uint8)
+    z = torch.randint(0, 256, (K // 128, N // 2), generator=g, device=dev, dtype=torch.uint8)
+    s = (torch.rand(K // 128, N, generator=g, device=dev) * 0.019 + 0.001).half()
+    x = torch.randn(M, K, generator=g, device=dev).half()
+    zero = torch.stack([z & 15, z >> 4], 2).reshape(K // 128, N).half().repeat_interleave(128, 0)
+    w = ((torch.stack([q & 15, q >> 4], 1).reshape(K, N).half() - zero) * s.repeat_interleave(128, 0)).double()
+    want, room = x.double() @ w, (x.double().abs() @ w.abs()) * K * 2.0 ** -24
+    gate, up = want[:, :N // 2], want[:, N // 2:]
+    rg, ru = room[:, :N // 2] + gate.abs() * 2.0 ** -11, room[:, N // 2:] + up.abs() * 2.0 ** -11
+    silu = torch.nn.functional.silu(gate)
+    for code in (256 + 2, 512 + 3, 1024 + 2, 2304 + 2, 2304 + 9, 2560 + 3, 2816 + 2):
+        if (code >> 8) >= 9 and M > (512 if code >> 8 == 11 else 256):
+            continue                                         # more rows than eight of the small blocks
+        for tail in (0, 1) if N % 32 == 0 else (0,):
+            note(f'splits by eighths or rows M={M} N={N} code={code} tail={tail}')
+            assert lib.art_gemm_w4a16_form(M, K, N, tail, 0, code) == code
+            out = torch.full((M, N >> tail), float('nan'), dtype=torch.float16, device=dev)
+            capi.check((lib.art_gemm_w4a16_swiglu if tail else lib.art_gemm_w4a16_tuned)(*(c_void_p(t.data_ptr()) for t in (x, q, s, z, out)), M, K, N, code, stream))
+            if tail:
+                near(out, silu * up, 1.1 * rg * up.abs() + silu.abs() * ru + 1.1 * rg * ru + (silu * up).abs() * 2.0 ** -20)
+            else:
+                near(out, want, room)
+
+
 @pytest.mark.parametrize('form', [9, 10, 11])
 @pytest.mark.parametrize('M', [1, 4, 16, 17, 32, 33, 64, 65, 131, 250])
 def test_int4_products_in_small_blocks_by_their_launch_parameter(autort, M, form):
