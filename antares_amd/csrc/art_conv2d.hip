@@ -292,10 +292,10 @@ size_t lds_of(int span) { return (size_t)span * (2 * kPitchBytes + 4); }
 
 // Forms: 1 = 64 features x 64 points per block, 2 = 64 x 128, 3 = 128 x 128; 4, 5, 6 the same over the staged image, 7 = 64 x 64
 // there with short sums (float32), plus 256 x slices of the channels (0: one); 8, 9, 10 = 16 features x 16, 32, 64 points (art_conv2d_direct.hip).
-bool direct(int form) { return (form & 255) > 7; }
+bool direct(int form) { return form >= 8 && form <= 10; }
 int shape_of(int form) { return (form & 255) % 3; }
 int features_of(int form) { return direct(form) ? 16 : shape_of(form) == 0 ? 128 : 64; }
-int points_of(int form) { return direct(form) ? 16 << ((form & 255) - 8) : shape_of(form) == 1 ? 64 : 128; }
+int points_of(int form) { return direct(form) ? 16 << (form - 8) : shape_of(form) == 1 ? 64 : 128; }
 int slices_of(int form) { return form >> 8 ? form >> 8 : 1; }
 
 bool geometry(Geometry& g, int f16, int N, int C, int H, int W, int F, int HO, int WO, int ph, int pw) {

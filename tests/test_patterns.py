@@ -177,6 +177,15 @@ def test_convolutions_in_one_launch_take_whole_pieces_of_the_filter_and_short_ru
     assert [v for v in (8, 9, 10) if capi.lib().art_conv2d_form(f16, n, c, hw, hw, 32, hw, hw, 1, 1, v)] == forms
 
 
+@pytest.mark.parametrize('form', [-8, 11, 12, 40, 41, 255, 256 + 8, 256 + 40, 512 + 10, 1 << 30])
+@pytest.mark.parametrize('f16', [0, 1])
+def test_convolutions_refuse_forms_that_there_are_not(f16, form):
+    """No entry works with a number that names no form (a shift by the difference to 8 is as long as one likes)."""
+    lib, shape = capi.lib(), (f16, 2, 16, 9, 9, 32, 9, 9, 1, 1)
+    assert lib.art_conv2d_form(*shape, form) == lib.art_conv2d_exact_enough(*shape, form) == lib.art_conv2d_scratch_bytes(*shape, form) == 0
+    assert lib.art_conv2d(None, None, None, None, *shape, form, None) != 0 and f'form {form}' in lib.art_last_error().decode()
+
+
 @pytest.mark.parametrize('f16,n,c,h,w,f', [(1, 64, 512, 128, 128, 512), (0, 64, 64, 100, 100, 17), (1, 256, 64, 112, 112, 64), (0, 32, 256, 56, 56, 256),
                                            (1, 2, 2048, 14, 14, 2048), (0, 1, 40, 12000, 60, 48), (0, 9, 216, 17, 17, 64)])
 def test_convolutions_take_a_bounded_copy_of_the_image(f16, n, c, h, w, f):
