@@ -356,13 +356,14 @@ __global__ __launch_bounds__(kThreads, TM * TN == 4 || (sizeof(T) == 4 && (TN ==
 // C = sum of the slices' tiles, in order.  Block b takes the eighth b % 8 of the columns of `rows` rows of 4 `quads` elements (rows 1: of all
 // elements; 0: blocks in order).  Four neighbouring elements per thread, eight slices requested at a time.
 template <typename Sum, typename Total, typename Out>
-__global__ __launch_bounds__(256) void gemm_tile_sum_kernel(const Sum* __restrict__ partial, Out* __restrict__ C, long long count, int splits, int rows, int quads, art::Div eighth) {
+__global__ __launch_bounds__(256) void gemm_tile_sum_kernel(const Sum* __restrict__ partial, Out* __restrict__ C, long long count, int splits, int rows, int quads,
+                                                           unsigned mul, unsigned shift, unsigned by) {      // Div of an eighth, as numbers: these are in registers when a kernel starts
   typedef Sum sum4 __attribute__((ext_vector_type(4), aligned(4)));
   typedef Total total4 __attribute__((ext_vector_type(4)));
   long long i = (long long)blockIdx.x * 256 + threadIdx.x;
   if (rows > 0) {
-    const unsigned at = (blockIdx.x >> 3) * 256 + threadIdx.x, row = rows > 1 ? art::over(at, eighth) : at < eighth.by ? 0 : 1;
-    const unsigned quad = (blockIdx.x & 7) * eighth.by + at - row * eighth.by;
+    const unsigned at = (blockIdx.x >> 3) * 256 + threadIdx.x, row = rows > 1 ? art::over(at, art::Div{mul, shift, by}) : at < by ? 0 : 1;
+    const unsigned quad = (blockIdx.x & 7) * by + at - row * by;
     if ((int)row >= rows || (int)quad >= quads) return;
     i = (long long)row * quads + quad;
   }
@@ -391,17 +392,27 @@ __global__ __launch_bounds__(256) void gemm_tile_sum_kernel(const Sum* __restric
 
 // Where the slices are added.  Blocks run on the XCDs in runs; numbered by tile, an XCD has all slices of an eighth of the tiles, which is an
 // eighth of the rows or, where there are more columns of tiles, of the columns, and the pass adds them on that XCD, from its L2.  Numbered by
-// slice, every XCD reads but its part of k of the operands, which is better for few tiles: with 8 to 15 of them 0.98 times as fast by tile, with
-// fewer 0.94.  From 16 on by tile, and columns only where an eighth of them is a line and more of partial sums: 248 such products of up to
-// 4096 x 4096 x 4096 are 1.05 times as fast, five of them more than 3 % slower (up to 9).  us: float16 448 x 512 x 1344 8.0 -> 7.2, 704 x 472 x 2128 11.9 -> 10.2, float32 128 x 1600 x 640
+// slice, every XCD reads but its part of k of the operands.  By tile
+//  * from 16 tiles on: with 8 to 15 of them 0.98 times as fast by tile, with fewer 0.94;
+//  * an eighth of the columns only with 800 of them and more, or of whole lines (partial sums, N % 256 == 0): of 640 to 800 others 8 of 21 were 3 to
+//    5 % slower by tile, 1.00 times as fast in the mean;
+//  * as long as an XCD's L2 (4 MiB) holds the operands that it reads then, an eighth of the longer one and all of the other.  Beyond that
+//    0.97 times as fast in float16 (633 x 1136 x 3597 20.9 us by slice, 24.0 by tile), up to it 1.05; float32, more bound by its products, 1.015 between 4 and
+//    6 MiB, 0.99 beyond.
+// Over 490 products of 16 tiles and more, up to 4096 x 4096 x 4096, 1.03 times as fast as all by slice, at worst 7 % slower.  us, by slice and by tile: float16 448 x 512 x 1344 8.0 -> 7.2, 704 x 472 x 2128 11.9 -> 10.2, float32 128 x 1600 x 640
 // 10.1 -> 9.0, int8 3592 x 64 x 3048 8.5 -> 7.3; by slice it stays at 6.2 for int8 128 x 192 x 3328 (7.6 by tile).
-bool in_columns(int N, int row_tiles, int col_tiles) { return row_tiles < col_tiles && N % 4 == 0 && N >= 640; }
+bool numbered_by_tile(int type, int M, int N, int K, int row_tiles, int col_tiles) {
+  const long long longer = M > N ? M : N, shorter = M > N ? N : M;
+  return (long long)row_tiles * col_tiles >= 16 && (row_tiles >= col_tiles || (N % 4 == 0 && N >= 640 && (N >= 800 || N % 256 == 0))) &&
+         (longer / 8 + shorter) * K * (type == 0 ? 2 : type == 1 ? 4 : 1) <= (type == 1 ? 6LL << 20 : 4LL << 20);
+}
 
 template <typename Sum, typename Total, typename Out>
 void launch_sum(const Sum* partial, Out* C, long long count, int splits, int rows, hipStream_t stream) {
   const long long quads = (count / (rows > 0 ? rows : 1) + 3) / 4, eighth = (quads + 7) / 8;
   const unsigned blocks = rows > 0 ? 8u * (unsigned)((rows * eighth + 255) / 256) : (unsigned)((quads + 255) / 256);
-  gemm_tile_sum_kernel<Sum, Total, Out><<<dim3(blocks), dim3(256), 0, stream>>>(partial, C, count, splits, rows, (int)quads, art::make_div((unsigned)eighth));
+  const art::Div of = art::make_div((unsigned)eighth);
+  gemm_tile_sum_kernel<Sum, Total, Out><<<dim3(blocks), dim3(256), 0, stream>>>(partial, C, count, splits, rows, (int)quads, of.mul, of.shift, of.by);
 }
 
 // Forms: 1 = 64 x 64 per block, 2 = 64 x 128, 3 = 128 x 128 (not float32: no registers left for the chunk's sums), 4 = 64 x 64
@@ -590,7 +601,7 @@ extern "C" int art_gemm_tile(const void* a_dev, const void* b_dev, void* c_dev, 
   ART_REQUIRE(!art::overlaps(c_dev, (size_t)M * N * out, a_dev, (size_t)M * K * s) && !art::overlaps(c_dev, (size_t)M * N * out, b_dev, (size_t)N * K * s),
               "art_gemm_tile: the result must not overlap an operand");
   const int row_tiles = (M + rows_of(form) - 1) / rows_of(form), col_tiles = (N + columns_of(form) - 1) / columns_of(form);
-  const int tiles = row_tiles * col_tiles, by_tile = splits > 1 && tiles >= 16 && (row_tiles >= col_tiles || in_columns(N, row_tiles, col_tiles));
+  const int tiles = row_tiles * col_tiles, by_tile = splits > 1 && numbered_by_tile(type, M, N, K, row_tiles, col_tiles);
   const Sizes z{M, N, K, row_tiles, col_tiles, chunks, splits, chunks / splits, chunks % splits, tiles * splits,
                 by_tile, art::make_div((unsigned)(by_tile ? splits : tiles)), art::make_div((unsigned)(row_tiles < col_tiles ? row_tiles : col_tiles))};
   hipStream_t st = (hipStream_t)stream;

@@ -208,6 +208,35 @@ def test_sliced_tile_products_of_sixteen_tiles_and_more(dtype, M, N):
             assert bool(((got - want).abs() <= (K + slices) * 2.0 ** -24 * size + 2.0 ** -11 * want.abs() + 2.0 ** -24).all())
 
 
+# on both sides of what an XCD's L2 holds (an eighth of the longer operand and the other: 4 MiB, float32 6), and of the widths whose columns are cut
+@pytest.mark.parametrize('M,N,K', [('L2', 0, 0), ('L2', 0, 64), ('L2', 1, 0), ('L2', 1, 64), (64, 768, 704), (64, 784, 704), (64, 796, 700), (64, 800, 704), (130, 640, 715)])
+@pytest.mark.parametrize('dtype', list(TILE_TYPES))
+def test_sliced_tile_products_numbered_by_tile_and_by_slice(dtype, M, N, K):
+    """As above: int8 exact, the others within their bounds."""
+    from ctypes import c_void_p
+    from antares_amd.runtime import capi
+    capi.init(0)
+    dev, lib = torch.device('cuda', 0), capi.lib()
+    kind, per = TILE_TYPES[dtype]
+    if M == 'L2':
+        most, (M, N) = (4 << 20, 6 << 20, 4 << 20)[kind] // (2, 4, 1)[kind], ((576, 192), (192, 832))[N]
+        K += most // (max(M, N) // 8 + min(M, N)) // 16 * 16
+    a, b, want, size = _tile_operands(dtype, M, N, K, dev, 1)
+    for form, slices in ((1, 2), (1, 5), (2, 3)):
+        print(f'[case] art_gemm_tile {dtype} {M}x{N}x{K} form {form} slices {slices}', flush=True)
+        c = torch.zeros(M, N, dtype=torch.int32 if kind == 2 else getattr(torch, dtype), device=dev)
+        partial = torch.full((slices * M * N,), -7, dtype=torch.int32, device=dev)          # NaN as float32
+        capi.check(lib.art_gemm_tile(*(c_void_p(t.data_ptr()) for t in (a, b, c, partial)), kind, M, N, K, form, slices,
+                                     c_void_p(torch.cuda.current_stream().cuda_stream)))
+        got = c.cpu().double()
+        if kind == 2:
+            assert torch.equal(got, want)
+        elif kind == 1:
+            assert bool(((got - want).abs() <= (32 + (K + 31) // 32 + slices) * 2.0 ** -24 * size).all())
+        else:
+            assert bool(((got - want).abs() <= (K + slices) * 2.0 ** -24 * size + 2.0 ** -11 * want.abs() + 2.0 ** -24).all())
+
+
 @pytest.mark.parametrize('chunks,rest', [(1, 0), (2, 3), (3, 0), (4, -1), (7, 5)])
 def test_tile_products_of_more_blocks_than_compute_units(chunks, rest):
     """float16 puts the next chunk into LDS in front of the products with up to 256 blocks, behind them with more: the same sums in
