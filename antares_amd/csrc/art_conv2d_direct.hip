@@ -254,6 +254,11 @@ Layout layout_of(const Geometry& g, int f16, int NT) {
   return l;
 }
 
+size_t lds_of(const Layout& l, int NT) {
+  const size_t sums = (size_t)l.waves * 16 * 16 * NT * 8, own = (size_t)l.waves * l.wave_bytes;
+  return own > sums ? own : sums;
+}
+
 template <typename T, int NT, int KP>
 int launch(const void* x, const void* w, void* y, const Geometry& g, const Layout& l, hipStream_t st) {
   static bool configured = false;
@@ -262,8 +267,7 @@ int launch(const void* x, const void* w, void* y, const Geometry& g, const Layou
     configured = true;
   }
   const Direct d{l.units, l.segment, make_div((unsigned)((l.segment + 16 * NT - 1) / (16 * NT))), l.pitch, l.wave_bytes, (uintptr_t)w % 16 == 0};
-  const size_t sums = (size_t)l.waves * 16 * 16 * NT * 8, bytes = (size_t)l.waves * l.wave_bytes > sums ? (size_t)l.waves * l.wave_bytes : sums;
-  conv2d_direct_kernel<T, NT, KP><<<dim3((unsigned)l.blocks), dim3(64 * l.waves), bytes, st>>>((const T*)x, (const T*)w, (float*)y, g, d);
+  conv2d_direct_kernel<T, NT, KP><<<dim3((unsigned)l.blocks), dim3(64 * l.waves), lds_of(l, NT), st>>>((const T*)x, (const T*)w, (float*)y, g, d);
   ART_LAUNCH_CHECK();
   return 0;
 }
@@ -284,6 +288,10 @@ bool art::conv::direct_fits(const Geometry& g, int f16, int form) {
 // What a form takes, in microseconds: a fixed part, for each round of a block's wavefronts over the channels a time that grows with
 // their number and with the points that a lane brings, and for blocks that share a compute unit, or do so unevenly, a time per unit of
 // channels.  Fitted to 1465 times of 580 sizes, a third of them outside of 16 to 256 channels and features and 7 to 56 squared: 6 to 8 % off.
+// Float16 blocks of which LDS holds two to a compute unit, five to seven wavefronts that take all channels in one turn over rows of some 40 to 128 points, take 1.3
+// times that beyond one round (up to 2.0): 47 x 80 x 16 x 104 -> 11 34.6 us in another form, 59.9 here.  What is taken instead is 1.30 times as fast
+// in the mean of 32 sizes of 60000 (up to 256 images, 1024 channels, 512 features, 128 x 128).  Not in float32 or for several turns: where it chose
+// between the forms here, 0.90 and 0.75 to 0.95 times.
 double art::conv::direct_time(const Geometry& g, int f16, int form) {
   struct Cost { double fixed, round, image, wave, shared, image_shared, uneven, image_uneven; };
   static const Cost cost[2][3] = {{{3.538, 0.0, 0.183, 0.183, 0.223, 0.058, 0.309, 0.026}, {4.356, 0.0, 0.178, 0.270, 0.362, 0.046, 0.0, 0.182}, {4.910, 1.472, 0.231, 0.290, 0.884, 0.010, 1.080, 0.0}},
@@ -292,8 +300,9 @@ double art::conv::direct_time(const Geometry& g, int f16, int form) {
   const Layout l = layout_of(g, f16, 1 << (form - 8));
   const int items = (l.points + 63) / 64, turns = (l.units + l.waves - 1) / l.waves;
   const double rounds = (double)l.blocks / 256, full = rounds > 1 ? rounds : 1, uneven = ceil(rounds) > full ? ceil(rounds) - full : 0;
-  return c.fixed + turns * (c.round + c.image * items + c.wave * l.waves) +
-         l.units * ((c.shared + c.image_shared * items) * (full - 1) + (c.uneven + c.image_uneven * items) * uneven);
+  const bool pairs = f16 && items == kMostPoints && turns == 1 && rounds > 1 && kLds / lds_of(l, 1 << (form - 8)) == 2;
+  return c.fixed + (pairs ? 1.3 : 1.0) * (turns * (c.round + c.image * items + c.wave * l.waves) +
+                                          l.units * ((c.shared + c.image_shared * items) * (full - 1) + (c.uneven + c.image_uneven * items) * uneven));
 }
 
 int art::conv::run_direct(const void* x, const void* w, void* y, const Geometry& g, int f16, int form, hipStream_t st) {

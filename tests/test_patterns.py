@@ -170,6 +170,14 @@ def test_convolutions_in_one_launch_where_that_was_measured_to_be_faster(f16, n,
     assert bool(capi.lib().art_conv2d_direct(f16, n, c, hw, hw, f, hw, hw, 1, 1)) == (direct < before)
 
 
+@pytest.mark.parametrize('f16,n,c,f,h,w,before,direct', [
+    (1, 47, 80, 11, 16, 104, 34.6, 59.9), (1, 72, 88, 4, 14, 103, 46.8, 79.9), (1, 95, 88, 1, 16, 83, 40.5, 58.9), (1, 37, 80, 2, 3, 97, 10.8, 13.1),
+    (0, 22, 88, 10, 116, 65, 333, 136), (0, 87, 36, 6, 3, 63, 35.3, 14.5)])
+def test_convolutions_of_wide_images_in_one_launch_where_that_was_measured_to_be_faster(f16, n, c, f, h, w, before, direct):
+    """Blocks of which a compute unit holds two; times in us on an MI355X."""
+    assert bool(capi.lib().art_conv2d_direct(f16, n, c, h, w, f, h, w, 1, 1)) == (direct < before)
+
+
 @pytest.mark.parametrize('f16,n,c,hw,forms', [(1, 2, 8, 9, [8, 9, 10]), (1, 2, 12, 9, []), (0, 2, 12, 9, [8, 9, 10]), (0, 2, 6, 9, []), (0, 2, 8, 100, [8, 9]), (0, 2, 8, 110, [8]),
                                               (0, 2, 8, 120, []), (0, 1, 8, 15, [8, 9, 10])])
 def test_convolutions_in_one_launch_take_whole_pieces_of_the_filter_and_short_runs(f16, n, c, hw, forms):
