@@ -331,7 +331,8 @@ long long blocks_of(const Geometry& g, int form) {
 // What a form takes, in microseconds, both launches: a fixed part, per chunk of a block a time that grows with the blocks that
 // share a compute unit and with how unevenly they do, a ramp per further round, and the stores.  Fitted to 330 sizes a form in float16 and
 // 310 in float32, two thirds of them of 16 to 256 channels and features, images of 7 to 56 squared and batches of 1 to 32: 5 and 1 to 3 % off.
-// (float16 64 x 64: 0.45 above the fit; where it is that close, the staged form with its shorter first fetch stays.)
+// (float16 64 x 64: its fixed part, 5.95, is 0.45 above that fit, which would have it taken at 7 % of 20000 sizes where now another form, mostly the staged
+// 64 x 64, is.  At 200 of these the one taken now is 1.064 times as fast in the mean, at 127 by more than 5 %, at six slower by more than 5 %, up to 8.)
 constexpr int kUnits = 256;                      // compute units of an MI355X
 double launch_time(const Geometry& g, int f16, int form) {
   struct Cost { double fixed, alone, shared, uneven, again, store; };

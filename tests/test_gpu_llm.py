@@ -312,7 +312,6 @@ def test_fused_decode_attention_against_the_oracle(parts, pos):
     assert np.array_equal(kg[keep], kc.numpy()[keep]) and np.array_equal(vg[keep], vc.numpy()[keep])
 
 
-@pytest.mark.usefixtures('oracle_built')
 @pytest.mark.parametrize('stride', [256, 264, (1 << 26) - 8, 1 << 26])       # halves from row to row; from the last on, a tile of them takes 4 GiB
 @pytest.mark.parametrize('T', [1, 31, 32, 33, 40])
 def test_causal_attention_reads_no_row_past_the_prompt(stride, T):
@@ -344,6 +343,7 @@ def test_causal_attention_reads_no_row_past_the_prompt(stride, T):
     assert torch.allclose(call(k, v, H * D).double().cpu(), want, rtol=1e-2, atol=1e-2)
 
 
+@pytest.mark.usefixtures('oracle_built')
 @pytest.mark.parametrize('T,H', [(1, 4), (5, 4), (31, 4), (32, 32), (33, 4), (100, 32), (128, 32), (200, 4), (384, 32)])
 def test_causal_attention_over_a_prompt_against_the_oracle(T, H):
     """attention_causal_f16 (matrix cores, a block of 32 queries) against the oracle's attention applied position by
