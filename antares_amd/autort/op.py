@@ -251,7 +251,7 @@ class ExportedOp(calls.Operator):
                 if not grid:
                     sym, grid = group.choose_short(env, pointers)
                 if grid:
-                    call.kernel(module.function(sym), grid, 256, [bound[n] for n in group.args] + dims)
+                    call.kernel(module.function(group.choose_stores(sym, env)), grid, 256, [bound[n] for n in group.args] + dims)
                     skip = group.count - 1
                     continue
             for n in plan.args:

@@ -149,10 +149,10 @@ def _lower_row_group(graph, i: int, count: int, sym: str) -> Tuple[str, RowGroup
     vector_ok = vmax > 1 and all(e is None or _multiple_of(e, vmax, r_ax) for _, e, _ in slots.values()) and \
         all(tensors[n.name].shape[-1] == r_ext or len(n.args) == 1 for n, _, _ in slots.values())
 
-    # written once and read by nobody here: past the caches (softmax of 32096 x 1003 50.0 -> 46.5 us, of 8192 x 500 11.9 -> 11.1)
+    # written once and read by nobody here: large results go past the caches, in kernels of their own (RowGroup.choose_stores)
     streamed = m is not None and sum(1 for st in graph.statements if m.output in st.reads or m.output == st.output) == 1
 
-    def emit(symbol: str, team: int, V: int, E: int, ragged: bool = False) -> str:
+    def emit(symbol: str, team: int, V: int, E: int, ragged: bool = False, past: bool = False) -> str:
         """team lanes per row, E vectors of V elements per lane held in registers (E == 0: the row is walked).  ragged: rows of
         any length from V on that start anywhere: the vectors are aligned like their elements, and the last one of a row ends with
         it - what it shares with the one before is left out of the reductions and stored twice."""
@@ -236,7 +236,7 @@ def _lower_row_group(graph, i: int, count: int, sym: str) -> Tuple[str, RowGroup
             body += [f'    const {oct_} __t_{st.output} = ({oct_}){meet};',
                      f'    if ({lane} == 0) {st.output}[{plain.offset(st.output, [plain.expr(ix) for ix in st.out_index])}] = __t_{st.output};']
         def store(value, to):
-            return f'__builtin_nontemporal_store({value}, {to});' if streamed else f'*{to} = {value};'
+            return f'__builtin_nontemporal_store({value}, {to});' if past else f'*{to} = {value};'
         if m is not None and V > 1:
             to = f'(__{"mem" if ragged else "vec"}_out*)&{m.output}[{plain.offset(m.output, d_idx + ["__r0"])}]'
             body += over_row(['__vec_out __out;'], [f'__out[__k] = ({oct_m})({em.expr(m.root)});'], [store('__out', to)])
@@ -245,25 +245,28 @@ def _lower_row_group(graph, i: int, count: int, sym: str) -> Tuple[str, RowGroup
         body += ['  }', '}']
         return '\n'.join(body)
 
-    group = RowGroup(symbol=sym, args=args, count=count, row_axes=D, red_axis=(r_ax, r_ext), pure=m is None)
-    code = [emit(sym, BLOCK, 1, 0)]
+    group = RowGroup(symbol=sym, args=args, count=count, row_axes=D, red_axis=(r_ax, r_ext), pure=m is None, out_bytes=ITEMSIZE[m.out_dtype] if m is not None else 0)
+    code = []
+
+    def add(name: str, team: int, V: int, E: int, ragged: bool = False, past: bool = streamed) -> str:
+        code.append(emit(name, team, V, E, ragged))
+        if past:
+            group.past[name] = name + '_past'
+            code.append(emit(name + '_past', team, V, E, ragged, past=True))
+        return name
+    add(sym, BLOCK, 1, 0)
     if slots:
         group.vec_tensors = sorted(set(row_tensors) | ({m.output} if m is not None else set()))
         for V in sorted({1, vmax if vector_ok else 1}):
             for team, E in ((64, 4), (BLOCK, 4), (BLOCK, 16)):
-                name = f'{sym}_{"w" if team == 64 else "b"}{E}' + (f'v{V}' if V > 1 else '')
-                group.cached.append((team, V, E, name))
-                code.append(emit(name, team, V, E))
+                group.cached.append((team, V, E, add(f'{sym}_{"w" if team == 64 else "b"}{E}' + (f'v{V}' if V > 1 else ''), team, V, E)))
         if m is not None and widest == 4 and all(ITEMSIZE[tensors[t].dtype] == 4 for t in row_tensors + [m.output]):
             for team, E in ((64, 1), (64, 2), (64, 4), (BLOCK, 2), (BLOCK, 8)):
-                name = f'{sym}_r{"w" if team == 64 else "b"}{E}'
-                group.ragged.append((team, vmax, E, name))
-                code.append(emit(name, team, vmax, E, ragged=True))
+                # (the first is taken for fewer rows than a large result has)
+                group.ragged.append((team, vmax, E, add(f'{sym}_r{"w" if team == 64 else "b"}{E}', team, vmax, E, ragged=True, past=streamed and (team, E) != (64, 1))))
         if m is not None and (not isinstance(r_ext, int) or 16 <= r_ext < 128):
             for V, E in ((1, 2), (1, 4), (1, 8)) + (((min(vmax, 4), 8 // min(vmax, 4)),) if vector_ok else ()):
-                name = f'{sym}_q{E}' + (f'v{V}' if V > 1 else '')
-                group.short.append((V, E, name))
-                code.append(emit(name, 16, V, E))
+                group.short.append((V, E, add(f'{sym}_q{E}' + (f'v{V}' if V > 1 else ''), 16, V, E)))
         if group.short:
             code.insert(0, _ROW16)
     return '\n\n'.join(code), group

@@ -1307,6 +1307,25 @@ def test_rows_in_vectors_that_start_anywhere(autort, program, dtype, rows, n, of
         assert bool(((got.double() - want)[fine].abs() <= want[fine] * (n + 60) * eps + torch.finfo(t).tiny).all())
 
 
+@pytest.mark.parametrize('rows,n,form', [(65537, 67, 'q8'), (8193, 255 + 1, 'w4v4'), (8193, 257, 'rw2'), (8193, 601, 'rw4'), (2049, 1024, 'b4v4'), (2101, 1025, 'rb2'), (1100, 4100, 'rb8'), (257, 8196, 'b16v4'), (129, 16391, '')])
+def test_large_results_of_rows_past_the_caches(autort, rows, n, form):
+    """A kernel that stores past the caches gives the bits of the one that does not."""
+    note(f'rows past the caches {rows} x {n}')
+    op = autort.export(ir=SHORT_ROWS['softmax'], inputs=['input0=float32[N:64, C:100]'], name='past_softmax')
+    x = torch.randn(rows, n, generator=torch.Generator().manual_seed(n)).to(autort.device())
+    group, taken = op.plans[0].row_group, []
+    choose = group.choose_stores
+    try:
+        group.choose_stores = lambda sym, env: taken.append(choose(sym, env)) or taken[-1]
+        past = op(x).clone()
+        group.choose_stores = lambda sym, env: sym
+        through = op(x)
+    finally:
+        del group.choose_stores
+    assert taken == [f'{group.symbol}{"_" + form if form else ""}_past']
+    assert torch.equal(past, through) and torch.allclose(past, torch.softmax(x, 1), rtol=1e-4, atol=1e-7)
+
+
 @pytest.mark.parametrize('reduce', ['>', '<'])
 @pytest.mark.parametrize('rows,n,offset', [(36, 129, 0), (38, 254, 0), (37, 255, 1), (258, 511, 0), (8195, 601, 0), (36, 1026, 0), (41, 4099, 0), (1025, 4100, 0)])       # a form of these kernels each
 def test_extremes_of_rows_in_vectors_that_start_anywhere_skip_a_nan(autort, reduce, rows, n, offset):

@@ -56,6 +56,19 @@ def test_rows_take_vectors_that_start_anywhere_where_they_are_faster(rows, n, of
     assert not lowered(SOFTMAX, ['input0=float16[N:32, C:1024]'])[1][0].row_group.ragged
 
 
+def test_results_of_rows_go_past_the_caches_from_eight_megabytes_on():
+    src, plans = lowered(SOFTMAX, ['input0=float32[N:32, C:1024]'])
+    group = plans[0].row_group
+    kernels = [group.symbol] + [k[-1] for k in group.cached + group.ragged + group.short]
+    assert set(kernels) - set(group.past) == {f'{group.symbol}_rw1'}          # taken up to 8191 rows of 256 columns
+    assert group.choose_stores(kernels[1], {'N': 2047, 'C': 1024}) == kernels[1]
+    assert group.choose_stores(kernels[1], {'N': 2048, 'C': 1024}) == group.past[kernels[1]]
+    bodies = dict(re.findall(r'void (\w+)\((.*?)(?=extern|\Z)', src, re.S))
+    for sym in kernels:
+        assert '__builtin_nontemporal_store' not in bodies[sym]
+        assert sym not in group.past or '__builtin_nontemporal_store' in bodies[group.past[sym]]
+
+
 @pytest.mark.parametrize('reduce', ['>', '<'])
 def test_no_kernel_over_rows_lets_a_value_be_the_first_operand_of_a_maximum(reduce):
     """A NaN as second operand is skipped, as the first it stays and takes the other's place: within a lane the first is always what the
