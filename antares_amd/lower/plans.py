@@ -89,8 +89,8 @@ class RowGroup(_Rule):
         elements to 16 bytes, softmax and layer normalisation in float32, `choose` / this (us):
           * up to 64 V, a wavefront per row: 4487 x 167 6.9 / 4.8, 912 x 152 3.9 / 3.1, 2 x 140 3.2 / 2.7; there is one in `choose` for 8192 rows
             and more (10806 x 132 4.8 / 4.9, 56548 x 157 18.8 / 24.4);
-          * up to 128 V, with 256 rows and more (in whole vectors below 8192): 62446 x 339 65.7 / 43.3, 5045 x 435 6.7 / 5.4, 418 x 344 3.8 / 3.5; with
-            fewer rows a block has each of them sooner (60 x 470 3.3 / 3.6);
+          * up to 128 V, with 512 rows and more (in whole vectors below 8192): 62446 x 339 65.7 / 43.3, 5045 x 435 6.7 / 5.4; with 256 to 511 a block has
+            each of them sooner (66 sizes, 0.93 to 0.95 times as fast here; with 512 to 767 0.99 to 1.01, beyond 1.02 to 1.08), with fewer too (60 x 470 3.3 / 3.6);
           * up to 256 V, with 8192 rows and more that are not whole vectors: 30000 x 701 31 / 27, 10328 x 513 11.0 / 9.9; 2400 x 555 5.7 / 6.2;
           * 256 to 512 V, not whole vectors, a block per row: 766 x 1113 5.5 / 4.8, 8814 x 1454 25.8 / 24.3;
           * 1024 to 2048 V, eight vectors per lane: rows that are not whole vectors were walked (6012 x 4973 77 / 51, 70 x 7558 8.9 / 6.6); whole
@@ -105,7 +105,7 @@ class RowGroup(_Rule):
         if n <= 64 * V:
             form = (64, 1) if rows < 8192 else None
         elif n <= 128 * V:
-            form = (64, 2) if rows >= 256 and (rows < 8192 or not whole) else None
+            form = (64, 2) if rows >= 512 and (rows < 8192 or not whole) else None
         elif n <= 256 * V:
             form = (64, 4) if rows >= 8192 and not whole else None
         elif n <= 512 * V:

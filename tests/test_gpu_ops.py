@@ -1274,7 +1274,7 @@ def test_rows_of_fewer_than_two_wavefronts(autort, program, dtype, rows, n, offs
 
 # vectors that start anywhere: the first and the last length of every form, rows of whole vectors at odd addresses, rows that end inside a block
 @pytest.mark.parametrize('program,dtype', [('softmax', 'float32'), ('sum', 'int32')])
-@pytest.mark.parametrize('rows,n,offset', [(3, 128, 0), (7, 129, 0), (5, 253, 1), (1001, 256, 0), (259, 257, 0), (258, 511, 0), (257, 512, 1), (8195, 513, 0), (8193, 1023, 0), (8193, 1024, 3),
+@pytest.mark.parametrize('rows,n,offset', [(3, 128, 0), (7, 129, 0), (5, 253, 1), (1001, 256, 0), (515, 257, 0), (514, 511, 0), (513, 512, 1), (8195, 513, 0), (8193, 1023, 0), (8193, 1024, 3),
                                            (2, 1025, 0), (1, 2047, 2), (3, 4097, 0), (2, 8191, 0), (1025, 8192, 0)])
 def test_rows_in_vectors_that_start_anywhere(autort, program, dtype, rows, n, offset):
     """One kernel, and the statements one by one: exact for whole numbers, else both within (n + 8) roundings of the sums, the exponentials and the
@@ -1327,7 +1327,7 @@ def test_large_results_of_rows_past_the_caches(autort, rows, n, form):
 
 
 @pytest.mark.parametrize('reduce', ['>', '<'])
-@pytest.mark.parametrize('rows,n,offset', [(36, 129, 0), (38, 254, 0), (37, 255, 1), (258, 511, 0), (8195, 601, 0), (36, 1026, 0), (41, 4099, 0), (1025, 4100, 0)])       # a form of these kernels each
+@pytest.mark.parametrize('rows,n,offset', [(36, 129, 0), (38, 254, 0), (37, 255, 1), (514, 511, 0), (8195, 601, 0), (36, 1026, 0), (41, 4099, 0), (1025, 4100, 0)])       # a form of these kernels each
 def test_extremes_of_rows_in_vectors_that_start_anywhere_skip_a_nan(autort, reduce, rows, n, offset):
     """A NaN at each place of the first, an inner and the last vector of a row (which overlaps the one before), beside the row's extreme at each
     other place: as the statements one by one, the row minus the extreme of its other values, to the bit."""

@@ -44,7 +44,7 @@ def test_softmax_is_one_row_group_with_kernels_for_short_and_long_rows():
 
 
 @pytest.mark.parametrize('rows,n,offset,form', [
-    (32, 128, 0, 'rw1'), (32, 255, 4, 'rw1'), (8192, 255, 0, None), (255, 300, 0, None), (256, 300, 0, 'rw2'), (8192, 300, 0, None), (8192, 301, 0, 'rw2'), (8192, 300, 4, 'rw2'),
+    (32, 128, 0, 'rw1'), (32, 255, 4, 'rw1'), (8192, 255, 0, None), (511, 300, 0, None), (512, 300, 0, 'rw2'), (8192, 300, 0, None), (8192, 301, 0, 'rw2'), (8192, 300, 4, 'rw2'),
     (8191, 600, 4, None), (8192, 601, 0, 'rw4'), (8192, 600, 0, None), (5, 1025, 0, 'rb2'), (5, 1028, 0, None), (5, 2049, 0, None), (5, 4097, 0, 'rb8'), (1023, 4100, 0, None),
     (1024, 4100, 0, 'rb8'), (1024, 8193, 0, None), (32, 127, 0, None)])
 def test_rows_take_vectors_that_start_anywhere_where_they_are_faster(rows, n, offset, form):
