@@ -15,8 +15,8 @@
 //     number, so that both are in one row): what bounds a chunk beside its products is the number of these loads and of the lines
 //     that each touches.  16-byte LDS writes put a lane's 8 or 4 channels side by side; 80 bytes from point to point keep reads
 //     and writes on distinct banks.  Against a point per load, padding read from the first point of the image, and all loads
-//     with the first three taps (one card, us): float16 32 x 128 x 28 x 28 -> 128 19.3 -> 17.7, 32 x 256 x 14 x 14 -> 256 28.1 -> 22.9, 16 x 256 x 28 x 28 -> 256
-//     31.5 -> 27.4, 26 x 120 x 37 x 37 -> 32 18.6 -> 16.7; float32 32 x 128 x 28 x 28 -> 128 79.7 -> 77.5;
+//     with the first three taps (one card, us; in float16 with the scalar bases below): float16 32 x 128 x 28 x 28 -> 128 18.3 -> 16.0, 32 x 256 x 14 x 14 -> 256
+//     28.0 -> 22.6, 16 x 256 x 28 x 28 -> 256 31.1 -> 26.7, 26 x 120 x 37 x 37 -> 32 18.7 -> 17.9; float32 32 x 128 x 28 x 28 -> 128 79.8 -> 78.2;
 //   * the offset of each pair of points, and which of them are inside, is worked out once per block;
 //   * the filter is packed first, by a launch of its own, in the order in which wavefronts feed it to the matrix
 //     instructions: [64 bytes of channels][tap][32 features][half][lane] with 16 bytes per lane, so that a wavefront's
@@ -27,9 +27,9 @@
 //     20 x 24 -> 64, 20 x 20 12.0 -> 10.5 us (generic 11.4), float16 19 x 19 of 16 channels 8.8 -> 7.3 (7.7 to 8.4);
 //   * 2 x 2 wavefronts of MT x NT tiles of 32 features x 32 points; blocks of one run of points are neighbours on one XCD.
 // Measured, padding 1, both launches, against the generic lowering (a padded copy, then a gathering product): float16
-// 32 x 128 x 28 x 28 -> 128 40.2 -> 16.3 us, 24 x 200 x 33 x 33 -> 48 89 -> 23 us, 2 x 160 x 18 x 18 -> 64 57 -> 14 us;
-// float32 32 x 128 x 28 x 28 -> 128 113 -> 81 us (the matrix instructions alone take 47), 23 x 128 x 30 x 30 -> 176 119 -> 86.
-// The first of these (clocks of a block, 27500 in all at 2.1 GHz; its products alone are 9200): 1150 for the places, 3700 until the first
+// 32 x 128 x 28 x 28 -> 128 40.2 -> 16.0 us, 24 x 200 x 33 x 33 -> 48 89 -> 23 us, 2 x 160 x 18 x 18 -> 64 57 -> 14 us;
+// float32 32 x 128 x 28 x 28 -> 128 113 -> 78 us (the matrix instructions alone take 47), 23 x 128 x 30 x 30 -> 176 119 -> 86.
+// The first of these, before its loads had scalar bases (17 us; clocks of a block, 27500 in all at 2.1 GHz; its products alone are 9200): 1150 for the places, 3700 until the first
 // image is in LDS, three chunks of 5150 and the last of 3400 (2600 without the filter's loads, which half fill the load path), 2900 for
 // the stores of 12.8 MB; packing the filter takes 2.3 us.  Without effect: the filter nine taps ahead, and blocks of four wavefronts
 // along the features, which load the filter once and read each point four times from LDS.
