@@ -13,7 +13,7 @@
 //            the caller chooses otherwise, served by L2) to get the number of
 //            evens up to the end of its span and the total; then, tile by tile, from the last
 //            one to the first (what count read last is still in the L2 of the XCD that
-//            both blocks b run on: 16777216 values 35.8 -> 34.0 us, 33554432 66.7 -> 64.9, up to 8388608 the same), it ranks
+//            both blocks b run on: 16777216 values 35.8 -> 34.0 us, 33554432 66.7 -> 64.9, up to 4000000 the same, 8000000 15.4 -> 15.7), it ranks
 //            the even values with wavefront ballots (v_mbcnt for the lanes below,
 //            a population count for the total) + a 4-wave prefix through LDS, compacts evens
 //            and odds of the tile in LDS and writes both runs with fully
